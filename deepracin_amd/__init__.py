@@ -119,6 +119,8 @@ def load_library(path=None):
         "dR_printNetObject": (None, [vp, c_char_p]),
         "dR_getOutputShape": (POINTER(Shape3), [vp]),
         "dR_getFeedNodeInputShape": (POINTER(Shape3), [vp]),
+        "dR_feedDataHWC": (None, [vp, vp, vp]),
+        "dR_downloadOutputs": (c_int, [vp, POINTER(vp), c_int]),
         "dR_downloadArray": (None, [vp, c_char_p, vp, c_size_t, c_size_t, vp]),
         "dR_uploadArray": (c_int, [vp, c_char_p, vp, c_size_t, c_size_t, vp]),
         "dR_createFloatBuffer": (c_int, [vp, POINTER(vp), c_int, c_int]),
@@ -192,6 +194,8 @@ def load_library(path=None):
         "drhip_staging_download_capacity": (c_size_t, [vp]),
         "drhip_upload_staged": (c_int, [vp, vp, c_size_t, vp, c_size_t, vp]),
         "drhip_download_staged": (c_int, [vp, vp, vp, c_size_t, c_size_t, vp]),
+        "drhip_upload_staged_interleaved": (c_int, [vp, vp, vp, c_size_t, c_int, vp]),
+        "drhip_download_staged_many": (c_int, [vp, c_int, POINTER(vp), POINTER(vp), POINTER(c_size_t), vp]),
         "drhip_fc_permute_rows_f32": (c_int, [vp, vp] + [c_int] * 4 + [vp]),
         "drhip_softmax_f32": (c_int, [vp, vp, c_int, vp]),
         "drhip_copy3d_f32": (c_int, [vp] + [c_int] * 5 + [vp] + [c_int] * 8 + [vp]),
@@ -346,17 +350,15 @@ def _from_chw(graph, flat, shape):
 
 def download_outputs(graph, squeeze=True):
     """Fetch every output buffer (blocking) in the graph's interface layout."""
-    lib = graph.lib
-    mem = (c_void_p * max(graph.num_outputs, 1))()
-    n = lib.dR_getOutputBuffers(graph.ptr, mem)
-    outs = []
-    for i in range(n):
-        s = graph.outnodes[i].out_shape
-        flat = np.empty(s[0] * s[1] * s[2], np.float32)
-        lib.dR_downloadArray(graph.ptr, b"output", mem[i], 0, flat.nbytes, flat.ctypes.data_as(c_void_p))
-        arr = _from_chw(graph, flat, s)
-        outs.append(np.squeeze(arr) if squeeze else arr)
-    return outs
+    n = min(graph.num_outputs, 10)
+    shapes = [node.out_shape for node in graph.outnodes[:n]]
+    flats = [np.empty(s[0] * s[1] * s[2], np.float32) for s in shapes]
+    hosts = (c_void_p * max(n, 1))(*[f.__array_interface__["data"][0] for f in flats])
+    got = graph.lib.dR_downloadOutputs(graph.ptr, hosts, n)
+    if n and not got:
+        raise RuntimeError("DR Error: deepRACIN downloading the outputs failed!")
+    outs = [_from_chw(graph, f, s) for f, s in zip(flats[:got], shapes)]
+    return [np.squeeze(a) for a in outs] if squeeze else outs
 
 
 def apply(graph):
@@ -379,13 +381,15 @@ def feed_data(node, data):
         raise TypeError("DR Error: data fed to a feed_node is " + str(data.dtype) + " but needs to be an array of type float32!")
     layout = node.graph.layout
     d = _dr_shape3(layout, list(data.shape))
-    if layout == "WHC":
-        data = data.transpose([2, 1, 0])
-    elif layout == "HWC":
-        data = data.transpose([2, 0, 1])
-    data = np.ascontiguousarray(data)
     if d != list(node.shape):
         raise ValueError("DR Error: data array's dimensions %s do not match node's dimensions %s!" % (d, node.shape))
+    if layout == "HWC":         # goes over as it is; the library brings it into planes on the way to the device
+        data = np.ascontiguousarray(data)
+        node.graph.lib.dR_feedDataHWC(node.graph.ptr, node.ptr, data.__array_interface__["data"][0])
+        return
+    if layout == "WHC":
+        data = data.transpose([2, 1, 0])
+    data = np.ascontiguousarray(data)
     node.graph.lib.dR_feedData(node.graph.ptr, node.ptr, _fptr(data), 0, d[0] * d[1] * d[2])
 
 

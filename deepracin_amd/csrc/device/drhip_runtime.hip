@@ -11,6 +11,8 @@
 
 namespace drhip {
 
+constexpr int kStagingSegments = 10;    // arrays one staged download can take (a graph reports at most 10 outputs)
+
 char* error_slot() {
     static thread_local char msg[512] = "no error";
     return msg;
@@ -57,6 +59,54 @@ __global__ void __launch_bounds__(256) copy_from_host_kernel(float* __restrict__
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride)
         ((f4*)dst)[i] = __builtin_nontemporal_load((const f4*)src + i);
     if (blockIdx.x == 0 && threadIdx.x < n - 4 * n4) dst[4 * n4 + threadIdx.x] = src[4 * n4 + threadIdx.x];
+}
+
+// dst [C][P] (device) = src [P][C] (pinned host memory): an interleaved image on its way to the planar layout.  A
+// workgroup takes 1024 pixels: it reads them over the bus in their own order, 16 bytes per lane and turn (a wave's load
+// is 1 KiB in a row, which is what the bus wants; the bus is what bounds this kernel), and every lane writes four
+// pixels of each channel out of LDS.  The array may end anywhere: the ragged end is moved sample by sample.
+// (224x224x3: 5.6 us on top of the launch, 107 GB/s through memory, like the plain copy above; numpy's transposition
+// of the same array takes the host 70 us.)
+constexpr int kHwcPixels = 1024;
+template <int C>
+__global__ void __launch_bounds__(256) hwc_from_host_kernel(float* __restrict__ dst, const float* __restrict__ src, size_t P, size_t pixels) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));     // (a channel plane starts at any multiple of 4 bytes)
+    __shared__ __attribute__((aligned(16))) float px[kHwcPixels * C];
+    const size_t p0 = (size_t)blockIdx.x * kHwcPixels;
+    const int n = (int)(pixels - p0 < kHwcPixels ? pixels - p0 : kHwcPixels);
+    const int t = threadIdx.x;
+    if (n == kHwcPixels) {
+        f4 v[C];
+#pragma unroll
+        for (int k = 0; k < C; ++k) v[k] = __builtin_nontemporal_load((const f4*)(src + p0 * C) + t + 256 * k);
+#pragma unroll
+        for (int k = 0; k < C; ++k) ((f4*)px)[t + 256 * k] = v[k];
+    } else {
+        for (int i = t; i < n * C; i += 256) px[i] = src[p0 * C + i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        float* d = dst + (size_t)c * P + p0 + 4 * t;
+        if (4 * t + 4 <= n) {
+            *(f4u*)d = f4u{px[4 * t * C + c], px[(4 * t + 1) * C + c], px[(4 * t + 2) * C + c], px[(4 * t + 3) * C + c]};
+        } else {
+            for (int i = 4 * t; i < n; ++i) d[i - 4 * t] = px[i * C + c];
+        }
+    }
+}
+
+// Several device arrays into one host area, each at its own place, and then the flag: copy_then_flag_kernel for all
+// outputs of a graph at once.
+struct CopySegments { const float* src[kStagingSegments]; unsigned n[kStagingSegments], at[kStagingSegments]; };
+__global__ void __launch_bounds__(1024) copy_many_then_flag_kernel(float* __restrict__ dst, CopySegments seg, int count, unsigned* flag, unsigned value) {
+    for (int k = 0; k < count; ++k)
+        for (unsigned i = threadIdx.x; i < seg.n[k]; i += blockDim.x)
+            __hip_atomic_store((unsigned*)dst + seg.at[k] + i, __float_as_uint(seg.src[k][i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this lane's stores have been accepted
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Measurement aid: what the shader clock does under a stream of fp32 MFMAs.  Every wave issues `iters` rounds of 8
@@ -286,6 +336,7 @@ struct Staging {
 };
 constexpr size_t kStagingDownBytes = 64 * 1024;    // + 64 bytes behind it for the flag
 constexpr size_t kStagingKernelUpload = 4u << 20;
+constexpr size_t kStagingHalves = 256u << 10;      // uploads by kernel of this size and more go in two pieces
 
 int drhip_staging_create(void** handle, size_t upload_bytes) {
     DRHIP_REQUIRE(handle && upload_bytes > 0, "drhip_staging_create: NULL handle or zero size");
@@ -344,15 +395,12 @@ static void upload_areas_done(Staging* s, hipStream_t stream) {
         if (s->up[a].pending && s->up[a].stream == stream) s->up[a].pending = s->up[a].recorded = false;
 }
 
-int drhip_upload_staged(void* handle, void* dst, size_t off, const void* src, size_t bytes, void* stream) {
-    Staging* s = (Staging*)handle;
-    DRHIP_REQUIRE(s && dst && src, "drhip_upload_staged: NULL pointer");
-    DRHIP_REQUIRE(bytes <= s->cap, "drhip_upload_staged: %zu bytes do not fit the staging area of %zu", bytes, s->cap);
-    if (bytes == 0) return DRHIP_OK;
+// The area the next upload may fill.  (The upload before the last may still be reading it.)
+static int acquire_area(Staging* s, UploadArea** out) {
     UploadArea& area = s->up[s->next];
     UploadArea& other = s->up[s->next ^ 1];
     s->next ^= 1;
-    if (area.pending) {         // the upload before the last may still be reading this area
+    if (area.pending) {
         if (area.recorded) {
             if (int rc = check(hipEventSynchronize(area.done), "hipEventSynchronize(staging)")) return rc;
         } else if (other.pending && other.recorded && other.stream == area.stream) {
@@ -361,32 +409,110 @@ int drhip_upload_staged(void* handle, void* dst, size_t off, const void* src, si
         } else if (int rc = check(hipStreamSynchronize(area.stream), "hipStreamSynchronize(staging)")) return rc;
         area.pending = area.recorded = false;
     }
+    *out = &area;
+    return DRHIP_OK;
+}
+
+// The upload out of `area` has been enqueued.
+static int release_area(Staging* s, UploadArea& area, hipStream_t stream) {
+    area.pending = true;
+    area.recorded = false;
+    area.stream = stream;
+    if (s->up[&area == &s->up[0]].pending) {    // no download has completed since the previous feed: this caller runs ahead of the device
+        if (int rc = check(hipEventRecord(area.done, stream), "hipEventRecord(staging)")) return rc;
+        area.recorded = true;
+    }
+    return DRHIP_OK;
+}
+
+int drhip_upload_staged(void* handle, void* dst, size_t off, const void* src, size_t bytes, void* stream) {
+    Staging* s = (Staging*)handle;
+    DRHIP_REQUIRE(s && dst && src, "drhip_upload_staged: NULL pointer");
+    DRHIP_REQUIRE(bytes <= s->cap, "drhip_upload_staged: %zu bytes do not fit the staging area of %zu", bytes, s->cap);
+    if (bytes == 0) return DRHIP_OK;
+    UploadArea* area = nullptr;
+    if (int rc = acquire_area(s, &area)) return rc;
     // A few hundred KiB: a kernel that reads the pinned area over the bus starts sooner than the DMA engine
     // (602 KB image: 4 us less per pass).  From 256 KiB on in two pieces: the kernel of the first half runs while
     // the host copies the second (2 us less per 602 KB image; with five pieces moved by the DMA engine the calls cost
     // the host more than the overlap returned, 0.414 vs 0.386 ms per VGG16 image).
     if (s->uploadByKernel && bytes <= kStagingKernelUpload && ((size_t)((char*)dst + off) % 16 == 0) && bytes % 4 == 0) {
-        const size_t first = bytes >= (256u << 10) ? (bytes / 2) & ~(size_t)15 : bytes;
+        const size_t first = bytes >= kStagingHalves ? (bytes / 2) & ~(size_t)15 : bytes;
         const size_t begins[2] = {0, first}, lens[2] = {first, bytes - first};
         for (int piece = 0; piece < 2 && lens[piece] > 0; ++piece) {
             const size_t begin = begins[piece], len = lens[piece];
-            memcpy(area.mem + begin, (const char*)src + begin, len);
+            memcpy(area->mem + begin, (const char*)src + begin, len);
             const size_t n = len / 4, n4 = n / 4;
             launch(copy_from_host_kernel, dim3((unsigned)std::max<size_t>(1, std::min<size_t>((n4 + 255) / 256, 512))), dim3(256), 0, as_stream(stream),
-                   (float*)((char*)dst + off + begin), (const float*)(area.mem + begin), n4, n);
+                   (float*)((char*)dst + off + begin), (const float*)(area->mem + begin), n4, n);
             if (int rc = launched("copy_from_host_kernel")) return rc;
         }
     } else {
-        memcpy(area.mem, src, bytes);
-        if (int rc = check(hipMemcpyAsync((char*)dst + off, area.mem, bytes, hipMemcpyHostToDevice, as_stream(stream)), "hipMemcpyAsync(H2D, staged)")) return rc;
+        memcpy(area->mem, src, bytes);
+        if (int rc = check(hipMemcpyAsync((char*)dst + off, area->mem, bytes, hipMemcpyHostToDevice, as_stream(stream)), "hipMemcpyAsync(H2D, staged)")) return rc;
     }
-    area.pending = true;
-    area.recorded = false;
-    area.stream = as_stream(stream);
-    if (other.pending) {        // no download has completed since the previous feed: this caller runs ahead of the device
-        if (int rc = check(hipEventRecord(area.done, as_stream(stream)), "hipEventRecord(staging)")) return rc;
-        area.recorded = true;
+    return release_area(s, *area, as_stream(stream));
+}
+
+int drhip_upload_staged_interleaved(void* handle, float* dst, const float* src, size_t pixels, int channels, void* stream) {
+    Staging* s = (Staging*)handle;
+    DRHIP_REQUIRE(s && dst && src && channels > 0, "drhip_upload_staged_interleaved: NULL pointer or no channels");
+    const size_t C = (size_t)channels, bytes = pixels * C * sizeof(float);
+    DRHIP_REQUIRE(bytes <= s->cap, "drhip_upload_staged_interleaved: %zu bytes do not fit the staging area of %zu", bytes, s->cap);
+    if (channels == 1 || pixels <= 1) return drhip_upload_staged(handle, dst, 0, src, bytes, stream);      // the two layouts are one
+    UploadArea* area = nullptr;
+    if (int rc = acquire_area(s, &area)) return rc;
+    float* const mem = (float*)area->mem;
+    if (channels <= 4 && s->uploadByKernel && bytes <= kStagingKernelUpload) {
+        // An image: the kernel that fetches it from the pinned area brings it into planes on the way; the host only
+        // copies.  In two pieces from 256 KiB on, for the reason given above.
+        const size_t half = (pixels / 2 + kHwcPixels - 1) / kHwcPixels * kHwcPixels;
+        const size_t first = bytes >= kStagingHalves && half < pixels ? half : pixels;
+        const size_t begins[2] = {0, first}, lens[2] = {first, pixels - first};
+        for (int piece = 0; piece < 2 && lens[piece] > 0; ++piece) {
+            const size_t begin = begins[piece], len = lens[piece];
+            memcpy(mem + begin * C, src + begin * C, len * C * sizeof(float));
+            const dim3 grid((unsigned)((len + kHwcPixels - 1) / kHwcPixels));
+            auto go = [&](auto kernel) { launch(kernel, grid, dim3(256), 0, as_stream(stream), dst + begin, (const float*)(mem + begin * C), pixels, len); };
+            if (channels == 2) go(hwc_from_host_kernel<2>);
+            else if (channels == 3) go(hwc_from_host_kernel<3>);
+            else go(hwc_from_host_kernel<4>);
+            if (int rc = launched("hwc_from_host_kernel")) return rc;
+        }
+    } else {
+        // Many channels, or more than a kernel should fetch: the host transposes while it fills the area, 64 pixels
+        // at a time so that the lines it reads are still in its cache when the next channel wants them.
+        for (size_t p0 = 0; p0 < pixels; p0 += 64) {
+            const size_t p1 = std::min(pixels, p0 + 64);
+            for (size_t c = 0; c < C; ++c)
+                for (size_t p = p0; p < p1; ++p) mem[c * pixels + p] = src[p * C + c];
+        }
+        if (int rc = check(hipMemcpyAsync(dst, mem, bytes, hipMemcpyHostToDevice, as_stream(stream)), "hipMemcpyAsync(H2D, staged)")) return rc;
     }
+    return release_area(s, *area, as_stream(stream));
+}
+
+// Value the next flagged download's kernel raises its flag to: never 0, the flag's initial value.
+static unsigned next_flag_value(Staging* s) { return ++s->seq ? s->seq : ++s->seq; }
+static unsigned* flag_of(Staging* s) { return (unsigned*)(s->down + kStagingDownBytes); }
+
+// The host watches the flag the download's kernel raises behind the data: the stream's own completion path
+// (signal, interrupt, wake-up) takes some 20 us longer than the data needs to arrive.
+static int wait_for_flag(Staging* s, unsigned want, hipStream_t stream) {
+    const auto t0 = std::chrono::steady_clock::now();
+    bool seen = false;
+    for (unsigned spins = 0;; ++spins) {
+        if (__atomic_load_n((const unsigned*)flag_of(s), __ATOMIC_ACQUIRE) == want) { seen = true; break; }
+        if ((spins & 255) == 255 && std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0).count() > s->spinUs) break;
+        __builtin_ia32_pause();
+    }
+    if (!seen) {        // a long pass, or a failed one: wait the ordinary way (and learn of any error)
+        if (int rc = check(hipStreamSynchronize(stream), "hipStreamSynchronize(D2H, staged)")) return rc;
+    }
+    // (Flag seen: the stream is not asked for its status here - hipStreamQuery costs 25-30 us, more than the
+    // flag saves.  A launch that failed was reported when it was enqueued; the next waiting call on the
+    // stream reports anything else.)
+    upload_areas_done(s, stream);
     return DRHIP_OK;
 }
 
@@ -400,27 +526,11 @@ int drhip_download_staged(void* handle, void* dst, const void* src, size_t off, 
     if (((size_t)((const char*)src + off) | bytes) % 4 == 0) {
         const size_t n = bytes / 4;
         if (s->spinUs > 0) {
-            // The host watches a flag the kernel raises behind the data: the stream's own completion path
-            // (signal, interrupt, wake-up) takes some 20 us longer than the data needs to arrive.
-            volatile unsigned* flag = (volatile unsigned*)(s->down + kStagingDownBytes);
-            const unsigned want = ++s->seq ? s->seq : ++s->seq;     // never 0, the flag's initial value
+            const unsigned want = next_flag_value(s);
             launch(copy_then_flag_kernel, dim3(1), dim3(1024), 0, as_stream(stream), (float*)s->down, (const float*)((const char*)src + off), n,
-                   (unsigned*)flag, want);
+                   flag_of(s), want);
             if (int rc = launched("copy_then_flag_kernel")) return rc;
-            const auto t0 = std::chrono::steady_clock::now();
-            bool seen = false;
-            for (unsigned spins = 0;; ++spins) {
-                if (__atomic_load_n((const unsigned*)flag, __ATOMIC_ACQUIRE) == want) { seen = true; break; }
-                if ((spins & 255) == 255 && std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0).count() > s->spinUs) break;
-                __builtin_ia32_pause();
-            }
-            if (!seen) {        // a long pass, or a failed one: wait the ordinary way (and learn of any error)
-                if (int rc = check(hipStreamSynchronize(as_stream(stream)), "hipStreamSynchronize(D2H, staged)")) return rc;
-            }
-            // (Flag seen: the stream is not asked for its status here - hipStreamQuery costs 25-30 us, more than the
-            // flag saves.  A launch that failed was reported when it was enqueued; the next waiting call on the
-            // stream reports anything else.)
-            upload_areas_done(s, as_stream(stream));
+            if (int rc = wait_for_flag(s, want, as_stream(stream))) return rc;
             memcpy(dst, s->down, bytes);
             return DRHIP_OK;
         }
@@ -430,6 +540,34 @@ int drhip_download_staged(void* handle, void* dst, const void* src, size_t off, 
     if (int rc = check(hipStreamSynchronize(as_stream(stream)), "hipStreamSynchronize(D2H, staged)")) return rc;
     upload_areas_done(s, as_stream(stream));
     memcpy(dst, s->down, bytes);
+    return DRHIP_OK;
+}
+
+int drhip_download_staged_many(void* handle, int count, float* const* dst, const float* const* src, const size_t* floats, void* stream) {
+    Staging* s = (Staging*)handle;
+    DRHIP_REQUIRE(s && count >= 0 && (count == 0 || (dst && src && floats)), "drhip_download_staged_many: NULL pointer");
+    size_t total = 0;
+    for (int k = 0; k < count; ++k) {
+        DRHIP_REQUIRE(dst[k] && src[k], "drhip_download_staged_many: NULL array %d", k);
+        total += floats[k];
+    }
+    if (count > 1 && count <= kStagingSegments && s->spinUs > 0 && total * sizeof(float) <= kStagingDownBytes) {
+        CopySegments seg = {};
+        size_t at = 0;
+        for (int k = 0; k < count; ++k) { seg.src[k] = src[k]; seg.n[k] = (unsigned)floats[k]; seg.at[k] = (unsigned)at; at += floats[k]; }
+        const unsigned want = next_flag_value(s);
+        launch(copy_many_then_flag_kernel, dim3(1), dim3(1024), 0, as_stream(stream), (float*)s->down, seg, count, flag_of(s), want);
+        if (int rc = launched("copy_many_then_flag_kernel")) return rc;
+        if (int rc = wait_for_flag(s, want, as_stream(stream))) return rc;
+        for (int k = 0; k < count; ++k) memcpy(dst[k], (const float*)s->down + seg.at[k], floats[k] * sizeof(float));
+        return DRHIP_OK;
+    }
+    for (int k = 0; k < count; ++k) {
+        const size_t bytes = floats[k] * sizeof(float);
+        const int rc = bytes <= kStagingDownBytes ? drhip_download_staged(handle, dst[k], src[k], 0, bytes, stream)
+                                                  : drhip_download(dst[k], src[k], 0, bytes, stream);
+        if (rc) return rc;
+    }
     return DRHIP_OK;
 }
 

@@ -246,6 +246,42 @@ void dR_feedData(dR_Graph* net, dR_Node* feednode, gfloat* data, gint offset, gi
     dR_uploadArray(net, (gchar*)"", data, (size_t)offset * sizeof(float), bytes, feednode->outputBuf->buf);
 }
 
+void dR_feedDataHWC(dR_Graph* net, dR_Node* feednode, gfloat* data) {
+    if (!feednode || !feednode->outputBuf || !data) {
+        say("dR_feedDataHWC: feed node has no buffer yet (call dR_prepare first) or no data\n");
+        return;
+    }
+    const size_t pixels = (size_t)feednode->oshape.s0 * feednode->oshape.s1, C = (size_t)feednode->oshape.s2;
+    float* dst = (float*)feednode->outputBuf->buf;
+    if (net->drStaging && pixels * C * sizeof(float) <= drhip_staging_upload_capacity(net->drStaging)) {
+        device_failed(net, drhip_upload_staged_interleaved(net->drStaging, dst, data, pixels, (int)C, stream_of(net)), "dR_feedDataHWC");
+        return;
+    }
+    std::vector<float> planes(pixels * C);
+    for (size_t p = 0; p < pixels; ++p)
+        for (size_t c = 0; c < C; ++c) planes[c * pixels + p] = data[p * C + c];
+    dR_uploadArray(net, (gchar*)"", planes.data(), 0, planes.size() * sizeof(float), feednode->outputBuf->buf);
+}
+
+gint dR_downloadOutputs(dR_Graph* net, gfloat** hosts, gint n) {
+    if (!net->prepared || n < 0 || (n > 0 && !hosts)) {
+        say("dR_downloadOutputs: the graph is not prepared, or no arrays were given\n");
+        return 0;
+    }
+    const float* src[10];
+    size_t floats[10];
+    int k = 0;
+    for (dR_ListElement* e = net->output_layers->first; e && k < n && k < 10; e = e->next, ++k) {
+        dR_Node* node = (dR_Node*)e->element;
+        src[k] = dev_out(node);
+        floats[k] = (size_t)node->oshape.s0 * node->oshape.s1 * node->oshape.s2;
+    }
+    if (net->drStaging) return device_failed(net, drhip_download_staged_many(net->drStaging, k, hosts, src, floats, stream_of(net)), "dR_downloadOutputs") ? 0 : k;
+    for (int i = 0; i < k; ++i)
+        if (device_failed(net, drhip_download(hosts[i], src[i], 0, floats[i] * sizeof(float), stream_of(net)), "dR_downloadOutputs")) return 0;
+    return k;
+}
+
 // One forward pass: walks the schedule and lets every node enqueue its kernels.  Asynchronous
 // unless profiling is enabled (reference src/deepRACIN.c:204-270: clFlush only).  With DR_HIPGRAPH=1
 // in the environment the first plain pass records the node walk into a hipGraph and later passes

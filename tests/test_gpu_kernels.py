@@ -589,6 +589,42 @@ def test_staged_transfers_carry_every_byte(lib, dev, env):
         lib.drhip_staging_destroy(h)
 
 
+@pytest.mark.parametrize("pixels,channels", [(1, 3), (5, 2), (1023, 3), (1025, 4), (50176, 3), (65537, 2), (4097, 1), (700, 7), (9, 64), (400001, 3)])
+@pytest.mark.parametrize("env", [{}, {"DR_UPLOAD_KERNEL": "0"}])
+def test_interleaved_upload_and_joint_download(lib, dev, pixels, channels, env):
+    """[pixels][channels] on the host -> [channels][pixels] on the device: by kernel in one and in two pieces, at the
+    edges of its 1024-pixel blocks, beyond 4 MiB and with many channels (host), each twice; then several arrays back
+    in one trip, and in several where they do not fit the download area."""
+    import os
+    os.environ.update(env)
+    try:
+        h = ctypes.c_void_p()
+        ok(lib, lib.drhip_staging_create(ctypes.byref(h), 4 * pixels * channels))
+    finally:
+        for k in env:
+            os.environ.pop(k, None)
+    vp = ctypes.c_void_p
+    try:
+        rng = np.random.default_rng(pixels)
+        buf = dev.empty(pixels * channels)
+        for _ in range(2):
+            a = rng.standard_normal((pixels, channels)).astype(np.float32)
+            want = a.T.copy()
+            ok(lib, lib.drhip_upload_staged_interleaved(h, buf, a.ctypes.data_as(vp), pixels, channels, None))
+            a[...] = np.nan                                                    # the caller's array is free again
+            lengths = [min(pixels, 9000), 1, min(pixels, 17)] if channels > 1 else [pixels]
+            backs = [np.full(n, -1.0, np.float32) for n in lengths]
+            addr = buf.value if isinstance(buf, vp) else buf
+            srcs = (vp * len(lengths))(*[addr + 4 * k * pixels * (channels > k) for k in range(len(lengths))])
+            dsts = (vp * len(lengths))(*[b.ctypes.data for b in backs])
+            ok(lib, lib.drhip_download_staged_many(h, len(lengths), dsts, srcs, (ctypes.c_size_t * len(lengths))(*lengths), None))
+            for k, b in enumerate(backs):
+                assert np.array_equal(b, want[k * (channels > k)][:lengths[k]]), k
+            assert np.array_equal(dev.get(buf, want.shape), want)
+    finally:
+        lib.drhip_staging_destroy(h)
+
+
 def test_copy3d_and_scalar(lib, dev, oracle):
     x = rnd(6, 9, 11)
     out = dev.empty(3 * 4 * 5)
