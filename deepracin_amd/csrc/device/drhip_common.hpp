@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <vector>
@@ -61,6 +62,21 @@ inline void launch(Kernel kernel, dim3 grid, dim3 block, size_t ldsBytes, hipStr
     }
     hipExtLaunchKernelGGL(kernel, grid, block, ldsBytes, stream, t.events[t.used], t.events[t.used + 1], 0, args...);
     t.used += 2;
+}
+
+// More than 64 KiB of dynamic LDS has to be asked for once per kernel and device (the attribute belongs to the kernel's
+// code object on ONE device); `asked` is the kernel's own memory of that, one bit per device.  Graphs may be prepared
+// and applied from several host threads.
+constexpr int kMaxDynamicLds = 159 * 1024;           // (of 160 KiB: what a kernel declares statically comes on top)
+inline int allow_lds(const void* kernel, size_t bytes, std::atomic<unsigned long long>& asked) {
+    if (bytes <= 65536) return DRHIP_OK;
+    int device = 0;
+    if (int rc = check(hipGetDevice(&device), "hipGetDevice")) return rc;
+    const unsigned long long bit = device >= 0 && device < 64 ? 1ull << device : 0;
+    if (asked.load(std::memory_order_acquire) & bit) return DRHIP_OK;
+    if (int rc = check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxDynamicLds), "hipFuncSetAttribute(max dynamic LDS)")) return rc;
+    asked.fetch_or(bit, std::memory_order_acq_rel);
+    return DRHIP_OK;
 }
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

@@ -1,0 +1,399 @@
+// Convolution with any odd filter and any stride as an implicit GEMM on the bf16 matrix cores, at fp32 accuracy (see
+// bf16x3.hpp): everything that is neither 3x3/stride 1 (Winograd) nor 1x1 (GEMM), such as 7x7/2 first layers and 5x5
+// layers.
+//
+//   out[o][p] = act(b[o] + sum over k-steps of F[k][o] . in[k][pixel p shifted by the step's tap])
+//
+// What bounds it: the matrix cores on large layers (2 * 6 * Ho*Wo * I*O*kh*kw FLOP of bf16 MFMA), one workgroup's chain
+// of staging, matrix steps and store on small ones; figures stand at the choice of the tile.
+//
+// A workgroup owns a tile of 32*MT output pixels and 32*WO output channels:
+//   * The input patch under the tile is staged in LDS once per 16 channels, zero padding included, ALREADY SPLIT into
+//     its three bf16 parts and with the eight channels an MFMA lane wants next to each other: inside the tap loop a
+//     B operand is one 16-byte LDS read whatever the tap (a tap is an address offset), and there is no vector arithmetic at all.
+//     Reading the samples from global memory per tap would cost a dword gather and a split per sample and tap, 25 times
+//     for a 5x5 filter.  The next 16 channels are fetched into registers while the taps run and go to the other half of LDS.
+//   * The filters come from a bank laid out and split once, when the layer is prepared, so that an A operand is one 16-byte
+//     buffer load per lane and 1 KiB in a row per wave.  Every wave reads only its own 32 channels, several steps ahead.
+//   * Two, four or eight waves share the k-steps of one channel block round-robin and meet in LDS at the end, in wave order: layers with
+//     few tiles fill the chip that way without a second kernel.
+// Layers with at most four input channels (images) put four neighbouring pixels x four channels into one step of 16 k
+// (CP = 4) instead of 16 channels of one pixel, most of which would be zero: a 7x7 filter over RGB is 14 steps, not 49.
+#include "bf16x3.hpp"
+
+#include <algorithm>
+
+namespace drhip {
+
+constexpr unsigned kBankBufferFlags = 0x00020000u;      // dword 3 of a gfx9 raw buffer resource (32-bit data format)
+constexpr unsigned kBankOutOfRange = 0x80000000u;       // byte offset no resource of at most 2 GiB contains
+constexpr int kBankThreads = 512;                       // eight waves: two per SIMD, one reads and counts while the other multiplies
+
+struct BankShape {                                      // everything but the pointers; by value to the kernel
+    int W, H, I, O, Wo, Ho;
+    int kw, sx, sy, padX, padY;
+    int lgBW;                                           // 32 pixels of one MFMA = 2^lgBW columns x the rest rows
+    int pw, patchN;                                     // patch width, patch pixels
+    int spr, steps, nChunks, oBlocks;                   // k-steps per filter row, per chunk; chunks; 32-channel blocks in the bank
+    unsigned pwMul, pwShift, sprMul;                    // division by pw; j = step * sprMul >> 16
+    int relu;
+};
+
+__device__ inline u32x4b bank_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, unsigned soffset) {
+    return __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voffset, (int)soffset, 0));
+}
+
+// F[chunk][step][part][o/32][lane][8] (bf16) from w[c][o][kh][kw]: lane l of a wave holds output channel o = l%32 and
+// the values k = 8*(l/32) .. +7 of the step.  CP = 16: k is the channel within the chunk, the step a tap.  CP = 4: k is
+// (pixel within a group of four, channel).  What does not exist is zero.
+__global__ void __launch_bounds__(256)
+conv_bank_layout_kernel(const float* __restrict__ w, unsigned short* __restrict__ F, int I, int O, int kw, int kh, int cp, int spr, int steps, int nChunks, int oBlocks) {
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;          // (chunk, step, oblock, lane, e)
+    const size_t total = (size_t)nChunks * steps * oBlocks * 512;
+    if (idx >= total) return;
+    const int e = (int)(idx & 7), lane = (int)((idx >> 3) & 63);
+    const size_t rest = idx >> 9;
+    const int ob = (int)(rest % oBlocks);
+    const int step = (int)(rest / oBlocks % steps), chunk = (int)(rest / oBlocks / steps);
+    const int k = 8 * (lane >> 5) + e, o = 32 * ob + (lane & 31);
+    const int j = step / spr;
+    const int c = cp == 16 ? 16 * chunk + k : (k & 3), i = cp == 16 ? step % spr : 4 * (step % spr) + (k >> 2);
+    const float v = (c < I && o < O && i < kw) ? w[(((size_t)c * O + o) * kh + j) * kw + i] : 0.0f;
+    unsigned short part[3];
+    split_one(v, part);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) F[((((size_t)chunk * steps + step) * 3 + q) * oBlocks + ob) * 512 + lane * 8 + e] = part[q];
+}
+
+// PF: staging rounds (512 units each) of the next 16 channels that are kept in registers.
+template <int CP, int MT, int WO, int WK, int PF>
+__global__ void __launch_bounds__(kBankThreads)
+conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __restrict__ F, const float* __restrict__ bias,
+                      float* __restrict__ out, BankShape s) {
+    static_assert(WO * WK * 64 == kBankThreads, "eight waves");
+    static_assert(CP == 4 || CP == 16, "channels of one pixel in a k-step");
+    constexpr int kGroups = CP == 16 ? 2 : 1;           // staging units per pixel, 8 (4) channels each
+    constexpr int kUnitBytes = CP == 16 ? 16 : 8;
+    __shared__ float biasT[32 * WO];                    // (a load in the epilogue would wait for the stores in front of it)
+    constexpr int kDepth = 4;                           // k-steps whose filters are in flight (even: two operand buffers alternate)
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wo = wave % WO, wk = wave / WO;
+    const int l32 = lane & 31, half = lane >> 5;
+    const int BW = 1 << s.lgBW, BH = 32 >> s.lgBW;
+    const int x0 = blockIdx.x << s.lgBW, y0 = blockIdx.y * (BH * MT);
+    const int ob = blockIdx.z * WO + wo;                // this wave's 32 output channels
+    const int bx = l32 & (BW - 1), by = l32 >> s.lgBW;
+    const int plane = s.H * s.W;
+
+    // ---- staging: unit u -> (channel group, patch pixel); a unit is 8 (4) channels of one pixel, split ----------------
+    const int units = s.patchN * kGroups;
+    const int rounds = (units + kBankThreads - 1) / kBankThreads;
+    const int partBytes = (s.patchN * kGroups * kUnitBytes + 15) & ~15;
+    const int bufBytes = 3 * partBytes;
+    const FastDiv pwd = {(unsigned)s.pw, s.pwMul, s.pwShift};
+    const int px0 = x0 * s.sx - s.padX, py0 = y0 * s.sy - s.padY;
+    constexpr int kUC = CP == 16 ? 8 : 4;               // channels of a unit
+    auto unit_offset = [&](int u, unsigned& off) {
+        const int grp = (kGroups == 2 && u >= s.patchN) ? 1 : 0, q = u - grp * s.patchN;
+        const int py = fast_div(q, pwd), px = q - py * s.pw;
+        const int ix = px0 + px, iy = py0 + py;
+        const bool ok = u < units && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
+        off = ok ? 4u * (unsigned)(grp * 8 * plane + iy * s.W + ix) : kBankOutOfRange;
+    };
+    auto load_unit = [&](float (&v)[kUC], unsigned off, int chunk) {
+#pragma unroll
+        for (int q = 0; q < kUC; ++q) {                 // (channels past the last one: a resource that ends in front of them)
+            const int c = chunk * 16 + q, left = max(s.I - c, 0);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(in + (size_t)min(c, s.I) * plane), 0, left * plane * 4, kBankBufferFlags);
+            v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
+        }
+    };
+    auto store_unit = [&](char* buf, const float (&v)[kUC], int u) {
+        if (u >= units) return;
+        Bf16Pair3 p[kUC / 2];
+#pragma unroll
+        for (int q = 0; q < kUC / 2; ++q) p[q] = split_pair(v[2 * q], v[2 * q + 1]);
+        char* d = buf + u * kUnitBytes;
+        if constexpr (CP == 16) {
+            *(u32x4b*)d = u32x4b{p[0].hi, p[1].hi, p[2].hi, p[3].hi};
+            *(u32x4b*)(d + partBytes) = u32x4b{p[0].mid, p[1].mid, p[2].mid, p[3].mid};
+            *(u32x4b*)(d + 2 * partBytes) = u32x4b{p[0].lo, p[1].lo, p[2].lo, p[3].lo};
+        } else {
+            *(u32x2b*)d = u32x2b{p[0].hi, p[1].hi};
+            *(u32x2b*)(d + partBytes) = u32x2b{p[0].mid, p[1].mid};
+            *(u32x2b*)(d + 2 * partBytes) = u32x2b{p[0].lo, p[1].lo};
+        }
+    };
+
+    // ---- filters: the steps of this wave, wk, wk + WK, ..., -------------------------------------
+    const int bankBytes = s.nChunks * s.steps * 3 * s.oBlocks * 1024;
+    const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, bankBytes, kBankBufferFlags);
+    const unsigned fLane = ob < s.oBlocks ? (unsigned)(ob * 1024 + lane * 16) : kBankOutOfRange;    // (a wave without channels multiplies zeros)
+    auto load_filters = [&](u32x4b (&f)[3], int chunk, int step) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) f[q] = bank_load4(rF, fLane, (unsigned)(((chunk * s.steps + step) * 3 + q) * s.oBlocks) * 1024u);
+    };
+    const int mySteps = wk < s.steps ? (s.steps - wk + WK - 1) / WK : 0;
+    u32x4b f[kDepth][3];
+#pragma unroll
+    for (int g = 0; g < kDepth; ++g) load_filters(f[g], 0, min(wk + g * WK, s.steps - 1));
+
+    unsigned off[PF];
+    float raw[PF][kUC];
+#pragma unroll
+    for (int r = 0; r < PF; ++r) {
+        unit_offset(tid + kBankThreads * r, off[r]);
+        load_unit(raw[r], off[r], 0);
+    }
+    if (tid < 32 * WO) biasT[tid] = bias ? bias[min((int)blockIdx.z * 32 * WO + tid, s.O - 1)] : 0.0f;
+    // what of the patch does not fit the prefetch registers is loaded when it is stored
+    auto stage = [&](char* buf, int chunk) {
+#pragma unroll
+        for (int r = 0; r < PF; ++r) store_unit(buf, raw[r], tid + kBankThreads * r);
+        for (int r = PF; r < rounds; ++r) {
+            unsigned o;
+            float v[kUC];
+            unit_offset(tid + kBankThreads * r, o);
+            load_unit(v, o, chunk);
+            store_unit(buf, v, tid + kBankThreads * r);
+        }
+    };
+
+    // MT = 1 keeps three accumulators, so that the MFMAs of a step do not wait for each other
+    constexpr int NA = MT == 1 ? 3 : 1;
+    f32x16b acc[MT][NA];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][a][r] = 0.0f;
+
+    // byte offset of this lane's operand for tap (0, 0), per 32-pixel block
+    int bBase[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int q = (by + BH * m) * s.sy * s.pw + bx * s.sx;
+        bBase[m] = CP == 16 ? (half * s.patchN + q) * 16 : q * 8 + half * 16;
+    }
+
+    stage(lds, 0);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+
+    auto read_operands = [&](const char* buf, u32x4b (&b)[MT][3], int step) {
+        const int j = (int)(((unsigned)step * s.sprMul) >> 16), i = step - j * s.spr;
+        const char* at = buf + (CP == 16 ? (j * s.pw + i) * 16 : (j * s.pw + 4 * i) * 8);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const char* p = at + q * partBytes + bBase[m];
+                if constexpr (CP == 16) b[m][q] = *(const u32x4b*)p;
+                else {
+                    const u32x2b lo = *(const u32x2b*)p, hi = *(const u32x2b*)(p + 8);
+                    b[m][q] = u32x4b{lo[0], lo[1], hi[0], hi[1]};
+                }
+            }
+    };
+    auto multiply = [&](const u32x4b (&fs)[3], const u32x4b (&b)[MT][3]) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m][q % NA] = mfma_bf16(fs[kProdA[q]], b[m][kProdB[q]], acc[m][q % NA]);
+    };
+
+    for (int chunk = 0; chunk < s.nChunks; ++chunk) {
+        const char* buf = lds + (chunk & 1) * bufBytes;
+        const bool more = chunk + 1 < s.nChunks;
+        if (more) {
+#pragma unroll
+            for (int r = 0; r < PF; ++r) load_unit(raw[r], off[r], chunk + 1);
+        }
+        // A step's operands are read from LDS while the step in front of it multiplies (a wave is often alone on its SIMD, and
+        // a trip to LDS is as long as six MFMAs); its filters were requested kDepth steps ago.  The loads of a group go
+        // out whether or not the steps exist, so that the number of loads in flight is known where it is waited for.
+        u32x4b b[2][MT][3];
+        read_operands(buf, b[0], wk);
+        for (int n = 0; n < mySteps; n += kDepth) {
+#pragma unroll
+            for (int g = 0; g < kDepth; ++g) {
+                const int t = n + g;
+                if (t < mySteps) {
+                    read_operands(buf, b[(g + 1) & 1], wk + min(t + 1, mySteps - 1) * WK);
+                    multiply(f[g], b[g & 1]);
+                }
+                // the step that takes this slot next: kDepth on, or the slot's first one in the next 16 channels
+                const bool here = t + kDepth < mySteps;
+                load_filters(f[g], here ? chunk : min(chunk + 1, s.nChunks - 1), min(wk + (here ? t + kDepth : g) * WK, s.steps - 1));
+            }
+        }
+        if (more) {
+            stage(lds + ((chunk + 1) & 1) * bufBytes, chunk + 1);       // (read last before the barrier in front of this chunk)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+    }
+
+    // D of the 32x32 MFMA: lane -> pixel lane%32; register r -> channel 8*(r/4) + 4*(lane/32) + r%4
+    const int P = s.Wo * s.Ho;
+    if constexpr (NA > 1) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][0][r] = (acc[m][0][r] + acc[m][1][r]) + acc[m][2][r];
+    }
+    constexpr int kPitch = 33;
+    float* part = (float*)lds;                          // [WK][32*WO channels][MT][33]
+    __syncthreads();                                    // the patch has been read for the last time
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            part[((wk * 32 * WO + 32 * wo + 8 * (r / 4) + 4 * half + r % 4) * MT + m) * kPitch + l32] = acc[m][0][r];
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 2 * WO * MT; ++n) {             // 512 lanes: 16 (channel, block) pairs of 32 pixels a turn
+        const int pair = 16 * n + (tid >> 5), m = pair % MT, oc = pair / MT, pl = tid & 31;
+        float v = 0.0f;
+#pragma unroll
+        for (int k = 0; k < WK; ++k) v += part[((k * 32 * WO + oc) * MT + m) * kPitch + pl];
+        const int o = blockIdx.z * (32 * WO) + oc;
+        const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
+        v += biasT[oc];
+        if (s.relu) v = fmaxf(v, 0.0f);
+        if (o < s.O && x < s.Wo && y < s.Ho) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
+    }
+}
+
+struct BankPlan { int cp, mt, wo, wk, pf; BankShape s; size_t lds; };
+
+static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int mt, int wo, int wk, int lgBW, BankPlan* p) {
+    p->cp = I <= 4 ? 4 : 16;
+    p->mt = mt; p->wo = wo; p->wk = wk;
+    BankShape& s = p->s;
+    s.W = W; s.H = H; s.I = I; s.O = O; s.Wo = W / sx; s.Ho = H / sy;
+    s.kw = kw; s.sx = sx; s.sy = sy; s.padX = kw / 2; s.padY = kh / 2;
+    s.lgBW = lgBW;
+    const int BW = 1 << lgBW, BH = (32 >> lgBW) * mt;
+    s.spr = p->cp == 16 ? kw : ceil_div(kw, 4);
+    s.steps = s.spr * kh;
+    s.pw = (BW - 1) * sx + (p->cp == 16 ? kw : 4 * s.spr);
+    s.patchN = s.pw * ((BH - 1) * sy + kh);
+    s.nChunks = p->cp == 16 ? ceil_div(I, 16) : 1;
+    s.oBlocks = ceil_div(O, 32);
+    const FastDiv d = make_fastdiv(s.pw);
+    s.pwMul = d.mul; s.pwShift = d.shift;
+    s.sprMul = (unsigned)(65536 / s.spr + 1);
+    const size_t partBytes = ((size_t)s.patchN * (p->cp == 16 ? 32 : 8) + 15) & ~(size_t)15;
+    p->pf = s.patchN * (p->cp == 16 ? 2 : 1) <= kBankThreads ? 1 : 2;
+    p->lds = 3 * partBytes * (s.nChunks > 1 ? 2 : 1);
+    p->lds = std::max(p->lds, (size_t)wk * 32 * wo * mt * 33 * sizeof(float));
+    return p->lds <= kMaxDynamicLds && s.steps * s.spr < 65536;      // (the kernel's division of a step number by spr)
+}
+
+// The tile that finishes first, by a count of what the busiest CU does, in clocks: per workgroup a fixed 2000 for the first
+// loads and the store, 1200 per round of staging 16 channels (the address unit takes one dword gather every 8 to 16
+// clocks), and the MFMAs of one of its four SIMDs at 33 clocks plus what is lost around them.  Pixel tiles wider than the
+// map or hanging over its edge count in full, which picks the tile shape as well.  Measured, us per launch, this choice / the
+// other tiles: 56x56 64->96 5x5 10.9 / 11.5 to 24.7, 224x224 3->64 7x7/2 5.8 / 7.1 to 12.7, 56x56 256->256 3x3 29.7 / 33 to 78,
+// 96x70 50->75 5x5 17.4 / 17.2 to 24.8, 112x112 64->128 3x3/2 8.5 / 8.6 to 15, 14x14 16->32 5x5 4.3 / 4.8 to 8.2.  The kernel
+// that staged the same patch for vector FMAs took 123 us on the first and 31.4 us on the last.
+static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, BankPlan* best) {
+    double bestCost = 0;
+    bool found = false;
+    for (int wsel = 0; wsel < 3; ++wsel)
+        for (int lgM = 0; lgM < 2; ++lgM) {
+            const int wo = 4 >> wsel, wk = 2 << wsel, mt = 1 << lgM;
+            if (variant && variant != (0x100 | wsel << 4 | lgM)) continue;
+            for (int lgBW = 3; lgBW <= 5; ++lgBW) {
+                BankPlan p;
+                if (!bank_shape(W, H, I, O, kw, kh, sx, sy, mt, wo, wk, lgBW, &p)) continue;
+                const BankShape& s = p.s;
+                const double wgs = (double)ceil_div(s.Wo, 1 << lgBW) * ceil_div(s.Ho, (32 >> lgBW) * mt) * ceil_div(s.oBlocks, wo);
+                const double mfma = (double)s.nChunks * s.steps * 6 * 33 * wo * mt / 4 * (mt == 1 ? 1.25 : 1.1);
+                const double cost = 2000 + std::ceil(wgs / num_cu()) * (2000 + (double)s.nChunks * p.pf * 1200 + mfma);
+                if (!found || cost < bestCost) { found = true; bestCost = cost; *best = p; }
+            }
+        }
+    return found;
+}
+
+template <int CP, int MT, int WO, int WK, int PF>
+static int launch_bank_pf(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
+    const BankShape& s = p.s;
+    const dim3 grid(ceil_div(s.Wo, 1 << s.lgBW), ceil_div(s.Ho, (32 >> s.lgBW) * MT), ceil_div(s.oBlocks, WO));
+    static std::atomic<unsigned long long> asked{0};
+    if (int rc = allow_lds((const void*)conv_bank_mfma_kernel<CP, MT, WO, WK, PF>, p.lds, asked)) return rc;
+    launch((conv_bank_mfma_kernel<CP, MT, WO, WK, PF>), grid, dim3(kBankThreads), p.lds, st, in, F, bias, out, s);
+    return launched("conv_bank_mfma_kernel");
+}
+
+template <int CP, int MT, int WO, int WK>
+static int launch_bank(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
+    return p.pf == 1 ? launch_bank_pf<CP, MT, WO, WK, 1>(in, F, bias, out, p, st) : launch_bank_pf<CP, MT, WO, WK, 2>(in, F, bias, out, p, st);
+}
+
+template <int CP, int MT>
+static int launch_bank_w(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
+    if (p.wk == 2) return launch_bank<CP, MT, 4, 2>(in, F, bias, out, p, st);
+    if (p.wk == 4) return launch_bank<CP, MT, 2, 4>(in, F, bias, out, p, st);
+    return launch_bank<CP, MT, 1, 8>(in, F, bias, out, p, st);
+}
+
+template <int CP>
+static int launch_bank_m(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
+    if (p.mt == 1) return launch_bank_w<CP, 1>(in, F, bias, out, p, st);
+    return launch_bank_w<CP, 2>(in, F, bias, out, p, st);
+}
+
+}  // namespace drhip
+
+using namespace drhip;
+
+static size_t bank_blocks(int I, int O, int kw, int kh) {      // KiB of the bank per part
+    const size_t steps = (size_t)kh * (I <= 4 ? ceil_div(kw, 4) : kw), chunks = I <= 4 ? 1 : ceil_div(I, 16);
+    return steps * chunks * ceil_div(O, 32);
+}
+
+extern "C" size_t drhip_conv_bank_floats(int I, int O, int kw, int kh) {
+    if (I <= 0 || O <= 0 || kw <= 0 || kh <= 0) return 0;
+    return bank_blocks(I, O, kw, kh) * 3 * 256;
+}
+
+extern "C" int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
+    if (W <= 0 || H <= 0 || I <= 0 || O <= 0 || kw <= 0 || kh <= 0 || !(kw & 1) || !(kh & 1) || strideX <= 0 || strideY <= 0) return 0;
+    if (W / strideX <= 0 || H / strideY <= 0) return 0;
+    // byte offsets into the input and the bank are 32-bit, and 0x80000000 must lie outside both
+    if ((long long)W * H * (I + 15) >= (1ll << 29) || (long long)(W / strideX) * (H / strideY) * O >= (1ll << 31)) return 0;
+    if (bank_blocks(I, O, kw, kh) * 3 * 1024 >= (1ull << 31)) return 0;
+    if (H / strideY > 65535 || ceil_div(O, 32) > 65535) return 0;
+    BankPlan p;
+    return bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, &p) ? 1 : 0;
+}
+
+extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O, int kw, int kh, void* stream) {
+    DRHIP_REQUIRE(w && F, "drhip_conv_bank_layout_f32: NULL tensor");
+    DRHIP_REQUIRE(I > 0 && O > 0 && kw > 0 && kh > 0 && bank_blocks(I, O, kw, kh) * 3 * 1024 < (1ull << 31), "drhip_conv_bank_layout_f32: bad shape I=%d O=%d %dx%d", I, O, kw, kh);
+    const int cp = I <= 4 ? 4 : 16, spr = cp == 4 ? ceil_div(kw, 4) : kw, chunks = cp == 4 ? 1 : ceil_div(I, 16);
+    launch(conv_bank_layout_kernel, dim3((unsigned)(bank_blocks(I, O, kw, kh) * 2)), dim3(256), 0, as_stream(stream), w, (unsigned short*)F, I, O, kw, kh, cp, spr,
+           spr * kh, chunks, ceil_div(O, 32));
+    return launched("conv_bank_layout_kernel");
+}
+
+extern "C" int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                                   int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
+    DRHIP_REQUIRE(in && F && out, "drhip_conv_bank_f32: NULL tensor");
+    DRHIP_REQUIRE(drhip_conv_bank_usable(W, H, I, O, kw, kh, strideX, strideY), "drhip_conv_bank_f32: shape %dx%dx%d -> %d, %dx%d/%dx%d not covered", W, H, I, O, kw, kh, strideX, strideY);
+    DRHIP_REQUIRE(((size_t)F & 15) == 0, "drhip_conv_bank_f32: the filter bank must be 16-byte aligned");
+    BankPlan p;
+    DRHIP_REQUIRE(bank_plan(W, H, I, O, kw, kh, strideX, strideY, variant, &p), "drhip_conv_bank_f32: variant %#x does not fit this shape", variant);
+    p.s.relu = relu ? 1 : 0;
+    if (p.cp == 4) return launch_bank_m<4>(in, (const unsigned short*)F, bias, out, p, as_stream(stream));
+    return launch_bank_m<16>(in, (const unsigned short*)F, bias, out, p, as_stream(stream));
+}

@@ -155,6 +155,19 @@ int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O);
 int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* bias, float* out,
                                   int W, int H, int I, int O, int stride, int relu, int variant, void* stream);
 
+/* The same convolution for any odd filter and any stride on the bf16 matrix cores at fp32 accuracy: operands are split
+ * into three bf16 parts each, which together hold all 24 significant bits, and six partial products are accumulated
+ * in fp32.  F is the filter bank in the layout the kernel streams, produced once at prepare time from
+ * w [I][O][kh][kw]; drhip_conv_bank_floats(I,O,kw,kh) floats, 16-byte aligned.  drhip_conv_bank_usable: whether the
+ * shape is covered (the patch of a tile fits LDS, 32-bit byte offsets).  `variant` 0 lets the launcher pick; otherwise
+ * 0x100 | log2(32-pixel blocks per workgroup, 0..1) | n << 4 for 2 << n waves sharing a channel block (n = 0..2).
+ * Replaces the per-layer generated kernel of filters other than 3x3 (src/dR_nodes_conv2d.c:364-420, 481-773). */
+int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY);
+size_t drhip_conv_bank_floats(int I, int O, int kw, int kh);
+int drhip_conv_bank_layout_f32(const float* w /* [I][O][kh][kw] */, float* F, int I, int O, int kw, int kh, void* stream);
+int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                        int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
+
 /* First layer (1 to 4 input channels, 3x3, any stride, zero padding, bias, optional ReLU) followed by
  * a 3x3 / stride-2 max pooling with the reference's pooling rules (out = ceil(in/2), samples outside
  * the map read 0.0): out[O][ceil(Ho/2)][ceil(Wo/2)], Wo = W/strideX, Ho = H/strideY.  The

@@ -84,6 +84,30 @@ def test_conv3x3_direct_mfma(lib, dev, oracle, variant, W, H, I, O, s):
         assert lib.drhip_conv3x3_direct_mfma_f32(xd, F, None, out, W, H, I, O, s, 0, 3, None) == -1      # 3 waves
 
 
+@pytest.mark.parametrize("variant", [0, 0x100, 0x101, 0x110, 0x111, 0x120, 0x121])
+@pytest.mark.parametrize("W,H,I,O,kw,kh,sx,sy", [
+    (56, 56, 64, 96, 5, 5, 1, 1), (224, 224, 3, 64, 7, 7, 2, 2), (28, 28, 1, 16, 5, 5, 1, 1), (14, 14, 16, 32, 5, 5, 1, 1),
+    (33, 9, 17, 33, 3, 3, 2, 2), (7, 5, 5, 3, 7, 3, 1, 1), (1, 1, 1, 1, 1, 1, 1, 1), (19, 21, 48, 70, 1, 5, 3, 2), (40, 17, 4, 129, 3, 5, 2, 1),
+    (9, 70, 40, 24, 1, 1, 2, 2)])
+def test_conv_split_bank(lib, dev, oracle, variant, W, H, I, O, kw, kh, sx, sy):
+    """Any filter and stride on the bf16 matrix cores, operands split into three parts: every tile and wave split, maps
+    smaller than a tile, ragged channel counts on both sides, and the image form (at most 4 input channels).  Held to a
+    twentieth of the layer bar: the parts carry all 24 bits."""
+    if variant and not lib.drhip_conv_bank_usable(W, H, I, O, kw, kh, sx, sy):
+        pytest.skip("not covered")
+    x, w, b = rnd(I, H, W), rnd(I, O, kh, kw, scale=(2.0 / (I * kw * kh)) ** 0.5), rnd(O, scale=0.1)
+    F = dev.empty(lib.drhip_conv_bank_floats(I, O, kw, kh))
+    ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, kw, kh, None))
+    Wo, Ho = W // sx, H // sy
+    for relu, bias in ((1, b), (0, None)):
+        y = dev.empty(O * Ho * Wo)
+        ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, dev.put(bias) if bias is not None else None, y, W, H, I, O, kw, kh, sx, sy, relu, variant, None))
+        want = oracle.conv_direct(x, w, bias, stride=(sx, sy), relu=bool(relu))
+        got = dev.get(y, want.shape)
+        assert_close(got, want, "split bank")
+        assert rel_err(got, want) <= TOL / 20
+
+
 @pytest.mark.parametrize("W,H,I,O,sx,sy", [(224, 224, 3, 64, 2, 2), (33, 31, 3, 9, 2, 2), (17, 13, 1, 5, 1, 1), (20, 18, 4, 70, 1, 2),
                                             (8, 5, 2, 16, 3, 1), (2, 2, 3, 2, 1, 1), (9, 9, 4, 33, 2, 2), (64, 48, 3, 32, 1, 1)])
 @pytest.mark.parametrize("relu", [1, 0])
