@@ -24,7 +24,7 @@
 // atomics, no device-scope fences) - by a small second kernel, or, when all workgroups of the launch
 // are resident at once, by the splits themselves: every split finishes a slice of its panel and
 // waits for the other splits' partial tiles by watching the workspace slots themselves.
-#include "drhip_common.hpp"
+#include "wino_common.hpp"
 
 #include <atomic>
 #include <cstdlib>
@@ -34,13 +34,9 @@
 namespace drhip {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWinoThreads = 256;       // 4 waves, one per row of the 4x4 transform
 constexpr int kWinoKC = 8;          // input channels per stage (4 MFMA k-steps)
-constexpr int kXcds = 8;            // L2 domains of MI355X
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Layout of the transformed filters:  U[xi][chunk][o][8], chunk = c / 8, and inside a chunk the
 // channel c%8 sits at position (c & 1) * 4 + ((c % 8) >> 1).  The MFMA A operand of k-step ks needs
@@ -62,57 +58,13 @@ winograd_filter_transform_kernel(const float* __restrict__ w, float* __restrict_
     const int c = idx / Opad, o = idx % Opad;
     float u[16];
     if (c < I && o < O) {
-        const float* g = w + ((size_t)c * O + o) * 9;
-        float t[4][3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const float g0 = g[j], g1 = g[3 + j], g2 = g[6 + j];
-            t[0][j] = g0;
-            t[1][j] = 0.5f * g0 + 0.5f * g1 + 0.5f * g2;
-            t[2][j] = 0.5f * g0 - 0.5f * g1 + 0.5f * g2;
-            t[3][j] = g2;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float a = t[r][0], b = t[r][1], cc = t[r][2];
-            u[4 * r + 0] = a;
-            u[4 * r + 1] = 0.5f * a + 0.5f * b + 0.5f * cc;
-            u[4 * r + 2] = 0.5f * a - 0.5f * b + 0.5f * cc;
-            u[4 * r + 3] = cc;
-        }
+        wino_filter_transform(w + ((size_t)c * O + o) * 9, u);
     } else {
 #pragma unroll
         for (int k = 0; k < 16; ++k) u[k] = 0.0f;
     }
 #pragma unroll
     for (int k = 0; k < 16; ++k) U[wino_u_index(k, c, o, nChunks, Opad)] = u[k];
-}
-
-// Output stores are written through (system-scope store: sc0 sc1) instead of being left dirty in this XCD's L2:
-// the consumer is the next kernel, whose workgroups mostly sit on other XCDs and read from memory anyway, and
-// what is written during the kernel need not be written back when it ends (224x224x64: 23.5 vs 25.0 us).
-__device__ inline void store1_through(float* p, float a) {
-    __hip_atomic_store((unsigned*)p, __float_as_uint(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-__device__ inline void store2_through(float* p, float a, float b) {
-    const f32x2 v = {a, b};
-    __hip_atomic_store((unsigned long long*)p, __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// 2x2 store with edge guards; vec2: W even and the base 8-byte aligned.
-__device__ inline void wino_store_tile(float* po, int W, int H, int ox, int oy, int vec2,
-                                       float y00, float y01, float y10, float y11) {
-    if (vec2) {
-        store2_through(po, y00, y01);
-        if (oy + 1 < H) store2_through(po + W, y10, y11);
-    } else {
-        po[0] = y00;
-        if (ox + 1 < W) po[1] = y01;
-        if (oy + 1 < H) {
-            po[W] = y10;
-            if (ox + 1 < W) po[W + 1] = y11;
-        }
-    }
 }
 
 // One wavefront per row of the 4x4 transform.
@@ -169,10 +121,6 @@ __device__ inline void wino_store_tile(float* po, int W, int H, int ox, int oy, 
     const bool joined = (cfg0 >> 31) != 0u, tiered = ((cfg0 >> 30) & 1u) != 0u;                          \
     const int chunksPerSplit = (int)(cfg1 & 0xffffu), lgSplits = (int)((cfg1 >> 24) & 15u);
 struct WinoPackedArgs { unsigned wh, io, mulX, mulTB, cfg0, cfg1; };
-
-constexpr unsigned kBufferFlags = 0x00020000u;      // dword 3 of a gfx9 raw buffer resource (32-bit data format)
-constexpr int kEpiRelu = DRHIP_EPILOGUE_RELU, kEpiMaxPool2 = DRHIP_EPILOGUE_MAXPOOL2;   // bits of the `relu` argument
-constexpr unsigned kOutOfRange = 0x80000000u;       // byte offset no resource of at most 2 GiB contains
 
 // Joined splits (see the kernel's epilogue).
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));

@@ -1,0 +1,378 @@
+// Winograd F(2x2,3x3) on the bf16 matrix cores, at fp32 accuracy: the large layers of k_winograd.hip, with the same
+// transforms, the same grouping into 16 products of filters and tiles and the same fusions, each product as six partial
+// products of bf16 parts (bf16x3.hpp).  That is 2.67 times the matrix rate of fp32, and vector instructions run beside a
+// bf16 MFMA where they exclude an fp32 one.
+//
+// What bounds it: the address unit of a CU.  Operands come as 16-byte loads per lane, 1 KiB each and 20 to 26 clocks; two
+// workgroups on a CU need 192 of them for filters and 40 for samples per 16 channels, about 5100 clocks beside 3200 of
+// MFMAs, 2700 of vector instructions and 2000 of LDS reads, and take 6300.  (A filter fragment serves two MFMAs here.  With two
+// blocks of tiles per wave it would serve four, but then the transform and the split of the samples, which every wave does
+// for its own row of the transform, take as long as the loads; splitting the positions of a row over two waves balances all
+// four units on paper and measured 5750 to 6300 with nothing left to overlap the first loads and the stores with.)
+// Measured per layer, normally distributed data, us, fp32 kernel / this one: 448x448 64->64 78 / 61, 224x224 64->64 22.8 / 18.6,
+// 224x224 128->128 75 / 57, 320x240 128->128 90 / 72, 160x120 256->256 107 / 84, 112x112 128->128 21.1 / 17.7,
+// 80x60 512->512 105 / 84, 56x56 512->512 73 / 52.
+//
+// A workgroup owns 32 consecutive tiles and 64 output channels; each of four waves owns one row of the 4x4 transform, 16
+// input channels per step:
+//   * The samples under the tiles go from global memory straight to LDS (buffer load with the LDS destination), two steps
+//     ahead, raw and row by row: no registers, no instructions, any alignment, and what lies outside the map or beyond the
+//     last channel arrives as zeros.
+//   * A lane reads the two window rows of its tile that its row of the transform combines, transforms and splits them;
+//     that work is cut into ticks and dealt out between the MFMAs of the position in front of it (without that the
+//     compiler gathers it in front of the MFMAs, and the matrix cores wait).
+//   * Filters are transformed and split once, when the layer is prepared, and come as 1 KiB fragments a step or half a step ahead.
+// With KW = 2 two such sets of four waves share the tiles and take alternate steps; their sums meet in LDS.  That is for
+// launches that leave at most one workgroup per CU, where a single set is alone on its SIMDs and waits for its own loads.
+#include "bf16x3.hpp"
+#include "wino_common.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+
+namespace drhip {
+
+constexpr int kWsKC = 16;               // input channels per step
+constexpr int kWsChunks = 20;           // 16-byte pieces of a window row of one channel in LDS
+constexpr int kWsSegments = (4 * kWsChunks - 72) / 4 + 1;               // rows of tiles whose samples fit: 2*31 + 3 floats, 4 more per row, 4 in front
+
+struct WsShape {                            // everything but the pointers; by value to the kernel
+    int W, H, I, O, tilesX, T, nTB, nBlocks, nC, nOB;   // tiles, panels of 32 tiles, workgroups; 16-channel chunks, 32-channel blocks of filters
+    unsigned mulX, shX, mulTB, shTB;                    // division by tilesX and by nTB
+    int flags, vec2, steps;                             // steps of a wave set
+};
+
+// U[row][chunk][o/32][position in the row][part][lane][8] (bf16): lane l of a wave holds output channel o = l%32 and input
+// channels 8*(l/32) .. +7 of the chunk's 16.  What does not exist is zero.
+__global__ void __launch_bounds__(256)
+wino_split_filter_kernel(const float* __restrict__ w, unsigned short* __restrict__ U, int I, int O, int nC, int nOB) {
+    const int row = threadIdx.x >> 6, lane = threadIdx.x & 63, ob = blockIdx.x % nOB, chunk = blockIdx.x / nOB;
+    const int c0 = chunk * 16 + 8 * (lane >> 5), o = ob * 32 + (lane & 31);
+    float u[8][4];                                  // the row's four positions of eight channels
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float all[16] = {};
+        if (c0 + e < I && o < O) wino_filter_transform(w + ((size_t)(c0 + e) * O + o) * 9, all);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) u[e][x] = row == 0 ? all[x] : row == 1 ? all[4 + x] : row == 2 ? all[8 + x] : all[12 + x];
+    }
+    u32x4b* d = (u32x4b*)U + ((size_t)(row * nC + chunk) * nOB + ob) * 12 * 64 + lane;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        u32x4b part[3];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const Bf16Pair3 s = split_pair(u[2 * p][x], u[2 * p + 1][x]);
+            part[0][p] = s.hi;
+            part[1][p] = s.mid;
+            part[2][p] = s.lo;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) d[(x * 3 + q) * 64] = part[q];
+    }
+}
+
+template <int KW>
+__global__ void __launch_bounds__(256 * KW, 2)
+winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __restrict__ U, const float* __restrict__ bias,
+                          float* __restrict__ out, WsShape s) {
+    constexpr int NT = 2, OB = 32 * NT;
+    constexpr int CHB = kWsChunks * 16, ROWB = kWsKC * CHB, BUFB = 4 * ROWB;    // bytes of a window row of one channel, of 16, of a step's samples
+    constexpr int NDMA = ROWB / 1024;               // loads of a wave for them: one window row each
+    constexpr int kPA[6] = {0, 0, 0, 1, 1, 2}, kPB[6] = {2, 1, 0, 1, 0, 0}; // partial products: part of the filter, part of the sample
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ float biasT[OB];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, set = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int l32 = lane & 31, half = lane >> 5;
+    const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX}, nTBd = {(unsigned)s.nTB, s.mulTB, s.shTB};
+
+    const int perXcd = (s.nBlocks + kXcds - 1) / kXcds;
+    const int slot = (int)(blockIdx.x >> 3), logical = (int)(blockIdx.x & 7) * perXcd + slot;     // (an XCD works on neighbouring panels)
+    if (slot >= perXcd || logical >= s.nBlocks) return;
+    const int oBlock = fast_div(logical, nTBd);
+    const int o0 = oBlock * OB, t0 = (logical - oBlock * s.nTB) * 32;
+    const int W = s.W, H = s.H, I = s.I, plane = W * H;
+
+    // ---- samples: global memory -> LDS -------------------------------------------------------------------------------
+    // A segment is the part of the panel's 32 tiles that lies in one row of tiles; its samples lie in a row in LDS, from a
+    // multiple of 16 bytes on: from column 2*tx-1 of its first tile, or from column 0 where that is left of the map (the sample
+    // in front of it is then whatever lies in front of it: it is multiplied by zero).
+    const int ty0 = fast_div(t0, tilesXd), off0 = t0 - ty0 * s.tilesX;
+    auto segment_at = [&](int k) { return k == 0 ? 4 : (2 * (k * s.tilesX - off0) + 4 * k + 6) & ~3; };     // in floats
+    unsigned voff[NDMA];
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+        const int idx = i * 64 + lane, ch = idx / kWsChunks, f = 4 * (idx % kWsChunks);
+        int k = 0;
+#pragma unroll
+        for (int q = 1; q < kWsSegments; ++q) k += f >= segment_at(q) ? 1 : 0;
+        const int x = (k == 0 && off0 > 0 ? 2 * off0 - 1 : 0) + f - segment_at(k), iy = 2 * (ty0 + k) - 1 + wave;
+        const bool ok = f >= 4 && x < W && iy >= 0 && iy < H;
+        voff[i] = ok ? 4u * (unsigned)((16 * set + ch) * plane + iy * W + x) : kOutOfRange;
+    }
+    const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, I * plane * 4, kBufferFlags);
+    const unsigned stepB = 64u * KW * (unsigned)plane;
+    const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(set * 3 * BUFB);
+    // 16 bytes per lane, lane by lane, to LDS at M0.  The compiler does not count these loads: where it waits for a filter
+    // it waits for a few more loads than it means to, and for the samples this kernel waits itself.
+    auto fetch_sample = [&](int buf, int i) {
+        const unsigned at = ldsBase + (unsigned)(buf * BUFB + wave * ROWB);
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff[i]), "s"(rIn), "s"(at + 1024u * i) : "memory");
+        voff[i] += stepB;
+    };
+
+    // ---- filters ---------------------------------------------------------------------------------------------------
+    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)U, 0, 16 * s.nC * 3 * s.nOB * 1024, kBufferFlags);
+    unsigned uOb[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) uOb[nt] = (unsigned)((wave * s.nC * s.nOB + min(oBlock * NT + nt, s.nOB - 1)) * 12288);
+    const unsigned uStep = (unsigned)s.nOB * 12288u;
+    // the first part of two positions and the others of one: no more registers are left
+    u32x4b f0[2][NT], f12[NT][2];
+    auto filter = [&](int e, int nt, int q) -> u32x4b& { return q == 0 ? f0[e & 1][nt] : f12[nt][q - 1]; };
+    auto load_filter = [&](int e, int nt, int q, int step) {
+        filter(e, nt, q) = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(rU, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 3072)), 0));
+    };
+
+    // ---- operands --------------------------------------------------------------------------------------------------
+    const int rowA = wave, rowB = wave < 2 ? 2 : 1;
+    const float sgn = wave == 1 ? 1.0f : -1.0f;
+    const int lr = fast_div(l32 + off0, tilesXd), tx = l32 + off0 - lr * s.tilesX;
+    const int firstTx = lr == 0 ? off0 : 0;
+    const int rLds = half * 8 * CHB + 4 * (segment_at(lr) + 2 * (tx - firstTx) - (firstTx == 0 ? 1 : 0));
+    const float k0f = tx > 0 ? 1.0f : 0.0f, k3f = 2 * tx + 2 < W ? 1.0f : 0.0f;
+    const bool c2ok = 2 * tx + 1 < W;
+    float mm[8][4];                                 // combined window rows of this lane's tile, 8 channels
+    float ra[4], rb[4];                             // a channel's rows on their way from LDS
+    const char* samples = lds + set * 3 * BUFB;
+    auto read_rows = [&](int buf, int j) {
+        const float* a = (const float*)(samples + buf * BUFB + rowA * ROWB + rLds + j * CHB);
+        const float* b = (const float*)(samples + buf * BUFB + rowB * ROWB + rLds + j * CHB);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { ra[c] = a[c]; rb[c] = b[c]; }
+    };
+    auto combine = [&](int j) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mm[j][c] = fmaf(sgn, rb[c], ra[c]);
+        mm[j][2] = c2ok ? mm[j][2] : 0.0f;
+    };
+    u32x4b B[2][3];                                 // [position parity][part]
+    float va[2], vb[2], xa[2], xb[2];               // the two items being split
+    auto vvalue = [&](int e, int c) {
+        return e == 0 ? fmaf(k0f, mm[c][0], -mm[c][2]) : e == 1 ? mm[c][1] + mm[c][2] : e == 2 ? mm[c][2] - mm[c][1] : fmaf(k3f, mm[c][3], -mm[c][1]);
+    };
+    auto pack = [&](float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2b{a, b}, bf16x2)); };
+    // The operands of position e out of mm: 12 ticks for two items (an item is two channels), whose instructions
+    // alternate: a vector instruction that needs the result of the one in front of it waits for it.
+    auto split_tick = [&](int e, int tick) {
+        const int u = tick / 12, k = tick % 12;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int p = 2 * u + x;
+            u32x4b(&d)[3] = B[e & 1];
+            if (k == 0) va[x] = vvalue(e, 2 * p);
+            if (k == 1) vb[x] = vvalue(e, 2 * p + 1);
+            if (k == 2 || k == 7 || k == 11) d[k == 2 ? 0 : k == 7 ? 1 : 2][p] = pack(va[x], vb[x]);
+            if (k == 3 || k == 8) xa[x] = __builtin_bit_cast(float, d[k == 3 ? 0 : 1][p] << 16);
+            if (k == 4 || k == 8) xb[x] = __builtin_bit_cast(float, d[k == 4 ? 0 : 1][p] & 0xffff0000u);
+            if (k == 5 || k == 9) va[x] -= xa[x];
+            if (k == 6 || k == 10) vb[x] -= xb[x];
+        }
+    };
+
+    f32x16b acc[4][NT];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[e][nt][r] = 0.0f;
+
+    auto barrier = [&] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+
+    // ---- prologue --------------------------------------------------------------------------------------------------
+#pragma unroll
+    for (int i = 0; i < 2 * NDMA; ++i) fetch_sample(i / NDMA, i % NDMA);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int q = 0; q < (e == 0 ? 3 : 1); ++q) load_filter(e, nt, q, set);
+    if (tid < OB) biasT[tid] = bias ? bias[min(o0 + tid, s.O - 1)] : 0.0f;
+    // (the first step's samples have arrived once no more than the second step's and the filters are under way)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
+    barrier();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { read_rows(0, j); combine(j); }
+#pragma unroll
+    for (int t = 0; t < 24; ++t) split_tick(0, t);
+
+    // ---- steps -----------------------------------------------------------------------------------------------------
+    // A position is 12 MFMAs, one per slot; with each go two ticks of the next position's operands and what else is due.
+    auto position = [&](auto ec, int step, int nxt, int nxt2) {
+        constexpr int e = decltype(ec)::value;
+#pragma unroll
+        for (int i = 0; i < 6 * NT; ++i) {
+            const int q = i / NT, nt = i % NT;
+            acc[e][nt] = mfma_bf16(filter(e, nt, kPA[q]), B[e & 1][kPB[q]], acc[e][nt]);
+            // a part's last product has been issued: its registers take the filters that come next
+            if (q == 2 || q == 4 || q == 5) {
+                const int by = q == 2 ? 2 : 1;
+                load_filter((e + by) & 3, nt, kPA[q], e + by >= 4 ? step + KW : step);
+            }
+#pragma unroll
+            for (int tk = 2 * i; tk < 2 * i + 2; ++tk) {
+                split_tick((e + 1) & 3, tk);
+                const int at = 24 * e + tk;         // 0..95 over the step
+                if (at % 4 == 0 && at / 4 < NDMA) fetch_sample(nxt2, at / 4);
+                // Rows of the next step, one channel after the other: read, and some ticks later combined, behind the last
+                // use of what they replace and in front of their own first use.
+                constexpr int kRead[8] = {46, 52, 57, 62, 67, 71, 76, 80}, kComb[8] = {51, 56, 61, 66, 70, 75, 79, 83};
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if (at == kComb[j]) combine(j);
+                    if (at == kRead[j]) read_rows(nxt, j);
+                }
+            }
+            // The next step's samples, requested a step ago, have to be visible before they are read.  (Younger than them are this
+            // step's fetch and at least the filters of a position: more than the count waited for.)
+            if (24 * e + 2 * i + 2 == 36) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
+                barrier();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using std::integral_constant;
+    int nxt = 1, nxt2 = 2;
+    for (int n = 0, step = set; n < s.steps; ++n, step += KW) {
+        position(integral_constant<int, 0>{}, step, nxt, nxt2);
+        position(integral_constant<int, 1>{}, step, nxt, nxt2);
+        position(integral_constant<int, 2>{}, step, nxt, nxt2);
+        position(integral_constant<int, 3>{}, step, nxt, nxt2);
+        nxt = nxt2;
+        nxt2 = nxt2 == 2 ? 0 : nxt2 + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (fetches beyond the last step: LDS is about to be used for something else)
+
+    // ---- epilogue --------------------------------------------------------------------------------------------------
+    // D of the 32x32 MFMA: lane -> tile lane%32; register r -> channel 8*(r/4) + 4*(lane/32) + r%4.  Each wave reduces its row of the
+    // transform to two columns, the rows (and the two sets) meet in LDS.
+    float* P = (float*)lds;                         // [set][row][2][OB][32]
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float m0 = acc[0][nt][r], m1 = acc[1][nt][r], m2 = acc[2][nt][r], m3 = acc[3][nt][r];
+            const int ol = 32 * nt + 8 * (r / 4) + 4 * half + (r % 4);
+            P[(((set * 4 + wave) * 2 + 0) * OB + ol) * 32 + l32] = m0 + m1 + m2;
+            P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + l32] = m1 - m2 + m3;
+        }
+    barrier();
+    constexpr int EO = 8 * KW;                      // output channels finished per pass
+    const int et = tid & 31, eo = tid >> 5;
+    const int etg = t0 + et;
+    const bool eOk = etg < s.T;
+    const int eTy = eOk ? fast_div(etg, tilesXd) : 0;
+    const int ox = eOk ? 2 * (etg - eTy * s.tilesX) : 0, oy = 2 * eTy;
+    auto tile_of = [&](int ol) {
+        float p[4][2];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                p[r][x] = P[((r * 2 + x) * OB + ol) * 32 + et];
+                if (KW == 2) p[r][x] += P[(((4 + r) * 2 + x) * OB + ol) * 32 + et];
+            }
+        return f32x4{p[0][0] + p[1][0] + p[2][0], p[0][1] + p[1][1] + p[2][1], p[1][0] - p[2][0] + p[3][0], p[1][1] - p[2][1] + p[3][1]};
+    };
+#pragma unroll
+    for (int q = 0; q < OB / EO; ++q) {
+        const int ol = eo + EO * q;
+        const f32x4 y = tile_of(ol);
+        if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2);
+    }
+}
+
+struct WsPlan { int kw; size_t lds; WsShape s; };
+
+static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
+    if ((variant & ~1) != 0x100 || W < 1 || H < 1 || I < 1 || O < 1) return false;
+    p->kw = 1 + (variant & 1);
+    WsShape& s = p->s;
+    s.W = W; s.H = H; s.I = I; s.O = O;
+    s.tilesX = (W + 1) / 2;
+    if ((31 + s.tilesX - 1) / s.tilesX + 1 > kWsSegments) return false;     // rows of tiles that a panel can touch
+    // 32-bit byte offsets on the input (a set's last step may lie beyond the last channel) and on the filters
+    if ((long long)W * H * (I + 31) >= (1ll << 29) || (long long)W * H * O >= (1ll << 31) ||
+        (long long)ceil_div(I, kWsKC) * ceil_div(O, 32) * 12288 * 4 >= (1ll << 31)) return false;
+    s.T = s.tilesX * ((H + 1) / 2);
+    s.nC = ceil_div(I, kWsKC);
+    s.nOB = ceil_div(O, 32);
+    s.nTB = ceil_div(s.T, 32);
+    s.nBlocks = s.nTB * ceil_div(O, 64);
+    const FastDiv dx = make_fastdiv(s.tilesX), dt = make_fastdiv(s.nTB);
+    s.mulX = dx.mul; s.shX = dx.shift; s.mulTB = dt.mul; s.shTB = dt.shift;
+    s.steps = ceil_div(s.nC, p->kw);
+    p->lds = (size_t)p->kw * std::max<size_t>(3 * 4 * kWsKC * kWsChunks * 16, 8 * 64 * 32 * sizeof(float));
+    return true;
+}
+
+template <int KW>
+static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, const WsPlan& p, hipStream_t st) {
+    static std::atomic<unsigned long long> asked{0};
+    if (int rc = allow_lds((const void*)winograd_f23_split_kernel<KW>, p.lds, asked)) return rc;
+    launch((winograd_f23_split_kernel<KW>), dim3(ceil_div(p.s.nBlocks, kXcds) * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s);
+    return launched("winograd_f23_split_kernel");
+}
+
+}  // namespace drhip
+
+using namespace drhip;
+
+// Against the fp32 kernel this one gains with the work of a CU and loses with the time of its first loads and its stores, 6 us.
+// Measured, ratio of the times: where every CU has more than one workgroup 0.65 to 0.93 with at least 64 input channels (4
+// steps), 0.91 with 32 channels and 1.5 workgroups per CU and 1.08 to 1.4 with fewer, at best 0.93 with 16; with one
+// workgroup for 0.6 to 1 of the CUs 0.71 to 0.92 from 128 channels on, 0.9 to 1.06 with 64, and with fewer workgroups 1.1 to 1.5
+// (72x72 128->128 1.21, 56x56 256->256 1.26).
+// Up to 32 output channels half of a workgroup would be padding.  Two wave sets where a CU gets one workgroup or none
+// (112x112 128->128 17.7 us against 20.0, 56x56 512->512 52 against 61), one where it gets more (112x112 128->256 29.4 against 34.5).
+extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, int O) {
+    WsPlan p;
+    if (O <= 32 || !ws_plan(W, H, I, O, 0x100, &p)) return 0;
+    const int blocks = p.s.nBlocks, cus = num_cu();
+    if (blocks <= cus) return p.s.steps >= 8 && 20 * blocks >= 11 * cus ? 0x101 : 0;
+    return p.s.steps >= 4 || (p.s.steps >= 2 && 2 * blocks >= 3 * cus) ? 0x100 : 0;
+}
+
+extern "C" size_t drhip_conv3x3_winograd_split_filter_floats(int I, int O) {
+    return I <= 0 || O <= 0 ? 0 : (size_t)ceil_div(I, kWsKC) * ceil_div(O, 32) * 12288;
+}
+
+extern "C" int drhip_winograd_split_filter_transform_f32(const float* w, float* U, int I, int O, void* stream) {
+    DRHIP_REQUIRE(w && U && I > 0 && O > 0, "drhip_winograd_split_filter_transform_f32: bad arguments");
+    const long long fragments = (long long)ceil_div(I, kWsKC) * ceil_div(O, 32);
+    DRHIP_REQUIRE(fragments * 12288 * 4 < (1ll << 31), "drhip_winograd_split_filter_transform_f32: %dx%d filters are too many", I, O);
+    launch(wino_split_filter_kernel, dim3((unsigned)fragments), dim3(256), 0, as_stream(stream), w, (unsigned short*)U, I, O, ceil_div(I, kWsKC), ceil_div(O, 32));
+    return launched("wino_split_filter_kernel");
+}
+
+extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int flags, int variant, void* stream) {
+    DRHIP_REQUIRE(in && U && out, "drhip_conv3x3_winograd_split_f32: NULL tensor");
+    DRHIP_REQUIRE((flags & ~(kEpiRelu | kEpiMaxPool2)) == 0, "drhip_conv3x3_winograd_split_f32: unknown epilogue flags %#x", flags);
+    DRHIP_REQUIRE(!(flags & kEpiMaxPool2) || ((W | H) & 1) == 0, "drhip_conv3x3_winograd_split_f32: fused max pooling needs an even map, not %dx%d", W, H);
+    WsPlan p;
+    DRHIP_REQUIRE(ws_plan(W, H, I, O, variant, &p), "drhip_conv3x3_winograd_split_f32: variant %#x does not cover %dx%dx%d -> %d", variant, W, H, I, O);
+    p.s.flags = flags;
+    p.s.vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
+    const unsigned short* F = (const unsigned short*)U;
+    return p.kw == 1 ? launch_ws<1>(in, F, bias, out, p, as_stream(stream)) : launch_ws<2>(in, F, bias, out, p, as_stream(stream));
+}

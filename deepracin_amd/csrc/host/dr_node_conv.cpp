@@ -69,6 +69,14 @@ gchar* conv_print(dR_Node* node) {
                    algos[c->algo], c->variant);
 }
 
+// A Winograd layer with O output channels: the split-operand kernel where it is the faster one, the fp32 kernel otherwise.
+void pick_winograd(dR_Conv2d_Data* c, int O) {
+    const int W = c->ishape.s0, H = c->ishape.s1, I = c->shape.s2;
+    c->variant = drhip_conv3x3_winograd_split_pick_variant(W, H, I, O);
+    c->drWinoSplit = c->variant != 0;
+    if (!c->drWinoSplit) c->variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
+}
+
 // ---- schedule: kernel variant and tile parameters for gfx950 -------------------------------------
 gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
@@ -81,7 +89,7 @@ gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
                           (long long)W * H * O < (1ll << 31) && (long long)(I + 7) * (O + 31) * 16 < (1ll << 29);
     if (c->algo == drConvWinograd && !packable) c->algo = drConvDirect;
     switch (c->algo) {
-        case drConvWinograd: c->variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O); break;
+        case drConvWinograd: pick_winograd(c, O); break;
         case drConv1x1Gemm:  c->variant = drhip_conv1x1_pick_variant(W * H, I, O); break;
         default: {
             // 3x3, stride 1 or 2, more than 4 input channels: the implicit GEMM on the matrix cores over a filter
@@ -124,14 +132,14 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     if (c->drAbsorbedBy) return TRUE;           // the 3x3 sibling carries this node's filters and bias
     const bool wino = c->algo == drConvWinograd;
     const int O = launch_channels(c);
-    if (c->drAbsorbed1x1)                       // the joint layer is wider than the one schedule() saw
-        c->variant = drhip_conv3x3_winograd_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
-    const int n = wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
+    if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
+    const int n = c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
+                       : wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
                        : c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)
                        : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1) : weight_count(c);
     gboolean ok = dR_createFloatBuffer(net, &c->weightsBuf, n, CL_MEM_READ_ONLY);
     if (launch_has_bias(c)) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, O, CL_MEM_READ_ONLY);
-    const size_t ws = wino ? drhip_conv3x3_winograd_workspace_floats(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->variant) : 0;
+    const size_t ws = wino && !c->drWinoSplit ? drhip_conv3x3_winograd_workspace_floats(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->variant) : 0;
     if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);   // split-K partial tiles
     if (c->drFusedAvgPool)                      // per-tile pixel sums for the pooling behind this layer
         ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, drhip_conv1x1_poolsum_slices(c->ishape.s0 * c->ishape.s1) * O, CL_MEM_READ_WRITE);
@@ -164,7 +172,8 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         cl_mem raw = NULL;
         if (!dR_createFloatBuffer(net, &raw, I * O * 9, CL_MEM_READ_ONLY)) return FALSE;
         ok = dR_uploadArray(net, (gchar*)"", (void*)host, 0, rawBytes, raw);
-        if (ok) ok = !device_failed(net, drhip_winograd_filter_transform_f32((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net)),
+        if (ok) ok = !device_failed(net, c->drWinoSplit ? drhip_winograd_split_filter_transform_f32((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net))
+                                                       : drhip_winograd_filter_transform_f32((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net)),
                                     "winograd filter transform");
         if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "winograd filter transform (sync)");
         dR_clMemoryBufferCleanup(net, raw);
@@ -213,11 +222,12 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
     const int relu = c->activation == tReLU;
     int rc;
     switch (c->algo) {
-        case drConvWinograd:
-            rc = drhip_conv3x3_winograd_f32(in, w, b, out, W, H, I, O,
-                                            (relu ? DRHIP_EPILOGUE_RELU : 0) | (c->drFusedPool ? DRHIP_EPILOGUE_MAXPOOL2 : 0),
-                                            c->variant, (float*)c->workspaceBuf, stream_of(net));
+        case drConvWinograd: {
+            const int flags = (relu ? DRHIP_EPILOGUE_RELU : 0) | (c->drFusedPool ? DRHIP_EPILOGUE_MAXPOOL2 : 0);
+            rc = c->drWinoSplit ? drhip_conv3x3_winograd_split_f32(in, w, b, out, W, H, I, O, flags, c->variant, stream_of(net))
+                                : drhip_conv3x3_winograd_f32(in, w, b, out, W, H, I, O, flags, c->variant, (float*)c->workspaceBuf, stream_of(net));
             break;
+        }
         case drConv1x1Gemm:
             if (c->drFusedAvgPool)
                 rc = drhip_conv1x1_poolsum_f32(in, w, b, (float*)c->workspaceBuf, W * H, I, O, relu, stream_of(net));
