@@ -261,7 +261,8 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
         nxt = nxt2;
         nxt2 = nxt2 == 2 ? 0 : nxt2 + 1;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (fetches beyond the last step: LDS is about to be used for something else)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (fetches beyond the last step, of every wave: LDS is about to be used for
+    barrier();                                              // something else)
 
     // ---- epilogue --------------------------------------------------------------------------------------------------
     // D of the 32x32 MFMA: lane -> tile lane%32; register r -> channel 8*(r/4) + 4*(lane/32) + r%4.  Each wave reduces its row of the
