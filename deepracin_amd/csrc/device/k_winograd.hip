@@ -123,12 +123,7 @@ winograd_filter_transform_kernel(const float* __restrict__ w, float* __restrict_
 struct WinoPackedArgs { unsigned wh, io, mulX, mulTB, cfg0, cfg1; };
 
 // Joined splits (see the kernel's epilogue).
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-constexpr unsigned kWinoEmpty = 0xffa5c3e1u;        // a signalling NaN: marks a workspace slot whose partial tile has not arrived
 constexpr int kWinoMaxJoin = 16;                    // most splits a joined launch can have
-constexpr int kWinoJoinSpins = 1 << 18;             // bound on the wait for a partner's partial tile (some 0.2 s)
-constexpr int kAuxThrough = 1 | 16;                 // cache policy of a buffer access: sc0 sc1, written through to memory
-constexpr int kAuxDeviceVolatile = 16 | (int)0x80000000u;   // sc1 (device scope: not served from this CU's vector cache), reloaded every time
 __device__ unsigned g_wino_join_timeouts;           // partial tiles that never arrived, over the life of the process
 
 __device__ inline f32x4 buf_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, unsigned soffset) {
@@ -962,7 +957,11 @@ extern "C" int drhip_conv3x3_winograd_workspace_prepare_f32(float* workspace, si
 
 extern "C" int drhip_conv3x3_winograd_join_timeouts(unsigned* count) {
     DRHIP_REQUIRE(count, "drhip_conv3x3_winograd_join_timeouts: NULL result pointer");
-    return check(hipMemcpyFromSymbol(count, HIP_SYMBOL(g_wino_join_timeouts), sizeof(unsigned)), "hipMemcpyFromSymbol(join timeouts)");
+    unsigned split = 0;
+    if (int rc = ws_join_timeouts(&split)) return rc;
+    if (int rc = check(hipMemcpyFromSymbol(count, HIP_SYMBOL(g_wino_join_timeouts), sizeof(unsigned)), "hipMemcpyFromSymbol(join timeouts)")) return rc;
+    *count += split;
+    return DRHIP_OK;
 }
 
 extern "C" size_t drhip_conv3x3_winograd_filter_floats(int I, int O) {

@@ -24,24 +24,33 @@
 //   * Filters are transformed and split once, when the layer is prepared, and come as 1 KiB fragments a step or half a step ahead.
 // With KW = 2 two such sets of four waves share the tiles and take alternate steps; their sums meet in LDS.  That is for
 // launches that leave at most one workgroup per CU, where a single set is alone on its SIMDs and waits for its own loads.
+// Launches whose panels do not fill the CUs evenly cut the input channels of all or of the last panels into pieces, which add their
+// sums up inside the launch (the rule, and what it measured, stands at the choice of the variant).
 #include "bf16x3.hpp"
 #include "wino_common.hpp"
 
 #include <algorithm>
 #include <atomic>
+#include <cstdlib>
 #include <type_traits>
 
 namespace drhip {
 
 constexpr int kWsKC = 16;               // input channels per step
-constexpr int kWsChunks = 20;           // 16-byte pieces of a window row of one channel in LDS
-constexpr int kWsSegments = (4 * kWsChunks - 72) / 4 + 1;               // rows of tiles whose samples fit: 2*31 + 3 floats, 4 more per row, 4 in front
+// WC: 16-byte pieces of a window row of one channel in LDS, 20 or (narrow maps) 24.  The rows of tiles whose samples fit:
+// 2*31 + 3 floats, 4 more per row, 4 in front.
+constexpr int ws_segments(int WC) { return (4 * WC - 72) / 4 + 1; }
 
 struct WsShape {                            // everything but the pointers; by value to the kernel
-    int W, H, I, O, tilesX, T, nTB, nBlocks, nC, nOB;   // tiles, panels of 32 tiles, workgroups; 16-channel chunks, 32-channel blocks of filters
+    int W, H, I, O, tilesX, T, nTB, nBlocks, nC, nOB;   // tiles, panels of 32 tiles, panels of outputs; 16-channel chunks, 32-channel blocks of filters
     unsigned mulX, shX, mulTB, shTB;                    // division by tilesX and by nTB
-    int flags, vec2, steps;                             // steps of a wave set
+    int flags, vec2;
+    // The first nA output panels of an XCD are cut into sA splits of perA chunks (in nA * sA workgroups), the others into sB of
+    // perB; mulA, mulB: division by sA and sB
+    int wgsA, nA, sA, sB, perA, perB, mulA, mulB;
 };
+
+__device__ unsigned g_ws_join_timeouts;     // partial tiles that never arrived, over the life of the process
 
 // U[row][chunk][o/32][position in the row][part][lane][8] (bf16): lane l of a wave holds output channel o = l%32 and input
 // channels 8*(l/32) .. +7 of the chunk's 16.  What does not exist is zero.
@@ -73,12 +82,12 @@ wino_split_filter_kernel(const float* __restrict__ w, unsigned short* __restrict
     }
 }
 
-template <int KW>
+template <int KW, int WC>
 __global__ void __launch_bounds__(256 * KW, 2)
 winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __restrict__ U, const float* __restrict__ bias,
-                          float* __restrict__ out, WsShape s) {
+                          float* __restrict__ out, WsShape s, float* __restrict__ ws) {
     constexpr int NT = 2, OB = 32 * NT;
-    constexpr int CHB = kWsChunks * 16, ROWB = kWsKC * CHB, BUFB = 4 * ROWB;    // bytes of a window row of one channel, of 16, of a step's samples
+    constexpr int CHB = WC * 16, ROWB = kWsKC * CHB, BUFB = 4 * ROWB;    // bytes of a window row of one channel, of 16, of a step's samples
     constexpr int NDMA = ROWB / 1024;               // loads of a wave for them: one window row each
     constexpr int kPA[6] = {0, 0, 0, 1, 1, 2}, kPB[6] = {2, 1, 0, 1, 0, 0}; // partial products: part of the filter, part of the sample
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -90,8 +99,13 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX}, nTBd = {(unsigned)s.nTB, s.mulTB, s.shTB};
 
     const int perXcd = (s.nBlocks + kXcds - 1) / kXcds;
-    const int slot = (int)(blockIdx.x >> 3), logical = (int)(blockIdx.x & 7) * perXcd + slot;     // (an XCD works on neighbouring panels)
-    if (slot >= perXcd || logical >= s.nBlocks) return;
+    const int slot = (int)(blockIdx.x >> 3), later = slot - s.wgsA;        // (an XCD works on neighbouring panels)
+    const int nSp = later < 0 ? s.sA : s.sB;
+    const int place = later < 0 ? slot : later, panel = nSp == 1 ? place : place * (later < 0 ? s.mulA : s.mulB) >> 16;
+    const int split = nSp == 1 ? 0 : place - panel * nSp;
+    const int inXcd = (later < 0 ? 0 : s.nA) + panel, logical = (int)(blockIdx.x & 7) * perXcd + inXcd;
+    if (inXcd >= perXcd || logical >= s.nBlocks) return;
+    const int perSplit = later < 0 ? s.perA : s.perB, first = split * perSplit, steps = (perSplit + KW - 1) / KW;
     const int oBlock = fast_div(logical, nTBd);
     const int o0 = oBlock * OB, t0 = (logical - oBlock * s.nTB) * 32;
     const int W = s.W, H = s.H, I = s.I, plane = W * H;
@@ -105,15 +119,15 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     unsigned voff[NDMA];
 #pragma unroll
     for (int i = 0; i < NDMA; ++i) {
-        const int idx = i * 64 + lane, ch = idx / kWsChunks, f = 4 * (idx % kWsChunks);
+        const int idx = i * 64 + lane, ch = idx / WC, f = 4 * (idx % WC);
         int k = 0;
 #pragma unroll
-        for (int q = 1; q < kWsSegments; ++q) k += f >= segment_at(q) ? 1 : 0;
+        for (int q = 1; q < ws_segments(WC); ++q) k += f >= segment_at(q) ? 1 : 0;
         const int x = (k == 0 && off0 > 0 ? 2 * off0 - 1 : 0) + f - segment_at(k), iy = 2 * (ty0 + k) - 1 + wave;
         const bool ok = f >= 4 && x < W && iy >= 0 && iy < H;
-        voff[i] = ok ? 4u * (unsigned)((16 * set + ch) * plane + iy * W + x) : kOutOfRange;
+        voff[i] = ok ? 4u * (unsigned)((16 * (first + set) + ch) * plane + iy * W + x) : kOutOfRange;
     }
-    const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, I * plane * 4, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, min(I, 16 * (first + perSplit)) * plane * 4, kBufferFlags);    // (ends with the split)
     const unsigned stepB = 64u * KW * (unsigned)plane;
     const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(set * 3 * BUFB);
     // 16 bytes per lane, lane by lane, to LDS at M0.  The compiler does not count these loads: where it waits for a filter
@@ -205,7 +219,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int q = 0; q < (e == 0 ? 3 : 1); ++q) load_filter(e, nt, q, set);
+            for (int q = 0; q < (e == 0 ? 3 : 1); ++q) load_filter(e, nt, q, first + set);
     if (tid < OB) biasT[tid] = bias ? bias[min(o0 + tid, s.O - 1)] : 0.0f;
     // (the first step's samples have arrived once no more than the second step's and the filters are under way)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
@@ -253,7 +267,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     };
     using std::integral_constant;
     int nxt = 1, nxt2 = 2;
-    for (int n = 0, step = set; n < s.steps; ++n, step += KW) {
+    for (int n = 0, step = first + set; n < steps; ++n, step += KW) {
         position(integral_constant<int, 0>{}, step, nxt, nxt2);
         position(integral_constant<int, 1>{}, step, nxt, nxt2);
         position(integral_constant<int, 2>{}, step, nxt, nxt2);
@@ -295,6 +309,64 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             }
         return f32x4{p[0][0] + p[1][0] + p[2][0], p[0][1] + p[1][1] + p[2][1], p[1][0] - p[2][0] + p[3][0], p[1][1] - p[2][1] + p[3][1]};
     };
+    if (nSp > 1) {
+        // The splits of a panel add their partial tiles up as those of the fp32 kernel do: each finishes its share of the
+        // passes, stores the others' shares and then looks for its own in the slots of the other splits, whose contents
+        // say themselves whether they have arrived.  (Slots lie at a workgroup's own place in the grid, 8 apart within a panel.)
+        constexpr int NP = OB / EO;
+        const __amdgpu_buffer_rsrc_t rWs = __builtin_amdgcn_make_buffer_rsrc((void*)ws, 0, 0x7ffffff0, kBufferFlags);
+        const unsigned group0 = blockIdx.x - (unsigned)(kXcds * split);
+        // The whole offset goes in the vector register.  With the region in the scalar one the compiler lets the next vector
+        // instruction overwrite the data of a 16-byte store, and on gfx950 the store then now and then takes the new value.
+        auto slot_of = [&](int u, int q) { return (int)((group0 + (unsigned)(kXcds * u)) * (unsigned)(OB * 32 * 16)) + 16 * ((eo + EO * q) * 32 + et); };
+        auto join = [&](auto splitsConst) {
+            constexpr int S = decltype(splitsConst)::value, C = (NP + S - 1) / S;       // C: passes of a split, at most
+            const int q0 = (split * NP + S - 1) / S, count = ((split + 1) * NP + S - 1) / S - q0;
+#pragma unroll
+            for (int q = 0; q < NP; ++q)
+                if (q < q0 || q >= q0 + count)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(eo + EO * q)), rWs, slot_of(split, q), 0, kAuxThrough);
+            const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
+            f32x4 own[C];
+            u32x4 part[C][S];
+#pragma unroll
+            for (int i = 0; i < C; ++i) own[i] = tile_of(eo + EO * (q0 + min(i, count - 1)));
+            bool ready = false;
+            for (int spins = 0; spins < kWinoJoinSpins && !ready; ++spins) {
+                asm volatile("" ::: "memory");          // (to the compiler these loads are invariant)
+                ready = true;
+#pragma unroll
+                for (int i = 0; i < C; ++i)
+#pragma unroll
+                    for (int u = 0; u < S; ++u) part[i][u] = __builtin_amdgcn_raw_buffer_load_b128(rWs, slot_of(u, q0 + min(i, count - 1)), 0, kAuxDeviceVolatile);
+#pragma unroll
+                for (int i = 0; i < C; ++i)
+#pragma unroll
+                    for (int u = 0; u < S; ++u)
+                        ready = ready && (u == split || (part[i][u][0] != kWinoEmpty && part[i][u][1] != kWinoEmpty && part[i][u][2] != kWinoEmpty && part[i][u][3] != kWinoEmpty));
+            }
+#pragma unroll
+            for (int i = 0; i < C; ++i) {
+                if (i >= count) continue;
+                const int q = q0 + i, ol = eo + EO * q;
+                f32x4 y = {0.f, 0.f, 0.f, 0.f};         // splits in order
+#pragma unroll
+                for (int u = 0; u < S; ++u) y += u == split ? own[i] : __builtin_bit_cast(f32x4, part[i][u]);
+#pragma unroll
+                for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, slot_of(u, q), 0, kAuxThrough);
+                if (!ready) {                           // a partner never delivered: say so in the result and in the counter
+                    y = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+                    atomicAdd(&g_ws_join_timeouts, 1u);
+                }
+                if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2);
+            }
+        };
+        if (nSp == 2) join(integral_constant<int, 2>{});
+        else if (nSp == 3) join(integral_constant<int, 3>{});
+        else if (nSp == 4) join(integral_constant<int, 4>{});
+        else if constexpr (KW == 1) join(integral_constant<int, 8>{});
+        return;
+    }
 #pragma unroll
     for (int q = 0; q < OB / EO; ++q) {
         const int ol = eo + EO * q;
@@ -303,15 +375,19 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     }
 }
 
-struct WsPlan { int kw; size_t lds; WsShape s; };
+struct WsPlan { int kw, wc, perXcd; size_t lds; WsShape s; };
 
+// Variant: 0x100 | wave sets - 1 | sA << 12 | sB << 16 | nA << 20, where the first nA output panels of every XCD are cut into
+// sA splits (1, 2, 3, 4 or, with one wave set, 8) of their input channels and the others into sB; all zero: nothing is split.
 static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
-    if ((variant & ~1) != 0x100 || W < 1 || H < 1 || I < 1 || O < 1) return false;
+    if (variant < 0 || (variant & 0xffe) != 0x100 || W < 1 || H < 1 || I < 1 || O < 1) return false;
     p->kw = 1 + (variant & 1);
     WsShape& s = p->s;
     s.W = W; s.H = H; s.I = I; s.O = O;
     s.tilesX = (W + 1) / 2;
-    if ((31 + s.tilesX - 1) / s.tilesX + 1 > kWsSegments) return false;     // rows of tiles that a panel can touch
+    const int segments = (31 + s.tilesX - 1) / s.tilesX + 1;                // rows of tiles that a panel can touch
+    p->wc = segments <= ws_segments(20) ? 20 : 24;
+    if (segments > ws_segments(p->wc)) return false;
     // 32-bit byte offsets on the input (a set's last step may lie beyond the last channel) and on the filters
     if ((long long)W * H * (I + 31) >= (1ll << 29) || (long long)W * H * O >= (1ll << 31) ||
         (long long)ceil_div(I, kWsKC) * ceil_div(O, 32) * 12288 * 4 >= (1ll << 31)) return false;
@@ -322,17 +398,33 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     s.nBlocks = s.nTB * ceil_div(O, 64);
     const FastDiv dx = make_fastdiv(s.tilesX), dt = make_fastdiv(s.nTB);
     s.mulX = dx.mul; s.shX = dx.shift; s.mulTB = dt.mul; s.shTB = dt.shift;
-    s.steps = ceil_div(s.nC, p->kw);
-    p->lds = (size_t)p->kw * std::max<size_t>(3 * 4 * kWsKC * kWsChunks * 16, 8 * 64 * 32 * sizeof(float));
-    return true;
+    p->lds = (size_t)p->kw * std::max<size_t>(3 * 4 * kWsKC * p->wc * 16, 8 * 64 * 32 * sizeof(float));
+    const int panels = ceil_div(s.nBlocks, kXcds);
+    s.nA = variant >> 20; s.sA = variant >> 12 & 15; s.sB = variant >> 16 & 15;
+    if (variant >> 12 == 0) { s.sA = s.sB = 1; s.nA = 0; }
+    s.wgsA = s.nA * s.sA;
+    p->perXcd = s.wgsA + (panels - s.nA) * s.sB;
+    if (s.sA < 1 || s.sB < 1) return false;
+    s.perA = ceil_div(s.nC, s.sA); s.perB = ceil_div(s.nC, s.sB);
+    s.mulA = 65536 / s.sA + 1; s.mulB = 65536 / s.sB + 1;                   // (exact up to 8192 workgroups)
+    if (s.sA == 1 && s.sB == 1) return true;
+    // A workgroup waits for the other splits of its panel, which are its neighbours in dispatch order on the same XCD: as long
+    // as one XCD holds more workgroups than a panel has splits, they all get to run.
+    auto allowed = [&](int n) { return n >= 1 && (n <= 4 || (n == 8 && p->kw == 1)) && (n - 1) * ceil_div(s.nC, n) < s.nC; };
+    return s.nA <= panels && allowed(s.sA) && allowed(s.sB) && std::max(s.sA, s.sB) < num_cu() / kXcds && p->perXcd < 8192 &&
+           (long long)p->perXcd * kXcds * 32768 < (1ll << 31);
 }
 
-template <int KW>
-static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, const WsPlan& p, hipStream_t st) {
+template <int KW, int WC>
+static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, float* ws, const WsPlan& p, hipStream_t st) {
     static std::atomic<unsigned long long> asked{0};
-    if (int rc = allow_lds((const void*)winograd_f23_split_kernel<KW>, p.lds, asked)) return rc;
-    launch((winograd_f23_split_kernel<KW>), dim3(ceil_div(p.s.nBlocks, kXcds) * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s);
+    if (int rc = allow_lds((const void*)winograd_f23_split_kernel<KW, WC>, p.lds, asked)) return rc;
+    launch((winograd_f23_split_kernel<KW, WC>), dim3(p.perXcd * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s, ws);
     return launched("winograd_f23_split_kernel");
+}
+
+int ws_join_timeouts(unsigned* count) {
+    return check(hipMemcpyFromSymbol(count, HIP_SYMBOL(g_ws_join_timeouts), sizeof(unsigned)), "hipMemcpyFromSymbol(join timeouts)");
 }
 
 }  // namespace drhip
@@ -346,16 +438,54 @@ using namespace drhip;
 // (72x72 128->128 1.21, 56x56 256->256 1.26).
 // Up to 32 output channels half of a workgroup would be padding.  Two wave sets where a CU gets one workgroup or none
 // (112x112 128->128 17.7 us against 20.0, 56x56 512->512 52 against 61), one where it gets more (112x112 128->256 29.4 against 34.5).
+//
+// Splits even out what the panels leave uneven, and cost 2.6 us where they are joined (all times here: one layer launched over
+// and over; between other layers the filters come from memory first).  n is the panels per XCD, of 32 CUs:
+//   * n <= 16: all panels in 2 to 4 pieces, as many as leave one workgroup per CU.  That takes 2.75 us per pair of chunks and
+//     10.6 more; the fp32 kernel takes 0.56 us per 8-channel stage of its busiest CU, 3 more and 1.5 for joining.  (40x30
+//     512->512 27.9 us against 36.9; 56x56 256->256 20.8 against 20.7 and 28x28 512->512 21.4 against 21.6 stay there.)
+//   * a few panels more than CUs: two wave sets, a round of whole panels and the rest in 3 or 4 pieces (80x60 512->512
+//     74.4 us, 83.5 with one wave set unsplit; 256->512 43.8 and 45.4).  More than 10 of 32 left over, or below 384
+//     channels more than 6: nothing gained (81x239 256->128, 7 over: 48.6 against 47.6).
+//   * a few more than two per CU: the rest in halves (160x120 256->256 76.1 us against 84.3, 128->256 43.8 against 46.5).
+//     After more rounds than one the workgroups do not end together any more (320x240 128->128, 2.3 rounds: 80 against 74).
 extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, int O) {
     WsPlan p;
     if (O <= 32 || !ws_plan(W, H, I, O, 0x100, &p)) return 0;
-    const int blocks = p.s.nBlocks, cus = num_cu();
-    if (blocks <= cus) return p.s.steps >= 8 && 20 * blocks >= 11 * cus ? 0x101 : 0;
-    return p.s.steps >= 4 || (p.s.steps >= 2 && 2 * blocks >= 3 * cus) ? 0x100 : 0;
+    const int blocks = p.s.nBlocks, nC = p.s.nC, cus = num_cu(), cusPerXcd = cus / kXcds, n = ceil_div(blocks, kXcds);
+    const bool wide = p.wc == 20;                       // (narrower maps are taken only as pieces)
+    static const bool joins = [] { const char* e = getenv("DR_WINO_JOIN"); return !(e && e[0] == '0'); }();
+    auto split = [&](int base, int nA, int sA, int sB) {
+        const int v = base | sA << 12 | sB << 16 | nA << 20;
+        return ws_plan(W, H, I, O, v, &p) ? v : 0;
+    };
+    if (joins && 2 * n <= cusPerXcd) {
+        const int S = std::min(4, cusPerXcd / n), old = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
+        if (!(old & 0x100)) {                           // (layers of its 16-tile form are too small)
+            const int lg = old >> 4 & 15, panels32 = p.s.nTB * ceil_div(O, 32);
+            const double stages = (double)ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus);
+            if (2.75 * ceil_div(ceil_div(nC, S), 2) + 10.6 < 0.93 * (0.56 * stages + (lg > 0 ? 4.5 : 3)))
+                if (const int v = split(0x101, 0, S, S)) return v;
+        }
+    }
+    if (!wide) return 0;
+    const int over = n - cusPerXcd, over2 = n - 2 * cusPerXcd;
+    if (joins && over > 0 && (nC >= 24 ? 3 * over <= cusPerXcd : nC >= 16 && 5 * over <= cusPerXcd))
+        if (const int v = split(0x101, cusPerXcd, 1, 4 * over <= cusPerXcd ? 4 : 3)) return v;
+    if (joins && nC >= 8 && over2 > 0 && 2 * over2 <= cusPerXcd)
+        if (const int v = split(0x100, 2 * cusPerXcd, 1, 2)) return v;
+    if (blocks <= cus) return nC >= 8 && 20 * blocks >= 11 * cus ? 0x101 : 0;
+    return nC >= 4 || (nC >= 2 && 2 * blocks >= 3 * cus) ? 0x100 : 0;
 }
 
 extern "C" size_t drhip_conv3x3_winograd_split_filter_floats(int I, int O) {
     return I <= 0 || O <= 0 ? 0 : (size_t)ceil_div(I, kWsKC) * ceil_div(O, 32) * 12288;
+}
+
+extern "C" size_t drhip_conv3x3_winograd_split_workspace_floats(int W, int H, int I, int O, int variant) {
+    WsPlan p;
+    if (!ws_plan(W, H, I, O, variant, &p) || (p.s.sA == 1 && p.s.sB == 1)) return 0;
+    return (size_t)p.perXcd * kXcds * 8192;
 }
 
 extern "C" int drhip_winograd_split_filter_transform_f32(const float* w, float* U, int I, int O, void* stream) {
@@ -366,14 +496,17 @@ extern "C" int drhip_winograd_split_filter_transform_f32(const float* w, float* 
     return launched("wino_split_filter_kernel");
 }
 
-extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int flags, int variant, void* stream) {
+extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int flags, int variant, float* workspace, void* stream) {
     DRHIP_REQUIRE(in && U && out, "drhip_conv3x3_winograd_split_f32: NULL tensor");
     DRHIP_REQUIRE((flags & ~(kEpiRelu | kEpiMaxPool2)) == 0, "drhip_conv3x3_winograd_split_f32: unknown epilogue flags %#x", flags);
     DRHIP_REQUIRE(!(flags & kEpiMaxPool2) || ((W | H) & 1) == 0, "drhip_conv3x3_winograd_split_f32: fused max pooling needs an even map, not %dx%d", W, H);
     WsPlan p;
     DRHIP_REQUIRE(ws_plan(W, H, I, O, variant, &p), "drhip_conv3x3_winograd_split_f32: variant %#x does not cover %dx%dx%d -> %d", variant, W, H, I, O);
+    DRHIP_REQUIRE(workspace || (p.s.sA == 1 && p.s.sB == 1), "drhip_conv3x3_winograd_split_f32: variant %#x joins splits and needs a prepared workspace", variant);
     p.s.flags = flags;
     p.s.vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
     const unsigned short* F = (const unsigned short*)U;
-    return p.kw == 1 ? launch_ws<1>(in, F, bias, out, p, as_stream(stream)) : launch_ws<2>(in, F, bias, out, p, as_stream(stream));
+    hipStream_t st = as_stream(stream);
+    if (p.wc == 20) return p.kw == 1 ? launch_ws<1, 20>(in, F, bias, out, workspace, p, st) : launch_ws<2, 20>(in, F, bias, out, workspace, p, st);
+    return p.kw == 1 ? launch_ws<1, 24>(in, F, bias, out, workspace, p, st) : launch_ws<2, 24>(in, F, bias, out, workspace, p, st);
 }

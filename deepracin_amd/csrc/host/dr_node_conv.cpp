@@ -77,6 +77,10 @@ void pick_winograd(dR_Conv2d_Data* c, int O) {
     if (!c->drWinoSplit) c->variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
 }
 
+size_t winograd_workspace_floats(const dR_Conv2d_Data* c, int O) {
+    return (c->drWinoSplit ? drhip_conv3x3_winograd_split_workspace_floats : drhip_conv3x3_winograd_workspace_floats)(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->variant);
+}
+
 // ---- schedule: kernel variant and tile parameters for gfx950 -------------------------------------
 gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
@@ -139,7 +143,7 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
                        : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1) : weight_count(c);
     gboolean ok = dR_createFloatBuffer(net, &c->weightsBuf, n, CL_MEM_READ_ONLY);
     if (launch_has_bias(c)) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, O, CL_MEM_READ_ONLY);
-    const size_t ws = wino && !c->drWinoSplit ? drhip_conv3x3_winograd_workspace_floats(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->variant) : 0;
+    const size_t ws = wino ? winograd_workspace_floats(c, O) : 0;
     if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);   // split-K partial tiles
     if (c->drFusedAvgPool)                      // per-tile pixel sums for the pooling behind this layer
         ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, drhip_conv1x1_poolsum_slices(c->ishape.s0 * c->ishape.s1) * O, CL_MEM_READ_WRITE);
@@ -178,10 +182,9 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "winograd filter transform (sync)");
         dR_clMemoryBufferCleanup(net, raw);
         net->clConfig->memConsumptionGPU -= (glong)rawBytes;
-        if (ok && c->workspaceBuf && (c->variant & 0x800))     // joined splits recognise missing partial tiles by a marker
-            ok = !device_failed(net, drhip_conv3x3_winograd_workspace_prepare_f32(
-                                         (float*)c->workspaceBuf, drhip_conv3x3_winograd_workspace_floats(c->ishape.s0, c->ishape.s1, I, O, c->variant),
-                                         stream_of(net)), "winograd workspace");
+        if (ok && c->workspaceBuf && (c->drWinoSplit || (c->variant & 0x800)))     // joined splits recognise missing partial tiles by a marker
+            ok = !device_failed(net, drhip_conv3x3_winograd_workspace_prepare_f32((float*)c->workspaceBuf, winograd_workspace_floats(c, O), stream_of(net)),
+                                "winograd workspace");
         if (ok && a && launch_has_bias(c)) {
             std::vector<float> bias((size_t)O, 0.0f);
             if (a->useBias) memcpy(bias.data(), a->biases, (size_t)O1 * sizeof(float));
@@ -224,7 +227,7 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
     switch (c->algo) {
         case drConvWinograd: {
             const int flags = (relu ? DRHIP_EPILOGUE_RELU : 0) | (c->drFusedPool ? DRHIP_EPILOGUE_MAXPOOL2 : 0);
-            rc = c->drWinoSplit ? drhip_conv3x3_winograd_split_f32(in, w, b, out, W, H, I, O, flags, c->variant, stream_of(net))
+            rc = c->drWinoSplit ? drhip_conv3x3_winograd_split_f32(in, w, b, out, W, H, I, O, flags, c->variant, (float*)c->workspaceBuf, stream_of(net))
                                 : drhip_conv3x3_winograd_f32(in, w, b, out, W, H, I, O, flags, c->variant, (float*)c->workspaceBuf, stream_of(net));
             break;
         }

@@ -228,30 +228,47 @@ def test_winograd_fused_maxpool(lib, dev, oracle, variant, W, H, I, O):
     assert lib.drhip_conv3x3_winograd_f32(p, U, None, p, 4, 4, I, O, 4, 1, None, None) == -1      # unknown flag
 
 
-@pytest.mark.parametrize("variant", [0x100, 0x101])
-@pytest.mark.parametrize("W,H,I,O", [(33, 17, 16, 33), (31, 40, 17, 70), (61, 63, 64, 128), (32, 2, 33, 65), (224, 20, 3, 64), (75, 1, 48, 1), (320, 6, 40, 96)])
+SPLIT_HALVES, SPLIT_MIXED = 2 << 12 | 2 << 16, 1 << 12 | 4 << 16 | 1 << 20
+
+
+@pytest.mark.parametrize("variant", [0x100, 0x101, 0x100 | SPLIT_HALVES, 0x101 | SPLIT_HALVES, 0x101 | 3 << 12 | 3 << 16, 0x101 | SPLIT_MIXED,
+                                     0x100 | 3 << 12 | 8 << 16 | 1 << 20])
+@pytest.mark.parametrize("W,H,I,O", [(33, 17, 16, 33), (31, 40, 17, 70), (61, 63, 64, 128), (32, 2, 33, 65), (224, 20, 3, 64), (75, 1, 48, 1), (320, 6, 40, 96),
+                                     (11, 30, 33, 40), (14, 14, 130, 65), (28, 28, 256, 512), (27, 13, 112, 512)])
 def test_winograd_split_operands(lib, dev, oracle, variant, W, H, I, O):
     """Winograd on the bf16 matrix cores, operands split into three parts: ragged channels on both sides, a last step without
-    channels, panels over up to three rows of tiles and over the end of the map, one-row maps, the pooling epilogue.
+    channels, panels over up to six rows of tiles and over the end of the map, one-row maps, the pooling epilogue; input channels in
+    equal and ragged pieces that are joined inside the launch, two launches on one workspace.
     Held to a twentieth of the layer bar: the parts carry all 24 bits."""
     x, w, b = rnd(I, H, W), rnd(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I))), rnd(O, scale=0.1)
     F = dev.empty(lib.drhip_conv3x3_winograd_split_filter_floats(I, O))
     ok(lib, lib.drhip_winograd_split_filter_transform_f32(dev.put(w), F, I, O, None))
     xd, bd = dev.put(x), dev.put(b)
+    n, ws = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant), None
+    if variant >> 12 and n == 0:                # fewer panels or chunks than the variant needs: refused
+        assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, dev.empty(O * H * W), W, H, I, O, 0, variant, xd, None) == -1
+        return
+    if n:
+        assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, dev.empty(O * H * W), W, H, I, O, 0, variant, None, None) == -1      # no workspace
+        ws = dev.empty(n)
+        ok(lib, lib.drhip_conv3x3_winograd_workspace_prepare_f32(ws, n, None))
     for relu, bias in ((1, b), (0, None)):
         y = dev.empty(O * H * W)
-        ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, bd if bias is not None else None, y, W, H, I, O, relu, variant, None))
+        ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, bd if bias is not None else None, y, W, H, I, O, relu, variant, ws, None))
         want = oracle.conv_f64(x, w, bias, relu=bool(relu))
         got = dev.get(y, want.shape)
         assert_close(got, want, "split operands")
         assert rel_err(got, want) <= TOL / 20
         pooled = dev.empty(O * (H // 2) * (W // 2))
-        rc = lib.drhip_conv3x3_winograd_split_f32(xd, F, bd if bias is not None else None, pooled, W, H, I, O, relu | 2, variant, None)
+        rc = lib.drhip_conv3x3_winograd_split_f32(xd, F, bd if bias is not None else None, pooled, W, H, I, O, relu | 2, variant, ws, None)
         assert rc == (-1 if W % 2 or H % 2 else 0)
         if rc == 0:
             mx = oracle.pool(got, (2, 2, 1), (2, 2, 1), 0)
             assert np.array_equal(dev.get(pooled, mx.shape), mx)
-    assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, xd, 30, 4, I, O, 0, variant, None) == -1      # more than three rows of tiles in a panel
+    late = ctypes.c_uint(1)
+    ok(lib, lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)))
+    assert late.value == 0
+    assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, xd, 10, 4, I, O, 0, variant, ws, None) == -1      # more rows of tiles in a panel than LDS has room for
 
 
 @pytest.mark.parametrize("variant", [0x811, 0x812, 0x821, 0x831, 0xc11, 0xc12, 0xc21, 0xc22, 0xc31])
