@@ -82,7 +82,8 @@ wino_split_filter_kernel(const float* __restrict__ w, unsigned short* __restrict
     }
 }
 
-template <int KW, int WC>
+// TURNS: see `turn`.  (Of its own, because even its few instructions show on layers of three steps: 41x53 254->254 0.17 us.)
+template <int KW, int WC, bool TURNS>
 __global__ void __launch_bounds__(256 * KW, 2)
 winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __restrict__ U, const float* __restrict__ bias,
                           float* __restrict__ out, WsShape s, float* __restrict__ ws) {
@@ -115,8 +116,12 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     // multiple of 16 bytes on: from column 2*tx-1 of its first tile, or from column 0 where that is left of the map (the sample
     // in front of it is then whatever lies in front of it: it is multiplied by zero).
     const int ty0 = fast_div(t0, tilesXd), off0 = t0 - ty0 * s.tilesX;
+    // Panels of an XCD begin at different channels and go round: the first to reach a fragment of the filters brings it from
+    // memory, the others find it in L2, and they take turns at that instead of all waiting for it together.
+    const int turn = TURNS ? min(inXcd & 31, steps - 1) : 0;
     auto segment_at = [&](int k) { return k == 0 ? 4 : (2 * (k * s.tilesX - off0) + 4 * k + 6) & ~3; };     // in floats
-    unsigned voff[NDMA];
+    const unsigned stepB = 64u * KW * (unsigned)plane;
+    unsigned voff[NDMA];                                // (never below kOutOfRange where it started from that)
 #pragma unroll
     for (int i = 0; i < NDMA; ++i) {
         const int idx = i * 64 + lane, ch = idx / WC, f = 4 * (idx % WC);
@@ -125,17 +130,25 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
         for (int q = 1; q < ws_segments(WC); ++q) k += f >= segment_at(q) ? 1 : 0;
         const int x = (k == 0 && off0 > 0 ? 2 * off0 - 1 : 0) + f - segment_at(k), iy = 2 * (ty0 + k) - 1 + wave;
         const bool ok = f >= 4 && x < W && iy >= 0 && iy < H;
-        voff[i] = ok ? 4u * (unsigned)((16 * (first + set) + ch) * plane + iy * W + x) : kOutOfRange;
+        voff[i] = (ok ? 4u * (unsigned)((16 * (first + set) + ch) * plane + iy * W + x) : kOutOfRange) + (unsigned)turn * stepB;
     }
     const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, min(I, 16 * (first + perSplit)) * plane * 4, kBufferFlags);    // (ends with the split)
-    const unsigned stepB = 64u * KW * (unsigned)plane;
     const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(set * 3 * BUFB);
     // 16 bytes per lane, lane by lane, to LDS at M0.  The compiler does not count these loads: where it waits for a filter
     // it waits for a few more loads than it means to, and for the samples this kernel waits itself.
+    int fetching = turn, left = steps;                  // the step whose samples are fetched next; how many are to come
+    unsigned toNext = 0;
     auto fetch_sample = [&](int buf, int i) {
+        if (i == 0) {
+            const bool last = TURNS && fetching == steps - 1;
+            // (behind the last one out of the map: zeros that nobody uses cost no trip to memory)
+            toNext = TURNS && left == 1 ? kOutOfRange : TURNS && left < 1 ? 0 : last ? stepB - (unsigned)steps * stepB : stepB;
+            --left;
+            if (TURNS) fetching = last ? 0 : fetching + 1;
+        }
         const unsigned at = ldsBase + (unsigned)(buf * BUFB + wave * ROWB);
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff[i]), "s"(rIn), "s"(at + 1024u * i) : "memory");
-        voff[i] += stepB;
+        voff[i] += toNext;
     };
 
     // ---- filters ---------------------------------------------------------------------------------------------------
@@ -219,7 +232,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int q = 0; q < (e == 0 ? 3 : 1); ++q) load_filter(e, nt, q, first + set);
+            for (int q = 0; q < (e == 0 ? 3 : 1); ++q) load_filter(e, nt, q, first + set + KW * turn);
     if (tid < OB) biasT[tid] = bias ? bias[min(o0 + tid, s.O - 1)] : 0.0f;
     // (the first step's samples have arrived once no more than the second step's and the filters are under way)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
@@ -231,7 +244,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
 
     // ---- steps -----------------------------------------------------------------------------------------------------
     // A position is 12 MFMAs, one per slot; with each go two ticks of the next position's operands and what else is due.
-    auto position = [&](auto ec, int step, int nxt, int nxt2) {
+    auto position = [&](auto ec, int step, int stepNext, int nxt, int nxt2) {
         constexpr int e = decltype(ec)::value;
 #pragma unroll
         for (int i = 0; i < 6 * NT; ++i) {
@@ -240,7 +253,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             // a part's last product has been issued: its registers take the filters that come next
             if (q == 2 || q == 4 || q == 5) {
                 const int by = q == 2 ? 2 : 1;
-                load_filter((e + by) & 3, nt, kPA[q], e + by >= 4 ? step + KW : step);
+                load_filter((e + by) & 3, nt, kPA[q], e + by >= 4 ? stepNext : step);
             }
 #pragma unroll
             for (int tk = 2 * i; tk < 2 * i + 2; ++tk) {
@@ -267,11 +280,14 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     };
     using std::integral_constant;
     int nxt = 1, nxt2 = 2;
-    for (int n = 0, step = first + set; n < steps; ++n, step += KW) {
-        position(integral_constant<int, 0>{}, step, nxt, nxt2);
-        position(integral_constant<int, 1>{}, step, nxt, nxt2);
-        position(integral_constant<int, 2>{}, step, nxt, nxt2);
-        position(integral_constant<int, 3>{}, step, nxt, nxt2);
+    for (int n = 0, m = turn; n < steps; ++n) {
+        const int step = first + set + KW * m;
+        m = TURNS && m == steps - 1 ? 0 : m + 1;
+        const int stepNext = first + set + KW * m;
+        position(integral_constant<int, 0>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 1>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 2>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 3>{}, step, stepNext, nxt, nxt2);
         nxt = nxt2;
         nxt2 = nxt2 == 2 ? 0 : nxt2 + 1;
     }
@@ -375,7 +391,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     }
 }
 
-struct WsPlan { int kw, wc, perXcd; size_t lds; WsShape s; };
+struct WsPlan { int kw, wc, perXcd; bool turns; size_t lds; WsShape s; };
 
 // Variant: 0x100 | wave sets - 1 | sA << 12 | sB << 16 | nA << 20, where the first nA output panels of every XCD are cut into
 // sA splits (1, 2, 3, 4 or, with one wave set, 8) of their input channels and the others into sB; all zero: nothing is split.
@@ -387,7 +403,7 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     s.tilesX = (W + 1) / 2;
     const int segments = (31 + s.tilesX - 1) / s.tilesX + 1;                // rows of tiles that a panel can touch
     p->wc = segments <= ws_segments(20) ? 20 : 24;
-    if (segments > ws_segments(p->wc)) return false;
+    if (segments > ws_segments(p->wc) || (p->wc == 24 && p->kw == 1)) return false;     // (one wave set never gained on narrow maps)
     // 32-bit byte offsets on the input (a set's last step may lie beyond the last channel) and on the filters
     if ((long long)W * H * (I + 31) >= (1ll << 29) || (long long)W * H * O >= (1ll << 31) ||
         (long long)ceil_div(I, kWsKC) * ceil_div(O, 32) * 12288 * 4 >= (1ll << 31)) return false;
@@ -399,7 +415,7 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     const FastDiv dx = make_fastdiv(s.tilesX), dt = make_fastdiv(s.nTB);
     s.mulX = dx.mul; s.shX = dx.shift; s.mulTB = dt.mul; s.shTB = dt.shift;
     p->lds = (size_t)p->kw * std::max<size_t>(3 * 4 * kWsKC * p->wc * 16, 8 * 64 * 32 * sizeof(float));
-    const int panels = ceil_div(s.nBlocks, kXcds);
+    const int panels = ceil_div(s.nBlocks, kXcds), cusPerXcd = num_cu() / kXcds;
     s.nA = variant >> 20; s.sA = variant >> 12 & 15; s.sB = variant >> 16 & 15;
     if (variant >> 12 == 0) { s.sA = s.sB = 1; s.nA = 0; }
     s.wgsA = s.nA * s.sA;
@@ -407,6 +423,14 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     if (s.sA < 1 || s.sB < 1) return false;
     s.perA = ceil_div(s.nC, s.sA); s.perB = ceil_div(s.nC, s.sB);
     s.mulA = 65536 / s.sA + 1; s.mulB = 65536 / s.sB + 1;                   // (exact up to 8192 workgroups)
+    // Beginning at different channels.  Measured with other filters and maps for every launch, us, all from the first channel
+    // on / in 32 turns: two wave sets, 80x60 512->512 87.7 / 82.1, 80x60 256->512 51.4 / 46.2, 56x56 512->512 63.5 / 59.3, 40x30
+    // 512->512 32.4 / 31.1; one set in one to two rounds, 160x120 256->256 84.1 / 78.4, 128->256 49.4 / 47.0.  With one set in
+    // less than a round a CU's two workgroups read the same filters and lose that (80x60 512->512 93 / 100); over more rounds
+    // the panels drift apart by themselves (320x240 128->128 87.0 / 87.7).
+    // (Pieces of fewer than 8 chunks have no turns to take: 41x53 254->254 in thirds 0.1 us slower.)
+    const int longest = s.nA > 0 ? s.perA : s.perB;
+    p->turns = longest >= 8 && (p->kw == 2 || (panels > 2 * cusPerXcd && panels <= 4 * cusPerXcd));
     if (s.sA == 1 && s.sB == 1) return true;
     // A workgroup waits for the other splits of its panel, which are its neighbours in dispatch order on the same XCD: as long
     // as one XCD holds more workgroups than a panel has splits, they all get to run.
@@ -415,11 +439,11 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
            (long long)p->perXcd * kXcds * 32768 < (1ll << 31);
 }
 
-template <int KW, int WC>
+template <int KW, int WC, bool TURNS>
 static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, float* ws, const WsPlan& p, hipStream_t st) {
     static std::atomic<unsigned long long> asked{0};
-    if (int rc = allow_lds((const void*)winograd_f23_split_kernel<KW, WC>, p.lds, asked)) return rc;
-    launch((winograd_f23_split_kernel<KW, WC>), dim3(p.perXcd * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s, ws);
+    if (int rc = allow_lds((const void*)winograd_f23_split_kernel<KW, WC, TURNS>, p.lds, asked)) return rc;
+    launch((winograd_f23_split_kernel<KW, WC, TURNS>), dim3(p.perXcd * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s, ws);
     return launched("winograd_f23_split_kernel");
 }
 
@@ -451,7 +475,7 @@ using namespace drhip;
 //     After more rounds than one the workgroups do not end together any more (320x240 128->128, 2.3 rounds: 80 against 74).
 extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, int O) {
     WsPlan p;
-    if (O <= 32 || !ws_plan(W, H, I, O, 0x100, &p)) return 0;
+    if (O <= 32 || !ws_plan(W, H, I, O, 0x101, &p)) return 0;
     const int blocks = p.s.nBlocks, nC = p.s.nC, cus = num_cu(), cusPerXcd = cus / kXcds, n = ceil_div(blocks, kXcds);
     const bool wide = p.wc == 20;                       // (narrower maps are taken only as pieces)
     static const bool joins = [] { const char* e = getenv("DR_WINO_JOIN"); return !(e && e[0] == '0'); }();
@@ -507,6 +531,7 @@ extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U,
     p.s.vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
     const unsigned short* F = (const unsigned short*)U;
     hipStream_t st = as_stream(stream);
-    if (p.wc == 20) return p.kw == 1 ? launch_ws<1, 20>(in, F, bias, out, workspace, p, st) : launch_ws<2, 20>(in, F, bias, out, workspace, p, st);
-    return p.kw == 1 ? launch_ws<1, 24>(in, F, bias, out, workspace, p, st) : launch_ws<2, 24>(in, F, bias, out, workspace, p, st);
+    if (p.wc == 24) return p.turns ? launch_ws<2, 24, true>(in, F, bias, out, workspace, p, st) : launch_ws<2, 24, false>(in, F, bias, out, workspace, p, st);
+    if (p.kw == 2) return p.turns ? launch_ws<2, 20, true>(in, F, bias, out, workspace, p, st) : launch_ws<2, 20, false>(in, F, bias, out, workspace, p, st);
+    return p.turns ? launch_ws<1, 20, true>(in, F, bias, out, workspace, p, st) : launch_ws<1, 20, false>(in, F, bias, out, workspace, p, st);
 }

@@ -236,8 +236,8 @@ int drhip_conv3x3_winograd_join_timeouts(unsigned* count);
  * partial products, fp32 accumulation), for large layers.  F is the transformed and split filter bank, made once at
  * prepare time from w [I][O][3][3]; drhip_conv3x3_winograd_split_filter_floats(I,O) floats, 16-byte aligned.
  * drhip_conv3x3_winograd_split_pick_variant returns 0 where drhip_conv3x3_winograd_f32 is the faster one (or this one
- * does not cover the shape: maps less than 11 wide, tensors beyond 32-bit byte offsets), else the variant to pass: 0x100 for
- * one set of four waves per workgroup, 0x101 for two that take alternate groups of 16 input channels, | sA << 12 | sB << 16 | nA << 20
+ * does not cover the shape: maps less than 11 wide, tensors beyond 32-bit byte offsets), else the variant to pass: 0x100 for one
+ * set of four waves per workgroup (maps from 31 wide on), 0x101 for two that take alternate groups of 16 input channels, | sA << 12 | sB << 16 | nA << 20
  * if the input channels are split: the first nA panels of outputs on each XCD into sA pieces, the others into sB.  Such a launch
  * joins the pieces itself and needs a workspace of drhip_conv3x3_winograd_split_workspace_floats floats that has been
  * through drhip_conv3x3_winograd_workspace_prepare_f32, for one launch at a time. */

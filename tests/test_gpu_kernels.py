@@ -234,7 +234,7 @@ SPLIT_HALVES, SPLIT_MIXED = 2 << 12 | 2 << 16, 1 << 12 | 4 << 16 | 1 << 20
 @pytest.mark.parametrize("variant", [0x100, 0x101, 0x100 | SPLIT_HALVES, 0x101 | SPLIT_HALVES, 0x101 | 3 << 12 | 3 << 16, 0x101 | SPLIT_MIXED,
                                      0x100 | 3 << 12 | 8 << 16 | 1 << 20])
 @pytest.mark.parametrize("W,H,I,O", [(33, 17, 16, 33), (31, 40, 17, 70), (61, 63, 64, 128), (32, 2, 33, 65), (224, 20, 3, 64), (75, 1, 48, 1), (320, 6, 40, 96),
-                                     (11, 30, 33, 40), (14, 14, 130, 65), (28, 28, 256, 512), (27, 13, 112, 512)])
+                                     (11, 30, 33, 40), (14, 14, 130, 65), (28, 28, 256, 512), (27, 13, 112, 512), (14, 30, 272, 64)])
 def test_winograd_split_operands(lib, dev, oracle, variant, W, H, I, O):
     """Winograd on the bf16 matrix cores, operands split into three parts: ragged channels on both sides, a last step without
     channels, panels over up to six rows of tiles and over the end of the map, one-row maps, the pooling epilogue; input channels in
@@ -245,7 +245,7 @@ def test_winograd_split_operands(lib, dev, oracle, variant, W, H, I, O):
     ok(lib, lib.drhip_winograd_split_filter_transform_f32(dev.put(w), F, I, O, None))
     xd, bd = dev.put(x), dev.put(b)
     n, ws = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant), None
-    if variant >> 12 and n == 0:                # fewer panels or chunks than the variant needs: refused
+    if n == 0 and (variant >> 12 or (W < 31 and variant == 0x100)):     # fewer panels or chunks than the variant needs, or a narrow map: refused
         assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, dev.empty(O * H * W), W, H, I, O, 0, variant, xd, None) == -1
         return
     if n:
@@ -269,6 +269,23 @@ def test_winograd_split_operands(lib, dev, oracle, variant, W, H, I, O):
     ok(lib, lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)))
     assert late.value == 0
     assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, xd, 10, 4, I, O, 0, variant, ws, None) == -1      # more rows of tiles in a panel than LDS has room for
+
+
+@pytest.mark.parametrize("W,H,I,O", [(257, 129, 113, 65), (21, 48, 400, 512), (33, 31, 256, 512)])
+def test_winograd_split_picked(lib, dev, oracle, W, H, I, O):
+    """The variant that the rule picks: a round of whole panels and halves behind it, narrow and wide maps in pieces, panels
+    that begin at different channels."""
+    variant = lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O)
+    n = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant)
+    assert variant >> 12 and n
+    x, w = rnd(I, H, W), rnd(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I)))
+    F, ws, y, xd = dev.empty(lib.drhip_conv3x3_winograd_split_filter_floats(I, O)), dev.empty(n), dev.empty(O * H * W), dev.put(x)
+    ok(lib, lib.drhip_winograd_split_filter_transform_f32(dev.put(w), F, I, O, None))
+    ok(lib, lib.drhip_conv3x3_winograd_workspace_prepare_f32(ws, n, None))
+    want = oracle.conv_f64(x, w, None, relu=False)
+    for _ in range(3):
+        ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, None, y, W, H, I, O, 0, variant, ws, None))
+        assert rel_err(dev.get(y, want.shape), want) <= TOL / 20
 
 
 @pytest.mark.parametrize("variant", [0x811, 0x812, 0x821, 0x831, 0xc11, 0xc12, 0xc21, 0xc22, 0xc31])
