@@ -18,8 +18,9 @@ of 20 passes is a few milliseconds long and a single sample of it says little), 
                  that, so `frac` is credit for the algorithm, NOT matrix-pipe utilisation: that is
                  `issued_tflops` (the FLOPs the kernel really issues, 2*16*tiles*I*O with tiles, I and O
                  padded to its blocks -- the counter SQ_INSTS_VALU_MFMA_MOPS_F32 reads exactly this, see
-                 profiles/) and `mfma_busy_frac` = issued_tflops / 157.3, the share of the data-sheet
-                 matrix peak the pipe was issuing at; the >= 50 % target is judged on `mfma_busy_frac`.
+                 profiles/; six bf16 products each on the layers of the split-operand kernel) and
+                 `mfma_busy_frac`, the share of the data-sheet matrix peaks (157.3 fp32, 2500 bf16) the
+                 pipe was issuing at; the >= 50 % target is judged on `mfma_busy_frac`.
                  `mfma_busy_frac_counters` is the same share from SQ_VALU_MFMA_BUSY_CYCLES of the
                  committed rocprofv3 run (profiles/counters.json: busy cycles per SIMD / (this run's device
                  time x 2.4 GHz)), `mfma_busy_frac_profiled` the share over the profiler's own, longer,
@@ -69,6 +70,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 PEAK_MFMA_F32_TFLOPS = 157.3
+PEAK_MFMA_BF16_TFLOPS = 2500.0      # dense
 PEAK_HBM_GBS = 8000.0
 PEAK_CLOCK_GHZ = 2.4            # the clock the data-sheet peak is quoted at
 COUNTERS_JSON = os.path.join(ROOT, "profiles", "counters.json")
@@ -106,16 +108,19 @@ KERNEL_NAMES = {"winograd": "winograd_f23_mfma_kernel", "conv1x1": "conv1x1_mfma
 def winograd_issued_flops(lib, W, H, I, O):
     """FLOPs the Winograd kernel issues for a layer: 16 GEMMs over tiles x I x O, each padded to the blocks of
     the variant the scheduler picks (tile blocks of 32 or 16, 8 input channels per stage, 32/64/128 or 16/32/64
-    output channels per workgroup); drhip_conv3x3_winograd_f32 decides the same way."""
+    output channels per workgroup); drhip_conv3x3_winograd_f32 decides the same way.  With it the peak of the matrix cores it
+    runs on: large layers take the split-operand kernel, six bf16 products (32 tiles x 16 channels x 64 channels) for each fp32 one."""
     v = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O)
     tb = 16 if v & 0x100 else 32
     ob = tb * {1: 1, 2: 2, 3: 4}[v & 0xf]
     tiles = ((W + 1) // 2) * ((H + 1) // 2)
     pad = lambda n, m: -(-n // m) * m
+    if lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O):
+        return 6 * 2 * 16 * pad(tiles, 32) * pad(I, 16) * pad(O, 64), PEAK_MFMA_BF16_TFLOPS
     # (an image layer -- at most 4 input channels, 32-tile blocks, unsplit, four waves -- runs its one stage without
     # the two k-steps that would multiply zeros)
     few = I <= 4 and tb == 32 and (v & 0xf) <= 2 and not (v & 0x400) and not (v >> 4) & 0xf
-    return 2 * 16 * pad(tiles, tb) * (4 if few else pad(I, 8)) * pad(O, ob)
+    return 2 * 16 * pad(tiles, tb) * (4 if few else pad(I, 8)) * pad(O, ob), PEAK_MFMA_F32_TFLOPS
 
 
 def measure(workload, seed, steps, warmup, blocks=BLOCKS, instrument=True, env_vars=None):
@@ -226,7 +231,7 @@ def analyse(lib, m, workload, counters):
         if n["op"] == "feed":
             continue
         k = kind_of(n)
-        gk = groups.setdefault(k, {"ms": 0.0, "flops": 0, "issued": 0, "bytes": 0, "launches": 0})
+        gk = groups.setdefault(k, {"ms": 0.0, "flops": 0, "issued": 0, "busy_ms": 0.0, "bytes": 0, "launches": 0})
         gk["ms"] += ms[i]
         gk["flops"] += merged.get(i, 0)
         gk["launches"] += 1 if ms[i] > 0 else 0
@@ -238,13 +243,14 @@ def analyse(lib, m, workload, counters):
         if k == "winograd" and ms[i] > 0:
             W, H, _ = shapes[n["in"]]
             I, O = n["w"].shape[0], joint_o.get(i, n["w"].shape[1])
-            issued = winograd_issued_flops(lib, W, H, I, O)
+            issued, peak = winograd_issued_flops(lib, W, H, I, O)
             gk["issued"] += issued
+            gk["busy_ms"] += issued / peak / 1e9
             v = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O)
-            if (v >> 4) & 0xf and not v & 0x800:       # split layers whose partial tiles are summed by a second kernel
+            if peak == PEAK_MFMA_F32_TFLOPS and (v >> 4) & 0xf and not v & 0x800:       # split layers whose partial tiles are summed by a second kernel
                 gk["kernels"] += 1
             row["issued_tflops"] = round(issued / (ms[i] * 1e-3) / 1e12, 2)
-            row["mfma_busy_frac"] = round(issued / (ms[i] * 1e-3) / 1e12 / PEAK_MFMA_F32_TFLOPS, 4)
+            row["mfma_busy_frac"] = round(issued / (ms[i] * 1e-3) / 1e12 / peak, 4)
         if k == "fc" and ms[i] > 0:
             K, N = n["w"].shape
             b = 4 * (K * N + K + 2 * N)
@@ -272,8 +278,8 @@ def analyse(lib, m, workload, counters):
             # counters of the committed rocprofv3 run: busy cycles per SIMD over THIS run's device time (the profiler's own
             # timestamps run ~10 % long), and the share under the profiler itself
             cyc = rec.get("mfma_busy_cycles_per_simd")
-            roofline.update({"issued_tflops": round(issued, 3), "frac_issued": round(issued / PEAK_MFMA_F32_TFLOPS, 4),
-                             "mfma_busy_frac": round(issued / PEAK_MFMA_F32_TFLOPS, 4),
+            roofline.update({"issued_tflops": round(issued, 3), "frac_issued": round(gk["busy_ms"] / gk["ms"], 4),
+                             "mfma_busy_frac": round(gk["busy_ms"] / gk["ms"], 4),
                              "mfma_busy_frac_counters": round(cyc / (gk["ms"] * 1e3 * PEAK_CLOCK_GHZ * 1e3), 4) if cyc else None,
                              "mfma_busy_frac_profiled": rec.get("mfma_busy_frac"),
                              "target": "mfma_busy_frac >= 0.50"})
