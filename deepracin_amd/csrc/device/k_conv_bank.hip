@@ -65,6 +65,29 @@ conv_bank_layout_kernel(const float* __restrict__ w, unsigned short* __restrict_
     for (int q = 0; q < 3; ++q) F[((((size_t)chunk * steps + step) * 3 + q) * oBlocks + ob) * 512 + lane * 8 + e] = part[q];
 }
 
+// One output in fp32, without the bias: an infinite sample (or one that bf16 rounds to infinity) has no three-part form and
+// leaves NaN behind, so an output that came out as NaN is worked out again from the samples and the filters put together.
+template <int CP>
+__device__ __forceinline__ float conv_bank_exact(const float* in, const unsigned short* F, const BankShape& s, int o, int x, int y) {
+    const int kh = s.steps / s.spr;
+    float v = 0.0f;
+#pragma clang loop unroll(disable)
+    for (int c = 0; c < s.I; ++c)
+#pragma clang loop unroll(disable)
+        for (int j = 0; j < kh; ++j)
+#pragma clang loop unroll(disable)
+            for (int i = 0; i < s.kw; ++i) {
+                const int ix = x * s.sx - s.padX + i, iy = y * s.sy - s.padY + j;
+                if (ix < 0 || ix >= s.W || iy < 0 || iy >= s.H) continue;
+                const int chunk = CP == 16 ? c >> 4 : 0, k = CP == 16 ? c & 15 : 4 * (i & 3) + c, step = j * s.spr + (CP == 16 ? i : i >> 2);
+                float w = 0.0f;
+                for (int q = 2; q >= 0; --q)
+                    w += __uint_as_float((unsigned)F[((((size_t)chunk * s.steps + step) * 3 + q) * s.oBlocks + (o >> 5)) * 512 + ((k >> 3) * 32 + (o & 31)) * 8 + (k & 7)] << 16);
+                v = fmaf(w, in[((size_t)c * s.H + iy) * s.W + ix], v);
+            }
+    return v;
+}
+
 // PF: staging rounds (512 units each) of the next 16 channels that are kept in registers.
 template <int CP, int MT, int WO, int WK, int PF>
 __global__ void __launch_bounds__(kBankThreads)
@@ -265,9 +288,11 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         for (int k = 0; k < WK; ++k) v += part[((k * 32 * WO + oc) * MT + m) * kPitch + pl];
         const int o = blockIdx.z * (32 * WO) + oc;
         const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
+        const bool ok = o < s.O && x < s.Wo && y < s.Ho;
+        if (ok && v != v) v = conv_bank_exact<CP>(in, F, s, o, x, y);
         v += biasT[oc];
         if (s.relu) v = fmaxf(v, 0.0f);
-        if (o < s.O && x < s.Wo && y < s.Ho) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
+        if (ok) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
     }
 }
 

@@ -228,6 +228,30 @@ def test_winograd_fused_maxpool(lib, dev, oracle, variant, W, H, I, O):
     assert lib.drhip_conv3x3_winograd_f32(p, U, None, p, 4, 4, I, O, 4, 1, None, None) == -1      # unknown flag
 
 
+@pytest.mark.parametrize("I,k,stride", [(3, 7, 2), (4, 5, 1), (20, 5, 1), (17, 3, 3)])
+def test_conv_bank_keeps_infinities(lib, dev, I, k, stride):
+    """An infinite sample gives what fp32 arithmetic gives, in the filter's reach and nowhere else."""
+    W, H, O = 23, 19, 40
+    x, w = rnd(I, H, W), rnd(I, O, k, k)
+    x[1, 9, 12], x[I - 1, 0, 0], x[0, H - 1, W - 1] = np.inf, -np.inf, np.nan
+    F = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k))
+    ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
+    Wo, Ho = W // stride, H // stride
+    y = dev.empty(O * Ho * Wo)
+    ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, None, y, W, H, I, O, k, k, stride, stride, 0, 0, None))
+    got, want = dev.get(y, (O, Ho, Wo)), np.zeros((O, Ho, Wo))
+    pad = np.pad(x.astype(np.float64), ((0, 0), (k // 2, k // 2), (k // 2, k // 2)))
+    for oy in range(Ho):
+        for ox in range(Wo):
+            s = pad[:, oy * stride:oy * stride + k, ox * stride:ox * stride + k]
+            want[:, oy, ox] = (w.astype(np.float64) * s[:, None]).sum((0, 2, 3))
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isinf(want).any()
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    f = np.isfinite(want)
+    assert np.abs(got[f] - want[f]).max() <= TOL / 20 * np.abs(want[f]).max()
+
+
 SPLIT_HALVES, SPLIT_MIXED = 2 << 12 | 2 << 16, 1 << 12 | 4 << 16 | 1 << 20
 
 
