@@ -147,7 +147,9 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             if (TURNS) fetching = last ? 0 : fetching + 1;
         }
         const unsigned at = ldsBase + (unsigned)(buf * BUFB + wave * ROWB);
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff[i]), "s"(rIn), "s"(at + 1024u * i) : "memory");
+        unsigned m0;                                    // (put back: the compiler may keep a value there, and takes no clobber for it)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 m0, %0"
+                     : "=&s"(m0) : "v"(voff[i]), "s"(rIn), "s"(at + 1024u * i) : "memory");
         voff[i] += toNext;
     };
 

@@ -563,3 +563,36 @@ def test_bench_refuses_more_than_one_gpu():
     assert r.returncode != 0
     assert "exactly one GPU" in (r.stdout + r.stderr)
     assert not r.stdout.strip().startswith("{")
+
+
+@pytest.fixture(scope="module")
+def split_kernel_code(tmp_path_factory):
+    """{kernel: lines} of the assembly that the build's compiler and flags make of k_winograd_split.hip."""
+    import subprocess
+    from deepracin_amd import build
+    out = str(tmp_path_factory.mktemp("asm") / "split.s")
+    src = os.path.join(build.CSRC, "device", "k_winograd_split.hip")
+    subprocess.run([build.HIPCC] + build.COMMON + build.DEVICE + ["--cuda-device-only", "-S", src, "-o", out], check=True, capture_output=True)
+    kernels, name = {}, None
+    for line in open(out):
+        if line.startswith("_ZN5drhip25winograd_f23_split_kernel") and line.split(";")[0].strip().endswith(":"):
+            name = line.split(":")[0]
+            kernels[name] = []
+        elif name and line.strip().startswith(".section"):
+            name = None
+        elif name:
+            kernels[name].append(line.strip())
+    assert len(kernels) == 6
+    return kernels
+
+
+def test_split_kernel_leaves_m0_as_the_compiler_has_it(split_kernel_code):
+    """The fetches to LDS take their destination from M0, which no inline assembly can declare as overwritten: each puts it back."""
+    for name, lines in split_kernel_code.items():
+        n = 0
+        for k, line in enumerate(lines):
+            if line.startswith("buffer_load") and line.endswith(" lds"):
+                n += 1
+                saved = lines[k - 3].split()[1].rstrip(",")
+                assert lines[k - 3].split()[2] == "m0" and lines[k - 2].startswith("s_mov_b32 m0, ") and lines[k + 1] == "s_mov_b32 m0, " + saved, (name, lines[k - 4:k + 2])
+        assert n >= 15, (name, n)
