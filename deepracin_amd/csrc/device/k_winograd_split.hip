@@ -154,7 +154,11 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     };
 
     // ---- filters ---------------------------------------------------------------------------------------------------
-    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)U, 0, 16 * s.nC * 3 * s.nOB * 1024, kBufferFlags);
+    // The waits for samples count the filter loads issued behind them, so these must stay where they stand: an address whose
+    // origin the compiler does not see keeps it from taking them for loads that no memory clobber concerns.
+    const unsigned short* uHere = U;
+    asm volatile("" : "+s"(uHere));
+    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, 16 * s.nC * 3 * s.nOB * 1024, kBufferFlags);
     unsigned uOb[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) uOb[nt] = (unsigned)((wave * s.nC * s.nOB + min(oBlock * NT + nt, s.nOB - 1)) * 12288);

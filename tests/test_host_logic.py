@@ -596,3 +596,31 @@ def test_split_kernel_leaves_m0_as_the_compiler_has_it(split_kernel_code):
                 saved = lines[k - 3].split()[1].rstrip(",")
                 assert lines[k - 3].split()[2] == "m0" and lines[k - 2].startswith("s_mov_b32 m0, ") and lines[k + 1] == "s_mov_b32 m0, " + saved, (name, lines[k - 4:k + 2])
         assert n >= 15, (name, n)
+
+
+def test_split_kernel_waits_for_its_samples(split_kernel_code):
+    """The split-operand Winograd kernel waits for its fetches to LDS by hand: a wait for all but the last n memory instructions
+    covers a fetch only if at least n were issued behind it.  Counted in the assembly: behind the first step's fetch in
+    front of the loop, and behind a step's fetch once round the loop to the wait of the next step."""
+    for name, lines in split_kernel_code.items():
+        fetches = 6 if "ILi2ELi24E" in name else 5      # of a wave per step
+        blocks, inline = [[]], False                    # of code; F fetch, M other memory instruction, (n) a wait by hand
+        for line in lines:
+            inline = (inline or line == ";;#ASMSTART") and line != ";;#ASMEND"
+            if line.startswith(".LBB"):
+                blocks.append([line.split(":")[0]])
+            elif re.match(r"(buffer|global|flat|scratch)_(load|store|atomic)", line):
+                blocks[-1].append("F" if line.endswith(" lds") else "M")
+            elif inline and line.startswith("s_waitcnt vmcnt"):
+                blocks[-1].append(int(re.search(r"\((\d+)\)", line).group(1)))
+        memory = lambda events: sum(e in ("F", "M") for e in events)
+        fetching = [b for b in blocks if "F" in b]      # straight on through these: the blocks between them only choose addresses
+        body, front = fetching[-1][1:], [e for b in fetching[:-1] for e in b if e in ("F", "M")]
+        assert body.count("F") == fetches and front.count("F") == 2 * fetches, name
+        waits = [k for k, e in enumerate(body) if isinstance(e, int)]
+        last = max(k for k, e in enumerate(body) if e == "F")
+        assert len(waits) == 1 and last < waits[0], name
+        assert memory(body[last + 1:]) + memory(body[:waits[0]]) >= body[waits[0]], name
+        first = [k for k, e in enumerate(front) if e == "F"][fetches - 1]
+        wait = next(e for b in blocks for e in b if isinstance(e, int))
+        assert memory(front[first + 1:]) >= wait > 0, (name, front, wait)
