@@ -314,7 +314,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + l32] = m1 - m2 + m3;
         }
     barrier();
-    constexpr int EO = 8 * KW;                      // output channels finished per pass
+    constexpr int EO = 8 * KW, NP = OB / EO;        // output channels finished per pass, passes
     const int et = tid & 31, eo = tid >> 5;
     const int etg = t0 + et;
     const bool eOk = etg < s.T;
@@ -331,11 +331,14 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             }
         return f32x4{p[0][0] + p[1][0] + p[2][0], p[0][1] + p[1][1] + p[2][1], p[1][0] - p[2][0] + p[3][0], p[1][1] - p[2][1] + p[3][1]};
     };
+    // An infinity, or a value that bf16 rounds to one, has no three-part form and has left NaN behind, and so has the sample beside
+    // the map that is multiplied by zero where it is one of those: what came out as NaN is noted, by pass, for the end.
+    unsigned again = 0;
+    auto note = [&](int q, f32x4 y) { again |= __builtin_isunordered(y[0], y[1]) || __builtin_isunordered(y[2], y[3]) ? 1u << q : 0u; };
     if (nSp > 1) {
         // The splits of a panel add their partial tiles up as those of the fp32 kernel do: each finishes its share of the
         // passes, stores the others' shares and then looks for its own in the slots of the other splits, whose contents
         // say themselves whether they have arrived.  (Slots lie at a workgroup's own place in the grid, 8 apart within a panel.)
-        constexpr int NP = OB / EO;
         const __amdgpu_buffer_rsrc_t rWs = __builtin_amdgcn_make_buffer_rsrc((void*)ws, 0, 0x7ffffff0, kBufferFlags);
         const unsigned group0 = blockIdx.x - (unsigned)(kXcds * split);
         // The whole offset goes in the vector register.  With the region in the scalar one the compiler lets the next vector
@@ -376,8 +379,10 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                 for (int u = 0; u < S; ++u) y += u == split ? own[i] : __builtin_bit_cast(f32x4, part[i][u]);
 #pragma unroll
                 for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, slot_of(u, q), 0, kAuxThrough);
+                note(q, y);
                 if (!ready) {                           // a partner never delivered: say so in the result and in the counter
                     y = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+                    again &= ~(1u << q);
                     atomicAdd(&g_ws_join_timeouts, 1u);
                 }
                 if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2);
@@ -387,13 +392,86 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
         else if (nSp == 3) join(integral_constant<int, 3>{});
         else if (nSp == 4) join(integral_constant<int, 4>{});
         else if constexpr (KW == 1) join(integral_constant<int, 8>{});
-        return;
-    }
+    } else {
+        f32x4 y[NP];                                    // (read in one go: with each store behind its own reads the notes cost the trunk
+        float b[NP];                                    // 4.5 us)
 #pragma unroll
-    for (int q = 0; q < OB / EO; ++q) {
-        const int ol = eo + EO * q;
-        const f32x4 y = tile_of(ol);
-        if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2);
+        for (int q = 0; q < NP; ++q) {
+            y[q] = tile_of(eo + EO * q);
+            b[q] = biasT[eo + EO * q];
+            note(q, y[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+            if (eOk && o0 + eo + EO * q < s.O) wino_finish(out, y[q], b[q], s.flags, o0 + eo + EO * q, plane, W, H, ox, oy, s.vec2);
+    }
+
+    // ---- tiles that came out as NaN --------------------------------------------------------------------------------
+    // Once more in fp32, step by step as the fp32 kernel does it, and with the samples beside the map left out.  Every wave
+    // for itself, tile by tile: its 2 * NP output channels side by side, the lanes left over share the input channels.  (Us, without
+    // and with one NaN and one infinity among the samples: 56x56 512->512 58 / 241, 224x224 64->64 18 / 39; all NaN 68 and 30.)
+    const unsigned long long any = __builtin_amdgcn_ballot_w64(eOk && again != 0u);
+    if (__builtin_expect(any == 0, 1)) return;          // (expected: otherwise what follows lies between instructions that every launch
+                                                        // fetches, and a trunk of 640x480 takes 713 us instead of 702)
+    constexpr int C = 2 * NP, S = 64 / C;               // channels of this wave, lanes per channel
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
+    const __amdgpu_buffer_rsrc_t rAll = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, I * plane * 4, kBufferFlags);
+    const int part = lane / C, pass = lane % C >> 1, ol = 2 * (tid >> 6) + (lane & 1) + EO * pass;
+    const u32x4b* uLane = (const u32x4b*)U + (size_t)min(oBlock * NT + (ol >> 5), s.nOB - 1) * 768 + (ol & 31);
+    for (unsigned bad = (unsigned)any | (unsigned)(any >> 32); bad != 0; bad &= bad - 1) {
+        const int t = __builtin_ctz(bad), ty = fast_div(t0 + t, tilesXd), x0 = 2 * (t0 + t - ty * s.tilesX) - 1, y0 = 2 * ty - 1;
+        // A NaN among the samples at the tile's own four pixels reaches all four outputs, whatever the others are.
+        bool own = false;
+        for (int c = 0; c < I && !own; c += 64) {
+            const float* at = in + (size_t)min(c + lane, I - 1) * plane + x0 + 1;
+            const int right = x0 + 2 < W ? 1 : 0, r0 = (y0 + 1) * W, r1 = min(y0 + 2, H - 1) * W;
+            own = __builtin_amdgcn_ballot_w64(__builtin_isunordered(at[r0], at[r0 + right]) || __builtin_isunordered(at[r1], at[r1 + right])) != 0;
+        }
+        if (own) continue;
+        const int shift = x0 < 0 ? 1 : 0;               // (the first column's tiles load from column 0)
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma clang loop unroll(disable)
+        for (int r = 0; r < 4; ++r) {                   // a row of the transform
+            const int ya = y0 + r, yb = y0 + (r < 2 ? 2 : 1);
+            const float sign = r == 1 ? 1.0f : -1.0f;
+            float m[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma clang loop unroll(disable)
+            for (int c8 = part; c8 < 2 * s.nC; c8 += S) {       // eight channels, half of a chunk
+                const u32x4b* u = uLane + (size_t)(r * s.nC + (c8 >> 1)) * s.nOB * 768 + 32 * (c8 & 1);
+                float v[8][4];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    auto row = [&](int iy) {
+                        const unsigned at = iy >= 0 && iy < H ? 4u * (unsigned)((8 * c8 + j) * plane + iy * W + x0 + shift) : kOutOfRange;
+                        const f32x4 e = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rAll, (int)at, 0, 0));
+                        return shift ? f32x4{0.f, e[0], e[1], e[2]} : e;
+                    };
+                    const f32x4 a = row(ya), b = row(yb);
+                    float d[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) d[c] = x0 + c < W ? fmaf(sign, b[c], a[c]) : 0.0f;
+                    v[j][0] = d[0] - d[2]; v[j][1] = d[1] + d[2]; v[j][2] = d[2] - d[1]; v[j][3] = d[3] - d[1];
+                }
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const u32x4b hi = u[3 * x * 64], mid = u[(3 * x + 1) * 64], lo = u[(3 * x + 2) * 64];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        auto of = [&](u32x4b q) { return __builtin_bit_cast(float, j & 1 ? q[j / 2] & 0xffff0000u : q[j / 2] << 16); };
+                        m[x] = fmaf(of(lo) + of(mid) + of(hi), v[j][x], m[x]);
+                    }
+                }
+            }
+            const float p0 = m[0] + m[1] + m[2], p1 = m[1] - m[2] + m[3], back = r == 2 ? -1.0f : 1.0f;
+            if (r < 3) { y[0] += p0; y[1] += p1; }
+            if (r > 0) { y[2] = fmaf(back, p0, y[2]); y[3] = fmaf(back, p1, y[3]); }
+        }
+#pragma unroll
+        for (int k = C; k < 64; k *= 2)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) y[c] += __shfl_xor(y[c], k);
+        const unsigned noted = (unsigned)__shfl((int)again, 32 * (lane & 1) + t);
+        if (part == 0 && (noted >> pass & 1u) && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, x0 + 1, y0 + 1, s.vec2);
     }
 }
 

@@ -295,6 +295,65 @@ def test_winograd_split_operands(lib, dev, oracle, variant, W, H, I, O):
     assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, xd, 10, 4, I, O, 0, variant, ws, None) == -1      # more rows of tiles in a panel than LDS has room for
 
 
+def winograd_replay(x, w):
+    """Winograd F(2x2,3x3) step by step in float64: what fp32 arithmetic makes of infinities and NaN, tile by tile."""
+    (I, H, W), O = x.shape, w.shape[1]
+    th, tw = -(-H // 2), -(-W // 2)
+    pad = np.zeros((I, 2 * th + 2, 2 * tw + 2))
+    pad[:, 1:H + 1, 1:W + 1] = x
+    d = np.stack([[pad[:, r:r + 2 * th:2, c:c + 2 * tw:2] for c in range(4)] for r in range(4)])       # [4][4][I][th][tw]
+    rows = lambda a: np.stack([a[0] - a[2], a[1] + a[2], a[2] - a[1], a[3] - a[1]])
+    G = np.array([[1, 0, 0], [.5, .5, .5], [.5, -.5, .5], [0, 0, 1]])
+    u = np.einsum("ri,coij,sj->rsco", G, w.astype(np.float64), G)
+    y = np.zeros((O, 2 * th, 2 * tw))
+    with np.errstate(invalid="ignore"):
+        v = np.swapaxes(rows(np.swapaxes(rows(d), 0, 1)), 0, 1)
+        m = np.stack([[sum(u[r, s, c][:, None, None] * v[r, s, c] for c in range(I)) for s in range(4)] for r in range(4)])
+        half = np.stack([m[0] + m[1] + m[2], m[1] - m[2] + m[3]])                                       # [2][4][O][th][tw]
+        for a in range(2):
+            y[:, a::2, 0::2] = half[a, 0] + half[a, 1] + half[a, 2]
+            y[:, a::2, 1::2] = half[a, 1] - half[a, 2] + half[a, 3]
+    return y[:, :H, :W]
+
+
+def assert_same_extremes(got, want):
+    """NaN where NaN is wanted, the same infinities, the finite rest within a twentieth of the layer bar of what is near it in size."""
+    assert np.array_equal(np.isnan(got), np.isnan(want)), np.argwhere(np.isnan(got) != np.isnan(want))[:5]
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    for part in (np.abs(want) < 1e6, (np.abs(want) >= 1e6) & np.isfinite(want)):
+        if part.any():
+            assert np.abs(got[part] - want[part]).max() <= TOL / 20 * np.abs(want[part]).max()
+
+
+def split_winograd(lib, dev, x, w, variant, flags=0):
+    (I, H, W), O = x.shape, w.shape[1]
+    F = dev.empty(lib.drhip_conv3x3_winograd_split_filter_floats(I, O))
+    ok(lib, lib.drhip_winograd_split_filter_transform_f32(dev.put(w), F, I, O, None))
+    n, ws = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant), None
+    if n:
+        ws = dev.empty(n)
+        ok(lib, lib.drhip_conv3x3_winograd_workspace_prepare_f32(ws, n, None))
+    y = dev.empty(O * H * W)
+    go = lambda xd: ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, None, y, W, H, I, O, flags, variant, ws, None))
+    go(dev.put(x))
+    return dev.get(y, (O, H, W)), go
+
+
+@pytest.mark.parametrize("variant", [0x100, 0x101, 0x100 | SPLIT_HALVES, 0x101 | 3 << 12 | 3 << 16])
+@pytest.mark.parametrize("W,H,I,O", [(33, 9, 70, 70), (40, 10, 100, 33)])
+def test_winograd_split_keeps_infinities(lib, dev, variant, W, H, I, O):
+    """Infinite samples, NaN and samples that bf16 rounds to infinity come out as fp32 Winograd has them, at the edges of the
+    map too, where the kernel's loads reach into the next row, and with the input channels in pieces."""
+    x, w = rnd(I, H, W), rnd(I, O, 3, 3, scale=0.02)
+    x[1, 4, 12], x[0, 0, 0], x[I - 1, H - 1, W - 1], x[I - 2, 3, 0], x[2, 5, W - 1] = np.inf, -np.inf, np.inf, -np.inf, np.inf
+    x[3, 2, 26], x[4, 2, 27], x[2, 6, 20] = np.inf, -np.inf, np.nan
+    x[5, 7, 5] = x[I - 1, 1, 22] = 3.399e38
+    got, _ = split_winograd(lib, dev, x, w, variant)
+    want = winograd_replay(x, w)
+    assert np.isinf(want).sum() > O and np.isnan(want).any()
+    assert_same_extremes(got, want)
+
+
 @pytest.mark.parametrize("W,H,I,O", [(257, 129, 113, 65), (21, 48, 400, 512), (33, 31, 256, 512)])
 def test_winograd_split_picked(lib, dev, oracle, W, H, I, O):
     """The variant that the rule picks: a round of whole panels and halves behind it, narrow and wide maps in pieces, panels
