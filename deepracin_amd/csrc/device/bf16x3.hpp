@@ -45,9 +45,19 @@ __device__ inline f32x16b mfma_bf16(u32x4b a, u32x4b b, f32x16b c) {
 constexpr int kProdA[6] = {2, 1, 0, 1, 0, 0};
 constexpr int kProdB[6] = {0, 1, 2, 0, 1, 0};
 
-// One element's parts as 16-bit patterns (filter banks, written once when a layer is prepared).
+// One element's parts as 16-bit patterns (filter banks, written once when a layer is prepared).  Here there is time for every
+// value: an infinity or NaN is its own first part, and a finite value that bf16 rounds to infinity is cut off instead of rounded,
+// so that the sum of the parts is the value itself.
 __device__ inline void split_one(float x, unsigned short (&part)[3]) {
-    const Bf16Pair3 p = split_pair(x, 0.0f);
+    const unsigned bits = __float_as_uint(x);
+    Bf16Pair3 p = split_pair(x, 0.0f);
+    if ((p.hi & 0x7fffu) >= 0x7f80u) {
+        const bool finite = (bits & 0x7fffffffu) < 0x7f800000u;
+        const Bf16Pair3 rest = split_pair(finite ? x - __uint_as_float(bits & 0xffff0000u) : 0.0f, 0.0f);
+        if (finite) p.hi = bits >> 16;                 // (a NaN keeps what the conversion made of it)
+        p.mid = rest.hi;
+        p.lo = rest.mid;
+    }
     part[0] = (unsigned short)p.hi;
     part[1] = (unsigned short)p.mid;
     part[2] = (unsigned short)p.lo;

@@ -66,7 +66,7 @@ conv_bank_layout_kernel(const float* __restrict__ w, unsigned short* __restrict_
 }
 
 // One output in fp32, without the bias: an infinite sample (or one that bf16 rounds to infinity) has no three-part form and
-// leaves NaN behind, so an output that came out as NaN is worked out again from the samples and the filters put together.
+// leaves NaN behind, and so do the parts of ordinary samples times an infinite weight, so an output that came out as NaN is worked out again from the samples and the filters put together.
 template <int CP>
 __device__ __forceinline__ float conv_bank_exact(const float* in, const unsigned short* F, const BankShape& s, int o, int x, int y) {
     const int kh = s.steps / s.spr;

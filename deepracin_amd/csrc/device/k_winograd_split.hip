@@ -72,10 +72,11 @@ wino_split_filter_kernel(const float* __restrict__ w, unsigned short* __restrict
         u32x4b part[3];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const Bf16Pair3 s = split_pair(u[2 * p][x], u[2 * p + 1][x]);
-            part[0][p] = s.hi;
-            part[1][p] = s.mid;
-            part[2][p] = s.lo;
+            unsigned short a[3], b[3];
+            split_one(u[2 * p][x], a);
+            split_one(u[2 * p + 1][x], b);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) part[q][p] = a[q] | (unsigned)b[q] << 16;
         }
 #pragma unroll
         for (int q = 0; q < 3; ++q) d[(x * 3 + q) * 64] = part[q];

@@ -303,10 +303,10 @@ def winograd_replay(x, w):
     pad[:, 1:H + 1, 1:W + 1] = x
     d = np.stack([[pad[:, r:r + 2 * th:2, c:c + 2 * tw:2] for c in range(4)] for r in range(4)])       # [4][4][I][th][tw]
     rows = lambda a: np.stack([a[0] - a[2], a[1] + a[2], a[2] - a[1], a[3] - a[1]])
-    G = np.array([[1, 0, 0], [.5, .5, .5], [.5, -.5, .5], [0, 0, 1]])
-    u = np.einsum("ri,coij,sj->rsco", G, w.astype(np.float64), G)
+    taps = lambda g: np.stack([g[0], .5 * g[0] + .5 * g[1] + .5 * g[2], .5 * g[0] - .5 * g[1] + .5 * g[2], g[2]])
     y = np.zeros((O, 2 * th, 2 * tw))
     with np.errstate(invalid="ignore"):
+        u = np.swapaxes(taps(np.swapaxes(taps(w.astype(np.float64).transpose(2, 3, 0, 1)), 0, 1)), 0, 1)    # [4][4][I][O]
         v = np.swapaxes(rows(np.swapaxes(rows(d), 0, 1)), 0, 1)
         m = np.stack([[sum(u[r, s, c][:, None, None] * v[r, s, c] for c in range(I)) for s in range(4)] for r in range(4)])
         half = np.stack([m[0] + m[1] + m[2], m[1] - m[2] + m[3]])                                       # [2][4][O][th][tw]
@@ -316,11 +316,13 @@ def winograd_replay(x, w):
     return y[:, :H, :W]
 
 
-def assert_same_extremes(got, want):
-    """NaN where NaN is wanted, the same infinities, the finite rest within a twentieth of the layer bar of what is near it in size."""
+def assert_same_extremes(got, want, by_channel=False):
+    """NaN where NaN is wanted, the same infinities, the finite rest within a twentieth of the layer bar: of the ordinary and of the huge
+    outputs, or of each output channel's largest."""
     assert np.array_equal(np.isnan(got), np.isnan(want)), np.argwhere(np.isnan(got) != np.isnan(want))[:5]
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
-    for part in (np.abs(want) < 1e6, (np.abs(want) >= 1e6) & np.isfinite(want)):
+    finite = np.isfinite(want)
+    for part in finite & (np.arange(len(want))[:, None, None, None] == np.arange(len(want))[:, None, None]) if by_channel else (finite & (np.abs(want) < 1e6), finite & (np.abs(want) >= 1e6)):
         if part.any():
             assert np.abs(got[part] - want[part]).max() <= TOL / 20 * np.abs(want[part]).max()
 
@@ -351,6 +353,45 @@ def test_winograd_split_keeps_infinities(lib, dev, variant, W, H, I, O):
     got, _ = split_winograd(lib, dev, x, w, variant)
     want = winograd_replay(x, w)
     assert np.isinf(want).sum() > O and np.isnan(want).any()
+    assert_same_extremes(got, want)
+
+
+@pytest.mark.parametrize("variant", [0x100, 0x101 | SPLIT_HALVES])
+@pytest.mark.parametrize("infinite", [True, False])
+def test_winograd_split_keeps_extreme_weights(lib, dev, variant, infinite):
+    """Filters with an infinite or NaN weight, and finite ones that bf16 rounds to infinity, as fp32 Winograd has them."""
+    W, H, I, O = 35, 7, 40, 40
+    x, w = rnd(I, H, W, scale=0.01), rnd(I, O, 3, 3)
+    x[:, 3:5, 4:6] = 0
+    if infinite:
+        w[1, 3, 0, 0], w[I - 1, 7, 2, 2], w[0, 8, 0, 2], w[1, 8, 0, 0], w[0, 39, 1, 2] = np.inf, -np.inf, np.inf, -np.inf, np.nan
+    w[1, 11, 0, 0], w[I - 1, 33, 2, 2] = 3.399e38, -np.finfo(np.float32).max
+    got, _ = split_winograd(lib, dev, x, w, variant)
+    # (the transforms mix the taps of a filter: the rounding of the largest tap is in every output of its channel)
+    assert_same_extremes(got, winograd_replay(x, w), by_channel=True)
+
+
+@pytest.mark.parametrize("I,k,stride,infinite", [(3, 7, 2, True), (4, 5, 1, True), (20, 5, 1, True), (17, 3, 3, True), (3, 7, 2, False), (20, 5, 1, False)])
+def test_conv_bank_keeps_extreme_weights(lib, dev, I, k, stride, infinite):
+    """Infinite weights, and finite ones that bf16 rounds to infinity, are what they are in fp32."""
+    W, H, O = 23, 19, 40
+    x, w = np.abs(rnd(I, H, W, scale=0.01)), rnd(I, O, k, k)
+    x[:, 3, 4] = 0
+    if infinite:
+        w[1, 3, 1, 1], w[I - 1, 7, 0, 0], w[0, 8, 0, 0], w[1, 8, 1, 1], w[0, 39, 1, 2] = np.inf, -np.inf, np.inf, -np.inf, np.nan
+    w[1, 11, 1, 1], w[I - 1, 33, k - 1, 0] = 3.399e38, -np.finfo(np.float32).max
+    F = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k))
+    ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
+    Wo, Ho = W // stride, H // stride
+    y = dev.empty(O * Ho * Wo)
+    ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, None, y, W, H, I, O, k, k, stride, stride, 0, 0, None))
+    got, want = dev.get(y, (O, Ho, Wo)), np.zeros((O, Ho, Wo))
+    for oy in range(Ho):
+        for ox in range(Wo):
+            ys, xs = np.arange(k) + oy * stride - k // 2, np.arange(k) + ox * stride - k // 2
+            j, i = (ys >= 0) & (ys < H), (xs >= 0) & (xs < W)
+            with np.errstate(invalid="ignore"):         # (a weight over the edge of the map is not multiplied by anything)
+                want[:, oy, ox] = (w.astype(np.float64)[:, :, j][:, :, :, i] * x[:, ys[j]][:, :, xs[i]][:, None]).sum((0, 2, 3))
     assert_same_extremes(got, want)
 
 
