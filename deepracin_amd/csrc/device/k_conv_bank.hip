@@ -65,29 +65,6 @@ conv_bank_layout_kernel(const float* __restrict__ w, unsigned short* __restrict_
     for (int q = 0; q < 3; ++q) F[((((size_t)chunk * steps + step) * 3 + q) * oBlocks + ob) * 512 + lane * 8 + e] = part[q];
 }
 
-// One output in fp32, without the bias: an infinite sample (or one that bf16 rounds to infinity) has no three-part form and
-// leaves NaN behind, and so do the parts of ordinary samples times an infinite weight, so an output that came out as NaN is worked out again from the samples and the filters put together.
-template <int CP>
-__device__ __forceinline__ float conv_bank_exact(const float* in, const unsigned short* F, const BankShape& s, int o, int x, int y) {
-    const int kh = s.steps / s.spr;
-    float v = 0.0f;
-#pragma clang loop unroll(disable)
-    for (int c = 0; c < s.I; ++c)
-#pragma clang loop unroll(disable)
-        for (int j = 0; j < kh; ++j)
-#pragma clang loop unroll(disable)
-            for (int i = 0; i < s.kw; ++i) {
-                const int ix = x * s.sx - s.padX + i, iy = y * s.sy - s.padY + j;
-                if (ix < 0 || ix >= s.W || iy < 0 || iy >= s.H) continue;
-                const int chunk = CP == 16 ? c >> 4 : 0, k = CP == 16 ? c & 15 : 4 * (i & 3) + c, step = j * s.spr + (CP == 16 ? i : i >> 2);
-                float w = 0.0f;
-                for (int q = 2; q >= 0; --q)
-                    w += __uint_as_float((unsigned)F[((((size_t)chunk * s.steps + step) * 3 + q) * s.oBlocks + (o >> 5)) * 512 + ((k >> 3) * 32 + (o & 31)) * 8 + (k & 7)] << 16);
-                v = fmaf(w, in[((size_t)c * s.H + iy) * s.W + ix], v);
-            }
-    return v;
-}
-
 // PF: staging rounds (512 units each) of the next 16 channels that are kept in registers.
 template <int CP, int MT, int WO, int WK, int PF>
 __global__ void __launch_bounds__(kBankThreads)
@@ -280,19 +257,73 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         for (int r = 0; r < 16; ++r)
             part[((wk * 32 * WO + 32 * wo + 8 * (r / 4) + 4 * half + r % 4) * MT + m) * kPitch + l32] = acc[m][0][r];
     __syncthreads();
+    unsigned again = 0;                                 // turns whose output came out as NaN
 #pragma unroll
     for (int n = 0; n < 2 * WO * MT; ++n) {             // 512 lanes: 16 (channel, block) pairs of 32 pixels a turn
         const int pair = 16 * n + (tid >> 5), m = pair % MT, oc = pair / MT, pl = tid & 31;
         float v = 0.0f;
 #pragma unroll
         for (int k = 0; k < WK; ++k) v += part[((k * 32 * WO + oc) * MT + m) * kPitch + pl];
+        again |= v != v ? 1u << n : 0u;
         const int o = blockIdx.z * (32 * WO) + oc;
         const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
-        const bool ok = o < s.O && x < s.Wo && y < s.Ho;
-        if (ok && v != v) v = conv_bank_exact<CP>(in, F, s, o, x, y);
         v += biasT[oc];
         if (s.relu) v = fmaxf(v, 0.0f);
-        if (ok) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
+        if (o < s.O && x < s.Wo && y < s.Ho) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
+    }
+
+    // ---- outputs that came out as NaN ------------------------------------------------------------------------------
+    // An infinite sample (or one that bf16 rounds to infinity) has no three-part form and leaves NaN behind, and so do the parts of
+    // ordinary samples times an infinite weight: such outputs are worked out again in fp32 from the samples and the filters put
+    // together.  Every wave for itself, pixel by pixel: its output channels side by side, the lanes left over share the k-steps.  A
+    // pixel with a NaN in its window stays one.  (56x56 64->96 5x5, us: 12.6, with a NaN and an infinity among the samples 346, all NaN
+    // 81; by one lane each the second took 2000.)
+    const unsigned long long any = __builtin_amdgcn_ballot_w64(again != 0u);
+    if (__builtin_expect(any == 0, 1)) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
+    constexpr int CH = 4 * WO;                          // channels of this wave
+    const int ci = lane % CH, oc = MT == 1 ? 16 * (ci >> 1) + 2 * wave + (ci & 1) : 8 * ci + wave, o = blockIdx.z * (32 * WO) + oc;
+    const int kh = s.steps / s.spr;
+    const unsigned fAgain = (unsigned)(min(o >> 5, s.oBlocks - 1) * 1024 + (o & 31) * 16);
+    for (unsigned long long bad = MT == 1 ? (any | any >> 32) & 0xffffffffull : any; bad != 0; bad &= bad - 1) {
+        const int px = __builtin_ctzll(bad), pl = px & 31, m = px >> 5;
+        const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
+        if (x >= s.Wo || y >= s.Ho) continue;
+        const int left = x * s.sx - s.padX, top = y * s.sy - s.padY;
+        bool stays = false;
+        for (int j = 0; j < kh && !stays; ++j) {
+            const float* row = in + (size_t)min(max(top + j, 0), s.H - 1) * s.W;        // (a row beside the map stands for one that is in the window)
+            bool nan = false;
+            for (int c = lane; c < s.I; c += 64)
+                for (int i = 0; i < s.kw; ++i) {
+                    const float v = row[(size_t)c * plane + min(max(left + i, 0), s.W - 1)];
+                    nan = nan || v != v;
+                }
+            stays = __builtin_amdgcn_ballot_w64(nan) != 0;
+        }
+        if (stays) continue;
+        float v = 0.0f;
+        for (int chunk = 0; chunk < s.nChunks; ++chunk)
+            for (int u = lane / CH; u < 2 * s.steps; u += 64 / CH) {            // half a k-step: eight values of k
+                const int step = u >> 1, h = u & 1, j = (int)(((unsigned)step * s.sprMul) >> 16), i0 = step - j * s.spr;
+                const unsigned f = fAgain + (unsigned)((chunk * s.steps + step) * 3 * s.oBlocks * 1024 + 512 * h), partF = (unsigned)s.oBlocks * 1024u;
+                const u32x4b hi = bank_load4(rF, f, 0), mid = bank_load4(rF, f + partF, 0), lo = bank_load4(rF, f + 2 * partF, 0);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int c = CP == 16 ? 16 * chunk + 8 * h + e : e & 3, i = CP == 16 ? i0 : 4 * i0 + 2 * h + (e >> 2);
+                    const int ix = left + i, iy = top + j;
+                    const bool ok = c < s.I && i < s.kw && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
+                    const float sample = in[ok ? (size_t)c * plane + iy * s.W + ix : 0];
+                    auto of = [&](u32x4b q) { return __builtin_bit_cast(float, e & 1 ? q[e / 2] & 0xffff0000u : q[e / 2] << 16); };
+                    v = ok ? fmaf(of(lo) + of(mid) + of(hi), sample, v) : v;
+                }
+            }
+#pragma unroll
+        for (int k = CH; k < 64; k *= 2) v += __shfl_xor(v, k);
+        const unsigned noted = (unsigned)__shfl((int)again, MT == 1 ? 32 * (ci & 1) + pl : px) >> (MT == 1 ? ci >> 1 : ci);
+        v += biasT[oc];
+        if (s.relu) v = fmaxf(v, 0.0f);
+        if (lane < CH && (noted & 1u) && o < s.O) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
     }
 }
 

@@ -395,6 +395,37 @@ def test_conv_bank_keeps_extreme_weights(lib, dev, I, k, stride, infinite):
     assert_same_extremes(got, want)
 
 
+def kernel_us(lib, go, arg, repeats=5):
+    """Shortest execution time of the kernels that go(arg) launches."""
+    best = 1e30
+    for _ in range(repeats):
+        ms, count = (ctypes.c_float * 64)(), ctypes.c_int()
+        ok(lib, lib.drhip_timing_begin())
+        go(arg)
+        ok(lib, lib.drhip_timing_end(ms, 64, ctypes.byref(count)))
+        assert count.value
+        best = min(best, 1e3 * sum(ms[:count.value]))
+    return best
+
+
+def test_a_sample_that_is_nan_does_not_hold_a_launch_up(lib, dev):
+    """What the split-operand kernels do about outputs that came out as NaN is work for whole waves, and none where a sample is NaN: such
+    a launch takes a multiple of its time, not milliseconds."""
+    W, H, I, O = 56, 56, 64, 96
+    x, w = rnd(I, H, W), rnd(I, O, 5, 5, scale=0.05)
+    bad = x.copy()
+    bad[10, 20, 30] = np.nan
+    bad[11, 40, 9] = np.inf
+    F, y = dev.empty(lib.drhip_conv_bank_floats(I, O, 5, 5)), dev.empty(O * H * W)
+    ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, 5, 5, None))
+    bank = lambda xd: ok(lib, lib.drhip_conv_bank_f32(xd, F, None, y, W, H, I, O, 5, 5, 1, 1, 0, 0, None))
+    _, wino = split_winograd(lib, dev, x, rnd(I, O, 3, 3, scale=0.05), 0x101)
+    for what, go in (("bank", bank), ("winograd", wino)):
+        good, worse, none = [kernel_us(lib, go, dev.put(a)) for a in (x, bad, np.full_like(x, np.nan))]
+        print("%s: %.1f us, with a NaN and an infinity %.1f us, all NaN %.1f us" % (what, good, worse, none))
+        assert worse <= 40 * good and none <= 20 * good     # (by one lane each: 160 times)
+
+
 @pytest.mark.parametrize("W,H,I,O", [(257, 129, 113, 65), (21, 48, 400, 512), (33, 31, 256, 512)])
 def test_winograd_split_picked(lib, dev, oracle, W, H, I, O):
     """The variant that the rule picks: a round of whole panels and halves behind it, narrow and wide maps in pieces, panels
