@@ -35,6 +35,8 @@ inline int launched(const char* kernel) { return check(hipGetLastError(), kernel
 inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 
 constexpr int kWave = 64;   // CDNA wavefront width
+constexpr unsigned kBufferFlags = 0x00020000u;      // dword 3 of a gfx9 raw buffer resource (32-bit data format)
+constexpr unsigned kOutOfRange = 0x80000000u;       // byte offset no resource of at most 2 GiB contains
 
 // Per-thread record of kernel execution times (drhip_timing_begin / drhip_timing_end).  While it is
 // on, every launch carries its own start and stop event (hipExtLaunchKernelGGL attaches them to the

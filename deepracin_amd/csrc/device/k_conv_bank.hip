@@ -25,8 +25,6 @@
 
 namespace drhip {
 
-constexpr unsigned kBankBufferFlags = 0x00020000u;      // dword 3 of a gfx9 raw buffer resource (32-bit data format)
-constexpr unsigned kBankOutOfRange = 0x80000000u;       // byte offset no resource of at most 2 GiB contains
 constexpr int kBankThreads = 512;                       // eight waves: two per SIMD, one reads and counts while the other multiplies
 
 struct BankShape {                                      // everything but the pointers; by value to the kernel
@@ -101,13 +99,13 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         const int py = fast_div(q, pwd), px = q - py * s.pw;
         const int ix = px0 + px, iy = py0 + py;
         const bool ok = u < units && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
-        off = ok ? 4u * (unsigned)(grp * 8 * plane + iy * s.W + ix) : kBankOutOfRange;
+        off = ok ? 4u * (unsigned)(grp * 8 * plane + iy * s.W + ix) : kOutOfRange;
     };
     auto load_unit = [&](float (&v)[kUC], unsigned off, int chunk) {
 #pragma unroll
         for (int q = 0; q < kUC; ++q) {                 // (channels past the last one: a resource that ends in front of them)
             const int c = chunk * 16 + q, left = max(s.I - c, 0);
-            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(in + (size_t)min(c, s.I) * plane), 0, left * plane * 4, kBankBufferFlags);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(in + (size_t)min(c, s.I) * plane), 0, left * plane * 4, kBufferFlags);
             v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
         }
     };
@@ -130,8 +128,8 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
 
     // ---- filters: the steps of this wave, wk, wk + WK, ..., -------------------------------------
     const int bankBytes = s.nChunks * s.steps * 3 * s.oBlocks * 1024;
-    const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, bankBytes, kBankBufferFlags);
-    const unsigned fLane = ob < s.oBlocks ? (unsigned)(ob * 1024 + lane * 16) : kBankOutOfRange;    // (a wave without channels multiplies zeros)
+    const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, bankBytes, kBufferFlags);
+    const unsigned fLane = ob < s.oBlocks ? (unsigned)(ob * 1024 + lane * 16) : kOutOfRange;    // (a wave without channels multiplies zeros)
     auto load_filters = [&](u32x4b (&f)[3], int chunk, int step) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) f[q] = bank_load4(rF, fLane, (unsigned)(((chunk * s.steps + step) * 3 + q) * s.oBlocks) * 1024u);

@@ -66,9 +66,7 @@ constexpr int kAuxThrough = 1 | 16;                 // cache policy of a buffer 
 constexpr int kAuxDeviceVolatile = 16 | (int)0x80000000u;   // sc1 (device scope: not served from this CU's vector cache), reloaded every time
 int ws_join_timeouts(unsigned* count);              // of the split-operand kernel
 
-constexpr unsigned kBufferFlags = 0x00020000u;      // dword 3 of a gfx9 raw buffer resource (32-bit data format)
 constexpr int kEpiRelu = DRHIP_EPILOGUE_RELU, kEpiMaxPool2 = DRHIP_EPILOGUE_MAXPOOL2;   // bits of the `relu` argument
-constexpr unsigned kOutOfRange = 0x80000000u;       // byte offset no resource of at most 2 GiB contains
 
 // Bias, ReLU and store of one 2x2 tile of channel o, or of its maximum (a following 2x2/2 max pooling; W and H even).
 __device__ inline void wino_finish(float* out, f32x4 y, float bias, int flags, int o, int plane, int W, int H, int ox, int oy, int vec2) {

@@ -61,12 +61,14 @@ gchar* conv_serialize(dR_Node* node, gchar* params[], gint* numParams, gfloat* v
 gchar* conv_print(dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     static const char* acts[] = { "Linear", "ReLU", "Sigmoid", "Tan" };
-    static const char* algos[] = { "direct", "Winograd F(2x2,3x3) MFMA", "1x1 MFMA GEMM" };
+    // (variant numbers are each kernel's own)
+    const char* kernel = c->algo == drConv1x1Gemm ? "1x1 MFMA GEMM"
+                       : c->algo == drConvWinograd ? (c->drWinoSplit ? "Winograd F(2x2,3x3) split-operand bf16 MFMA" : "Winograd F(2x2,3x3) MFMA")
+                       : c->drSplitBank ? "direct, split-operand bf16 MFMA" : c->drDirectBank ? "direct MFMA" : "direct";
     return fmt_dup("Conv2d Layer: %d\n Filter dimensions: %dx%d\n Input channels: %d\n Output channels: %d\n"
                    " Activation: %s\n Stride: %d, %d, %d, %d\n Use bias: %s\n Kernel: %s (variant %d)\n",
                    node->layerID, c->shape.s0, c->shape.s1, c->shape.s2, c->shape.s3, acts[c->activation & 3],
-                   c->stride.s0, c->stride.s1, c->stride.s2, c->stride.s3, c->useBias ? "Yes" : "No",
-                   algos[c->algo], c->variant);
+                   c->stride.s0, c->stride.s1, c->stride.s2, c->stride.s3, c->useBias ? "Yes" : "No", kernel, c->variant);
 }
 
 // A Winograd layer with O output channels: the split-operand kernel where it is the faster one, the fp32 kernel otherwise.

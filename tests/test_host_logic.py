@@ -507,6 +507,19 @@ def test_layers_beyond_the_packed_argument_fields_take_the_general_kernel(lib):
                 assert plan[0][0] != plan[1][0]                  # the convolution keeps a tensor of its own
 
 
+@pytest.mark.parametrize("W,H,I,O,k,stride,kernel", [
+    (112, 112, 128, 128, 3, 1, "Winograd F(2x2,3x3) split-operand bf16 MFMA"), (14, 14, 16, 64, 3, 1, "Winograd F(2x2,3x3) MFMA"),
+    (56, 56, 64, 96, 5, 1, "direct, split-operand bf16 MFMA"), (56, 56, 64, 96, 3, 2, "direct MFMA"), (33, 31, 3, 9, 3, 2, "direct"), (9, 9, 8, 8, 1, 1, "1x1 MFMA GEMM")])
+def test_a_layer_says_which_kernel_it_runs(lib, W, H, I, O, k, stride, kernel):
+    with dr.Environment() as env:
+        g = env.create_graph()
+        x = dr.feed_node(g, [H, W, I])
+        c = dr.Conv2d_raw(x, np.ones((I, O, k, k), np.float32), None, (stride, stride), "relu")
+        dr.mark_as_output(c)
+        assert lib.dR_propagateShapesAndSchedule(g.ptr) == 1
+        assert re.fullmatch(" Kernel: %s \\(variant \\d+\\)" % re.escape(kernel), _kernel_line(c)), _kernel_line(c)
+
+
 def test_layers_beyond_32_bit_byte_offsets_take_the_general_kernels(lib):
     """Every dimension fits the 16-bit argument fields, but the input holds 2^29 elements or more: the matrix-core
     3x3 kernels and the pooling-on-load 1x1 kernel (32-bit byte offsets) are not scheduled for such a layer."""
