@@ -10,6 +10,11 @@
 // 16x32 with operands in [-0.5, 0.5): 3.3e-8 relative against 7.3e-8 for a chain of fp32 FMAs; 2.34 PFLOP/s of matrix
 // instructions sustained, and up to six vector instructions per matrix instruction ride along for nothing, where
 // an fp32 MFMA and a vector instruction exclude each other.)
+//
+// bf16 ends at 2^-133, so that below 2^-110 the third part would lose bits that fp32 has.  Both operands are therefore multiplied by
+// 2^16 when they are split, which puts the last bit of the smallest fp32 number there, and results by 2^-32.  What that takes
+// out of range at the other end (operands above 2^111, results above 2^95) comes out as infinity or NaN, which the kernels that
+// use this look for and work out again in fp32.
 #pragma once
 
 #include "drhip_common.hpp"
@@ -22,6 +27,8 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4b __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2b __attribute__((ext_vector_type(2)));
+
+constexpr float kSplitScale = 0x1p16f, kSplitUnscaleOne = 0x1p-16f, kSplitUnscale = 0x1p-32f;
 
 struct Bf16Pair3 { unsigned hi, mid, lo; };         // two values, each as three parts, packed by part
 
@@ -45,22 +52,19 @@ __device__ inline f32x16b mfma_bf16(u32x4b a, u32x4b b, f32x16b c) {
 constexpr int kProdA[6] = {2, 1, 0, 1, 0, 0};
 constexpr int kProdB[6] = {0, 1, 2, 0, 1, 0};
 
-// One element's parts as 16-bit patterns (filter banks, written once when a layer is prepared).  Here there is time for every
-// value: an infinity or NaN is its own first part, and a finite value that bf16 rounds to infinity is cut off instead of rounded,
-// so that the sum of the parts is the value itself.
+// One element's parts as 16-bit patterns (filter banks, written once when a layer is prepared).  What has no parts, an infinity,
+// a NaN or a value above 2^111, gets an infinite first part, so that nothing finite comes of it, and its own 32 bits as the others.
 __device__ inline void split_one(float x, unsigned short (&part)[3]) {
     const unsigned bits = __float_as_uint(x);
-    Bf16Pair3 p = split_pair(x, 0.0f);
-    if ((p.hi & 0x7fffu) >= 0x7f80u) {
-        const bool finite = (bits & 0x7fffffffu) < 0x7f800000u;
-        const Bf16Pair3 rest = split_pair(finite ? x - __uint_as_float(bits & 0xffff0000u) : 0.0f, 0.0f);
-        if (finite) p.hi = bits >> 16;                 // (a NaN keeps what the conversion made of it)
-        p.mid = rest.hi;
-        p.lo = rest.mid;
-    }
-    part[0] = (unsigned short)p.hi;
-    part[1] = (unsigned short)p.mid;
-    part[2] = (unsigned short)p.lo;
+    const bool fits = fabsf(x) < 0x1p111f;
+    const Bf16Pair3 p = split_pair(fits ? kSplitScale * x : 0.0f, 0.0f);
+    part[0] = (unsigned short)(fits ? p.hi : 0x7f80u);
+    part[1] = (unsigned short)(fits ? p.mid : bits >> 16);
+    part[2] = (unsigned short)(fits ? p.lo : bits);
+}
+__device__ inline float whole(unsigned hi, unsigned mid, unsigned lo) {
+    if (hi == 0x7f80u) return __uint_as_float(mid << 16 | lo);
+    return kSplitUnscaleOne * (__uint_as_float(lo << 16) + __uint_as_float(mid << 16) + __uint_as_float(hi << 16));
 }
 
 }  // namespace drhip

@@ -113,7 +113,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         if (u >= units) return;
         Bf16Pair3 p[kUC / 2];
 #pragma unroll
-        for (int q = 0; q < kUC / 2; ++q) p[q] = split_pair(v[2 * q], v[2 * q + 1]);
+        for (int q = 0; q < kUC / 2; ++q) p[q] = split_pair(kSplitScale * v[2 * q], kSplitScale * v[2 * q + 1]);
         char* d = buf + u * kUnitBytes;
         if constexpr (CP == 16) {
             *(u32x4b*)d = u32x4b{p[0].hi, p[1].hi, p[2].hi, p[3].hi};
@@ -255,23 +255,23 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         for (int r = 0; r < 16; ++r)
             part[((wk * 32 * WO + 32 * wo + 8 * (r / 4) + 4 * half + r % 4) * MT + m) * kPitch + l32] = acc[m][0][r];
     __syncthreads();
-    unsigned again = 0;                                 // turns whose output came out as NaN
+    unsigned again = 0;                                 // turns whose output did not come out finite
 #pragma unroll
     for (int n = 0; n < 2 * WO * MT; ++n) {             // 512 lanes: 16 (channel, block) pairs of 32 pixels a turn
         const int pair = 16 * n + (tid >> 5), m = pair % MT, oc = pair / MT, pl = tid & 31;
         float v = 0.0f;
 #pragma unroll
         for (int k = 0; k < WK; ++k) v += part[((k * 32 * WO + oc) * MT + m) * kPitch + pl];
-        again |= v != v ? 1u << n : 0u;
+        again |= fabsf(v) < __builtin_inff() ? 0u : 1u << n;
         const int o = blockIdx.z * (32 * WO) + oc;
         const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
-        v += biasT[oc];
+        v = fmaf(v, kSplitUnscale, biasT[oc]);
         if (s.relu) v = fmaxf(v, 0.0f);
         if (o < s.O && x < s.Wo && y < s.Ho) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
     }
 
-    // ---- outputs that came out as NaN ------------------------------------------------------------------------------
-    // An infinite sample (or one that bf16 rounds to infinity) has no three-part form and leaves NaN behind, and so do the parts of
+    // ---- outputs that did not come out finite ------------------------------------------------------------------------------
+    // An infinite sample (or one that is infinite once it is scaled) has no three-part form and leaves NaN behind, and so do the parts of
     // ordinary samples times an infinite weight: such outputs are worked out again in fp32 from the samples and the filters put
     // together.  Every wave for itself, pixel by pixel: its output channels side by side, the lanes left over share the k-steps.  A
     // pixel with a NaN in its window stays one.  (56x56 64->96 5x5, us: 12.6, with a NaN and an infinity among the samples 346, all NaN
@@ -312,8 +312,8 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
                     const int ix = left + i, iy = top + j;
                     const bool ok = c < s.I && i < s.kw && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
                     const float sample = in[ok ? (size_t)c * plane + iy * s.W + ix : 0];
-                    auto of = [&](u32x4b q) { return __builtin_bit_cast(float, e & 1 ? q[e / 2] & 0xffff0000u : q[e / 2] << 16); };
-                    v = ok ? fmaf(of(lo) + of(mid) + of(hi), sample, v) : v;
+                    auto of = [&](u32x4b q) { return e & 1 ? q[e / 2] >> 16 : q[e / 2] & 0xffffu; };
+                    v = ok ? fmaf(whole(of(hi), of(mid), of(lo)), sample, v) : v;
                 }
             }
 #pragma unroll

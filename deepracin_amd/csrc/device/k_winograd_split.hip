@@ -177,8 +177,8 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     const int lr = fast_div(l32 + off0, tilesXd), tx = l32 + off0 - lr * s.tilesX;
     const int firstTx = lr == 0 ? off0 : 0;
     const int rLds = half * 8 * CHB + 4 * (segment_at(lr) + 2 * (tx - firstTx) - (firstTx == 0 ? 1 : 0));
-    const float k0f = tx > 0 ? 1.0f : 0.0f, k3f = 2 * tx + 2 < W ? 1.0f : 0.0f;
-    const bool c2ok = 2 * tx + 1 < W;
+    // the masks of the samples beside the map carry the scale of the split as well
+    const float k0f = tx > 0 ? kSplitScale : 0.0f, k2f = 2 * tx + 1 < W ? kSplitScale : 0.0f, k3f = 2 * tx + 2 < W ? kSplitScale : 0.0f;
     float mm[8][4];                                 // combined window rows of this lane's tile, 8 channels
     float ra[4], rb[4];                             // a channel's rows on their way from LDS
     const char* samples = lds + set * 3 * BUFB;
@@ -191,7 +191,8 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     auto combine = [&](int j) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) mm[j][c] = fmaf(sgn, rb[c], ra[c]);
-        mm[j][2] = c2ok ? mm[j][2] : 0.0f;
+        mm[j][1] *= kSplitScale;                    // (the other two are multiplied where they are used)
+        mm[j][2] *= k2f;
     };
     u32x4b B[2][3];                                 // [position parity][part]
     float va[2], vb[2], xa[2], xb[2];               // the two items being split
@@ -332,10 +333,10 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             }
         return f32x4{p[0][0] + p[1][0] + p[2][0], p[0][1] + p[1][1] + p[2][1], p[1][0] - p[2][0] + p[3][0], p[1][1] - p[2][1] + p[3][1]};
     };
-    // An infinity, or a value that bf16 rounds to one, has no three-part form and has left NaN behind, and so has the sample beside
-    // the map that is multiplied by zero where it is one of those: what came out as NaN is noted, by pass, for the end.
+    // An infinity, or a value that is one once it is scaled, has no three-part form and has left NaN behind, and so has the sample
+    // beside the map that is multiplied by zero where it is one of those: what is not finite is noted, by pass, for the end.
     unsigned again = 0;
-    auto note = [&](int q, f32x4 y) { again |= __builtin_isunordered(y[0], y[1]) || __builtin_isunordered(y[2], y[3]) ? 1u << q : 0u; };
+    auto note = [&](int q, f32x4 y) { again |= (fabsf(y[0]) + fabsf(y[1])) + (fabsf(y[2]) + fabsf(y[3])) < __builtin_inff() ? 0u : 1u << q; };
     if (nSp > 1) {
         // The splits of a panel add their partial tiles up as those of the fp32 kernel do: each finishes its share of the
         // passes, stores the others' shares and then looks for its own in the slots of the other splits, whose contents
@@ -386,7 +387,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                     again &= ~(1u << q);
                     atomicAdd(&g_ws_join_timeouts, 1u);
                 }
-                if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2);
+                if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2, kSplitUnscale);
             }
         };
         if (nSp == 2) join(integral_constant<int, 2>{});
@@ -404,10 +405,10 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
         }
 #pragma unroll
         for (int q = 0; q < NP; ++q)
-            if (eOk && o0 + eo + EO * q < s.O) wino_finish(out, y[q], b[q], s.flags, o0 + eo + EO * q, plane, W, H, ox, oy, s.vec2);
+            if (eOk && o0 + eo + EO * q < s.O) wino_finish(out, y[q], b[q], s.flags, o0 + eo + EO * q, plane, W, H, ox, oy, s.vec2, kSplitUnscale);
     }
 
-    // ---- tiles that came out as NaN --------------------------------------------------------------------------------
+    // ---- tiles that did not come out finite --------------------------------------------------------------------------------
     // Once more in fp32, step by step as the fp32 kernel does it, and with the samples beside the map left out.  Every wave
     // for itself, tile by tile: its 2 * NP output channels side by side, the lanes left over share the input channels.  (Us, without
     // and with one NaN and one infinity among the samples: 56x56 512->512 58 / 241, 224x224 64->64 18 / 39; all NaN 68 and 30.)
@@ -458,8 +459,8 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                     const u32x4b hi = u[3 * x * 64], mid = u[(3 * x + 1) * 64], lo = u[(3 * x + 2) * 64];
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
-                        auto of = [&](u32x4b q) { return __builtin_bit_cast(float, j & 1 ? q[j / 2] & 0xffff0000u : q[j / 2] << 16); };
-                        m[x] = fmaf(of(lo) + of(mid) + of(hi), v[j][x], m[x]);
+                        auto of = [&](u32x4b q) { return j & 1 ? q[j / 2] >> 16 : q[j / 2] & 0xffffu; };
+                        m[x] = fmaf(whole(of(hi), of(mid), of(lo)), v[j][x], m[x]);
                     }
                 }
             }

@@ -69,8 +69,10 @@ int ws_join_timeouts(unsigned* count);              // of the split-operand kern
 constexpr int kEpiRelu = DRHIP_EPILOGUE_RELU, kEpiMaxPool2 = DRHIP_EPILOGUE_MAXPOOL2;   // bits of the `relu` argument
 
 // Bias, ReLU and store of one 2x2 tile of channel o, or of its maximum (a following 2x2/2 max pooling; W and H even).
-__device__ inline void wino_finish(float* out, f32x4 y, float bias, int flags, int o, int plane, int W, int H, int ox, int oy, int vec2) {
-    y += bias;
+// scale: a power of two that the sums are to be multiplied by.
+__device__ inline void wino_finish(float* out, f32x4 y, float bias, int flags, int o, int plane, int W, int H, int ox, int oy, int vec2, float scale = 1.0f) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y[k] = fmaf(y[k], scale, bias);
     if (flags & kEpiRelu) { y[0] = fmaxf(y[0], 0.f); y[1] = fmaxf(y[1], 0.f); y[2] = fmaxf(y[2], 0.f); y[3] = fmaxf(y[3], 0.f); }
     if (flags & kEpiMaxPool2)
         store1_through(out + (size_t)o * (plane >> 2) + (size_t)(oy >> 1) * (W >> 1) + (ox >> 1), fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])));

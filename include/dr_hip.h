@@ -156,8 +156,9 @@ int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* 
                                   int W, int H, int I, int O, int stride, int relu, int variant, void* stream);
 
 /* The same convolution for any odd filter and any stride on the bf16 matrix cores at fp32 accuracy: operands are split
- * into three bf16 parts each, which together hold all 24 significant bits, and six partial products are accumulated
- * in fp32.  F is the filter bank in the layout the kernel streams, produced once at prepare time from
+ * into three bf16 parts each, which together hold all 24 significant bits of any fp32 number up to 2^111, and six partial
+ * products are accumulated in fp32; outputs with larger or infinite operands, and results above 2^95, are worked out again in
+ * fp32, at a multiple of the time.  F is the filter bank in the layout the kernel streams, produced once at prepare time from
  * w [I][O][kh][kw]; drhip_conv_bank_floats(I,O,kw,kh) floats, 16-byte aligned.  drhip_conv_bank_usable: whether the
  * shape is covered (the patch of a tile fits LDS, 32-bit byte offsets).  `variant` 0 lets the launcher pick; otherwise
  * 0x100 | log2(32-pixel blocks per workgroup, 0..1) | n << 4 for 2 << n waves sharing a channel block (n = 0..2).

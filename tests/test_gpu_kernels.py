@@ -395,6 +395,26 @@ def test_conv_bank_keeps_extreme_weights(lib, dev, I, k, stride, infinite):
     assert_same_extremes(got, want)
 
 
+@pytest.mark.parametrize("operand,power", [(o, p) for o in ("samples", "weights") for p in (-146, -136, -126, -112, -60, 60, 100, 116, 124)])
+def test_split_kernels_hold_operands_of_any_size(lib, dev, oracle, operand, power):
+    """Samples and weights down to the smallest fp32 number keep all their bits, and what is too large for three parts once it is scaled, the
+    results included, is worked out in fp32."""
+    W, H, I, O = 23, 9, 20, 40
+    other = 2.0 ** (20 if power < 0 else -20)                       # results that fp32 has 24 bits for
+    scaled = lambda a, on: (a.astype(np.float64) * (2.0 ** power if on else other)).astype(np.float32)
+    x = scaled(rnd(I, H, W), operand == "samples")
+    for k in (3, 5):
+        w = scaled(rnd(I, O, k, k), operand == "weights")
+        F, y = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k)), dev.empty(O * H * W)
+        ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
+        ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, None, y, W, H, I, O, k, k, 1, 1, 0, 0, None))
+        want = oracle.conv_f64(x, w)
+        assert rel_err(dev.get(y, want.shape), want, floor=0.0) <= TOL / 20, k
+        if k == 3 and (operand == "samples" or power >= -126):      # (fp32 has no bits left for the transform of smaller filters)
+            for variant in (0x101, 0x101 | SPLIT_HALVES):
+                assert rel_err(split_winograd(lib, dev, x, w, variant)[0], want, floor=0.0) <= TOL / 20, hex(variant)
+
+
 def kernel_us(lib, go, arg, repeats=5):
     """Shortest execution time of the kernels that go(arg) launches."""
     best = 1e30
