@@ -361,6 +361,8 @@ def download_outputs(graph, squeeze=True):
     """Fetch every output buffer (blocking) in the graph's interface layout."""
     n = min(graph.num_outputs, 10)
     shapes = [node.out_shape for node in graph.outnodes[:n]]
+    if None in shapes:          # not prepared: there are none yet
+        return []
     flats = [np.empty(s[0] * s[1] * s[2], np.float32) for s in shapes]
     hosts = (c_void_p * max(n, 1))(*[f.__array_interface__["data"][0] for f in flats])
     got = graph.lib.dR_downloadOutputs(graph.ptr, hosts, n)

@@ -637,3 +637,12 @@ def test_split_kernel_waits_for_its_samples(split_kernel_code):
         first = [k for k, e in enumerate(front) if e == "F"][fetches - 1]
         wait = next(e for b in blocks for e in b if isinstance(e, int))
         assert memory(front[first + 1:]) >= wait > 0, (name, front, wait)
+
+
+def test_outputs_of_an_unprepared_graph_are_none_at_all(lib):
+    """download_outputs in front of prepare returns an empty list, as the reference's wrapper does: dR_getOutputBuffers counts none."""
+    with dr.Environment() as env:
+        g = env.create_graph()
+        x = dr.feed_node(g, [8, 8, 2])
+        dr.mark_as_output(dr.Pooling(x, "max", [1, 2, 2, 1], [1, 2, 2, 1]))
+        assert dr.download_outputs(g) == [] and dr.download_outputs(g, squeeze=False) == []
