@@ -216,7 +216,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         // a trip to LDS is as long as six MFMAs); its filters were requested kDepth steps ago.  The loads of a group go
         // out whether or not the steps exist, so that the number of loads in flight is known where it is waited for.
         u32x4b b[2][MT][3];
-        read_operands(buf, b[0], wk);
+        read_operands(buf, b[0], min(wk, s.steps - 1));                 // (a wave may have no step at all)
         for (int n = 0; n < mySteps; n += kDepth) {
 #pragma unroll
             for (int g = 0; g < kDepth; ++g) {
