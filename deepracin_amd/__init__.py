@@ -203,6 +203,7 @@ def load_library(path=None):
         "drhip_staging_download_capacity": (c_size_t, [vp]),
         "drhip_upload_staged": (c_int, [vp, vp, c_size_t, vp, c_size_t, vp]),
         "drhip_download_staged": (c_int, [vp, vp, vp, c_size_t, c_size_t, vp]),
+        "drhip_interleaved_to_planes": (None, [vp, vp, c_size_t, c_int]),
         "drhip_upload_staged_interleaved": (c_int, [vp, vp, vp, c_size_t, c_int, vp]),
         "drhip_download_staged_many": (c_int, [vp, c_int, POINTER(vp), POINTER(vp), POINTER(c_size_t), vp]),
         "drhip_fc_permute_rows_f32": (c_int, [vp, vp] + [c_int] * 4 + [vp]),

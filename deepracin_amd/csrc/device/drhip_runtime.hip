@@ -425,6 +425,13 @@ static int release_area(Staging* s, UploadArea& area, hipStream_t stream) {
     return DRHIP_OK;
 }
 
+// dst (16-byte aligned) = the pinned memory at src
+static int launch_copy_from_host(float* dst, const float* src, size_t n, hipStream_t stream) {
+    const size_t n4 = n / 4;
+    launch(copy_from_host_kernel, dim3((unsigned)std::max<size_t>(1, std::min<size_t>((n4 + 255) / 256, 512))), dim3(256), 0, stream, dst, src, n4, n);
+    return launched("copy_from_host_kernel");
+}
+
 int drhip_upload_staged(void* handle, void* dst, size_t off, const void* src, size_t bytes, void* stream) {
     Staging* s = (Staging*)handle;
     DRHIP_REQUIRE(s && dst && src, "drhip_upload_staged: NULL pointer");
@@ -442,16 +449,26 @@ int drhip_upload_staged(void* handle, void* dst, size_t off, const void* src, si
         for (int piece = 0; piece < 2 && lens[piece] > 0; ++piece) {
             const size_t begin = begins[piece], len = lens[piece];
             memcpy(area->mem + begin, (const char*)src + begin, len);
-            const size_t n = len / 4, n4 = n / 4;
-            launch(copy_from_host_kernel, dim3((unsigned)std::max<size_t>(1, std::min<size_t>((n4 + 255) / 256, 512))), dim3(256), 0, as_stream(stream),
-                   (float*)((char*)dst + off + begin), (const float*)(area->mem + begin), n4, n);
-            if (int rc = launched("copy_from_host_kernel")) return rc;
+            if (int rc = launch_copy_from_host((float*)((char*)dst + off + begin), (const float*)(area->mem + begin), len / 4, as_stream(stream))) return rc;
         }
     } else {
         memcpy(area->mem, src, bytes);
         if (int rc = check(hipMemcpyAsync((char*)dst + off, area->mem, bytes, hipMemcpyHostToDevice, as_stream(stream)), "hipMemcpyAsync(H2D, staged)")) return rc;
     }
     return release_area(s, *area, as_stream(stream));
+}
+
+// Channels c0 .. c1-1, 64 pixels at a time, so that the lines that are read are still in the cache when the next channel wants them.
+static void planes_of(float* planes, const float* src, size_t pixels, size_t C, size_t c0, size_t c1) {
+    for (size_t p0 = 0; p0 < pixels; p0 += 64) {
+        const size_t p1 = std::min(pixels, p0 + 64);
+        for (size_t c = c0; c < c1; ++c)
+            for (size_t p = p0; p < p1; ++p) planes[c * pixels + p] = src[p * C + c];
+    }
+}
+
+void drhip_interleaved_to_planes(float* planes, const float* src, size_t pixels, int channels) {
+    planes_of(planes, src, pixels, (size_t)channels, 0, (size_t)channels);
 }
 
 int drhip_upload_staged_interleaved(void* handle, float* dst, const float* src, size_t pixels, int channels, void* stream) {
@@ -480,14 +497,19 @@ int drhip_upload_staged_interleaved(void* handle, float* dst, const float* src, 
             if (int rc = launched("hwc_from_host_kernel")) return rc;
         }
     } else {
-        // Many channels, or more than a kernel should fetch: the host transposes while it fills the area, 64 pixels
-        // at a time so that the lines it reads are still in its cache when the next channel wants them.
-        for (size_t p0 = 0; p0 < pixels; p0 += 64) {
-            const size_t p1 = std::min(pixels, p0 + 64);
-            for (size_t c = 0; c < C; ++c)
-                for (size_t p = p0; p < p1; ++p) mem[c * pixels + p] = src[p * C + c];
-        }
-        if (int rc = check(hipMemcpyAsync(dst, mem, bytes, hipMemcpyHostToDevice, as_stream(stream)), "hipMemcpyAsync(H2D, staged)")) return rc;
+        // Many channels, or more than a kernel should fetch: the host transposes while it fills the area, which then goes
+        // over as any other upload does, in two pieces from 256 KiB on.  (Feed, a 1x1 layer and its output back, us, by the DMA
+        // engine / so: 28x28x32 36.1 / 24.7, 56x56x64 93 / 90, 64x64x200 238 / 220.)
+        const bool byKernel = s->uploadByKernel && bytes <= kStagingKernelUpload && (size_t)dst % 16 == 0;
+        const size_t half = C / 2 & ~(size_t)3, first = byKernel && bytes >= kStagingHalves && half > 0 ? half : C;      // (pieces start at a multiple of 16 bytes)
+        planes_of(mem, src, pixels, C, 0, first);
+        if (byKernel) {
+            if (int rc = launch_copy_from_host(dst, mem, pixels * first, as_stream(stream))) return rc;
+            if (first < C) {
+                planes_of(mem, src, pixels, C, first, C);
+                if (int rc = launch_copy_from_host(dst + pixels * first, mem + pixels * first, pixels * (C - first), as_stream(stream))) return rc;
+            }
+        } else if (int rc = check(hipMemcpyAsync(dst, mem, bytes, hipMemcpyHostToDevice, as_stream(stream)), "hipMemcpyAsync(H2D, staged)")) return rc;
     }
     return release_area(s, *area, as_stream(stream));
 }

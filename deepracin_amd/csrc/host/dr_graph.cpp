@@ -258,8 +258,7 @@ void dR_feedDataHWC(dR_Graph* net, dR_Node* feednode, gfloat* data) {
         return;
     }
     std::vector<float> planes(pixels * C);
-    for (size_t p = 0; p < pixels; ++p)
-        for (size_t c = 0; c < C; ++c) planes[c * pixels + p] = data[p * C + c];
+    drhip_interleaved_to_planes(planes.data(), data, pixels, (int)C);
     dR_uploadArray(net, (gchar*)"", planes.data(), 0, planes.size() * sizeof(float), feednode->outputBuf->buf);
 }
 

@@ -118,8 +118,10 @@ int    drhip_upload_staged(void* handle, void* dst_dev, size_t dst_byte_offset, 
 int    drhip_download_staged(void* handle, void* dst_host, const void* src_dev, size_t src_byte_offset, size_t bytes, void* stream);
 /* drhip_upload_staged for an interleaved image: dst [channels][pixels] (device) = src [pixels][channels] (host).  With
  * 2 to 4 channels and up to 4 MiB the kernel that fetches the pinned area brings the samples into planes on the way;
- * otherwise the host does while it fills the area. */
+ * otherwise the host does while it fills the area, from where it goes over like any other upload. */
 int    drhip_upload_staged_interleaved(void* handle, float* dst_dev, const float* src_host, size_t pixels, int channels, void* stream);
+/* planes [channels][pixels] = src [pixels][channels], both on the host */
+void   drhip_interleaved_to_planes(float* planes, const float* src, size_t pixels, int channels);
 /* drhip_download_staged for several arrays: one kernel and one wait for all of them where together they fit the
  * download area (at most 10), otherwise one after the other. */
 int    drhip_download_staged_many(void* handle, int count, float* const* dst_host, const float* const* src_dev, const size_t* floats, void* stream);

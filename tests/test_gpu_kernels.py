@@ -869,7 +869,11 @@ def test_interleaved_upload_and_joint_download(lib, dev, pixels, channels, env):
         for _ in range(2):
             a = rng.standard_normal((pixels, channels)).astype(np.float32)
             want = a.T.copy()
+            ok(lib, lib.drhip_timing_begin())
             ok(lib, lib.drhip_upload_staged_interleaved(h, buf, a.ctypes.data_as(vp), pixels, channels, None))
+            launches, ms = ctypes.c_int(), (ctypes.c_float * 8)()
+            ok(lib, lib.drhip_timing_end(ms, 8, ctypes.byref(launches)))
+            assert (launches.value > 0) == (not env and a.nbytes <= 4 << 20)      # by kernel up to 4 MiB, whatever the channels
             a[...] = np.nan                                                    # the caller's array is free again
             lengths = [min(pixels, 9000), 1, min(pixels, 17)] if channels > 1 else [pixels]
             backs = [np.full(n, -1.0, np.float32) for n in lengths]

@@ -646,3 +646,11 @@ def test_outputs_of_an_unprepared_graph_are_none_at_all(lib):
         x = dr.feed_node(g, [8, 8, 2])
         dr.mark_as_output(dr.Pooling(x, "max", [1, 2, 2, 1], [1, 2, 2, 1]))
         assert dr.download_outputs(g) == [] and dr.download_outputs(g, squeeze=False) == []
+
+
+@pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
+def test_interleaved_to_planes(lib, pixels, channels):
+    a = np.random.default_rng(0).standard_normal((pixels, channels)).astype(np.float32)
+    out = np.full((channels, pixels), np.nan, np.float32)
+    lib.drhip_interleaved_to_planes(out.ctypes.data, a.ctypes.data, pixels, channels)
+    assert np.array_equal(out, a.T)
