@@ -390,10 +390,11 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                 if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2, kSplitUnscale);
             }
         };
-        if (nSp == 2) join(integral_constant<int, 2>{});
-        else if (nSp == 3) join(integral_constant<int, 3>{});
-        else if (nSp == 4) join(integral_constant<int, 4>{});
-        else if constexpr (KW == 1) join(integral_constant<int, 8>{});
+        if (KW == 1 || nSp == 2) join(integral_constant<int, 2>{});
+        else if constexpr (KW == 2) {
+            if (nSp == 3) join(integral_constant<int, 3>{});
+            else join(integral_constant<int, 4>{});
+        }
     } else {
         f32x4 y[NP];                                    // (read in one go: with each store behind its own reads the notes cost the trunk
         float b[NP];                                    // 4.5 us)
@@ -480,7 +481,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
 struct WsPlan { int kw, wc, perXcd; bool turns; size_t lds; WsShape s; };
 
 // Variant: 0x100 | wave sets - 1 | sA << 12 | sB << 16 | nA << 20, where the first nA output panels of every XCD are cut into
-// sA splits (1, 2, 3, 4 or, with one wave set, 8) of their input channels and the others into sB; all zero: nothing is split.
+// sA splits (1 to 4, with one wave set 1 or 2) of their input channels and the others into sB; all zero: nothing is split.
 static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     if (variant < 0 || (variant & 0xffe) != 0x100 || W < 1 || H < 1 || I < 1 || O < 1) return false;
     p->kw = 1 + (variant & 1);
@@ -520,7 +521,7 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     if (s.sA == 1 && s.sB == 1) return true;
     // A workgroup waits for the other splits of its panel, which are its neighbours in dispatch order on the same XCD: as long
     // as one XCD holds more workgroups than a panel has splits, they all get to run.
-    auto allowed = [&](int n) { return n >= 1 && (n <= 4 || (n == 8 && p->kw == 1)) && (n - 1) * ceil_div(s.nC, n) < s.nC; };
+    auto allowed = [&](int n) { return n >= 1 && n <= 2 * p->kw && (n - 1) * ceil_div(s.nC, n) < s.nC; };
     return s.nA <= panels && allowed(s.sA) && allowed(s.sB) && std::max(s.sA, s.sB) < num_cu() / kXcds && p->perXcd < 8192 &&
            (long long)p->perXcd * kXcds * 32768 < (1ll << 31);
 }

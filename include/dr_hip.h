@@ -241,7 +241,7 @@ int drhip_conv3x3_winograd_join_timeouts(unsigned* count);
  * drhip_conv3x3_winograd_split_pick_variant returns 0 where drhip_conv3x3_winograd_f32 is the faster one (or this one
  * does not cover the shape: maps less than 11 wide, tensors beyond 32-bit byte offsets), else the variant to pass: 0x100 for one
  * set of four waves per workgroup (maps from 31 wide on), 0x101 for two that take alternate groups of 16 input channels, | sA << 12 | sB << 16 | nA << 20
- * if the input channels are split: the first nA panels of outputs on each XCD into sA pieces, the others into sB.  Such a launch
+ * if the input channels are split: the first nA panels of outputs on each XCD into sA pieces, the others into sB (1 to 4 pieces, with one set of waves 1 or 2).  Such a launch
  * joins the pieces itself and needs a workspace of drhip_conv3x3_winograd_split_workspace_floats floats that has been
  * through drhip_conv3x3_winograd_workspace_prepare_f32, for one launch at a time. */
 int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, int O);

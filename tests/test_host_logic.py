@@ -648,6 +648,12 @@ def test_outputs_of_an_unprepared_graph_are_none_at_all(lib):
         assert dr.download_outputs(g) == [] and dr.download_outputs(g, squeeze=False) == []
 
 
+def test_split_winograd_variants_are_those_that_the_rule_can_pick(lib):
+    """One set of waves joins halves, two join up to four pieces; other numbers of pieces are refused."""
+    joins = lambda base, n: lib.drhip_conv3x3_winograd_split_workspace_floats(160, 120, 256, 256, base | n << 12 | n << 16) > 0
+    assert [n for n in range(16) if joins(0x100, n)] == [2] and [n for n in range(16) if joins(0x101, n)] == [2, 3, 4]
+
+
 @pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
 def test_interleaved_to_planes(lib, pixels, channels):
     a = np.random.default_rng(0).standard_normal((pixels, channels)).astype(np.float32)
