@@ -340,9 +340,10 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     if (nSp > 1) {
         // The splits of a panel add their partial tiles up as those of the fp32 kernel do: each finishes its share of the
         // passes, stores the others' shares and then looks for its own in the slots of the other splits, whose contents
-        // say themselves whether they have arrived.  (Slots lie at a workgroup's own place in the grid, 8 apart within a panel.)
+        // say themselves whether they have arrived.  (Slots lie at a workgroup's place in the grid, whole panels in front left out, 8
+        // apart within a panel.)
         const __amdgpu_buffer_rsrc_t rWs = __builtin_amdgcn_make_buffer_rsrc((void*)ws, 0, 0x7ffffff0, kBufferFlags);
-        const unsigned group0 = blockIdx.x - (unsigned)(kXcds * split);
+        const unsigned group0 = blockIdx.x - (unsigned)(kXcds * (split + (s.sA == 1 ? s.wgsA : 0)));
         // The whole offset goes in the vector register.  With the region in the scalar one the compiler lets the next vector
         // instruction overwrite the data of a 16-byte store, and on gfx950 the store then now and then takes the new value.
         auto slot_of = [&](int u, int q) { return (int)((group0 + (unsigned)(kXcds * u)) * (unsigned)(OB * 32 * 16)) + 16 * ((eo + EO * q) * 32 + et); };
@@ -596,7 +597,8 @@ extern "C" size_t drhip_conv3x3_winograd_split_filter_floats(int I, int O) {
 extern "C" size_t drhip_conv3x3_winograd_split_workspace_floats(int W, int H, int I, int O, int variant) {
     WsPlan p;
     if (!ws_plan(W, H, I, O, variant, &p) || (p.s.sA == 1 && p.s.sB == 1)) return 0;
-    return (size_t)p.perXcd * kXcds * 8192;
+    const int slots = (p.s.sA > 1 ? p.s.wgsA : 0) + (p.s.sB > 1 ? p.perXcd - p.s.wgsA : 0);     // whole panels need none
+    return (size_t)std::max(slots, 1) * kXcds * 8192;       // (never 0 for a variant with pieces: that means it is refused)
 }
 
 extern "C" int drhip_winograd_split_filter_transform_f32(const float* w, float* U, int I, int O, void* stream) {

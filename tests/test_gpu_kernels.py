@@ -446,6 +446,25 @@ def test_a_sample_that_is_nan_does_not_hold_a_launch_up(lib, dev):
         assert worse <= 40 * good and none <= 20 * good     # (by one lane each: 160 times)
 
 
+@pytest.mark.parametrize("nA,sA,sB", [(1, 1, 2), (1, 2, 1), (1, 2, 2), (2, 1, 2), (0, 1, 2), (1, 4, 3), (1, 1, 4), (1, 3, 1)])
+def test_winograd_split_stays_inside_its_workspace(lib, dev, oracle, nA, sA, sB):
+    """Whole panels in front of cut ones, behind them, and pieces of two sizes: the result, every slot left with its marker, and
+    nothing written behind the workspace."""
+    W, H, I, O = 64, 36, 100, 70
+    variant = (0x101 if max(sA, sB) > 2 else 0x100) | nA << 20 | sA << 12 | sB << 16
+    x, w = rnd(I, H, W), rnd(I, O, 3, 3, scale=0.05)
+    n, guard = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant), 1 << 16
+    F, ws, y, xd = dev.empty(lib.drhip_conv3x3_winograd_split_filter_floats(I, O)), dev.empty(n + guard), dev.empty(O * H * W), dev.put(x)
+    ok(lib, lib.drhip_winograd_split_filter_transform_f32(dev.put(w), F, I, O, None))
+    ok(lib, lib.drhip_conv3x3_winograd_workspace_prepare_f32(ws, n, None))
+    want = oracle.conv_f64(x, w)
+    for _ in range(2):
+        ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, None, y, W, H, I, O, 0, variant, ws, None))
+        assert rel_err(dev.get(y, want.shape), want) <= TOL / 20
+        left = dev.get(ws, (n + guard,))
+        assert np.all(left[:n].view(np.uint32) == 0xffa5c3e1) and np.all(left[n:] == -777)
+
+
 @pytest.mark.parametrize("W,H,I,O", [(257, 129, 113, 65), (21, 48, 400, 512), (33, 31, 256, 512)])
 def test_winograd_split_picked(lib, dev, oracle, W, H, I, O):
     """The variant that the rule picks: a round of whole panels and halves behind it, narrow and wide maps in pieces, panels

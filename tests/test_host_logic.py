@@ -654,6 +654,14 @@ def test_split_winograd_variants_are_those_that_the_rule_can_pick(lib):
     assert [n for n in range(16) if joins(0x100, n)] == [2] and [n for n in range(16) if joins(0x101, n)] == [2, 3, 4]
 
 
+def test_split_winograd_workspace_holds_pieces_only(lib):
+    """160x120 256->256 is 600 panels, 75 per XCD: slots of 32 KiB for the pieces, none for panels that stay whole."""
+    floats = lambda v: lib.drhip_conv3x3_winograd_split_workspace_floats(160, 120, 256, 256, v)
+    assert lib.drhip_conv3x3_winograd_split_pick_variant(160, 120, 256, 256) == 0x100 | 64 << 20 | 1 << 12 | 2 << 16
+    for nA, sA, sB, slots in ((64, 1, 2, 22), (75, 1, 2, 1), (75, 2, 1, 150), (10, 2, 1, 20), (10, 2, 2, 150), (0, 1, 2, 150), (0, 1, 1, 0)):
+        assert floats(0x100 | nA << 20 | sA << 12 | sB << 16) == slots * 8 * 8192, (nA, sA, sB)
+
+
 @pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
 def test_interleaved_to_planes(lib, pixels, channels):
     a = np.random.default_rng(0).standard_normal((pixels, channels)).astype(np.float32)
