@@ -614,3 +614,37 @@ def test_random_topologies(oracle, gpu, seed):
                     for i, a in zip(outs, got):
                         assert_close(a, step[i], "seed %d node %d (%s) of %s" % (seed, i, spec[i]["op"], [s["op"] for s in spec]),
                                      terms=spec_terms(spec[i]))
+
+
+def test_joined_layers_of_two_graphs_on_two_streams(lib, gpu):
+    """Pieces of a split-operand layer wait for each other inside the launch.  Two graphs with such a layer, each on its own
+    stream, run at the same time: every pass as if it were alone, and no piece waited in vain."""
+    rng = np.random.default_rng(3)
+    W, H, I, O = 33, 31, 256, 512
+    assert lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O) >> 12
+    late = ctypes.c_uint(0)
+    assert lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)) == 0
+    before = late.value
+    with dr.Environment() as one, dr.Environment() as two:
+        graphs, alone, streams = [], [], []
+        for env in (one, two):
+            g = env.create_graph()
+            streams.append(ctypes.c_void_p())
+            assert lib.drhip_stream_create(ctypes.byref(streams[-1])) == 0
+            lib.dR_setClEnvironment(ctypes.c_void_p(g.ptr), None, None, streams[-1], None)
+            x = dr.feed_node(g, [H, W, I])
+            c = dr.Conv2d_raw(x, (rng.standard_normal((I, O, 3, 3)) * 0.03).astype(np.float32), None, (1, 1), "relu")
+            dr.mark_as_output(c)
+            dr.prepare(g)
+            dr.feed_data(x, rng.standard_normal((H, W, I)).astype(np.float32))
+            alone.append(dr.apply(g)[0])
+            graphs.append(g)
+        for _ in range(5):
+            for _ in range(20):
+                for g in graphs:
+                    assert lib.dR_apply(g.ptr)
+            for g, want in zip(graphs, alone):
+                assert np.array_equal(dr.download_outputs(g)[0], want)
+    for st in streams:
+        assert lib.drhip_stream_destroy(st) == 0
+    assert lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)) == 0 and late.value == before

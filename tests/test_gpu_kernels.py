@@ -271,7 +271,7 @@ def test_winograd_split_operands(lib, dev, oracle, variant, W, H, I, O):
     n, ws = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant), None
     if n == 0 and (variant >> 12 or (W < 31 and variant == 0x100)):     # fewer panels or chunks than the variant needs, or a narrow map: refused
         assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, dev.empty(O * H * W), W, H, I, O, 0, variant, xd, None) == -1
-        return
+        pytest.skip("refused, as it has to be")
     if n:
         assert lib.drhip_conv3x3_winograd_split_f32(xd, F, None, dev.empty(O * H * W), W, H, I, O, 0, variant, None, None) == -1      # no workspace
         ws = dev.empty(n)
