@@ -17,7 +17,7 @@ of 20 passes is a few milliseconds long and a single sample of it says little), 
                  achieved / 157.3 TFLOP/s.  Winograd F(2x2,3x3) issues 2.25x fewer multiplications than
                  that, so `frac` is credit for the algorithm, NOT matrix-pipe utilisation: that is
                  `issued_tflops` (the FLOPs the kernel really issues, 2*16*tiles*I*O with tiles, I and O
-                 padded to its blocks -- the counter SQ_INSTS_VALU_MFMA_MOPS_F32 reads exactly this, see
+                 padded to its blocks -- the counters SQ_INSTS_VALU_MFMA_MOPS_F32 and _BF16 read exactly this, see
                  profiles/; six bf16 products each on the layers of the split-operand kernel) and
                  `mfma_busy_frac`, the share of the data-sheet matrix peaks (157.3 fp32, 2500 bf16) the
                  pipe was issuing at; the >= 50 % target is judged on `mfma_busy_frac`.
@@ -51,7 +51,8 @@ This script drives exactly one GPU.
 *_results.db (from --kernel-trace --stats) gives the per-kernel duration table; directories with
 *_counter_collection.csv (from --pmc) give per-dispatch counter tables of the last forward pass --
 FETCH_SIZE and WRITE_SIZE scaled by what the same run read for the plain 256 MiB copies of
---calibrate-copy, the matrix-core counters as issued FLOPs and busy share per Winograd launch -- and
+--calibrate-copy, the matrix-core counters as issued FLOPs and busy share per Winograd launch, busy cycles of the
+address unit and LDS -- and
 `--counters-json FILE` stores the figures bench.py reports (`traffic`, `mfma_busy_frac_counters`).
 """
 import argparse
@@ -246,6 +247,8 @@ def analyse(lib, m, workload, counters):
             issued, peak = winograd_issued_flops(lib, W, H, I, O)
             gk["issued"] += issued
             gk["busy_ms"] += issued / peak / 1e9
+            name = "winograd_f23_split_kernel" if peak == PEAK_MFMA_BF16_TFLOPS else KERNEL_NAMES[k]
+            gk.setdefault("names", collections.Counter())[name] += 1
             v = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O)
             if peak == PEAK_MFMA_F32_TFLOPS and (v >> 4) & 0xf and not v & 0x800:       # split layers whose partial tiles are summed by a second kernel
                 gk["kernels"] += 1
@@ -267,7 +270,8 @@ def analyse(lib, m, workload, counters):
         gk = groups[dominant]
         ach = gk["flops"] / (gk["ms"] * 1e-3) / 1e12
         rec = (counters.get(workload) or {}).get(dominant) or {}
-        roofline = {"kernel": KERNEL_NAMES[dominant], "bound": "mfma", "achieved": round(ach, 3), "peak": PEAK_MFMA_F32_TFLOPS,
+        names = gk.get("names") or {KERNEL_NAMES[dominant]: gk["launches"]}
+        roofline = {"kernel": " + ".join(n if len(names) == 1 else "%s x%d" % (n, c) for n, c in names.items()), "bound": "mfma", "achieved": round(ach, 3), "peak": PEAK_MFMA_F32_TFLOPS,
                     "unit": "TFLOP/s", "frac": round(ach / PEAK_MFMA_F32_TFLOPS, 4),
                     "frac_is": "direct-equivalent FLOPs / peak (algorithmic credit)",
                     "traffic": rec.get("traffic_bytes_per_launch"),
@@ -410,7 +414,7 @@ def _load_counters(path):
 
 def summarise(dirs, workload, counters_json, last=0):
     import sqlite3
-    fetch = write = mfma = None
+    fetch = write = mfma = units = None
     record = {}
     for d in dirs:
         for db in sorted(glob.glob(os.path.join(d, "**", "*_results.db"), recursive=True)):
@@ -428,8 +432,13 @@ def summarise(dirs, workload, counters_json, last=0):
                 fetch = per["FETCH_SIZE"]
             if "WRITE_SIZE" in per:
                 write = per["WRITE_SIZE"]
+            if "TA_TA_BUSY_sum" in per:
+                units = per
             if "SQ_INSTS_VALU_MFMA_MOPS_F32" in per:
                 mfma = per
+                bf16 = {r["dispatch"]: r["value"] for r in per.get("SQ_INSTS_VALU_MFMA_MOPS_BF16", [])}
+                for r in per["SQ_INSTS_VALU_MFMA_MOPS_F32"]:        # a kernel issues the one or the other
+                    r["value"] += bf16.get(r["dispatch"], 0.0)
     if fetch and write:
         cf = [r["value"] for r in fetch if "copy3d" in r["kernel"]][1:]
         cw = [r["value"] for r in write if "copy3d" in r["kernel"]][1:]
@@ -453,7 +462,7 @@ def summarise(dirs, workload, counters_json, last=0):
         for k, (n, a, b) in tot.items():
             print("| `%s` | %d | %.1f | %.1f | %.1f |" % (k, n, a, b, (a + b) / n))
         print()
-        for group, match in (("winograd", "winograd_f23"), ("fc", "fc_gemv"), ("conv1x1", "conv1x1_mfma"), ("direct", "direct_mfma")):
+        for group, match in (("winograd", "winograd_f23"), ("fc", "fc_gemv"), ("conv1x1", "conv1x1_mfma"), ("direct", "direct_mfma"), ("bank", "conv_bank")):
             sel = [(n, a, b) for k, (n, a, b) in tot.items() if match in k]
             if sel:
                 n = sum(s[0] for s in sel)
@@ -461,12 +470,12 @@ def summarise(dirs, workload, counters_json, last=0):
     if mfma:
         mops = _last_pass(mfma["SQ_INSTS_VALU_MFMA_MOPS_F32"], last)
         busy = {r["dispatch"]: r["value"] for r in mfma.get("SQ_VALU_MFMA_BUSY_CYCLES", [])}
-        print("Matrix-core counters of the launches of the last forward pass that issue MFMAs.  SQ_INSTS_VALU_MFMA_MOPS_F32 counts "
-              "512 FLOP per unit; SQ_VALU_MFMA_BUSY_CYCLES is summed over the chip's 1024 SIMDs; `kernel us` is the dispatch's own "
+        print("Matrix-core counters of the launches of the last forward pass that issue MFMAs.  SQ_INSTS_VALU_MFMA_MOPS_F32 (and _BF16, on the "
+              "split-operand kernels) counts 512 FLOP per unit; SQ_VALU_MFMA_BUSY_CYCLES is summed over the chip's 1024 SIMDs; `kernel us` is the dispatch's own "
               "End - Start timestamp under the profiler (longer than in a plain run); busy = busy cycles per SIMD / (kernel us x 2.4 GHz).\n")
         print("| # | kernel | grid (lanes) | MOPS | issued GFLOP | MFMA busy cycles/SIMD | kernel us | busy |")
         print("|---:|---|---:|---:|---:|---:|---:|---:|")
-        families = (("winograd", "winograd_f23"), ("direct", "direct_mfma"), ("conv1x1", "conv1x1_mfma"), ("first_layer", "fewc"))
+        families = (("winograd", "winograd_f23"), ("direct", "direct_mfma"), ("conv1x1", "conv1x1_mfma"), ("first_layer", "fewc"), ("bank", "conv_bank"))
         tot = collections.OrderedDict()
         k = 0
         reduce_us = 0.0
@@ -495,6 +504,17 @@ def summarise(dirs, workload, counters_json, last=0):
             rec["issued_gflop"] = round(tc / 1e9, 4)
             rec["profiled_us"] = round(tt, 2)
             rec["mfma_busy_frac"] = round(tb / (tt * 1e3 * PEAK_CLOCK_GHZ), 4)
+        print()
+    if units:
+        print("Unit counters per dispatch of the last forward pass, per compute unit (sums over the chip / 256), in clocks: cycles a CU had waves, "
+              "cycles its address unit (TA) was busy, cycles its LDS was accessed and those of them that bank conflicts added.\n")
+        print("| # | kernel | grid (lanes) | kernel us | CU busy | TA busy | LDS active | LDS conflicts |")
+        print("|---:|---|---:|---:|---:|---:|---:|---:|")
+        at = lambda c: {r["dispatch"]: r["value"] / 256.0 for r in units[c]}
+        busy, lds, conflicts = at("SQ_BUSY_CU_CYCLES"), at("SQ_LDS_IDX_ACTIVE"), at("SQ_LDS_BANK_CONFLICT")
+        for k, r in enumerate(_last_pass(units["TA_TA_BUSY_sum"], last)):
+            print("| %d | `%s` | %d | %.1f | %.0f | %.0f | %.0f | %.0f |" % (k + 1, r["kernel"], r["grid"], (r["end"] - r["start"]) / 1e3, busy[r["dispatch"]],
+                                                                     r["value"] / 256.0, lds[r["dispatch"]], conflicts[r["dispatch"]]))
         print()
     if counters_json and record:
         data = json.load(open(counters_json)) if os.path.exists(counters_json) else {}

@@ -4,8 +4,9 @@
 // bf16 MFMA where they exclude an fp32 one.
 //
 // What bounds it: the address unit of a CU.  Operands come as 16-byte loads per lane, 1 KiB each and 20 to 26 clocks; two
-// workgroups on a CU need 192 of them for filters and 40 for samples per 16 channels, about 5100 clocks beside 3200 of
-// MFMAs, 2700 of vector instructions and 2000 of LDS reads, and take 6300.  (A filter fragment serves two MFMAs here.  With two
+// workgroups on a CU need 192 of them for filters and 40 for samples per 16 channels.  Counted on 320x240 128->128, per 16
+// channels of two workgroups with their share of the first loads and the stores: the CU busy for 7300 clocks, its address
+// unit for 6000, the MFMAs of a SIMD 3070, LDS 2600 (1150 of them bank conflicts).  (A filter fragment serves two MFMAs here.  With two
 // blocks of tiles per wave it would serve four, but then the transform and the split of the samples, which every wave does
 // for its own row of the transform, take as long as the loads; splitting the positions of a row over two waves balances all
 // four units on paper and measured 5750 to 6300 with nothing left to overlap the first loads and the stores with.)

@@ -228,17 +228,18 @@ def test_winograd_fused_maxpool(lib, dev, oracle, variant, W, H, I, O):
     assert lib.drhip_conv3x3_winograd_f32(p, U, None, p, 4, 4, I, O, 4, 1, None, None) == -1      # unknown flag
 
 
-@pytest.mark.parametrize("I,k,stride", [(3, 7, 2), (4, 5, 1), (20, 5, 1), (17, 3, 3)])
-def test_conv_bank_keeps_infinities(lib, dev, I, k, stride):
-    """An infinite sample gives what fp32 arithmetic gives, in the filter's reach and nowhere else."""
-    W, H, O = 23, 19, 40
+@pytest.mark.parametrize("I,k,stride,variant", [(3, 7, 2, 0), (4, 5, 1, 0), (20, 5, 1, 0), (17, 3, 3, 0)]
+                         + [(I, 5, 1, 0x100 | n << 4 | m) for I in (3, 20) for n in range(3) for m in range(2)])
+def test_conv_bank_keeps_infinities(lib, dev, I, k, stride, variant):
+    """An infinite sample gives what fp32 arithmetic gives, in the filter's reach and nowhere else, whatever the tile."""
+    W, H, O = 23, 19, 40 if variant == 0 else 140
     x, w = rnd(I, H, W), rnd(I, O, k, k)
     x[1, 9, 12], x[I - 1, 0, 0], x[0, H - 1, W - 1] = np.inf, -np.inf, np.nan
     F = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k))
     ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
     Wo, Ho = W // stride, H // stride
     y = dev.empty(O * Ho * Wo)
-    ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, None, y, W, H, I, O, k, k, stride, stride, 0, 0, None))
+    ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, None, y, W, H, I, O, k, k, stride, stride, 0, variant, None))
     got, want = dev.get(y, (O, Ho, Wo)), np.zeros((O, Ho, Wo))
     pad = np.pad(x.astype(np.float64), ((0, 0), (k // 2, k // 2), (k // 2, k // 2)))
     for oy in range(Ho):
@@ -335,17 +336,20 @@ def split_winograd(lib, dev, x, w, variant, flags=0):
     if n:
         ws = dev.empty(n)
         ok(lib, lib.drhip_conv3x3_winograd_workspace_prepare_f32(ws, n, None))
+    shape = (O, H // 2, W // 2) if flags & 2 else (O, H, W)
     y = dev.empty(O * H * W)
     go = lambda xd: ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, None, y, W, H, I, O, flags, variant, ws, None))
     go(dev.put(x))
-    return dev.get(y, (O, H, W)), go
+    return dev.get(y, shape), go
 
 
-@pytest.mark.parametrize("variant", [0x100, 0x101, 0x100 | SPLIT_HALVES, 0x101 | 3 << 12 | 3 << 16])
-@pytest.mark.parametrize("W,H,I,O", [(33, 9, 70, 70), (40, 10, 100, 33)])
+@pytest.mark.parametrize("variant,W,H,I,O", [(v, W, H, I, O) for v in (0x100, 0x101, 0x100 | SPLIT_HALVES, 0x101 | 3 << 12 | 3 << 16)
+                                             for W, H, I, O in ((33, 9, 70, 70), (40, 10, 100, 33))]
+                         + [(0x101, 33, 9, 272, 33), (0x101 | SPLIT_HALVES, 28, 9, 100, 70), (0x101 | SPLIT_HALVES, 28, 9, 272, 33)])
 def test_winograd_split_keeps_infinities(lib, dev, variant, W, H, I, O):
     """Infinite samples, NaN and samples that bf16 rounds to infinity come out as fp32 Winograd has them, at the edges of the
-    map too, where the kernel's loads reach into the next row, and with the input channels in pieces."""
+    map too, where the kernel's loads reach into the next row, with the input channels in pieces, from different channels on and on
+    narrow maps."""
     x, w = rnd(I, H, W), rnd(I, O, 3, 3, scale=0.02)
     x[1, 4, 12], x[0, 0, 0], x[I - 1, H - 1, W - 1], x[I - 2, 3, 0], x[2, 5, W - 1] = np.inf, -np.inf, np.inf, -np.inf, np.inf
     x[3, 2, 26], x[4, 2, 27], x[2, 6, 20] = np.inf, -np.inf, np.nan
@@ -354,6 +358,10 @@ def test_winograd_split_keeps_infinities(lib, dev, variant, W, H, I, O):
     want = winograd_replay(x, w)
     assert np.isinf(want).sum() > O and np.isnan(want).any()
     assert_same_extremes(got, want)
+    if H % 2 == 0 and W % 2 == 0:           # ReLU and the pooling epilogue: fmaxf passes a NaN over
+        pooled, _ = split_winograd(lib, dev, x, w, variant, flags=3)
+        act = np.fmax(got, 0)
+        assert np.array_equal(pooled, np.fmax(np.fmax(act[:, ::2, ::2], act[:, ::2, 1::2]), np.fmax(act[:, 1::2, ::2], act[:, 1::2, 1::2])))
 
 
 @pytest.mark.parametrize("variant", [0x100, 0x101 | SPLIT_HALVES])
