@@ -17,6 +17,7 @@
 //     buffer load per lane and 1 KiB in a row per wave.  Every wave reads only its own 32 channels, several steps ahead.
 //   * Two, four or eight waves share the k-steps of one channel block round-robin and meet in LDS at the end, in wave order: layers with
 //     few tiles fill the chip that way without a second kernel.
+//   * Outputs that do not come out finite are worked out again in fp32, at the end.
 // Layers with at most four input channels (images) put four neighbouring pixels x four channels into one step of 16 k
 // (CP = 4) instead of 16 channels of one pixel, most of which would be zero: a 7x7 filter over RGB is 14 steps, not 49.
 #include "bf16x3.hpp"

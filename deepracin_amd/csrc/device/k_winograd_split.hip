@@ -23,6 +23,7 @@
 //     that work is cut into ticks and dealt out between the MFMAs of the position in front of it (without that the
 //     compiler gathers it in front of the MFMAs, and the matrix cores wait).
 //   * Filters are transformed and split once, when the layer is prepared, and come as 1 KiB fragments a step or half a step ahead.
+//   * Tiles that do not come out finite are worked out again in fp32, at the end.
 // With KW = 2 two such sets of four waves share the tiles and take alternate steps; their sums meet in LDS.  That is for
 // launches that leave at most one workgroup per CU, where a single set is alone on its SIMDs and waits for its own loads.
 // Launches whose panels do not fill the CUs evenly cut the input channels of all or of the last panels into pieces, which add their

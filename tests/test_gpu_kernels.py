@@ -22,6 +22,14 @@ def rnd(*shape, scale=1.0):
     return (RNG.standard_normal(shape) * scale).astype(np.float32)
 
 
+# (tests that draw from this one leave the inputs of the others as they are)
+OWN = np.random.default_rng(8)
+
+
+def own(*shape, scale=1.0):
+    return (OWN.standard_normal(shape) * scale).astype(np.float32)
+
+
 def ok(lib, rc):
     assert rc == 0, lib.drhip_last_error().decode()
 
@@ -228,12 +236,21 @@ def test_winograd_fused_maxpool(lib, dev, oracle, variant, W, H, I, O):
     assert lib.drhip_conv3x3_winograd_f32(p, U, None, p, 4, 4, I, O, 4, 1, None, None) == -1      # unknown flag
 
 
-@pytest.mark.parametrize("I,k,stride,variant", [(3, 7, 2, 0), (4, 5, 1, 0), (20, 5, 1, 0), (17, 3, 3, 0)]
-                         + [(I, 5, 1, 0x100 | n << 4 | m) for I in (3, 20) for n in range(3) for m in range(2)])
-def test_conv_bank_keeps_infinities(lib, dev, I, k, stride, variant):
-    """An infinite sample gives what fp32 arithmetic gives, in the filter's reach and nowhere else, whatever the tile."""
-    W, H, O = 23, 19, 40 if variant == 0 else 140
-    x, w = rnd(I, H, W), rnd(I, O, k, k)
+@pytest.mark.parametrize("I,k,stride", [(3, 7, 2), (4, 5, 1), (20, 5, 1), (17, 3, 3)])
+def test_conv_bank_keeps_infinities(lib, dev, I, k, stride):
+    """An infinite sample gives what fp32 arithmetic gives, in the filter's reach and nowhere else."""
+    W, H, O = 23, 19, 40
+    bank_with_infinities(lib, dev, rnd(I, H, W), rnd(I, O, k, k), stride, 0)
+
+
+@pytest.mark.parametrize("I", [3, 20])
+@pytest.mark.parametrize("variant", [0x100, 0x101, 0x110, 0x111, 0x120, 0x121])
+def test_conv_bank_keeps_infinities_in_every_tile(lib, dev, I, variant):
+    bank_with_infinities(lib, dev, own(I, 19, 23), own(I, 140, 5, 5), 1, variant)
+
+
+def bank_with_infinities(lib, dev, x, w, stride, variant):
+    (I, H, W), O, k = x.shape, w.shape[1], w.shape[2]
     x[1, 9, 12], x[I - 1, 0, 0], x[0, H - 1, W - 1] = np.inf, -np.inf, np.nan
     F = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k))
     ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
@@ -350,7 +367,7 @@ def test_winograd_split_keeps_infinities(lib, dev, variant, W, H, I, O):
     """Infinite samples, NaN and samples that bf16 rounds to infinity come out as fp32 Winograd has them, at the edges of the
     map too, where the kernel's loads reach into the next row, with the input channels in pieces, from different channels on and on
     narrow maps."""
-    x, w = rnd(I, H, W), rnd(I, O, 3, 3, scale=0.02)
+    x, w = own(I, H, W), own(I, O, 3, 3, scale=0.02)
     x[1, 4, 12], x[0, 0, 0], x[I - 1, H - 1, W - 1], x[I - 2, 3, 0], x[2, 5, W - 1] = np.inf, -np.inf, np.inf, -np.inf, np.inf
     x[3, 2, 26], x[4, 2, 27], x[2, 6, 20] = np.inf, -np.inf, np.nan
     x[5, 7, 5] = x[I - 1, 1, 22] = 3.399e38
@@ -369,7 +386,7 @@ def test_winograd_split_keeps_infinities(lib, dev, variant, W, H, I, O):
 def test_winograd_split_keeps_extreme_weights(lib, dev, variant, infinite):
     """Filters with an infinite or NaN weight, and finite ones that bf16 rounds to infinity, as fp32 Winograd has them."""
     W, H, I, O = 35, 7, 40, 40
-    x, w = rnd(I, H, W, scale=0.01), rnd(I, O, 3, 3)
+    x, w = own(I, H, W, scale=0.01), own(I, O, 3, 3)
     x[:, 3:5, 4:6] = 0
     if infinite:
         w[1, 3, 0, 0], w[I - 1, 7, 2, 2], w[0, 8, 0, 2], w[1, 8, 0, 0], w[0, 39, 1, 2] = np.inf, -np.inf, np.inf, -np.inf, np.nan
@@ -383,7 +400,7 @@ def test_winograd_split_keeps_extreme_weights(lib, dev, variant, infinite):
 def test_conv_bank_keeps_extreme_weights(lib, dev, I, k, stride, infinite):
     """Infinite weights, and finite ones that bf16 rounds to infinity, are what they are in fp32."""
     W, H, O = 23, 19, 40
-    x, w = np.abs(rnd(I, H, W, scale=0.01)), rnd(I, O, k, k)
+    x, w = np.abs(own(I, H, W, scale=0.01)), own(I, O, k, k)
     x[:, 3, 4] = 0
     if infinite:
         w[1, 3, 1, 1], w[I - 1, 7, 0, 0], w[0, 8, 0, 0], w[1, 8, 1, 1], w[0, 39, 1, 2] = np.inf, -np.inf, np.inf, -np.inf, np.nan
@@ -410,9 +427,9 @@ def test_split_kernels_hold_operands_of_any_size(lib, dev, oracle, operand, powe
     W, H, I, O = 23, 9, 20, 40
     other = 2.0 ** (20 if power < 0 else -20)                       # results that fp32 has 24 bits for
     scaled = lambda a, on: (a.astype(np.float64) * (2.0 ** power if on else other)).astype(np.float32)
-    x = scaled(rnd(I, H, W), operand == "samples")
+    x = scaled(own(I, H, W), operand == "samples")
     for k in (3, 5):
-        w = scaled(rnd(I, O, k, k), operand == "weights")
+        w = scaled(own(I, O, k, k), operand == "weights")
         F, y = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k)), dev.empty(O * H * W)
         ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
         ok(lib, lib.drhip_conv_bank_f32(dev.put(x), F, None, y, W, H, I, O, k, k, 1, 1, 0, 0, None))
@@ -440,14 +457,14 @@ def test_a_sample_that_is_nan_does_not_hold_a_launch_up(lib, dev):
     """What the split-operand kernels do about outputs that came out as NaN is work for whole waves, and none where a sample is NaN: such
     a launch takes a multiple of its time, not milliseconds."""
     W, H, I, O = 56, 56, 64, 96
-    x, w = rnd(I, H, W), rnd(I, O, 5, 5, scale=0.05)
+    x, w = own(I, H, W), own(I, O, 5, 5, scale=0.05)
     bad = x.copy()
     bad[10, 20, 30] = np.nan
     bad[11, 40, 9] = np.inf
     F, y = dev.empty(lib.drhip_conv_bank_floats(I, O, 5, 5)), dev.empty(O * H * W)
     ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, 5, 5, None))
     bank = lambda xd: ok(lib, lib.drhip_conv_bank_f32(xd, F, None, y, W, H, I, O, 5, 5, 1, 1, 0, 0, None))
-    _, wino = split_winograd(lib, dev, x, rnd(I, O, 3, 3, scale=0.05), 0x101)
+    _, wino = split_winograd(lib, dev, x, own(I, O, 3, 3, scale=0.05), 0x101)
     for what, go in (("bank", bank), ("winograd", wino)):
         good, worse, none = [kernel_us(lib, go, dev.put(a)) for a in (x, bad, np.full_like(x, np.nan))]
         print("%s: %.1f us, with a NaN and an infinity %.1f us, all NaN %.1f us" % (what, good, worse, none))
@@ -460,7 +477,7 @@ def test_winograd_split_stays_inside_its_workspace(lib, dev, oracle, nA, sA, sB)
     nothing written behind the workspace."""
     W, H, I, O = 64, 36, 100, 70
     variant = (0x101 if max(sA, sB) > 2 else 0x100) | nA << 20 | sA << 12 | sB << 16
-    x, w = rnd(I, H, W), rnd(I, O, 3, 3, scale=0.05)
+    x, w = own(I, H, W), own(I, O, 3, 3, scale=0.05)
     n, guard = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant), 1 << 16
     F, ws, y, xd = dev.empty(lib.drhip_conv3x3_winograd_split_filter_floats(I, O)), dev.empty(n + guard), dev.empty(O * H * W), dev.put(x)
     ok(lib, lib.drhip_winograd_split_filter_transform_f32(dev.put(w), F, I, O, None))
