@@ -236,7 +236,7 @@ int drhip_conv3x3_winograd_workspace_prepare_f32(float* workspace, size_t floats
 int drhip_conv3x3_winograd_join_timeouts(unsigned* count);
 
 /* The same convolution with the same fusions on the bf16 matrix cores at fp32 accuracy (operands in three bf16 parts, six
- * partial products, fp32 accumulation), for large layers.  F is the transformed and split filter bank, made once at
+ * partial products, fp32 accumulation; what does not come out finite is worked out again in fp32), for large layers.  F is the transformed and split filter bank, made once at
  * prepare time from w [I][O][3][3]; drhip_conv3x3_winograd_split_filter_floats(I,O) floats, 16-byte aligned.
  * drhip_conv3x3_winograd_split_pick_variant returns 0 where drhip_conv3x3_winograd_f32 is the faster one (or this one
  * does not cover the shape: maps less than 11 wide, tensors beyond 32-bit byte offsets), else the variant to pass: 0x100 for one
