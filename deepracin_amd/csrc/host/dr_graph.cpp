@@ -299,8 +299,12 @@ gint dR_downloadOutputs(dR_Graph* net, gfloat** hosts, gint n) {
 static bool tensor_fused_away(const dR_Node* n) {
     if (n->type == tConv2d) {
         const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
-        return c->drFusedPool || c->drFusedAvgPool;
+        const dR_Conv2d_Data* pair = c->drAbsorbedBy ? (const dR_Conv2d_Data*)c->drAbsorbedBy->layer : c;
+        return c->drFusedPool || c->drFusedAvgPool || c->drFireFrom || pair->drFireNext;
     }
+    if (n->type == tConcat && ((const dR_Concat_Data*)n->layer)->drFused)
+        for (const dR_Node* p : nodes_of(n->previous_layers))
+            if (p->type == tConv2d && ((const dR_Conv2d_Data*)p->layer)->drFireNext) return true;
     if (n->type == tPooling && ((const dR_Pooling_Data*)n->layer)->drFused && n->next_layers && n->next_layers->length == 1) {
         const dR_Node* c = (const dR_Node*)n->next_layers->first->element;
         return c->type == tConv2d && ((const dR_Conv2d_Data*)c->layer)->drPooledInput == n;

@@ -62,7 +62,9 @@ gchar* conv_print(dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     static const char* acts[] = { "Linear", "ReLU", "Sigmoid", "Tan" };
     // (variant numbers are each kernel's own)
-    const char* kernel = c->algo == drConv1x1Gemm ? "1x1 MFMA GEMM"
+    const char* kernel = c->drFireFrom ? "in the launch of the fire module in front"
+                       : c->drFire ? (c->drFireNext ? "fire module and the squeeze layer behind it, fp32 MFMA" : "fire module, fp32 MFMA")
+                       : c->algo == drConv1x1Gemm ? "1x1 MFMA GEMM"
                        : c->algo == drConvWinograd ? (c->drWinoSplit ? "Winograd F(2x2,3x3) split-operand bf16 MFMA" : "Winograd F(2x2,3x3) MFMA")
                        : c->drSplitBank ? "direct, split-operand bf16 MFMA" : c->drDirectBank ? "direct MFMA" : "direct";
     return fmt_dup("Conv2d Layer: %d\n Filter dimensions: %dx%d\n Input channels: %d\n Output channels: %d\n"
@@ -133,9 +135,25 @@ inline bool launch_has_bias(const dR_Conv2d_Data* c) {
     return c->useBias || (c->drAbsorbed1x1 && conv_of(c->drAbsorbed1x1)->useBias);
 }
 
+// The shape arguments of the drhip_fire_* calls for an expand pair.
+struct FireArgs { int W, H, S, E, Sn, pool; };
+FireArgs fire_args(const dR_Conv2d_Data* c) {
+    return FireArgs{c->ishape.s0, c->ishape.s1, c->shape.s2, c->shape.s3, c->drFireNext ? conv_of(c->drFireNext)->shape.s3 : 0, c->drFirePool ? 1 : 0};
+}
+
 gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     if (c->drAbsorbedBy) return TRUE;           // the 3x3 sibling carries this node's filters and bias
+    if (c->drFireFrom) {                        // its filters are in the other launch's bank; its sums are kept here
+        const FireArgs f = fire_args(conv_of(c->drFireFrom));
+        gboolean ok = dR_createFloatBuffer(net, &c->workspaceBuf, (gint)drhip_fire_partials_floats(f.W, f.H, f.S, f.E, f.Sn, f.pool), CL_MEM_READ_WRITE);
+        if (c->useBias) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, (c->shape.s3 + 15) & ~15, CL_MEM_READ_ONLY);
+        return ok;
+    }
+    if (c->drFire) {
+        const FireArgs f = fire_args(c);
+        return dR_createFloatBuffer(net, &c->weightsBuf, (gint)drhip_fire_bank_floats(f.W, f.H, f.S, f.E, f.Sn, f.pool), CL_MEM_READ_ONLY);
+    }
     const bool wino = c->algo == drConvWinograd;
     const int O = launch_channels(c);
     if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
@@ -156,6 +174,20 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     if (!c->hasVariables) { say("Conv2d Layer %d has no weights: call dR_Conv2d_setVariables first! \n", node->layerID); return FALSE; }
     if (c->drAbsorbedBy) return TRUE;
+    if (c->drFireFrom) {
+        std::vector<float> bias((size_t)(c->shape.s3 + 15) & ~(size_t)15, 0.0f);
+        if (c->useBias) memcpy(bias.data(), c->biases, (size_t)c->shape.s3 * sizeof(float));
+        return c->useBias ? dR_uploadArray(net, (gchar*)"", bias.data(), 0, bias.size() * sizeof(float), c->biasBuf) : TRUE;
+    }
+    if (c->drFire) {
+        const FireArgs f = fire_args(c);
+        const dR_Conv2d_Data* a = conv_of(c->drAbsorbed1x1);
+        std::vector<float> bank(drhip_fire_bank_floats(f.W, f.H, f.S, f.E, f.Sn, f.pool));
+        return !device_failed(net, drhip_fire_layout_f32(a->weights, c->weights, a->useBias ? a->biases : NULL, c->useBias ? c->biases : NULL,
+                                                         c->drFireNext ? conv_of(c->drFireNext)->weights : NULL, bank.data(), f.W, f.H, f.S, f.E, f.Sn, f.pool),
+                              "fire module filter layout") &&
+               dR_uploadArray(net, (gchar*)"", bank.data(), 0, bank.size() * sizeof(float), c->weightsBuf);
+    }
     gboolean ok = TRUE;
     if (c->algo == drConvWinograd) {
         // raw weights go up once, U = G g G^T is produced on the device, the raw copy is dropped.
@@ -216,7 +248,18 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
 gboolean conv_compute(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     if (c->drAbsorbedBy) return TRUE;           // computed by the 3x3 sibling's launch
+    if (c->drFireFrom) return TRUE;             // by the expand pair in front, and finished by the pair behind
     dR_Node* src = first_input(node);
+    if (c->drFire) {
+        const FireArgs f = fire_args(c);
+        const dR_Conv2d_Data* squeeze = src->type == tConv2d && conv_of(src)->drFireFrom ? conv_of(src) : NULL;
+        const FireArgs fin = squeeze ? fire_args(conv_of(squeeze->drFireFrom)) : FireArgs{};
+        return !device_failed(net, drhip_fire_f32(squeeze ? (const float*)squeeze->workspaceBuf : dev_out(src),
+                                                  squeeze ? drhip_fire_slices(fin.W, fin.H, fin.S, fin.E, fin.Sn, fin.pool) : 0,
+                                                  squeeze && squeeze->useBias ? (const float*)squeeze->biasBuf : NULL, squeeze && squeeze->activation == tReLU,
+                                                  (const float*)c->weightsBuf, c->drFireNext ? (float*)conv_of(c->drFireNext)->workspaceBuf : dev_out(c->drAbsorbed1x1),
+                                                  f.W, f.H, f.S, f.E, f.Sn, f.pool, c->activation == tReLU, stream_of(net)), "deepRACIN:conv2d");
+    }
     const float* in = dev_out(src);
     // with drFusedPool this is the pooling node's buffer; with an absorbed 1x1 sibling the launch
     // starts at that sibling's channels, which lie directly below this node's in the concat buffer

@@ -152,6 +152,40 @@ dR_Node* avgpool_fusable_producer(const dR_Node* p) {
     return c;
 }
 
+// The expand pair of a fire module as one launch that may take the next module's squeeze layer along (DR_FUSE_FIRE=0 keeps
+// layers apart).  `concat` is fused and holds nothing but the pair; returns its 3x3 layer.
+dR_Node* fire_pair(const dR_Node* concat) {
+    if (concat->type != tConcat || !((const dR_Concat_Data*)concat->layer)->drFused) return nullptr;
+    std::vector<dR_Node*> ins = nodes_of(concat->previous_layers);
+    if (ins.size() != 2 || ins[1]->type != tConv2d) return nullptr;
+    const dR_Conv2d_Data* c3 = (const dR_Conv2d_Data*)ins[1]->layer;
+    if (c3->drAbsorbed1x1 != ins[0]) return nullptr;
+    const dR_Conv2d_Data* c1 = (const dR_Conv2d_Data*)ins[0]->layer;
+    if (c1->shape.s3 != c3->shape.s3 || !c1->hasVariables || !c3->hasVariables) return nullptr;
+    return drhip_fire_slices(c3->ishape.s0, c3->ishape.s1, c3->shape.s2, c3->shape.s3, 0, 0) > 0 ? ins[1] : nullptr;
+}
+
+// The squeeze layer that is the only reader of a pair's outputs, directly or through a 3x3/2 max pooling it takes on load, and is itself
+// read by nothing but another such pair.
+dR_Node* fire_next(const dR_Node* concat, const std::map<const dR_Node*, dR_Node*>& pairOf, bool* pool) {
+    auto hidden = [](const dR_Node* n) { return !tensor_wanted(n) && !n->outputBuf && n->next_layers; };
+    if (!hidden(concat) || concat->next_layers->length != 1) return nullptr;
+    dR_Node* n = nodes_of(concat->next_layers)[0];
+    *pool = n->type == tPooling;
+    const dR_Node* pooling = *pool ? n : nullptr;
+    if (pooling) {
+        if (!hidden(pooling) || pooling->next_layers->length != 1) return nullptr;
+        n = nodes_of(pooling->next_layers)[0];
+    }
+    if (n->type != tConv2d || !hidden(n) || n->next_layers->length != 2) return nullptr;
+    const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
+    if (c->algo != drConv1x1Gemm || c->drFusedAvgPool || c->drFusedPool || c->drAbsorbedBy || c->drPooledInput != pooling || !c->hasVariables) return nullptr;
+    std::vector<dR_Node*> readers = nodes_of(n->next_layers);
+    if (readers[0] == readers[1]) return nullptr;
+    const std::map<const dR_Node*, dR_Node*>::const_iterator a = pairOf.find(readers[0]), b = pairOf.find(readers[1]);
+    return a != pairOf.end() && b != pairOf.end() && a->second == b->second ? n : nullptr;
+}
+
 }  // namespace
 
 extern "C" {
@@ -326,6 +360,35 @@ gboolean dR_planBuffers(dR_Graph* net) {
         if (dR_Node* pool = pooled_input_of(n)) {
             ((dR_Conv2d_Data*)n->layer)->drPooledInput = pool;
             ((dR_Pooling_Data*)pool->layer)->drFused = TRUE;
+        }
+    }
+    // Fire modules in a chain (after the fusions above, on which the rule rests)
+    for (dR_Node* n : sched)
+        if (n->type == tConv2d) {
+            dR_Conv2d_Data* c = (dR_Conv2d_Data*)n->layer;
+            c->drFire = c->drFirePool = FALSE;
+            c->drFireNext = c->drFireFrom = nullptr;
+        }
+    const char* fuseFire = getenv("DR_FUSE_FIRE");
+    if (!(fuseFire && strcmp(fuseFire, "0") == 0)) {
+        std::map<const dR_Node*, dR_Node*> pairOf;              // either layer of a pair -> its 3x3 layer
+        for (dR_Node* n : sched)
+            if (dR_Node* e3 = fire_pair(n)) pairOf[e3] = pairOf[((dR_Conv2d_Data*)e3->layer)->drAbsorbed1x1] = e3;
+        for (dR_Node* n : sched) {
+            dR_Node* e3 = fire_pair(n);
+            bool pool = false;
+            dR_Node* next = e3 ? fire_next(n, pairOf, &pool) : nullptr;
+            if (!next) continue;
+            dR_Conv2d_Data* c3 = (dR_Conv2d_Data*)e3->layer;
+            // (a chain does not begin behind a plain tensor with a pooling in it; in execution order, so what is in front is decided)
+            const dR_Node* squeeze = nodes_of(e3->previous_layers)[0];
+            if (pool && !(squeeze->type == tConv2d && ((const dR_Conv2d_Data*)squeeze->layer)->drFireFrom)) continue;
+            if (drhip_fire_slices(c3->ishape.s0, c3->ishape.s1, c3->shape.s2, c3->shape.s3, ((dR_Conv2d_Data*)next->layer)->shape.s3, pool) == 0) continue;
+            c3->drFire = TRUE;
+            c3->drFireNext = next;
+            c3->drFirePool = pool;
+            ((dR_Conv2d_Data*)next->layer)->drFireFrom = e3;
+            ((dR_Conv2d_Data*)pairOf[nodes_of(next->next_layers)[0]]->layer)->drFire = TRUE;       // (reads sums, whether it takes a layer along or not)
         }
     }
     auto root_of = [&](dR_Node* n, int* offset) {

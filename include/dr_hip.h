@@ -279,6 +279,24 @@ int drhip_conv1x1_pooled3s2_f32(const float* in, const float* w, const float* bi
  * variant 0 in drhip_conv1x1_f32 = let the launcher pick. */
 int drhip_conv1x1_pick_variant(int P, int I, int O);
 
+/* Fire modules in a chain, one launch each: the two expand layers of a module (1x1 and 3x3, E channels each, on the S channels of
+ * its squeeze layer) and the squeeze layer of the next module (1x1, Sn channels, on both outputs, 1x1 layer's first), with
+ * pool != 0 behind a 3x3 / stride-2 max pooling of them (rules as drhip_pool_f32).  out: that layer's sums without bias and
+ * activation, [slices][pixel][Sn rounded up to 16] with slices = drhip_fire_slices, to be added by the reader;
+ * Sn = 0: the expand outputs themselves, [2E][H][W].  in: a plain tensor [S][H][W] (slicesIn = 0; not with pool or
+ * Sn = 0) or the sums another launch has left, with the bias (S rounded up to 16, 16-byte
+ * aligned) and activation that belong to them.  drhip_fire_slices is 0 where a shape is not covered
+ * (S and Sn up to 64, E a multiple of 32).  bank: laid out once, on the host, from the layers' filters as they are handed over
+ * ([I][O][kh][kw]) and biases (NULL: none); drhip_fire_bank_floats floats, 16-byte aligned on the device.  No counterpart in the
+ * reference, which runs these layers one after the other (src/dR_nodes_conv2d.c:37-81, src/dR_nodes_pooling.c:277-401). */
+int    drhip_fire_slices(int W, int H, int S, int E, int Sn, int pool);
+size_t drhip_fire_bank_floats(int W, int H, int S, int E, int Sn, int pool);
+size_t drhip_fire_partials_floats(int W, int H, int S, int E, int Sn, int pool);
+int    drhip_fire_layout_f32(const float* w1, const float* w3, const float* b1, const float* b3, const float* wn, float* bank,
+                             int W, int H, int S, int E, int Sn, int pool);
+int    drhip_fire_f32(const float* in, int slicesIn, const float* inBias, int inRelu, const float* bank, float* out,
+                      int W, int H, int S, int E, int Sn, int pool, int relu, void* stream);
+
 /* ---- pooling ----------------------------------------------------------------------------------
  * out dims = ceil(in/stride) per axis; window anchored at (x*stx, y*sty, z*stz); samples outside
  * the input count as 0.0f; type 0 = max (start value -FLT_MAX), 1 = average (sum / (sx*sy*sz)).

@@ -191,6 +191,62 @@ def test_maxpool_taken_on_load_by_the_1x1_layer_behind_it(oracle, gpu):
     assert_close(got_sq, want[sq], "squeeze, pool as output")
 
 
+FIRE_CHAINS = [
+    # w, h, input channels, modules (squeeze, expand, 'p' with a 3x3/2 max pooling behind it), relu, bias, squeeze layers computed in other launches
+    (1, 1, 3, [(1, 32, ""), (1, 32, "")], True, True, 1),                       # one pixel
+    (13, 9, 20, [(16, 64, ""), (16, 64, "p"), (32, 128, "")], True, True, 2),
+    (56, 56, 24, [(16, 64, ""), (16, 64, "p"), (32, 128, ""), (32, 128, "p"), (48, 192, "")], True, True, 4),   # SqueezeNet's maps
+    (14, 14, 64, [(48, 192, ""), (64, 256, ""), (64, 256, "")], True, True, 2),
+    (17, 2, 40, [(64, 32, "p"), (50, 96, ""), (7, 32, "p"), (33, 64, "")], False, False, 2),        # ragged channels, nothing clipped at 0; pooled behind a plain tensor: apart
+    (113, 75, 16, [(16, 64, ""), (16, 64, "p"), (24, 32, "")], True, False, 2),
+    (9, 11, 8, [(65, 32, ""), (16, 48, ""), (64, 64, ""), (64, 32, "p")], True, True, 1),           # 65 and 48 are not covered: kernels of their own
+]
+
+
+@pytest.mark.parametrize("chain", FIRE_CHAINS, ids=lambda c: "%dx%d" % c[:2])
+def test_fire_modules_in_a_chain(oracle, gpu, chain):
+    """The expand layers of a module and the next module's squeeze layer in one launch, against the oracle and against
+    kernels of their own (DR_FUSE_FIRE=0)."""
+    w, h, cin, modules, relu, bias, hidden = chain
+    st = configs._Streams(77)
+    spec = [{"op": "feed", "shape": (w, h, cin)}]
+    cur, squeezes, tail = 0, [], None
+    for squeeze, expand, pool in modules:
+        spec.append(configs._conv(st, cur, 1, cin, squeeze, relu=relu, bias=bias)); s = len(spec) - 1
+        squeezes.append(s)
+        spec.append(configs._conv(st, s, 1, squeeze, expand, relu=relu, bias=bias))
+        spec.append(configs._conv(st, s, 3, squeeze, expand, relu=relu, bias=bias))
+        spec.append({"op": "concat", "ins": [s + 1, s + 2], "dim": 2}); cur, cin = s + 3, 2 * expand
+        if pool:
+            spec.append(configs._maxpool(cur, 3, 2)); cur = len(spec) - 1
+    feeds = {0: configs.image_input(st, w, h, spec[0]["shape"][2], 2.0) - np.float32(1)}
+    want = oracle.run_spec(spec, feeds)[cur]
+    res = {}
+    for flag in ("1", "0"):
+        os.environ["DR_FUSE_FIRE"] = flag
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, [cur])
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], feeds[0])
+                dr.graph_config(g).profilingGPU = 1
+                assert g.lib.dR_apply(g.ptr)
+                silent = sum(dr.node_struct(nodes[i]).drLastKernelMs == 0.0 for i in squeezes)
+                dr.graph_config(g).profilingGPU = 0
+                first = configs.fetch_chw(g)[0]
+                assert g.lib.dR_apply(g.ptr)
+                res[flag] = configs.fetch_chw(g)[0]
+                assert np.array_equal(first, res[flag])
+        finally:
+            os.environ.pop("DR_FUSE_FIRE", None)
+        assert silent == (hidden if flag == "1" else 0)
+        # (every layer rounds like a sum of at most 10 * 64 or 2 * 256 products; a chain of n of them carries n times that)
+        assert_close(res[flag], want, "chain, DR_FUSE_FIRE=%s" % flag, terms=1024 * len(modules) ** 2)
+    # another order of the same sums
+    assert rel_err(res["1"], res["0"]) <= 2e-6 * len(modules)
+
+
 def test_fc_chain_fused(oracle, gpu):
     """FC -> FC -> softmax: the finishing kernels of the two GEMVs disappear into their consumers
     (3 launches instead of 5) and the probabilities do not change by a bit."""
