@@ -265,6 +265,119 @@ conv1x1_mfma16_kernel(const float* __restrict__ in, const float* __restrict__ w,
     }
 }
 
+// A 1x1 layer in front of a global average, on an input that lies pixel by pixel ([P][I]; the fire module in front stores
+// it so).  Both operands are then 16 bytes per lane for four k-steps: lane l of a fragment holds filter or pixel l%16 and
+// input channels 4*(l/16) .. +3 of sixteen, and the MFMA of k-step s contracts channels s, 4+s, 8+s and 12+s.  A workgroup has
+// 16*NC pixels, staged in LDS once, and 64 output channels, sixteen to each pair of waves, which take half of the input channels
+// each; the pixels of a tile are added up by lanes.  What bounds it: 16*I*NC/4 clocks of MFMA a SIMD, 1.7 us on 14x14 512->1000, behind
+// 2 us of launch and first loads: all filters of a wave are under way at once (fetched anew as they are used they took a second trip,
+// 1 us more), and a second wave per SIMD takes the places where the first one waits (four waves: 6.4 us).  us a launch, with the
+// kernel above / this one: 14x14 512->1000 6.7 / 5.9, 29x19 15.9 / 11.6.
+template <int NC>
+__global__ void __launch_bounds__(512, 2)
+conv1x1_pixels_poolsum_kernel(const float* __restrict__ in, const float* __restrict__ F, const float* __restrict__ bias, float* __restrict__ partials, int P, int I, int O, int relu) {
+    constexpr int D = 16, U = 4;                    // fragments and quads of the tile under way
+    extern __shared__ __attribute__((aligned(16))) float part[];            // [16*NC][I + 4], then the second halves' sums
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lk = lane >> 4, half = wave >> 2;
+    const int ob = blockIdx.x * 4 + (wave & 3), p0 = blockIdx.y * 16 * NC, n = I >> 5, quads = I >> 2, pitch = I + 4;     // (items of this wave)
+    const int oBlocks = (O + 15) >> 4;
+    const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, P * I * 4, kC1BufferFlags);     // (zeros behind the last pixel)
+    const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, oBlocks * I * 64, kC1BufferFlags);
+    const __amdgpu_buffer_rsrc_t rBias = __builtin_amdgcn_make_buffer_rsrc((void*)bias, 0, bias ? O * 4 : 0, kC1BufferFlags);
+    auto load = [](const __amdgpu_buffer_rsrc_t& r, int v, int sOff) { return __builtin_bit_cast(f32x4ld, __builtin_amdgcn_raw_buffer_load_b128(r, v, sOff, 0)); };
+    // the tile's samples lie in a row: thread after thread, 8 KiB a round
+    f32x4ld v[U];
+    const int base = p0 * I * 4 + 16 * tid, total = 16 * NC * quads;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (u * 512 < total) v[u] = load(rIn, base, u * 8192);
+    asm volatile("" ::: "memory");
+    f32x4ld a[D];
+    const int f0 = (2 * min(ob, oBlocks - 1) + half) * n;                   // (a wave without channels repeats the last ones)
+#pragma unroll
+    for (int u = 0; u < D; ++u) a[u] = load(rF, 16 * lane, (f0 + min(u, n - 1)) << 10);
+    f32x4ld b0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b0[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rBias, 4 * (16 * ob + 4 * lk + r), 0, 0));
+    asm volatile("" ::: "memory");
+    auto put = [&](int i, const f32x4ld& q) {       // quad i of the tile: a pixel's quads lie together
+        const int px = i / quads;
+        if (i < total) *(f32x4ld*)(part + px * pitch + 4 * (i - px * quads)) = q;
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (u * 512 < total) put(u * 512 + tid, v[u]);
+    for (int i = U * 512; i < total; i += 512) put(i + tid, load(rIn, base, i * 16));
+    auto barrier = [] {                             // (LDS only: loads stay under way)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    barrier();
+
+    f32x4v acc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    const float* mine = part + l16 * pitch + 4 * lk + half * 16 * n;
+    f32x4ld b[2][NC];
+    auto read_b = [&](int u, int i) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) b[u & 1][c] = *(const f32x4ld*)(mine + 16 * c * pitch + 16 * min(i, n - 1));
+    };
+    read_b(0, 0);
+    for (int i0 = 0; i0 < n; i0 += D) {             // (loads go out whether or not there is an item for them: then it is known how many are under way)
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            if (u % 2 == 0 && u > 0 && i0 + u >= n) break;                  // (n is a multiple of 2)
+            read_b(u + 1, i0 + u + 1);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][k], b[u & 1][c][k], acc[c], 0, 0, 0);
+            a[u] = load(rF, 16 * lane, (f0 + min(i0 + D + u, n - 1)) << 10);
+        }
+    }
+    float* second = part + 16 * NC * pitch + ((wave & 3) * NC * 64 + lane) * 4;
+    if (half) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) *(f32x4v*)(second + c * 256) = acc[c];
+    }
+    barrier();
+    if (half) return;
+    // D: lane -> pixel l16, register r -> channel 4*lk + r
+    f32x4v sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const f32x4v other = *(const f32x4v*)(second + c * 256);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float y = acc[c][r] + other[r] + b0[r];
+            if (relu) y = fmaxf(y, 0.0f);
+            sum[r] += p0 + 16 * c + l16 < P ? y : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int m = 8; m >= 1; m >>= 1)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] += __shfl_xor(sum[r], m, 64);
+    if (l16 == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = 16 * ob + 4 * lk + r;
+            if (o < O) store_through(partials + (size_t)blockIdx.y * O + o, sum[r]);
+        }
+    }
+}
+
+// F[o/16][c/16][lane][4] from w[c][o]; what does not exist is zero
+__global__ void __launch_bounds__(256)
+conv1x1_pixels_layout_kernel(const float* __restrict__ w, float* __restrict__ F, int I, int O) {
+    const int n = I >> 4, lane = threadIdx.x >> 2, k = threadIdx.x & 3;
+    const int ob = blockIdx.x / n, c = 16 * (blockIdx.x - ob * n) + 4 * (lane >> 4) + k, o = 16 * ob + (lane & 15);
+    F[(size_t)blockIdx.x * 256 + threadIdx.x] = o < O ? w[(size_t)c * O + o] : 0.0f;
+}
+
 }  // namespace drhip
 
 using namespace drhip;
@@ -350,4 +463,28 @@ extern "C" int drhip_conv1x1_pooled3s2_f32(const float* in, const float* w, cons
     launch(conv1x1_mfma16_kernel<true>, dim3(nPT16, nOT16), dim3(64 * kw), (size_t)kw * 16 * kC1Pad16 * sizeof(float), as_stream(stream),
            in, w, bias, out, P, I, O, kw, (relu ? 1 : 0) | (int)(dWp.shift << 8), Win, Hin, dWp.mul);
     return launched("conv1x1_mfma16_kernel<pooled input>");
+}
+
+// 16 pixels a workgroup, 32 where that makes more slices than the reader has under way twice.
+extern "C" int drhip_conv1x1_pixels_tile(int P) { return P > 1024 ? 32 : 16; }
+
+extern "C" int drhip_conv1x1_pixels_layout_f32(const float* w, float* F, int I, int O, void* stream) {
+    DRHIP_REQUIRE(w && F && I > 0 && I % 16 == 0 && O > 0 && (long long)I * O < (1ll << 28), "drhip_conv1x1_pixels_layout_f32: bad arguments");
+    launch(conv1x1_pixels_layout_kernel, dim3(ceil_div(O, 16) * (I / 16)), dim3(256), 0, as_stream(stream), w, F, I, O);
+    return launched("conv1x1_pixels_layout_kernel");
+}
+
+extern "C" int drhip_conv1x1_pixels_poolsum_f32(const float* in, const float* F, const float* bias, float* partials, int P, int I, int O, int relu, void* stream) {
+    DRHIP_REQUIRE(in && F && partials, "drhip_conv1x1_pixels_poolsum_f32: NULL tensor");
+    DRHIP_REQUIRE(P > 0 && I > 0 && I % 64 == 0 && I <= 1024 && O > 0 && O <= 65535 && (long long)P * I < (1ll << 28), "drhip_conv1x1_pixels_poolsum_f32: bad shape P=%d I=%d O=%d", P, I, O);
+    DRHIP_REQUIRE((((size_t)in | (size_t)F) & 15) == 0, "drhip_conv1x1_pixels_poolsum_f32: input and filters need 16-byte alignment");
+    const int tile = drhip_conv1x1_pixels_tile(P);
+    const size_t ldsBytes = (size_t)tile * (I + 4 + 64) * sizeof(float);
+    const dim3 grid(ceil_div(O, 64), ceil_div(P, tile));
+    DRHIP_REQUIRE(grid.y <= 65535, "drhip_conv1x1_pixels_poolsum_f32: %d pixels are too many", P);
+    static std::atomic<unsigned long long> asked1{0}, asked2{0};
+    if (int rc = tile == 16 ? allow_lds((const void*)conv1x1_pixels_poolsum_kernel<1>, ldsBytes, asked1) : allow_lds((const void*)conv1x1_pixels_poolsum_kernel<2>, ldsBytes, asked2)) return rc;
+    if (tile == 16) launch(conv1x1_pixels_poolsum_kernel<1>, grid, dim3(512), ldsBytes, as_stream(stream), in, F, bias, partials, P, I, O, relu);
+    else launch(conv1x1_pixels_poolsum_kernel<2>, grid, dim3(512), ldsBytes, as_stream(stream), in, F, bias, partials, P, I, O, relu);
+    return launched("conv1x1_pixels_poolsum_kernel");
 }

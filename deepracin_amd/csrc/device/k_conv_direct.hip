@@ -181,12 +181,14 @@ constexpr int kFpThreads = 64 * kFpWaves;
 constexpr int kFpPitch = 16 * kFpWaves + 1;         // LDS row pitch (floats)
 typedef float f32x4d __attribute__((ext_vector_type(4)));
 
-template <int MB, int KS>                           // KS = k-steps = ceil(9*I / 4)
+// SQUEEZE: a 1x1 layer behind the pooling, for which all its input channels (at most 16*MB) are here: the pooled pixels meet its
+// filters (wn, fragments as the fire modules have them) right away, and its sums are what is stored, [pixel][16*MBn].
+template <int MB, int KS, bool SQUEEZE>             // KS = k-steps = ceil(9*I / 4)
 __global__ void __launch_bounds__(kFpThreads)
 conv3x3_fewc_pool3s2_kernel(const float* __restrict__ in, const float* __restrict__ w, const float* __restrict__ bias,
-                            float* __restrict__ out, unsigned wh, unsigned io, unsigned woho, unsigned cfg) {
+                            float* __restrict__ out, unsigned wh, unsigned io, unsigned woho, unsigned cfg, const float* __restrict__ wn) {
     // (12 dwords of arguments, which arrive in SGPRs with the wave: wh = W | H << 16, io = I | O << 16,
-    // woho = Wo | Ho << 16, cfg = sx | sy << 4 | relu << 8)
+    // woho = Wo | Ho << 16, cfg = sx | sy << 4 | relu << 8 | MBn << 9)
     const int W = (int)(wh & 0xffffu), H = (int)(wh >> 16), I = (int)(io & 0xffffu), O = (int)(io >> 16);
     const int Wo = (int)(woho & 0xffffu), Ho = (int)(woho >> 16), Wp = (Wo + 1) >> 1, Hp = (Ho + 1) >> 1;
     const int sx = (int)(cfg & 15u), sy = (int)((cfg >> 4) & 15u), relu = (int)((cfg >> 8) & 1u);
@@ -236,6 +238,12 @@ conv3x3_fewc_pool3s2_kernel(const float* __restrict__ in, const float* __restric
     }
     float bv = 0.0f;                                // the bias comes along in the same trip
     if (tid < OBc && bias) bv = bias[min(o0 + tid, O - 1)];
+    f32x4d a2[MB];
+    const int MBn = SQUEEZE ? (int)(cfg >> 9) : 0;
+    if (SQUEEZE && wave < MBn) {
+#pragma unroll
+        for (int c = 0; c < MB; ++c) a2[c] = *(const f32x4d*)(wn + (((wave * MB + c) << 8) + 4 * lane));
+    }
 #pragma unroll
     for (int u = 0; u < kRounds; ++u)
         if (dst[u] >= 0) wT[dst[u]] = fv[u];
@@ -266,11 +274,13 @@ conv3x3_fewc_pool3s2_kernel(const float* __restrict__ in, const float* __restric
         }
     __syncthreads();
 
+    constexpr int kPooledPitch = 16 * MB + 4;       // (in front of it lie the filters, which are in registers by now)
+    static_assert(!SQUEEZE || 16 * kPooledPitch <= 4 * KS * 16 * MB, "pooled pixels take the place of the filters");
     for (int idx = tid; idx < 16 * MB * kFpPool * kFpPool; idx += kFpThreads) {
         const int ch = idx / (kFpPool * kFpPool), pp = idx % (kFpPool * kFpPool);
         const int ppy = pp / kFpPool, ppx = pp % kFpPool;
         const int py = kFpPool * tileY + ppy, px = kFpPool * tileX + ppx;
-        if (py < Hp && px < Wp && o0 + ch < O) {
+        if (SQUEEZE || (py < Hp && px < Wp && o0 + ch < O)) {
             float r = -FLT_MAX;
 #pragma unroll
             for (int dy = 0; dy < 3; ++dy)
@@ -279,8 +289,25 @@ conv3x3_fewc_pool3s2_kernel(const float* __restrict__ in, const float* __restric
                     const float v = convT[ch * kFpPitch + (2 * ppy + dy) * kFpConv + 2 * ppx + dx];
                     if (v > r) r = v;
                 }
-            store_through(out + ((size_t)(o0 + ch) * Hp + py) * Wp + px, r);
+            if constexpr (SQUEEZE) wT[pp * kPooledPitch + ch] = ch < O ? r : 0.0f;
+            else store_through(out + ((size_t)(o0 + ch) * Hp + py) * Wp + px, r);
         }
+    }
+    if constexpr (SQUEEZE) {
+        __syncthreads();
+        if (wave >= MBn) return;
+        f32x4d sums = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < MB; ++c) {
+            const f32x4d v = *(const f32x4d*)(wT + j * kPooledPitch + 16 * c + 4 * lk);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[c][k], v[k], sums, 0, 0, 0);
+        }
+        const int py = kFpPool * tileY + j / kFpPool, px = kFpPool * tileX + j % kFpPool;
+        const __amdgpu_buffer_rsrc_t rOut = __builtin_amdgcn_make_buffer_rsrc((void*)out, 0, 0x7ffffff0, kBufferFlags);
+        typedef unsigned u32x4d __attribute__((ext_vector_type(4)));
+        if (py < Hp && px < Wp)                     // (sc0 sc1: written through)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4d, sums), rOut, 4 * ((py * Wp + px) * 16 * MBn + 16 * wave + 4 * lk), 0, 1 | 16);
     }
 }
 
@@ -648,8 +675,8 @@ extern "C" int drhip_conv2d_direct_f32(const float* in, const float* w, const fl
     return launch_direct<4>(in, w, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, s);
 }
 
-extern "C" int drhip_conv3x3_pool3s2_f32(const float* in, const float* w, const float* bias, float* out,
-                                         int W, int H, int I, int O, int strideX, int strideY, int relu, void* stream) {
+static int conv3x3_pool3s2(const float* in, const float* w, const float* bias, const float* wn, float* out, int W, int H, int I, int O, int Sn,
+                           int strideX, int strideY, int relu, void* stream) {
     DRHIP_REQUIRE(in && w && out, "drhip_conv3x3_pool3s2_f32: NULL tensor");
     DRHIP_REQUIRE(W > 0 && H > 0 && O > 0 && I >= 1 && I <= 4, "drhip_conv3x3_pool3s2_f32: bad shape %dx%dx%d -> %d (1 to 4 input channels)", W, H, I, O);
     DRHIP_REQUIRE(strideX > 0 && strideY > 0 && W / strideX > 0 && H / strideY > 0, "drhip_conv3x3_pool3s2_f32: bad stride or empty output");
@@ -662,12 +689,27 @@ extern "C" int drhip_conv3x3_pool3s2_f32(const float* in, const float* w, const 
     const bool wide = O > 32;                       // 64 channels per workgroup, else 32
     DRHIP_REQUIRE(tilesY <= 65535 && O <= 32 * 65535, "drhip_conv3x3_pool3s2_f32: tensor exceeds the launch grid");
     const dim3 grid(tilesX, tilesY, ceil_div(O, wide ? 64 : 32)), block(kFpThreads);
-#define DRHIP_FP(MBV, KSV) launch((conv3x3_fewc_pool3s2_kernel<MBV, KSV>), grid, block, 0, s, in, w, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, (unsigned)Wo | (unsigned)Ho << 16, (unsigned)strideX | (unsigned)strideY << 4 | (relu ? 256u : 0u))
-#define DRHIP_FP_K(MBV) do { if (ks == 3) DRHIP_FP(MBV, 3); else if (ks == 5) DRHIP_FP(MBV, 5); else if (ks == 7) DRHIP_FP(MBV, 7); else DRHIP_FP(MBV, 9); } while (0)
+#define DRHIP_FPS(MBV, KSV, SQ) launch((conv3x3_fewc_pool3s2_kernel<MBV, KSV, SQ>), grid, block, 0, s, in, w, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, (unsigned)Wo | (unsigned)Ho << 16, (unsigned)strideX | (unsigned)strideY << 4 | (relu ? 256u : 0u) | (unsigned)ceil_div(Sn, 16) << 9, wn)
+#define DRHIP_FP(MBV, KSV) do { if (wn) DRHIP_FPS(MBV, KSV, true); else DRHIP_FPS(MBV, KSV, false); } while (0)
+#define DRHIP_FP_K(MBV) do { if (ks == 3) DRHIP_FPS(MBV, 3, false); else if (ks == 5) DRHIP_FP(MBV, 5); else if (ks == 7) DRHIP_FP(MBV, 7); else DRHIP_FP(MBV, 9); } while (0)
     if (wide) DRHIP_FP_K(4); else DRHIP_FP_K(2);
 #undef DRHIP_FP_K
 #undef DRHIP_FP
+#undef DRHIP_FPS
     return launched("conv3x3_fewc_pool3s2_kernel");
+}
+
+extern "C" int drhip_conv3x3_pool3s2_f32(const float* in, const float* w, const float* bias, float* out,
+                                         int W, int H, int I, int O, int strideX, int strideY, int relu, void* stream) {
+    return conv3x3_pool3s2(in, w, bias, nullptr, out, W, H, I, O, 0, strideX, strideY, relu, stream);
+}
+
+extern "C" int drhip_conv3x3_pool3s2_squeeze_f32(const float* in, const float* w, const float* bias, const float* wn, float* out,
+                                                 int W, int H, int I, int O, int Sn, int strideX, int strideY, int relu, void* stream) {
+    DRHIP_REQUIRE(wn && (((size_t)wn | (size_t)out) & 15) == 0, "drhip_conv3x3_pool3s2_squeeze_f32: the squeeze layer's filters and sums need 16-byte alignment");
+    DRHIP_REQUIRE(O >= 1 && O <= 64 && Sn >= 1 && Sn <= 64 && I >= 2, "drhip_conv3x3_pool3s2_squeeze_f32: %d -> %d -> %d channels are not covered", I, O, Sn);
+    DRHIP_REQUIRE(strideX > 0 && strideY > 0 && (long long)(W / strideX / 2 + 1) * (H / strideY / 2 + 1) * 64 < (1ll << 28), "drhip_conv3x3_pool3s2_squeeze_f32: %dx%d is too large", W, H);
+    return conv3x3_pool3s2(in, w, bias, wn, out, W, H, I, O, Sn, strideX, strideY, relu, stream);
 }
 
 extern "C" size_t drhip_conv3x3_direct_filter_floats(int I, int O) {

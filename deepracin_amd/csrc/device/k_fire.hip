@@ -68,7 +68,7 @@ constexpr int fire_outs(int Q, bool pool) { return (16 * fire_columns(pool) + (p
 constexpr int fire_quads(int S16, bool pool) { return pool ? (S16 > 1 ? 3 : 2) : (S16 > 1 ? 2 : 1); }
 
 // Q: sixteens of channels of either layer per slice.  STORE: the expand outputs themselves are
-// stored, 1x1 layer first, [2E][H][W].  PLAIN: the input is a tensor [S][H][W].  Grid: slices x blocks across x blocks down (eight slices: one per XCD and its L2).
+// stored, 1x1 layer first, [2E][H][W] or, with bit 31 of outWh, [H][W][2E].  PLAIN: the input is a tensor [S][H][W].  Grid: slices x blocks across x blocks down (eight slices: one per XCD and its L2).
 // wh: W | H << 16.  block: bw | bh << 8 (output pixels of a workgroup) | ew << 16 | epx << 24 (expand pixels under them: columns, number).
 // misc: patch pixels | S << 8 | slices of the input << 16 | ReLU of the input << 24 | ReLU << 25 | MB << 26 |
 // log2(waves of different mb) << 29.  outWh: map of what is stored, Wo | Ho << 16 (STORE: E).
@@ -241,10 +241,13 @@ fire_kernel(const float* __restrict__ in, const float* __restrict__ bank, unsign
 #pragma unroll
         for (int c = 0; c < NCW; ++c) {
             if constexpr (STORE) {
-                float* o = out + (size_t)(k * (int)outWh + blockIdx.x * 16 * Q + 16 * q + 4 * lk) * plane + place[c];
-                if (inMap[c]) {
+                const int E = outWh & 0x7fffffff, o = k * E + blockIdx.x * 16 * Q + 16 * q + 4 * lk;
+                if (outWh >> 31) {
+                    const __amdgpu_buffer_rsrc_t rOut = __builtin_amdgcn_make_buffer_rsrc((void*)out, 0, 0x7ffffff0, kBufferFlags);
+                    if (inMap[c]) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4f, sum[c]), rOut, 4 * (place[c] * 2 * E + o), 0, kAuxThrough16);
+                } else if (inMap[c]) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) store_through(o + (size_t)r * plane, sum[c][r]);
+                    for (int r = 0; r < 4; ++r) store_through(out + (size_t)(o + r) * plane + place[c], sum[c][r]);
                 }
             } else {
                 if (POOL && !inMap[c]) sum[c] = f32x4f{0.f, 0.f, 0.f, 0.f};     // (samples beside the map count as 0.0)
@@ -444,12 +447,13 @@ extern "C" int drhip_fire_layout_f32(const float* w1, const float* w3, const flo
 }
 
 extern "C" int drhip_fire_f32(const float* in, int slicesIn, const float* inBias, int inRelu, const float* bank, float* out,
-                              int W, int H, int S, int E, int Sn, int pool, int relu, void* stream) {
+                              int W, int H, int S, int E, int Sn, int pool, int relu, int pixels, void* stream) {
     DRHIP_REQUIRE(in && bank && out, "drhip_fire_f32: NULL tensor");
     DRHIP_REQUIRE(slicesIn >= 0 && slicesIn <= 32, "drhip_fire_f32: %d slices", slicesIn);
     DRHIP_REQUIRE(slicesIn > 0 || (Sn > 0 && !pool), "drhip_fire_f32: a plain input is not covered where the expand outputs are stored or pooled");
-    DRHIP_REQUIRE((((size_t)bank | (size_t)(slicesIn > 0 ? in : nullptr) | (size_t)(slicesIn > 0 ? inBias : nullptr) | (size_t)(Sn > 0 ? out : nullptr)) & 15) == 0,
-                  "drhip_fire_f32: banks, partial sums and their bias need 16-byte alignment");
+    DRHIP_REQUIRE(!pixels || (Sn == 0 && (long long)W * H * 2 * E < (1ll << 28)), "drhip_fire_f32: [H][W][2E] is for expand outputs of less than 1 GiB");
+    DRHIP_REQUIRE((((size_t)bank | (size_t)(slicesIn > 0 ? in : nullptr) | (size_t)(slicesIn > 0 ? inBias : nullptr) | (size_t)(Sn > 0 || pixels ? out : nullptr)) & 15) == 0,
+                  "drhip_fire_f32: banks, partial sums, their bias and outputs by pixel need 16-byte alignment");
     FirePlan p;
     DRHIP_REQUIRE(fire_plan(W, H, S, E, Sn, pool, &p), "drhip_fire_f32: %dx%d, %d -> 2 x %d -> %d is not covered", W, H, S, E, Sn);
     DRHIP_REQUIRE((long long)slicesIn * W * H * 16 * p.S16 < (1ll << 29), "drhip_fire_f32: %d slices of %dx%dx%d are too large", slicesIn, W, H, S);
@@ -457,7 +461,7 @@ extern "C" int drhip_fire_f32(const float* in, int slicesIn, const float* inBias
     c.wh = (unsigned)(W | H << 16);
     c.block = (unsigned)(p.bw | p.bh << 8 | p.ew << 16) | (unsigned)(p.ew * p.eh) << 24;
     c.misc = (unsigned)(p.hpx | S << 8 | slicesIn << 16) | (inRelu ? 1u << 24 : 0u) | (relu ? 1u << 25 : 0u) | (unsigned)p.MB << 26 | (p.MB > 2 ? 2u : p.MB > 1 ? 1u : 0u) << 29;
-    c.outWh = Sn > 0 ? (unsigned)(p.Wo | p.Ho << 16) : (unsigned)E;
+    c.outWh = Sn > 0 ? (unsigned)(p.Wo | p.Ho << 16) : (unsigned)E | (pixels ? 1u << 31 : 0u);
     switch (p.S16) {
         case 1: return launch_fire_s<1>(p, c, pool != 0, Sn == 0, slicesIn == 0);
         case 2: return launch_fire_s<2>(p, c, pool != 0, Sn == 0, slicesIn == 0);

@@ -300,14 +300,16 @@ static bool tensor_fused_away(const dR_Node* n) {
     if (n->type == tConv2d) {
         const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
         const dR_Conv2d_Data* pair = c->drAbsorbedBy ? (const dR_Conv2d_Data*)c->drAbsorbedBy->layer : c;
-        return c->drFusedPool || c->drFusedAvgPool || c->drFireFrom || pair->drFireNext;
+        return c->drFusedPool || c->drFusedAvgPool || c->drFireFrom || pair->drFireNext || pair->drByPixel;
     }
     if (n->type == tConcat && ((const dR_Concat_Data*)n->layer)->drFused)
         for (const dR_Node* p : nodes_of(n->previous_layers))
-            if (p->type == tConv2d && ((const dR_Conv2d_Data*)p->layer)->drFireNext) return true;
+            if (p->type == tConv2d && (((const dR_Conv2d_Data*)p->layer)->drFireNext || ((const dR_Conv2d_Data*)p->layer)->drByPixel)) return true;
     if (n->type == tPooling && ((const dR_Pooling_Data*)n->layer)->drFused && n->next_layers && n->next_layers->length == 1) {
         const dR_Node* c = (const dR_Node*)n->next_layers->first->element;
-        return c->type == tConv2d && ((const dR_Conv2d_Data*)c->layer)->drPooledInput == n;
+        if (c->type != tConv2d) return false;
+        const dR_Node* from = ((const dR_Conv2d_Data*)c->layer)->drFireFrom;
+        return ((const dR_Conv2d_Data*)c->layer)->drPooledInput == n || (from && ((const dR_Conv2d_Data*)from->layer)->drSqueezeNext);
     }
     if (n->type == tFullyConnected) return ((const dR_FC_Data*)n->layer)->drDeferReduce && !n->output;
     return false;

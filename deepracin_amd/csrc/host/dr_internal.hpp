@@ -62,6 +62,8 @@ inline void*  stream_of(const dR_Graph* net) { return net->clConfig->hipStream; 
 void link_single_input(dR_Node* node, dR_Node* input, const char* what);
 // Report a failed drhip_* call the way dR_openCLError does: message to stdout, FALSE to the caller.
 gboolean device_failed(dR_Graph* net, int status, const char* what);
+// Slices of the pixel sums that a 1x1 layer with drFusedAvgPool leaves.
+int avgpool_slices(const dR_Conv2d_Data* conv);
 // Copy caller-owned floats.
 float* dup_floats(const float* src, size_t n);
 // While dR_parseGraph builds a node, the float counts of the variable files it read for that node

@@ -62,7 +62,7 @@ gchar* conv_print(dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     static const char* acts[] = { "Linear", "ReLU", "Sigmoid", "Tan" };
     // (variant numbers are each kernel's own)
-    const char* kernel = c->drFireFrom ? "in the launch of the fire module in front"
+    const char* kernel = c->drFireFrom ? "in the launch of the layers in front"
                        : c->drFire ? (c->drFireNext ? "fire module and the squeeze layer behind it, fp32 MFMA" : "fire module, fp32 MFMA")
                        : c->algo == drConv1x1Gemm ? "1x1 MFMA GEMM"
                        : c->algo == drConvWinograd ? (c->drWinoSplit ? "Winograd F(2x2,3x3) split-operand bf16 MFMA" : "Winograd F(2x2,3x3) MFMA")
@@ -127,6 +127,21 @@ gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
 
 gboolean conv_create_kernel(dR_Graph*, dR_Node*) { return TRUE; }   // kernels are built into the library
 
+// The shape arguments of the drhip_fire_* calls for an expand pair.
+struct FireArgs { int W, H, S, E, Sn, pool; };
+FireArgs fire_args(const dR_Conv2d_Data* c) {
+    return FireArgs{c->ishape.s0, c->ishape.s1, c->shape.s2, c->shape.s3, c->drFireNext ? conv_of(c->drFireNext)->shape.s3 : 0, c->drFirePool ? 1 : 0};
+}
+// Slices of the sums of a squeeze layer that another launch leaves, and the floats of all of them.
+int squeeze_slices(const dR_Conv2d_Data* squeeze) {
+    const dR_Conv2d_Data* from = conv_of(squeeze->drFireFrom);
+    const FireArgs f = fire_args(from);
+    return from->drSqueezeNext ? 1 : drhip_fire_slices(f.W, f.H, f.S, f.E, f.Sn, f.pool);
+}
+size_t squeeze_floats(const dR_Conv2d_Data* squeeze) {
+    return (size_t)squeeze_slices(squeeze) * squeeze->ishape.s0 * squeeze->ishape.s1 * ((squeeze->shape.s3 + 15) & ~15);
+}
+
 // Output channels the node's launch produces: its own plus those of an absorbed 1x1 sibling.
 inline int launch_channels(const dR_Conv2d_Data* c) {
     return c->shape.s3 + (c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1)->shape.s3 : 0);
@@ -135,18 +150,12 @@ inline bool launch_has_bias(const dR_Conv2d_Data* c) {
     return c->useBias || (c->drAbsorbed1x1 && conv_of(c->drAbsorbed1x1)->useBias);
 }
 
-// The shape arguments of the drhip_fire_* calls for an expand pair.
-struct FireArgs { int W, H, S, E, Sn, pool; };
-FireArgs fire_args(const dR_Conv2d_Data* c) {
-    return FireArgs{c->ishape.s0, c->ishape.s1, c->shape.s2, c->shape.s3, c->drFireNext ? conv_of(c->drFireNext)->shape.s3 : 0, c->drFirePool ? 1 : 0};
-}
-
 gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     if (c->drAbsorbedBy) return TRUE;           // the 3x3 sibling carries this node's filters and bias
-    if (c->drFireFrom) {                        // its filters are in the other launch's bank; its sums are kept here
-        const FireArgs f = fire_args(conv_of(c->drFireFrom));
-        gboolean ok = dR_createFloatBuffer(net, &c->workspaceBuf, (gint)drhip_fire_partials_floats(f.W, f.H, f.S, f.E, f.Sn, f.pool), CL_MEM_READ_WRITE);
+    if (c->drFireFrom) {                        // its filters are in the other launch's bank (behind a first layer: here); its sums are kept here
+        gboolean ok = dR_createFloatBuffer(net, &c->workspaceBuf, (gint)squeeze_floats(c), CL_MEM_READ_WRITE);
+        if (conv_of(c->drFireFrom)->drSqueezeNext) ok = ok && dR_createFloatBuffer(net, &c->weightsBuf, ((c->shape.s3 + 15) & ~15) * (c->shape.s2 > 32 ? 64 : 32), CL_MEM_READ_ONLY);
         if (c->useBias) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, (c->shape.s3 + 15) & ~15, CL_MEM_READ_ONLY);
         return ok;
     }
@@ -160,13 +169,27 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     const int n = c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
                        : wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
                        : c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)
-                       : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1) : weight_count(c);
+                       : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1)
+                       : c->drByPixel ? ((O + 15) & ~15) * c->shape.s2 : weight_count(c);
     gboolean ok = dR_createFloatBuffer(net, &c->weightsBuf, n, CL_MEM_READ_ONLY);
     if (launch_has_bias(c)) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, O, CL_MEM_READ_ONLY);
     const size_t ws = wino ? winograd_workspace_floats(c, O) : 0;
     if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);   // split-K partial tiles
     if (c->drFusedAvgPool)                      // per-tile pixel sums for the pooling behind this layer
-        ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, drhip_conv1x1_poolsum_slices(c->ishape.s0 * c->ishape.s1) * O, CL_MEM_READ_WRITE);
+        ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, avgpool_slices(c) * O, CL_MEM_READ_WRITE);
+    return ok;
+}
+
+// weightsBuf of a 1x1 layer in fragments: raw weights [I][O] go up once, are laid out on the device and dropped.
+gboolean fill_by_pixel(dR_Graph* net, dR_Conv2d_Data* c, const float* rows, int I) {
+    const size_t rawBytes = (size_t)I * c->shape.s3 * sizeof(float);
+    cl_mem raw = NULL;
+    if (!dR_createFloatBuffer(net, &raw, I * c->shape.s3, CL_MEM_READ_ONLY)) return FALSE;
+    gboolean ok = dR_uploadArray(net, (gchar*)"", (void*)rows, 0, rawBytes, raw);
+    if (ok) ok = !device_failed(net, drhip_conv1x1_pixels_layout_f32((const float*)raw, (float*)c->weightsBuf, I, c->shape.s3, stream_of(net)), "1x1 filter layout");
+    if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "1x1 filter layout (sync)");
+    dR_clMemoryBufferCleanup(net, raw);
+    net->clConfig->memConsumptionGPU -= (glong)rawBytes;
     return ok;
 }
 
@@ -177,6 +200,12 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
     if (c->drFireFrom) {
         std::vector<float> bias((size_t)(c->shape.s3 + 15) & ~(size_t)15, 0.0f);
         if (c->useBias) memcpy(bias.data(), c->biases, (size_t)c->shape.s3 * sizeof(float));
+        if (conv_of(c->drFireFrom)->drSqueezeNext) {
+            const int I = c->shape.s2 > 32 ? 64 : 32;
+            std::vector<float> rows((size_t)I * c->shape.s3, 0.0f);
+            memcpy(rows.data(), c->weights, (size_t)weight_count(c) * sizeof(float));
+            if (!fill_by_pixel(net, c, rows.data(), I)) return FALSE;
+        }
         return c->useBias ? dR_uploadArray(net, (gchar*)"", bias.data(), 0, bias.size() * sizeof(float), c->biasBuf) : TRUE;
     }
     if (c->drFire) {
@@ -238,6 +267,8 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "direct filter layout (sync)");
         dR_clMemoryBufferCleanup(net, raw);
         net->clConfig->memConsumptionGPU -= (glong)rawBytes;
+    } else if (c->drByPixel) {
+        ok = fill_by_pixel(net, c, c->weights, c->shape.s2);
     } else {
         ok = dR_uploadArray(net, (gchar*)"", c->weights, 0, (size_t)weight_count(c) * sizeof(float), c->weightsBuf);
     }
@@ -253,12 +284,11 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
     if (c->drFire) {
         const FireArgs f = fire_args(c);
         const dR_Conv2d_Data* squeeze = src->type == tConv2d && conv_of(src)->drFireFrom ? conv_of(src) : NULL;
-        const FireArgs fin = squeeze ? fire_args(conv_of(squeeze->drFireFrom)) : FireArgs{};
         return !device_failed(net, drhip_fire_f32(squeeze ? (const float*)squeeze->workspaceBuf : dev_out(src),
-                                                  squeeze ? drhip_fire_slices(fin.W, fin.H, fin.S, fin.E, fin.Sn, fin.pool) : 0,
+                                                  squeeze ? squeeze_slices(squeeze) : 0,
                                                   squeeze && squeeze->useBias ? (const float*)squeeze->biasBuf : NULL, squeeze && squeeze->activation == tReLU,
                                                   (const float*)c->weightsBuf, c->drFireNext ? (float*)conv_of(c->drFireNext)->workspaceBuf : dev_out(c->drAbsorbed1x1),
-                                                  f.W, f.H, f.S, f.E, f.Sn, f.pool, c->activation == tReLU, stream_of(net)), "deepRACIN:conv2d");
+                                                  f.W, f.H, f.S, f.E, f.Sn, f.pool, c->activation == tReLU, c->drByPixel, stream_of(net)), "deepRACIN:conv2d");
     }
     const float* in = dev_out(src);
     // with drFusedPool this is the pooling node's buffer; with an absorbed 1x1 sibling the launch
@@ -277,7 +307,9 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
             break;
         }
         case drConv1x1Gemm:
-            if (c->drFusedAvgPool)
+            if (c->drByPixel)
+                rc = drhip_conv1x1_pixels_poolsum_f32(in, w, b, (float*)c->workspaceBuf, W * H, I, O, relu, stream_of(net));
+            else if (c->drFusedAvgPool)
                 rc = drhip_conv1x1_poolsum_f32(in, w, b, (float*)c->workspaceBuf, W * H, I, O, relu, stream_of(net));
             else if (c->drPooledInput) {        // the 3x3/2 max pooling in front is taken while loading its input
                 const dR_Pooling_Data* pd = (const dR_Pooling_Data*)c->drPooledInput->layer;
@@ -287,7 +319,10 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
                 rc = drhip_conv1x1_f32(in, w, b, out, W * H, I, O, relu, c->variant, stream_of(net));
             break;
         default:
-            if (c->drFusedPool)                 // first layer + the 3x3/2 max pool behind it (out = the pool's buffer)
+            if (c->drSqueezeNext) {             // and the squeeze layer behind that
+                const dR_Conv2d_Data* sq = conv_of(c->drSqueezeNext);
+                rc = drhip_conv3x3_pool3s2_squeeze_f32(in, w, b, (const float*)sq->weightsBuf, (float*)sq->workspaceBuf, W, H, I, O, sq->shape.s3, c->stride.s1, c->stride.s2, relu, stream_of(net));
+            } else if (c->drFusedPool)          // first layer + the 3x3/2 max pool behind it (out = the pool's buffer)
                 rc = drhip_conv3x3_pool3s2_f32(in, w, b, out, W, H, I, O, c->stride.s1, c->stride.s2, relu, stream_of(net));
             else if (c->drDirectBank)
                 rc = drhip_conv3x3_direct_mfma_f32(in, w, b, out, W, H, I, O, c->stride.s1, relu, c->variant, stream_of(net));
@@ -319,6 +354,11 @@ gboolean conv_cleanup_layer(dR_Graph*, dR_Node* node) {
 }
 
 }  // namespace
+
+int dr::avgpool_slices(const dR_Conv2d_Data* c) {
+    const int P = c->ishape.s0 * c->ishape.s1;
+    return c->drByPixel ? (P + drhip_conv1x1_pixels_tile(P) - 1) / drhip_conv1x1_pixels_tile(P) : drhip_conv1x1_poolsum_slices(P);
+}
 
 extern "C" {
 

@@ -155,7 +155,7 @@ drhip_deferred_vec deferred_output_of(dR_Node* producer) {
         const int P = c->ishape.s0 * c->ishape.s1;
         d.partials = (const float*)c->workspaceBuf;
         d.bias = NULL;
-        d.slices = drhip_conv1x1_poolsum_slices(P);
+        d.slices = avgpool_slices(c);
         d.n = c->shape.s3;
         d.relu = 0;
         d.finished = producer->output ? dev_out(producer) : NULL;

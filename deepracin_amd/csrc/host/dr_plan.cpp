@@ -165,27 +165,43 @@ dR_Node* fire_pair(const dR_Node* concat) {
     return drhip_fire_slices(c3->ishape.s0, c3->ishape.s1, c3->shape.s2, c3->shape.s3, 0, 0) > 0 ? ins[1] : nullptr;
 }
 
-// The squeeze layer that is the only reader of a pair's outputs, directly or through a 3x3/2 max pooling it takes on load, and is itself
-// read by nothing but another such pair.
+inline bool tensor_hidden(const dR_Node* n) { return !tensor_wanted(n) && !n->outputBuf && n->next_layers; }
+
+// Is n a squeeze layer (taking `pooling` on load, where that is given) that nothing but a pair of expand layers reads?
+bool fire_squeeze(const dR_Node* n, const dR_Node* pooling, const std::map<const dR_Node*, dR_Node*>& pairOf) {
+    if (n->type != tConv2d || !tensor_hidden(n) || n->next_layers->length != 2) return false;
+    const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
+    if (c->algo != drConv1x1Gemm || c->drFusedAvgPool || c->drFusedPool || c->drAbsorbedBy || c->drPooledInput != pooling || !c->hasVariables) return false;
+    std::vector<dR_Node*> readers = nodes_of(n->next_layers);
+    if (readers[0] == readers[1]) return false;
+    const std::map<const dR_Node*, dR_Node*>::const_iterator a = pairOf.find(readers[0]), b = pairOf.find(readers[1]);
+    return a != pairOf.end() && b != pairOf.end() && a->second == b->second;
+}
+
+// The squeeze layer that is the only reader of a pair's outputs, directly or through a 3x3/2 max pooling it takes on load.
 dR_Node* fire_next(const dR_Node* concat, const std::map<const dR_Node*, dR_Node*>& pairOf, bool* pool) {
-    auto hidden = [](const dR_Node* n) { return !tensor_wanted(n) && !n->outputBuf && n->next_layers; };
-    if (!hidden(concat) || concat->next_layers->length != 1) return nullptr;
+    if (!tensor_hidden(concat) || concat->next_layers->length != 1) return nullptr;
     dR_Node* n = nodes_of(concat->next_layers)[0];
     *pool = n->type == tPooling;
     const dR_Node* pooling = *pool ? n : nullptr;
     if (pooling) {
-        if (!hidden(pooling) || pooling->next_layers->length != 1) return nullptr;
+        if (!tensor_hidden(pooling) || pooling->next_layers->length != 1) return nullptr;
         n = nodes_of(pooling->next_layers)[0];
     }
-    if (n->type != tConv2d || !hidden(n) || n->next_layers->length != 2) return nullptr;
-    const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
-    if (c->algo != drConv1x1Gemm || c->drFusedAvgPool || c->drFusedPool || c->drAbsorbedBy || c->drPooledInput != pooling || !c->hasVariables) return nullptr;
-    std::vector<dR_Node*> readers = nodes_of(n->next_layers);
-    if (readers[0] == readers[1]) return nullptr;
-    const std::map<const dR_Node*, dR_Node*>::const_iterator a = pairOf.find(readers[0]), b = pairOf.find(readers[1]);
-    return a != pairOf.end() && b != pairOf.end() && a->second == b->second ? n : nullptr;
+    return fire_squeeze(n, pooling, pairOf) ? n : nullptr;
 }
 
+// The squeeze layer behind a first layer and its pooling that has all its input channels in one workgroup of theirs.
+dR_Node* first_layer_squeeze(const dR_Node* n, const std::map<const dR_Node*, dR_Node*>& pairOf) {
+    if (n->type != tConv2d || !((const dR_Conv2d_Data*)n->layer)->drFusedPool) return nullptr;
+    const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
+    if (c->algo != drConvDirect || c->shape.s2 < 2 || c->shape.s3 > 64) return nullptr;
+    const dR_Node* pooling = nodes_of(n->next_layers)[0];
+    if (!tensor_hidden(pooling) || pooling->next_layers->length != 1) return nullptr;
+    dR_Node* squeeze = nodes_of(pooling->next_layers)[0];
+    return fire_squeeze(squeeze, nullptr, pairOf) && ((const dR_Conv2d_Data*)squeeze->layer)->shape.s3 <= 64 &&
+           (long long)(pooling->oshape.s0 + 1) * (pooling->oshape.s1 + 1) * 64 < (1ll << 28) ? squeeze : nullptr;
+}
 }  // namespace
 
 extern "C" {
@@ -366,14 +382,21 @@ gboolean dR_planBuffers(dR_Graph* net) {
     for (dR_Node* n : sched)
         if (n->type == tConv2d) {
             dR_Conv2d_Data* c = (dR_Conv2d_Data*)n->layer;
-            c->drFire = c->drFirePool = FALSE;
-            c->drFireNext = c->drFireFrom = nullptr;
+            c->drFire = c->drFirePool = c->drByPixel = FALSE;
+            c->drFireNext = c->drFireFrom = c->drSqueezeNext = nullptr;
         }
     const char* fuseFire = getenv("DR_FUSE_FIRE");
     if (!(fuseFire && strcmp(fuseFire, "0") == 0)) {
         std::map<const dR_Node*, dR_Node*> pairOf;              // either layer of a pair -> its 3x3 layer
         for (dR_Node* n : sched)
             if (dR_Node* e3 = fire_pair(n)) pairOf[e3] = pairOf[((dR_Conv2d_Data*)e3->layer)->drAbsorbed1x1] = e3;
+        auto pair_behind = [&](dR_Node* squeeze) { return (dR_Conv2d_Data*)pairOf[nodes_of(squeeze->next_layers)[0]]->layer; };
+        for (dR_Node* n : sched)
+            if (dR_Node* squeeze = first_layer_squeeze(n, pairOf)) {
+                ((dR_Conv2d_Data*)n->layer)->drSqueezeNext = squeeze;
+                ((dR_Conv2d_Data*)squeeze->layer)->drFireFrom = n;
+                pair_behind(squeeze)->drFire = TRUE;            // (reads sums, whether it takes a layer along or not)
+            }
         for (dR_Node* n : sched) {
             dR_Node* e3 = fire_pair(n);
             bool pool = false;
@@ -388,7 +411,18 @@ gboolean dR_planBuffers(dR_Graph* net) {
             c3->drFireNext = next;
             c3->drFirePool = pool;
             ((dR_Conv2d_Data*)next->layer)->drFireFrom = e3;
-            ((dR_Conv2d_Data*)pairOf[nodes_of(next->next_layers)[0]]->layer)->drFire = TRUE;       // (reads sums, whether it takes a layer along or not)
+            pair_behind(next)->drFire = TRUE;
+        }
+        // The last pair of a chain in front of a 1x1 layer and a global average: by pixel
+        for (dR_Node* n : sched) {
+            dR_Node* e3 = fire_pair(n);
+            if (!e3 || !tensor_hidden(n) || n->next_layers->length != 1) continue;
+            dR_Conv2d_Data* c3 = (dR_Conv2d_Data*)e3->layer;
+            dR_Node* reader = nodes_of(n->next_layers)[0];
+            if (!c3->drFire || c3->drFireNext || reader->type != tConv2d || (long long)n->oshape.s0 * n->oshape.s1 * n->oshape.s2 >= (1ll << 28)) continue;
+            dR_Conv2d_Data* c = (dR_Conv2d_Data*)reader->layer;
+            if (!c->drFusedAvgPool || c->shape.s2 > 1024 || c->shape.s3 > 65535) continue;
+            c3->drByPixel = c->drByPixel = TRUE;
         }
     }
     auto root_of = [&](dR_Node* n, int* offset) {

@@ -179,6 +179,11 @@ int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, floa
  * pooling kernel of such a pair (src/dR_nodes_conv2d.c:481-773, src/dR_nodes_pooling.c:277-401). */
 int drhip_conv3x3_pool3s2_f32(const float* in, const float* w, const float* bias, float* out,
                               int W, int H, int I, int O, int strideX, int strideY, int relu, void* stream);
+/* The same with a 1x1 layer of Sn channels (O and Sn at most 64) behind the pooling: out holds that layer's sums without bias and
+ * activation, [pixel][Sn rounded up to 16], for a reader that takes one slice of such sums (drhip_fire_f32).  wn: its filters as
+ * drhip_conv1x1_pixels_layout_f32 lays them out for I = O rounded up to 32 (64 above 32), rows that do not exist zero; out and wn 16-byte aligned. */
+int drhip_conv3x3_pool3s2_squeeze_f32(const float* in, const float* w, const float* bias, const float* wn, float* out,
+                                      int W, int H, int I, int O, int Sn, int strideX, int strideY, int relu, void* stream);
 
 /* Winograd F(2x2,3x3) filter transform U = G g G^T for every (c,o).  Runs once per layer at
  * dR_prepare time.  U holds drhip_conv3x3_winograd_filter_floats(I,O) floats in the layout the MFMA
@@ -264,6 +269,12 @@ int drhip_conv1x1_f32(const float* in, const float* w, const float* bias, float*
 int drhip_conv1x1_poolsum_slices(int P);
 int drhip_conv1x1_poolsum_f32(const float* in, const float* w, const float* bias, float* partials,
                               int P, int I, int O, int relu, void* stream);
+/* drhip_conv1x1_poolsum_f32 for an input by pixel, in [P][I] (I a multiple of 64, at most 1024; 16-byte aligned), with filters laid
+ * out for it once: F = ceil(O/16) * I * 16 floats, 16-byte aligned, from w [I][O].  partials[t*O + o]: tiles of
+ * drhip_conv1x1_pixels_tile(P) pixels. */
+int drhip_conv1x1_pixels_tile(int P);
+int drhip_conv1x1_pixels_layout_f32(const float* w /* [I][O] */, float* F, int I, int O, void* stream);
+int drhip_conv1x1_pixels_poolsum_f32(const float* in, const float* F, const float* bias, float* partials, int P, int I, int O, int relu, void* stream);
 /* A 3x3 / stride-2 max pooling followed by a 1x1 convolution, without the pooled tensor in between:
  * in is the pooling's input [I][Hin][Win]; the convolution works on the pooled map of
  * ceil(Win/2) x ceil(Hin/2) pixels, whose samples it takes while loading (maximum over the window
@@ -283,7 +294,7 @@ int drhip_conv1x1_pick_variant(int P, int I, int O);
  * its squeeze layer) and the squeeze layer of the next module (1x1, Sn channels, on both outputs, 1x1 layer's first), with
  * pool != 0 behind a 3x3 / stride-2 max pooling of them (rules as drhip_pool_f32).  out: that layer's sums without bias and
  * activation, [slices][pixel][Sn rounded up to 16] with slices = drhip_fire_slices, to be added by the reader;
- * Sn = 0: the expand outputs themselves, [2E][H][W].  in: a plain tensor [S][H][W] (slicesIn = 0; not with pool or
+ * Sn = 0: the expand outputs themselves, [2E][H][W] or, with pixels != 0, [H][W][2E].  in: a plain tensor [S][H][W] (slicesIn = 0; not with pool or
  * Sn = 0) or the sums another launch has left, with the bias (S rounded up to 16, 16-byte
  * aligned) and activation that belong to them.  drhip_fire_slices is 0 where a shape is not covered
  * (S and Sn up to 64, E a multiple of 32).  bank: laid out once, on the host, from the layers' filters as they are handed over
@@ -295,7 +306,7 @@ size_t drhip_fire_partials_floats(int W, int H, int S, int E, int Sn, int pool);
 int    drhip_fire_layout_f32(const float* w1, const float* w3, const float* b1, const float* b3, const float* wn, float* bank,
                              int W, int H, int S, int E, int Sn, int pool);
 int    drhip_fire_f32(const float* in, int slicesIn, const float* inBias, int inRelu, const float* bank, float* out,
-                      int W, int H, int S, int E, int Sn, int pool, int relu, void* stream);
+                      int W, int H, int S, int E, int Sn, int pool, int relu, int pixels, void* stream);
 
 /* ---- pooling ----------------------------------------------------------------------------------
  * out dims = ceil(in/stride) per axis; window anchored at (x*stx, y*sty, z*stz); samples outside

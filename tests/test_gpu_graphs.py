@@ -247,6 +247,47 @@ def test_fire_modules_in_a_chain(oracle, gpu, chain):
     assert rel_err(res["1"], res["0"]) <= 2e-6 * len(modules)
 
 
+@pytest.mark.parametrize("w,h,cin,first,squeeze,expand,classes,bias", [
+    (91, 74, 3, 64, 16, 64, 1000, True),        # SqueezeNet's ends around one module; odd maps
+    (18, 14, 4, 20, 33, 32, 17, False),         # ragged channels, one block of pooled pixels and a bit
+    (132, 260, 2, 64, 64, 256, 10, True),       # 33 x 65 pixels: tiles of 32 in front of the average
+    (24, 10, 1, 8, 8, 32, 5, True),             # one input channel: the squeeze layer stays a kernel of its own
+], ids=lambda v: str(v))
+def test_fire_chain_with_both_ends(oracle, gpu, w, h, cin, first, squeeze, expand, classes, bias):
+    """First layer, pooling and squeeze layer in one launch in front of a module, and behind it a 1x1 layer with a global average
+    that reads the module's outputs pixel by pixel: against the oracle, and against the kernels apart."""
+    st = configs._Streams(78)
+    spec = [{"op": "feed", "shape": (w, h, cin)}, configs._conv(st, 0, 3, cin, first, stride=2, bias=bias), configs._maxpool(1, 3, 2),
+            configs._conv(st, 2, 1, first, squeeze, bias=bias), configs._conv(st, 3, 1, squeeze, expand, bias=bias), configs._conv(st, 3, 3, squeeze, expand, bias=bias),
+            {"op": "concat", "ins": [4, 5], "dim": 2}, configs._conv(st, 6, 1, 2 * expand, classes, bias=bias)]
+    wp, hp = -(-(w // 2) // 2), -(-(h // 2) // 2)
+    spec += [{"op": "pool", "in": 7, "window": (wp, hp, 1), "stride": (wp, hp, 1), "kind": 1}, {"op": "softmax", "in": 8}]
+    feeds = {0: configs.image_input(st, w, h, cin, 2.0) - np.float32(1)}
+    want = oracle.run_spec(spec, feeds)
+    res = {}
+    for flag in ("1", "0"):
+        os.environ["DR_FUSE_FIRE"] = flag
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, [9, 8])
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], feeds[0])
+                dr.graph_config(g).profilingGPU = 1
+                assert g.lib.dR_apply(g.ptr)
+                silent = dr.node_struct(nodes[3]).drLastKernelMs == 0.0
+                dr.graph_config(g).profilingGPU = 0
+                assert g.lib.dR_apply(g.ptr)
+                res[flag] = configs.fetch_chw(g)
+        finally:
+            os.environ.pop("DR_FUSE_FIRE", None)
+        assert silent == (flag == "1" and cin > 1)
+        assert_close(res[flag][1].reshape(-1), want[8].reshape(-1), "average, DR_FUSE_FIRE=%s" % flag, terms=4096)
+        assert np.abs(res[flag][0].reshape(-1) - want[9].reshape(-1)).max() <= 1e-5
+    # another order of the same sums
+    assert rel_err(res["1"][1], res["0"][1]) <= 5e-6
+
+
 def test_fc_chain_fused(oracle, gpu):
     """FC -> FC -> softmax: the finishing kernels of the two GEMVs disappear into their consumers
     (3 launches instead of 5) and the probabilities do not change by a bit."""
