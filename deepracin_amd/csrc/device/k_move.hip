@@ -18,11 +18,17 @@ copy3d_kernel(const float* __restrict__ src, int sW, int sH, int sx0, int sy0, i
     }
 }
 
+// Up to four tensors into one: a picture whose channels have a mean of their own each is three of them, and took three slices and
+// three of these, 14 us of launches in a row (one: 2.4).
+struct ScalarOps { const float* x[4]; size_t n[4], at[4]; int op[4]; float s[4]; };
+
 __global__ void __launch_bounds__(256)
-scalar_op_kernel(const float* __restrict__ x, float* __restrict__ y, size_t n, int op, float s) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) {
+scalar_op_kernel(ScalarOps ops, float* __restrict__ y) {
+    const int k = blockIdx.y, op = ops.op[k];
+    const float* __restrict__ x = ops.x[k];
+    const float s = ops.s[k];
+    float* const d = y + ops.at[k];
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < ops.n[k]; i += (size_t)gridDim.x * 256) {
         const float v = x[i];
         float r;
         switch (op) {
@@ -36,7 +42,7 @@ scalar_op_kernel(const float* __restrict__ x, float* __restrict__ y, size_t n, i
             case 7: r = s; break;
             default: r = powf(v, s); break;
         }
-        y[i] = r;
+        d[i] = r;
     }
 }
 
@@ -61,13 +67,25 @@ extern "C" int drhip_copy3d_f32(const float* src, int sW, int sH, int sx0, int s
     return launched("copy3d_kernel");
 }
 
+extern "C" int drhip_scalar_ops_f32(int count, const float* const* x, const size_t* n, const int* op, const float* s, float* y, void* stream) {
+    DRHIP_REQUIRE(count >= 1 && count <= 4 && x && n && op && s && y, "drhip_scalar_ops_f32: %d operations", count);
+    ScalarOps ops = {};
+    size_t at = 0, most = 0;
+    for (int k = 0; k < count; ++k) {
+        DRHIP_REQUIRE(x[k], "drhip_scalar_op_f32: NULL tensor");
+        DRHIP_REQUIRE(op[k] >= 0 && op[k] <= 8, "drhip_scalar_op_f32: unknown op %d", op[k]);
+        ops.x[k] = x[k]; ops.n[k] = n[k]; ops.at[k] = at; ops.op[k] = op[k]; ops.s[k] = s[k];
+        at += n[k];
+        most = n[k] > most ? n[k] : most;
+    }
+    if (most == 0) return DRHIP_OK;
+    size_t blocks = (most + 255) / 256;
+    if (blocks > (size_t)16 * num_cu()) blocks = (size_t)16 * num_cu();
+    launch(scalar_op_kernel, dim3((unsigned)blocks, count), dim3(256), 0, as_stream(stream), ops, y);
+    return launched("scalar_op_kernel");
+}
+
 extern "C" int drhip_scalar_op_f32(const float* x, float* y, size_t n, int op, float s, void* stream) {
     DRHIP_REQUIRE(x && y, "drhip_scalar_op_f32: NULL tensor");
-    DRHIP_REQUIRE(op >= 0 && op <= 8, "drhip_scalar_op_f32: unknown op %d", op);
-    if (n == 0) return DRHIP_OK;
-    const int block = 256;
-    size_t blocks = (n + block - 1) / block;
-    if (blocks > (size_t)16 * num_cu()) blocks = (size_t)16 * num_cu();
-    launch(scalar_op_kernel, dim3((unsigned)blocks), dim3(block), 0, as_stream(stream), x, y, n, op, s);
-    return launched("scalar_op_kernel");
+    return drhip_scalar_ops_f32(1, &x, &n, &op, &s, y, stream);
 }

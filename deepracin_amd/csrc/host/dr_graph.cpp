@@ -311,6 +311,8 @@ static bool tensor_fused_away(const dR_Node* n) {
         const dR_Node* from = ((const dR_Conv2d_Data*)c->layer)->drFireFrom;
         return ((const dR_Conv2d_Data*)c->layer)->drPooledInput == n || (from && ((const dR_Conv2d_Data*)from->layer)->drSqueezeNext);
     }
+    if (n->type == tSlice) return ((const dR_Slice_Data*)n->layer)->drReadThrough;
+    if (n->type == tElemWise1Op) return ((const dR_ElemWise1Op_Data*)n->layer)->drInConcat;     // (not stored yet where a debug layer is read)
     if (n->type == tFullyConnected) return ((const dR_FC_Data*)n->layer)->drDeferReduce && !n->output;
     return false;
 }

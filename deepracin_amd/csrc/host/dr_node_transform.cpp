@@ -56,6 +56,27 @@ gboolean concat_schedule(dR_Graph* net, dR_Node* node) {
 
 gboolean concat_compute(dR_Graph* net, dR_Node* node) {
     dR_Concat_Data* c = concat_of(node);
+    if (c->drScalarOps) {              // the producers' work, read through the slices in front of them
+        const float* x[4];
+        size_t n[4];
+        int op[4], k = 0;
+        float s[4];
+        for (dR_Node* p : nodes_of(node->previous_layers)) {
+            const dR_ElemWise1Op_Data* e = (const dR_ElemWise1Op_Data*)p->layer;
+            dR_Node* in = first_input(p);
+            size_t skip = 0;
+            if (in->type == tSlice && ((const dR_Slice_Data*)in->layer)->drReadThrough) {
+                const dR_Slice_Data* slice = (const dR_Slice_Data*)in->layer;
+                skip = (size_t)slice->origin.s2 * slice->ishape.s0 * slice->ishape.s1;
+                in = first_input(in);
+            }
+            x[k] = dev_out(in) + skip;
+            n[k] = (size_t)out_volume(p);
+            op[k] = (int)e->op;
+            s[k++] = e->scalar;
+        }
+        return !device_failed(net, drhip_scalar_ops_f32(k, x, n, op, s, dev_out(node), stream_of(net)), "deepRACIN:elemwise1op");
+    }
     if (c->drFused) return TRUE;       // the producers already wrote into this node's buffer
     int off[3] = { 0, 0, 0 };
     for (dR_Node* in : nodes_of(node->previous_layers)) {
@@ -112,6 +133,7 @@ gboolean slice_propagate(dR_Graph* net, dR_Node* node) {
 
 gboolean slice_compute(dR_Graph* net, dR_Node* node) {
     dR_Slice_Data* s = slice_of(node);
+    if (s->drReadThrough) return TRUE;
     int rc = drhip_copy3d_f32(dev_out(first_input(node)), s->ishape.s0, s->ishape.s1, s->origin.s0, s->origin.s1, s->origin.s2,
                               dev_out(node), s->oshape.s0, s->oshape.s1, 0, 0, 0,
                               s->oshape.s0, s->oshape.s1, s->oshape.s2, stream_of(net));
@@ -151,6 +173,7 @@ gboolean ew_propagate(dR_Graph* net, dR_Node* node) {
 
 gboolean ew_compute(dR_Graph* net, dR_Node* node) {
     dR_ElemWise1Op_Data* e = ew_of(node);
+    if (e->drInConcat) return TRUE;
     int rc = drhip_scalar_op_f32(dev_out(first_input(node)), dev_out(node), (size_t)out_volume(node), (int)e->op, e->scalar, stream_of(net));
     return !device_failed(net, rc, "deepRACIN:elemwise1op");
 }

@@ -378,6 +378,29 @@ gboolean dR_planBuffers(dR_Graph* net) {
             ((dR_Pooling_Data*)pool->layer)->drFused = TRUE;
         }
     }
+    // Scalar operations that fill a concat between them: one launch, and whole channels are taken from the tensor that they are
+    // sliced from (DR_FUSE_SCALAR=0 keeps them apart)
+    for (dR_Node* n : sched) {
+        if (n->type == tSlice) ((dR_Slice_Data*)n->layer)->drReadThrough = FALSE;
+        if (n->type == tElemWise1Op) ((dR_ElemWise1Op_Data*)n->layer)->drInConcat = FALSE;
+        if (n->type == tConcat) ((dR_Concat_Data*)n->layer)->drScalarOps = FALSE;
+    }
+    const char* fuseScalar = getenv("DR_FUSE_SCALAR");
+    for (dR_Node* n : sched) {
+        if (n->type != tConcat || !((dR_Concat_Data*)n->layer)->drFused || (fuseScalar && strcmp(fuseScalar, "0") == 0)) continue;
+        std::vector<dR_Node*> ins = nodes_of(n->previous_layers);
+        bool all = ins.size() >= 2 && ins.size() <= 4;
+        for (dR_Node* p : ins) all = all && p->type == tElemWise1Op;
+        if (!all) continue;
+        ((dR_Concat_Data*)n->layer)->drScalarOps = TRUE;
+        for (dR_Node* p : ins) {
+            ((dR_ElemWise1Op_Data*)p->layer)->drInConcat = TRUE;
+            dR_Node* slice = nodes_of(p->previous_layers)[0];
+            if (slice->type != tSlice || !tensor_hidden(slice) || slice->next_layers->length != 1) continue;
+            dR_Slice_Data* s = (dR_Slice_Data*)slice->layer;
+            s->drReadThrough = s->origin.s0 == 0 && s->origin.s1 == 0 && s->oshape.s0 == s->ishape.s0 && s->oshape.s1 == s->ishape.s1;
+        }
+    }
     // Fire modules in a chain (after the fusions above, on which the rule rests)
     for (dR_Node* n : sched)
         if (n->type == tConv2d) {
@@ -457,6 +480,14 @@ gboolean dR_planBuffers(dR_Graph* net) {
             Root& rp = touch(root_of(p, nullptr));
             rp.lastUse = std::max(rp.lastUse, n->drSchedulePos);
         }
+        // scalar operations done by the concat behind them read what they, or the slices in front of them, are made of
+        if (n->type == tConcat && ((dR_Concat_Data*)n->layer)->drScalarOps)
+            for (dR_Node* p : nodes_of(n->previous_layers)) {
+                dR_Node* in = nodes_of(p->previous_layers)[0];
+                if (in->type == tSlice && ((dR_Slice_Data*)in->layer)->drReadThrough) in = nodes_of(in->previous_layers)[0];
+                Root& rp = touch(root_of(in, nullptr));
+                rp.lastUse = std::max(rp.lastUse, n->drSchedulePos);
+            }
         // a convolution that pools while loading reads the tensor in front of the pooling node
         if (n->type == tConv2d && ((dR_Conv2d_Data*)n->layer)->drPooledInput) {
             for (dR_Node* p : nodes_of(((dR_Conv2d_Data*)n->layer)->drPooledInput->previous_layers)) {

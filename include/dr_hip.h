@@ -393,6 +393,8 @@ int drhip_copy3d_f32(const float* src, int sW, int sH, int sx0, int sy0, int sz0
                      int w, int h, int c, void* stream);
 /* y = f(x, s); op numbering = dR_ElemWise1OperationType: 0 x+s, 1 x-s, 2 x*s, 3 x/s, 4 log x, 5 exp x,
  * 6 sqrt x, 7 s, 8 pow(x,s)  (`addScalar` ... `powScalar`, Kernels/dR_math.cl:170-341) */
+/* Several of them, each on n[k] elements, one after the other into y: one launch for up to 4. */
+int drhip_scalar_ops_f32(int count, const float* const* x, const size_t* n, const int* op, const float* s, float* y, void* stream);
 int drhip_scalar_op_f32(const float* x, float* y, size_t n, int op, float s, void* stream);
 
 #ifdef __cplusplus

@@ -288,6 +288,54 @@ def test_fire_chain_with_both_ends(oracle, gpu, w, h, cin, first, squeeze, expan
     assert rel_err(res["1"][1], res["0"][1]) <= 5e-6
 
 
+@pytest.mark.parametrize("case", ["means", "ragged", "mixed", "shared"])
+def test_scalar_operations_in_front_of_a_concat(oracle, gpu, case):
+    """Slices, scalar operations and the concat they fill in one launch (DR_FUSE_SCALAR=0: kernels apart): the same numbers."""
+    w, h, c = (23, 17, 5) if case != "ragged" else (1, 1, 3)
+    spec = [{"op": "feed", "shape": (w, h, c)}]
+    def ew(src, kind, value):
+        spec.append({"op": "scalar", "in": src, "kind": kind, "value": value})
+        return len(spec) - 1
+    def part(origin, shape):
+        spec.append({"op": "slice", "in": 0, "origin": origin, "shape": shape})
+        return len(spec) - 1
+    if case == "mixed":                         # two channels, a box that has to be copied, and a tensor that is no slice
+        base = ew(0, 2, 3.0)
+        spec.append({"op": "slice", "in": base, "origin": (0, 0, 1), "shape": (w, h, 2)})
+        ins = [ew(len(spec) - 1, 0, 1.5), ew(base, 1, 0.25)]
+    elif case == "shared":                      # a slice with another reader stays
+        one = part((0, 0, 2), (w, h, 1))
+        ins = [ew(one, 3, 7.0), ew(one, 7, 2.0), ew(part((0, 0, 0), (w, h, 1)), 2, -1.0)]
+    else:
+        ins = [ew(part((0, 0, k), (w, h, 1)), 1, 10.0 * k) for k in (2, 0, 1)]
+    spec.append({"op": "concat", "ins": ins, "dim": 2}); cat = len(spec) - 1
+    if case == "mixed":
+        spec.append({"op": "slice", "in": 0, "origin": (1, 2, 0), "shape": (5, 4, 2)}); box = len(spec) - 1
+        a, b = ew(box, 1, 4.0), ew(box, 0, 4.0)
+        spec.append({"op": "concat", "ins": [a, b], "dim": 2})
+    outs = [cat] if case != "mixed" else [cat, len(spec) - 1]
+    feeds = {0: configs.image_input(configs._Streams(79), w, h, c, 255.0)}
+    want = oracle.run_spec(spec, feeds)
+    for flag in ("1", "0"):
+        os.environ["DR_FUSE_SCALAR"] = flag
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, outs)
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], feeds[0])
+                dr.graph_config(g).profilingGPU = 1
+                assert g.lib.dR_apply(g.ptr)
+                assert (dr.node_struct(nodes[ins[0]]).drLastKernelMs == 0.0) == (flag == "1")
+                dr.graph_config(g).profilingGPU = 0
+                assert g.lib.dR_apply(g.ptr)
+                got = configs.fetch_chw(g)
+        finally:
+            os.environ.pop("DR_FUSE_SCALAR", None)
+        for x, i in zip(got, outs):
+            assert np.array_equal(x, want[i]) or np.abs(x - want[i]).max() <= 2.0 ** -23 * np.abs(want[i]).max()     # (a division's last bit)
+
+
 def test_fc_chain_fused(oracle, gpu):
     """FC -> FC -> softmax: the finishing kernels of the two GEMVs disappear into their consumers
     (3 launches instead of 5) and the probabilities do not change by a bit."""
