@@ -23,6 +23,8 @@
 // OpenCL device; any partitioning gives the same sum up to fp32 rounding.
 #include "drhip_common.hpp"
 
+#include <algorithm>
+
 namespace drhip {
 
 constexpr int kFcThreads = 256;
@@ -57,7 +59,10 @@ static FcPlan fc_plan(int K, int N) {
     // layer that sums them while it loads its input (4096 x 4096 behind 16 instead of 56 slices: 12.2 against 13.3 us).
     const int target = num_cu();                     // workgroups wanted in flight
     int slices = ceil_div(target, p.panels);
-    const int maxSlices = ceil_div(K, 4 * kWave);    // at least 256 rows per workgroup (4096 x 4096: 13.7 us with 16 slices, 14.8 with 32)
+    // at least 256 rows per workgroup (4096 x 4096: 13.7 us with 16 slices, 14.8 with 32).  A matrix of at most 4 MiB is a few workgroups
+    // whose time is that of their trips to memory: 64 rows, 16 a wave, are one, and 32 slices one for the reader (1568 x 128: 5.2 us with 7
+    // slices, 2.5 with 25; 192 x 1000 4.9 with 1, 3.2 with 3).
+    const int maxSlices = (long long)K * N <= 1 << 20 ? std::min(32, ceil_div(K, kWave)) : ceil_div(K, 4 * kWave);
     if (slices > maxSlices) slices = maxSlices;
     if (slices < 1) slices = 1;
     p.rowsPerSlice = ceil_div(ceil_div(K, slices), kWave) * kWave;   // whole chunks
