@@ -104,6 +104,16 @@ __device__ inline void store_through(float* p, float v) {
     __hip_atomic_store((unsigned*)p, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A value for the host (drhip_push), and, by every lane of the workgroup behind its last one, the flag that tells it of them.
+__device__ inline void push_value(const drhip_push& p, unsigned at, float v) {
+    __hip_atomic_store((unsigned*)p.host + at, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ inline void push_flag(const drhip_push& p) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this lane's stores have been accepted
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(p.flag, p.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Element `row` of an activation vector that a split GEMV left as partial sums: slices added in
 // order, then bias and ReLU -- bit for bit what the GEMV's finishing kernel stores.
 __device__ inline float deferred_element(const drhip_deferred_vec& d, int row) {
@@ -119,14 +129,26 @@ __device__ inline float deferred_element(const drhip_deferred_vec& d, int row) {
 #pragma unroll
         for (int u = 0; u < 32; ++u) s += v[u];
     }
-    for (; sl + 16 <= d.slices; sl += 16) {         // (a GEMV that fills the chip leaves 16 slices: one round, not two)
+    for (; sl + 16 == d.slices; sl += 16) {         // (a GEMV that fills the chip leaves 16 slices: one round, not two)
         float v[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) v[u] = pp[(size_t)(sl + u) * d.n];
 #pragma unroll
         for (int u = 0; u < 16; ++u) s += v[u];
     }
-    for (; sl < d.slices; sl += 8) {                // the ragged end too: clamped loads, zeros by select
+    if (d.slices - sl > 8) {                        // the ragged end in one round as well: clamped loads, zeros by select
+        float v[32];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = pp[(size_t)min(sl + u, d.slices - 1) * d.n];
+        if (d.slices - sl > 16) {
+#pragma unroll
+            for (int u = 16; u < 32; ++u) v[u] = pp[(size_t)min(sl + u, d.slices - 1) * d.n];
+        }
+#pragma unroll
+        for (int u = 0; u < 32; ++u) s = (sl + u < d.slices) ? s + v[u] : s;
+        sl = d.slices;
+    }
+    for (; sl < d.slices; sl += 8) {
         float v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) v[u] = pp[(size_t)min(sl + u, d.slices - 1) * d.n];

@@ -565,6 +565,24 @@ int drhip_download_staged(void* handle, void* dst, const void* src, size_t off, 
     return DRHIP_OK;
 }
 
+int drhip_push_begin(void* handle, size_t floats, drhip_push* push) {
+    Staging* s = (Staging*)handle;
+    if (!s || !push || s->spinUs <= 0 || floats * sizeof(float) > kStagingDownBytes) return DRHIP_EINVAL;      // (no message: the caller takes the other way)
+    *push = drhip_push{(float*)s->down, 0, 0xffffffffu, flag_of(s), next_flag_value(s)};
+    return DRHIP_OK;
+}
+
+int drhip_push_collect(void* handle, const drhip_push* push, int count, float* const* dst, const unsigned* at, const size_t* floats, void* stream) {
+    Staging* s = (Staging*)handle;
+    DRHIP_REQUIRE(s && push && push->host == (float*)s->down && count >= 0 && (count == 0 || (dst && at && floats)), "drhip_push_collect: bad arguments");
+    if (int rc = wait_for_flag(s, push->value, as_stream(stream))) return rc;
+    for (int k = 0; k < count; ++k) {
+        DRHIP_REQUIRE(dst[k] && (at[k] + floats[k]) * sizeof(float) <= kStagingDownBytes, "drhip_push_collect: array %d", k);
+        memcpy(dst[k], push->host + at[k], floats[k] * sizeof(float));
+    }
+    return DRHIP_OK;
+}
+
 int drhip_download_staged_many(void* handle, int count, float* const* dst, const float* const* src, const size_t* floats, void* stream) {
     Staging* s = (Staging*)handle;
     DRHIP_REQUIRE(s && count >= 0 && (count == 0 || (dst && src && floats)), "drhip_download_staged_many: NULL pointer");

@@ -46,7 +46,7 @@ __device__ inline float block_reduce(float v, float* red) {
 // caller wants to read the logits too).
 template <bool SMALL>
 __global__ void __launch_bounds__(kSoftmaxThreads)
-softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef) {     // no __restrict__: x may become y
+softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef, drhip_push push) {    // no __restrict__: x may become y
     __shared__ float red[kSoftmaxThreads / kWave];
     const int tid = threadIdx.x;
     if (SMALL) {                                    // n <= kSoftmaxThreads * kSoftmaxRegs
@@ -64,6 +64,11 @@ softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef) {     /
                 if (i < n) xdef.finished[i] = v[u];
             }
         }
+        if (push.host && push.atInput != 0xffffffffu) {
+#pragma unroll
+            for (int u = 0; u < kSoftmaxRegs; ++u)
+                if (tid + u * kSoftmaxThreads < n) push_value(push, push.atInput + tid + u * kSoftmaxThreads, v[u]);
+        }
         float m = -FLT_MAX;
 #pragma unroll
         for (int u = 0; u < kSoftmaxRegs; ++u) m = fmaxf(m, v[u]);
@@ -79,7 +84,9 @@ softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef) {     /
         for (int u = 0; u < kSoftmaxRegs; ++u) {
             const int i = tid + u * kSoftmaxThreads;
             if (i < n) store_through(y + i, v[u] * inv);
+            if (push.host && i < n) push_value(push, push.at + i, v[u] * inv);
         }
+        if (push.host) push_flag(push);
         return;
     }
     if (xdef.partials) {
@@ -99,20 +106,94 @@ softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef) {     /
     for (int i = tid; i < n; i += kSoftmaxThreads) store_through(y + i, expf(x[i] - m) * inv);
 }
 
+// A small layer and the softmax behind it.  As a launch of its own such a layer is one or two workgroups that wait for one trip to
+// memory; here the waves that wait for the logits do it.  A thread has column n and every T-th row, so that neighbouring
+// threads read neighbouring weights, and the T sums of a column are added in order.
+// (128 -> 10 behind 25 slices: 2.8 + 2.8 us as two launches; a thumbnail classifier's call 44 -> 40 us, and 36 with its outputs on
+// their way to the host from here.)
+constexpr int kFcSoftmaxRows = 16;                  // rows of a thread under way
+constexpr int kFcSoftmaxGroups = 32;                // T at most
+__global__ void __launch_bounds__(kSoftmaxThreads)
+fc_softmax_kernel(const float* __restrict__ Wt, const float* x, const float* __restrict__ bias, float* z, float* y, int K, int N, int T, unsigned mulN, unsigned shN, int relu,
+                  drhip_deferred_vec xdef, drhip_push push) {
+    __shared__ float xs[1024], part[kSoftmaxThreads], red[kSoftmaxThreads / kWave];
+    const int tid = threadIdx.x;
+    const FastDiv nd = {(unsigned)N, mulN, shN};
+    const int g = fast_div(tid, nd), n = tid - g * N;
+    float w[kFcSoftmaxRows];
+    const float* column = Wt + n;
+#pragma unroll
+    for (int u = 0; u < kFcSoftmaxRows; ++u) w[u] = column[(size_t)min(g + u * T, K - 1) * N];
+    const float b = bias && tid < N ? bias[tid] : 0.0f;
+    const float xv = tid < K ? (xdef.partials ? deferred_element(xdef, tid) : x[tid]) : 0.0f;
+    if (tid < K) xs[tid] = xv;
+    __syncthreads();
+    float s = 0.0f;
+    for (int k0 = g; k0 < K; k0 += kFcSoftmaxRows * T) {
+#pragma unroll
+        for (int u = 0; u < kFcSoftmaxRows; ++u) s = k0 + u * T < K ? fmaf(w[u], xs[min(k0 + u * T, K - 1)], s) : s;
+        if (k0 + kFcSoftmaxRows * T < K) {
+#pragma unroll
+            for (int u = 0; u < kFcSoftmaxRows; ++u) w[u] = column[(size_t)min(k0 + (kFcSoftmaxRows + u) * T, K - 1) * N];
+        }
+    }
+    if (g < T) part[g * N + n] = s;
+    __syncthreads();
+    float v = -FLT_MAX;
+    if (tid < N) {
+        v = part[tid];
+        for (int k = 1; k < T; ++k) v += part[k * N + tid];
+        v += b;
+        if (relu) v = fmaxf(v, 0.0f);
+        if (z) z[tid] = v;
+        if (push.host && push.atInput != 0xffffffffu) push_value(push, push.atInput + tid, v);
+    }
+    if (xdef.partials && xdef.finished && tid < K) xdef.finished[tid] = xv;
+    const float m = block_reduce<true>(v, red);
+    const float e = tid < N ? expf(v - m) : 0.0f;
+    const float inv = 1.0f / block_reduce<false>(e, red);
+    if (tid < N) {
+        store_through(y + tid, e * inv);
+        if (push.host) push_value(push, push.at + tid, e * inv);
+    }
+    if (push.host) push_flag(push);
+}
+
 }  // namespace drhip
 
 using namespace drhip;
 
+extern "C" int drhip_fc_softmax_usable(int K, int N) { return K >= 1 && N >= 1 && K <= 1024 && N <= 1024 && K * N <= 32768; }
+
+extern "C" int drhip_fc_softmax_f32(const float* x, const drhip_deferred_vec* xdef, const float* Wt, const float* bias, float* z, float* y, int K, int N, int relu,
+                                    const drhip_push* push, void* stream) {
+    DRHIP_REQUIRE((x || xdef) && Wt && y && y != z, "drhip_fc_softmax_f32: NULL tensor");
+    DRHIP_REQUIRE(drhip_fc_softmax_usable(K, N), "drhip_fc_softmax_f32: %d -> %d is not covered", K, N);
+    DRHIP_REQUIRE(!xdef || (xdef->partials && xdef->slices > 0 && xdef->n == K), "drhip_fc_softmax_f32: deferred input must carry partial sums of a vector of length %d", K);
+    const drhip_deferred_vec none = {nullptr, nullptr, 0, 0, 0, nullptr, 0.0f};
+    const drhip_push nowhere = {nullptr, 0, 0, nullptr, 0};
+    const FastDiv nd = make_fastdiv(N);
+    const int most = kSoftmaxThreads / N, T = most < kFcSoftmaxGroups ? most : kFcSoftmaxGroups;
+    launch(fc_softmax_kernel, dim3(1), dim3(kSoftmaxThreads), 0, as_stream(stream), Wt, x, bias, z, y, K, N, T, nd.mul, nd.shift, relu, xdef ? *xdef : none, push ? *push : nowhere);
+    return launched("fc_softmax_kernel");
+}
+
 extern "C" int drhip_softmax_ex_f32(const float* x, const drhip_deferred_vec* xdef, float* y, int n, void* stream) {
+    return drhip_softmax_push_f32(x, xdef, y, n, nullptr, stream);
+}
+
+extern "C" int drhip_softmax_push_f32(const float* x, const drhip_deferred_vec* xdef, float* y, int n, const drhip_push* push, void* stream) {
     DRHIP_REQUIRE((x || xdef) && y, "drhip_softmax_f32: NULL tensor");
     DRHIP_REQUIRE(n > 0, "drhip_softmax_f32: n = %d", n);
     DRHIP_REQUIRE(!xdef || (xdef->partials && xdef->slices > 0 && xdef->n == n), "drhip_softmax_f32: deferred input must carry partial sums of a vector of length %d", n);
     DRHIP_REQUIRE(!xdef || xdef->finished != y, "drhip_softmax_f32: the finished logits and the probabilities need separate arrays");
+    DRHIP_REQUIRE(!push || n <= kSoftmaxThreads * kSoftmaxRegs, "drhip_softmax_push_f32: %d values are too many", n);
     const drhip_deferred_vec none = {nullptr, nullptr, 0, 0, 0, nullptr, 0.0f};
+    const drhip_push nowhere = {nullptr, 0, 0, nullptr, 0};
     if (n <= kSoftmaxThreads * kSoftmaxRegs)
-        launch(softmax_kernel<true>, dim3(1), dim3(kSoftmaxThreads), 0, as_stream(stream), x, y, n, xdef ? *xdef : none);
+        launch(softmax_kernel<true>, dim3(1), dim3(kSoftmaxThreads), 0, as_stream(stream), x, y, n, xdef ? *xdef : none, push ? *push : nowhere);
     else
-        launch(softmax_kernel<false>, dim3(1), dim3(kSoftmaxThreads), 0, as_stream(stream), x, y, n, xdef ? *xdef : none);
+        launch(softmax_kernel<false>, dim3(1), dim3(kSoftmaxThreads), 0, as_stream(stream), x, y, n, xdef ? *xdef : none, nowhere);
     return launched("softmax_kernel");
 }
 

@@ -313,7 +313,7 @@ static bool tensor_fused_away(const dR_Node* n) {
     }
     if (n->type == tSlice) return ((const dR_Slice_Data*)n->layer)->drReadThrough;
     if (n->type == tElemWise1Op) return ((const dR_ElemWise1Op_Data*)n->layer)->drInConcat;     // (not stored yet where a debug layer is read)
-    if (n->type == tFullyConnected) return ((const dR_FC_Data*)n->layer)->drDeferReduce && !n->output;
+    if (n->type == tFullyConnected) return ((const dR_FC_Data*)n->layer)->drInSoftmax || (((const dR_FC_Data*)n->layer)->drDeferReduce && !n->output);
     return false;
 }
 
@@ -410,6 +410,46 @@ gboolean dR_apply(dR_Graph* net) {
     }
     if (net->config->debugInfo) say("Done.\n\n");
     return TRUE;
+}
+
+// The node whose kernel makes every output of the pass: a softmax that is an output, with its finished input, where that is one too.
+static dR_Node* all_outputs_node(const dR_Graph* net) {
+    dR_Node* last = NULL;
+    for (dR_Node* n : nodes_of(net->output_layers))
+        if (n->type == tSoftmax) { if (last) return NULL; last = n; }
+    if (!last || last->oshape.s0 * last->oshape.s1 * last->oshape.s2 > 2048) return NULL;
+    const dR_Softmax_Data* s = (const dR_Softmax_Data*)last->layer;
+    for (dR_Node* n : nodes_of(net->output_layers))
+        if (n != last && n != s->drDeferredInput && n != s->drFcInput) return NULL;
+    return last;
+}
+
+gint dR_applyAndDownload(dR_Graph* net, gfloat** hosts, gint n) {
+    if (!net->prepared || n < 0 || (n > 0 && !hosts)) {
+        say("dR_applyAndDownload: the graph is not prepared, or no arrays were given\n");
+        return -1;
+    }
+    const char* replay = getenv("DR_HIPGRAPH");
+    const bool plain = net->drStaging && !net->config->profilingGPU && net->debugLayer < 0 && !net->drGraphExec && !(replay && strcmp(replay, "1") == 0);
+    dR_Node* last = plain && n >= net->output_layers->length ? all_outputs_node(net) : NULL;
+    drhip_push push;
+    const unsigned values = last ? (unsigned)(last->oshape.s0 * last->oshape.s1 * last->oshape.s2) : 0;
+    if (!last || drhip_push_begin(net->drStaging, 2 * (size_t)values, &push) != DRHIP_OK) return dR_apply(net) ? dR_downloadOutputs(net, hosts, n) : -1;
+    unsigned at[2];
+    size_t floats[2];
+    int k = 0;
+    for (dR_Node* node : nodes_of(net->output_layers)) {
+        at[k] = node == last ? 0 : values;
+        floats[k++] = values;
+        if (node != last) push.atInput = values;
+    }
+    net->drPush = &push;
+    net->drPushNode = last;
+    const gboolean ok = dR_apply(net);
+    net->drPush = NULL;
+    net->drPushNode = NULL;
+    if (!ok) return -1;
+    return device_failed(net, drhip_push_collect(net->drStaging, &push, k, hosts, at, floats, stream_of(net)), "dR_applyAndDownload") ? 0 : k;
 }
 
 void dR_cleanup(dR_Graph* net, gboolean cleanupcl) {

@@ -175,6 +175,7 @@ drhip_deferred_vec deferred_output_of(dR_Node* producer) {
 
 gboolean fc_compute(dR_Graph* net, dR_Node* node) {
     dR_FC_Data* f = fc_of(node);
+    if (f->drInSoftmax) return TRUE;
     drhip_deferred_vec xdef;
     if (f->drDeferredInput) xdef = deferred_output_of(f->drDeferredInput);
     int rc = drhip_fc_ex_f32(dev_out(first_input(node)), f->drDeferredInput ? &xdef : NULL, (const float*)f->weightsBuf,
@@ -241,10 +242,18 @@ gboolean softmax_propagate(dR_Graph* net, dR_Node* node) {
 
 gboolean softmax_compute(dR_Graph* net, dR_Node* node) {
     dR_Softmax_Data* s = (dR_Softmax_Data*)node->layer;
+    const drhip_push* push = net->drPushNode == node ? (const drhip_push*)net->drPush : NULL;
     drhip_deferred_vec xdef;
+    if (s->drFcInput) {
+        dR_FC_Data* f = fc_of(s->drFcInput);
+        if (f->drDeferredInput) xdef = deferred_output_of(f->drDeferredInput);
+        return !device_failed(net, drhip_fc_softmax_f32(dev_out(first_input(s->drFcInput)), f->drDeferredInput ? &xdef : NULL, (const float*)f->weightsBuf,
+                                                        f->useBias ? (const float*)f->biasBuf : NULL, s->drFcInput->output ? dev_out(s->drFcInput) : NULL, dev_out(node),
+                                                        f->shape.s0, f->shape.s1, f->activation == tReLU, push, stream_of(net)), "deepRACIN:softmax");
+    }
     if (s->drDeferredInput) xdef = deferred_output_of(s->drDeferredInput);
-    int rc = drhip_softmax_ex_f32(dev_out(first_input(node)), s->drDeferredInput ? &xdef : NULL, dev_out(node),
-                                  s->ishape.s0 * s->ishape.s1 * s->ishape.s2, stream_of(net));
+    int rc = drhip_softmax_push_f32(dev_out(first_input(node)), s->drDeferredInput ? &xdef : NULL, dev_out(node),
+                                    s->ishape.s0 * s->ishape.s1 * s->ishape.s2, push, stream_of(net));
     return !device_failed(net, rc, "deepRACIN:softmax");
 }
 

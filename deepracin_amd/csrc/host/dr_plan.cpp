@@ -319,8 +319,11 @@ gboolean dR_planBuffers(dR_Graph* net) {
     // FC -> FC and FC -> softmax: the consumer sums the producer's split-K partials while it loads
     // its input, the producer's finishing kernel is not launched (DR_FUSE_FC=0 keeps it).
     for (dR_Node* n : sched) {
-        if (n->type == tFullyConnected) { ((dR_FC_Data*)n->layer)->drDeferReduce = FALSE; ((dR_FC_Data*)n->layer)->drDeferredInput = nullptr; }
-        if (n->type == tSoftmax) ((dR_Softmax_Data*)n->layer)->drDeferredInput = nullptr;
+        if (n->type == tFullyConnected) {
+            ((dR_FC_Data*)n->layer)->drDeferReduce = ((dR_FC_Data*)n->layer)->drInSoftmax = FALSE;
+            ((dR_FC_Data*)n->layer)->drDeferredInput = nullptr;
+        }
+        if (n->type == tSoftmax) ((dR_Softmax_Data*)n->layer)->drDeferredInput = ((dR_Softmax_Data*)n->layer)->drFcInput = nullptr;
     }
     const char* fuseFc = getenv("DR_FUSE_FC");
     for (dR_Node* n : sched) {
@@ -328,8 +331,13 @@ gboolean dR_planBuffers(dR_Graph* net) {
         dR_FC_Data* fd = (dR_FC_Data*)n->layer;
         // an output node can defer too: its consumer stores the finished vector into its buffer
         if (n->outputBuf || !n->next_layers || n->next_layers->length != 1 || n->layerID == g_debugLayerAtPlanTime) continue;
-        if (drhip_fc_slices(fd->shape.s0, fd->shape.s1) <= 1) continue;
         dR_Node* c = nodes_of(n->next_layers)[0];
+        if (c->type == tSoftmax && drhip_fc_softmax_usable(fd->shape.s0, fd->shape.s1)) {       // a small layer: in the softmax's launch
+            fd->drInSoftmax = TRUE;
+            ((dR_Softmax_Data*)c->layer)->drFcInput = n;
+            continue;
+        }
+        if (drhip_fc_slices(fd->shape.s0, fd->shape.s1) <= 1) continue;
         if (c->type == tFullyConnected) ((dR_FC_Data*)c->layer)->drDeferredInput = n;
         else if (c->type == tSoftmax) ((dR_Softmax_Data*)c->layer)->drDeferredInput = n;
         else continue;
@@ -480,6 +488,12 @@ gboolean dR_planBuffers(dR_Graph* net) {
             Root& rp = touch(root_of(p, nullptr));
             rp.lastUse = std::max(rp.lastUse, n->drSchedulePos);
         }
+        // a softmax that computes the layer in front of it reads that layer's input
+        if (n->type == tSoftmax && ((dR_Softmax_Data*)n->layer)->drFcInput)
+            for (dR_Node* p : nodes_of(((dR_Softmax_Data*)n->layer)->drFcInput->previous_layers)) {
+                Root& rp = touch(root_of(p, nullptr));
+                rp.lastUse = std::max(rp.lastUse, n->drSchedulePos);
+            }
         // scalar operations done by the concat behind them read what they, or the slices in front of them, are made of
         if (n->type == tConcat && ((dR_Concat_Data*)n->layer)->drScalarOps)
             for (dR_Node* p : nodes_of(n->previous_layers)) {

@@ -126,6 +126,15 @@ void   drhip_interleaved_to_planes(float* planes, const float* src, size_t pixel
  * download area (at most 10), otherwise one after the other. */
 int    drhip_download_staged_many(void* handle, int count, float* const* dst_host, const float* const* src_dev, const size_t* floats, void* stream);
 
+/* Results that go to the host as they are made: the kernel that makes them stores them into the staging's download area as
+ * well, at `at`, and its input at `atInput` (0xffffffff: not), and raises the flag behind them.  drhip_push_begin prepares
+ * that for `floats` values in all (DRHIP_EINVAL: they do not fit, or flags are not watched), a drhip_*_push_f32 call takes it, and
+ * drhip_push_collect waits for the flag and copies out, dst[k] = floats[k] values from at[k].  Saves the copy kernel's launch
+ * behind the last layer of a pass. */
+typedef struct drhip_push { float* host; unsigned at, atInput; unsigned* flag; unsigned value; } drhip_push;
+int drhip_push_begin(void* handle, size_t floats, drhip_push* push);
+int drhip_push_collect(void* handle, const drhip_push* push, int count, float* const* dst_host, const unsigned* at, const size_t* floats, void* stream);
+
 /* ---- convolution ------------------------------------------------------------------------------
  * Common meaning: in [I][H][W]; out [O][Ho][Wo] with Wo = W/strideX, Ho = H/strideY (floor);
  * zero padding of kw/2, kh/2; bias may be NULL; relu != 0 applies max(v,0) after the bias. */
@@ -382,6 +391,14 @@ int drhip_normalize_f32(const float* x, float* y, size_t n, int type, float targ
  * shuffles.  Replaces computeExp + host-side sum + mulScalar (src/dR_nodes_math.c:620-678,
  * Kernels/dR_math.cl:216-227,295-305). */
 int drhip_softmax_f32(const float* x, float* y, int n, void* stream);
+/* drhip_softmax_ex_f32 that also stores y, and the finished input of a deferred one, for the host (push may be NULL; n at most 2048) */
+int drhip_softmax_push_f32(const float* x, const drhip_deferred_vec* xdef, float* y, int n, const drhip_push* push, void* stream);
+/* A small fully connected layer and the softmax behind it in one workgroup: y = softmax(act(bias + x . Wt)), K and N at most 1024 and
+ * K*N at most 32768 (drhip_fc_softmax_usable); z (may be NULL) receives the layer's own output.  Replaces `matrixVectorMultFirst`,
+ * `matrixVectorMultSecond` and the softmax kernels of such a pair (Kernels/dR_fcl.cl:59-120, src/dR_nodes_math.c:620-678). */
+int drhip_fc_softmax_usable(int K, int N);
+int drhip_fc_softmax_f32(const float* x, const drhip_deferred_vec* xdef, const float* Wt, const float* bias, float* z, float* y, int K, int N, int relu,
+                         const drhip_push* push, void* stream);
 int drhip_softmax_ex_f32(const float* x, const drhip_deferred_vec* xdef, float* y, int n, void* stream);
 
 /* ---- data movement nodes ------------------------------------------------------------------------

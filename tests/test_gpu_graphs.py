@@ -288,6 +288,44 @@ def test_fire_chain_with_both_ends(oracle, gpu, w, h, cin, first, squeeze, expan
     assert rel_err(res["1"][1], res["0"][1]) <= 5e-6
 
 
+@pytest.mark.parametrize("K,N,front,logits", [(1, 1, 0, True), (1024, 32, 0, False), (32, 1024, 40, True), (333, 98, 900, True), (128, 10, 1568, True), (5, 700, 0, True)],
+                         ids=lambda v: str(v))
+def test_small_layer_in_the_softmax(oracle, gpu, K, N, front, logits):
+    """A small fully connected layer in the launch of the softmax behind it, on a plain or an unfinished input, and outputs that go to the
+    host from that launch: against the oracle, the kernels apart (DR_FUSE_FC=0) and dR_apply with a download."""
+    st = configs._Streams(81)
+    spec = [{"op": "feed", "shape": (front or K, 1, 1)}]
+    if front:
+        spec.append(configs._fc(st, 0, front, K, True))
+    spec.append(configs._fc(st, len(spec) - 1, K, N, False)); fc = len(spec) - 1
+    spec.append({"op": "softmax", "in": fc})
+    outs = [fc, fc + 1] if logits else [fc + 1]
+    x = configs.image_input(st, front or K, 1, 1)
+    want = oracle.run_spec(spec, {0: x})
+    for flag in ("1", "0"):
+        os.environ["DR_FUSE_FC"] = flag
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, outs)
+                dr.prepare(g)
+                for k in (0, 1, 2):             # (another input in between: what comes back is this pass's)
+                    configs.feed_chw(nodes[0], x if k != 1 else 1 - x)
+                    got = dr.apply(g)
+                assert g.lib.dR_apply(g.ptr)
+                again = dr.download_outputs(g)
+                dr.graph_config(g).profilingGPU = 1         # (apart: a profiled pass is waited for)
+                slow = dr.apply(g)
+                ms = dr.node_struct(nodes[fc]).drLastKernelMs
+        finally:
+            os.environ.pop("DR_FUSE_FC", None)
+        assert (ms == 0.0) == (flag == "1")
+        for u, v, w, i in zip(got, again, slow, outs):
+            assert np.array_equal(u, v) and np.array_equal(u, w)
+            # (a sum of K products that are themselves rounded sums)
+            assert_close(np.reshape(u, -1), want[i].reshape(-1), "node %d" % i, terms=max(K, front) * (4 if front else 1), floor=0.01)
+
+
 @pytest.mark.parametrize("case", ["means", "ragged", "mixed", "shared"])
 def test_scalar_operations_in_front_of_a_concat(oracle, gpu, case):
     """Slices, scalar operations and the concat they fill in one launch (DR_FUSE_SCALAR=0: kernels apart): the same numbers."""
