@@ -17,12 +17,16 @@
 //     buffer load per lane and 1 KiB in a row per wave.  Every wave reads only its own 32 channels, several steps ahead.
 //   * Two, four or eight waves share the k-steps of one channel block round-robin and meet in LDS at the end, in wave order: layers with
 //     few tiles fill the chip that way without a second kernel.
+//   * A 2x2/2 max pooling behind the layer is taken from these sums: a pooled pixel a lane.  (28x28 with 5x5 filters and poolings, 16
+//     and 32 channels, its image from the host and its results back: 36.4 -> 32.2 us, two launches less.)
 //   * Outputs that do not come out finite are worked out again in fp32, at the end.
 // Layers with at most four input channels (images) put four neighbouring pixels x four channels into one step of 16 k
 // (CP = 4) instead of 16 channels of one pixel, most of which would be zero: a 7x7 filter over RGB is 14 steps, not 49.
 #include "bf16x3.hpp"
 
 #include <algorithm>
+#include <cfloat>
+#include <type_traits>
 
 namespace drhip {
 
@@ -35,7 +39,7 @@ struct BankShape {                                      // everything but the po
     int pw, patchN;                                     // patch width, patch pixels
     int spr, steps, nChunks, oBlocks;                   // k-steps per filter row, per chunk; chunks; 32-channel blocks in the bank
     unsigned pwMul, pwShift, sprMul;                    // division by pw; j = step * sprMul >> 16
-    int relu;
+    int relu, pool;                                     // pool: a 2x2/2 max pooling stands behind the layer, `out` is its tensor
 };
 
 __device__ inline u32x4b bank_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, unsigned soffset) {
@@ -257,6 +261,39 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
             part[((wk * 32 * WO + 32 * wo + 8 * (r / 4) + 4 * half + r % 4) * MT + m) * kPitch + l32] = acc[m][0][r];
     __syncthreads();
     unsigned again = 0;                                 // turns whose output did not come out finite
+    auto finish = [&](float v, float scale, float b) {
+        v = fmaf(v, scale, b);
+        return s.relu ? fmaxf(v, 0.0f) : v;
+    };
+    // Pooled: 512 lanes, 64 (channel, block) pairs of 8 pooled pixels a turn.  The maximum as the pooling's own kernel takes it: in scan
+    // order from the lowest number on, what lies beside the map counts as 0.
+    constexpr int kPooled = WO * MT / 2 > 0 ? WO * MT / 2 : 1;
+    const int px2 = tid & ((BW >> 1) - 1), py2 = (tid & 7) >> (s.lgBW - 1), Wp = (s.Wo + 1) >> 1, Pp = Wp * ((s.Ho + 1) >> 1);
+    auto pooled_of = [&](int n, int& oc, int& x, int& y) {
+        const int pair = 64 * n + (tid >> 3), m = pair % MT;
+        oc = pair / MT; x = x0 + 2 * px2; y = y0 + 2 * py2 + BH * m;
+        return ((oc * MT) + m) * kPitch + 2 * py2 * BW + 2 * px2;
+    };
+    auto larger = [](float best, float v) { return v > best ? v : best; };
+    if (s.pool) {
+#pragma unroll
+        for (int n = 0; n < kPooled; ++n) {
+            int oc, x, y;
+            const int at = pooled_of(n, oc, x, y);
+            if (oc >= 32 * WO) break;                   // (a single block for half of the lanes)
+            const int o = blockIdx.z * (32 * WO) + oc;
+            float best = -FLT_MAX;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = 0.0f;
+#pragma unroll
+                for (int k = 0; k < WK; ++k) v += part[k * 32 * WO * MT * kPitch + at + (e & 1) + (e >> 1) * BW];
+                again |= fabsf(v) < __builtin_inff() ? 0u : 1u << n;
+                best = larger(best, x + (e & 1) < s.Wo && y + (e >> 1) < s.Ho ? finish(v, kSplitUnscale, biasT[oc]) : 0.0f);
+            }
+            if (o < s.O && x < s.Wo && y < s.Ho) store_through(out + (size_t)o * Pp + (size_t)(y >> 1) * Wp + (x >> 1), best);
+        }
+    } else
 #pragma unroll
     for (int n = 0; n < 2 * WO * MT; ++n) {             // 512 lanes: 16 (channel, block) pairs of 32 pixels a turn
         const int pair = 16 * n + (tid >> 5), m = pair % MT, oc = pair / MT, pl = tid & 31;
@@ -266,8 +303,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         again |= fabsf(v) < __builtin_inff() ? 0u : 1u << n;
         const int o = blockIdx.z * (32 * WO) + oc;
         const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
-        v = fmaf(v, kSplitUnscale, biasT[oc]);
-        if (s.relu) v = fmaxf(v, 0.0f);
+        v = finish(v, kSplitUnscale, biasT[oc]);
         if (o < s.O && x < s.Wo && y < s.Ho) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
     }
 
@@ -280,17 +316,14 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     const unsigned long long any = __builtin_amdgcn_ballot_w64(again != 0u);
     if (__builtin_expect(any == 0, 1)) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
-    constexpr int CH = 4 * WO;                          // channels of this wave
-    const int ci = lane % CH, oc = MT == 1 ? 16 * (ci >> 1) + 2 * wave + (ci & 1) : 8 * ci + wave, o = blockIdx.z * (32 * WO) + oc;
     const int kh = s.steps / s.spr;
-    const unsigned fAgain = (unsigned)(min(o >> 5, s.oBlocks - 1) * 1024 + (o & 31) * 16);
-    for (unsigned long long bad = MT == 1 ? (any | any >> 32) & 0xffffffffull : any; bad != 0; bad &= bad - 1) {
-        const int px = __builtin_ctzll(bad), pl = px & 31, m = px >> 5;
-        const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
-        if (x >= s.Wo || y >= s.Ho) continue;
+    // The sum at pixel (x, y) of the map for channel oc of the workgroup: CH channels side by side, 64 / CH lanes for each.
+    auto once_more = [&](auto channels, int x, int y, int oc) {
+        constexpr int CH = decltype(channels)::value;
+        const int o = blockIdx.z * (32 * WO) + oc;
+        const unsigned fAgain = (unsigned)(min(o >> 5, s.oBlocks - 1) * 1024 + (o & 31) * 16);
         const int left = x * s.sx - s.padX, top = y * s.sy - s.padY;
-        bool stays = false;
-        for (int j = 0; j < kh && !stays; ++j) {
+        for (int j = 0; j < kh; ++j) {
             const float* row = in + (size_t)min(max(top + j, 0), s.H - 1) * s.W;        // (a row beside the map stands for one that is in the window)
             bool nan = false;
             for (int c = lane; c < s.I; c += 64)
@@ -298,9 +331,8 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
                     const float v = row[(size_t)c * plane + min(max(left + i, 0), s.W - 1)];
                     nan = nan || v != v;
                 }
-            stays = __builtin_amdgcn_ballot_w64(nan) != 0;
+            if (__builtin_amdgcn_ballot_w64(nan) != 0) return __builtin_nanf("");
         }
-        if (stays) continue;
         float v = 0.0f;
         for (int chunk = 0; chunk < s.nChunks; ++chunk)
             for (int u = lane / CH; u < 2 * s.steps; u += 64 / CH) {            // half a k-step: eight values of k
@@ -319,9 +351,34 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
             }
 #pragma unroll
         for (int k = CH; k < 64; k *= 2) v += __shfl_xor(v, k);
+        return v;
+    };
+    if (s.pool) {                                       // output by output, the four of its window by the whole wave
+        for (int n = 0; n < kPooled; ++n)
+            for (unsigned long long bad = __builtin_amdgcn_ballot_w64((again >> n & 1u) != 0); bad != 0; bad &= bad - 1) {
+                const int src = __builtin_ctzll(bad);
+                int oc, x, y;
+                pooled_of(n, oc, x, y);
+                oc = __shfl(oc, src); x = __shfl(x, src); y = __shfl(y, src);
+                const int o = blockIdx.z * (32 * WO) + oc;
+                if (o >= s.O || x >= s.Wo || y >= s.Ho) continue;
+                float best = -FLT_MAX;
+                for (int e = 0; e < 4; ++e) {
+                    const int xe = x + (e & 1), ye = y + (e >> 1);
+                    best = larger(best, xe < s.Wo && ye < s.Ho ? finish(once_more(std::integral_constant<int, 1>{}, xe, ye, oc), 1.0f, biasT[oc]) : 0.0f);
+                }
+                if (lane == src) store_through(out + (size_t)o * Pp + (size_t)(y >> 1) * Wp + (x >> 1), best);
+            }
+        return;
+    }
+    constexpr int CH = 4 * WO;                          // channels of this wave
+    const int ci = lane % CH, oc = MT == 1 ? 16 * (ci >> 1) + 2 * wave + (ci & 1) : 8 * ci + wave, o = blockIdx.z * (32 * WO) + oc;
+    for (unsigned long long bad = MT == 1 ? (any | any >> 32) & 0xffffffffull : any; bad != 0; bad &= bad - 1) {
+        const int px = __builtin_ctzll(bad), pl = px & 31, m = px >> 5;
+        const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
+        if (x >= s.Wo || y >= s.Ho) continue;
+        const float v = finish(once_more(std::integral_constant<int, CH>{}, x, y, oc), 1.0f, biasT[oc]);
         const unsigned noted = (unsigned)__shfl((int)again, MT == 1 ? 32 * (ci & 1) + pl : px) >> (MT == 1 ? ci >> 1 : ci);
-        v += biasT[oc];
-        if (s.relu) v = fmaxf(v, 0.0f);
         if (lane < CH && (noted & 1u) && o < s.O) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
     }
 }
@@ -359,14 +416,14 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
 // other tiles: 56x56 64->96 5x5 10.9 / 11.5 to 24.7, 224x224 3->64 7x7/2 5.8 / 7.1 to 12.7, 56x56 256->256 3x3 29.7 / 33 to 78,
 // 96x70 50->75 5x5 17.4 / 17.2 to 24.8, 112x112 64->128 3x3/2 8.5 / 8.6 to 15, 14x14 16->32 5x5 4.3 / 4.8 to 8.2.  The kernel
 // that staged the same patch for vector FMAs took 123 us on the first and 31.4 us on the last.
-static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, BankPlan* best) {
+static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, bool pool, BankPlan* best) {
     double bestCost = 0;
     bool found = false;
     for (int wsel = 0; wsel < 3; ++wsel)
         for (int lgM = 0; lgM < 2; ++lgM) {
             const int wo = 4 >> wsel, wk = 2 << wsel, mt = 1 << lgM;
             if (variant && variant != (0x100 | wsel << 4 | lgM)) continue;
-            for (int lgBW = 3; lgBW <= 5; ++lgBW) {
+            for (int lgBW = 3; lgBW <= (pool ? 4 : 5); ++lgBW) {       // (pooled: two rows of a window in one block)
                 BankPlan p;
                 if (!bank_shape(W, H, I, O, kw, kh, sx, sy, mt, wo, wk, lgBW, &p)) continue;
                 const BankShape& s = p.s;
@@ -429,7 +486,12 @@ extern "C" int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh
     if (bank_blocks(I, O, kw, kh) * 3 * 1024 >= (1ull << 31)) return 0;
     if (H / strideY > 65535 || ceil_div(O, 32) > 65535) return 0;
     BankPlan p;
-    return bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, &p) ? 1 : 0;
+    return bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, false, &p) ? 1 : 0;
+}
+
+extern "C" int drhip_conv_bank_maxpool2_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
+    BankPlan p;
+    return drhip_conv_bank_usable(W, H, I, O, kw, kh, strideX, strideY) && bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, true, &p) ? 1 : 0;
 }
 
 extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O, int kw, int kh, void* stream) {
@@ -441,14 +503,25 @@ extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O
     return launched("conv_bank_layout_kernel");
 }
 
-extern "C" int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
-                                   int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
-    DRHIP_REQUIRE(in && F && out, "drhip_conv_bank_f32: NULL tensor");
-    DRHIP_REQUIRE(drhip_conv_bank_usable(W, H, I, O, kw, kh, strideX, strideY), "drhip_conv_bank_f32: shape %dx%dx%d -> %d, %dx%d/%dx%d not covered", W, H, I, O, kw, kh, strideX, strideY);
-    DRHIP_REQUIRE(((size_t)F & 15) == 0, "drhip_conv_bank_f32: the filter bank must be 16-byte aligned");
+static int conv_bank(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                     int kw, int kh, int strideX, int strideY, int relu, bool pool, int variant, void* stream, const char* who) {
+    DRHIP_REQUIRE(in && F && out, "%s: NULL tensor", who);
+    DRHIP_REQUIRE(drhip_conv_bank_usable(W, H, I, O, kw, kh, strideX, strideY), "%s: shape %dx%dx%d -> %d, %dx%d/%dx%d not covered", who, W, H, I, O, kw, kh, strideX, strideY);
+    DRHIP_REQUIRE(((size_t)F & 15) == 0, "%s: the filter bank must be 16-byte aligned", who);
     BankPlan p;
-    DRHIP_REQUIRE(bank_plan(W, H, I, O, kw, kh, strideX, strideY, variant, &p), "drhip_conv_bank_f32: variant %#x does not fit this shape", variant);
+    DRHIP_REQUIRE(bank_plan(W, H, I, O, kw, kh, strideX, strideY, variant, pool, &p), "%s: variant %#x does not fit this shape", who, variant);
     p.s.relu = relu ? 1 : 0;
+    p.s.pool = pool ? 1 : 0;
     if (p.cp == 4) return launch_bank_m<4>(in, (const unsigned short*)F, bias, out, p, as_stream(stream));
     return launch_bank_m<16>(in, (const unsigned short*)F, bias, out, p, as_stream(stream));
+}
+
+extern "C" int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                                   int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
+    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, false, variant, stream, "drhip_conv_bank_f32");
+}
+
+extern "C" int drhip_conv_bank_maxpool2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                                            int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
+    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, true, variant, stream, "drhip_conv_bank_maxpool2_f32");
 }

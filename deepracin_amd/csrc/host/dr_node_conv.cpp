@@ -322,7 +322,9 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
             if (c->drSqueezeNext) {             // and the squeeze layer behind that
                 const dR_Conv2d_Data* sq = conv_of(c->drSqueezeNext);
                 rc = drhip_conv3x3_pool3s2_squeeze_f32(in, w, b, (const float*)sq->weightsBuf, (float*)sq->workspaceBuf, W, H, I, O, sq->shape.s3, c->stride.s1, c->stride.s2, relu, stream_of(net));
-            } else if (c->drFusedPool)          // first layer + the 3x3/2 max pool behind it (out = the pool's buffer)
+            } else if (c->drFusedPool && c->drSplitBank)
+                rc = drhip_conv_bank_maxpool2_f32(in, w, b, out, W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, relu, c->variant, stream_of(net));
+            else if (c->drFusedPool)            // first layer + the 3x3/2 max pool behind it (out = the pool's buffer)
                 rc = drhip_conv3x3_pool3s2_f32(in, w, b, out, W, H, I, O, c->stride.s1, c->stride.s2, relu, stream_of(net));
             else if (c->drDirectBank)
                 rc = drhip_conv3x3_direct_mfma_f32(in, w, b, out, W, H, I, O, c->stride.s1, relu, c->variant, stream_of(net));

@@ -179,6 +179,10 @@ size_t drhip_conv_bank_floats(int I, int O, int kw, int kh);
 int drhip_conv_bank_layout_f32(const float* w /* [I][O][kh][kw] */, float* F, int I, int O, int kw, int kh, void* stream);
 int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                         int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
+/* With a 2x2/2 max pooling behind it, by drhip_pool_f32's rules: out[O][ceil(Ho/2)][ceil(Wo/2)]. */
+int drhip_conv_bank_maxpool2_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY);
+int drhip_conv_bank_maxpool2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                                 int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
 
 /* First layer (1 to 4 input channels, 3x3, any stride, zero padding, bias, optional ReLU) followed by
  * a 3x3 / stride-2 max pooling with the reference's pooling rules (out = ceil(in/2), samples outside

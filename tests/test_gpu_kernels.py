@@ -116,6 +116,33 @@ def test_conv_split_bank(lib, dev, oracle, variant, W, H, I, O, kw, kh, sx, sy):
         assert rel_err(got, want) <= TOL / 20
 
 
+@pytest.mark.parametrize("variant", [0x100, 0x101, 0x110, 0x111, 0x120, 0x121])
+@pytest.mark.parametrize("W,H,I,O,k,s", [(28, 28, 1, 16, 5, 1), (14, 14, 16, 32, 5, 1), (27, 9, 17, 33, 5, 1), (1, 1, 3, 70, 7, 1), (33, 40, 4, 129, 5, 2), (18, 5, 40, 9, 3, 3)])
+def test_conv_split_bank_with_maxpool(lib, dev, oracle, variant, W, H, I, O, k, s):
+    """The same with a 2x2/2 max pooling behind it: the pooling kernel's results bit for bit, on odd maps (where the pooling counts zeros)
+    too; an infinity and a NaN reach what they reach without it."""
+    x, w, b = own(I, H, W), own(I, O, k, k, scale=(2.0 / (I * k * k)) ** 0.5), own(O, scale=0.1) - 0.1
+    F = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k))
+    ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
+    Wo, Ho, bd = W // s, H // s, dev.put(b)
+    full, pooled = dev.empty(O * Ho * Wo), dev.empty(O * -(-Ho // 2) * -(-Wo // 2))
+    for relu, extremes in ((1, False), (0, False), (0, True)):
+        if extremes:
+            x[0, H // 2, W // 2], x[I - 1, 0, 0], x[I // 2, H - 1, W - 1] = np.inf, -np.inf, np.nan
+        xd = dev.put(x)
+        ok(lib, lib.drhip_conv_bank_f32(xd, F, bd, full, W, H, I, O, k, k, s, s, relu, variant, None))
+        ok(lib, lib.drhip_conv_bank_maxpool2_f32(xd, F, bd, pooled, W, H, I, O, k, k, s, s, relu, variant, None))
+        two = dev.empty(O * -(-Ho // 2) * -(-Wo // 2))
+        ok(lib, lib.drhip_pool_f32(full, two, None, Wo, Ho, O, 2, 2, 1, 2, 2, 1, 0, None))
+        got, want = (dev.get(p, (O, -(-Ho // 2), -(-Wo // 2))) for p in (pooled, two))
+        if extremes:                        # (the four of such a window are worked out again together, in another order of the sums)
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]) and not np.isnan(got).any()
+            f = np.isfinite(want)
+            assert not f.any() or np.all(np.abs(got[f] - want[f]) <= TOL / 20 * np.abs(w).sum((0, 2, 3)).max())
+        else:
+            assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("W,H,I,O,sx,sy", [(224, 224, 3, 64, 2, 2), (33, 31, 3, 9, 2, 2), (17, 13, 1, 5, 1, 1), (20, 18, 4, 70, 1, 2),
                                             (8, 5, 2, 16, 3, 1), (2, 2, 3, 2, 1, 1), (9, 9, 4, 33, 2, 2), (64, 48, 3, 32, 1, 1)])
 @pytest.mark.parametrize("relu", [1, 0])
