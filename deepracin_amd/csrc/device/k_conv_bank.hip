@@ -8,14 +8,14 @@
 // of staging, matrix steps and store on small ones; figures stand at the choice of the tile.
 //
 // A workgroup owns a tile of 32*MT output pixels and 32*WO output channels:
-//   * The input patch under the tile is staged in LDS once per 16 channels, zero padding included, ALREADY SPLIT into
+//   * The input patch under the tile is staged in LDS, 16 to 128 channels at a time, zero padding included, ALREADY SPLIT into
 //     its three bf16 parts and with the eight channels an MFMA lane wants next to each other: inside the tap loop a
 //     B operand is one 16-byte LDS read whatever the tap (a tap is an address offset), and there is no vector arithmetic at all.
 //     Reading the samples from global memory per tap would cost a dword gather and a split per sample and tap, 25 times
-//     for a 5x5 filter.  The next 16 channels are fetched into registers while the taps run and go to the other half of LDS.
+//     for a 5x5 filter.  The next stage's are fetched into registers while the taps run and go to the other half of LDS.
 //   * The filters come from a bank laid out and split once, when the layer is prepared, so that an A operand is one 16-byte
 //     buffer load per lane and 1 KiB in a row per wave.  Every wave reads only its own 32 channels, several steps ahead.
-//   * Two, four or eight waves share the k-steps of one channel block round-robin and meet in LDS at the end, in wave order: layers with
+//   * Two, four or eight waves share the k-steps of a stage and 32 output channels round-robin and meet in LDS at the end, in wave order: layers with
 //     few tiles fill the chip that way without a second kernel.
 //   * A 2x2/2 max pooling behind the layer is taken from these sums: a pooled pixel a lane.  (28x28 with 5x5 filters and poolings, 16
 //     and 32 channels, its image from the host and its results back: 36.4 -> 32.2 us, two launches less.)
@@ -38,7 +38,9 @@ struct BankShape {                                      // everything but the po
     int lgBW;                                           // 32 pixels of one MFMA = 2^lgBW columns x the rest rows
     int pw, patchN;                                     // patch width, patch pixels
     int spr, steps, nChunks, oBlocks;                   // k-steps per filter row, per chunk; chunks; 32-channel blocks in the bank
-    unsigned pwMul, pwShift, sprMul;                    // division by pw; j = step * sprMul >> 16
+    int group, nStages;                                 // chunks that are staged together; stages
+    unsigned pwMul, pwShift, patchMul, patchShift;      // division by pw and patchN
+    unsigned sprMul, stepsMul;                          // j = tap * sprMul >> 16, chunk of a stage = step * stepsMul >> 16
     int relu, pool;                                     // pool: a 2x2/2 max pooling stands behind the layer, `out` is its tensor
 };
 
@@ -68,7 +70,7 @@ conv_bank_layout_kernel(const float* __restrict__ w, unsigned short* __restrict_
     for (int q = 0; q < 3; ++q) F[((((size_t)chunk * steps + step) * 3 + q) * oBlocks + ob) * 512 + lane * 8 + e] = part[q];
 }
 
-// PF: staging rounds (512 units each) of the next 16 channels that are kept in registers.
+// PF: staging rounds (512 units each) of the next stage that are kept in registers.
 template <int CP, int MT, int WO, int WK, int PF>
 __global__ void __launch_bounds__(kBankThreads)
 conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __restrict__ F, const float* __restrict__ bias,
@@ -92,24 +94,24 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     const int plane = s.H * s.W;
 
     // ---- staging: unit u -> (channel group, patch pixel); a unit is 8 (4) channels of one pixel, split ----------------
-    const int units = s.patchN * kGroups;
+    const int units = s.patchN * kGroups * s.group;
     const int rounds = (units + kBankThreads - 1) / kBankThreads;
-    const int partBytes = (s.patchN * kGroups * kUnitBytes + 15) & ~15;
+    const int partBytes = (units * kUnitBytes + 15) & ~15;
     const int bufBytes = 3 * partBytes;
-    const FastDiv pwd = {(unsigned)s.pw, s.pwMul, s.pwShift};
+    const FastDiv pwd = {(unsigned)s.pw, s.pwMul, s.pwShift}, patchd = {(unsigned)s.patchN, s.patchMul, s.patchShift};
     const int px0 = x0 * s.sx - s.padX, py0 = y0 * s.sy - s.padY;
     constexpr int kUC = CP == 16 ? 8 : 4;               // channels of a unit
     auto unit_offset = [&](int u, unsigned& off) {
-        const int grp = (kGroups == 2 && u >= s.patchN) ? 1 : 0, q = u - grp * s.patchN;
+        const int grp = kGroups == 2 ? fast_div(u, patchd) : 0, q = u - grp * s.patchN;
         const int py = fast_div(q, pwd), px = q - py * s.pw;
         const int ix = px0 + px, iy = py0 + py;
         const bool ok = u < units && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
         off = ok ? 4u * (unsigned)(grp * 8 * plane + iy * s.W + ix) : kOutOfRange;
     };
-    auto load_unit = [&](float (&v)[kUC], unsigned off, int chunk) {
+    auto load_unit = [&](float (&v)[kUC], unsigned off, int stage) {
 #pragma unroll
         for (int q = 0; q < kUC; ++q) {                 // (channels past the last one: a resource that ends in front of them)
-            const int c = chunk * 16 + q, left = max(s.I - c, 0);
+            const int c = stage * s.group * 16 + q, left = max(s.I - c, 0);
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(in + (size_t)min(c, s.I) * plane), 0, left * plane * 4, kBufferFlags);
             v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
         }
@@ -132,17 +134,17 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     };
 
     // ---- filters: the steps of this wave, wk, wk + WK, ..., -------------------------------------
-    const int bankBytes = s.nChunks * s.steps * 3 * s.oBlocks * 1024;
+    const int allSteps = s.nChunks * s.steps;
+    const int bankBytes = allSteps * 3 * s.oBlocks * 1024;
     const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, bankBytes, kBufferFlags);
     const unsigned fLane = ob < s.oBlocks ? (unsigned)(ob * 1024 + lane * 16) : kOutOfRange;    // (a wave without channels multiplies zeros)
-    auto load_filters = [&](u32x4b (&f)[3], int chunk, int step) {
+    auto load_filters = [&](u32x4b (&f)[3], int step) {     // (of the whole layer)
 #pragma unroll
-        for (int q = 0; q < 3; ++q) f[q] = bank_load4(rF, fLane, (unsigned)(((chunk * s.steps + step) * 3 + q) * s.oBlocks) * 1024u);
+        for (int q = 0; q < 3; ++q) f[q] = bank_load4(rF, fLane, (unsigned)((min(step, allSteps - 1) * 3 + q) * s.oBlocks) * 1024u);
     };
-    const int mySteps = wk < s.steps ? (s.steps - wk + WK - 1) / WK : 0;
     u32x4b f[kDepth][3];
 #pragma unroll
-    for (int g = 0; g < kDepth; ++g) load_filters(f[g], 0, min(wk + g * WK, s.steps - 1));
+    for (int g = 0; g < kDepth; ++g) load_filters(f[g], wk + g * WK);
 
     unsigned off[PF];
     float raw[PF][kUC];
@@ -153,14 +155,14 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     }
     if (tid < 32 * WO) biasT[tid] = bias ? bias[min((int)blockIdx.z * 32 * WO + tid, s.O - 1)] : 0.0f;
     // what of the patch does not fit the prefetch registers is loaded when it is stored
-    auto stage = [&](char* buf, int chunk) {
+    auto stage = [&](char* buf, int n) {
 #pragma unroll
         for (int r = 0; r < PF; ++r) store_unit(buf, raw[r], tid + kBankThreads * r);
         for (int r = PF; r < rounds; ++r) {
             unsigned o;
             float v[kUC];
             unit_offset(tid + kBankThreads * r, o);
-            load_unit(v, o, chunk);
+            load_unit(v, o, n);
             store_unit(buf, v, tid + kBankThreads * r);
         }
     };
@@ -189,8 +191,9 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 
     auto read_operands = [&](const char* buf, u32x4b (&b)[MT][3], int step) {
-        const int j = (int)(((unsigned)step * s.sprMul) >> 16), i = step - j * s.spr;
-        const char* at = buf + (CP == 16 ? (j * s.pw + i) * 16 : (j * s.pw + 4 * i) * 8);
+        const int c = CP == 16 ? (int)(((unsigned)step * s.stepsMul) >> 16) : 0, tap = step - c * s.steps;
+        const int j = (int)(((unsigned)tap * s.sprMul) >> 16), i = tap - j * s.spr;
+        const char* at = buf + (CP == 16 ? (2 * c * s.patchN + j * s.pw + i) * 16 : (j * s.pw + 4 * i) * 8);
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -210,18 +213,19 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
             for (int m = 0; m < MT; ++m) acc[m][q % NA] = mfma_bf16(fs[kProdA[q]], b[m][kProdB[q]], acc[m][q % NA]);
     };
 
-    for (int chunk = 0; chunk < s.nChunks; ++chunk) {
-        const char* buf = lds + (chunk & 1) * bufBytes;
-        const bool more = chunk + 1 < s.nChunks;
+    for (int n0 = 0; n0 < s.nStages; ++n0) {
+        const char* buf = lds + (n0 & 1) * bufBytes;
+        const bool more = n0 + 1 < s.nStages;
+        const int first = n0 * s.group * s.steps, steps = min(s.group * s.steps, allSteps - first), mySteps = wk < steps ? (steps - wk + WK - 1) / WK : 0;
         if (more) {
 #pragma unroll
-            for (int r = 0; r < PF; ++r) load_unit(raw[r], off[r], chunk + 1);
+            for (int r = 0; r < PF; ++r) load_unit(raw[r], off[r], n0 + 1);
         }
         // A step's operands are read from LDS while the step in front of it multiplies (a wave is often alone on its SIMD, and
         // a trip to LDS is as long as six MFMAs); its filters were requested kDepth steps ago.  The loads of a group go
         // out whether or not the steps exist, so that the number of loads in flight is known where it is waited for.
         u32x4b b[2][MT][3];
-        read_operands(buf, b[0], min(wk, s.steps - 1));                 // (a wave may have no step at all)
+        read_operands(buf, b[0], min(wk, steps - 1));                   // (a wave may have no step at all)
         for (int n = 0; n < mySteps; n += kDepth) {
 #pragma unroll
             for (int g = 0; g < kDepth; ++g) {
@@ -230,13 +234,12 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
                     read_operands(buf, b[(g + 1) & 1], wk + min(t + 1, mySteps - 1) * WK);
                     multiply(f[g], b[g & 1]);
                 }
-                // the step that takes this slot next: kDepth on, or the slot's first one in the next 16 channels
-                const bool here = t + kDepth < mySteps;
-                load_filters(f[g], here ? chunk : min(chunk + 1, s.nChunks - 1), min(wk + (here ? t + kDepth : g) * WK, s.steps - 1));
+                // the step that takes this slot next: kDepth on, or the slot's first one in the next stage
+                load_filters(f[g], first + wk + (t + kDepth < mySteps ? (t + kDepth) * WK : s.group * s.steps + g * WK));
             }
         }
         if (more) {
-            stage(lds + ((chunk + 1) & 1) * bufBytes, chunk + 1);       // (read last before the barrier in front of this chunk)
+            stage(lds + ((n0 + 1) & 1) * bufBytes, n0 + 1);             // (read last before the barrier in front of this stage)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -399,23 +402,35 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
     s.patchN = s.pw * ((BH - 1) * sy + kh);
     s.nChunks = p->cp == 16 ? ceil_div(I, 16) : 1;
     s.oBlocks = ceil_div(O, 32);
-    const FastDiv d = make_fastdiv(s.pw);
+    const FastDiv d = make_fastdiv(s.pw), dp = make_fastdiv(s.patchN);
     s.pwMul = d.mul; s.pwShift = d.shift;
+    s.patchMul = dp.mul; s.patchShift = dp.shift;
     s.sprMul = (unsigned)(65536 / s.spr + 1);
-    const size_t partBytes = ((size_t)s.patchN * (p->cp == 16 ? 32 : 8) + 15) & ~(size_t)15;
-    p->pf = s.patchN * (p->cp == 16 ? 2 : 1) <= kBankThreads ? 1 : 2;
-    p->lds = 3 * partBytes * (s.nChunks > 1 ? 2 : 1);
-    p->lds = std::max(p->lds, (size_t)wk * 32 * wo * mt * 33 * sizeof(float));
+    const size_t sums = (size_t)wk * 32 * wo * mt * 33 * sizeof(float);
+    const long long wgs = (long long)ceil_div(s.Wo, BW) * ceil_div(s.Ho, BH) * ceil_div(s.oBlocks, wo);
+    // As few stages as LDS allows (half of it where a CU is to hold two workgroups), of the same number of chunks: the loads of a stage are
+    // one trip to memory, and every stage leaves waves without a last step.  56x56 64->96 5x5 12.9 us by single chunks, 11.4 in one stage of
+    // four; 28x28 128->128 5x5 14.5 and 11.7 in two of four.
+    s.nStages = 0;
+    do {
+        s.group = ceil_div(s.nChunks, ++s.nStages);
+        const int units = s.patchN * (p->cp == 16 ? 2 : 1) * s.group;
+        const size_t partBytes = ((size_t)units * (p->cp == 16 ? 16 : 8) + 15) & ~(size_t)15;
+        p->pf = std::min(ceil_div(units, kBankThreads), p->cp == 16 ? 4 : 2);
+        p->lds = std::max(3 * partBytes * (s.nStages > 1 ? 2 : 1), sums);
+        if (s.group <= 8 && units <= 4 * kBankThreads && p->lds <= (wgs > num_cu() ? kMaxDynamicLds / 2 : kMaxDynamicLds) && s.group * s.steps * s.steps < 65536) break;
+    } while (s.group > 1);
+    s.nStages = ceil_div(s.nChunks, s.group);
+    s.stepsMul = s.group > 1 ? (unsigned)(65536 / s.steps + 1) : 0;         // (exact by the last condition)
     return p->lds <= kMaxDynamicLds && s.steps * s.spr < 65536;      // (the kernel's division of a step number by spr)
 }
 
-// The tile that finishes first, by a count of what the busiest CU does, in clocks: per workgroup a fixed 2000 for the first
-// loads and the store, 1200 per round of staging 16 channels (the address unit takes one dword gather every 8 to 16
-// clocks), and the MFMAs of one of its four SIMDs at 33 clocks plus what is lost around them.  Pixel tiles wider than the
-// map or hanging over its edge count in full, which picks the tile shape as well.  Measured, us per launch, this choice / the
-// other tiles: 56x56 64->96 5x5 10.9 / 11.5 to 24.7, 224x224 3->64 7x7/2 5.8 / 7.1 to 12.7, 56x56 256->256 3x3 29.7 / 33 to 78,
-// 96x70 50->75 5x5 17.4 / 17.2 to 24.8, 112x112 64->128 3x3/2 8.5 / 8.6 to 15, 14x14 16->32 5x5 4.3 / 4.8 to 8.2.  The kernel
-// that staged the same patch for vector FMAs took 123 us on the first and 31.4 us on the last.
+// The tile that finishes first, by a count of what the busiest CU does, in clocks: per workgroup a fixed 1500 for the store, per stage 1200
+// for the trip to memory and 1200 per round of staging (the address unit takes one dword gather every 8 to 16 clocks), and the MFMAs of
+// one of its four SIMDs at 42 clocks or, if that is more, the filters at 42 bytes a clock.  Pixel tiles wider than the map or
+// hanging over its edge count in full, which picks the tile shape as well.  Measured, us per layer, this choice / the
+// other tiles: 56x56 64->96 5x5 11.4 / 11.5 to 25, 224x224 3->64 7x7/2 6.1 / 7.7 to 13.7, 96x70 50->75 5x5 17.7 / 19.5 to 25, 28x28 128->128 5x5
+// 11.7 / 16 to 47, 112x112 64->128 3x3/2 9.2 / 10.1 to 15.5, 14x14 16->32 5x5 4.3 / 5 to 9.
 static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, bool pool, BankPlan* best) {
     double bestCost = 0;
     bool found = false;
@@ -428,8 +443,10 @@ static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy
                 if (!bank_shape(W, H, I, O, kw, kh, sx, sy, mt, wo, wk, lgBW, &p)) continue;
                 const BankShape& s = p.s;
                 const double wgs = (double)ceil_div(s.Wo, 1 << lgBW) * ceil_div(s.Ho, (32 >> lgBW) * mt) * ceil_div(s.oBlocks, wo);
-                const double mfma = (double)s.nChunks * s.steps * 6 * 33 * wo * mt / 4 * (mt == 1 ? 1.25 : 1.1);
-                const double cost = 2000 + std::ceil(wgs / num_cu()) * (2000 + (double)s.nChunks * p.pf * 1200 + mfma);
+                const double waveSteps = (s.nStages - 1.0) * ceil_div(s.group * s.steps, wk) + ceil_div((s.nChunks - (s.nStages - 1) * s.group) * s.steps, wk);
+                const double staging = s.nStages * 1200.0 * (1 + ceil_div(s.patchN * (p.cp == 16 ? 2 : 1) * s.group, kBankThreads));
+                const double work = std::max(1.3 * waveSteps * 2 * 6 * 32 * mt, (double)s.nChunks * s.steps * wo * 3072 / 42);
+                const double cost = 6000 + std::ceil(wgs / num_cu()) * (1500 + staging + work);
                 if (!found || cost < bestCost) { found = true; bestCost = cost; *best = p; }
             }
         }
@@ -448,6 +465,10 @@ static int launch_bank_pf(const float* in, const unsigned short* F, const float*
 
 template <int CP, int MT, int WO, int WK>
 static int launch_bank(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
+    if constexpr (CP == 16) {
+        if (p.pf == 4) return launch_bank_pf<CP, MT, WO, WK, 4>(in, F, bias, out, p, st);
+        if (p.pf == 3) return launch_bank_pf<CP, MT, WO, WK, 3>(in, F, bias, out, p, st);
+    }
     return p.pf == 1 ? launch_bank_pf<CP, MT, WO, WK, 1>(in, F, bias, out, p, st) : launch_bank_pf<CP, MT, WO, WK, 2>(in, F, bias, out, p, st);
 }
 
