@@ -171,7 +171,7 @@ def load_library(path=None):
         "drhip_conv_bank_floats": (c_size_t, [c_int] * 4),
         "drhip_conv_bank_layout_f32": (c_int, [vp, vp] + [c_int] * 4 + [vp]),
         "drhip_conv_bank_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 10 + [vp]),
-        "drhip_conv_bank_maxpool2_usable": (c_int, [c_int] * 8),
+        "drhip_conv_bank_pick_variant": (c_int, [c_int] * 9),
         "drhip_conv_bank_maxpool2_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 10 + [vp]),
         "drhip_conv3x3_pool3s2_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 7 + [vp]),
         "drhip_conv1x1_poolsum_f32": (c_int, [vp, vp, vp, vp, c_int, c_int, c_int, c_int, vp]),

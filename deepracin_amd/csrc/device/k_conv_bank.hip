@@ -434,6 +434,10 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
 static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, bool pool, BankPlan* best) {
     double bestCost = 0;
     bool found = false;
+    if (variant >> 12) {                                // everything chosen beforehand
+        const int wsel = variant >> 4 & 3, lgBW = variant >> 12;
+        return (variant & 0xfce) == 0x100 && wsel < 3 && lgBW >= 3 && lgBW <= (pool ? 4 : 5) && bank_shape(W, H, I, O, kw, kh, sx, sy, 1 << (variant & 1), 4 >> wsel, 2 << wsel, lgBW, best);
+    }
     for (int wsel = 0; wsel < 3; ++wsel)
         for (int lgM = 0; lgM < 2; ++lgM) {
             const int wo = 4 >> wsel, wk = 2 << wsel, mt = 1 << lgM;
@@ -499,20 +503,25 @@ extern "C" size_t drhip_conv_bank_floats(int I, int O, int kw, int kh) {
     return bank_blocks(I, O, kw, kh) * 3 * 256;
 }
 
-extern "C" int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
-    if (W <= 0 || H <= 0 || I <= 0 || O <= 0 || kw <= 0 || kh <= 0 || !(kw & 1) || !(kh & 1) || strideX <= 0 || strideY <= 0) return 0;
-    if (W / strideX <= 0 || H / strideY <= 0) return 0;
+static bool bank_limits(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
+    if (W <= 0 || H <= 0 || I <= 0 || O <= 0 || kw <= 0 || kh <= 0 || !(kw & 1) || !(kh & 1) || strideX <= 0 || strideY <= 0) return false;
+    if (W / strideX <= 0 || H / strideY <= 0) return false;
     // byte offsets into the input and the bank are 32-bit, and 0x80000000 must lie outside both
-    if ((long long)W * H * (I + 15) >= (1ll << 29) || (long long)(W / strideX) * (H / strideY) * O >= (1ll << 31)) return 0;
-    if (bank_blocks(I, O, kw, kh) * 3 * 1024 >= (1ull << 31)) return 0;
-    if (H / strideY > 65535 || ceil_div(O, 32) > 65535) return 0;
-    BankPlan p;
-    return bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, false, &p) ? 1 : 0;
+    if ((long long)W * H * (I + 15) >= (1ll << 29) || (long long)(W / strideX) * (H / strideY) * O >= (1ll << 31)) return false;
+    if (bank_blocks(I, O, kw, kh) * 3 * 1024 >= (1ull << 31)) return false;
+    return H / strideY <= 65535 && ceil_div(O, 32) <= 65535;
 }
 
-extern "C" int drhip_conv_bank_maxpool2_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
+extern "C" int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
     BankPlan p;
-    return drhip_conv_bank_usable(W, H, I, O, kw, kh, strideX, strideY) && bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, true, &p) ? 1 : 0;
+    return bank_limits(W, H, I, O, kw, kh, strideX, strideY) && bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, false, &p) ? 1 : 0;
+}
+
+// (Choosing a tile costs the host a microsecond or two: once when a layer is scheduled, not at every launch.)
+extern "C" int drhip_conv_bank_pick_variant(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY, int maxpool2) {
+    BankPlan p;
+    if (!bank_limits(W, H, I, O, kw, kh, strideX, strideY) || !bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, maxpool2 != 0, &p)) return 0;
+    return 0x100 | (p.wk == 2 ? 0 : p.wk == 4 ? 0x10 : 0x20) | (p.mt - 1) | p.s.lgBW << 12;
 }
 
 extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O, int kw, int kh, void* stream) {
@@ -527,7 +536,7 @@ extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O
 static int conv_bank(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                      int kw, int kh, int strideX, int strideY, int relu, bool pool, int variant, void* stream, const char* who) {
     DRHIP_REQUIRE(in && F && out, "%s: NULL tensor", who);
-    DRHIP_REQUIRE(drhip_conv_bank_usable(W, H, I, O, kw, kh, strideX, strideY), "%s: shape %dx%dx%d -> %d, %dx%d/%dx%d not covered", who, W, H, I, O, kw, kh, strideX, strideY);
+    DRHIP_REQUIRE(bank_limits(W, H, I, O, kw, kh, strideX, strideY), "%s: shape %dx%dx%d -> %d, %dx%d/%dx%d not covered", who, W, H, I, O, kw, kh, strideX, strideY);
     DRHIP_REQUIRE(((size_t)F & 15) == 0, "%s: the filter bank must be 16-byte aligned", who);
     BankPlan p;
     DRHIP_REQUIRE(bank_plan(W, H, I, O, kw, kh, strideX, strideY, variant, pool, &p), "%s: variant %#x does not fit this shape", who, variant);

@@ -106,10 +106,17 @@ gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
             c->drDirectBank = packable && c->shape.s0 == 3 && c->shape.s1 == 3 && I > 4 && c->stride.s1 == c->stride.s2 &&
                               (c->stride.s1 == 1 || c->stride.s1 == 2) && !(valu && strcmp(valu, "1") == 0);
             c->variant = c->drDirectBank ? drhip_conv3x3_direct_pick_variant(W / c->stride.s1, H / c->stride.s2, I, O) : 0;
+            // At stride 2 that kernel is the faster one where eight of its waves share the channels, which is where it has less than a
+            // workgroup per CU; elsewhere the split bank is: 300x200 48->96 17.7 us against 26.6, 96x96 36->48 5.8 / 7.8, 224x224 64->128
+            // 19.7 / 32.3, 30x30 24->32 4.9 / 10.6, 56x56 128->512 13.7 / 14.6; with eight waves 56x56 96->128 7.9 / 6.9, 28x28 512->512 30.2 / 21.7,
+            // 48x48 72->96 6.7 / 6.6, 20x20 64->64 5.9 / 5.6.
+            const int bank = drhip_conv_bank_pick_variant(W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 0);
+            if (c->drDirectBank && c->stride.s1 == 2 && (c->variant & 15) != 8 && bank) c->drDirectBank = FALSE;
             // Other filters and strides: the split filter bank.  (3x3 filters over an image have kernels of their own, one of
             // which pools as well.)
             c->drSplitBank = !c->drDirectBank && !(c->shape.s0 == 3 && c->shape.s1 == 3 && I <= 4) && !(valu && strcmp(valu, "1") == 0) &&
-                             drhip_conv_bank_usable(W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2);
+                             bank != 0;
+            if (!c->drDirectBank) c->variant = c->drSplitBank ? bank : 0;
             break;
         }
     }
@@ -166,6 +173,7 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     const bool wino = c->algo == drConvWinograd;
     const int O = launch_channels(c);
     if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
+    if (c->drSplitBank && c->drFusedPool) c->variant = drhip_conv_bank_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 1);
     const int n = c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
                        : wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
                        : c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)

@@ -99,7 +99,7 @@ dR_Node* pool_fusable_producer(const dR_Node* p) {
     if (tensor_wanted(c) || c->outputBuf || !c->next_layers || c->next_layers->length != 1) return nullptr;
     if (two) {
         const bool even = !((c->oshape.s0 | c->oshape.s1) & 1);
-        const bool bank = cd->drSplitBank && drhip_conv_bank_maxpool2_usable(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->shape.s0, cd->shape.s1, cd->stride.s1, cd->stride.s2);
+        const bool bank = cd->drSplitBank && drhip_conv_bank_pick_variant(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->shape.s0, cd->shape.s1, cd->stride.s1, cd->stride.s2, 1);
         if (!bank && !(cd->algo == drConvWinograd && even)) return nullptr;
     } else {
         if (cd->algo != drConvDirect || cd->shape.s0 != 3 || cd->shape.s1 != 3 || cd->shape.s2 > 4) return nullptr;

@@ -172,15 +172,17 @@ int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* 
  * fp32, at a multiple of the time.  F is the filter bank in the layout the kernel streams, produced once at prepare time from
  * w [I][O][kh][kw]; drhip_conv_bank_floats(I,O,kw,kh) floats, 16-byte aligned.  drhip_conv_bank_usable: whether the
  * shape is covered (the patch of a tile fits LDS, 32-bit byte offsets).  `variant` 0 lets the launcher pick; otherwise
- * 0x100 | log2(32-pixel blocks per workgroup, 0..1) | n << 4 for 2 << n waves sharing a channel block (n = 0..2).
+ * 0x100 | log2(32-pixel blocks per workgroup, 0..1) | n << 4 for 2 << n waves sharing a channel block (n = 0..2), and
+ * | log2(columns of a block, 3..5) << 12 or none of those bits.  drhip_conv_bank_pick_variant: what 0 stands for, in full, with
+ * or without the pooling; 0 if the shape is not covered.
  * Replaces the per-layer generated kernel of filters other than 3x3 (src/dR_nodes_conv2d.c:364-420, 481-773). */
 int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY);
+int drhip_conv_bank_pick_variant(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY, int maxpool2);
 size_t drhip_conv_bank_floats(int I, int O, int kw, int kh);
 int drhip_conv_bank_layout_f32(const float* w /* [I][O][kh][kw] */, float* F, int I, int O, int kw, int kh, void* stream);
 int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                         int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
 /* With a 2x2/2 max pooling behind it, by drhip_pool_f32's rules: out[O][ceil(Ho/2)][ceil(Wo/2)]. */
-int drhip_conv_bank_maxpool2_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY);
 int drhip_conv_bank_maxpool2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                                  int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
 

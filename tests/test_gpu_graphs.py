@@ -326,6 +326,30 @@ def test_small_layer_in_the_softmax(oracle, gpu, K, N, front, logits):
             assert_close(np.reshape(u, -1), want[i].reshape(-1), "node %d" % i, terms=max(K, front) * (4 if front else 1), floor=0.01)
 
 
+@pytest.mark.parametrize("W,H,I,O,split", [(30, 30, 24, 32, True), (33, 47, 36, 50, True), (7, 5, 9, 3, True), (90, 62, 70, 300, True), (20, 20, 64, 64, False), (41, 40, 80, 70, False)])
+def test_strided_layers_by_either_kernel(oracle, gpu, W, H, I, O, split):
+    """3x3/2 layers on both sides of the rule that chooses their kernel, and by the general one (DR_DIRECT_VALU=1)."""
+    st = configs._Streams(91)
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, 3, I, O, stride=2)]
+    x = configs.image_input(st, W, H, I)
+    want = oracle.conv_f64(x, spec[1]["w"], spec[1]["b"], stride=(2, 2), relu=True)
+    for flag in ("0", "1"):
+        os.environ["DR_DIRECT_VALU"] = flag
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, [1])
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], x)
+                assert g.lib.dR_apply(g.ptr)
+                got = configs.fetch_chw(g)[0]
+                line = ctypes.string_at(ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_void_p)(dr.node_struct(nodes[1]).printLayer)(nodes[1].ptr)).decode()
+                assert ("split-operand" in line) == (split and flag == "0")
+        finally:
+            os.environ.pop("DR_DIRECT_VALU", None)
+        assert_close(got, want, "DR_DIRECT_VALU=" + flag, terms=9 * I)
+
+
 @pytest.mark.parametrize("case", ["means", "ragged", "mixed", "shared"])
 def test_scalar_operations_in_front_of_a_concat(oracle, gpu, case):
     """Slices, scalar operations and the concat they fill in one launch (DR_FUSE_SCALAR=0: kernels apart): the same numbers."""
