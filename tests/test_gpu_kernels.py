@@ -846,6 +846,19 @@ def test_normalize(lib, dev, oracle, C, H, W):
     assert lib.drhip_normalize_f32(xd, y, 0, 2, 0.0, 1.0, scratch, None) == -1
 
 
+@pytest.mark.parametrize("n", [1, 3, 5, 1023, 1027, 1024 * 256 * 4 + 2, 1024 * 256 * 16 + 1024 * 128 + 3])
+def test_normalize_merges_what_workgroups_leave(lib, dev, oracle, n):
+    """The deviation out of sums about the workgroups' own means, which lie far apart here: one workgroup, ragged ends, all of its elements
+    in registers and more than those."""
+    x = (OWN.random(n, dtype=np.float32) + 100.0 * np.sin(np.arange(n) / 4096.0)).astype(np.float32)
+    xd, y, scratch = dev.put(x), dev.empty(n), dev.empty(lib.drhip_normalize_scratch_floats(n))
+    for kind, tm, td in [(1, 0.0, 2.0), (2, 0.5, 1.5)] if n > 1 else [(0, 3.0, 1.0)]:
+        ok(lib, lib.drhip_normalize_f32(xd, y, n, kind, tm, td, scratch, None))
+        want = oracle.normalize_f64(x.reshape(1, 1, n), kind, tm, td).reshape(-1)
+        # (sums of n terms in a tree of at least 256 lanes: n / 2^18 terms one after the other, each step half a unit of 2^-23)
+        assert np.abs(dev.get(y, (n,)) - want).max() <= (16 + n / 2 ** 18) * 2.0 ** -23 * max(np.abs(want).max(), np.abs(x).max() * td / max(x.std(), 1e-3))
+
+
 def test_softmax(lib, dev, oracle):
     for n, scale in [(1000, 3.0), (10, 1.0), (5000, 5.0), (1, 1.0), (2048, 2.0), (2049, 2.0), (257, 1.0)]:
         x = rnd(n, scale=scale)
