@@ -443,12 +443,14 @@ conv3x3_direct_mfma_kernel(const float* __restrict__ in, const float* __restrict
     // 12 dwords of arguments, all of which arrive in SGPRs with the wave (nothing is read from the dispatch packet:
     // a scalar load in front of the first vector loads is a round trip of its own in every workgroup):
     // wh = W | H << 16, io = I | O << 16, WoMul / cfg & 31 = multiplier / shift of the division by Wo,
-    // cfg bit 5 = ReLU, cfg >> 8 = waves per workgroup.
+    // cfg bit 5 = ReLU, bit 6 = a global average behind the layer: out[tile][o] takes the sums over the tile's 32 pixels,
+    // cfg >> 8 = waves per workgroup.
     constexpr int OB = 32 * NT, KC = kDmKC;
     const int W = (int)(wh & 0xffffu), H = (int)(wh >> 16), I = (int)(io & 0xffffu), O = (int)(io >> 16);
     const int Wo = W / S, Ho = H / S;
     const FastDiv Wod = {(unsigned)Wo, WoMul, cfg & 31u};
     const int relu = (int)((cfg >> 5) & 1u), KW = (int)(cfg >> 8);
+    const bool sums = (cfg >> 6 & 1u) != 0;
     constexpr int NA = NT == 1 ? 2 : 1;     // accumulators per channel block: two independent MFMA chains at least
     extern __shared__ float part[];         // [KW][OB][kDmPartPitch]
 
@@ -584,9 +586,14 @@ conv3x3_direct_mfma_kernel(const float* __restrict__ in, const float* __restrict
         const int o = o0 + ol, pp = p0 + pl;
         float v = 0.0f;
         for (int k = 0; k < KW; ++k) v += part[(k * OB + ol) * kDmPartPitch + pl];
-        if (o < O && pp < P) {
-            v += biasValue;
-            if (relu) v = fmaxf(v, 0.0f);
+        v += biasValue;
+        if (relu) v = fmaxf(v, 0.0f);
+        if (sums) {
+            v = pp < P ? v : 0.0f;
+#pragma unroll
+            for (int k = 1; k < 32; k *= 2) v += __shfl_xor(v, k);
+            if (o < O && pl == 0) store_through(out + (size_t)blockIdx.x * O + o, v);
+        } else if (o < O && pp < P) {
             store_through(out + (size_t)o * P + pp, v);
         }
     };
@@ -740,8 +747,8 @@ extern "C" int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O) {
     return kw | (wide ? 0x10 : 0);
 }
 
-extern "C" int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* bias, float* out,
-                                             int W, int H, int I, int O, int stride, int relu, int variant, void* stream) {
+static int conv3x3_direct_mfma(const float* in, const float* F, const float* bias, float* out,
+                               int W, int H, int I, int O, int stride, int relu, bool sums, int variant, void* stream) {
     DRHIP_REQUIRE(in && F && out, "drhip_conv3x3_direct_mfma_f32: NULL tensor");
     DRHIP_REQUIRE(W > 0 && H > 0 && I > 0 && O > 0, "drhip_conv3x3_direct_mfma_f32: bad shape %dx%dx%d -> %d", W, H, I, O);
     DRHIP_REQUIRE(stride == 1 || stride == 2, "drhip_conv3x3_direct_mfma_f32: stride %d (1 or 2)", stride);
@@ -762,9 +769,19 @@ extern "C" int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, co
     const size_t ldsBytes = (size_t)kw * OB * kDmPartPitch * sizeof(float);
     hipStream_t s = as_stream(stream);
     const FastDiv dWo = make_fastdiv(Wo);
-#define DRHIP_DM(NTV, SV) launch((conv3x3_direct_mfma_kernel<NTV, SV>), grid, block, ldsBytes, s, in, F, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dWo.mul, dWo.shift | (relu ? 32u : 0u) | (unsigned)kw << 8)
+#define DRHIP_DM(NTV, SV) launch((conv3x3_direct_mfma_kernel<NTV, SV>), grid, block, ldsBytes, s, in, F, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dWo.mul, dWo.shift | (relu ? 32u : 0u) | (sums ? 64u : 0u) | (unsigned)kw << 8)
     if (wide) { if (stride == 1) DRHIP_DM(2, 1); else DRHIP_DM(2, 2); }
     else { if (stride == 1) DRHIP_DM(1, 1); else DRHIP_DM(1, 2); }
 #undef DRHIP_DM
     return launched("conv3x3_direct_mfma_kernel");
+}
+
+extern "C" int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* bias, float* out,
+                                             int W, int H, int I, int O, int stride, int relu, int variant, void* stream) {
+    return conv3x3_direct_mfma(in, F, bias, out, W, H, I, O, stride, relu, false, variant, stream);
+}
+
+extern "C" int drhip_conv3x3_direct_poolsum_f32(const float* in, const float* F, const float* bias, float* partials,
+                                                int W, int H, int I, int O, int stride, int relu, int variant, void* stream) {
+    return conv3x3_direct_mfma(in, F, bias, partials, W, H, I, O, stride, relu, true, variant, stream);
 }

@@ -334,6 +334,8 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
                 rc = drhip_conv_bank_maxpool2_f32(in, w, b, out, W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, relu, c->variant, stream_of(net));
             else if (c->drFusedPool)            // first layer + the 3x3/2 max pool behind it (out = the pool's buffer)
                 rc = drhip_conv3x3_pool3s2_f32(in, w, b, out, W, H, I, O, c->stride.s1, c->stride.s2, relu, stream_of(net));
+            else if (c->drDirectBank && c->drFusedAvgPool)
+                rc = drhip_conv3x3_direct_poolsum_f32(in, w, b, (float*)c->workspaceBuf, W, H, I, O, c->stride.s1, relu, c->variant, stream_of(net));
             else if (c->drDirectBank)
                 rc = drhip_conv3x3_direct_mfma_f32(in, w, b, out, W, H, I, O, c->stride.s1, relu, c->variant, stream_of(net));
             else if (c->drSplitBank)
@@ -366,7 +368,8 @@ gboolean conv_cleanup_layer(dR_Graph*, dR_Node* node) {
 }  // namespace
 
 int dr::avgpool_slices(const dR_Conv2d_Data* c) {
-    const int P = c->ishape.s0 * c->ishape.s1;
+    const int P = (c->ishape.s0 / c->stride.s1) * (c->ishape.s1 / c->stride.s2);
+    if (c->drDirectBank) return (P + 31) / 32;
     return c->drByPixel ? (P + drhip_conv1x1_pixels_tile(P) - 1) / drhip_conv1x1_pixels_tile(P) : drhip_conv1x1_poolsum_slices(P);
 }
 

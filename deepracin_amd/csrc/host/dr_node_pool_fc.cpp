@@ -146,13 +146,13 @@ gboolean fc_fill(dR_Graph* net, dR_Node* node) {
 }
 
 // Where a node that skipped its finishing kernel left its output: an FC node its slice sums, a
-// global average pooling behind a 1x1 convolution the convolution's per-tile pixel sums.
+// global average pooling behind a 1x1 or strided convolution the convolution's per-tile pixel sums.
 drhip_deferred_vec deferred_output_of(dR_Node* producer) {
     drhip_deferred_vec d;
     if (producer->type == tPooling) {
         dR_Node* conv = first_input(producer);
         dR_Conv2d_Data* c = (dR_Conv2d_Data*)conv->layer;
-        const int P = c->ishape.s0 * c->ishape.s1;
+        const int P = conv->oshape.s0 * conv->oshape.s1;
         d.partials = (const float*)c->workspaceBuf;
         d.bias = NULL;
         d.slices = avgpool_slices(c);

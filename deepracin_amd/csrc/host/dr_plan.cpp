@@ -131,7 +131,8 @@ dR_Node* pooled_input_of(const dR_Node* c) {
     return p;
 }
 
-// A global average pooling (one window = the whole map) behind a 1x1 convolution and in front of an
+// A global average pooling (one window = the whole map) behind a 1x1 convolution, or a strided 3x3 one of at most 64 tiles of
+// pixels (every workgroup of the reader adds all of them up; 28x28 128->192 3x3/2, the average and 192x1000 behind other layers: 2.3 us less), and in front of an
 // FC or softmax node: the convolution's epilogue sums its pixels per tile, the consumer adds the
 // tile sums and divides, and neither the convolution's tensor nor a pooling kernel is needed
 // (DR_FUSE_AVGPOOL=0 keeps them).  The pooled tensor may still be an output: the consumer stores it.
@@ -149,7 +150,9 @@ dR_Node* avgpool_fusable_producer(const dR_Node* p) {
     std::vector<dR_Node*> ins = nodes_of(p->previous_layers);
     if (ins.size() != 1) return nullptr;
     dR_Node* c = ins[0];
-    if (c->type != tConv2d || ((const dR_Conv2d_Data*)c->layer)->algo != drConv1x1Gemm) return nullptr;
+    if (c->type != tConv2d) return nullptr;
+    const dR_Conv2d_Data* cd = (const dR_Conv2d_Data*)c->layer;
+    if (cd->algo != drConv1x1Gemm && !(cd->drDirectBank && (long long)c->oshape.s0 * c->oshape.s1 <= 64 * 32)) return nullptr;
     if (tensor_wanted(c) || c->outputBuf || !c->next_layers || c->next_layers->length != 1) return nullptr;
     return c;
 }
@@ -454,7 +457,7 @@ gboolean dR_planBuffers(dR_Graph* net) {
             dR_Node* reader = nodes_of(n->next_layers)[0];
             if (!c3->drFire || c3->drFireNext || reader->type != tConv2d || (long long)n->oshape.s0 * n->oshape.s1 * n->oshape.s2 >= (1ll << 28)) continue;
             dR_Conv2d_Data* c = (dR_Conv2d_Data*)reader->layer;
-            if (!c->drFusedAvgPool || c->shape.s2 > 1024 || c->shape.s3 > 65535) continue;
+            if (c->algo != drConv1x1Gemm || !c->drFusedAvgPool || c->shape.s2 > 1024 || c->shape.s3 > 65535) continue;
             c3->drByPixel = c->drByPixel = TRUE;
         }
     }

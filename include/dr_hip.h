@@ -165,6 +165,10 @@ int drhip_conv3x3_direct_filter_layout_f32(const float* w /* [I][O][3][3] */, fl
 int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O);
 int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* bias, float* out,
                                   int W, int H, int I, int O, int stride, int relu, int variant, void* stream);
+/* With a global average behind it: partials[t*O + o] = sum over the pixels of tile t (32 pixels each, ceil(Wo*Ho/32) tiles), for a
+ * drhip_deferred_vec as drhip_conv1x1_poolsum_f32's. */
+int drhip_conv3x3_direct_poolsum_f32(const float* in, const float* F, const float* bias, float* partials,
+                                     int W, int H, int I, int O, int stride, int relu, int variant, void* stream);
 
 /* The same convolution for any odd filter and any stride on the bf16 matrix cores at fp32 accuracy: operands are split
  * into three bf16 parts each, which together hold all 24 significant bits of any fp32 number up to 2^111, and six partial

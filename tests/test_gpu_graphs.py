@@ -479,6 +479,36 @@ def test_conv_global_average_softmax_fused(oracle, gpu):
             assert rel_err(res["1"][k], want[2 + k]) <= LAYER_TOL and rel_err(res["1"][k], res["0"][k]) <= 1e-5
 
 
+@pytest.mark.parametrize("W,H,I,O,tail", [(29, 23, 64, 70, "fc"), (5, 2, 60, 33, "fc"), (20, 20, 96, 9, "softmax"), (86, 94, 64, 32, "fc"), (92, 90, 64, 32, "fc")])
+def test_global_average_behind_a_strided_layer(oracle, gpu, W, H, I, O, tail):
+    """A 3x3/2 layer that leaves its pixel sums to the reader of the average behind it, up to 64 tiles of pixels, and the kernels apart
+    (DR_FUSE_AVGPOOL=0)."""
+    st = configs._Streams(93)
+    Wo, Ho = W // 2, H // 2
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, 3, I, O, stride=2), {"op": "pool", "in": 1, "window": (Wo, Ho, 1), "stride": (Wo, Ho, 1), "kind": 1}]
+    spec.append(configs._fc(st, 2, O, 300, False) if tail == "fc" else {"op": "softmax", "in": 2})
+    x = configs.image_input(st, W, H, I)
+    want, res, launches = oracle.run_spec(spec, {0: x}), {}, {}
+    for mode in ("1", "0"):
+        os.environ["DR_FUSE_AVGPOOL"] = mode
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, [2, 3])
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], x)
+                assert g.lib.dR_apply(g.ptr) and g.lib.dR_apply(g.ptr)
+                res[mode] = [a.copy() for a in configs.fetch_chw(g)]
+                dr.graph_config(g).profilingGPU = 1
+                assert g.lib.dR_apply(g.ptr)
+                launches[mode] = g.lib.drhip_timing_count()
+        finally:
+            os.environ.pop("DR_FUSE_AVGPOOL", None)
+    assert launches["0"] - launches["1"] == (1 if Wo * Ho <= 64 * 32 else 0), launches
+    for k in range(2):
+        assert rel_err(res["1"][k], want[2 + k]) <= LAYER_TOL and rel_err(res["1"][k], res["0"][k]) <= 1e-5
+
+
 def test_squeezenet_with_normalization_node(oracle, gpu):
     """Config 4 with its per-image normalisation moved into the graph: raw U[0,255) image in, a
     Normalization node (mean 0, deviation 1) in front of conv1."""
