@@ -167,6 +167,8 @@ def load_library(path=None):
         "drhip_timing_count": (c_int, []),
         "drhip_timing_end": (c_int, [POINTER(c_float), c_int, POINTER(c_int)]),
         "drhip_conv2d_direct_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 9 + [vp]),
+        "drhip_conv3x3_image_avgpool2_usable": (c_int, [c_int] * 5),
+        "drhip_conv3x3_image_avgpool2_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 6 + [vp]),
         "drhip_conv_bank_usable": (c_int, [c_int] * 8),
         "drhip_conv_bank_floats": (c_size_t, [c_int] * 4),
         "drhip_conv_bank_layout_f32": (c_int, [vp, vp] + [c_int] * 4 + [vp]),

@@ -107,7 +107,7 @@ winograd_filter_transform_kernel(const float* __restrict__ w, float* __restrict_
 // is a round trip of its own at the start of every workgroup (~0.07 us each).
 //   wh = W | H << 16, io = I | O << 16 (each at most 65535),
 //   mulX, mulTB = multipliers of the divisions by tilesX and by the number of tile panels,
-//   cfg0 = shiftX | shiftTB << 5 | epilogue flags << 10 (2 bits) | vec2 << 12 | splits << 13 (16 bits) | tiered << 30 | joined << 31,
+//   cfg0 = shiftX | shiftTB << 5 | epilogue flags << 10 (2 bits) | vec2 << 12 | splits << 13 (16 bits) | average << 29 (FEWC) | tiered << 30 | joined << 31,
 //   cfg1 = chunks per split (16 bits) | log2 splits << 24 (joined launches)
 //   tiered launches: the splits field holds log2 splits of up to four tiers (4 bits each) and cfg1 their panel
 //   counts per XCD (8 bits each)
@@ -460,7 +460,11 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                 if (eTileOk && o < O) {
                     if (bias) { const float bv = kBiasEarly ? biasEarly[kBiasEarly ? q : 0] : bias[o]; y00 += bv; y01 += bv; y10 += bv; y11 += bv; }
                     if (relu & kEpiRelu) { y00 = fmaxf(y00, 0.f); y01 = fmaxf(y01, 0.f); y10 = fmaxf(y10, 0.f); y11 = fmaxf(y11, 0.f); }
-                    if (relu & kEpiMaxPool2)        // W, H even: the tile is one window of a 2x2/2 max pool
+                    // W, H even: the tile is one window of a 2x2/2 pooling.  (An average only behind images, by the pooling kernel's order:
+                    // 224x224 3->64 and the pooling 6.3 + 5.1 us -> 6.1; in the other kernels the code alone would cost more than it gains.)
+                    if (FEWC && (cfg0 >> 29 & 1u))
+                        store1_through(out + (size_t)o * (plane >> 2) + (size_t)(oy >> 1) * (W >> 1) + (ox >> 1), (((y00 + y01) + y10) + y11) / 4.0f);
+                    else if (relu & kEpiMaxPool2)
                         store1_through(out + (size_t)o * (plane >> 2) + (size_t)(oy >> 1) * (W >> 1) + (ox >> 1), fmaxf(fmaxf(y00, y01), fmaxf(y10, y11)));
                     else
                         wino_store_tile(out + (size_t)o * plane + (size_t)oy * W + ox, W, H, ox, oy, vec2, y00, y01, y10, y11);
@@ -815,6 +819,8 @@ static bool wino_tiers(int nBlocks, int nChunks, int cus, WinoTiers* t) {
 
 // Workspace: [splits][panel][o in panel][tile in panel] partial 2x2 tiles (float4 each); tiered launches: one
 // panel-sized region per workgroup of the grid.
+constexpr int kEpiAvgPool2 = 4;     // (inside this file: of the kernels for images)
+
 template <int NT, int TB>
 static int launch_wino(const float* in, const float* U, const float* bias, float* out, float* workspace,
                        int W, int H, int I, int O, int relu, const WinoCfg& c, hipStream_t s) {
@@ -838,7 +844,7 @@ static int launch_wino(const float* in, const float* U, const float* bias, float
     }
     const WinoPackedArgs pa = {(unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dx.mul, dtb.mul,
                                dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | (unsigned)g.splits << 13 |
-                                   (joined ? 1u << 31 : 0u),
+                                   (relu & kEpiAvgPool2 ? 1u << 29 : 0u) | (joined ? 1u << 31 : 0u),
                                (unsigned)g.chunksPerSplit | (joined ? (unsigned)__builtin_ctz(g.splits) << 24 : 0u)};
     // joined: one grid row, the splits of a panel side by side on one XCD (see the kernel)
     const dim3 grid = joined ? dim3(gridX * g.splits) : dim3(gridX, g.splits);
@@ -1038,4 +1044,22 @@ extern "C" int drhip_conv3x3_winograd_f32(const float* in, const float* U, const
     if (c.nt == 1) return launch_wino<1, 32>(in, U, bias, out, workspace, W, H, I, O, relu, c, s);
     if (c.nt == 2) return launch_wino<2, 32>(in, U, bias, out, workspace, W, H, I, O, relu, c, s);
     return launch_wino<4, 32>(in, U, bias, out, workspace, W, H, I, O, relu, c, s);
+}
+
+extern "C" int drhip_conv3x3_image_avgpool2_usable(int W, int H, int I, int O, int variant) {
+    WinoCfg c;
+    if (W < 2 || H < 2 || ((W | H) & 1) || I < 1 || I > 4 || O < 1 || W > 65535 || H > 65535 || O > 65535 || variant <= 0 || !wino_variant(variant, &c)) return 0;
+    if ((long long)W * H * I >= (1ll << 29) || (long long)W * H * O >= (1ll << 31)) return 0;
+    return c.tb == 32 && c.nt <= 2 && c.waveSets != 2 && !c.tiered && wino_geom(W, H, I, O, c).splits == 1;
+}
+
+extern "C" int drhip_conv3x3_image_avgpool2_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int relu, int variant, void* stream) {
+    DRHIP_REQUIRE(in && U && out, "drhip_conv3x3_image_avgpool2_f32: NULL tensor");
+    DRHIP_REQUIRE(((size_t)U & 15) == 0, "drhip_conv3x3_image_avgpool2_f32: transformed filters must be 16-byte aligned");
+    DRHIP_REQUIRE(drhip_conv3x3_image_avgpool2_usable(W, H, I, O, variant), "drhip_conv3x3_image_avgpool2_f32: variant %#x does not cover %dx%dx%d -> %d", variant, W, H, I, O);
+    WinoCfg c;
+    wino_variant(variant, &c);
+    const int flags = (relu ? kEpiRelu : 0) | kEpiAvgPool2;
+    hipStream_t s = as_stream(stream);
+    return c.nt == 1 ? launch_wino<1, 32>(in, U, bias, out, nullptr, W, H, I, O, flags, c, s) : launch_wino<2, 32>(in, U, bias, out, nullptr, W, H, I, O, flags, c, s);
 }

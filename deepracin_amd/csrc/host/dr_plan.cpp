@@ -88,16 +88,19 @@ dR_Node* pool_fusable_producer(const dR_Node* p) {
     const char* env = getenv("DR_FUSE_POOL");
     if (env && strcmp(env, "0") == 0) return nullptr;
     const dR_Pooling_Data* pd = (const dR_Pooling_Data*)p->layer;
-    if (pd->poolingType != tMax || pd->shape.s3 != 1 || pd->stride.s1 != 2 || pd->stride.s2 != 2 || pd->stride.s3 != 1) return nullptr;
+    const bool average = pd->poolingType == tAverage;
+    if ((pd->poolingType != tMax && !average) || pd->shape.s3 != 1 || pd->stride.s1 != 2 || pd->stride.s2 != 2 || pd->stride.s3 != 1) return nullptr;
     const bool two = pd->shape.s1 == 2 && pd->shape.s2 == 2, three = pd->shape.s1 == 3 && pd->shape.s2 == 3;
-    if (!two && !three) return nullptr;
+    if (!two && (!three || average)) return nullptr;
     std::vector<dR_Node*> ins = nodes_of(p->previous_layers);
     if (ins.size() != 1) return nullptr;
     dR_Node* c = ins[0];
     if (c->type != tConv2d) return nullptr;
     const dR_Conv2d_Data* cd = (const dR_Conv2d_Data*)c->layer;
     if (tensor_wanted(c) || c->outputBuf || !c->next_layers || c->next_layers->length != 1) return nullptr;
-    if (two) {
+    if (average) {
+        if (cd->algo != drConvWinograd || cd->drWinoSplit || !drhip_conv3x3_image_avgpool2_usable(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->variant)) return nullptr;
+    } else if (two) {
         const bool even = !((c->oshape.s0 | c->oshape.s1) & 1);
         const bool bank = cd->drSplitBank && drhip_conv_bank_pick_variant(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->shape.s0, cd->shape.s1, cd->stride.s1, cd->stride.s2, 1);
         if (!bank && !(cd->algo == drConvWinograd && even)) return nullptr;
@@ -358,7 +361,7 @@ gboolean dR_planBuffers(dR_Graph* net) {
         if (n->type == tPooling) {
             dR_Node* c = pool_fusable_producer(n);
             ((dR_Pooling_Data*)n->layer)->drFused = c != nullptr;
-            if (c) { ((dR_Conv2d_Data*)c->layer)->drFusedPool = TRUE; parent[c] = std::make_pair(n, 0); }
+            if (c) { ((dR_Conv2d_Data*)c->layer)->drFusedPool = TRUE; ((dR_Conv2d_Data*)c->layer)->drPoolAverage = ((dR_Pooling_Data*)n->layer)->poolingType == tAverage; parent[c] = std::make_pair(n, 0); }
             else if ((c = avgpool_fusable_producer(n)) != nullptr) {
                 dR_Node* consumer = nodes_of(n->next_layers)[0];
                 if (consumer->type == tFullyConnected) ((dR_FC_Data*)consumer->layer)->drDeferredInput = n;

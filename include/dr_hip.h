@@ -259,6 +259,11 @@ size_t drhip_conv3x3_winograd_workspace_floats(int W, int H, int I, int O, int v
 int drhip_conv3x3_winograd_workspace_prepare_f32(float* workspace, size_t floats, void* stream);
 int drhip_conv3x3_winograd_join_timeouts(unsigned* count);
 
+/* A layer over an image (up to 4 channels, even sides) with a 2x2/2 average pooling behind it: out[O][H/2][W/2].  For the variants that
+ * drhip_conv3x3_image_avgpool2_usable says so of; filters as above. */
+int drhip_conv3x3_image_avgpool2_usable(int W, int H, int I, int O, int variant);
+int drhip_conv3x3_image_avgpool2_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int relu, int variant, void* stream);
+
 /* The same convolution with the same fusions on the bf16 matrix cores at fp32 accuracy (operands in three bf16 parts, six
  * partial products, fp32 accumulation; what does not come out finite is worked out again in fp32), for large layers.  F is the transformed and split filter bank, made once at
  * prepare time from w [I][O][3][3]; drhip_conv3x3_winograd_split_filter_floats(I,O) floats, 16-byte aligned.

@@ -145,6 +145,35 @@ def test_maxpool_fused_into_convolution(oracle, gpu):
         assert dr.node_struct(nodes[4]).drLastKernelMs == 0.0 and dr.node_struct(nodes[3]).drLastKernelMs > 0.0
 
 
+@pytest.mark.parametrize("W,H,I,O,relu", [(224, 224, 3, 64, True), (2, 2, 1, 1, False), (34, 18, 4, 33, False), (98, 66, 2, 70, True), (124, 70, 4, 33, False), (99, 66, 3, 33, False), (98, 66, 5, 33, True)])
+def test_average_pooling_behind_an_image_layer(oracle, gpu, W, H, I, O, relu):
+    """A 3x3 layer over an image and a 2x2/2 average pooling in one launch: the two kernels' numbers (DR_FUSE_POOL=0); small and odd maps
+    and layers of five channels stay apart."""
+    st = configs._Streams(95)
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, 3, I, O, relu=relu), {"op": "pool", "in": 1, "window": (2, 2, 1), "stride": (2, 2, 1), "kind": 1}]
+    x = configs.image_input(st, W, H, I)
+    want, res, launches = oracle.run_spec(spec, {0: x}), {}, {}
+    for mode in ("1", "0"):
+        os.environ["DR_FUSE_POOL"] = mode
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, [2])
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], x)
+                assert g.lib.dR_apply(g.ptr)
+                res[mode] = configs.fetch_chw(g)[0].copy()
+                dr.graph_config(g).profilingGPU = 1
+                assert g.lib.dR_apply(g.ptr)
+                launches[mode] = g.lib.drhip_timing_count()
+        finally:
+            os.environ.pop("DR_FUSE_POOL", None)
+    fused = bool(dr.load_library().drhip_conv3x3_image_avgpool2_usable(W, H, I, O, dr.load_library().drhip_conv3x3_winograd_pick_variant(W, H, I, O)))
+    assert launches["0"] - launches["1"] == fused and fused == (W % 2 == 0 and I <= 4 and W > 40)      # (small maps: the 16-tile kernel)
+    assert np.array_equal(res["1"], res["0"])
+    assert_close(res["1"], want[2], terms=9 * I)
+
+
 def test_maxpool_taken_on_load_by_the_1x1_layer_behind_it(oracle, gpu):
     """SqueezeNet's pool3 / pool5 pattern: fire module -> 3x3/2 max pool -> squeeze 1x1.  With only the last
     tensor requested the squeeze layer pools while it loads (no pooling launch, no pooled tensor); with
