@@ -13,7 +13,8 @@
 //     [slice][pixel][channel], and the next launch adds the slices (in order: the results do not depend on timing), bias and ReLU
 //     while it loads them.
 //   * Every load of a workgroup is issued at its start: the input, the filters (16 bytes per lane are four k-steps, see below)
-//     and the next layer's.
+//     and the next layer's; of the filters 20 packs, for behind other layers a pack is a trip to memory (12 / 16 / 20 / 24 packs: SqueezeNet at
+//     224x224 57.8 / 57.3 / 57.4 / 57.5 us a pass, at 451x299 84.7 / 83.9 / 83.1 / 82.8).
 //   * Four waves, one per SIMD, and few instructions: what a wave does once is paid per wave, 4 clocks an instruction.  A first form with
 //     eight waves and shapes known at run time issued its first loads a microsecond after its start and took 430 clocks for
 //     the four MFMAs of an item.  So the item loop is unrolled over constants (S/16 is a template parameter, rows of the patch lie 12
@@ -43,7 +44,7 @@ typedef float f32x2f __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4f __attribute__((ext_vector_type(4)));
 constexpr int kAuxThrough16 = 1 | 16;           // sc0 sc1: written through to memory
 constexpr int kFireThreads = 256;
-constexpr int kFireAhead = 12;                  // packs of filters a wave has under way at most
+constexpr int kFireAhead = 20;                  // packs of filters a wave has under way at most
 constexpr int kFireSlices = 8;                  // slices of a quad of the patch that are under way together
 constexpr int kFireRow = 12;                    // pixels from row to row of the patch in LDS
 
