@@ -62,14 +62,15 @@ __global__ void __launch_bounds__(256) copy_from_host_kernel(float* __restrict__
 }
 
 // dst [C][P] (device) = src [P][C] (pinned host memory): an interleaved image on its way to the planar layout.  A
-// workgroup takes 1024 pixels: it reads them over the bus in their own order, 16 bytes per lane and turn (a wave's load
+// workgroup of two waves takes 512 pixels: it reads them over the bus in their own order, 16 bytes per lane and turn (a wave's load
 // is 1 KiB in a row, which is what the bus wants; the bus is what bounds this kernel), and every lane writes four
 // pixels of each channel out of LDS.  The array may end anywhere: the ragged end is moved sample by sample.
 // (224x224x3: 5.6 us on top of the launch, 107 GB/s through memory, like the plain copy above; numpy's transposition
-// of the same array takes the host 70 us.)
-constexpr int kHwcPixels = 1024;
+// of the same array takes the host 70 us.  Four waves and 1024 pixels wait longer for their last sample: a photograph of 451x299 in
+// and its classes out 152.8 us, 148.5 with two; one wave and 256 pixels 156.7; at 224x224 all the same.)
+constexpr int kHwcPixels = 512;
 template <int C>
-__global__ void __launch_bounds__(256) hwc_from_host_kernel(float* __restrict__ dst, const float* __restrict__ src, size_t P, size_t pixels) {
+__global__ void __launch_bounds__(128) hwc_from_host_kernel(float* __restrict__ dst, const float* __restrict__ src, size_t P, size_t pixels) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));     // (a channel plane starts at any multiple of 4 bytes)
     __shared__ __attribute__((aligned(16))) float px[kHwcPixels * C];
@@ -79,11 +80,11 @@ __global__ void __launch_bounds__(256) hwc_from_host_kernel(float* __restrict__ 
     if (n == kHwcPixels) {
         f4 v[C];
 #pragma unroll
-        for (int k = 0; k < C; ++k) v[k] = __builtin_nontemporal_load((const f4*)(src + p0 * C) + t + 256 * k);
+        for (int k = 0; k < C; ++k) v[k] = __builtin_nontemporal_load((const f4*)(src + p0 * C) + t + 128 * k);
 #pragma unroll
-        for (int k = 0; k < C; ++k) ((f4*)px)[t + 256 * k] = v[k];
+        for (int k = 0; k < C; ++k) ((f4*)px)[t + 128 * k] = v[k];
     } else {
-        for (int i = t; i < n * C; i += 256) px[i] = src[p0 * C + i];
+        for (int i = t; i < n * C; i += 128) px[i] = src[p0 * C + i];
     }
     __syncthreads();
 #pragma unroll
@@ -490,7 +491,7 @@ int drhip_upload_staged_interleaved(void* handle, float* dst, const float* src, 
             const size_t begin = begins[piece], len = lens[piece];
             memcpy(mem + begin * C, src + begin * C, len * C * sizeof(float));
             const dim3 grid((unsigned)((len + kHwcPixels - 1) / kHwcPixels));
-            auto go = [&](auto kernel) { launch(kernel, grid, dim3(256), 0, as_stream(stream), dst + begin, (const float*)(mem + begin * C), pixels, len); };
+            auto go = [&](auto kernel) { launch(kernel, grid, dim3(128), 0, as_stream(stream), dst + begin, (const float*)(mem + begin * C), pixels, len); };
             if (channels == 2) go(hwc_from_host_kernel<2>);
             else if (channels == 3) go(hwc_from_host_kernel<3>);
             else go(hwc_from_host_kernel<4>);
