@@ -1,6 +1,7 @@
-// Softmax over a flat fp32 vector in ONE workgroup of sixteen waves: wavefront-level butterfly
-// reductions (ds_bpermute via __shfl_xor) for max and sum, one small LDS exchange between the waves;
-// vectors of up to 2048 elements are read once and kept in registers.  (Sixteen waves, not four: a lane then
+// Softmax over a flat fp32 vector in ONE workgroup of sixteen waves: reductions within a wave in registers, one
+// small LDS exchange between the waves for the maximum and one for the sum, behind barriers that wait for LDS only: the
+// logits on their way to memory or the host stay under way (0.45 us a pass less than with butterflies and full barriers).
+// Vectors of up to 2048 elements are read once and kept in registers.  (Sixteen waves, not four: a lane then
 // finishes one or two logits of a deferred input, and each of them is a round of dependent loads -- 1000 logits
 // behind 16 slices: 4.0 against 8.8 us.)
 //
@@ -11,30 +12,47 @@
 #include "drhip_common.hpp"
 
 #include <cfloat>
+#include <type_traits>
 
 namespace drhip {
 
 constexpr int kSoftmaxThreads = 1024;
 constexpr int kSoftmaxRegs = 2;     // vectors of up to 2048 elements live in registers: one read of x
 
-__device__ inline float wave_max(float v) {
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-__device__ inline float wave_sum(float v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// Maximum / sum over a wave, in registers: within rows of sixteen lanes, across two rows, across four; the last lane has it.  (A
+// butterfly through LDS is six dependent trips of 100 clocks.)
+template <bool MAX>
+__device__ inline float wave_reduce(float v) {
+    constexpr float none = MAX ? -FLT_MAX : 0.0f;
+    auto with = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+    auto from = [none](float a, auto ctrl, auto rows) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, a), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+    };
+    using std::integral_constant;
+    v = with(v, from(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{}));      // row_shr:1
+    v = with(v, from(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{}));
+    v = with(v, from(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{}));
+    v = with(v, from(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{}));
+    v = with(v, from(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{}));      // row_bcast:15
+    v = with(v, from(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{}));      // row_bcast:31
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-// Workgroup-wide maximum / sum; the result is valid in every lane.  `red` has one slot per wave.
+// LDS only: what has been stored for other kernels or the host stays under way.
+__device__ inline void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Workgroup-wide maximum / sum; the result is valid in every lane.  `red` has one slot per wave, and is of this reduction alone.
 template <bool MAX>
 __device__ inline float block_reduce(float v, float* red) {
     constexpr int nwaves = kSoftmaxThreads / kWave;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    v = MAX ? wave_max(v) : wave_sum(v);
-    __syncthreads();                    // red may still be read from the previous reduction
+    v = wave_reduce<MAX>(v);
     if (lane == 0) red[wave] = v;
-    __syncthreads();
+    lds_barrier();
     float r = red[0];
 #pragma unroll
     for (int w = 1; w < nwaves; ++w) r = MAX ? fmaxf(r, red[w]) : r + red[w];
@@ -47,7 +65,7 @@ __device__ inline float block_reduce(float v, float* red) {
 template <bool SMALL>
 __global__ void __launch_bounds__(kSoftmaxThreads)
 softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef, drhip_push push) {    // no __restrict__: x may become y
-    __shared__ float red[kSoftmaxThreads / kWave];
+    __shared__ __attribute__((aligned(16))) float red[2][kSoftmaxThreads / kWave];
     const int tid = threadIdx.x;
     if (SMALL) {                                    // n <= kSoftmaxThreads * kSoftmaxRegs
         float v[kSoftmaxRegs];
@@ -72,14 +90,14 @@ softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef, drhip_p
         float m = -FLT_MAX;
 #pragma unroll
         for (int u = 0; u < kSoftmaxRegs; ++u) m = fmaxf(m, v[u]);
-        m = block_reduce<true>(m, red);
+        m = block_reduce<true>(m, red[0]);
         float s = 0.0f;
 #pragma unroll
         for (int u = 0; u < kSoftmaxRegs; ++u) {
             v[u] = (tid + u * kSoftmaxThreads < n) ? expf(v[u] - m) : 0.0f;
             s += v[u];
         }
-        const float inv = 1.0f / block_reduce<false>(s, red);
+        const float inv = 1.0f / block_reduce<false>(s, red[1]);
 #pragma unroll
         for (int u = 0; u < kSoftmaxRegs; ++u) {
             const int i = tid + u * kSoftmaxThreads;
@@ -99,10 +117,10 @@ softmax_kernel(const float* x, float* y, int n, drhip_deferred_vec xdef, drhip_p
     }
     float m = -FLT_MAX;
     for (int i = tid; i < n; i += kSoftmaxThreads) m = fmaxf(m, x[i]);
-    m = block_reduce<true>(m, red);
+    m = block_reduce<true>(m, red[0]);
     float s = 0.0f;
     for (int i = tid; i < n; i += kSoftmaxThreads) s += expf(x[i] - m);
-    const float inv = 1.0f / block_reduce<false>(s, red);
+    const float inv = 1.0f / block_reduce<false>(s, red[1]);
     for (int i = tid; i < n; i += kSoftmaxThreads) store_through(y + i, expf(x[i] - m) * inv);
 }
 
@@ -116,7 +134,8 @@ constexpr int kFcSoftmaxGroups = 32;                // T at most
 __global__ void __launch_bounds__(kSoftmaxThreads)
 fc_softmax_kernel(const float* __restrict__ Wt, const float* x, const float* __restrict__ bias, float* z, float* y, int K, int N, int T, unsigned mulN, unsigned shN, int relu,
                   drhip_deferred_vec xdef, drhip_push push) {
-    __shared__ float xs[1024], part[kSoftmaxThreads], red[kSoftmaxThreads / kWave];
+    __shared__ float xs[1024], part[kSoftmaxThreads];
+    __shared__ __attribute__((aligned(16))) float red[2][kSoftmaxThreads / kWave];
     const int tid = threadIdx.x;
     const FastDiv nd = {(unsigned)N, mulN, shN};
     const int g = fast_div(tid, nd), n = tid - g * N;
@@ -127,7 +146,7 @@ fc_softmax_kernel(const float* __restrict__ Wt, const float* x, const float* __r
     const float b = bias && tid < N ? bias[tid] : 0.0f;
     const float xv = tid < K ? (xdef.partials ? deferred_element(xdef, tid) : x[tid]) : 0.0f;
     if (tid < K) xs[tid] = xv;
-    __syncthreads();
+    lds_barrier();
     float s = 0.0f;
     for (int k0 = g; k0 < K; k0 += kFcSoftmaxRows * T) {
 #pragma unroll
@@ -138,7 +157,7 @@ fc_softmax_kernel(const float* __restrict__ Wt, const float* x, const float* __r
         }
     }
     if (g < T) part[g * N + n] = s;
-    __syncthreads();
+    lds_barrier();
     float v = -FLT_MAX;
     if (tid < N) {
         v = part[tid];
@@ -149,9 +168,9 @@ fc_softmax_kernel(const float* __restrict__ Wt, const float* x, const float* __r
         if (push.host && push.atInput != 0xffffffffu) push_value(push, push.atInput + tid, v);
     }
     if (xdef.partials && xdef.finished && tid < K) xdef.finished[tid] = xv;
-    const float m = block_reduce<true>(v, red);
+    const float m = block_reduce<true>(v, red[0]);
     const float e = tid < N ? expf(v - m) : 0.0f;
-    const float inv = 1.0f / block_reduce<false>(e, red);
+    const float inv = 1.0f / block_reduce<false>(e, red[1]);
     if (tid < N) {
         store_through(y + tid, e * inv);
         if (push.host) push_value(push, push.at + tid, e * inv);
