@@ -310,7 +310,7 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
     switch (c->algo) {
         case drConvWinograd: {
             const int flags = (relu ? DRHIP_EPILOGUE_RELU : 0) | (c->drFusedPool ? DRHIP_EPILOGUE_MAXPOOL2 : 0);
-            rc = c->drFusedPool && c->drPoolAverage ? drhip_conv3x3_image_avgpool2_f32(in, w, b, out, W, H, I, O, relu, c->variant, stream_of(net))
+            rc = c->drFusedPool && c->drPoolAverage ? drhip_conv3x3_image_avgpool2_f32(in, w, b, dev_out((dR_Node*)node->next_layers->first->element), W, H, I, O, relu, c->variant, stream_of(net))
                : c->drWinoSplit ? drhip_conv3x3_winograd_split_f32(in, w, b, out, W, H, I, O, flags, c->variant, (float*)c->workspaceBuf, stream_of(net))
                                 : drhip_conv3x3_winograd_f32(in, w, b, out, W, H, I, O, flags, c->variant, (float*)c->workspaceBuf, stream_of(net));
             break;

@@ -361,7 +361,12 @@ gboolean dR_planBuffers(dR_Graph* net) {
         if (n->type == tPooling) {
             dR_Node* c = pool_fusable_producer(n);
             ((dR_Pooling_Data*)n->layer)->drFused = c != nullptr;
-            if (c) { ((dR_Conv2d_Data*)c->layer)->drFusedPool = TRUE; ((dR_Conv2d_Data*)c->layer)->drPoolAverage = ((dR_Pooling_Data*)n->layer)->poolingType == tAverage; parent[c] = std::make_pair(n, 0); }
+            if (c) {
+                dR_Conv2d_Data* cd = (dR_Conv2d_Data*)c->layer;
+                cd->drFusedPool = TRUE;
+                cd->drPoolAverage = ((dR_Pooling_Data*)n->layer)->poolingType == tAverage;
+                if (!cd->drPoolAverage) parent[c] = std::make_pair(n, 0);       // (an average goes to the pooling's buffer from here)
+            }
             else if ((c = avgpool_fusable_producer(n)) != nullptr) {
                 dR_Node* consumer = nodes_of(n->next_layers)[0];
                 if (consumer->type == tFullyConnected) ((dR_FC_Data*)consumer->layer)->drDeferredInput = n;
@@ -510,6 +515,11 @@ gboolean dR_planBuffers(dR_Graph* net) {
                 Root& rp = touch(root_of(in, nullptr));
                 rp.lastUse = std::max(rp.lastUse, n->drSchedulePos);
             }
+        // a layer that averages writes the pooling's tensor before that node's turn
+        if (n->type == tConv2d && ((dR_Conv2d_Data*)n->layer)->drFusedPool && ((dR_Conv2d_Data*)n->layer)->drPoolAverage) {
+            Root& rp = touch(root_of(nodes_of(n->next_layers)[0], nullptr));
+            rp.firstDef = std::min(rp.firstDef, n->drSchedulePos);
+        }
         // a convolution that pools while loading reads the tensor in front of the pooling node
         if (n->type == tConv2d && ((dR_Conv2d_Data*)n->layer)->drPooledInput) {
             for (dR_Node* p : nodes_of(((dR_Conv2d_Data*)n->layer)->drPooledInput->previous_layers)) {
