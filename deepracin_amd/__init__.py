@@ -121,6 +121,7 @@ def load_library(path=None):
         "dR_getFeedNodeInputShape": (POINTER(Shape3), [vp]),
         "dR_feedDataHWC": (None, [vp, vp, vp]),
         "dR_downloadOutputs": (c_int, [vp, POINTER(vp), c_int]),
+        "dR_applyAhead": (c_int, [vp]),
         "dR_applyAndDownload": (c_int, [vp, POINTER(vp), c_int]),
         "dR_downloadArray": (None, [vp, c_char_p, vp, c_size_t, c_size_t, vp]),
         "dR_uploadArray": (c_int, [vp, c_char_p, vp, c_size_t, c_size_t, vp]),
@@ -366,19 +367,17 @@ def _from_chw(graph, flat, shape):
 
 def download_outputs(graph, squeeze=True):
     """Fetch every output buffer (blocking) in the graph's interface layout."""
-    return _outputs(graph, squeeze, False)
+    return _outputs(graph, squeeze)
 
 
-def _outputs(graph, squeeze, run):
+def _outputs(graph, squeeze):
     n = min(graph.num_outputs, 10)
     shapes = [node.out_shape for node in graph.outnodes[:n]]
     if None in shapes:          # not prepared: there are none yet
         return []
     flats = [np.empty(s[0] * s[1] * s[2], np.float32) for s in shapes]
     hosts = (c_void_p * max(n, 1))(*[f.__array_interface__["data"][0] for f in flats])
-    got = (graph.lib.dR_applyAndDownload if run else graph.lib.dR_downloadOutputs)(graph.ptr, hosts, n)
-    if run and got < 0:
-        raise RuntimeError("DR Error: deepRACIN apply failed!")
+    got = graph.lib.dR_downloadOutputs(graph.ptr, hosts, n)
     if n and not got:
         raise RuntimeError("DR Error: deepRACIN downloading the outputs failed!")
     outs = [_from_chw(graph, f, s) for f, s in zip(flats[:got], shapes)]
@@ -387,10 +386,9 @@ def _outputs(graph, squeeze, run):
 
 def apply(graph):
     """Run the graph once and return the outputs (reference :444-465)."""
-    if None in [node.out_shape for node in graph.outnodes]:         # not prepared
-        if not graph.lib.dR_apply(graph.ptr):
-            raise RuntimeError("DR Error: deepRACIN apply failed!")
-    return _outputs(graph, True, True)
+    if not graph.lib.dR_applyAhead(graph.ptr):          # (the arrays are made while it runs)
+        raise RuntimeError("DR Error: deepRACIN apply failed!")
+    return _outputs(graph, True)
 
 
 def mark_as_output(node):

@@ -573,6 +573,11 @@ int drhip_push_begin(void* handle, size_t floats, drhip_push* push) {
     return DRHIP_OK;
 }
 
+int drhip_push_current(void* handle, const drhip_push* push) {
+    const Staging* s = (const Staging*)handle;
+    return s && push && push->host == (const float*)s->down && push->value == s->seq;
+}
+
 int drhip_push_collect(void* handle, const drhip_push* push, int count, float* const* dst, const unsigned* at, const size_t* floats, void* stream) {
     Staging* s = (Staging*)handle;
     DRHIP_REQUIRE(s && push && push->host == (float*)s->down && count >= 0 && (count == 0 || (dst && at && floats)), "drhip_push_collect: bad arguments");

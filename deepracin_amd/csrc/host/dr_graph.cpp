@@ -262,10 +262,19 @@ void dR_feedDataHWC(dR_Graph* net, dR_Node* feednode, gfloat* data) {
     dR_uploadArray(net, (gchar*)"", planes.data(), 0, planes.size() * sizeof(float), feednode->outputBuf->buf);
 }
 
+struct Pending { drhip_push push; int count; unsigned at[2]; size_t floats[2]; };      // what dR_Graph::drPending holds
+
 gint dR_downloadOutputs(dR_Graph* net, gfloat** hosts, gint n) {
     if (!net->prepared || n < 0 || (n > 0 && !hosts)) {
         say("dR_downloadOutputs: the graph is not prepared, or no arrays were given\n");
         return 0;
+    }
+    Pending* pushed = (Pending*)net->drPending;
+    if (pushed && pushed->count > 0) {                  // on their way, unless something else has used the area since
+        const Pending p = *pushed;
+        pushed->count = 0;
+        const int k = n < p.count ? n : p.count;
+        if (drhip_push_current(net->drStaging, &p.push)) return device_failed(net, drhip_push_collect(net->drStaging, &p.push, k, hosts, p.at, p.floats, stream_of(net)), "dR_downloadOutputs") ? 0 : k;
     }
     const float* src[10];
     size_t floats[10];
@@ -319,6 +328,7 @@ static bool tensor_fused_away(const dR_Node* n) {
 
 gboolean dR_apply(dR_Graph* net) {
     if (!net->prepared) { say("dR_apply: graph is not prepared. Call dR_prepare first! \n"); return FALSE; }
+    if (net->drPending) ((Pending*)net->drPending)->count = 0;      // (of an earlier pass)
     dR_ClConfig* cc = net->clConfig;
     const bool profGPU = net->config->profilingGPU, profCPU = net->config->profilingCPU;
     if (net->config->debugInfo) say("Applying graph...\n");
@@ -424,32 +434,35 @@ static dR_Node* all_outputs_node(const dR_Graph* net) {
     return last;
 }
 
+gboolean dR_applyAhead(dR_Graph* net) {
+    const char* replay = getenv("DR_HIPGRAPH");
+    const bool plain = net->prepared && net->drStaging && !net->config->profilingGPU && net->debugLayer < 0 && !net->drGraphExec && !(replay && strcmp(replay, "1") == 0);
+    dR_Node* last = plain ? all_outputs_node(net) : NULL;
+    const unsigned values = last ? (unsigned)(last->oshape.s0 * last->oshape.s1 * last->oshape.s2) : 0;
+    Pending p = {};
+    if (!last || drhip_push_begin(net->drStaging, 2 * (size_t)values, &p.push) != DRHIP_OK) return dR_apply(net);
+    for (dR_Node* node : nodes_of(net->output_layers)) {
+        p.at[p.count] = node == last ? 0 : values;
+        p.floats[p.count++] = values;
+        if (node != last) p.push.atInput = values;
+    }
+    net->drPush = &p.push;
+    net->drPushNode = last;
+    const gboolean ok = dR_apply(net);
+    net->drPush = NULL;
+    net->drPushNode = NULL;
+    if (!ok) return FALSE;
+    if (!net->drPending) net->drPending = zalloc<Pending>();
+    *(Pending*)net->drPending = p;
+    return TRUE;
+}
+
 gint dR_applyAndDownload(dR_Graph* net, gfloat** hosts, gint n) {
     if (!net->prepared || n < 0 || (n > 0 && !hosts)) {
         say("dR_applyAndDownload: the graph is not prepared, or no arrays were given\n");
         return -1;
     }
-    const char* replay = getenv("DR_HIPGRAPH");
-    const bool plain = net->drStaging && !net->config->profilingGPU && net->debugLayer < 0 && !net->drGraphExec && !(replay && strcmp(replay, "1") == 0);
-    dR_Node* last = plain && n >= net->output_layers->length ? all_outputs_node(net) : NULL;
-    drhip_push push;
-    const unsigned values = last ? (unsigned)(last->oshape.s0 * last->oshape.s1 * last->oshape.s2) : 0;
-    if (!last || drhip_push_begin(net->drStaging, 2 * (size_t)values, &push) != DRHIP_OK) return dR_apply(net) ? dR_downloadOutputs(net, hosts, n) : -1;
-    unsigned at[2];
-    size_t floats[2];
-    int k = 0;
-    for (dR_Node* node : nodes_of(net->output_layers)) {
-        at[k] = node == last ? 0 : values;
-        floats[k++] = values;
-        if (node != last) push.atInput = values;
-    }
-    net->drPush = &push;
-    net->drPushNode = last;
-    const gboolean ok = dR_apply(net);
-    net->drPush = NULL;
-    net->drPushNode = NULL;
-    if (!ok) return -1;
-    return device_failed(net, drhip_push_collect(net->drStaging, &push, k, hosts, at, floats, stream_of(net)), "dR_applyAndDownload") ? 0 : k;
+    return dR_applyAhead(net) ? dR_downloadOutputs(net, hosts, n) : -1;
 }
 
 void dR_cleanup(dR_Graph* net, gboolean cleanupcl) {
@@ -464,6 +477,8 @@ void dR_cleanup(dR_Graph* net, gboolean cleanupcl) {
     }
     if (net->drGraphExec) { drhip_graph_destroy(net->drGraphExec); net->drGraphExec = NULL; }
     if (net->drStaging) { drhip_staging_destroy(net->drStaging); net->drStaging = NULL; }
+    free(net->drPending);
+    net->drPending = NULL;
     for (int k = 0; k < 4; ++k) { drhip_event_destroy(net->drBranchEvents[k]); net->drBranchEvents[k] = NULL; }
     for (int k = 0; k < 3; ++k) { drhip_stream_destroy(net->drSideStreams[k]); net->drSideStreams[k] = NULL; }
     if (net->prepared) dR_cleanupBuffers(net);

@@ -133,6 +133,7 @@ int    drhip_download_staged_many(void* handle, int count, float* const* dst_hos
  * behind the last layer of a pass. */
 typedef struct drhip_push { float* host; unsigned at, atInput; unsigned* flag; unsigned value; } drhip_push;
 int drhip_push_begin(void* handle, size_t floats, drhip_push* push);
+int drhip_push_current(void* handle, const drhip_push* push);    /* nothing else has used the area since */
 int drhip_push_collect(void* handle, const drhip_push* push, int count, float* const* dst_host, const unsigned* at, const size_t* floats, void* stream);
 
 /* ---- convolution ------------------------------------------------------------------------------

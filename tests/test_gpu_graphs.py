@@ -355,6 +355,43 @@ def test_small_layer_in_the_softmax(oracle, gpu, K, N, front, logits):
             assert_close(np.reshape(u, -1), want[i].reshape(-1), "node %d" % i, terms=max(K, front) * (4 if front else 1), floor=0.01)
 
 
+def test_outputs_on_their_way_to_the_host(gpu):
+    """Outputs that the last kernel pushes: fetched late, twice, behind another pass, another download, a new image, and by one call."""
+    st = configs._Streams(99)
+    spec = [{"op": "feed", "shape": (9, 7, 3)}, configs._fc(st, 0, 189, 40, False), {"op": "softmax", "in": 1}]
+    a, b = configs.image_input(st, 9, 7, 3), configs.image_input(st, 9, 7, 3)
+    with dr.Environment() as env:
+        g = env.create_graph()
+        nodes = configs.build_graph(g, spec, [1, 2])
+        dr.prepare(g)
+        want = {}
+        for name, x in (("a", a), ("b", b)):
+            configs.feed_chw(nodes[0], x)
+            assert g.lib.dR_apply(g.ptr)
+            want[name] = [o.copy() for o in dr.download_outputs(g)]
+        same = lambda got, name: all(np.array_equal(u, v) for u, v in zip(got, want[name])) and len(got) == 2
+        configs.feed_chw(nodes[0], a)
+        assert g.lib.dR_applyAhead(g.ptr)
+        configs.feed_chw(nodes[0], b)                       # (behind the pass)
+        assert same(dr.download_outputs(g), "a") and same(dr.download_outputs(g), "a")
+        assert g.lib.dR_applyAhead(g.ptr)
+        assert np.array_equal(np.squeeze(configs.fetch_chw(g)[1]), want["b"][1])        # one by one, through the same area
+        assert same(dr.download_outputs(g), "b")
+        configs.feed_chw(nodes[0], a)
+        assert g.lib.dR_applyAhead(g.ptr)
+        configs.feed_chw(nodes[0], b)
+        assert g.lib.dR_apply(g.ptr) and same(dr.download_outputs(g), "b")              # an ordinary pass behind it
+        configs.feed_chw(nodes[0], a)
+        assert same(dr.apply(g), "a")
+        flats = [np.empty(40, np.float32) for _ in range(2)]
+        hosts = (ctypes.c_void_p * 2)(*[f.ctypes.data for f in flats])
+        configs.feed_chw(nodes[0], b)
+        assert g.lib.dR_applyAndDownload(g.ptr, hosts, 2) == 2 and same(flats, "b")
+        configs.feed_chw(nodes[0], a)
+        assert g.lib.dR_applyAndDownload(g.ptr, hosts, 1) == 1 and np.array_equal(flats[0], want["a"][0]) and np.array_equal(flats[1], want["b"][1])
+        assert g.lib.dR_applyAhead(g.ptr)                   # (and nobody fetches them)
+
+
 @pytest.mark.parametrize("W,H,I,O,split", [(30, 30, 24, 32, True), (33, 47, 36, 50, True), (7, 5, 9, 3, True), (90, 62, 70, 300, True), (20, 20, 64, 64, False), (41, 40, 80, 70, False)])
 def test_strided_layers_by_either_kernel(oracle, gpu, W, H, I, O, split):
     """3x3/2 layers on both sides of the rule that chooses their kernel, and by the general one (DR_DIRECT_VALU=1)."""
