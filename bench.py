@@ -103,7 +103,7 @@ def kind_of(node):
     return node["op"]
 
 
-KERNEL_NAMES = {"winograd": "winograd_f23_mfma_kernel", "conv1x1": "conv1x1_mfma_kernel", "direct": "conv3x3_direct_mfma_kernel"}
+KERNEL_NAMES = {"fire": "fire_kernel", "winograd": "winograd_f23_mfma_kernel", "conv1x1": "conv1x1_mfma_kernel", "direct": "conv3x3_direct_mfma_kernel"}
 
 
 def winograd_issued_flops(lib, W, H, I, O):
@@ -164,6 +164,8 @@ def measure(workload, seed, steps, warmup, blocks=BLOCKS, instrument=True, env_v
         res = {"spec": spec, "feeds": feeds, "flops": flops, "shapes": shapes, "outs": outs,
                "ms_per_step": statistics.median(block_ms), "ms_min": min(block_ms), "ms_max": max(block_ms),
                "launch_graph": bool(dr.graph_struct(g).drGraphExec)}
+        said = lambda n: ctypes.string_at(ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_void_p)(dr.node_struct(n).printLayer)(n.ptr)).decode()
+        res["fire_nodes"] = {i for i, n in enumerate(spec) if n["op"] == "conv" and "Kernel: fire module" in said(nodes[i])}
 
         # wall-clock rate of the loop the reference's users run: feed (H2D over PCIe), pass, download of the output
         # (the three C calls with buffers set up once, as a C caller has them: no array is created inside the loop)
@@ -217,6 +219,8 @@ def analyse(lib, m, workload, counters):
     """Per-layer rows, kernel groups and the roofline blocks of one measured workload."""
     spec, flops, shapes, per_node = m["spec"], m["flops"], m["shapes"], m["per_node"]
     ms = [float(v) for v in per_node]
+    fire = m["fire_nodes"]                  # 3x3 layers of fire modules that run with their neighbours in one launch of another kernel
+    kind = lambda i: "fire" if i in fire else kind_of(spec[i])
     # an expand 1x1 that rides in its 3x3 sibling's Winograd launch has no kernel of its own: its work is
     # credited to the launch that does it
     merged, joint_o = dict(flops), {}
@@ -227,11 +231,16 @@ def analyse(lib, m, workload, counters):
                     merged[j] = merged.get(j, 0) + merged.pop(i, 0)
                     joint_o[j] = o["w"].shape[1] + n["w"].shape[1]      # the 1x1 channels travel as centre-tap 3x3 filters
                     break
+            else:                           # a squeeze layer in the launch in front of it, through a pooling or not
+                j = n["in"]
+                while spec[j]["op"] in ("pool", "concat"):
+                    j = spec[j]["ins"][-1] if spec[j]["op"] == "concat" else spec[j]["in"]
+                merged[j] = merged.get(j, 0) + merged.pop(i, 0)
     groups, layers = {}, []
     for i, n in enumerate(spec):
         if n["op"] == "feed":
             continue
-        k = kind_of(n)
+        k = kind(i)
         gk = groups.setdefault(k, {"ms": 0.0, "flops": 0, "issued": 0, "busy_ms": 0.0, "bytes": 0, "launches": 0})
         gk["ms"] += ms[i]
         gk["flops"] += merged.get(i, 0)
@@ -263,7 +272,7 @@ def analyse(lib, m, workload, counters):
         if row:
             layers.append(row)
 
-    conv_kinds = [k for k in ("winograd", "conv1x1", "direct") if k in groups and groups[k]["ms"] > 0]
+    conv_kinds = [k for k in ("winograd", "fire", "conv1x1", "direct") if k in groups and groups[k]["ms"] > 0]
     dominant = max(conv_kinds, key=lambda k: groups[k]["ms"]) if conv_kinds else None
     roofline = None
     if dominant:
@@ -462,7 +471,7 @@ def summarise(dirs, workload, counters_json, last=0):
         for k, (n, a, b) in tot.items():
             print("| `%s` | %d | %.1f | %.1f | %.1f |" % (k, n, a, b, (a + b) / n))
         print()
-        for group, match in (("winograd", "winograd_f23"), ("fc", "fc_gemv"), ("conv1x1", "conv1x1_mfma"), ("direct", "direct_mfma"), ("bank", "conv_bank")):
+        for group, match in (("winograd", "winograd_f23"), ("fire", "fire_kernel"), ("fc", "fc_gemv"), ("conv1x1", "conv1x1_"), ("direct", "direct_mfma"), ("bank", "conv_bank")):
             sel = [(n, a, b) for k, (n, a, b) in tot.items() if match in k]
             if sel:
                 n = sum(s[0] for s in sel)
@@ -475,7 +484,7 @@ def summarise(dirs, workload, counters_json, last=0):
               "End - Start timestamp under the profiler (longer than in a plain run); busy = busy cycles per SIMD / (kernel us x 2.4 GHz).\n")
         print("| # | kernel | grid (lanes) | MOPS | issued GFLOP | MFMA busy cycles/SIMD | kernel us | busy |")
         print("|---:|---|---:|---:|---:|---:|---:|---:|")
-        families = (("winograd", "winograd_f23"), ("direct", "direct_mfma"), ("conv1x1", "conv1x1_mfma"), ("first_layer", "fewc"), ("bank", "conv_bank"))
+        families = (("winograd", "winograd_f23"), ("fire", "fire_kernel"), ("direct", "direct_mfma"), ("conv1x1", "conv1x1_"), ("first_layer", "fewc"), ("bank", "conv_bank"))
         tot = collections.OrderedDict()
         k = 0
         reduce_us = 0.0
