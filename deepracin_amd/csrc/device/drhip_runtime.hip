@@ -337,7 +337,8 @@ struct Staging {
 };
 constexpr size_t kStagingDownBytes = 64 * 1024;    // + 64 bytes behind it for the flag
 constexpr size_t kStagingKernelUpload = 4u << 20;
-constexpr size_t kStagingHalves = 256u << 10;      // uploads by kernel of this size and more go in two pieces
+constexpr size_t kStagingHalves = 256u << 10;      // uploads by kernel of this size and more go in two pieces,
+constexpr size_t kStagingPiece = 450u << 10;       // images of three times this and more in pieces of this size at least
 
 int drhip_staging_create(void** handle, size_t upload_bytes) {
     DRHIP_REQUIRE(handle && upload_bytes > 0, "drhip_staging_create: NULL handle or zero size");
@@ -483,12 +484,14 @@ int drhip_upload_staged_interleaved(void* handle, float* dst, const float* src, 
     float* const mem = (float*)area->mem;
     if (channels <= 4 && s->uploadByKernel && bytes <= kStagingKernelUpload) {
         // An image: the kernel that fetches it from the pinned area brings it into planes on the way; the host only
-        // copies.  In two pieces from 256 KiB on, for the reason given above.
-        const size_t half = (pixels / 2 + kHwcPixels - 1) / kHwcPixels * kHwcPixels;
-        const size_t first = bytes >= kStagingHalves && half < pixels ? half : pixels;
-        const size_t begins[2] = {0, first}, lens[2] = {first, pixels - first};
-        for (int piece = 0; piece < 2 && lens[piece] > 0; ++piece) {
-            const size_t begin = begins[piece], len = lens[piece];
+        // copies.  In two pieces from 256 KiB on, for the reason given above, and from three times 450 KiB on in as many
+        // as are 450 KiB each: a piece of much more than 1 MB is fetched at a lower rate.  (An image through SqueezeNet
+        // and its classes back, us, in two pieces / in pieces of 300, 450 and 600 KiB: 512x512 223 / 199, 196, 196,
+        // 400x400 160 / 157, 155, 157, 451x299 148.0 / 145.3, 145.7, 147.8.)
+        const size_t pieces = bytes < kStagingHalves ? 1 : std::max<size_t>(2, bytes / kStagingPiece);
+        const size_t each = (pixels + pieces * kHwcPixels - 1) / (pieces * kHwcPixels) * kHwcPixels;
+        for (size_t begin = 0; begin < pixels; begin += each) {
+            const size_t len = std::min(each, pixels - begin);
             memcpy(mem + begin * C, src + begin * C, len * C * sizeof(float));
             const dim3 grid((unsigned)((len + kHwcPixels - 1) / kHwcPixels));
             auto go = [&](auto kernel) { launch(kernel, grid, dim3(128), 0, as_stream(stream), dst + begin, (const float*)(mem + begin * C), pixels, len); };

@@ -932,10 +932,10 @@ def test_staged_transfers_carry_every_byte(lib, dev, env):
         lib.drhip_staging_destroy(h)
 
 
-@pytest.mark.parametrize("pixels,channels", [(1, 3), (5, 2), (1023, 3), (1025, 4), (50176, 3), (65537, 2), (4097, 1), (700, 7), (9, 64), (400001, 3)])
+@pytest.mark.parametrize("pixels,channels", [(1, 3), (5, 2), (1023, 3), (1025, 4), (50176, 3), (65537, 2), (4097, 1), (700, 7), (9, 64), (400001, 3), (115210, 3), (307201, 3)])
 @pytest.mark.parametrize("env", [{}, {"DR_UPLOAD_KERNEL": "0"}])
 def test_interleaved_upload_and_joint_download(lib, dev, pixels, channels, env):
-    """[pixels][channels] on the host -> [channels][pixels] on the device: by kernel in one and in two pieces, at the
+    """[pixels][channels] on the host -> [channels][pixels] on the device: by kernel in one, two, three and eight pieces, at the
     edges of its 1024-pixel blocks, beyond 4 MiB and with many channels (host), each twice; then several arrays back
     in one trip, and in several where they do not fit the download area."""
     import os
