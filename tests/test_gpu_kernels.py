@@ -936,7 +936,7 @@ def test_staged_transfers_carry_every_byte(lib, dev, env):
 @pytest.mark.parametrize("env", [{}, {"DR_UPLOAD_KERNEL": "0"}])
 def test_interleaved_upload_and_joint_download(lib, dev, pixels, channels, env):
     """[pixels][channels] on the host -> [channels][pixels] on the device: by kernel in one, two, three and eight pieces, at the
-    edges of its 1024-pixel blocks, beyond 4 MiB and with many channels (host), each twice; then several arrays back
+    edges of its 512-pixel blocks, beyond 4 MiB and with many channels (host), each twice; then several arrays back
     in one trip, and in several where they do not fit the download area."""
     import os
     os.environ.update(env)
