@@ -77,6 +77,11 @@ bool expand_pair(const dR_Node* a, const dR_Node* b) {
     return ia.size() == 1 && ib.size() == 1 && ia[0] == ib[0];
 }
 
+// A 3x3 filter over an image (at most 4 input channels) outside Winograd: the layers whose kernel takes a 3x3/2 pooling along.
+bool direct_image_layer(const dR_Conv2d_Data* c) {
+    return c->algo == drConvDirect && !c->drDirectBank && !c->drSplitBank && c->shape.s0 == 3 && c->shape.s1 == 3 && c->shape.s2 <= 4;
+}
+
 // Max pooling stored by the convolution in front of it, so that the full-resolution tensor never
 // exists (only when nobody else wants that tensor; DR_FUSE_POOL=0 keeps the two apart):
 //  - a 2x2 / stride-2 pool behind a Winograd convolution: every 2x2 output tile of the convolution
@@ -105,7 +110,7 @@ dR_Node* pool_fusable_producer(const dR_Node* p) {
         const bool bank = cd->drSplitBank && drhip_conv_bank_pick_variant(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->shape.s0, cd->shape.s1, cd->stride.s1, cd->stride.s2, 1);
         if (!bank && !(cd->algo == drConvWinograd && even)) return nullptr;
     } else {
-        if (cd->algo != drConvDirect || cd->shape.s0 != 3 || cd->shape.s1 != 3 || cd->shape.s2 > 4) return nullptr;
+        if (!direct_image_layer(cd)) return nullptr;
         // (that kernel carries its shape in 16-bit fields and its strides in 4-bit fields)
         if (cd->ishape.s0 > 65535 || cd->ishape.s1 > 65535 || cd->shape.s3 > 65535 || cd->stride.s1 > 15 || cd->stride.s2 > 15) return nullptr;
     }
@@ -203,8 +208,9 @@ dR_Node* fire_next(const dR_Node* concat, const std::map<const dR_Node*, dR_Node
 dR_Node* first_layer_squeeze(const dR_Node* n, const std::map<const dR_Node*, dR_Node*>& pairOf) {
     if (n->type != tConv2d || !((const dR_Conv2d_Data*)n->layer)->drFusedPool) return nullptr;
     const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
-    if (c->algo != drConvDirect || c->shape.s2 < 2 || c->shape.s3 > 64) return nullptr;
     const dR_Node* pooling = nodes_of(n->next_layers)[0];
+    // (layers of other filters take a pooling along as well, a 2x2 one, in a kernel that knows no layer behind it)
+    if (!direct_image_layer(c) || ((const dR_Pooling_Data*)pooling->layer)->shape.s1 != 3 || c->shape.s2 < 2 || c->shape.s3 > 64) return nullptr;
     if (!tensor_hidden(pooling) || pooling->next_layers->length != 1) return nullptr;
     dR_Node* squeeze = nodes_of(pooling->next_layers)[0];
     return fire_squeeze(squeeze, nullptr, pairOf) && ((const dR_Conv2d_Data*)squeeze->layer)->shape.s3 <= 64 &&

@@ -317,6 +317,29 @@ def test_fire_chain_with_both_ends(oracle, gpu, w, h, cin, first, squeeze, expan
     assert rel_err(res["1"][1], res["0"][1]) <= 5e-6
 
 
+@pytest.mark.parametrize("w,h,cin,first,k,stride", [(65, 47, 3, 64, 7, 2), (30, 34, 8, 64, 5, 1), (60, 52, 16, 32, 3, 2), (41, 37, 4, 24, 5, 2)])
+def test_fire_module_behind_a_pooled_layer_of_other_filters(oracle, gpu, w, h, cin, first, k, stride):
+    """A layer on the split filter bank with a 2x2 pooling in its launch, then two modules: the squeeze layer behind the pooling is
+    a launch of its own, in front of a chain."""
+    st = configs._Streams(79)
+    spec = [{"op": "feed", "shape": (w, h, cin)}, configs._conv(st, 0, k, cin, first, stride=stride), configs._maxpool(1, 2, 2)]
+    channels = first
+    for squeeze, expand in ((16, 32), (20, 64)):
+        s = len(spec)
+        spec += [configs._conv(st, s - 1, 1, channels, squeeze), configs._conv(st, s, 1, squeeze, expand), configs._conv(st, s, 3, squeeze, expand),
+                 {"op": "concat", "ins": [s + 1, s + 2], "dim": 2}]
+        channels = 2 * expand
+    x = configs.image_input(st, w, h, cin, 2.0) - np.float32(1)
+    want = oracle.run_spec(spec, {0: x})
+    with dr.Environment() as env:
+        g = env.create_graph()
+        nodes = configs.build_graph(g, spec, [len(spec) - 1])
+        dr.prepare(g)
+        configs.feed_chw(nodes[0], x)
+        assert g.lib.dR_apply(g.ptr)
+        assert rel_err(configs.fetch_chw(g)[0], want[-1]) <= LAYER_TOL
+
+
 @pytest.mark.parametrize("K,N,front,logits", [(1, 1, 0, True), (1024, 32, 0, False), (32, 1024, 40, True), (333, 98, 900, True), (128, 10, 1568, True), (5, 700, 0, True)],
                          ids=lambda v: str(v))
 def test_small_layer_in_the_softmax(oracle, gpu, K, N, front, logits):
@@ -857,6 +880,8 @@ def _random_spec(seed):
         elif kind == "fire":
             s = conv(cur, 1, int(rng.integers(1, 12)))
             e = int(rng.integers(1, 40))
+            if e % 4 == 0:                           # what the launches of whole fire modules cover
+                e = 32 if e % 8 == 0 else 64
             a, b = conv(s, 1, e), conv(s, 3, e)
             spec.append({"op": "concat", "ins": [a, b], "dim": 2}); shapes.append((w_, h_, 2 * e)); cur = len(spec) - 1
         elif kind == "branch3":                      # three producers, one of them read twice

@@ -520,6 +520,23 @@ def test_a_layer_says_which_kernel_it_runs(lib, W, H, I, O, k, stride, kernel):
         assert re.fullmatch(" Kernel: %s \\(variant \\d+\\)" % re.escape(kernel), _kernel_line(c)), _kernel_line(c)
 
 
+@pytest.mark.parametrize("W,H,I,O,k,stride,pool,taken", [
+    (65, 47, 3, 64, 3, 2, 3, True), (64, 48, 2, 33, 3, 2, 3, True), (65, 47, 3, 64, 7, 2, 2, False), (64, 48, 4, 32, 5, 1, 2, False),
+    (30, 34, 8, 64, 5, 1, 2, False), (60, 52, 16, 32, 3, 2, 2, False), (65, 47, 3, 64, 7, 2, 3, False), (65, 47, 1, 64, 3, 2, 3, False)])
+def test_a_squeeze_layer_rides_with_image_layers_only(lib, W, H, I, O, k, stride, pool, taken):
+    """Layer -> pooling -> fire module: the launch of the first two takes the squeeze layer along where it is a 3x3 layer over an image
+    with a 3x3/2 pooling, and no other layer that has its pooling in its launch does."""
+    w = lambda i, o, side: np.ones((i, o, side, side), np.float32)
+    with dr.Environment() as env:
+        g = env.create_graph()
+        c = dr.Conv2d_raw(dr.feed_node(g, [H, W, I]), w(I, O, k), None, (stride, stride), "relu")
+        squeeze = dr.Conv2d_raw(dr.Pooling(c, "max", [1, pool, pool, 1], [1, 2, 2, 1]), w(O, 16, 1), None, (1, 1), "relu")
+        one, three = dr.Conv2d_raw(squeeze, w(16, 32, 1), None, (1, 1), "relu"), dr.Conv2d_raw(squeeze, w(16, 32, 3), None, (1, 1), "relu")
+        dr.mark_as_output(dr.Concat([one, three], 2))
+        assert lib.dR_propagateShapesAndSchedule(g.ptr) == 1 and lib.dR_planBuffers(g.ptr) == 1
+        assert ("in the launch of the layers in front" in _kernel_line(squeeze)) == taken, _kernel_line(squeeze)
+
+
 def test_layers_beyond_32_bit_byte_offsets_take_the_general_kernels(lib):
     """Every dimension fits the 16-bit argument fields, but the input holds 2^29 elements or more: the matrix-core
     3x3 kernels and the pooling-on-load 1x1 kernel (32-bit byte offsets) are not scheduled for such a layer."""
