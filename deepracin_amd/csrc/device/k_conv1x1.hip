@@ -286,12 +286,12 @@ conv1x1_pixels_poolsum_kernel(const float* __restrict__ in, const float* __restr
     const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, oBlocks * I * 64, kC1BufferFlags);
     const __amdgpu_buffer_rsrc_t rBias = __builtin_amdgcn_make_buffer_rsrc((void*)bias, 0, bias ? O * 4 : 0, kC1BufferFlags);
     auto load = [](const __amdgpu_buffer_rsrc_t& r, int v, int sOff) { return __builtin_bit_cast(f32x4ld, __builtin_amdgcn_raw_buffer_load_b128(r, v, sOff, 0)); };
-    // the tile's samples lie in a row: thread after thread, 8 KiB a round
+    // the tile's samples lie in a row: thread after thread, 8 KiB a round (in the vector offset, which is the one that the range check sees)
     f32x4ld v[U];
     const int base = p0 * I * 4 + 16 * tid, total = 16 * NC * quads;
 #pragma unroll
     for (int u = 0; u < U; ++u)
-        if (u * 512 < total) v[u] = load(rIn, base, u * 8192);
+        if (u * 512 < total) v[u] = load(rIn, base + u * 8192, 0);
     asm volatile("" ::: "memory");
     f32x4ld a[D];
     const int f0 = (2 * min(ob, oBlocks - 1) + half) * n;                   // (a wave without channels repeats the last ones)
@@ -308,7 +308,7 @@ conv1x1_pixels_poolsum_kernel(const float* __restrict__ in, const float* __restr
 #pragma unroll
     for (int u = 0; u < U; ++u)
         if (u * 512 < total) put(u * 512 + tid, v[u]);
-    for (int i = U * 512; i < total; i += 512) put(i + tid, load(rIn, base, i * 16));
+    for (int i = U * 512; i < total; i += 512) put(i + tid, load(rIn, base + i * 16, 0));
     auto barrier = [] {                             // (LDS only: loads stay under way)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();

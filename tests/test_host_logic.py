@@ -711,3 +711,24 @@ def test_wide_stores_keep_their_data(tmp_path, source):
                 lo, hi = (int(w[1]), int(w[1])) if w[1] else (int(w[2]), int(w[3]))
                 assert hi < int(m[1]) or lo > int(m[2]), (line, after)
     assert stores
+
+
+def test_pixel_loads_end_with_the_tensor(tmp_path):
+    """The 1x1 kernel in front of a global average takes zeros behind the last pixel from the range check of its input's resource,
+    which need not see scalar offsets: in the assembly only the filters' resource is read at one, and the input's is another."""
+    import subprocess
+    from deepracin_amd import build
+    out = str(tmp_path / "k.s")
+    subprocess.run([build.HIPCC] + build.COMMON + build.DEVICE + ["--cuda-device-only", "-S", os.path.join(build.CSRC, "device", "k_conv1x1.hip"), "-o", out],
+                   check=True, capture_output=True)
+    kernels, loads = 0, None
+    for line in open(out):
+        if line.startswith("_ZN5drhip29conv1x1_pixels_poolsum_kernel") and line.split(";")[0].strip().endswith(":"):
+            kernels, loads = kernels + 1, []
+        elif loads is not None and line.strip().startswith("buffer_load_dwordx4"):
+            loads.append(re.match(r"\s+buffer_load_dwordx4 v\[\d+:\d+\], v\d+, (s\[\d+:\d+\]), (\S+) offen", line).groups())
+        elif loads and "s_endpgm" in line:
+            scalar = {resource for resource, offset in loads if offset != "0"}
+            assert len(scalar) == 1 and loads[0][0] not in scalar and sum(r == loads[0][0] for r, _ in loads) == 5, loads
+            loads = None
+    assert kernels == 2
