@@ -480,7 +480,9 @@ conv3x3_direct_mfma_kernel(const float* __restrict__ in, const float* __restrict
 
     const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, I * plane * 4, kDmBufferFlags);
     const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, 9 * nChunks * Opad * 8 * 4, kDmBufferFlags);
-    const unsigned fOff = 4u * (unsigned)((o0 + l32) * 8 + 4 * lhi);
+    unsigned fOff[NT];                      // (a block of channels behind the bank's last one reads zeros: the range check sees this offset only)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) fOff[nt] = nt == 0 || o0 + 32 * nt < Opad ? 4u * (unsigned)((o0 + 32 * nt + l32) * 8 + 4 * lhi) : kDmOutOfRange;
 
     // rows of channels cbase + 2ks + lhi, ks = 0..3.  Plain form: one resource for the tensor, the channel in the
     // scalar offset (chunks known to lie inside the tensor).  Ranged form: the resource starts at channel cbase and
@@ -503,7 +505,7 @@ conv3x3_direct_mfma_kernel(const float* __restrict__ in, const float* __restrict
     auto load_filters = [&](f32x4d (&f)[NT], int tap, int chunk) {
         const unsigned soff = 4u * (unsigned)((tap * nChunks + chunk) * Opad * 8);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) f[nt] = dm_buf_load4(rF, fOff + 4u * (unsigned)(nt * 32 * 8), soff);
+        for (int nt = 0; nt < NT; ++nt) f[nt] = dm_buf_load4(rF, fOff[nt], soff);
     };
 
     // the epilogue's bias values are requested now: thread tid finishes the elements tid + q*blockDim.x of the tile

@@ -243,11 +243,13 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         };
         // filters of one xi for a whole stage: component ks of the 16-byte load = k-step ks
         const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)U, 0, 16 * nChunksAll * Opad * 8 * 4, kBufferFlags);
-        const unsigned fOff = 4u * (unsigned)((o0 + l32) * 8 + 4 * lhi);
+        unsigned fOff[NT];                              // (a block of channels behind the bank's last one reads zeros: the range check sees this offset only)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) fOff[nt] = nt == 0 || o0 + 32 * nt < Opad ? 4u * (unsigned)((o0 + 32 * nt + l32) * 8 + 4 * lhi) : kOutOfRange;
         auto load_filters = [&](f32x4 (&f)[NT], int e, int chunk) {
             const unsigned soff = 4u * (unsigned)(((4 * wave + e) * nChunksAll + chunk) * Opad * 8);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) f[nt] = buf_load4(rU, fOff + 4u * (unsigned)(nt * 32 * 8), soff);
+            for (int nt = 0; nt < NT; ++nt) f[nt] = buf_load4(rU, fOff[nt], soff);
         };
 
         // The epilogue's bias values are fetched now: a load issued there would add a trip to memory
@@ -557,12 +559,14 @@ winograd_f23_mfma16_kernel(const float* __restrict__ in, const float* __restrict
         load_rows(d, r, 0u);
     };
     const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)U, 0, 16 * nChunksAll * Opad * 8 * 4, kBufferFlags);
-    const unsigned fOff = 4u * (unsigned)((o0 + l16) * 8 + 4 * (lk & 1));
+    unsigned fOff[NB];                              // (as in the 32-tile kernel)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) fOff[nb] = nb < 2 || o0 + 16 * nb < Opad ? 4u * (unsigned)((o0 + 16 * nb + l16) * 8 + 4 * (lk & 1)) : kOutOfRange;
     const bool oddPair = (lk >> 1) != 0;            // which components of the 16 bytes: {0,2} or {1,3}
     auto load_filters = [&](f32x4 (&f)[NB], int e, int chunk) {
         const unsigned soff = 4u * (unsigned)(((4 * wave + e) * nChunksAll + chunk) * Opad * 8);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) f[nb] = buf_load4(rU, fOff + 4u * (unsigned)(nb * 16 * 8), soff);
+        for (int nb = 0; nb < NB; ++nb) f[nb] = buf_load4(rU, fOff[nb], soff);
     };
 
     constexpr int EO = 16 * KW;                     // output channels finished per pass of the epilogue

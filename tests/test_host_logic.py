@@ -732,3 +732,25 @@ def test_pixel_loads_end_with_the_tensor(tmp_path):
             assert len(scalar) == 1 and loads[0][0] not in scalar and sum(r == loads[0][0] for r, _ in loads) == 5, loads
             loads = None
     assert kernels == 2
+
+
+@pytest.mark.parametrize("source,kernels", [("k_conv_direct.hip", 2), ("k_winograd.hip", 6)])
+def test_filter_loads_end_with_the_bank(tmp_path, source, kernels):
+    """Filter banks of the fp32 3x3 kernels are padded to 32 output channels, and a panel may be wider: the blocks of 32 channels that the bank
+    lacks read zeros by the range check, which need not see the scalar offset.  So such a block has a vector offset of its
+    own: with a scalar one no load goes 1024 bytes (a block) on from another's place by its immediate offset."""
+    import subprocess
+    from deepracin_amd import build
+    out = str(tmp_path / "k.s")
+    subprocess.run([build.HIPCC] + build.COMMON + build.DEVICE + ["--cuda-device-only", "-S", os.path.join(build.CSRC, "device", source), "-o", out],
+                   check=True, capture_output=True)
+    name, places = None, {}
+    for line in open(out):
+        if re.match(r"_ZN5drhip\S+:", line):
+            name = line.split(":")[0]
+        m = re.match(r"\s+buffer_load_dwordx4 v\[\d+:\d+\], (v\d+), s\[\d+:\d+\], s\d+ offen(?: offset:(\d+))?", line)
+        if m:
+            places.setdefault(name, set()).add(m[1])
+            assert int(m[2] or 0) < 1024, (name, line)
+    wide = [n for n in places if re.search(r"direct_mfma_kernelILi2|f23_mfma_kernelILi[24]|f23_mfma16_kernelILi4", n)]
+    assert len(wide) == kernels and all(len(places[n]) >= 2 for n in wide), (wide, places)
