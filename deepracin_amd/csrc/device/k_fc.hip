@@ -60,9 +60,12 @@ static FcPlan fc_plan(int K, int N) {
     const int target = num_cu();                     // workgroups wanted in flight
     int slices = ceil_div(target, p.panels);
     // at least 256 rows per workgroup (4096 x 4096: 13.7 us with 16 slices, 14.8 with 32).  A matrix of at most 4 MiB is a few workgroups
-    // whose time is that of their trips to memory: 64 rows, 16 a wave, are one, and 32 slices one for the reader (1568 x 128: 5.2 us with 7
-    // slices, 2.5 with 25; 192 x 1000 4.9 with 1, 3.2 with 3).
-    const int maxSlices = (long long)K * N <= 1 << 20 ? std::min(32, ceil_div(K, kWave)) : ceil_div(K, 4 * kWave);
+    // whose time is that of their trips to memory: 64 rows, 16 a wave, are one, and 32 slices one for the reader (64 / 256 rows, us of the layer and a
+    // softmax, or another layer and a softmax, behind it: 1024 x 1000 6.8 / 7.4 and 9.7 / 10.4; 256 x 2048 7.4 / 8.3 and 9.5 / 11.5; 512 x 30 - and
+    // 5.9 / 6.5; 2048 x 100 6.6 / 7.0 and 7.6 / 8.3).  Beyond 8192 rows 32 slices would have more than 256 rows each, and 256 are the better ones again
+    // (32 slices / 256 rows: 16384 x 60 8.9 / 7.4 and 10.5 / 9.0, 100032 x 10 26.1 / 10.9 and 27.5 / 11.8).
+    int maxSlices = ceil_div(K, 4 * kWave);
+    if ((long long)K * N <= 1 << 20) maxSlices = std::max(maxSlices, std::min(32, ceil_div(K, kWave)));
     if (slices > maxSlices) slices = maxSlices;
     if (slices < 1) slices = 1;
     p.rowsPerSlice = ceil_div(ceil_div(K, slices), kWave) * kWave;   // whole chunks
@@ -133,10 +136,13 @@ fc_gemv_kernel(const float* __restrict__ Wt, const float* __restrict__ x, int K,
                     fma_row<VEC>(acc, wb[u], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xl), j0 + kFcUnroll + u)));
             }
         } else {
-            for (int j = 0; j < rows; ++j) {
-                const float xv = __shfl(xl, j, 64);
-                vec_t w = __builtin_nontemporal_load((const vec_t*)(wp + (size_t)j * N));
-                fma_row<VEC>(acc, w, xv);
+            // the last rows, fewer than a turn's: eight loads at a time as well (row after row they were a trip to memory each, 5 us for 48 rows)
+            for (int j0 = 0; j0 < rows; j0 += kFcUnroll) {
+#pragma unroll
+                for (int u = 0; u < kFcUnroll; ++u) wa[u] = __builtin_nontemporal_load((const vec_t*)(wp + (size_t)min(j0 + u, rows - 1) * N));
+#pragma unroll
+                for (int u = 0; u < kFcUnroll; ++u)
+                    if (j0 + u < rows) fma_row<VEC>(acc, wa[u], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xl), j0 + u)));
             }
         }
     }

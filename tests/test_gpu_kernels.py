@@ -1102,6 +1102,23 @@ def test_fc_sweep(lib, dev, oracle, C, H, W, N):
     assert_close(got, oracle.fc_f64(x, Wt, b).reshape(-1), terms=K)
 
 
+@pytest.mark.parametrize("K,N", [(7, 10), (15, 1000), (48, 98), (191, 300), (1000, 10), (8240, 10)])
+def test_fc_last_rows(lib, dev, K, N):
+    """Rows left over behind whole turns, eight at a time: against float64 (an fp32 sum of K products, so eps sqrt(K) of the sum of their
+    amounts), and an infinite weight in the last row, whose place stands in for rows that do not exist, stays an infinity."""
+    x, Wt = np.abs(rnd(K)) + np.float32(0.1), rnd(K, N, scale=np.sqrt(2.0 / K))
+    n = lib.drhip_fc_scratch_floats(K, N)
+    for inf in (False, True):
+        if inf:
+            Wt[K - 1, 0] = np.inf
+        y = dev.empty(N)
+        ok(lib, lib.drhip_fc_f32(dev.put(x), dev.put(Wt), None, y, dev.empty(n) if n else None, K, N, 0, None))
+        got = dev.get(y, (N,)).astype(np.float64)
+        assert not inf or got[0] == np.inf
+        x64, w64 = x.astype(np.float64), Wt.astype(np.float64)[:, 1:]
+        assert (np.abs(got[1:] - x64 @ w64) <= 2.0 ** -23 * np.sqrt(K) * (x64 @ np.abs(w64))).all()
+
+
 def test_mfma_clock_probe(lib, gpu):
     """The measurement aid of bench.py: shader clock under a stream of fp32 MFMAs, from the two clock counters a wave
     can read.  Somewhere between idle clocks and the 2.4 GHz of the data sheet."""

@@ -585,6 +585,17 @@ def test_pick_variants_are_launchable(lib):
         assert (c in (1, 2, 4, 8)) or (c & 0x100 and (c & 0xff) in (1, 2, 4, 8, 16) and c >> 9 == 0)
 
 
+@pytest.mark.parametrize("K,N", [(1, 1), (64, 10), (65, 1000), (1024, 1000), (8192, 100), (8256, 20), (16384, 60), (30000, 30), (100032, 10), (25088, 4096), (4096, 1000)])
+def test_fc_slices_hold_no_more_than_256_rows(lib, K, N):
+    """No slice has more than 256 rows unless 256 workgroups, one per CU, have more to share between them (columns go out in panels
+    of 64, from 1024 on in 16 and more); up to 8192 rows a matrix of at most 2^20 weights is cut finer, into 32 slices at most."""
+    slices, panels = lib.drhip_fc_slices(K, N), -(-N // 64) if N < 1024 else 16
+    rows, shared = -(-K // slices), 64 * -(-K // (64 * -(-256 // panels)))
+    assert rows <= max(256, shared)
+    if K * N <= 1 << 20 and K <= 8192:
+        assert slices <= 32 and rows <= max(64 * -(-K // 2048), shared)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU: any other --gpus value ends with a message, not with a number."""
     import subprocess
