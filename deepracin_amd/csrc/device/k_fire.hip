@@ -348,31 +348,38 @@ struct FirePlan {
 // 3.1 (Q = 4; 196 workgroups), 56x56 16->2x64->32 behind a pooling 4.4 (Q = 2; Q = 1 4.6), 28x28 32->2x128->48 behind one 4.9 (Q = 1,
 // 8 slices; Q = 2 5.9), 14x14 64->2x256->64 5.5 (Q = 2, 8 slices; Q = 4 6.2), 29x19 64->2x256->64 6.1 (Q = 4), 128x128 16->2x64->16 5.6
 // (1024 workgroups of 16 pixels; 256 of 64 pixels, which load a filter once for four columns, 6.3).
-static bool fire_plan(int W, int H, int S, int E, int Sn, int pool, FirePlan* best) {
+//
+// rows: the expand outputs are stored in rows of a map.  Then a block's rows count too: each is a piece of a line for every channel, written through, some 7
+// clocks each where there are many (85x96 12->2x128 stored from blocks of 1x16 pixels 36 us, from 8x2 8 us, and so the Winograd kernel behind
+// a squeeze layer 10 us).  Only the block is chosen by that, the channels of a slice are those of the bank.
+static bool fire_plan(int W, int H, int S, int E, int Sn, int pool, FirePlan* best, bool rows = false) {
     if (W < 1 || H < 1 || S < 1 || S > 64 || E < 32 || E % 32 != 0 || E > 2048 || Sn < 0 || Sn > 64 || (pool && Sn == 0)) return false;
     if (W > 16384 || H > 16384 || (long long)W * H * 64 >= (1ll << 26)) return false;
     const int S16 = ceil_div(S, 16), SP = 16 * S16, MB = ceil_div(Sn, 16), Wo = pool ? (W + 1) / 2 : W, Ho = pool ? (H + 1) / 2 : H;
     const int columns = fire_columns(pool), atOnce = kFireThreads * fire_quads(S16, pool), resident = S16 == 1 ? 4 : 2;
-    double least = 0;
-    for (int Q = pool ? 1 : 2; Q <= 4; Q *= 2) {
-        const int slices = E / 16 / Q;
-        if (slices * 16 * Q != E || slices > 32 || (long long)Wo * Ho * 16 * std::max(MB, 1) * slices >= (1ll << 28)) continue;
-        for (int bw = 1; bw <= (pool ? (kFireRow - 3) / 2 : kFireRow - 2); ++bw)
-            for (int bh = 1; bw * bh <= 16; ++bh) {
-                const int ew = pool ? 2 * bw + 1 : bw, eh = pool ? 2 * bh + 1 : bh, hpx = (ew + 2) * (eh + 2), nbx = ceil_div(Wo, bw), nby = ceil_div(Ho, bh);
-                if (ew * eh > 16 * columns) break;
-                if (nbx > 65535 || nby > 65535) continue;
-                const double perCu = std::ceil((double)nbx * nby * slices / num_cu()), filters = (10 * S16 + 2 * MB) * Q * 1024 / 48.0;
-                // (the last two: smaller patches, and longer runs of addresses, where nothing else decides)
-                const double work = 320.0 * S16 * Q * columns + filters + ceil_div(hpx * SP / 4, atOnce) * atOnce * 64 / 48.0 + hpx * SP / 48.0 + 300.0 / bw;
-                const double cost = std::ceil(perCu / resident) * 2500 + perCu * work + slices * 36 * 16 * MB * 4 / 48.0 + std::max(0, slices - kFireSlices) * 900.0;
-                if (least != 0 && cost >= least) continue;
-                const size_t lds = (size_t)(fire_sums(Q, pool) + (Sn > 0 ? fire_outs(Q, pool) : 0) + (eh + 2) * kFireRow * (SP + 4)) * sizeof(float);
-                least = cost;
-                *best = FirePlan{Q, bw, bh, ew, eh, hpx, nbx, nby, slices, S16, MB, lds, Wo, Ho};
-            }
-    }
-    return least != 0;
+    auto search = [&](int firstQ, int lastQ, double clocksPerRow) {
+        double least = 0;
+        for (int Q = firstQ; Q <= lastQ; Q *= 2) {
+            const int slices = E / 16 / Q;
+            if (slices * 16 * Q != E || slices > 32 || (long long)Wo * Ho * 16 * std::max(MB, 1) * slices >= (1ll << 28)) continue;
+            for (int bw = 1; bw <= (pool ? (kFireRow - 3) / 2 : kFireRow - 2); ++bw)
+                for (int bh = 1; bw * bh <= 16; ++bh) {
+                    const int ew = pool ? 2 * bw + 1 : bw, eh = pool ? 2 * bh + 1 : bh, hpx = (ew + 2) * (eh + 2), nbx = ceil_div(Wo, bw), nby = ceil_div(Ho, bh);
+                    if (ew * eh > 16 * columns) break;
+                    if (nbx > 65535 || nby > 65535) continue;
+                    const double perCu = std::ceil((double)nbx * nby * slices / num_cu()), filters = (10 * S16 + 2 * MB) * Q * 1024 / 48.0;
+                    // (the last two: smaller patches, and longer runs of addresses, where nothing else decides)
+                    const double work = 320.0 * S16 * Q * columns + filters + ceil_div(hpx * SP / 4, atOnce) * atOnce * 64 / 48.0 + hpx * SP / 48.0 + 300.0 / bw + 32 * Q * bh * clocksPerRow;
+                    const double cost = std::ceil(perCu / resident) * 2500 + perCu * work + slices * 36 * 16 * MB * 4 / 48.0 + std::max(0, slices - kFireSlices) * 900.0;
+                    if (least != 0 && cost >= least) continue;
+                    const size_t lds = (size_t)(fire_sums(Q, pool) + (Sn > 0 ? fire_outs(Q, pool) : 0) + (eh + 2) * kFireRow * (SP + 4)) * sizeof(float);
+                    least = cost;
+                    *best = FirePlan{Q, bw, bh, ew, eh, hpx, nbx, nby, slices, S16, MB, lds, Wo, Ho};
+                }
+        }
+        return least != 0;
+    };
+    return search(pool ? 1 : 2, 4, 0.0) && (!rows || search(best->Q, best->Q, 7.0));
 }
 
 struct FireCall { const float *in, *bank, *inBias; float* out; unsigned wh, block, misc, outWh; hipStream_t st; };
@@ -456,7 +463,7 @@ extern "C" int drhip_fire_f32(const float* in, int slicesIn, const float* inBias
     DRHIP_REQUIRE((((size_t)bank | (size_t)(slicesIn > 0 ? in : nullptr) | (size_t)(slicesIn > 0 ? inBias : nullptr) | (size_t)(Sn > 0 || pixels ? out : nullptr)) & 15) == 0,
                   "drhip_fire_f32: banks, partial sums, their bias and outputs by pixel need 16-byte alignment");
     FirePlan p;
-    DRHIP_REQUIRE(fire_plan(W, H, S, E, Sn, pool, &p), "drhip_fire_f32: %dx%d, %d -> 2 x %d -> %d is not covered", W, H, S, E, Sn);
+    DRHIP_REQUIRE(fire_plan(W, H, S, E, Sn, pool, &p, Sn == 0 && !pixels), "drhip_fire_f32: %dx%d, %d -> 2 x %d -> %d is not covered", W, H, S, E, Sn);
     DRHIP_REQUIRE((long long)slicesIn * W * H * 16 * p.S16 < (1ll << 29), "drhip_fire_f32: %d slices of %dx%dx%d are too large", slicesIn, W, H, S);
     FireCall c = {in, bank, inBias, out, 0, 0, 0, 0, as_stream(stream)};
     c.wh = (unsigned)(W | H << 16);

@@ -228,6 +228,8 @@ FIRE_CHAINS = [
     (14, 14, 64, [(48, 192, ""), (64, 256, ""), (64, 256, "")], True, True, 2),
     (17, 2, 40, [(64, 32, "p"), (50, 96, ""), (7, 32, "p"), (33, 64, "")], False, False, 2),        # ragged channels, nothing clipped at 0; pooled behind a plain tensor: apart
     (113, 75, 16, [(16, 64, ""), (16, 64, "p"), (24, 32, "")], True, False, 2),
+    (85, 23, 16, [(12, 32, ""), (12, 64, "")], True, True, 1),                  # last module stored in rows: widths that no block of them divides
+    (59, 7, 8, [(40, 32, ""), (33, 96, "")], True, True, 1),
     (9, 11, 8, [(65, 32, ""), (16, 48, ""), (64, 64, ""), (64, 32, "p")], True, True, 1),           # 65 and 48 are not covered: kernels of their own
 ]
 
