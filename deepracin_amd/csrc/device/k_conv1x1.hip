@@ -468,6 +468,18 @@ extern "C" int drhip_conv1x1_pooled3s2_f32(const float* in, const float* w, cons
 // 16 pixels a workgroup, 32 where that makes more slices than the reader has under way twice.
 extern "C" int drhip_conv1x1_pixels_tile(int P) { return P > 1024 ? 32 : 16; }
 
+// What either kernel takes in a pass: most of it by whole rounds of workgroups on the CUs.  Fitted to 327 shapes, 7x7 to 80x80 pixels of 64 to
+// 1024 channels to 10, 100 and 1000; half of them within 8 %.  One by pixel does 64 output channels at least, so that few of them are better off
+// apart (us: 56x56 1024->10 9.8 / 15.4, 40x40 512->10 6.0 / 8.6; 14x14 512->1000 6.7 / 5.9, 56x56 512->1000 66.6 / 49.3).
+extern "C" float drhip_conv1x1_poolsum_us(int P, int I, int O) {
+    const int wgs = ceil_div(O, 32) * ceil_div(P, 32);
+    return (float)(2.7 + (0.0057 * ceil_div(wgs, num_cu()) + 0.0043 * wgs / num_cu()) * I);
+}
+extern "C" float drhip_conv1x1_pixels_us(int P, int I, int O) {
+    const int tile = drhip_conv1x1_pixels_tile(P), wgs = ceil_div(O, 64) * ceil_div(P, tile);
+    return (float)(2.7 + (0.0047 * ceil_div(wgs, num_cu()) + 0.0029 * wgs / num_cu()) * I * tile / 16);
+}
+
 extern "C" int drhip_conv1x1_pixels_layout_f32(const float* w, float* F, int I, int O, void* stream) {
     DRHIP_REQUIRE(w && F && I > 0 && I % 16 == 0 && O > 0 && (long long)I * O < (1ll << 28), "drhip_conv1x1_pixels_layout_f32: bad arguments");
     launch(conv1x1_pixels_layout_kernel, dim3(ceil_div(O, 16) * (I / 16)), dim3(256), 0, as_stream(stream), w, F, I, O);

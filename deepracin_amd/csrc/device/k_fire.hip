@@ -339,6 +339,7 @@ struct FirePlan {
     int Q, bw, bh, ew, eh, hpx, nbx, nby, slices, S16, MB;
     size_t lds;
     int Wo, Ho;
+    double clocks;
 };
 
 // The shape of a launch: the block of output pixels and the channels of a slice that take the fewest clocks.  A workgroup takes
@@ -374,7 +375,7 @@ static bool fire_plan(int W, int H, int S, int E, int Sn, int pool, FirePlan* be
                     if (least != 0 && cost >= least) continue;
                     const size_t lds = (size_t)(fire_sums(Q, pool) + (Sn > 0 ? fire_outs(Q, pool) : 0) + (eh + 2) * kFireRow * (SP + 4)) * sizeof(float);
                     least = cost;
-                    *best = FirePlan{Q, bw, bh, ew, eh, hpx, nbx, nby, slices, S16, MB, lds, Wo, Ho};
+                    *best = FirePlan{Q, bw, bh, ew, eh, hpx, nbx, nby, slices, S16, MB, lds, Wo, Ho, cost};
                 }
         }
         return least != 0;
@@ -408,6 +409,29 @@ using namespace drhip;
 extern "C" int drhip_fire_slices(int W, int H, int S, int E, int Sn, int pool) {
     FirePlan p;
     return fire_plan(W, H, S, E, Sn, pool, &p) ? p.slices : 0;
+}
+
+// What the launches of a module take in a pass, us, for the choice between them: the launch above from the clocks of its plan, the others from the
+// products they do and the numbers they move (mpx: millions of pixels; the Winograd kernels store maps of odd width less well).  Fitted to 330 shapes, maps
+// of 13x13 to 320x320, 16 to 64 channels to 2x32 to 2x1024: half of them come out within 7 % and nine of ten within 20 %.  The launch above is put a tenth
+// lower, which lost least: on 450 random networks of one to six modules the choice is 0.8 % slower than the best side on average and 12 % at most, always
+// taking the next layer along 0.8 and 18 %, never doing so 20 and 90 %; in runs of alike modules always doing so lost up to 70 % (80x80 32->2x1024).
+extern "C" float drhip_fire_us(int W, int H, int S, int E, int Sn, int pool, int slicesIn) {
+    FirePlan p;
+    if (!fire_plan(W, H, S, E, Sn, pool, &p)) return 0.0f;
+    // (every workgroup adds up all slices of its patch: with sixteen of them 10 to 30 us of 50 to 100 on large maps)
+    const double patches = 16.0 * p.S16 * 4 / 48 / 2400 * p.hpx * slicesIn * ceil_div(p.nbx * p.nby * p.slices, num_cu());
+    return 0.9f * (float)((pool ? 1.5 + 1.15 * p.clocks / 2400 : 1.8 + 0.92 * p.clocks / 2400) + 1.8 * std::max(0.0, patches - 2));
+}
+extern "C" float drhip_fire_expand_us(int W, int H, int S, int E) {
+    const double mpx = 1e-6 * W * H;
+    const int variant = drhip_conv3x3_winograd_split_pick_variant(W, H, S, 2 * E) ? 0 : drhip_conv3x3_winograd_pick_variant(W, H, S, 2 * E);
+    const double second = (variant & 0xf0) != 0 && (variant & 0x800) == 0 ? 4.0 : 0.0;         // (a kernel that adds up splits)
+    return (float)(3.7 + second + (W & 1 ? 5.8 : 2.4) * mpx * E + 0.133 * mpx * E * S + 0.00002 * E * S);
+}
+extern "C" float drhip_fire_squeeze_us(int W, int H, int C, int Sn, int pool) {
+    const double mpx = 1e-6 * W * H;
+    return (float)(pool ? 2.5 + 0.89 * mpx * C + 0.035 * mpx * C * Sn + 0.000114 * C * Sn : 2.8 + 0.63 * mpx * C + 0.026 * mpx * C * Sn + 0.000024 * C * Sn);
 }
 
 extern "C" size_t drhip_fire_bank_floats(int W, int H, int S, int E, int Sn, int pool) {

@@ -204,6 +204,69 @@ dR_Node* fire_next(const dR_Node* concat, const std::map<const dR_Node*, dR_Node
     return fire_squeeze(n, pooling, pairOf) ? n : nullptr;
 }
 
+// A module of a run in which each one's squeeze layer may ride in the launch in front.
+struct FireModule {
+    dR_Node *e3 = nullptr, *front = nullptr, *next = nullptr;   // its 3x3 layer; the layer whose launch may take its squeeze layer along; the next squeeze layer
+    dR_Conv2d_Data* conv = nullptr;                             // of e3
+    dR_Conv2d_Data* average = nullptr;                          // a 1x1 layer with a global average that reads it, where there is no next one
+    bool pool = false, joined = false, joins = false;           // a pooling in front of the next one; its squeeze layer rides in front, the next one's rides here
+};
+
+// The 1x1 layer in front of a global average that is the only reader of a pair's outputs and can take them pixel by pixel.
+dR_Conv2d_Data* fire_average(const dR_Node* concat) {
+    if (!tensor_hidden(concat) || concat->next_layers->length != 1) return nullptr;
+    const dR_Node* reader = nodes_of(concat->next_layers)[0];
+    if (reader->type != tConv2d || (long long)concat->oshape.s0 * concat->oshape.s1 * concat->oshape.s2 >= (1ll << 28)) return nullptr;
+    dR_Conv2d_Data* c = (dR_Conv2d_Data*)reader->layer;
+    return c->algo == drConv1x1Gemm && c->drFusedAvgPool && c->shape.s2 <= 1024 && c->shape.s3 <= 65535 ? c : nullptr;
+}
+
+// Whether it takes them so (the pair stores both forms in the same time).
+bool by_pixel_pays(const dR_Conv2d_Data* average) {
+    const int P = average->ishape.s0 * average->ishape.s1;
+    return drhip_conv1x1_pixels_us(P, average->shape.s2, average->shape.s3) < drhip_conv1x1_poolsum_us(P, average->shape.s2, average->shape.s3);
+}
+
+// Which squeeze layers of a run ride along: the cheapest way through it.  A launch that takes one along spares a launch and the trip of
+// 2E channels through memory, and does direct products on the fp32 matrix cores, filters loaded again for every 16 pixels, where
+// the Winograd kernels do fewer on faster ones: wide modules on large maps are better apart (us of a run of two modules, apart / together: 56x56 64->2x1024 99
+// / 153, 80x80 32->2x1024 122 / 180, 224x224 64->2x32 81 / 103; 14x14 64->2x256 19.6 / 17.9, 56x56 16->2x512 48 / 30), and
+// what a run gains in the middle may be worth its ends.
+void choose_fire_launches(std::vector<FireModule>& run) {
+    const float never = 1e30f;
+    std::vector<std::pair<bool, bool>> came(run.size());        // of module k: whether its squeeze layer rides, where the next one's does not / does
+    float cost[2] = {0.0f, run[0].front ? 0.0f : never};        // where this module's squeeze layer does not ride / rides
+    for (size_t k = 0; k < run.size(); ++k) {
+        const dR_Conv2d_Data* c = run[k].conv;
+        const int W = c->ishape.s0, H = c->ishape.s1, S = c->shape.s2, E = c->shape.s3;
+        float alone = 0.0f;
+        if (run[k].front) {                                     // (otherwise it is a launch of its own either way)
+            const bool pool = k > 0 && run[k - 1].pool;
+            const dR_Conv2d_Data* from = k > 0 ? run[k - 1].conv : c;
+            alone = drhip_fire_squeeze_us(from->ishape.s0, from->ishape.s1, k > 0 ? 2 * from->shape.s3 : ((const dR_Conv2d_Data*)run[0].front->layer)->shape.s3, S, pool);
+        }
+        const float apart = cost[0] + alone + drhip_fire_expand_us(W, H, S, E);
+        const int slices = k > 0 ? drhip_fire_slices(run[k - 1].conv->ishape.s0, run[k - 1].conv->ishape.s1, run[k - 1].conv->shape.s2, run[k - 1].conv->shape.s3, S, run[k - 1].pool) : 1;
+        float last = cost[1] + drhip_fire_us(W, H, S, E, 0, 0, slices);
+        if (run[k].average && by_pixel_pays(run[k].average))    // (which only a pair of this kind can lay out)
+            last -= drhip_conv1x1_poolsum_us(W * H, 2 * E, run[k].average->shape.s3) - drhip_conv1x1_pixels_us(W * H, 2 * E, run[k].average->shape.s3);
+        float on = never, first = never;
+        if (run[k].next) {
+            const int Sn = ((const dR_Conv2d_Data*)run[k].next->layer)->shape.s3;
+            on = cost[1] + drhip_fire_us(W, H, S, E, Sn, run[k].pool, slices);
+            if (!run[k].pool) first = cost[0] + alone + drhip_fire_us(W, H, S, E, Sn, 0, 0);    // (no launch pools behind a plain tensor)
+        }
+        came[k] = std::make_pair(last < apart, on < first);
+        cost[0] = std::min(apart, last);
+        cost[1] = std::min(on, first);
+    }
+    bool joins = false;                                         // (no module behind the last one)
+    for (size_t k = run.size(); k-- > 0;) {
+        run[k].joins = joins;
+        joins = run[k].joined = joins ? came[k].second : came[k].first;
+    }
+}
+
 // The squeeze layer behind a first layer and its pooling that has all its input channels in one workgroup of theirs.
 dR_Node* first_layer_squeeze(const dR_Node* n, const std::map<const dR_Node*, dR_Node*>& pairOf) {
     if (n->type != tConv2d || !((const dR_Conv2d_Data*)n->layer)->drFusedPool) return nullptr;
@@ -440,39 +503,40 @@ gboolean dR_planBuffers(dR_Graph* net) {
         std::map<const dR_Node*, dR_Node*> pairOf;              // either layer of a pair -> its 3x3 layer
         for (dR_Node* n : sched)
             if (dR_Node* e3 = fire_pair(n)) pairOf[e3] = pairOf[((dR_Conv2d_Data*)e3->layer)->drAbsorbed1x1] = e3;
-        auto pair_behind = [&](dR_Node* squeeze) { return (dR_Conv2d_Data*)pairOf[nodes_of(squeeze->next_layers)[0]]->layer; };
-        for (dR_Node* n : sched)
-            if (dR_Node* squeeze = first_layer_squeeze(n, pairOf)) {
-                ((dR_Conv2d_Data*)n->layer)->drSqueezeNext = squeeze;
-                ((dR_Conv2d_Data*)squeeze->layer)->drFireFrom = n;
-                pair_behind(squeeze)->drFire = TRUE;            // (reads sums, whether it takes a layer along or not)
-            }
+        auto pair_behind = [&](dR_Node* squeeze) { return pairOf[nodes_of(squeeze->next_layers)[0]]; };
+        std::map<const dR_Node*, FireModule> modules;           // by 3x3 layer
         for (dR_Node* n : sched) {
             dR_Node* e3 = fire_pair(n);
-            bool pool = false;
-            dR_Node* next = e3 ? fire_next(n, pairOf, &pool) : nullptr;
-            if (!next) continue;
-            dR_Conv2d_Data* c3 = (dR_Conv2d_Data*)e3->layer;
-            // (a chain does not begin behind a plain tensor with a pooling in it; in execution order, so what is in front is decided)
-            const dR_Node* squeeze = nodes_of(e3->previous_layers)[0];
-            if (pool && !(squeeze->type == tConv2d && ((const dR_Conv2d_Data*)squeeze->layer)->drFireFrom)) continue;
-            if (drhip_fire_slices(c3->ishape.s0, c3->ishape.s1, c3->shape.s2, c3->shape.s3, ((dR_Conv2d_Data*)next->layer)->shape.s3, pool) == 0) continue;
-            c3->drFire = TRUE;
-            c3->drFireNext = next;
-            c3->drFirePool = pool;
-            ((dR_Conv2d_Data*)next->layer)->drFireFrom = e3;
-            pair_behind(next)->drFire = TRUE;
+            if (!e3) continue;
+            FireModule& m = modules[e3];
+            m.conv = (dR_Conv2d_Data*)e3->layer;
+            m.e3 = e3;
+            m.next = fire_next(n, pairOf, &m.pool);
+            m.average = fire_average(n);
+            if (m.next && drhip_fire_slices(m.conv->ishape.s0, m.conv->ishape.s1, m.conv->shape.s2, m.conv->shape.s3, ((dR_Conv2d_Data*)m.next->layer)->shape.s3, m.pool) == 0) m.next = nullptr;
         }
-        // The last pair of a chain in front of a 1x1 layer and a global average: by pixel
         for (dR_Node* n : sched) {
-            dR_Node* e3 = fire_pair(n);
-            if (!e3 || !tensor_hidden(n) || n->next_layers->length != 1) continue;
-            dR_Conv2d_Data* c3 = (dR_Conv2d_Data*)e3->layer;
-            dR_Node* reader = nodes_of(n->next_layers)[0];
-            if (!c3->drFire || c3->drFireNext || reader->type != tConv2d || (long long)n->oshape.s0 * n->oshape.s1 * n->oshape.s2 >= (1ll << 28)) continue;
-            dR_Conv2d_Data* c = (dR_Conv2d_Data*)reader->layer;
-            if (c->algo != drConv1x1Gemm || !c->drFusedAvgPool || c->shape.s2 > 1024 || c->shape.s3 > 65535) continue;
-            c3->drByPixel = c->drByPixel = TRUE;
+            if (dR_Node* squeeze = first_layer_squeeze(n, pairOf)) modules[pair_behind(squeeze)].front = n;
+            std::map<const dR_Node*, FireModule>::iterator m = modules.find(n);
+            if (m != modules.end() && m->second.next) modules[pair_behind(m->second.next)].front = n;
+        }
+        for (dR_Node* n : sched) {
+            std::map<const dR_Node*, FireModule>::iterator m = modules.find(n);
+            if (m == modules.end() || (m->second.front && modules.count(m->second.front))) continue;        // (not where a run begins)
+            std::vector<FireModule> run(1, m->second);
+            while (run.back().next) run.push_back(modules[pair_behind(run.back().next)]);
+            choose_fire_launches(run);
+            for (const FireModule& k : run) {
+                k.conv->drFire = k.joined || k.joins;
+                if (k.joined) {
+                    dR_Node* squeeze = nodes_of(k.e3->previous_layers)[0];
+                    dR_Conv2d_Data* front = (dR_Conv2d_Data*)k.front->layer;
+                    ((dR_Conv2d_Data*)squeeze->layer)->drFireFrom = k.front;
+                    (modules.count(k.front) ? front->drFireNext : front->drSqueezeNext) = squeeze;
+                }
+                k.conv->drFirePool = k.joins && k.pool;
+                if (k.conv->drFire && k.average && by_pixel_pays(k.average)) k.conv->drByPixel = k.average->drByPixel = TRUE;
+            }
         }
     }
     auto root_of = [&](dR_Node* n, int* offset) {

@@ -300,6 +300,9 @@ int drhip_conv1x1_poolsum_f32(const float* in, const float* w, const float* bias
 int drhip_conv1x1_pixels_tile(int P);
 int drhip_conv1x1_pixels_layout_f32(const float* w /* [I][O] */, float* F, int I, int O, void* stream);
 int drhip_conv1x1_pixels_poolsum_f32(const float* in, const float* F, const float* bias, float* partials, int P, int I, int O, int relu, void* stream);
+/* Estimates of either launch's microseconds in a pass, for the choice. */
+float drhip_conv1x1_poolsum_us(int P, int I, int O);
+float drhip_conv1x1_pixels_us(int P, int I, int O);
 /* A 3x3 / stride-2 max pooling followed by a 1x1 convolution, without the pooled tensor in between:
  * in is the pooling's input [I][Hin][Win]; the convolution works on the pooled map of
  * ceil(Win/2) x ceil(Hin/2) pixels, whose samples it takes while loading (maximum over the window
@@ -326,6 +329,11 @@ int drhip_conv1x1_pick_variant(int P, int I, int O);
  * ([I][O][kh][kw]) and biases (NULL: none); drhip_fire_bank_floats floats, 16-byte aligned on the device.  No counterpart in the
  * reference, which runs these layers one after the other (src/dR_nodes_conv2d.c:37-81, src/dR_nodes_pooling.c:277-401). */
 int    drhip_fire_slices(int W, int H, int S, int E, int Sn, int pool);
+/* Estimates of microseconds in a pass, for the choice: such a launch (0 where a shape is not covered; slicesIn as below), the expand layers as a launch of their own
+ * (drhip_conv3x3_winograd_*), and the squeeze layer (Sn channels on C of a WxH map, pooled 3x3/2 on load with pool != 0) as one. */
+float  drhip_fire_us(int W, int H, int S, int E, int Sn, int pool, int slicesIn);
+float  drhip_fire_expand_us(int W, int H, int S, int E);
+float  drhip_fire_squeeze_us(int W, int H, int C, int Sn, int pool);
 size_t drhip_fire_bank_floats(int W, int H, int S, int E, int Sn, int pool);
 size_t drhip_fire_partials_floats(int W, int H, int S, int E, int Sn, int pool);
 int    drhip_fire_layout_f32(const float* w1, const float* w3, const float* b1, const float* b3, const float* wn, float* bank,

@@ -282,6 +282,7 @@ def test_fire_modules_in_a_chain(oracle, gpu, chain):
     (91, 74, 3, 64, 16, 64, 1000, True),        # SqueezeNet's ends around one module; odd maps
     (18, 14, 4, 20, 33, 32, 17, False),         # ragged channels, one block of pooled pixels and a bit
     (132, 260, 2, 64, 64, 256, 10, True),       # 33 x 65 pixels: tiles of 32 in front of the average
+    (132, 260, 2, 64, 64, 256, 333, True),      # the same pixel by pixel
     (24, 10, 1, 8, 8, 32, 5, True),             # one input channel: the squeeze layer stays a kernel of its own
 ], ids=lambda v: str(v))
 def test_fire_chain_with_both_ends(oracle, gpu, w, h, cin, first, squeeze, expand, classes, bias):
