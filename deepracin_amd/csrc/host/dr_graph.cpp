@@ -304,26 +304,20 @@ gint dR_downloadOutputs(dR_Graph* net, gfloat** hosts, gint n) {
 // without waiting; after the last node the pass is awaited once, a node's device time
 // (node->drLastKernelMs) is the sum over its kernels, and their sum goes to
 // clConfig->totalKernelGPUTime, printed like the reference does.
-// Fusions decided by the buffer planner leave some nodes without a stored tensor of their own.
+// Fusions decided by the buffer planner leave some nodes without a tensor that a debug layer could be read from: not stored at
+// all, or in another layer's place, by pixel, or later in the pass.
 static bool tensor_fused_away(const dR_Node* n) {
+    if (n->type != tFullyConnected || !n->output || ((const dR_FC_Data*)n->layer)->drInSoftmax)
+        if (tensor_unstored(n)) return true;
     if (n->type == tConv2d) {
         const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
         const dR_Conv2d_Data* pair = c->drAbsorbedBy ? (const dR_Conv2d_Data*)c->drAbsorbedBy->layer : c;
-        return c->drFusedPool || c->drFusedAvgPool || c->drFireFrom || pair->drFireNext || pair->drByPixel;
+        return c->drFusedPool || pair->drFireNext || pair->drByPixel;
     }
     if (n->type == tConcat && ((const dR_Concat_Data*)n->layer)->drFused)
         for (const dR_Node* p : nodes_of(n->previous_layers))
-            if (p->type == tConv2d && (((const dR_Conv2d_Data*)p->layer)->drFireNext || ((const dR_Conv2d_Data*)p->layer)->drByPixel)) return true;
-    if (n->type == tPooling && ((const dR_Pooling_Data*)n->layer)->drFused && n->next_layers && n->next_layers->length == 1) {
-        const dR_Node* c = (const dR_Node*)n->next_layers->first->element;
-        if (c->type != tConv2d) return false;
-        const dR_Node* from = ((const dR_Conv2d_Data*)c->layer)->drFireFrom;
-        return ((const dR_Conv2d_Data*)c->layer)->drPooledInput == n || (from && ((const dR_Conv2d_Data*)from->layer)->drSqueezeNext);
-    }
-    if (n->type == tSlice) return ((const dR_Slice_Data*)n->layer)->drReadThrough;
-    if (n->type == tElemWise1Op) return ((const dR_ElemWise1Op_Data*)n->layer)->drInConcat;     // (not stored yet where a debug layer is read)
-    if (n->type == tFullyConnected) return ((const dR_FC_Data*)n->layer)->drInSoftmax || (((const dR_FC_Data*)n->layer)->drDeferReduce && !n->output);
-    return false;
+            if (p->type == tConv2d && ((const dR_Conv2d_Data*)p->layer)->drByPixel) return true;
+    return n->type == tElemWise1Op && ((const dR_ElemWise1Op_Data*)n->layer)->drInConcat;
 }
 
 gboolean dR_apply(dR_Graph* net) {

@@ -62,7 +62,9 @@ inline void*  stream_of(const dR_Graph* net) { return net->clConfig->hipStream; 
 void link_single_input(dR_Node* node, dR_Node* input, const char* what);
 // Report a failed drhip_* call the way dR_openCLError does: message to stdout, FALSE to the caller.
 gboolean device_failed(dR_Graph* net, int status, const char* what);
-// Slices of the pixel sums that a 1x1 layer with drFusedAvgPool leaves.
+// Does a fusion of the buffer planner leave no launch that writes or reads the tensor of n (unless it is an output)?  Valid once buffers are planned.
+bool tensor_unstored(const dR_Node* n);
+// Slices of the pixel sums that a layer with drFusedAvgPool (1x1 or strided 3x3) leaves.
 int avgpool_slices(const dR_Conv2d_Data* conv);
 // Copy caller-owned floats.
 float* dup_floats(const float* src, size_t n);

@@ -30,6 +30,7 @@ struct Root {
     int firstDef = 1 << 30;   // schedule position of the earliest writer
     int lastUse = -1;         // schedule position of the latest reader
     bool pinned = false;      // feed/output/caller-supplied: never shares storage
+    bool unstored = false;    // no launch writes or reads it: shares a place without memory
     dR_MemoryHandler* phys = nullptr;
 };
 
@@ -280,6 +281,31 @@ dR_Node* first_layer_squeeze(const dR_Node* n, const std::map<const dR_Node*, dR
            (long long)(pooling->oshape.s0 + 1) * (pooling->oshape.s1 + 1) * 64 < (1ll << 28) ? squeeze : nullptr;
 }
 }  // namespace
+
+bool dr::tensor_unstored(const dR_Node* n) {
+    auto next_conv = [](const dR_Node* p) -> const dR_Conv2d_Data* {
+        const std::vector<dR_Node*> readers = nodes_of(p->next_layers);
+        return readers.size() == 1 && readers[0]->type == tConv2d ? (const dR_Conv2d_Data*)readers[0]->layer : nullptr;
+    };
+    switch (n->type) {
+        case tConv2d: {                 // (a maximum behind it: its tensor is the pooling's)
+            const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
+            return c->drFusedAvgPool || c->drFireFrom || (c->drFusedPool && c->drPoolAverage);
+        }
+        case tConcat:
+            if (((const dR_Concat_Data*)n->layer)->drFused)
+                for (const dR_Node* p : nodes_of(n->previous_layers))
+                    if (p->type == tConv2d && ((const dR_Conv2d_Data*)p->layer)->drFireNext) return true;
+            return false;
+        case tPooling:
+            if (const dR_Conv2d_Data* c = ((const dR_Pooling_Data*)n->layer)->drFused ? next_conv(n) : nullptr)
+                return c->drPooledInput == n || (c->drFireFrom && ((const dR_Conv2d_Data*)c->drFireFrom->layer)->drSqueezeNext);
+            return false;
+        case tSlice: return ((const dR_Slice_Data*)n->layer)->drReadThrough;
+        case tFullyConnected: return ((const dR_FC_Data*)n->layer)->drInSoftmax || ((const dR_FC_Data*)n->layer)->drDeferReduce;
+        default: return false;
+    }
+}
 
 extern "C" {
 
@@ -557,6 +583,7 @@ gboolean dR_planBuffers(dR_Graph* net) {
             r.owner = owner;
             r.size = owner->getRequiredOutputBufferSize(owner);
             r.pinned = owner->type == tDataFeedNode || owner->output || (owner->outputBuf && owner->outputBuf->outputBuf);
+            r.unstored = !r.pinned && tensor_unstored(owner);
             it = roots.insert(std::make_pair(owner, r)).first;
             rootOrder.push_back(owner);
         }
@@ -617,14 +644,14 @@ gboolean dR_planBuffers(dR_Graph* net) {
         } else {
             int best = -1;
             for (size_t i = 0; i < pool.size(); ++i) {
-                if (pool[i]->drLastUse >= r.firstDef) continue;          // still being read
+                if (pool[i]->drLastUse >= r.firstDef || (bool)pool[i]->drUnstored != r.unstored) continue;       // still being read
                 if (best < 0) { best = (int)i; continue; }
                 const int sb = pool[best]->size, si = pool[i]->size;
                 const bool fitb = sb >= r.size, fiti = si >= r.size;
                 if ((fiti && !fitb) || (fiti && fitb && si < sb) || (!fiti && !fitb && si > sb)) best = (int)i;
             }
             if (best >= 0) h = pool[best];
-            else { h = dR_newMemoryHandler(FALSE); pool.push_back(h); dR_list_append(handlers, h); }
+            else { h = dR_newMemoryHandler(FALSE); h->drUnstored = r.unstored; pool.push_back(h); dR_list_append(handlers, h); }
         }
         h->size = std::max(h->size, r.size);
         h->drFirstDef = std::min(h->drFirstDef, r.firstDef);
@@ -669,13 +696,14 @@ gboolean dR_estimateAndAllocateBuffers(dR_Graph* net) {
     for_each(net->streamBufferHandlers, [&](void* p) {
         dR_MemoryHandler* h = (dR_MemoryHandler*)p;
         h->bufptr = &h->buf;
+        if (h->drUnstored) return;
         ok = ok && dR_createFloatBuffer(net, h->bufptr, h->size, CL_MEM_READ_WRITE);
         if (debug(net)) say("Stream buffer with size %d created!\n", h->size);
     });
     if (!ok) return FALSE;
     for_each(net->drViewHandlers, [&](void* p) {
         dR_MemoryHandler* v = (dR_MemoryHandler*)p;
-        v->buf = (cl_mem)((float*)v->drViewOf->buf + v->drViewOffset);
+        v->buf = v->drViewOf->drUnstored ? NULL : (cl_mem)((float*)v->drViewOf->buf + v->drViewOffset);
         v->bufptr = &v->buf;
     });
     // per-node parameter buffers (weights, biases, scratch)

@@ -389,6 +389,33 @@ def test_schedule_order_and_buffer_plan(lib, oracle, name):
         assert len({p[0] for p in plan}) < len(spec) // 2
 
 
+def test_tensors_that_fusions_remove_have_no_memory(lib):
+    """SqueezeNet's fire modules leave sums in workspaces: of its tensors there is memory for the image, the last module's outputs
+    (pixel by pixel) and the outputs of the graph, and for all of them where every layer is an output."""
+    class Handler(ctypes.Structure):
+        _fields_ = FullHandler._fields_ + [("drUnstored", ctypes.c_int)]
+
+    def planned(outputs):
+        spec, _, outs = configs.CONFIGS["squeezenet"](seed=2)
+        with dr.Environment() as env:
+            g = env.create_graph()
+            nodes = configs.build_graph(g, spec, outs if outputs is None else [i for i in range(1, len(spec))])
+            assert lib.dR_propagateShapesAndSchedule(g.ptr) == 1 and lib.dR_planBuffers(g.ptr) == 1
+            stored, removed = {}, 0
+            for n in nodes:
+                h = ctypes.cast(dr.node_struct(n).outputBuf, ctypes.POINTER(Handler))
+                if h.contents.drViewOf:
+                    h = ctypes.cast(h.contents.drViewOf, ctypes.POINTER(Handler))
+                if h.contents.drUnstored:
+                    removed += 1
+                else:
+                    stored[ctypes.addressof(h.contents)] = h.contents.size
+            return len(nodes), removed, sum(stored.values())
+    nodes, removed, floats = planned(None)
+    assert removed > nodes // 2 and floats <= 224 * 224 * 3 + 14 * 14 * 512 + 2 * 1000 + 14 * 14 * 64
+    assert planned("all")[1] == 0
+
+
 def _odd_offset_norm_spec():
     """feed 5x5x3 -> {1x1 conv to 3 channels (75 floats), Normalization} -> channel concat."""
     rng = np.random.default_rng(5)
