@@ -367,10 +367,6 @@ def _from_chw(graph, flat, shape):
 
 def download_outputs(graph, squeeze=True):
     """Fetch every output buffer (blocking) in the graph's interface layout."""
-    return _outputs(graph, squeeze)
-
-
-def _outputs(graph, squeeze):
     n = min(graph.num_outputs, 10)
     shapes = [node.out_shape for node in graph.outnodes[:n]]
     if None in shapes:          # not prepared: there are none yet
@@ -388,7 +384,7 @@ def apply(graph):
     """Run the graph once and return the outputs (reference :444-465)."""
     if not graph.lib.dR_applyAhead(graph.ptr):          # (the arrays are made while it runs)
         raise RuntimeError("DR Error: deepRACIN apply failed!")
-    return _outputs(graph, True)
+    return download_outputs(graph)
 
 
 def mark_as_output(node):

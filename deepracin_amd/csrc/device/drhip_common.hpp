@@ -129,12 +129,13 @@ __device__ inline float deferred_element(const drhip_deferred_vec& d, int row) {
 #pragma unroll
         for (int u = 0; u < 32; ++u) s += v[u];
     }
-    for (; sl + 16 == d.slices; sl += 16) {         // (a GEMV that fills the chip leaves 16 slices: one round, not two)
+    if (sl + 16 == d.slices) {                      // (a GEMV that fills the chip leaves 16 slices: one round, not two)
         float v[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) v[u] = pp[(size_t)(sl + u) * d.n];
 #pragma unroll
         for (int u = 0; u < 16; ++u) s += v[u];
+        sl += 16;
     }
     if (d.slices - sl > 8) {                        // the ragged end in one round as well: clamped loads, zeros by select
         float v[32];
