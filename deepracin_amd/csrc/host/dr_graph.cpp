@@ -28,13 +28,35 @@ static Range out_range(dR_Node* n) {
 }
 static bool overlap(const Range& a, const Range& b) { return a.lo && b.lo && a.lo < b.hi && b.lo < a.hi; }
 
+// What the launch of a node reads and writes of the planned memory: fusions read tensors in front of the node's own inputs, and
+// write those of other nodes.
+struct Touched { std::vector<Range> reads, writes; };
+static Touched touched_by(dR_Node* n) {
+    Touched t;
+    if (n->type == tConv2d && ((const dR_Conv2d_Data*)n->layer)->drAbsorbedBy) return t;       // (its sibling's launch)
+    auto reads_inputs_of = [&](const dR_Node* of) { for (dR_Node* p : nodes_of(of->previous_layers)) t.reads.push_back(out_range(p)); };
+    reads_inputs_of(n);
+    t.writes.push_back(out_range(n));
+    if (n->type == tConv2d) {
+        const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
+        if (c->drPooledInput) reads_inputs_of(c->drPooledInput);
+        if (c->drAbsorbed1x1) t.writes.push_back(out_range(c->drAbsorbed1x1));
+        if (c->drFusedPool && c->drPoolAverage) t.writes.push_back(out_range((dR_Node*)n->next_layers->first->element));
+    }
+    if (n->type == tSoftmax && ((const dR_Softmax_Data*)n->layer)->drFcInput) reads_inputs_of(((const dR_Softmax_Data*)n->layer)->drFcInput);
+    return t;
+}
+
 static bool can_run_beside(dR_Node* a, dR_Node* b) {
     for (dR_Node* p : nodes_of(b->previous_layers)) if (p == a) return false;
     for (dR_Node* p : nodes_of(a->previous_layers)) if (p == b) return false;
-    const Range wa = out_range(a), wb = out_range(b);
-    if (overlap(wa, wb)) return false;
-    for (dR_Node* p : nodes_of(a->previous_layers)) if (overlap(out_range(p), wb)) return false;
-    for (dR_Node* p : nodes_of(b->previous_layers)) if (overlap(out_range(p), wa)) return false;
+    const Touched ta = touched_by(a), tb = touched_by(b);
+    for (const Range& w : ta.writes) {
+        for (const Range& r : tb.writes) if (overlap(w, r)) return false;
+        for (const Range& r : tb.reads) if (overlap(w, r)) return false;
+    }
+    for (const Range& w : tb.writes)
+        for (const Range& r : ta.reads) if (overlap(w, r)) return false;
     return true;
 }
 

@@ -947,6 +947,42 @@ def test_random_topologies(oracle, gpu, seed):
                                      terms=spec_terms(spec[i]))
 
 
+def _branches_spec(kind):
+    """Graphs whose memory a launch touches beyond its own node's inputs and output, beside independent nodes that are planned into
+    the same places: a pooled layer that averages, one pooled on load, a small layer inside its softmax."""
+    st = configs._Streams(80)
+    conv, pool = configs._conv, configs._maxpool
+    if kind == "average":           # node 4 writes the average of node 5 where node 1 was, which node 3 in front of it reads
+        spec = [{"op": "feed", "shape": (124, 70, 3)}, conv(st, 0, 1, 3, 16), {"op": "scalar", "in": 0, "kind": 2, "value": 0.5}, conv(st, 1, 1, 16, 9), conv(st, 2, 3, 3, 33),
+                {"op": "pool", "in": 4, "window": (2, 2, 1), "stride": (2, 2, 1), "kind": 1}, conv(st, 3, 1, 9, 7), conv(st, 5, 1, 33, 5)]
+    elif kind == "on load":         # node 6 writes where node 1 was, which node 3 in front of it pools on load
+        spec = [{"op": "feed", "shape": (37, 29, 8)}, conv(st, 0, 5, 8, 16), pool(1, 3, 2), conv(st, 2, 1, 16, 24), conv(st, 0, 1, 8, 16), conv(st, 4, 3, 16, 12),
+                conv(st, 5, 1, 12, 16), conv(st, 3, 1, 24, 6), conv(st, 6, 1, 16, 4)]
+    else:                           # node 6 writes where node 1 was, which the softmax in front of it reads for the layer that it computes
+        fc = lambda src, k, n: {"op": "fc", "in": src, "w": (st.next().standard_normal((k, n)) * k ** -0.5).astype(np.float32), "b": None, "relu": True}
+        spec = [{"op": "feed", "shape": (60, 1, 1)}, fc(0, 60, 60), fc(1, 60, 20), {"op": "softmax", "in": 2}, fc(0, 60, 50), fc(4, 50, 60), fc(5, 60, 60), fc(6, 60, 30), {"op": "softmax", "in": 7}]
+    read = {n["in"] for n in spec[1:]}
+    return spec, [i for i in range(1, len(spec)) if i not in read]
+
+
+@pytest.mark.parametrize("kind", ["average", "on load", "softmax"])
+def test_branches_keep_off_memory_that_fusions_touch(oracle, gpu, kind):
+    """Independent nodes on side streams (DR_BRANCHES=1): every replay as node by node."""
+    spec, outs = _branches_spec(kind)
+    rng = np.random.default_rng(4)
+    w, h, c = spec[0]["shape"]
+    inputs = [rng.standard_normal((c, h, w)).astype(np.float32) for _ in range(4)]
+    eager, _ = _run_many(spec, outs, inputs, graph_mode=False)
+    forked, used = _run_many(spec, outs, inputs, graph_mode=True, branches=True)
+    assert used
+    want = oracle.run_spec(spec, {0: inputs[0]})
+    for i, a in zip(outs, eager[0]):
+        assert rel_err(a, want[i]) <= LAYER_TOL
+    for a, b in zip(eager, forked):
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
+
+
 def test_joined_layers_of_two_graphs_on_two_streams(lib, gpu):
     """Pieces of a split-operand layer wait for each other inside the launch.  Two graphs with such a layer, each on its own
     stream, run at the same time: every pass as if it were alone, and no piece waited in vain."""
