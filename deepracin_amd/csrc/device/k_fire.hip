@@ -412,22 +412,26 @@ extern "C" int drhip_fire_slices(int W, int H, int S, int E, int Sn, int pool) {
 }
 
 // What the launches of a module take in a pass, us, for the choice between them: the launch above from the clocks of its plan, the others from the
-// products they do and the numbers they move (mpx: millions of pixels; the Winograd kernels store maps of odd width less well).  Fitted to 330 shapes, maps
-// of 13x13 to 320x320, 16 to 64 channels to 2x32 to 2x1024: half of them come out within 7 % and nine of ten within 20 %.  The launch above is put a tenth
-// lower, which lost least: on 450 random networks of one to six modules the choice is 0.8 % slower than the best side on average and 12 % at most, always
-// taking the next layer along 0.8 and 18 %, never doing so 20 and 90 %; in runs of alike modules always doing so lost up to 70 % (80x80 32->2x1024).
+// products they do and the numbers they move (the Winograd kernels store maps of odd width less well).  Fitted to 330 shapes, maps of 13x13 to 320x320, 16 to 64
+// channels to 2x32 to 2x1024: half of them come out within 6 %, nine of ten within 17 %.  The launch above is put 3 % lower, which lost least.
+// On 450 random networks of one to six modules the choice is 0.8 % slower than the better side on average and 14 % at most, always taking the next layer
+// along 0.8 and 19 %, never doing so 19 and 94 %; runs of four alike modules, us apart / chosen / always along: 112x112 64->2x256 214 / 214 / 249, 80x80
+// 32->2x1024 242 / 240 / 382, 56x56 64->2x256 83 / 82 / 90, 28x28 64->2x256 46 / 38 / 38; left on the slower side: 64x64 64->2x256 87 / 95 / 95.
 extern "C" float drhip_fire_us(int W, int H, int S, int E, int Sn, int pool, int slicesIn) {
     FirePlan p;
     if (!fire_plan(W, H, S, E, Sn, pool, &p)) return 0.0f;
+    const int perCu = ceil_div(p.nbx * p.nby * p.slices, num_cu());
+    const double us = p.clocks / 2400;
     // (every workgroup adds up all slices of its patch: with sixteen of them 10 to 30 us of 50 to 100 on large maps)
-    const double patches = 16.0 * p.S16 * 4 / 48 / 2400 * p.hpx * slicesIn * ceil_div(p.nbx * p.nby * p.slices, num_cu());
-    return 0.9f * (float)((pool ? 1.5 + 1.15 * p.clocks / 2400 : 1.8 + 0.92 * p.clocks / 2400) + 1.8 * std::max(0.0, patches - 2));
+    const double patches = std::max(0.0, 16.0 * p.S16 * 4 / 48 / 2400 * p.hpx * slicesIn * perCu - 2);
+    return 0.97f * (float)(pool ? 1.6 + 1.12 * us + patches : Sn > 0 ? 2.1 + (0.73 + 0.06 * p.S16) * us + 1.8 * patches : 1.95 + 0.89 * us + 1.8 * patches);
 }
 extern "C" float drhip_fire_expand_us(int W, int H, int S, int E) {
-    const double mpx = 1e-6 * W * H;
-    const int variant = drhip_conv3x3_winograd_split_pick_variant(W, H, S, 2 * E) ? 0 : drhip_conv3x3_winograd_pick_variant(W, H, S, 2 * E);
-    const double second = (variant & 0xf0) != 0 && (variant & 0x800) == 0 ? 4.0 : 0.0;         // (a kernel that adds up splits)
-    return (float)(3.7 + second + (W & 1 ? 5.8 : 2.4) * mpx * E + 0.133 * mpx * E * S + 0.00002 * E * S);
+    const double mpxE = 1e-6 * W * H * E;
+    if (drhip_conv3x3_winograd_split_pick_variant(W, H, S, 2 * E)) return (float)(5.4 + (W & 1 ? 5.4 : 2.9) * mpxE + 0.094 * mpxE * S + 0.000009 * E * S);
+    const int variant = drhip_conv3x3_winograd_pick_variant(W, H, S, 2 * E);
+    const double second = (variant & 0xf0) != 0 && (variant & 0x800) == 0 ? 3.5 : 0.0;          // (a kernel that adds up splits)
+    return (float)(3.7 + second + (W & 1 ? 4.6 : 1.7) * mpxE + 0.186 * mpxE * S + 0.00001 * E * S);
 }
 extern "C" float drhip_fire_squeeze_us(int W, int H, int C, int Sn, int pool) {
     const double mpx = 1e-6 * W * H;
