@@ -608,6 +608,131 @@ conv3x3_direct_mfma_kernel(const float* __restrict__ in, const float* __restrict
         finish(idx, bias ? bias[min(o0 + (idx >> 5), O - 1)] : 0.0f);
 }
 
+// The same for layers with fewer 32x32 tiles than CUs: 16 pixels x 16*NB channels a workgroup on v_mfma_f32_16x16x4_f32, that is two or
+// four times the workgroups and a half or a quarter of the matrix work on the busiest CU.  Same filter bank: a lane has pixel or output
+// channel lane%16 and, of a chunk of eight channels, c = 4*(lane/32) + lane/16%2 for one k-step and c + 2 for the other, whose
+// filters are neighbours in the bank (8 bytes a lane and tap, 512 in a row).  The first two stages of a wave are requested at its
+// start, which with eight waves are all there are up to 128 channels: one trip to memory.
+// What bounds it: that trip, then the MFMAs of a SIMD and the loads of the CU's address unit, which take about as long as
+// each other (28x28 96->128 from 56x56: 3500 clocks).
+template <int NB, int S>
+__global__ void __launch_bounds__(512)
+conv3x3_direct_mfma16_kernel(const float* __restrict__ in, const float* __restrict__ F, const float* __restrict__ bias,
+                             float* __restrict__ out, unsigned wh, unsigned io, unsigned WoMul, unsigned cfg) {
+    // (arguments as above; with cfg bit 6 a tile is 16 pixels)
+    constexpr int OB = 16 * NB, KC = kDmKC, kPitch16 = 17, NA = 6;
+    typedef float f32x2d __attribute__((ext_vector_type(2)));
+    const int W = (int)(wh & 0xffffu), H = (int)(wh >> 16), I = (int)(io & 0xffffu), O = (int)(io >> 16);
+    const int Wo = W / S, Ho = H / S;
+    const FastDiv Wod = {(unsigned)Wo, WoMul, cfg & 31u};
+    const int relu = (int)((cfg >> 5) & 1u), KW = (int)(cfg >> 8);
+    const bool sums = (cfg >> 6 & 1u) != 0;
+    extern __shared__ float part[];         // [KW][OB][kPitch16]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, parity = lane >> 4 & 1, hi = lane >> 5;
+    const int o0 = blockIdx.y * OB, p0 = blockIdx.x * 16;
+    const int P = Wo * Ho, plane = H * W;
+    const int nChunks = (I + KC - 1) / KC, Opad = dm_opad(O);
+
+    const int p = p0 + l16, pc = min(p, P - 1);
+    const int y = fast_div(pc, Wod), x = pc - y * Wo;
+    const bool shifted = x == 0;            // (as above)
+    const int xLoad = x * S - 1 + (shifted ? 1 : 0), cLane = 4 * hi + parity;
+    const bool c2ok = x * S + 1 < W;
+    unsigned offRow[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int iy = y * S - 1 + d;
+        offRow[d] = (p < P && iy >= 0 && iy < H) ? 4u * (unsigned)(cLane * plane + iy * W + xLoad) : kDmOutOfRange;
+    }
+    const __amdgpu_buffer_rsrc_t rF = __builtin_amdgcn_make_buffer_rsrc((void*)F, 0, 9 * nChunks * Opad * 8 * 4, kDmBufferFlags);
+    const unsigned fOff = 4u * (unsigned)((o0 + l16) * 8 + 4 * parity + 2 * hi);
+
+    // Channels cbase + cLane and two on.  Every resource starts at its own channel and ends with the tensor: channels that do not exist read
+    // zeros, and nothing is read behind the last one's last sample.
+    f32x4d raw[2][2][3];
+    f32x2d f[2][9][NB];
+    auto load_stage = [&](int buf, int ch) {
+        const int chF = min(ch, nChunks - 1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int c = ch * KC + 2 * k, left = max(I - c, 0);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(in + (size_t)min(c, I) * plane), 0, left * plane * 4, kDmBufferFlags);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) raw[buf][k][d] = dm_buf_load4(r, offRow[d], 0u);
+        }
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                f[buf][tap][nb] = __builtin_bit_cast(f32x2d, __builtin_amdgcn_raw_buffer_load_b64(rF, (int)fOff + 512 * nb, (int)(4u * (unsigned)((tap * nChunks + chF) * Opad * 8)), 0));
+    };
+    load_stage(0, wave);
+    if (wave + KW < nChunks) load_stage(1, wave + KW);
+    const int ol = tid >> 4;                // this thread finishes pixel tid%16 of this channel (and with few waves of others)
+    const float biasEarly = bias && ol < OB ? bias[min(o0 + ol, O - 1)] : 0.0f;
+
+    f32x4d acc[NB][NA];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) acc[nb][a] = f32x4d{0.f, 0.f, 0.f, 0.f};
+    auto stage = [&](int buf, int ch) {
+        float b[2][9];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const f32x4d v = raw[buf][k][d];
+                b[k][3 * d + 0] = shifted ? 0.0f : v[0];
+                b[k][3 * d + 1] = shifted ? v[0] : v[1];
+                const float third = shifted ? v[1] : v[2];
+                b[k][3 * d + 2] = c2ok ? third : 0.0f;
+            }
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    acc[nb][(2 * tap + k) % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[buf][tap][nb][k], b[k][tap], acc[nb][(2 * tap + k) % NA], 0, 0, 0);
+        if (ch + 2 * KW < nChunks) load_stage(buf, ch + 2 * KW);
+    };
+    for (int ch = wave; ch < nChunks; ch += 2 * KW) {
+        stage(0, ch);
+        if (ch + KW < nChunks) stage(1, ch + KW);
+    }
+
+    // D: lane -> pixel lane%16, register r -> channel 4*(lane/16) + r; the waves' sums meet in LDS, added in wave order
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float v = ((acc[nb][0][r] + acc[nb][1][r]) + (acc[nb][2][r] + acc[nb][3][r])) + (acc[nb][4][r] + acc[nb][5][r]);
+            part[(wave * OB + 16 * nb + 4 * (lane >> 4) + r) * kPitch16 + l16] = v;
+        }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    for (int idx = tid; idx < OB * 16; idx += 64 * KW) {
+        const int oc = idx >> 4, o = o0 + oc, pp = p0 + (idx & 15);
+        float v = 0.0f;
+        for (int k = 0; k < KW; ++k) v += part[(k * OB + oc) * kPitch16 + (idx & 15)];
+        v += idx == tid ? biasEarly : bias ? bias[min(o, O - 1)] : 0.0f;
+        if (relu) v = fmaxf(v, 0.0f);
+        if (sums) {
+            v = pp < P ? v : 0.0f;
+#pragma unroll
+            for (int k = 1; k < 16; k *= 2) v += __shfl_xor(v, k);
+            if (o < O && (idx & 15) == 0) store_through(out + (size_t)blockIdx.x * O + o, v);
+        } else if (o < O && pp < P) {
+            store_through(out + (size_t)o * P + pp, v);
+        }
+    }
+}
+
 template <int OCT>
 static int launch_direct(const float* in, const float* w, const float* bias, float* out,
                          int W, int H, int I, int O, int kw, int kh, int sx, int sy, int relu, hipStream_t s) {
@@ -734,8 +859,9 @@ extern "C" int drhip_conv3x3_direct_filter_layout_f32(const float* w, float* F, 
     return launched("direct_filter_layout_kernel");
 }
 
-// variant = waves per workgroup (1, 2, 4, 8) | 0x10 for 64 output channels per workgroup (else 32)
-extern "C" int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O) {
+// variant = waves per workgroup (1, 2, 4, 8) | 0x10 for 64 output channels per workgroup (else 32); with 0x20 16 pixels (else 32) and 32
+// or 16 channels
+static int direct_pick32(int Wo, int Ho, int I, int O) {
     const int nChunks = ceil_div(I, kDmKC);
     const int tiles = ceil_div(Wo * Ho, 32);
     // 64 channels per workgroup share every window between two MFMA sets; taken once such blocks alone give every
@@ -747,6 +873,19 @@ extern "C" int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O) {
     while (kw < 4 && nChunks >= 4 * kw) kw *= 2;
     if (tiles * ceil_div(O, wide ? 64 : 32) < num_cu() && nChunks >= 8) kw = 8;
     return kw | (wide ? 0x10 : 0);
+}
+
+// Tiles of 16 pixels where those of 32 leave CUs idle: 16 channels each if that makes no more workgroups than CUs, else 32 (one workgroup a
+// CU of half of the matrix work each). A workgroup too many costs as much as a second round. us, 32 pixels / 16 pixels x 16 / x 32 channels / split
+// bank: from 28x28 by stride 2, 128->192 8.0 / 5.0 / 6.7 / 9.2, 512->512 21.5 / 21.1 / 18.6 / 30.3; 56x56 96->128 6.8 / 6.2 / 6.1 / 7.7, 128->256 8.5 / 11.3 /
+// 12.3 / 9.8; 48x48 72->96 6.5 / 4.2 / 5.6 / 6.9; 20x20 64->64 5.5 / 3.8 / 4.6 / 5.9; 14x14 256->256 by stride 1 12.3 / 7.3 / 10.5.
+// Error against 64 bits, rms relative, 32 / 16 pixels / split bank: 28x28 128->192 1.2e-7 / 9.8e-8 / 1.1e-7, 20x20 64->64 1.0e-7 / 9.3e-8 / 9.6e-8,
+// 28x28 512->512 2.2e-7 / 1.5e-7 / 1.9e-7 (six short chains a wave and block).
+extern "C" int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O) {
+    const int v = direct_pick32(Wo, Ho, I, O), nChunks = ceil_div(I, kDmKC), kw = nChunks >= 8 ? 8 : 4;
+    if ((v & 0x10) || (nChunks >= 8 && v != 8)) return v;          // (a workgroup per CU as it is)
+    const long long tiles = ceil_div(Wo * Ho, 16);
+    return tiles * ceil_div(O, 16) <= num_cu() ? 0x20 | kw : tiles * ceil_div(O, 32) <= num_cu() ? 0x30 | kw : v;
 }
 
 static int conv3x3_direct_mfma(const float* in, const float* F, const float* bias, float* out,
@@ -761,17 +900,17 @@ static int conv3x3_direct_mfma(const float* in, const float* F, const float* bia
     DRHIP_REQUIRE((long long)W * H * I < (1ll << 29) && (long long)Wo * Ho * O < (1ll << 31) && (long long)(I + 7) * (O + 31) * 9 < (1ll << 29),
                   "drhip_conv3x3_direct_mfma_f32: tensor too large for 32-bit byte offsets");
     DRHIP_REQUIRE(((size_t)F & 15) == 0, "drhip_conv3x3_direct_mfma_f32: the filter bank must be 16-byte aligned");
-    if (variant == 0) variant = drhip_conv3x3_direct_pick_variant(Wo, Ho, I, O);
-    const int kw = variant & 0xf, wide = (variant & 0x10) != 0;
-    DRHIP_REQUIRE((variant >> 5) == 0 && (kw == 1 || kw == 2 || kw == 4 || kw == 8), "drhip_conv3x3_direct_mfma_f32: unknown variant %#x", variant);
-    const int OB = wide ? 64 : 32;
-    const int nPT = ceil_div(Wo * Ho, 32);
+    if (variant == 0) variant = sums ? direct_pick32(Wo, Ho, I, O) : drhip_conv3x3_direct_pick_variant(Wo, Ho, I, O);     // (sums: tiles of 32 pixels)
+    const int kw = variant & 0xf, wide = (variant & 0x10) != 0, small = (variant & 0x20) != 0;
+    DRHIP_REQUIRE((variant >> 6) == 0 && (kw == 1 || kw == 2 || kw == 4 || kw == 8), "drhip_conv3x3_direct_mfma_f32: unknown variant %#x", variant);
+    const int OB = (wide ? 64 : 32) >> small;
+    const int nPT = ceil_div(Wo * Ho, small ? 16 : 32);
     DRHIP_REQUIRE(ceil_div(O, OB) <= 65535, "drhip_conv3x3_direct_mfma_f32: too many output channels (%d)", O);
     const dim3 grid(nPT, ceil_div(O, OB)), block(64 * kw);
-    const size_t ldsBytes = (size_t)kw * OB * kDmPartPitch * sizeof(float);
+    const size_t ldsBytes = (size_t)kw * OB * (small ? 17 : kDmPartPitch) * sizeof(float);
     hipStream_t s = as_stream(stream);
     const FastDiv dWo = make_fastdiv(Wo);
-#define DRHIP_DM(NTV, SV) launch((conv3x3_direct_mfma_kernel<NTV, SV>), grid, block, ldsBytes, s, in, F, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dWo.mul, dWo.shift | (relu ? 32u : 0u) | (sums ? 64u : 0u) | (unsigned)kw << 8)
+#define DRHIP_DM(NTV, SV) launch((small ? conv3x3_direct_mfma16_kernel<NTV, SV> : conv3x3_direct_mfma_kernel<NTV, SV>), grid, block, ldsBytes, s, in, F, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dWo.mul, dWo.shift | (relu ? 32u : 0u) | (sums ? 64u : 0u) | (unsigned)kw << 8)
     if (wide) { if (stride == 1) DRHIP_DM(2, 1); else DRHIP_DM(2, 2); }
     else { if (stride == 1) DRHIP_DM(1, 1); else DRHIP_DM(1, 2); }
 #undef DRHIP_DM

@@ -107,9 +107,9 @@ gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
                               (c->stride.s1 == 1 || c->stride.s1 == 2) && !(valu && strcmp(valu, "1") == 0);
             c->variant = c->drDirectBank ? drhip_conv3x3_direct_pick_variant(W / c->stride.s1, H / c->stride.s2, I, O) : 0;
             // At stride 2 that kernel is the faster one where eight of its waves share the channels, which is where it has less than a
-            // workgroup per CU; elsewhere the split bank is: 300x200 48->96 17.7 us against 26.6, 96x96 36->48 5.8 / 7.8, 224x224 64->128
-            // 19.7 / 32.3, 30x30 24->32 4.9 / 10.6, 56x56 128->512 13.7 / 14.6; with eight waves 56x56 96->128 7.9 / 6.9, 28x28 512->512 30.2 / 21.7,
-            // 48x48 72->96 6.7 / 6.6, 20x20 64->64 5.9 / 5.6.
+            // workgroup of 32 pixels and channels per CU; elsewhere the split bank is: 300x200 48->96 17.7 us against 26.6, 96x96 36->48 5.8 / 7.8,
+            // 224x224 64->128 19.7 / 32.3, 30x30 24->32 4.9 / 10.6, 56x56 128->512 13.7 / 14.6; with eight waves 56x56 96->128 7.7 / 6.1, 28x28
+            // 512->512 30.3 / 18.6, 48x48 72->96 6.9 / 4.2, 20x20 64->64 5.9 / 3.8.
             const int bank = drhip_conv_bank_pick_variant(W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 0);
             if (c->drDirectBank && c->stride.s1 == 2 && (c->variant & 15) != 8 && bank) c->drDirectBank = FALSE;
             // Other filters and strides: the split filter bank.  (3x3 filters over an image have kernels of their own, one of
@@ -370,7 +370,7 @@ gboolean conv_cleanup_layer(dR_Graph*, dR_Node* node) {
 
 int dr::avgpool_slices(const dR_Conv2d_Data* c) {
     const int P = (c->ishape.s0 / c->stride.s1) * (c->ishape.s1 / c->stride.s2);
-    if (c->drDirectBank) return (P + 31) / 32;
+    if (c->drDirectBank) return (c->variant & 0x20) ? (P + 15) / 16 : (P + 31) / 32;
     return c->drByPixel ? (P + drhip_conv1x1_pixels_tile(P) - 1) / drhip_conv1x1_pixels_tile(P) : drhip_conv1x1_poolsum_slices(P);
 }
 

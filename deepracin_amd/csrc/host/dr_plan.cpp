@@ -466,7 +466,10 @@ gboolean dR_planBuffers(dR_Graph* net) {
                 dR_Node* consumer = nodes_of(n->next_layers)[0];
                 if (consumer->type == tFullyConnected) ((dR_FC_Data*)consumer->layer)->drDeferredInput = n;
                 else ((dR_Softmax_Data*)consumer->layer)->drDeferredInput = n;
-                ((dR_Conv2d_Data*)c->layer)->drFusedAvgPool = TRUE;
+                dR_Conv2d_Data* cd = (dR_Conv2d_Data*)c->layer;
+                cd->drFusedAvgPool = TRUE;
+                // (at most 64 tiles for the reader to add up: of 32 pixels in larger maps)
+                if (cd->drDirectBank && (cd->variant & 0x20) && c->oshape.s0 * c->oshape.s1 > 64 * 16) cd->variant = 8;
                 ((dR_Pooling_Data*)n->layer)->drFused = TRUE;
             }
         }

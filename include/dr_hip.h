@@ -156,7 +156,8 @@ int drhip_conv2d_direct_f32(const float* in, const float* w, const float* bias, 
  * channels to a multiple of 32, and channel c%8 stored at position (c&1)*4 + (c%8)/2 of its group of 8;
  * drhip_conv3x3_direct_filter_floats(I,O) floats.  `variant` (0 = let the launcher pick) = waves per
  * workgroup (1, 2, 4, 8: they deal the 8-channel stages round-robin, partial tiles added in wave
- * order) | 0x10 for 64 instead of 32 output channels per workgroup.  Same function as
+ * order) | 0x10 for 64 instead of 32 output channels per workgroup, of 32 pixels, or | 0x20 for 16 (with 0x10: 32)
+ * output channels of 16 pixels.  Same function as
  * drhip_conv2d_direct_f32 with kw = kh = 3.  Replaces the per-layer generated kernel
  * `conv2d3x3x<O>_<id>_...` and its launch (src/dR_nodes_conv2d.c:364-420, 481-773); the reference
  * re-lays nothing (it reads [I][O][3][3] through __constant or global memory).
@@ -166,8 +167,8 @@ int drhip_conv3x3_direct_filter_layout_f32(const float* w /* [I][O][3][3] */, fl
 int drhip_conv3x3_direct_pick_variant(int Wo, int Ho, int I, int O);
 int drhip_conv3x3_direct_mfma_f32(const float* in, const float* F, const float* bias, float* out,
                                   int W, int H, int I, int O, int stride, int relu, int variant, void* stream);
-/* With a global average behind it: partials[t*O + o] = sum over the pixels of tile t (32 pixels each, ceil(Wo*Ho/32) tiles), for a
- * drhip_deferred_vec as drhip_conv1x1_poolsum_f32's. */
+/* With a global average behind it: partials[t*O + o] = sum over the pixels of tile t (32 pixels each, ceil(Wo*Ho/32) tiles; 16 pixels
+ * each if `variant` says 0x20, never with variant 0), for a drhip_deferred_vec as drhip_conv1x1_poolsum_f32's. */
 int drhip_conv3x3_direct_poolsum_f32(const float* in, const float* F, const float* bias, float* partials,
                                      int W, int H, int I, int O, int stride, int relu, int variant, void* stream);
 

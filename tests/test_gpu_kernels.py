@@ -92,6 +92,31 @@ def test_conv3x3_direct_mfma(lib, dev, oracle, variant, W, H, I, O, s):
         assert lib.drhip_conv3x3_direct_mfma_f32(xd, F, None, out, W, H, I, O, s, 0, 3, None) == -1      # 3 waves
 
 
+@pytest.mark.parametrize("variant", [0x21, 0x22, 0x24, 0x28, 0x31, 0x34, 0x38])
+@pytest.mark.parametrize("W,H,I,O,s", [
+    (28, 28, 128, 192, 2), (31, 33, 72, 97, 2), (1, 1, 5, 1, 1), (2, 3, 33, 65, 2), (17, 1, 6, 16, 1), (3, 11, 130, 31, 1), (9, 7, 24, 33, 2), (16, 2, 8, 15, 1)])
+def test_conv3x3_direct_tiles_of_16(lib, dev, oracle, variant, W, H, I, O, s):
+    """Tiles of 16 pixels: ragged pixels, channels and stages, and the sums for a global average (the same outputs added up tile by
+    tile: 16 of them in fp32, so 16 * 2^-24 of the sum of their magnitudes)."""
+    x, w, b = own(I, H, W), own(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I))), own(O, scale=0.01)
+    F = dev.empty(lib.drhip_conv3x3_direct_filter_floats(I, O))
+    ok(lib, lib.drhip_conv3x3_direct_filter_layout_f32(dev.put(w), F, I, O, None))
+    xd, bd = dev.put(x), dev.put(b)
+    for relu, bias in ((1, bd), (0, None)):
+        want = oracle.conv_direct(x, w, b if bias else None, (s, s), relu=bool(relu))
+        out = dev.empty(want.size)
+        ok(lib, lib.drhip_conv3x3_direct_mfma_f32(xd, F, bias, out, W, H, I, O, s, relu, variant, None))
+        got = dev.get(out, want.shape)
+        assert_close(got, want, terms=9 * I)
+        assert_close(got, oracle.conv_f64(x, w, b if bias else None, stride=(s, s), relu=bool(relu)), terms=9 * I)
+        flat = got.reshape(O, -1).astype(np.float64)
+        tiles = -(-flat.shape[1] // 16)
+        flat = np.pad(flat, ((0, 0), (0, 16 * tiles - flat.shape[1]))).reshape(O, tiles, 16)
+        parts = dev.empty(tiles * O)
+        ok(lib, lib.drhip_conv3x3_direct_poolsum_f32(xd, F, bias, parts, W, H, I, O, s, relu, variant, None))
+        assert np.all(np.abs(dev.get(parts, (tiles, O)) - flat.sum(2).T) <= 16 * 2.0 ** -24 * np.abs(flat).sum(2).T)
+
+
 @pytest.mark.parametrize("variant", [0, 0x100, 0x101, 0x110, 0x111, 0x120, 0x121])
 @pytest.mark.parametrize("W,H,I,O,kw,kh,sx,sy", [
     (56, 56, 64, 96, 5, 5, 1, 1), (224, 224, 3, 64, 7, 7, 2, 2), (28, 28, 1, 16, 5, 5, 1, 1), (14, 14, 16, 32, 5, 5, 1, 1),

@@ -811,3 +811,10 @@ def test_filter_loads_end_with_the_bank(tmp_path, source, kernels):
             assert int(m[2] or 0) < 1024, (name, line)
     wide = [n for n in places if re.search(r"direct_mfma_kernelILi2|f23_mfma_kernelILi[24]|f23_mfma16_kernelILi4", n)]
     assert len(wide) == kernels and all(len(places[n]) >= 2 for n in wide), (wide, places)
+
+
+def test_direct_variant_of_small_maps():
+    """Which direct 3x3 layers get tiles of 16 pixels: those that make no more workgroups than CUs (256) with 16 or 32 channels each."""
+    pick = dr.load_library().drhip_conv3x3_direct_pick_variant
+    assert [pick(14, 14, 128, 192), pick(28, 28, 96, 128), pick(64, 64, 64, 16), pick(64, 62, 64, 17), pick(14, 14, 32, 16)] == [0x28, 0x38, 0x28, 0x38, 0x24]
+    assert pick(62, 64, 64, 33) == 8 and pick(28, 28, 128, 288) == 8 and pick(56, 56, 256, 256) & 0x20 == 0
