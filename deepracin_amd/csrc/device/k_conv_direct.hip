@@ -165,148 +165,167 @@ conv_direct_fewc_kernel(const float* __restrict__ in, const float* __restrict__ 
 
 // First layer and the 3x3 / stride-2 max pooling behind it in one kernel, on the matrix cores.
 //
-// A workgroup owns a 4x4 tile of POOLED pixels x 16*MB channels.  The pooling windows of that tile
-// cover 9x9 convolution outputs (81, dealt to six wavefronts as six 16-pixel MFMA columns); each
-// wavefront computes its 16 pixels for all channels as a small GEMM over k = (channel, tap), 9*I <= 36
-// values = up to 9 k-steps of v_mfma_f32_16x16x4_f32 (B: gathered input samples, zero padding by
-// select; A: the filters [I][O][9] as they are), adds bias, applies ReLU, and parks the pixels in
-// LDS; then all lanes pool out of LDS in the pooling kernel's scan order.  Convolution outputs
-// outside the map count as 0.0, exactly what the pooling kernel reads there.  The full-resolution
-// tensor (3.2 MB for SqueezeNet's conv1) is never written; the halo costs (9/8)^2 = 1.27x the MFMAs.
-constexpr int kFpPool = 4;                          // pooled tile edge
-constexpr int kFpConv = 2 * kFpPool + 1;            // convolution tile edge
-constexpr int kFpPix = kFpConv * kFpConv;           // 81
-constexpr int kFpWaves = (kFpPix + 15) / 16;        // 6
-constexpr int kFpThreads = 64 * kFpWaves;
-constexpr int kFpPitch = 16 * kFpWaves + 1;         // LDS row pitch (floats)
+// A workgroup owns 4x3 POOLED pixels x 16*MB channels.  The pooling windows of that tile cover 9x7 convolution outputs (63,
+// dealt to four wavefronts, one per SIMD, as 16-pixel MFMA columns); each wavefront computes its 16 pixels for all channels as
+// a small GEMM on v_mfma_f32_16x16x4_f32 whose k-steps are the rows of the window, channel by channel: k = the three samples of
+// a row and a zero.  A lane then has one column of its window, the rows are three offsets and the channels scalar ones: next to no
+// index arithmetic, which is what this kernel was bound by (with k = 4 of the 9*I (channel, tap) pairs, seven steps for an RGB image instead of
+// nine, and tiles of 4x4 on six waves it took 1.8 us until the loads were out, now 0.7; SqueezeNet at 224x224 55.5 -> 54.6 us a pass,
+// at 451x299 with its feed and download 145.1 -> 141.6).  What lies beside the image is out of the resource's range and reads zeros.  The filters go through
+// LDS as they are.  Bias, ReLU, and the pixels are parked in LDS, pixel by pixel; then all lanes pool out of LDS in the pooling kernel's
+// scan order, four channels each.  Convolution outputs outside the map count as 0.0, exactly what the pooling kernel reads there.
+// The full-resolution tensor (3.2 MB for SqueezeNet's conv1) is never written; the halo costs 1.31x the MFMAs.
+constexpr int kFpX = 4, kFpY = 3;                   // pooled tile
+constexpr int kFpConvX = 2 * kFpX + 1, kFpConvY = 2 * kFpY + 1;
+constexpr int kFpThreads = 256;
+static_assert(kFpConvX * kFpConvY <= 64, "a wave has 16 pixels");
 typedef float f32x4d __attribute__((ext_vector_type(4)));
+constexpr unsigned kDmBufferFlags = 0x00020000u;    // dword 3 of a gfx9 raw buffer resource (32-bit data format)
+constexpr unsigned kDmOutOfRange = 0x80000000u;     // byte offset no resource of at most 2 GiB contains
 
 // SQUEEZE: a 1x1 layer behind the pooling, for which all its input channels (at most 16*MB) are here: the pooled pixels meet its
 // filters (wn, fragments as the fire modules have them) right away, and its sums are what is stored, [pixel][16*MBn].
-template <int MB, int KS, bool SQUEEZE>             // KS = k-steps = ceil(9*I / 4)
-__global__ void __launch_bounds__(kFpThreads)
+template <int MB, int I, bool SQUEEZE>              // I = input channels
+__global__ void __launch_bounds__(kFpThreads, 2)
 conv3x3_fewc_pool3s2_kernel(const float* __restrict__ in, const float* __restrict__ w, const float* __restrict__ bias,
-                            float* __restrict__ out, unsigned wh, unsigned io, unsigned woho, unsigned cfg, const float* __restrict__ wn) {
-    // (12 dwords of arguments, which arrive in SGPRs with the wave: wh = W | H << 16, io = I | O << 16,
+                            float* __restrict__ out, unsigned wh, unsigned outChannels, unsigned woho, unsigned cfg, const float* __restrict__ wn) {
+    // (12 dwords of arguments, which arrive in SGPRs with the wave: wh = W | H << 16,
     // woho = Wo | Ho << 16, cfg = sx | sy << 4 | relu << 8 | MBn << 9)
-    const int W = (int)(wh & 0xffffu), H = (int)(wh >> 16), I = (int)(io & 0xffffu), O = (int)(io >> 16);
+    constexpr int OBc = 16 * MB, kPitch = OBc + 4;
+    const int W = (int)(wh & 0xffffu), H = (int)(wh >> 16), O = (int)outChannels;
     const int Wo = (int)(woho & 0xffffu), Ho = (int)(woho >> 16), Wp = (Wo + 1) >> 1, Hp = (Ho + 1) >> 1;
     const int sx = (int)(cfg & 15u), sy = (int)((cfg >> 4) & 15u), relu = (int)((cfg >> 8) & 1u);
-    __shared__ float convT[16 * MB * kFpPitch];
-    __shared__ float wT[4 * KS * 16 * MB];          // filters as [k = (channel, tap)][channel out], zero padded
-    __shared__ float biasT[16 * MB];
+    __shared__ __attribute__((aligned(16))) float convT[64 * kPitch];       // [pixel][channel]
+    __shared__ __attribute__((aligned(16))) float wT[I * OBc * 9 + 1];      // the filters, [channel in][channel out][9]; then the pooled pixels
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 15, lk = lane >> 4;
     const int tileX = blockIdx.x, tileY = blockIdx.y;       // (a 3-D grid: no integer division in front of the first loads)
-    const int o0 = blockIdx.z * 16 * MB;
+    const int o0 = blockIdx.z * OBc;
 
-    const int q = 16 * wave + j;                    // convolution pixel within the 9x9 tile
-    const int ry = q / kFpConv, rx = q % kFpConv;
-    const int cy = 2 * kFpPool * tileY + ry, cx = 2 * kFpPool * tileX + rx;
-    const bool pixOk = q < kFpPix && cy < Ho && cx < Wo;
+    const int q = 16 * wave + j;                    // convolution pixel within the 9x7 tile
+    const int ry = q / kFpConvX, rx = q % kFpConvX;
+    const int cy = 2 * kFpY * tileY + ry, cx = 2 * kFpX * tileX + rx;
+    const bool pixOk = q < kFpConvX * kFpConvY && cy < Ho && cx < Wo;
 
-    // B operands: this lane's input samples, gathered now ...
-    float b[KS];
+    // B operands: column lk of this lane's window, row by row (lanes of the fourth column: zeros) ...
+    const int ix = cx * sx + lk - 1, iy0 = cy * sy - 1;
+    const bool columnOk = pixOk && lk < 3 && (unsigned)ix < (unsigned)W;
+    // (each channel's resource: the rows under the tile and no more, whatever the size of the image)
+    const int iyTop = max(2 * kFpY * tileY * sy - 1, 0), rows = min(H - iyTop, kFpConvY * 15 + 3);
+    unsigned row[3];
+    float b[I][3];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const int kidx = 4 * ks + lk;               // (channel, tap)
-        const int c = kidx / 9, tap = kidx % 9;
-        const int iy = cy * sy + tap / 3 - 1, ix = cx * sx + tap % 3 - 1;
-        const bool ok = pixOk && kidx < 9 * I && iy >= 0 && iy < H && ix >= 0 && ix < W;
-        const float v = in[((size_t)min(c, I - 1) * H + min(max(iy, 0), H - 1)) * W + min(max(ix, 0), W - 1)];
-        b[ks] = ok ? v : 0.0f;
-    }
-    // ... while the workgroup's filters go to LDS once, read in their own order (contiguous per
-    // input channel: w[c][o0 ..][9]) and written transposed, so that an MFMA A operand is 16
-    // consecutive floats.
-    constexpr int OBc = 16 * MB;
-    constexpr int kRounds = (4 * KS * OBc + kFpThreads - 1) / kFpThreads;
-    float fv[kRounds];
-    int dst[kRounds];
+    for (int d = 0; d < 3; ++d) row[d] = columnOk && (unsigned)(iy0 + d) < (unsigned)H ? 4u * (unsigned)((iy0 + d - iyTop) * W + ix) : kDmOutOfRange;
 #pragma unroll
-    for (int u = 0; u < kRounds; ++u) {             // all loads first (clamped addresses), one trip to memory
-        const int e = tid + u * kFpThreads;
-        // e -> (c, o local, tap) in memory order for real filter values, the zero padding after them
-        const bool real = e < 9 * I * OBc;
-        const int c = min(e / (9 * OBc), I - 1), rest = e % (9 * OBc);
-        const int ol = real ? rest / 9 : (e - 9 * I * OBc) % OBc;
-        const int kidx = real ? c * 9 + rest % 9 : 9 * I + (e - 9 * I * OBc) / OBc;
-        const float f = w[((size_t)c * O + min(o0 + ol, O - 1)) * 9 + rest % 9];
-        fv[u] = (real && o0 + ol < O) ? f : 0.0f;
-        dst[u] = e < 4 * KS * OBc ? kidx * OBc + ol : -1;
+    for (int c = 0; c < I; ++c) {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(in + ((size_t)c * H + iyTop) * W), 0, rows * W * 4, kDmBufferFlags);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) b[c][d] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)row[d], 0, 0));
     }
-    float bv = 0.0f;                                // the bias comes along in the same trip
-    if (tid < OBc && bias) bv = bias[min(o0 + tid, O - 1)];
+    // ... while the workgroup's filters go to LDS once, in their own order (zeros behind the last output channel)
+    constexpr int kRounds = (OBc * 9 + kFpThreads - 1) / kFpThreads;
+    float fv[I][kRounds];
+#pragma unroll
+    for (int c = 0; c < I; ++c) {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)c * O * 9), 0, O * 36, kDmBufferFlags);
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) fv[c][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (o0 * 9 + u * kFpThreads + tid), 0, 0));
+    }
+    const __amdgpu_buffer_rsrc_t rBias = __builtin_amdgcn_make_buffer_rsrc((void*)bias, 0, bias ? O * 4 : 0, kDmBufferFlags);
+    f32x4d biasE[MB];                               // (four channels a lane, as the sums come)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) biasE[m] = __builtin_bit_cast(f32x4d, __builtin_amdgcn_raw_buffer_load_b128(rBias, 4 * (o0 + 16 * m + 4 * lk), 0, 0));
     f32x4d a2[MB];
     const int MBn = SQUEEZE ? (int)(cfg >> 9) : 0;
     if (SQUEEZE && wave < MBn) {
 #pragma unroll
         for (int c = 0; c < MB; ++c) a2[c] = *(const f32x4d*)(wn + (((wave * MB + c) << 8) + 4 * lane));
     }
+    auto barrier = [] {                             // (LDS only: loads stay under way)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
 #pragma unroll
-    for (int u = 0; u < kRounds; ++u)
-        if (dst[u] >= 0) wT[dst[u]] = fv[u];
-    if (tid < OBc) biasT[tid] = bv;
-    __syncthreads();
-    float a[MB][KS];
+    for (int c = 0; c < I; ++c)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int m = 0; m < MB; ++m) a[m][ks] = wT[(4 * ks + lk) * OBc + 16 * m + j];
+        for (int u = 0; u < kRounds; ++u)
+            if ((u + 1) * kFpThreads <= OBc * 9 || u * kFpThreads + tid < OBc * 9) wT[c * OBc * 9 + u * kFpThreads + tid] = fv[c][u];
+    barrier();
     f32x4d acc[MB];
 #pragma unroll
     for (int m = 0; m < MB; ++m) acc[m] = f32x4d{0.f, 0.f, 0.f, 0.f};
+    // (all of them on their way before the first is waited for; the zero's filter is replaced by a zero, for it may not be finite)
+    const float* mine = wT + 9 * j + min(lk, 2);
+    float a[3 * I][MB];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int k = 0; k < 3 * I; ++k)
 #pragma unroll
-        for (int m = 0; m < MB; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][ks], b[ks], acc[m], 0, 0, 0);
+        for (int m = 0; m < MB; ++m) a[k][m] = mine[(k / 3 * OBc + 16 * m) * 9 + 3 * (k % 3)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 3 * I; ++k)
+#pragma unroll
+        for (int m = 0; m < MB; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(lk < 3 ? a[k][m] : 0.0f, b[k / 3][k % 3], acc[m], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
 
     // D: lane -> pixel j, register r -> channel 4*lk + r of block m
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+    for (int m = 0; m < MB; ++m) {
+        f32x4d v = acc[m] + biasE[m];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int ch = 16 * m + 4 * lk + r;
-            float v = acc[m][r] + biasT[ch];
-            if (relu) v = fmaxf(v, 0.0f);
-            convT[ch * kFpPitch + q] = pixOk ? v : 0.0f;
+            if (relu) v[r] = fmaxf(v[r], 0.0f);
+            v[r] = pixOk ? v[r] : 0.0f;
         }
-    __syncthreads();
+        *(f32x4d*)(convT + q * kPitch + 16 * m + 4 * lk) = v;
+    }
+    barrier();
 
-    constexpr int kPooledPitch = 16 * MB + 4;       // (in front of it lie the filters, which are in registers by now)
-    static_assert(!SQUEEZE || 16 * kPooledPitch <= 4 * KS * 16 * MB, "pooled pixels take the place of the filters");
-    for (int idx = tid; idx < 16 * MB * kFpPool * kFpPool; idx += kFpThreads) {
-        const int ch = idx / (kFpPool * kFpPool), pp = idx % (kFpPool * kFpPool);
-        const int ppy = pp / kFpPool, ppx = pp % kFpPool;
-        const int py = kFpPool * tileY + ppy, px = kFpPool * tileX + ppx;
-        if (SQUEEZE || (py < Hp && px < Wp && o0 + ch < O)) {
-            float r = -FLT_MAX;
+    // (where the filters were, which nobody needs any more, lie the pooled pixels, in front of the squeeze layer)
+    constexpr int kPooled = kFpX * kFpY;
+    static_assert(!SQUEEZE || 16 * kPitch <= I * OBc * 9, "pooled pixels take the place of the filters");
+    for (int idx = tid; idx < 4 * MB * (SQUEEZE ? 16 : kPooled); idx += kFpThreads) {
+        const int pp = SQUEEZE ? idx / (4 * MB) : idx % kPooled, ch = 4 * (SQUEEZE ? idx % (4 * MB) : idx / kPooled);
+        const int ppy = pp / kFpX, ppx = pp % kFpX;
+        const int py = kFpY * tileY + ppy, px = kFpX * tileX + ppx;
+        f32x4d r = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
+        const float* at = convT + ((2 * ppy) * kFpConvX + 2 * ppx) * kPitch + ch;
+        if (pp < kPooled) {
 #pragma unroll
             for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
                 for (int dx = 0; dx < 3; ++dx) {
-                    const float v = convT[ch * kFpPitch + (2 * ppy + dy) * kFpConv + 2 * ppx + dx];
-                    if (v > r) r = v;
+                    const f32x4d v = *(const f32x4d*)(at + (dy * kFpConvX + dx) * kPitch);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) r[k] = v[k] > r[k] ? v[k] : r[k];
                 }
-            if constexpr (SQUEEZE) wT[pp * kPooledPitch + ch] = ch < O ? r : 0.0f;
-            else store_through(out + ((size_t)(o0 + ch) * Hp + py) * Wp + px, r);
+        }
+        if constexpr (SQUEEZE) {                    // (columns without a pixel, channels that do not exist: zeros)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) r[k] = pp < kPooled && ch + k < O ? r[k] : 0.0f;
+            *(f32x4d*)(wT + pp * kPitch + ch) = r;
+        } else if (py < Hp && px < Wp) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (o0 + ch + k < O) store_through(out + ((size_t)(o0 + ch + k) * Hp + py) * Wp + px, r[k]);
         }
     }
     if constexpr (SQUEEZE) {
-        __syncthreads();
+        barrier();
         if (wave >= MBn) return;
         f32x4d sums = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < MB; ++c) {
-            const f32x4d v = *(const f32x4d*)(wT + j * kPooledPitch + 16 * c + 4 * lk);
+            const f32x4d v = *(const f32x4d*)(wT + j * kPitch + 16 * c + 4 * lk);
 #pragma unroll
             for (int k = 0; k < 4; ++k) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[c][k], v[k], sums, 0, 0, 0);
         }
-        const int py = kFpPool * tileY + j / kFpPool, px = kFpPool * tileX + j % kFpPool;
+        const int py = kFpY * tileY + j / kFpX, px = kFpX * tileX + j % kFpX;
         const __amdgpu_buffer_rsrc_t rOut = __builtin_amdgcn_make_buffer_rsrc((void*)out, 0, 0x7ffffff0, kBufferFlags);
         typedef unsigned u32x4d __attribute__((ext_vector_type(4)));
-        if (py < Hp && px < Wp)                     // (sc0 sc1: written through)
+        if (j < kPooled && py < Hp && px < Wp)      // (sc0 sc1: written through)
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4d, sums), rOut, 4 * ((py * Wp + px) * 16 * MBn + 16 * wave + 4 * lk), 0, 1 | 16);
     }
 }
@@ -408,9 +427,6 @@ conv3x3_fewc_mfma_kernel(const float* __restrict__ in, const float* __restrict__
 //     then bias, ReLU and 128-byte row stores.
 // Per stage and wave: 12 + 9*NT loads and ~50 VALU instructions (the selects) for 36*NT MFMAs.
 typedef float f32x16d __attribute__((ext_vector_type(16)));
-typedef float f32x4d __attribute__((ext_vector_type(4)));
-constexpr unsigned kDmBufferFlags = 0x00020000u;    // dword 3 of a gfx9 raw buffer resource (32-bit data format)
-constexpr unsigned kDmOutOfRange = 0x80000000u;     // byte offset no resource of at most 2 GiB contains
 constexpr int kDmKC = 8;                            // input channels per stage (4 MFMA k-steps)
 constexpr int kDmPartPitch = 33;
 
@@ -817,17 +833,16 @@ static int conv3x3_pool3s2(const float* in, const float* w, const float* bias, c
     DRHIP_REQUIRE((long long)W * H * I < (1ll << 31) && (long long)W * H * O < (1ll << 31), "drhip_conv3x3_pool3s2_f32: tensor too large");
     DRHIP_REQUIRE(W <= 65535 && H <= 65535 && O <= 65535 && strideX <= 15 && strideY <= 15, "drhip_conv3x3_pool3s2_f32: W, H and O are limited to 65535, strides to 15");
     const int Wo = W / strideX, Ho = H / strideY, Wp = ceil_div(Wo, 2), Hp = ceil_div(Ho, 2);
-    const int tilesX = ceil_div(Wp, kFpPool), tilesY = ceil_div(Hp, kFpPool);
+    const int tilesX = ceil_div(Wp, kFpX), tilesY = ceil_div(Hp, kFpY);
     hipStream_t s = as_stream(stream);
-    const int ks = ceil_div(9 * I, 4);              // 3, 5, 7 or 9
     const bool wide = O > 32;                       // 64 channels per workgroup, else 32
     DRHIP_REQUIRE(tilesY <= 65535 && O <= 32 * 65535, "drhip_conv3x3_pool3s2_f32: tensor exceeds the launch grid");
     const dim3 grid(tilesX, tilesY, ceil_div(O, wide ? 64 : 32)), block(kFpThreads);
-#define DRHIP_FPS(MBV, KSV, SQ) launch((conv3x3_fewc_pool3s2_kernel<MBV, KSV, SQ>), grid, block, 0, s, in, w, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, (unsigned)Wo | (unsigned)Ho << 16, (unsigned)strideX | (unsigned)strideY << 4 | (relu ? 256u : 0u) | (unsigned)ceil_div(Sn, 16) << 9, wn)
-#define DRHIP_FP(MBV, KSV) do { if (wn) DRHIP_FPS(MBV, KSV, true); else DRHIP_FPS(MBV, KSV, false); } while (0)
-#define DRHIP_FP_K(MBV) do { if (ks == 3) DRHIP_FPS(MBV, 3, false); else if (ks == 5) DRHIP_FP(MBV, 5); else if (ks == 7) DRHIP_FP(MBV, 7); else DRHIP_FP(MBV, 9); } while (0)
-    if (wide) DRHIP_FP_K(4); else DRHIP_FP_K(2);
-#undef DRHIP_FP_K
+#define DRHIP_FPS(MBV, IV, SQ) launch((conv3x3_fewc_pool3s2_kernel<MBV, IV, SQ>), grid, block, 0, s, in, w, bias, out, (unsigned)W | (unsigned)H << 16, (unsigned)O, (unsigned)Wo | (unsigned)Ho << 16, (unsigned)strideX | (unsigned)strideY << 4 | (relu ? 256u : 0u) | (unsigned)ceil_div(Sn, 16) << 9, wn)
+#define DRHIP_FP(MBV, IV) do { if (wn) DRHIP_FPS(MBV, IV, true); else DRHIP_FPS(MBV, IV, false); } while (0)
+#define DRHIP_FP_I(MBV) do { if (I == 1) DRHIP_FPS(MBV, 1, false); else if (I == 2) DRHIP_FP(MBV, 2); else if (I == 3) DRHIP_FP(MBV, 3); else DRHIP_FP(MBV, 4); } while (0)
+    if (wide) DRHIP_FP_I(4); else DRHIP_FP_I(2);
+#undef DRHIP_FP_I
 #undef DRHIP_FP
 #undef DRHIP_FPS
     return launched("conv3x3_fewc_pool3s2_kernel");

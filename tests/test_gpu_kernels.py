@@ -189,6 +189,25 @@ def test_first_layer_conv_with_maxpool(lib, dev, oracle, W, H, I, O, sx, sy, rel
     assert lib.drhip_conv3x3_pool3s2_f32(dev.put(x), dev.put(w), None, out, W, H, 5, O, sx, sy, relu, None) == -1
 
 
+@pytest.mark.parametrize("I", [1, 2, 3, 4])
+@pytest.mark.parametrize("W,H,O,sx,sy", [(7, 5, 31, 1, 1), (8, 6, 32, 1, 1), (9, 7, 33, 1, 1), (17, 13, 64, 1, 1), (1, 40, 65, 1, 2), (200, 31, 5, 15, 15), (31, 200, 48, 14, 15)])
+def test_first_layer_with_maxpool_tiles(lib, dev, oracle, I, W, H, O, sx, sy):
+    """Around its tiles of 4x3 pooled pixels and blocks of 32 and 64 channels, with the longest strides; and an infinite weight, which
+    spoils the outputs that its tap reaches and no others."""
+    x, w, b = own(I, H, W), own(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I))), own(O, scale=0.05)
+    conv = oracle.conv_direct(x, w, b, (sx, sy), relu=True)
+    want = oracle.pool(conv, (3, 3, 1), (2, 2, 1), 0)
+    out, xd, bd = dev.empty(want.size), dev.put(x), dev.put(b)
+    ok(lib, lib.drhip_conv3x3_pool3s2_f32(xd, dev.put(w), bd, out, W, H, I, O, sx, sy, 1, None))
+    got = dev.get(out, want.shape)
+    assert_close(got, want, terms=9 * I)
+    w[I - 1, O - 1, 1, 1] = np.inf                  # (the middle one: never beside the map)
+    ok(lib, lib.drhip_conv3x3_pool3s2_f32(xd, dev.put(w), bd, out, W, H, I, O, sx, sy, 1, None))
+    spoilt = dev.get(out, want.shape)
+    positive = oracle.pool((x[I - 1:, ::sy, ::sx][:, :conv.shape[1], :conv.shape[2]] > 0).astype(np.float32), (3, 3, 1), (2, 2, 1), 0)[0]
+    assert np.array_equal(spoilt[:-1], got[:-1]) and np.array_equal(spoilt[-1], np.where(positive > 0, np.float32(np.inf), np.float32(0)))
+
+
 def test_conv_direct_valu_kernels(lib, dev, oracle):
     """DR_DIRECT_VALU=1: the LDS-tiled / first-layer VALU kernels behind the matrix-core forms."""
     import os
