@@ -427,7 +427,8 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
 
 // The tile that finishes first, by a count of what the busiest CU does, in clocks: per workgroup a fixed 1500 for the store, per stage 1200
 // for the trip to memory and 1200 per round of staging (the address unit takes one dword gather every 8 to 16 clocks), and the MFMAs of
-// one of its four SIMDs at 42 clocks or, if that is more, the filters at 42 bytes a clock.  Pixel tiles wider than the map or
+// one of its four SIMDs at 42 clocks or, if that is more, the filters at 42 bytes a clock, and 2 clocks for every row of outputs of
+// a channel in a block, a piece of a line each (8 or 16 columns: 384x384 3->96 7x7/2 22.4 / 20.8 us, 224x224 3->64 7x7/2 6.2 / 5.9).  Pixel tiles wider than the map or
 // hanging over its edge count in full, which picks the tile shape as well.  Measured, us per layer, this choice / the
 // other tiles: 56x56 64->96 5x5 11.4 / 11.5 to 25, 224x224 3->64 7x7/2 6.1 / 7.7 to 13.7, 96x70 50->75 5x5 17.7 / 19.5 to 25, 28x28 128->128 5x5
 // 11.7 / 16 to 47, 112x112 64->128 3x3/2 9.2 / 10.1 to 15.5, 14x14 16->32 5x5 4.3 / 5 to 9.
@@ -450,7 +451,8 @@ static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy
                 const double waveSteps = (s.nStages - 1.0) * ceil_div(s.group * s.steps, wk) + ceil_div((s.nChunks - (s.nStages - 1) * s.group) * s.steps, wk);
                 const double staging = s.nStages * 1200.0 * (1 + ceil_div(s.patchN * (p.cp == 16 ? 2 : 1) * s.group, kBankThreads));
                 const double work = std::max(1.3 * waveSteps * 2 * 6 * 32 * mt, (double)s.nChunks * s.steps * wo * 3072 / 42);
-                const double cost = 6000 + std::ceil(wgs / num_cu()) * (1500 + staging + work);
+                const double rows = pool ? 0.0 : 2.0 * 32 * wo * mt * (32 >> lgBW);
+                const double cost = 6000 + std::ceil(wgs / num_cu()) * (1500 + staging + work + rows);
                 if (!found || cost < bestCost) { found = true; bestCost = cost; *best = p; }
             }
         }
