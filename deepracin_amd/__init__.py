@@ -176,6 +176,8 @@ def load_library(path=None):
         "drhip_conv_bank_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 10 + [vp]),
         "drhip_conv_bank_pick_variant": (c_int, [c_int] * 9),
         "drhip_conv_bank_maxpool2_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 10 + [vp]),
+        "drhip_conv_bank_maxpool3s2_pick_variant": (c_int, [c_int] * 9),
+        "drhip_conv_bank_maxpool3s2_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 10 + [vp]),
         "drhip_conv3x3_pool3s2_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 7 + [vp]),
         "drhip_conv1x1_poolsum_f32": (c_int, [vp, vp, vp, vp, c_int, c_int, c_int, c_int, vp]),
         "drhip_conv1x1_poolsum_slices": (c_int, [c_int]),

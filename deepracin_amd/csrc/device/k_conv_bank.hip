@@ -19,6 +19,8 @@
 //     few tiles fill the chip that way without a second kernel.
 //   * A 2x2/2 max pooling behind the layer is taken from these sums: a pooled pixel a lane.  (28x28 with 5x5 filters and poolings, 16
 //     and 32 channels, its image from the host and its results back: 36.4 -> 32.2 us, two launches less.)
+//   * So is a 3x3/2 max pooling (P3): the pixels of a workgroup are then the 9x7 or 9x9 under 4x3 or 4x4 pooled ones, so that
+//     1.3 times the products are done, and one launch less and a quarter of the outputs stored.  (Figures stand at the choice of the variant.)
 //   * Outputs that do not come out finite are worked out again in fp32, at the end.
 // Layers with at most four input channels (images) put four neighbouring pixels x four channels into one step of 16 k
 // (CP = 4) instead of 16 channels of one pixel, most of which would be zero: a 7x7 filter over RGB is 14 steps, not 49.
@@ -31,17 +33,20 @@
 namespace drhip {
 
 constexpr int kBankThreads = 512;                       // eight waves: two per SIMD, one reads and counts while the other multiplies
+// P3: 4 x 3 (two blocks) or 4 x 4 (three) pooled pixels of a workgroup, 9 columns of pixels under them, and what lgBW says then
+constexpr int kP3X = 4, kP3W = 2 * kP3X + 1, kP3Tile = 6;
+constexpr int p3_rows(int mt) { return mt + 1; }
 
 struct BankShape {                                      // everything but the pointers; by value to the kernel
     int W, H, I, O, Wo, Ho;
     int kw, sx, sy, padX, padY;
-    int lgBW;                                           // 32 pixels of one MFMA = 2^lgBW columns x the rest rows
+    int lgBW;                                           // 32 pixels of one MFMA = 2^lgBW columns x the rest rows (kP3Tile: see there)
     int pw, patchN;                                     // patch width, patch pixels
     int spr, steps, nChunks, oBlocks;                   // k-steps per filter row, per chunk; chunks; 32-channel blocks in the bank
     int group, nStages;                                 // chunks that are staged together; stages
     unsigned pwMul, pwShift, patchMul, patchShift;      // division by pw and patchN
     unsigned sprMul, stepsMul;                          // j = tap * sprMul >> 16, chunk of a stage = step * stepsMul >> 16
-    int relu, pool;                                     // pool: a 2x2/2 max pooling stands behind the layer, `out` is its tensor
+    int relu, pool;                                     // pool: a 2x2/2 (with P3: 3x3/2) max pooling stands behind the layer, `out` is its tensor
 };
 
 __device__ inline u32x4b bank_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, unsigned soffset) {
@@ -71,12 +76,14 @@ conv_bank_layout_kernel(const float* __restrict__ w, unsigned short* __restrict_
 }
 
 // PF: staging rounds (512 units each) of the next stage that are kept in registers.
-template <int CP, int MT, int WO, int WK, int PF>
+template <int CP, int MT, int WO, int WK, int PF, bool P3>
 __global__ void __launch_bounds__(kBankThreads)
 conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __restrict__ F, const float* __restrict__ bias,
                       float* __restrict__ out, BankShape s) {
     static_assert(WO * WK * 64 == kBankThreads, "eight waves");
     static_assert(CP == 4 || CP == 16, "channels of one pixel in a k-step");
+    constexpr int kP3Y = p3_rows(MT), kP3H = 2 * kP3Y + 1;
+    static_assert(!P3 || (MT >= 2 && kP3W * kP3H <= 32 * MT), "the pixels under a tile of pooled ones");
     constexpr int kGroups = CP == 16 ? 2 : 1;           // staging units per pixel, 8 (4) channels each
     constexpr int kUnitBytes = CP == 16 ? 16 : 8;
     __shared__ float biasT[32 * WO];                    // (a load in the epilogue would wait for the stores in front of it)
@@ -88,7 +95,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     const int wo = wave % WO, wk = wave / WO;
     const int l32 = lane & 31, half = lane >> 5;
     const int BW = 1 << s.lgBW, BH = 32 >> s.lgBW;
-    const int x0 = blockIdx.x << s.lgBW, y0 = blockIdx.y * (BH * MT);
+    const int x0 = P3 ? blockIdx.x * (2 * kP3X) : blockIdx.x << s.lgBW, y0 = blockIdx.y * (P3 ? 2 * kP3Y : BH * MT);
     const int ob = blockIdx.z * WO + wo;                // this wave's 32 output channels
     const int bx = l32 & (BW - 1), by = l32 >> s.lgBW;
     const int plane = s.H * s.W;
@@ -181,7 +188,8 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     int bBase[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int q = (by + BH * m) * s.sy * s.pw + bx * s.sx;
+        const int p3 = min(32 * m + l32, kP3W * kP3H - 1);
+        const int q = P3 ? (p3 / kP3W) * s.sy * s.pw + (p3 % kP3W) * s.sx : (by + BH * m) * s.sy * s.pw + bx * s.sx;
         bBase[m] = CP == 16 ? (half * s.patchN + q) * 16 : q * 8 + half * 16;
     }
 
@@ -256,6 +264,11 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     }
     constexpr int kPitch = 33;
     float* part = (float*)lds;                          // [WK][32*WO channels][MT][33]
+    auto barrier = [] {                                 // (LDS only)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
     __syncthreads();                                    // the patch has been read for the last time
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -268,6 +281,94 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         v = fmaf(v, scale, b);
         return s.relu ? fmaxf(v, 0.0f) : v;
     };
+    // The sum at pixel (x, y) of the map for channel oc of the workgroup: CH channels side by side, 64 / CH lanes for each.
+    auto once_more = [&](auto channels, int x, int y, int oc) {
+        constexpr int CH = decltype(channels)::value;
+        const int o = blockIdx.z * (32 * WO) + oc;
+        const unsigned fAgain = (unsigned)(min(o >> 5, s.oBlocks - 1) * 1024 + (o & 31) * 16);
+        const int left = x * s.sx - s.padX, top = y * s.sy - s.padY, kh = s.steps / s.spr;
+        for (int j = 0; j < kh; ++j) {
+            const float* row = in + (size_t)min(max(top + j, 0), s.H - 1) * s.W;        // (a row beside the map stands for one that is in the window)
+            bool nan = false;
+            for (int c = lane; c < s.I; c += 64)
+                for (int i = 0; i < s.kw; ++i) {
+                    const float v = row[(size_t)c * plane + min(max(left + i, 0), s.W - 1)];
+                    nan = nan || v != v;
+                }
+            if (__builtin_amdgcn_ballot_w64(nan) != 0) return __builtin_nanf("");
+        }
+        float v = 0.0f;
+        for (int chunk = 0; chunk < s.nChunks; ++chunk)
+            for (int u = lane / CH; u < 2 * s.steps; u += 64 / CH) {            // half a k-step: eight values of k
+                const int step = u >> 1, h = u & 1, j = (int)(((unsigned)step * s.sprMul) >> 16), i0 = step - j * s.spr;
+                const unsigned f = fAgain + (unsigned)((chunk * s.steps + step) * 3 * s.oBlocks * 1024 + 512 * h), partF = (unsigned)s.oBlocks * 1024u;
+                const u32x4b hi = bank_load4(rF, f, 0), mid = bank_load4(rF, f + partF, 0), lo = bank_load4(rF, f + 2 * partF, 0);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int c = CP == 16 ? 16 * chunk + 8 * h + e : e & 3, i = CP == 16 ? i0 : 4 * i0 + 2 * h + (e >> 2);
+                    const int ix = left + i, iy = top + j;
+                    const bool ok = c < s.I && i < s.kw && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
+                    const float sample = in[ok ? (size_t)c * plane + iy * s.W + ix : 0];
+                    auto of = [&](u32x4b q) { return e & 1 ? q[e / 2] >> 16 : q[e / 2] & 0xffffu; };
+                    v = ok ? fmaf(whole(of(hi), of(mid), of(lo)), sample, v) : v;
+                }
+            }
+#pragma unroll
+        for (int k = CH; k < 64; k *= 2) v += __shfl_xor(v, k);
+        return v;
+    };
+    if constexpr (P3) {
+        // Outputs first, each in the place of its first sum, zeros beside the map; then the pooling, by its own kernel's rules.  (A turn is 16
+        // channels of one block: no division.)
+        constexpr int NT = 2 * WO * MT;
+        float* const mine = part + (tid >> 5) * MT * kPitch + l32;
+        auto block_of = [](int n) { return n / (2 * WO); };
+        auto first_of = [](int n) { return 16 * (n % (2 * WO)); };         // channel, less tid / 32
+        float v[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            v[n] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) v[n] += mine[((k * 32 * WO + first_of(n)) * MT + block_of(n)) * kPitch];
+            again |= fabsf(v[n]) < __builtin_inff() ? 0u : 1u << n;
+            v[n] = finish(v[n], kSplitUnscale, biasT[first_of(n) + (tid >> 5)]);
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(again != 0u) != 0, 0)) {       // (as below, output by output)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                for (unsigned long long bad = __builtin_amdgcn_ballot_w64((again >> n & 1u) != 0); bad != 0; bad &= bad - 1) {
+                    const int src = __builtin_ctzll(bad), oc = first_of(n) + ((tid & ~63) + src) / 32, pl = 32 * block_of(n) + (src & 31);
+                    const int x = x0 + pl % kP3W, y = y0 + pl / kP3W;
+                    if (pl >= kP3W * kP3H || x >= s.Wo || y >= s.Ho) continue;
+                    const float once = finish(once_more(std::integral_constant<int, 1>{}, x, y, oc), 1.0f, biasT[oc]);
+                    v[n] = lane == src ? once : v[n];
+                }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int pl = 32 * m + l32;
+            const bool inMap = x0 + pl % kP3W < s.Wo && y0 + pl / kP3W < s.Ho;
+#pragma unroll
+            for (int n = 2 * WO * m; n < 2 * WO * (m + 1); ++n) mine[(first_of(n) * MT + m) * kPitch] = inMap ? v[n] : 0.0f;
+        }
+        barrier();
+        const int Wp = (s.Wo + 1) >> 1, Hp = (s.Ho + 1) >> 1;
+#pragma unroll
+        for (int i0 = 0; i0 < 32 * WO * kP3X * kP3Y; i0 += kBankThreads) {
+            const int i = i0 + tid, oc = i / (kP3X * kP3Y), pp = i % (kP3X * kP3Y), ppy = pp / kP3X, ppx = pp % kP3X;
+            if (32 * WO * kP3X * kP3Y < i0 + kBankThreads && oc >= 32 * WO) break;
+            float best = -FLT_MAX;
+#pragma unroll
+            for (int d = 0; d < 9; ++d) {
+                const int q = (2 * ppy + d / 3) * kP3W + 2 * ppx + d % 3;
+                const float u = part[(oc * MT + (q >> 5)) * kPitch + (q & 31)];
+                best = u > best ? u : best;
+            }
+            const int o = blockIdx.z * (32 * WO) + oc, px = (x0 >> 1) + ppx, py = (y0 >> 1) + ppy;
+            if (o < s.O && px < Wp && py < Hp) store_through(out + ((size_t)o * Hp + py) * Wp + px, best);
+        }
+        return;
+    }
     // Pooled: 512 lanes, 64 (channel, block) pairs of 8 pooled pixels a turn.  The maximum as the pooling's own kernel takes it: in scan
     // order from the lowest number on, what lies beside the map counts as 0.
     constexpr int kPooled = WO * MT / 2 > 0 ? WO * MT / 2 : 1;
@@ -319,43 +420,6 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     const unsigned long long any = __builtin_amdgcn_ballot_w64(again != 0u);
     if (__builtin_expect(any == 0, 1)) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
-    const int kh = s.steps / s.spr;
-    // The sum at pixel (x, y) of the map for channel oc of the workgroup: CH channels side by side, 64 / CH lanes for each.
-    auto once_more = [&](auto channels, int x, int y, int oc) {
-        constexpr int CH = decltype(channels)::value;
-        const int o = blockIdx.z * (32 * WO) + oc;
-        const unsigned fAgain = (unsigned)(min(o >> 5, s.oBlocks - 1) * 1024 + (o & 31) * 16);
-        const int left = x * s.sx - s.padX, top = y * s.sy - s.padY;
-        for (int j = 0; j < kh; ++j) {
-            const float* row = in + (size_t)min(max(top + j, 0), s.H - 1) * s.W;        // (a row beside the map stands for one that is in the window)
-            bool nan = false;
-            for (int c = lane; c < s.I; c += 64)
-                for (int i = 0; i < s.kw; ++i) {
-                    const float v = row[(size_t)c * plane + min(max(left + i, 0), s.W - 1)];
-                    nan = nan || v != v;
-                }
-            if (__builtin_amdgcn_ballot_w64(nan) != 0) return __builtin_nanf("");
-        }
-        float v = 0.0f;
-        for (int chunk = 0; chunk < s.nChunks; ++chunk)
-            for (int u = lane / CH; u < 2 * s.steps; u += 64 / CH) {            // half a k-step: eight values of k
-                const int step = u >> 1, h = u & 1, j = (int)(((unsigned)step * s.sprMul) >> 16), i0 = step - j * s.spr;
-                const unsigned f = fAgain + (unsigned)((chunk * s.steps + step) * 3 * s.oBlocks * 1024 + 512 * h), partF = (unsigned)s.oBlocks * 1024u;
-                const u32x4b hi = bank_load4(rF, f, 0), mid = bank_load4(rF, f + partF, 0), lo = bank_load4(rF, f + 2 * partF, 0);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int c = CP == 16 ? 16 * chunk + 8 * h + e : e & 3, i = CP == 16 ? i0 : 4 * i0 + 2 * h + (e >> 2);
-                    const int ix = left + i, iy = top + j;
-                    const bool ok = c < s.I && i < s.kw && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
-                    const float sample = in[ok ? (size_t)c * plane + iy * s.W + ix : 0];
-                    auto of = [&](u32x4b q) { return e & 1 ? q[e / 2] >> 16 : q[e / 2] & 0xffffu; };
-                    v = ok ? fmaf(whole(of(hi), of(mid), of(lo)), sample, v) : v;
-                }
-            }
-#pragma unroll
-        for (int k = CH; k < 64; k *= 2) v += __shfl_xor(v, k);
-        return v;
-    };
     if (s.pool) {                                       // output by output, the four of its window by the whole wave
         for (int n = 0; n < kPooled; ++n)
             for (unsigned long long bad = __builtin_amdgcn_ballot_w64((again >> n & 1u) != 0); bad != 0; bad &= bad - 1) {
@@ -386,7 +450,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     }
 }
 
-struct BankPlan { int cp, mt, wo, wk, pf; BankShape s; size_t lds; };
+struct BankPlan { int cp, mt, wo, wk, pf, tilesX, tilesY; BankShape s; size_t lds; double clocks; };
 
 static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int mt, int wo, int wk, int lgBW, BankPlan* p) {
     p->cp = I <= 4 ? 4 : 16;
@@ -395,7 +459,8 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
     s.W = W; s.H = H; s.I = I; s.O = O; s.Wo = W / sx; s.Ho = H / sy;
     s.kw = kw; s.sx = sx; s.sy = sy; s.padX = kw / 2; s.padY = kh / 2;
     s.lgBW = lgBW;
-    const int BW = 1 << lgBW, BH = (32 >> lgBW) * mt;
+    const bool p3 = lgBW >= kP3Tile;
+    const int BW = p3 ? kP3W : 1 << lgBW, BH = p3 ? 2 * p3_rows(mt) + 1 : (32 >> lgBW) * mt, stepX = p3 ? BW - 1 : BW, stepY = p3 ? BH - 1 : BH;
     s.spr = p->cp == 16 ? kw : ceil_div(kw, 4);
     s.steps = s.spr * kh;
     s.pw = (BW - 1) * sx + (p->cp == 16 ? kw : 4 * s.spr);
@@ -407,7 +472,8 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
     s.patchMul = dp.mul; s.patchShift = dp.shift;
     s.sprMul = (unsigned)(65536 / s.spr + 1);
     const size_t sums = (size_t)wk * 32 * wo * mt * 33 * sizeof(float);
-    const long long wgs = (long long)ceil_div(s.Wo, BW) * ceil_div(s.Ho, BH) * ceil_div(s.oBlocks, wo);
+    p->tilesX = ceil_div(s.Wo, stepX); p->tilesY = ceil_div(s.Ho, stepY);
+    const long long wgs = (long long)p->tilesX * p->tilesY * ceil_div(s.oBlocks, wo);
     // As few stages as LDS allows (half of it where a CU is to hold two workgroups), of the same number of chunks: the loads of a stage are
     // one trip to memory, and every stage leaves waves without a last step.  56x56 64->96 5x5 12.9 us by single chunks, 11.4 in one stage of
     // four; 28x28 128->128 5x5 14.5 and 11.7 in two of four.
@@ -432,63 +498,69 @@ static bool bank_shape(int W, int H, int I, int O, int kw, int kh, int sx, int s
 // hanging over its edge count in full, which picks the tile shape as well.  Measured, us per layer, this choice / the
 // other tiles: 56x56 64->96 5x5 11.4 / 11.5 to 25, 224x224 3->64 7x7/2 6.1 / 7.7 to 13.7, 96x70 50->75 5x5 17.7 / 19.5 to 25, 28x28 128->128 5x5
 // 11.7 / 16 to 47, 112x112 64->128 3x3/2 9.2 / 10.1 to 15.5, 14x14 16->32 5x5 4.3 / 5 to 9.
-static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, bool pool, BankPlan* best) {
-    double bestCost = 0;
+// pool: 0, 1 (2x2/2 behind the layer) or 2 (3x3/2: lgBW is kP3Tile or one more, and mt 2 or 3; never with waves for four blocks of channels,
+// whose sums and pooling take longer than they save).
+static bool bank_plan(int W, int H, int I, int O, int kw, int kh, int sx, int sy, int variant, int pool, BankPlan* best) {
     bool found = false;
+    const int firstBW = pool == 2 ? kP3Tile : 3, lastBW = pool == 2 ? kP3Tile + 1 : pool ? 4 : 5;       // (2x2: two rows of a window in one block)
+    auto blocks = [&](int lgM, int lgBW) { return pool == 2 ? 2 + lgBW - kP3Tile : 1 << lgM; };
     if (variant >> 12) {                                // everything chosen beforehand
         const int wsel = variant >> 4 & 3, lgBW = variant >> 12;
-        return (variant & 0xfce) == 0x100 && wsel < 3 && lgBW >= 3 && lgBW <= (pool ? 4 : 5) && bank_shape(W, H, I, O, kw, kh, sx, sy, 1 << (variant & 1), 4 >> wsel, 2 << wsel, lgBW, best);
+        return (variant & 0xfce) == 0x100 && wsel < 3 && lgBW >= firstBW && lgBW <= lastBW && (pool != 2 || ((variant & 1) && wsel > 0)) &&
+               bank_shape(W, H, I, O, kw, kh, sx, sy, blocks(variant & 1, lgBW), 4 >> wsel, 2 << wsel, lgBW, best);
     }
-    for (int wsel = 0; wsel < 3; ++wsel)
-        for (int lgM = 0; lgM < 2; ++lgM) {
-            const int wo = 4 >> wsel, wk = 2 << wsel, mt = 1 << lgM;
+    for (int wsel = pool == 2 ? 1 : 0; wsel < 3; ++wsel)
+        for (int lgM = pool == 2 ? 1 : 0; lgM < 2; ++lgM) {
+            const int wo = 4 >> wsel, wk = 2 << wsel;
             if (variant && variant != (0x100 | wsel << 4 | lgM)) continue;
-            for (int lgBW = 3; lgBW <= (pool ? 4 : 5); ++lgBW) {       // (pooled: two rows of a window in one block)
+            for (int lgBW = firstBW; lgBW <= lastBW; ++lgBW) {
+                const int mt = blocks(lgM, lgBW);
                 BankPlan p;
                 if (!bank_shape(W, H, I, O, kw, kh, sx, sy, mt, wo, wk, lgBW, &p)) continue;
                 const BankShape& s = p.s;
-                const double wgs = (double)ceil_div(s.Wo, 1 << lgBW) * ceil_div(s.Ho, (32 >> lgBW) * mt) * ceil_div(s.oBlocks, wo);
+                const double wgs = (double)p.tilesX * p.tilesY * ceil_div(s.oBlocks, wo);
                 const double waveSteps = (s.nStages - 1.0) * ceil_div(s.group * s.steps, wk) + ceil_div((s.nChunks - (s.nStages - 1) * s.group) * s.steps, wk);
                 const double staging = s.nStages * 1200.0 * (1 + ceil_div(s.patchN * (p.cp == 16 ? 2 : 1) * s.group, kBankThreads));
                 const double work = std::max(1.3 * waveSteps * 2 * 6 * 32 * mt, (double)s.nChunks * s.steps * wo * 3072 / 42);
-                const double rows = pool ? 0.0 : 2.0 * 32 * wo * mt * (32 >> lgBW);
-                const double cost = 6000 + std::ceil(wgs / num_cu()) * (1500 + staging + work + rows);
-                if (!found || cost < bestCost) { found = true; bestCost = cost; *best = p; }
+                const double rows = pool == 2 ? 800.0 + 1000.0 * wo : pool ? 0.0 : 2.0 * 32 * wo * mt * (32 >> lgBW);
+                p.clocks = 6000 + std::ceil(wgs / num_cu()) * (1500 + staging + work + rows);
+                if (!found || p.clocks < best->clocks) { found = true; *best = p; }
             }
         }
     return found;
 }
 
-template <int CP, int MT, int WO, int WK, int PF>
+template <int CP, int MT, int WO, int WK, int PF, bool P3>
 static int launch_bank_pf(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
-    const BankShape& s = p.s;
-    const dim3 grid(ceil_div(s.Wo, 1 << s.lgBW), ceil_div(s.Ho, (32 >> s.lgBW) * MT), ceil_div(s.oBlocks, WO));
+    const dim3 grid(p.tilesX, p.tilesY, ceil_div(p.s.oBlocks, WO));
     static std::atomic<unsigned long long> asked{0};
-    if (int rc = allow_lds((const void*)conv_bank_mfma_kernel<CP, MT, WO, WK, PF>, p.lds, asked)) return rc;
-    launch((conv_bank_mfma_kernel<CP, MT, WO, WK, PF>), grid, dim3(kBankThreads), p.lds, st, in, F, bias, out, s);
+    if (int rc = allow_lds((const void*)conv_bank_mfma_kernel<CP, MT, WO, WK, PF, P3>, p.lds, asked)) return rc;
+    launch((conv_bank_mfma_kernel<CP, MT, WO, WK, PF, P3>), grid, dim3(kBankThreads), p.lds, st, in, F, bias, out, p.s);
     return launched("conv_bank_mfma_kernel");
 }
 
-template <int CP, int MT, int WO, int WK>
+template <int CP, int MT, int WO, int WK, bool P3>
 static int launch_bank(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
     if constexpr (CP == 16) {
-        if (p.pf == 4) return launch_bank_pf<CP, MT, WO, WK, 4>(in, F, bias, out, p, st);
-        if (p.pf == 3) return launch_bank_pf<CP, MT, WO, WK, 3>(in, F, bias, out, p, st);
+        if (p.pf == 4) return launch_bank_pf<CP, MT, WO, WK, 4, P3>(in, F, bias, out, p, st);
+        if (p.pf == 3) return launch_bank_pf<CP, MT, WO, WK, 3, P3>(in, F, bias, out, p, st);
     }
-    return p.pf == 1 ? launch_bank_pf<CP, MT, WO, WK, 1>(in, F, bias, out, p, st) : launch_bank_pf<CP, MT, WO, WK, 2>(in, F, bias, out, p, st);
+    return p.pf == 1 ? launch_bank_pf<CP, MT, WO, WK, 1, P3>(in, F, bias, out, p, st) : launch_bank_pf<CP, MT, WO, WK, 2, P3>(in, F, bias, out, p, st);
 }
 
-template <int CP, int MT>
+template <int CP, int MT, bool P3>
 static int launch_bank_w(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
-    if (p.wk == 2) return launch_bank<CP, MT, 4, 2>(in, F, bias, out, p, st);
-    if (p.wk == 4) return launch_bank<CP, MT, 2, 4>(in, F, bias, out, p, st);
-    return launch_bank<CP, MT, 1, 8>(in, F, bias, out, p, st);
+    if constexpr (!P3)
+        if (p.wk == 2) return launch_bank<CP, MT, 4, 2, P3>(in, F, bias, out, p, st);
+    if (p.wk == 4) return launch_bank<CP, MT, 2, 4, P3>(in, F, bias, out, p, st);
+    return launch_bank<CP, MT, 1, 8, P3>(in, F, bias, out, p, st);
 }
 
 template <int CP>
 static int launch_bank_m(const float* in, const unsigned short* F, const float* bias, float* out, const BankPlan& p, hipStream_t st) {
-    if (p.mt == 1) return launch_bank_w<CP, 1>(in, F, bias, out, p, st);
-    return launch_bank_w<CP, 2>(in, F, bias, out, p, st);
+    if (p.s.lgBW >= kP3Tile) return p.mt == 2 ? launch_bank_w<CP, 2, true>(in, F, bias, out, p, st) : launch_bank_w<CP, 3, true>(in, F, bias, out, p, st);
+    if (p.mt == 1) return launch_bank_w<CP, 1, false>(in, F, bias, out, p, st);
+    return launch_bank_w<CP, 2, false>(in, F, bias, out, p, st);
 }
 
 }  // namespace drhip
@@ -516,14 +588,28 @@ static bool bank_limits(int W, int H, int I, int O, int kw, int kh, int strideX,
 
 extern "C" int drhip_conv_bank_usable(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY) {
     BankPlan p;
-    return bank_limits(W, H, I, O, kw, kh, strideX, strideY) && bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, false, &p) ? 1 : 0;
+    return bank_limits(W, H, I, O, kw, kh, strideX, strideY) && bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, 0, &p) ? 1 : 0;
 }
 
 // (Choosing a tile costs the host a microsecond or two: once when a layer is scheduled, not at every launch.)
+static int bank_variant(const BankPlan& p) { return 0x100 | (p.wk == 2 ? 0 : p.wk == 4 ? 0x10 : 0x20) | (p.mt > 1 ? 1 : 0) | p.s.lgBW << 12; }
+
 extern "C" int drhip_conv_bank_pick_variant(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY, int maxpool2) {
     BankPlan p;
     if (!bank_limits(W, H, I, O, kw, kh, strideX, strideY) || !bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, maxpool2 != 0, &p)) return 0;
-    return 0x100 | (p.wk == 2 ? 0 : p.wk == 4 ? 0x10 : 0x20) | (p.mt - 1) | p.s.lgBW << 12;
+    return bank_variant(p);
+}
+
+// A 3x3/2 pooling in the layer's launch, or apart: its own launch takes 3 us and its map's way to memory and back, 2500 bytes a clock; a 1x1 layer
+// behind it that takes it on load 0.7 us and 0.6 a megabyte.  us, apart / in one launch: 224x224 3->64 7x7/2 10.6 / 8.5 (in
+// tiles of 4x4; of 4x3, 266 workgroups on 256 CUs, 12.8), 200x200 3->64 9.9 / 7.3, 96x96 3->24 8.5 / 5.9; 384x384 3->96 26.4 / 27.1, 224x224 3->32
+// 5x5 19.2 / 19.2, 56x56 64->64 5x5 10.9 / 10.8, which stay apart: 7 % are asked for, as the estimates are no better.  With a 1x1 layer, taken on load / in
+// one launch: 300x300 3->64 20.4 / 17.8, 200x200 3->64 12.2 / 10.9, 224x224 3->64 11.3 / 11.5, 128x128 3->32 7.8 / 8.4.
+extern "C" int drhip_conv_bank_maxpool3s2_pick_variant(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY, int against) {
+    BankPlan p, apart;
+    if (!bank_limits(W, H, I, O, kw, kh, strideX, strideY) || !bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, 2, &p)) return 0;
+    const double bytes = 4.0 * (W / strideX) * (H / strideY) * O, pooling = against == 1 ? 1600 + bytes / 714 : 7000 + 1.25 * bytes / 2500;
+    return against != 2 && bank_plan(W, H, I, O, kw, kh, strideX, strideY, 0, 0, &apart) && 0.93 * (apart.clocks + pooling) < p.clocks ? 0 : bank_variant(p);
 }
 
 extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O, int kw, int kh, void* stream) {
@@ -536,24 +622,29 @@ extern "C" int drhip_conv_bank_layout_f32(const float* w, float* F, int I, int O
 }
 
 static int conv_bank(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
-                     int kw, int kh, int strideX, int strideY, int relu, bool pool, int variant, void* stream, const char* who) {
+                     int kw, int kh, int strideX, int strideY, int relu, int pool, int variant, void* stream, const char* who) {
     DRHIP_REQUIRE(in && F && out, "%s: NULL tensor", who);
     DRHIP_REQUIRE(bank_limits(W, H, I, O, kw, kh, strideX, strideY), "%s: shape %dx%dx%d -> %d, %dx%d/%dx%d not covered", who, W, H, I, O, kw, kh, strideX, strideY);
     DRHIP_REQUIRE(((size_t)F & 15) == 0, "%s: the filter bank must be 16-byte aligned", who);
     BankPlan p;
     DRHIP_REQUIRE(bank_plan(W, H, I, O, kw, kh, strideX, strideY, variant, pool, &p), "%s: variant %#x does not fit this shape", who, variant);
     p.s.relu = relu ? 1 : 0;
-    p.s.pool = pool ? 1 : 0;
+    p.s.pool = pool;
     if (p.cp == 4) return launch_bank_m<4>(in, (const unsigned short*)F, bias, out, p, as_stream(stream));
     return launch_bank_m<16>(in, (const unsigned short*)F, bias, out, p, as_stream(stream));
 }
 
 extern "C" int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                                    int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
-    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, false, variant, stream, "drhip_conv_bank_f32");
+    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, 0, variant, stream, "drhip_conv_bank_f32");
 }
 
 extern "C" int drhip_conv_bank_maxpool2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                                             int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
-    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, true, variant, stream, "drhip_conv_bank_maxpool2_f32");
+    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, 1, variant, stream, "drhip_conv_bank_maxpool2_f32");
+}
+
+extern "C" int drhip_conv_bank_maxpool3s2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                                              int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream) {
+    return conv_bank(in, F, bias, out, W, H, I, O, kw, kh, strideX, strideY, relu, 2, variant, stream, "drhip_conv_bank_maxpool3s2_f32");
 }

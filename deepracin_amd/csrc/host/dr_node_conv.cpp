@@ -13,6 +13,8 @@ using namespace dr;
 namespace {
 
 inline dR_Conv2d_Data* conv_of(dR_Node* n) { return (dR_Conv2d_Data*)n->layer; }
+// (with drFusedPool: the pooling that rides along has windows of 3x3)
+inline bool pools_by_three(dR_Node* n) { return ((const dR_Pooling_Data*)((dR_Node*)n->next_layers->first->element)->layer)->shape.s1 == 3; }
 inline int weight_count(const dR_Conv2d_Data* c) { return c->shape.s0 * c->shape.s1 * c->shape.s2 * c->shape.s3; }
 
 gboolean conv_propagate(dR_Graph* net, dR_Node* node) {
@@ -173,7 +175,9 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     const bool wino = c->algo == drConvWinograd;
     const int O = launch_channels(c);
     if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
-    if (c->drSplitBank && c->drFusedPool) c->variant = drhip_conv_bank_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 1);
+    if (c->drSplitBank && c->drFusedPool)
+        c->variant = pools_by_three(node) ? drhip_conv_bank_maxpool3s2_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 2)
+                                          : drhip_conv_bank_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 1);
     const int n = c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
                        : wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
                        : c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)
@@ -332,7 +336,7 @@ gboolean conv_compute(dR_Graph* net, dR_Node* node) {
                 const dR_Conv2d_Data* sq = conv_of(c->drSqueezeNext);
                 rc = drhip_conv3x3_pool3s2_squeeze_f32(in, w, b, (const float*)sq->weightsBuf, (float*)sq->workspaceBuf, W, H, I, O, sq->shape.s3, c->stride.s1, c->stride.s2, relu, stream_of(net));
             } else if (c->drFusedPool && c->drSplitBank)
-                rc = drhip_conv_bank_maxpool2_f32(in, w, b, out, W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, relu, c->variant, stream_of(net));
+                rc = (pools_by_three(node) ? drhip_conv_bank_maxpool3s2_f32 : drhip_conv_bank_maxpool2_f32)(in, w, b, out, W, H, I, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, relu, c->variant, stream_of(net));
             else if (c->drFusedPool)            // first layer + the 3x3/2 max pool behind it (out = the pool's buffer)
                 rc = drhip_conv3x3_pool3s2_f32(in, w, b, out, W, H, I, O, c->stride.s1, c->stride.s2, relu, stream_of(net));
             else if (c->drDirectBank && c->drFusedAvgPool)

@@ -83,12 +83,15 @@ bool direct_image_layer(const dR_Conv2d_Data* c) {
     return c->algo == drConvDirect && !c->drDirectBank && !c->drSplitBank && c->shape.s0 == 3 && c->shape.s1 == 3 && c->shape.s2 <= 4;
 }
 
+dR_Node* loads_pooled(const dR_Node* c);
+
 // Max pooling stored by the convolution in front of it, so that the full-resolution tensor never
 // exists (only when nobody else wants that tensor; DR_FUSE_POOL=0 keeps the two apart):
 //  - a 2x2 / stride-2 pool behind a Winograd convolution: every 2x2 output tile of the convolution
 //    is one pooling window;
-//  - a 3x3 / stride-2 pool behind a first layer (3x3 filter, at most 4 input channels): one kernel
-//    computes the convolution outputs of a pooled tile on the matrix cores and pools them in LDS.
+//  - a 3x3 / stride-2 pool behind a first layer (3x3 filter, at most 4 input channels), or behind a layer of the split filter bank
+//    where that is the faster way: one kernel computes the convolution outputs of a pooled tile on the matrix cores and pools
+//    them in LDS.
 dR_Node* pool_fusable_producer(const dR_Node* p) {
     if (p->type != tPooling) return nullptr;
     const char* env = getenv("DR_FUSE_POOL");
@@ -111,6 +114,9 @@ dR_Node* pool_fusable_producer(const dR_Node* p) {
         const bool bank = cd->drSplitBank && drhip_conv_bank_pick_variant(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->shape.s0, cd->shape.s1, cd->stride.s1, cd->stride.s2, 1);
         if (!bank && !(cd->algo == drConvWinograd && even)) return nullptr;
     } else {
+        if (cd->drSplitBank)
+            return drhip_conv_bank_maxpool3s2_pick_variant(cd->ishape.s0, cd->ishape.s1, cd->shape.s2, cd->shape.s3, cd->shape.s0, cd->shape.s1, cd->stride.s1, cd->stride.s2,
+                                                           p->next_layers && p->next_layers->length == 1 && loads_pooled(nodes_of(p->next_layers)[0]) == p) ? c : nullptr;
         if (!direct_image_layer(cd)) return nullptr;
         // (that kernel carries its shape in 16-bit fields and its strides in 4-bit fields)
         if (cd->ishape.s0 > 65535 || cd->ishape.s1 > 65535 || cd->shape.s3 > 65535 || cd->stride.s1 > 15 || cd->stride.s2 > 15) return nullptr;
@@ -121,7 +127,7 @@ dR_Node* pool_fusable_producer(const dR_Node* p) {
 // A 3x3 / stride-2 max pooling whose only reader is a 1x1 convolution: the convolution takes the window maxima
 // while it loads its input, the pooled tensor is never written and the pooling kernel is not launched
 // (DR_FUSE_POOLIN=0 keeps them apart).  Returns the pooling node in front of such a convolution.
-dR_Node* pooled_input_of(const dR_Node* c) {
+dR_Node* loads_pooled(const dR_Node* c) {
     if (c->type != tConv2d) return nullptr;
     const char* env = getenv("DR_FUSE_POOLIN");
     if (env && strcmp(env, "0") == 0) return nullptr;
@@ -134,10 +140,13 @@ dR_Node* pooled_input_of(const dR_Node* c) {
     if (pd->poolingType != tMax || pd->shape.s1 != 3 || pd->shape.s2 != 3 || pd->shape.s3 != 1) return nullptr;
     if (pd->stride.s1 != 2 || pd->stride.s2 != 2 || pd->stride.s3 != 1) return nullptr;
     if (tensor_wanted(p) || p->outputBuf || !p->next_layers || p->next_layers->length != 1) return nullptr;
-    if (pool_fusable_producer(p)) return nullptr;      // already stored by the convolution in front of it
     // (the pooling-on-load kernel addresses the unpooled tensor with 32-bit byte offsets)
     if ((long long)pd->ishape.s0 * pd->ishape.s1 * pd->ishape.s2 >= (1ll << 29)) return nullptr;
     return p;
+}
+dR_Node* pooled_input_of(const dR_Node* c) {
+    dR_Node* p = loads_pooled(c);
+    return p && pool_fusable_producer(p) ? nullptr : p;        // (already stored by the convolution in front of it)
 }
 
 // A global average pooling (one window = the whole map) behind a 1x1 convolution, or a strided 3x3 one of at most 64 tiles of

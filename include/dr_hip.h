@@ -191,6 +191,13 @@ int drhip_conv_bank_f32(const float* in, const float* F, const float* bias, floa
 /* With a 2x2/2 max pooling behind it, by drhip_pool_f32's rules: out[O][ceil(Ho/2)][ceil(Wo/2)]. */
 int drhip_conv_bank_maxpool2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
                                  int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
+/* With a 3x3/2 max pooling behind it, by the same rules: `variant` 0, or 0x101, 0x6101 (tiles of
+ * 4x3 pooled pixels) or 0x7101 (of 4x4) | n << 4, n = 1 or 2.
+ * pick_variant: 0 if the shape is not covered, or if the two are better apart, the pooling in a launch of its own (`against` 0) or taken
+ * on load by a 1x1 layer (1); 2: whatever is better. */
+int drhip_conv_bank_maxpool3s2_pick_variant(int W, int H, int I, int O, int kw, int kh, int strideX, int strideY, int against);
+int drhip_conv_bank_maxpool3s2_f32(const float* in, const float* F, const float* bias, float* out, int W, int H, int I, int O,
+                                   int kw, int kh, int strideX, int strideY, int relu, int variant, void* stream);
 
 /* First layer (1 to 4 input channels, 3x3, any stride, zero padding, bias, optional ReLU) followed by
  * a 3x3 / stride-2 max pooling with the reference's pooling rules (out = ceil(in/2), samples outside

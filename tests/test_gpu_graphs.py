@@ -174,6 +174,39 @@ def test_average_pooling_behind_an_image_layer(oracle, gpu, W, H, I, O, relu):
     assert_close(res["1"], want[2], terms=9 * I)
 
 
+@pytest.mark.parametrize("W,H,I,O,k,reader,fused", [(200, 200, 3, 64, 7, "", True), (47, 33, 3, 20, 7, "", True), (64, 63, 16, 33, 5, "", True), (33, 47, 64, 64, 5, "", False), (260, 260, 3, 160, 7, "", False),
+                                                  (200, 200, 3, 64, 7, "1x1", True), (96, 96, 3, 24, 7, "1x1", False)])
+def test_maxpool_of_three_behind_other_filters(oracle, gpu, W, H, I, O, k, reader, fused):
+    """A layer of other filters by stride 2 and the 3x3/2 pooling behind it, in one launch where that is the faster way, and apart (DR_FUSE_POOL=0); in front of a
+    1x1 layer, which otherwise takes the pooling on load, a launch more or less makes no difference in the count."""
+    st = configs._Streams(97)
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, k, I, O, stride=2), {"op": "pool", "in": 1, "window": (3, 3, 1), "stride": (2, 2, 1), "kind": 0}]
+    if reader:
+        spec.append(configs._conv(st, 2, 1, O, 16))
+    x = configs.image_input(st, W, H, I)
+    want, res, launches, variant = oracle.run_spec(spec, {0: x}), {}, {}, 0
+    lib = dr.load_library()
+    assert (lib.drhip_conv_bank_maxpool3s2_pick_variant(W, H, I, O, k, k, 2, 2, 1 if reader else 0) != 0) == fused
+    for mode in ("1", "0"):
+        os.environ["DR_FUSE_POOL"] = mode
+        try:
+            with dr.Environment() as env:
+                g = env.create_graph()
+                nodes = configs.build_graph(g, spec, [len(spec) - 1])
+                dr.prepare(g)
+                configs.feed_chw(nodes[0], x)
+                assert g.lib.dR_apply(g.ptr) and g.lib.dR_apply(g.ptr)
+                res[mode] = configs.fetch_chw(g)[0].copy()
+                dr.graph_config(g).profilingGPU = 1
+                assert g.lib.dR_apply(g.ptr)
+                launches[mode] = g.lib.drhip_timing_count()
+        finally:
+            os.environ.pop("DR_FUSE_POOL", None)
+    assert launches["0"] - launches["1"] == (1 if fused and not reader else 0), launches
+    for got in res.values():
+        assert_close(got, want[-1], terms=I * k * k)
+
+
 def test_maxpool_taken_on_load_by_the_1x1_layer_behind_it(oracle, gpu):
     """SqueezeNet's pool3 / pool5 pattern: fire module -> 3x3/2 max pool -> squeeze 1x1.  With only the last
     tensor requested the squeeze layer pools while it loads (no pooling launch, no pooled tensor); with

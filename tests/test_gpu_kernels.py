@@ -168,6 +168,33 @@ def test_conv_split_bank_with_maxpool(lib, dev, oracle, variant, W, H, I, O, k, 
             assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("variant", [0, 0x121, 0x6111, 0x6121, 0x7111, 0x7121])
+@pytest.mark.parametrize("W,H,I,O,k,s", [(112, 96, 3, 64, 7, 2), (35, 41, 4, 33, 5, 1), (17, 13, 20, 129, 3, 2), (8, 6, 1, 5, 5, 1), (9, 7, 16, 32, 3, 1), (1, 1, 2, 3, 7, 1), (50, 3, 70, 20, 5, 2)])
+def test_conv_split_bank_with_maxpool3(lib, dev, variant, W, H, I, O, k, s):
+    """A layer and the 3x3/2 max pooling behind it in one launch: what the two give apart, around its tiles of 4x3 and 4x4 pooled pixels; without ReLU, so
+    that what lies beside the map shows, and with samples that have no parts."""
+    x, w, b = own(I, H, W), own(I, O, k, k, scale=np.sqrt(2.0 / (k * k * I))), own(O, scale=0.05)
+    Wo, Ho = W // s, H // s
+    F = dev.empty(lib.drhip_conv_bank_floats(I, O, k, k))
+    ok(lib, lib.drhip_conv_bank_layout_f32(dev.put(w), F, I, O, k, k, None))
+    full, pooled, two, bd = dev.empty(O * Wo * Ho), dev.empty(O * -(-Ho // 2) * -(-Wo // 2)), dev.empty(O * -(-Ho // 2) * -(-Wo // 2)), dev.put(b)
+    for relu, extremes in ((1, False), (0, False), (0, True)):
+        if extremes:
+            x[0, H // 2, W // 2], x[I - 1, 0, 0], x[I // 2, H - 1, W - 1] = np.inf, -np.inf, np.nan
+        xd = dev.put(x)
+        ok(lib, lib.drhip_conv_bank_f32(xd, F, bd, full, W, H, I, O, k, k, s, s, relu, variant and variant & 0x130 | 1, None))
+        ok(lib, lib.drhip_pool_f32(full, two, None, Wo, Ho, O, 3, 3, 1, 2, 2, 1, 0, None))
+        ok(lib, lib.drhip_conv_bank_maxpool3s2_f32(xd, F, bd, pooled, W, H, I, O, k, k, s, s, relu, variant, None))
+        got, want = (dev.get(p, (O, -(-Ho // 2), -(-Wo // 2))) for p in (pooled, two))
+        if extremes:                        # (worked out again in another order of the sums: an error as of two such sums in fp32)
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]) and not np.isnan(got).any()
+            f = np.isfinite(want)
+            assert not f.any() or np.all(np.abs(got[f] - want[f]) <= TOL / 20 * np.abs(w).sum((0, 2, 3)).max())
+        else:
+            assert_close(got, want, terms=I * k * k)
+            assert np.array_equal(got, want) or variant == 0 or I > 16      # (otherwise the waves may share the steps another way)
+
+
 @pytest.mark.parametrize("W,H,I,O,sx,sy", [(224, 224, 3, 64, 2, 2), (33, 31, 3, 9, 2, 2), (17, 13, 1, 5, 1, 1), (20, 18, 4, 70, 1, 2),
                                             (8, 5, 2, 16, 3, 1), (2, 2, 3, 2, 1, 1), (9, 9, 4, 33, 2, 2), (64, 48, 3, 32, 1, 1)])
 @pytest.mark.parametrize("relu", [1, 0])
