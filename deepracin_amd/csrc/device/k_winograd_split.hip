@@ -124,16 +124,37 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     const int turn = TURNS ? min(inXcd & 31, steps - 1) : 0;
     auto segment_at = [&](int k) { return k == 0 ? 4 : (2 * (k * s.tilesX - off0) + 4 * k + 6) & ~3; };     // in floats
     const unsigned stepB = 64u * KW * (unsigned)plane;
+    const int first16 = 16 * (first + set);
+    // Segment by segment, for a wave's window row and the same in all lanes: where its samples lie in LDS, behind which of them the
+    // row ends (not one of them, for a row beside the map), and the address that the first would have at the row's beginning.
+    constexpr int SEG = ws_segments(WC);
+    const unsigned plane4 = 4u * (unsigned)plane;
+    int segAt[SEG], segEnd[SEG];
+    unsigned segBase[SEG];
+#pragma unroll
+    for (int k = 0; k < SEG; ++k) {
+        const int iy = 2 * (ty0 + k) - 1 + wave, left = k == 0 && off0 > 0 ? 2 * off0 - 1 : 0;
+        segAt[k] = segment_at(k);
+        segEnd[k] = iy >= 0 && iy < H ? W - left + segAt[k] : 0;
+        segBase[k] = 4u * (unsigned)(iy * W + left - segAt[k]) + (unsigned)first16 * plane4;
+    }
     unsigned voff[NDMA];                                // (never below kOutOfRange where it started from that)
+    int piece = lane % WC;
+    unsigned chOff = (unsigned)(lane / WC) * plane4;
 #pragma unroll
     for (int i = 0; i < NDMA; ++i) {
-        const int idx = i * 64 + lane, ch = idx / WC, f = 4 * (idx % WC);
-        int k = 0;
+        const int f = 4 * piece;
+        int end = segEnd[0];
+        unsigned base = segBase[0];
 #pragma unroll
-        for (int q = 1; q < ws_segments(WC); ++q) k += f >= segment_at(q) ? 1 : 0;
-        const int x = (k == 0 && off0 > 0 ? 2 * off0 - 1 : 0) + f - segment_at(k), iy = 2 * (ty0 + k) - 1 + wave;
-        const bool ok = f >= 4 && x < W && iy >= 0 && iy < H;
-        voff[i] = (ok ? 4u * (unsigned)((16 * (first + set) + ch) * plane + iy * W + x) : kOutOfRange) + (unsigned)turn * stepB;
+        for (int k = 1; k < SEG; ++k) {
+            end = f >= segAt[k] ? segEnd[k] : end;
+            base = f >= segAt[k] ? segBase[k] : base;
+        }
+        voff[i] = (f >= 4 && f < end ? base + 4u * (unsigned)f + chOff : kOutOfRange) + (unsigned)turn * stepB;
+        const bool wrap = piece >= WC - 64 % WC;        // 64 pieces on
+        piece += 64 % WC - (wrap ? WC : 0);
+        chOff += (unsigned)(64 / WC) * plane4 + (wrap ? plane4 : 0u);
     }
     const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, min(I, 16 * (first + perSplit)) * plane * 4, kBufferFlags);    // (ends with the split)
     const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(set * 3 * BUFB);
@@ -161,16 +182,19 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     // origin the compiler does not see keeps it from taking them for loads that no memory clobber concerns.
     const unsigned short* uHere = U;
     asm volatile("" : "+s"(uHere));
-    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, 16 * s.nC * 3 * s.nOB * 1024, kBufferFlags);
+    const int uBytes = 16 * s.nC * 3 * s.nOB * 1024;
+    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, uBytes, kBufferFlags);
     unsigned uOb[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) uOb[nt] = (unsigned)((wave * s.nC * s.nOB + min(oBlock * NT + nt, s.nOB - 1)) * 12288);
     const unsigned uStep = (unsigned)s.nOB * 12288u;
+    // (what the last step requests for one behind it comes from nowhere)
+    __amdgpu_buffer_rsrc_t rNext = rU;
     // the first part of two positions and the others of one: no more registers are left
     u32x4b f0[2][NT], f12[NT][2];
     auto filter = [&](int e, int nt, int q) -> u32x4b& { return q == 0 ? f0[e & 1][nt] : f12[nt][q - 1]; };
-    auto load_filter = [&](int e, int nt, int q, int step) {
-        filter(e, nt, q) = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(rU, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 3072)), 0));
+    auto load_filter = [&](const __amdgpu_buffer_rsrc_t& from, int e, int nt, int q, int step) {
+        filter(e, nt, q) = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 3072)), 0));
     };
 
     // ---- operands --------------------------------------------------------------------------------------------------
@@ -235,18 +259,23 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     };
 
     // ---- prologue --------------------------------------------------------------------------------------------------
+    float biasEarly = 0.0f;
+    if (tid < OB && bias) biasEarly = bias[min(o0 + tid, s.O - 1)];
+    asm volatile("" ::: "memory");
+    // What the first products need comes first, the rest behind the barrier.
 #pragma unroll
-    for (int i = 0; i < 2 * NDMA; ++i) fetch_sample(i / NDMA, i % NDMA);
+    for (int i = 0; i < (KW == 1 ? 2 : 1) * NDMA; ++i) fetch_sample(i / NDMA, i % NDMA);
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int q = 0; q < (e == 0 ? 3 : 1); ++q) load_filter(e, nt, q, first + set + KW * turn);
-    if (tid < OB) biasT[tid] = bias ? bias[min(o0 + tid, s.O - 1)] : 0.0f;
-    // (the first step's samples have arrived once no more than the second step's and the filters are under way)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
+        for (int q = 0; q < 3; ++q) load_filter(rU, 0, nt, q, first + set + KW * turn);
+    if (tid < OB) biasT[tid] = biasEarly;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NT + (KW == 1 ? NDMA : 0)) : "memory");
     barrier();
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) if (KW == 2) fetch_sample(1, i);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) load_filter(rU, 1, nt, 0, first + set + KW * turn);
 #pragma unroll
     for (int j = 0; j < 8; ++j) { read_rows(0, j); combine(j); }
 #pragma unroll
@@ -263,7 +292,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             // a part's last product has been issued: its registers take the filters that come next
             if (q == 2 || q == 4 || q == 5) {
                 const int by = q == 2 ? 2 : 1;
-                load_filter((e + by) & 3, nt, kPA[q], e + by >= 4 ? stepNext : step);
+                load_filter(e + by >= 4 ? rNext : rU, (e + by) & 3, nt, kPA[q], e + by >= 4 ? stepNext : step);
             }
 #pragma unroll
             for (int tk = 2 * i; tk < 2 * i + 2; ++tk) {
@@ -294,6 +323,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
         const int step = first + set + KW * m;
         m = TURNS && m == steps - 1 ? 0 : m + 1;
         const int stepNext = first + set + KW * m;
+        rNext = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, n + 1 < steps ? uBytes : 0, kBufferFlags);
         position(integral_constant<int, 0>{}, step, stepNext, nxt, nxt2);
         position(integral_constant<int, 1>{}, step, stepNext, nxt, nxt2);
         position(integral_constant<int, 2>{}, step, stepNext, nxt, nxt2);
