@@ -282,14 +282,15 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         return s.relu ? fmaxf(v, 0.0f) : v;
     };
     // The sum at pixel (x, y) of the map for channel oc of the workgroup: CH channels side by side, 64 / CH lanes for each.
-    auto once_more = [&](auto channels, int x, int y, int oc) {
+    // (kh by the caller, once: the division is not for every output)
+    auto once_more = [&](auto channels, int kh, int x, int y, int oc) {
         constexpr int CH = decltype(channels)::value;
         const int o = blockIdx.z * (32 * WO) + oc;
         const unsigned fAgain = (unsigned)(min(o >> 5, s.oBlocks - 1) * 1024 + (o & 31) * 16);
-        const int left = x * s.sx - s.padX, top = y * s.sy - s.padY, kh = s.steps / s.spr;
+        const int left = x * s.sx - s.padX, top = y * s.sy - s.padY;
         for (int j = 0; j < kh; ++j) {
-            const float* row = in + (size_t)min(max(top + j, 0), s.H - 1) * s.W;        // (a row beside the map stands for one that is in the window)
             bool nan = false;
+            const float* row = in + (size_t)min(max(top + j, 0), s.H - 1) * s.W;        // (a row beside the map stands for one that is in the window)
             for (int c = lane; c < s.I; c += 64)
                 for (int i = 0; i < s.kw; ++i) {
                     const float v = row[(size_t)c * plane + min(max(left + i, 0), s.W - 1)];
@@ -297,20 +298,34 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
                 }
             if (__builtin_amdgcn_ballot_w64(nan) != 0) return __builtin_nanf("");
         }
+        // (its instructions bound this, not its loads: one offset for the samples of a position, and channels that do not exist end the resource)
+        const __amdgpu_buffer_rsrc_t rAll = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, s.I * plane * 4, kBufferFlags);
         float v = 0.0f;
         for (int chunk = 0; chunk < s.nChunks; ++chunk)
             for (int u = lane / CH; u < 2 * s.steps; u += 64 / CH) {            // half a k-step: eight values of k
                 const int step = u >> 1, h = u & 1, j = (int)(((unsigned)step * s.sprMul) >> 16), i0 = step - j * s.spr;
                 const unsigned f = fAgain + (unsigned)((chunk * s.steps + step) * 3 * s.oBlocks * 1024 + 512 * h), partF = (unsigned)s.oBlocks * 1024u;
                 const u32x4b hi = bank_load4(rF, f, 0), mid = bank_load4(rF, f + partF, 0), lo = bank_load4(rF, f + 2 * partF, 0);
+                constexpr int G = CP == 16 ? 1 : 2;     // positions of eight values
+                bool ok[G];
+                float sample[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int c = CP == 16 ? 16 * chunk + 8 * h + e : e & 3, i = CP == 16 ? i0 : 4 * i0 + 2 * h + (e >> 2);
-                    const int ix = left + i, iy = top + j;
-                    const bool ok = c < s.I && i < s.kw && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
-                    const float sample = in[ok ? (size_t)c * plane + iy * s.W + ix : 0];
-                    auto of = [&](u32x4b q) { return e & 1 ? q[e / 2] >> 16 : q[e / 2] & 0xffffu; };
-                    v = ok ? fmaf(whole(of(hi), of(mid), of(lo)), sample, v) : v;
+                for (int g = 0; g < G; ++g) {
+                    const int i = CP == 16 ? i0 : 4 * i0 + 2 * h + g, ix = left + i, iy = top + j;
+                    ok[g] = i < s.kw && ix >= 0 && ix < s.W && iy >= 0 && iy < s.H;
+                    const int at = 4 * ((CP == 16 ? (16 * chunk + 8 * h) * plane : 0) + iy * s.W + ix);
+#pragma unroll
+                    for (int e = 0; e < 8 / G; ++e) sample[8 / G * g + e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rAll, (ok[g] ? at : 0) + 4 * e * plane, 0, 0));
+                }
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    float w = v;
+#pragma unroll
+                    for (int e = 8 / G * g; e < 8 / G * (g + 1); ++e) {
+                        auto of = [&](u32x4b q) { return e & 1 ? q[e / 2] >> 16 : q[e / 2] & 0xffffu; };
+                        w = fmaf(whole(of(hi), of(mid), of(lo)), sample[e], w);
+                    }
+                    v = ok[g] ? w : v;
                 }
             }
 #pragma unroll
@@ -334,13 +349,14 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
             v[n] = finish(v[n], kSplitUnscale, biasT[first_of(n) + (tid >> 5)]);
         }
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(again != 0u) != 0, 0)) {       // (as below, output by output)
+            const int kh = s.steps / s.spr;
 #pragma unroll
             for (int n = 0; n < NT; ++n)
                 for (unsigned long long bad = __builtin_amdgcn_ballot_w64((again >> n & 1u) != 0); bad != 0; bad &= bad - 1) {
                     const int src = __builtin_ctzll(bad), oc = first_of(n) + ((tid & ~63) + src) / 32, pl = 32 * block_of(n) + (src & 31);
                     const int x = x0 + pl % kP3W, y = y0 + pl / kP3W;
                     if (pl >= kP3W * kP3H || x >= s.Wo || y >= s.Ho) continue;
-                    const float once = finish(once_more(std::integral_constant<int, 1>{}, x, y, oc), 1.0f, biasT[oc]);
+                    const float once = finish(once_more(std::integral_constant<int, 1>{}, kh, x, y, oc), 1.0f, biasT[oc]);
                     v[n] = lane == src ? once : v[n];
                 }
         }
@@ -415,11 +431,12 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
     // An infinite sample (or one that is infinite once it is scaled) has no three-part form and leaves NaN behind, and so do the parts of
     // ordinary samples times an infinite weight: such outputs are worked out again in fp32 from the samples and the filters put
     // together.  Every wave for itself, pixel by pixel: its output channels side by side, the lanes left over share the k-steps.  A
-    // pixel with a NaN in its window stays one.  (56x56 64->96 5x5, us: 12.6, with a NaN and an infinity among the samples 346, all NaN
-    // 81; by one lane each the second took 2000.)
+    // pixel with a NaN in its window stays one.  (56x56 64->96 5x5, us: 11.1, with a NaN and an infinity among the samples 289 - 441
+    // with a 64-bit address and a check for every sample - and all NaN 113; by one lane each the second took 2000.)
     const unsigned long long any = __builtin_amdgcn_ballot_w64(again != 0u);
     if (__builtin_expect(any == 0, 1)) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
+    const int kh = s.steps / s.spr;
     if (s.pool) {                                       // output by output, the four of its window by the whole wave
         for (int n = 0; n < kPooled; ++n)
             for (unsigned long long bad = __builtin_amdgcn_ballot_w64((again >> n & 1u) != 0); bad != 0; bad &= bad - 1) {
@@ -432,7 +449,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
                 float best = -FLT_MAX;
                 for (int e = 0; e < 4; ++e) {
                     const int xe = x + (e & 1), ye = y + (e >> 1);
-                    best = larger(best, xe < s.Wo && ye < s.Ho ? finish(once_more(std::integral_constant<int, 1>{}, xe, ye, oc), 1.0f, biasT[oc]) : 0.0f);
+                    best = larger(best, xe < s.Wo && ye < s.Ho ? finish(once_more(std::integral_constant<int, 1>{}, kh, xe, ye, oc), 1.0f, biasT[oc]) : 0.0f);
                 }
                 if (lane == src) store_through(out + (size_t)o * Pp + (size_t)(y >> 1) * Wp + (x >> 1), best);
             }
@@ -444,7 +461,7 @@ conv_bank_mfma_kernel(const float* __restrict__ in, const unsigned short* __rest
         const int px = __builtin_ctzll(bad), pl = px & 31, m = px >> 5;
         const int x = x0 + (pl & (BW - 1)), y = y0 + (pl >> s.lgBW) + BH * m;
         if (x >= s.Wo || y >= s.Ho) continue;
-        const float v = finish(once_more(std::integral_constant<int, CH>{}, x, y, oc), 1.0f, biasT[oc]);
+        const float v = finish(once_more(std::integral_constant<int, CH>{}, kh, x, y, oc), 1.0f, biasT[oc]);
         const unsigned noted = (unsigned)__shfl((int)again, MT == 1 ? 32 * (ci & 1) + pl : px) >> (MT == 1 ? ci >> 1 : ci);
         if (lane < CH && (noted & 1u) && o < s.O) store_through(out + (size_t)o * P + (size_t)y * s.Wo + x, v);
     }
