@@ -137,7 +137,15 @@ __device__ inline f32x4 buf_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, un
 // without a second workgroup's share of partial tiles in memory.
 // FEWC: a layer with at most four input channels (an image): one stage whose third and fourth k-step would multiply
 // zeros are left out, and nothing is prefetched.
-template <int NT, int KW, bool FEWC = false>
+// HELP: a launch with helpers.  Panels that fill one round of the CUs only in part leave the others idle: 56x56 256->256 has 200 panels
+// for 256 CUs.  There the CUs without a panel of their own take the last stages (cfg1, bits 16 to 23: channels in eights) of
+// several panels each, one panel after the other, and leave the sums in the panel's slots of the workspace (as the joined splits do); the panel's
+// own workgroup adds them to its own.  What a helper has to do once per panel - first loads, sums, stores - takes as long as four stages of
+// eight channels, so the pieces are uneven and their size comes from a rule (wino_helpers).  A helper waits for nobody and stands
+// first in the grid, so whoever waits for it gets it.  us, without / with: 56x56 256->256 19.5 / 18.5, 52x52 256->256 19.5 / 17.2,
+// 36x36 256->512 20.4 / 17.9, 48x48 256->256 22.4 (as two launches) / 16.2, 48x48 128->256 14.1 / 10.3.  (A panel for each of a
+// helper's two wave sets: the same with four panels a helper, 18.4 / 17.3 with three; the next panel's first loads in front of this one's sums: nothing.)
+template <int NT, int KW, bool FEWC = false, bool HELP = false>
 __global__ void __launch_bounds__(kWinoThreads * KW, KW == 2 ? 1 : (NT == 1 ? 3 : (NT == 2 ? 2 : 1)))
 winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__ U, const float* __restrict__ bias,
                          WINO_ARGS, float* __restrict__ out, float* __restrict__ ws) {
@@ -153,7 +161,12 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
     // order (finest cut first, whole panels last): one workgroup of every full tier lands on each CU, so the
     // CUs end up with equal numbers of stages although the panel count is no multiple of the CU count.
     int slot = (int)(blockIdx.x / kXcds), split = (int)blockIdx.y, nSp = nSplits, lgSp = lgSplits, chunksHere = chunksPerSplit;
-    if (tiered) {
+    int donated = 0;
+    if constexpr (HELP) {
+        donated = (int)((cfg1 >> 16) & 255u);
+        nSp = 1;
+        slot -= nSplits;                                // (the first workgroups of an XCD are its helpers)
+    } else if (tiered) {
         int jj = slot, base = 0;
         bool found = false;
 #pragma unroll
@@ -171,11 +184,12 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         split = slot & (nSplits - 1);
         slot >>= lgSplits;
     }
-    const int logical = (blockIdx.x % kXcds) * perXcd + slot;
-    if (slot >= perXcd || logical >= nBlocks) return;
-    const int oBlock = fast_div(logical, nTBd);
-    const int o0 = oBlock * OB;
-    const int t0 = (logical - oBlock * (int)nTBd.d) * TB;
+    const bool helper = HELP && slot < 0;
+    int inXcd = helper ? slot + nSplits : slot, logical = (blockIdx.x % kXcds) * perXcd + inXcd;    // (a helper's first)
+    if (inXcd >= perXcd || logical >= nBlocks) return;
+    int oBlock = fast_div(logical, nTBd);
+    int o0 = oBlock * OB;
+    int t0 = (logical - oBlock * (int)nTBd.d) * TB;
     // The fewer stages a workgroup has, the sooner its partial tiles can be on their way: small pieces first,
     // so that the workgroups that end a CU's work are whole panels, which wait for nobody.
     if (tiered) {
@@ -188,7 +202,8 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
     // tile 0 carries the three selects per k-step that move that one lane's samples (`shifted` below); in every other
     // block they are constants and vanish.  (A branch inside the stage, and two copies of the channel loop alone, both cost more
     // than they saved: the first breaks the stage's instruction order, the second made the compiler spill.)
-    auto rest_of_kernel = [&](auto tile0Block) {
+    auto rest_of_kernel = [&](auto tile0Block, auto helping) {
+        constexpr bool kHelping = decltype(helping)::value;     // (of a launch with helpers: this is one)
         const int tid = threadIdx.x, lane = tid & 63;
         const int waveId = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int wave = waveId & 3;                    // = row of the transform
@@ -196,8 +211,8 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         const int l32 = lane & 31, lhi = lane >> 5;
         const int plane = H * W;
         const int nChunksAll = (I + KC - 1) / KC;
-        const int chBegin = split * chunksHere;
-        const int chEnd = min(nChunksAll, chBegin + chunksHere);        // > chBegin: the launcher creates no empty split
+        const int chBegin = HELP ? (kHelping ? nChunksAll - donated : 0) : split * chunksHere;
+        const int chEnd = HELP ? (kHelping ? nChunksAll : nChunksAll - donated) : min(nChunksAll, chBegin + chunksHere);        // > chBegin: the launcher creates no empty split
         const int Opad = wino_opad(O);
 
         // ---- this lane's tile and the byte offsets of the two window rows it reads ---------------
@@ -257,7 +272,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         constexpr bool kBiasEarly = NT <= 2;
         constexpr int EO = 8 * KW;                      // output channels finished per pass of the epilogue
         float biasEarly[kBiasEarly ? OB / EO : 1];
-        if (kBiasEarly && bias && (nSp == 1 || joined)) {
+        if (kBiasEarly && !kHelping && bias && (nSp == 1 || joined)) {
 #pragma unroll
             for (int q = 0; q < OB / EO; ++q) biasEarly[q] = bias[min(o0 + (tid >> 5) + EO * q, O - 1)];
         }
@@ -337,6 +352,18 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         for (; ch < chMain; ch += KW) stage(ch, std::true_type{});
         for (; ch < chEnd; ch += KW) stage(ch, std::false_type{});
 
+        // The slots of a panel's partial tiles (see the joined splits below): the helper fills them, the panel's own workgroup asks for
+        // its lanes' now and looks at them when its own sums are ready.
+        const __amdgpu_buffer_rsrc_t rHelp = __builtin_amdgcn_make_buffer_rsrc((void*)ws, 0, 0x7ffffff0, kBufferFlags);
+        const int helpRegion = (int)(4u * (unsigned)logical * (unsigned)(OB * TB * 4));
+        u32x4 helped[OB / EO];
+        auto ask_helper = [&] {
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < OB / EO; ++q) helped[q] = __builtin_amdgcn_raw_buffer_load_b128(rHelp, (int)(16u * (unsigned)(((tid >> 5) + EO * q) * TB + (tid & 31))), helpRegion, kAuxDeviceVolatile);
+        };
+        if constexpr (HELP && !kHelping) ask_helper();
+
         // ---- epilogue -----------------------------------------------------------------------------
         // Accumulator layout of the 32x32 MFMA: lane -> column (tile) lane%32; register r -> row
         // (output channel) 8*(r/4) + 4*(lane/32) + r%4.
@@ -380,7 +407,19 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             return f32x4{p[0][0] + p[1][0] + p[2][0], p[0][1] + p[1][1] + p[2][1],
                          p[1][0] - p[2][0] + p[3][0], p[1][1] - p[2][1] + p[3][1]};
         };
-        if (joined && nSp > 1) {
+        if constexpr (HELP) {
+            if constexpr (kHelping) {
+#pragma unroll
+                for (int q = 0; q < OB / EO; ++q)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(eo + EO * q)), rHelp, (int)(16u * (unsigned)((eo + EO * q) * TB + et)), helpRegion, kAuxThrough);
+                // (the next panel's sums go where these were)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                return;
+            }
+        }
+        if (!HELP && joined && nSp > 1) {
             // (the partial tiles go out and are looked for at the highest priority: the other workgroups on this CU
             // are in their channel loops, and a wave at their priority gets an issue slot only when they stall)
             if (tiered) __builtin_amdgcn_s_setprio(3);
@@ -453,10 +492,29 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             else collect(std::integral_constant<int, 16>{});
             return;
         }
+        bool arrived = true;
+        if constexpr (HELP && !kHelping) {
+            auto all_here = [&] {
+                bool r = true;
+#pragma unroll
+                for (int q = 0; q < OB / EO; ++q) r = r && helped[q][0] != kWinoEmpty && helped[q][1] != kWinoEmpty && helped[q][2] != kWinoEmpty && helped[q][3] != kWinoEmpty;
+                return r;
+            };
+            arrived = all_here();
+            for (int spins = 0; spins < kWinoJoinSpins && !arrived; ++spins) { ask_helper(); arrived = all_here(); }
+            const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
+#pragma unroll
+            for (int q = 0; q < OB / EO; ++q) __builtin_amdgcn_raw_buffer_store_b128(empty, rHelp, (int)(16u * (unsigned)((eo + EO * q) * TB + et)), helpRegion, kAuxThrough);
+            if (!arrived) atomicAdd(&g_wino_join_timeouts, 1u);
+        }
 #pragma unroll
         for (int q = 0; q < OB / EO; ++q) {
             const int ol = eo + EO * q, o = o0 + ol;
-            const f32x4 y = tile_of(ol);
+            f32x4 y = tile_of(ol);
+            if constexpr (HELP && !kHelping) {          // (a helper that never delivered shows in the result, too)
+                y += __builtin_bit_cast(f32x4, helped[q]);
+                if (!arrived) y = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+            }
             float y00 = y[0], y01 = y[1], y10 = y[2], y11 = y[3];
             if (direct) {
                 if (eTileOk && o < O) {
@@ -480,11 +538,24 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
     // (Only the eight-wave form pays back the second copy: the first layers' kernels are so short that fetching
     // twice the code costs them more - 224x224 3->64: 7.7-8.9 against 6.9 us - and the 32-channel four-wave form
     // gained nothing.)
+    if constexpr (HELP) {
+        if (helper) {
+            for (;;) {                                  // every nSplits-th panel of the XCD
+                rest_of_kernel(std::true_type{}, std::true_type{});
+                inXcd += nSplits;
+                logical += nSplits;
+                if (inXcd >= perXcd || logical >= nBlocks) return;
+                oBlock = fast_div(logical, nTBd);
+                o0 = oBlock * OB;
+                t0 = (logical - oBlock * (int)nTBd.d) * TB;
+            }
+        }
+    }
     if constexpr (KW == 2) {
-        if (t0 == 0) rest_of_kernel(std::true_type{});
-        else rest_of_kernel(std::false_type{});
+        if (t0 == 0) rest_of_kernel(std::true_type{}, std::false_type{});
+        else rest_of_kernel(std::false_type{}, std::false_type{});
     } else {
-        rest_of_kernel(std::true_type{});
+        rest_of_kernel(std::true_type{}, std::false_type{});
     }
 }
 
@@ -750,13 +821,19 @@ winograd_split_reduce_kernel(const float* __restrict__ ws, const float* __restri
 //         | 0x1000 (with 0x800, split bits 0): tiered joined splits - the panels of an XCD are dealt out in tiers
 //                  of whole panels, halves, quarters, ... so that every CU ends up with about the same number of
 //                  stages (see wino_tiers)
-struct WinoCfg { int nt, splits, tb, waveSets; bool joined, tiered; };
+//         | 0x2000 (0x2c01 only): idle CUs help the others out (see wino_helpers; the same workspace)
+struct WinoCfg { int nt, splits, tb, waveSets; bool joined, tiered, helped; };
 
 static bool wino_variant(int variant, WinoCfg* c) {
     c->waveSets = (variant & 0x400) ? 2 : 1;
     c->joined = (variant & 0x800) != 0;
     c->tiered = (variant & 0x1000) != 0;
-    if (variant >> 13) return false;
+    c->helped = (variant & 0x2000) != 0;
+    if (variant >> 14) return false;
+    if (c->helped) {
+        c->nt = 1; c->splits = 1; c->tb = 32;
+        return variant == 0x2c01;
+    }
     if (c->tiered && (!c->joined || c->waveSets == 2 || ((variant >> 4) & 0xf) != 0 || (variant & 0xf) > 2)) return false;
     if (c->joined && !c->tiered && ((variant & 0x100) || ((variant >> 4) & 0xf) < 1 || ((variant >> 4) & 0xf) > 4)) return false;
     if (c->joined && (variant & 0x100)) return false;
@@ -821,6 +898,20 @@ static bool wino_tiers(int nBlocks, int nChunks, int cus, WinoTiers* t) {
     return t->maxLg > 0;
 }
 
+// Who helps (see the kernel): an XCD has P panels and `cus` CUs; cus - P helpers have up to `each` panels each.  In stages of eight channels
+// (0.47 us on a CU) a panel's own workgroup needs n - d and 11 on top where something is joined, a helper each * (d + 4) and 5 or 6:
+// the largest even d for which the helper is done first.  Below 4 the join costs what is gained (57x55 256->256, d = 2: 20.1 / 20.0).
+// Measured, d = 2, 4, 6, 8, 10: 56x56 256->256 (four panels each) 19.4 18.7 21.3 24.9 28.9; 52x52 (three) 19.0 18.0 17.3 19.7 22.4; 48x48 (two)
+// 19.1 17.9 17.0 16.1 16.5.
+WinoHelpers wino_helpers(int nBlocks, int nChunks, int cus) {
+    const int P = ceil_div(nBlocks, kXcds);
+    WinoHelpers best = {0, 0};
+    if (P >= cus) return best;
+    const int each = ceil_div(P, cus - P);
+    for (int d = 4; d <= 254 && nChunks - d >= 2 && each * (d + 4) <= nChunks - d + 5; d += 2) best = {cus - P, d};
+    return best;
+}
+
 // Workspace: [splits][panel][o in panel][tile in panel] partial 2x2 tiles (float4 each); tiered launches: one
 // panel-sized region per workgroup of the grid.
 constexpr int kEpiAvgPool2 = 4;     // (inside this file: of the kernels for images)
@@ -835,6 +926,16 @@ static int launch_wino(const float* in, const float* U, const float* bias, float
     const int vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
     const FastDiv dx = make_fastdiv(g.tilesX), dtb = make_fastdiv(g.nTB);
     const bool joined = c.joined && g.splits > 1;   // (a layer with fewer stages than splits may end up unsplit)
+    if constexpr (TB == 32 && NT == 1) {
+        if (c.helped) {
+            const WinoHelpers h = wino_helpers(g.nBlocks, g.nChunks, num_cu() / kXcds);
+            static_assert(4 * 2 * OB * TB * sizeof(float) * 2 <= 65536, "no more LDS than any launch may have");
+            launch((winograd_f23_mfma_kernel<1, 2, false, true>), dim3(gridX + h.count * kXcds), dim3(2 * kWinoThreads), 2 * ldsBytes, s, in, U, bias,
+                   (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dx.mul, dtb.mul,
+                   dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | (unsigned)h.count << 13, (unsigned)h.donated << 16, out, workspace);
+            return launched("winograd_f23_mfma_kernel");
+        }
+    }
     if constexpr (TB == 32) {
         WinoTiers t;
         if (c.tiered && wino_tiers(g.nBlocks, g.nChunks, num_cu() / kXcds, &t)) {
@@ -921,7 +1022,10 @@ extern "C" int drhip_conv3x3_winograd_pick_variant(int W, int H, int I, int O) {
     // Small layers (SqueezeNet's expand convolutions: <= 8 stages, a few dozen 32x32 panels) are bound
     // by the latency of one workgroup, not by throughput: 16x16 blocks, unsplit, one launch
     // (in a replayed launch graph 4.2-5.8 us per layer against 5.1-7.1 us for the 32x32 forms).
-    if (ceil_div(T, 32) * ceil_div(O, 32) < cus / 2 && ceil_div(I, kWinoKC) <= 16)
+    // (Where they would need a second round of the CUs and halves of the 32x32 panels can be joined: those, from 10 stages on.
+    // 48x105 96->64 8.5 / 7.8, 34x32 128->256 10.2 / 8.2; with 8 stages 49x60 64->160 6.8 / 7.3)
+    if (ceil_div(T, 32) * ceil_div(O, 32) < cus / 2 && ceil_div(I, kWinoKC) <= 16 &&
+        !(ceil_div(I, kWinoKC) > 8 && ceil_div(T, 16) * ceil_div(O, 16) > cus && wino_join_flag(1, ceil_div(I, kWinoKC))))
         // 6+ stages and at most one workgroup per CU (14x14 maps; 56x56 64->64: 5.3 vs 5.5 us): two wave sets
         return (ceil_div(I, kWinoKC) >= 6 && ceil_div(T, 16) * ceil_div(O, 16) <= cus) ? 0x501 : 0x101;
     // (an image layer has next to no transform work to share, and twice the workgroups of half the size spread its
@@ -930,16 +1034,22 @@ extern "C" int drhip_conv3x3_winograd_pick_variant(int W, int H, int I, int O) {
     const int panels = ceil_div(T, 32) * ceil_div(O, code == 2 ? 64 : 32);
     const int nChunks = ceil_div(I, kWinoKC);
     int lg = 0;
-    // (a split costs a second kernel: below 6 stages in all it does not pay)
-    while (lg < 5 && nChunks >= 6 && (panels << lg) < (5 * cus) / 8 && (nChunks >> (lg + 1)) >= 2) ++lg;
+    // Panels for one round of the CUs and no halves of them: the CUs without one help the others.
+    if (code == 1 && 2 * panels > cus && wino_join_flag(1, 2) && wino_helpers(panels, nChunks, cus / kXcds).count) return 0x2c01;
+    // (a split costs a second kernel: below 6 stages in all it does not pay, nor where the next cut is too fine to be joined in one round
+    // and this one is whole or can be joined.  us, with / without that cut: 46x46 64->256 10.2 / 7.4, 34x32 256->256 13.7 / 12.4,
+    // 36x36 256->96 9.8 / 8.4)
+    auto enough = [&] { return (panels << (lg + 1)) > cus && (lg == 0 || wino_join_flag(lg, nChunks)); };
+    while (lg < 5 && nChunks >= 6 && !enough() && (panels << lg) < (5 * cus) / 8 && (nChunks >> (lg + 1)) >= 2) ++lg;
     // At most one workgroup per CU and at least two stages for each wave set: eight waves per workgroup,
     // so that every SIMD still has two waves to alternate between (56x56 256->256: 23.6 vs 24.8 us;
     // 28x28 512->512 as 112 panels x 2 splits: 26.3 vs 26.9 us for 64-channel panels x 4 splits).
     // A split whose workgroups are all resident at once (one per CU) adds its partial tiles up inside the launch.
-    // (joined splits of fewer than 16 stages each: four waves, 14x14 512->512 as 8 splits: 10.4 vs 11.1 us)
+    // (joined splits of fewer than 16 stages each, finer than halves: four waves, 14x14 512->512 as 8 splits: 10.4 vs 11.1 us, 36x36 256->96
+    // as 4 8.4 / 9.4; as halves 34x32 128->256 8.9 / 8.2, 192->256 11.0 / 10.1)
     if ((panels << lg) <= cus && (nChunks >> lg) >= 4) {
         const int join = wino_join_flag(lg, nChunks);
-        return ((join && (nChunks >> lg) < 16) ? 0 : 0x400) | code | (lg << 4) | join;
+        return ((join && lg > 1 && (nChunks >> lg) < 16) ? 0 : 0x400) | code | (lg << 4) | join;
     }
     // Unsplit layers with more 32-channel panels than CUs, but no multiple of them (112x112 128->128: 392 panels,
     // two on 136 CUs and one on 120): tiers of whole, halved, ... panels even the CUs out (in a replayed VGG16
@@ -985,6 +1095,7 @@ extern "C" size_t drhip_conv3x3_winograd_workspace_floats(int W, int H, int I, i
     const WinoGeom g = wino_geom(W, H, I, O, c);
     WinoTiers t;
     if (c.tiered) return wino_tiers(g.nBlocks, g.nChunks, num_cu() / kXcds, &t) ? (size_t)t.wgsPerXcd * kXcds * (c.tb * c.nt) * c.tb * 4 : 0;
+    if (c.helped) return wino_helpers(g.nBlocks, g.nChunks, num_cu() / kXcds).count ? (size_t)g.nBlocks * 32 * 32 * 4 : 0;
     if (g.splits <= 1) return 0;
     return (size_t)g.splits * g.nBlocks * (c.tb * c.nt) * c.tb * 4;
 }
@@ -1011,6 +1122,7 @@ extern "C" int drhip_conv3x3_winograd_f32(const float* in, const float* U, const
     DRHIP_REQUIRE(!(relu & DRHIP_EPILOGUE_MAXPOOL2) || ((W | H) & 1) == 0, "drhip_conv3x3_winograd_f32: the fused 2x2 max pool needs even W and H (got %dx%d)", W, H);
     if (variant == 0) {
         variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
+        if (variant & 0x2000) variant = 0x401;
         if (variant & 0x1000) variant = (variant & 0xf) == 2 ? 2 : 1;      // (joined splits need a prepared workspace: explicit variants only)
         variant &= ~0x800;
         if (!workspace) variant &= 0x50f;          // no workspace offered: stay unsplit
@@ -1020,7 +1132,11 @@ extern "C" int drhip_conv3x3_winograd_f32(const float* in, const float* U, const
     const WinoGeom g = wino_geom(W, H, I, O, c);
     DRHIP_REQUIRE(g.splits == 1 || workspace, "drhip_conv3x3_winograd_f32: variant %d splits the input channels and needs a workspace", variant);
     DRHIP_REQUIRE(g.splits <= 65535, "drhip_conv3x3_winograd_f32: too many input-channel splits");
-    if (c.tiered) {
+    if (c.helped) {
+        const WinoHelpers h = wino_helpers(g.nBlocks, g.nChunks, num_cu() / kXcds);
+        DRHIP_REQUIRE(h.count > 0, "drhip_conv3x3_winograd_f32: variant %#x: %d panels of %d stages leave nobody to help", variant, g.nBlocks, g.nChunks);
+        DRHIP_REQUIRE(workspace, "drhip_conv3x3_winograd_f32: variant %#x joins splits and needs a prepared workspace", variant);
+    } else if (c.tiered) {
         WinoTiers t;
         if (wino_tiers(g.nBlocks, g.nChunks, num_cu() / kXcds, &t)) {
             // A workgroup waits for the other splits of its panel, which follow it in dispatch order on the same

@@ -61,6 +61,8 @@ __device__ inline void wino_store_tile(float* po, int W, int H, int ox, int oy, 
 // Joined splits: the splits of a panel add their partial tiles up inside the one launch.
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr unsigned kWinoEmpty = 0xffa5c3e1u;        // a signalling NaN: marks a workspace slot whose partial tile has not arrived
+struct WinoHelpers { int count, donated; };          // of an XCD; stages of 8 channels they take off each of its panels (k_winograd.hip)
+WinoHelpers wino_helpers(int nBlocks, int nChunks, int cus);
 constexpr int kWinoJoinSpins = 1 << 18;             // bound on the wait for a partner's partial tile (some 0.2 s)
 constexpr int kAuxThrough = 1 | 16;                 // cache policy of a buffer access: sc0 sc1, written through to memory
 constexpr int kAuxDeviceVolatile = 16 | (int)0x80000000u;   // sc1 (device scope: not served from this CU's vector cache), reloaded every time

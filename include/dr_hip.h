@@ -264,6 +264,9 @@ size_t drhip_conv3x3_winograd_workspace_floats(int W, int H, int I, int O, int v
  * then the rest halved, quartered ... over the input channels (joined as above) so that every unit gets the same
  * number of channel stages; the number of splits then differs per block and is not the caller's to choose.
  * Environment DR_WINO_TIERS=0 keeps pick_variant from returning it.
+ * 0x2c01 ("helpers", eight waves, 32 channels per workgroup): compute units without a block of their own take the last
+ * channels of the others' blocks and leave partial tiles in the (prepared) workspace; for shapes with fewer blocks than
+ * compute units and long enough channel loops, refused for others.
  * No counterpart in the reference: its kernel never splits the channel sum (Kernels/dR_winograd2.cl:176-189). */
 int drhip_conv3x3_winograd_workspace_prepare_f32(float* workspace, size_t floats, void* stream);
 int drhip_conv3x3_winograd_join_timeouts(unsigned* count);

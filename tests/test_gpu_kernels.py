@@ -703,6 +703,50 @@ def test_winograd_tiered_splits(lib, dev, oracle, variant, W, H, I, O):
         assert lib.drhip_conv3x3_winograd_f32(xd, U, bd, out, W, H, I, O, 1, variant, None, None) == -1
 
 
+@pytest.mark.parametrize("W,H,I,O", [
+    (8, 8, 64, 32),          # one panel: its XCD has 31 helpers for it
+    (9, 7, 67, 40), (13, 9, 130, 33), (2, 2, 128, 300),     # ragged tiles, channels and outputs
+    (64, 40, 128, 224),      # 140 panels, two of an XCD's 18 for most of its 14 helpers
+    (52, 52, 250, 256),      # 176: three each
+    (56, 56, 256, 256),      # 200: four, the last XCD has none of its own in part
+])
+def test_winograd_helpers(lib, dev, oracle, W, H, I, O):
+    """Variant 0x2c01: CUs without a panel take the last stages of the others' panels.  As for the tiered splits."""
+    variant = 0x2c01
+    x, w, b = rnd(I, H, W), rnd(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I))), rnd(O, scale=0.01)
+    U, _ = wino_filters(lib, dev, w)
+    xd, bd = dev.put(x), dev.put(b)
+    out = dev.empty(O * H * W)
+    n = lib.drhip_conv3x3_winograd_workspace_floats(W, H, I, O, variant)
+    assert n == -(-(-(-W // 2) * -(-H // 2)) // 32) * -(-O // 32) * 4096
+    ws = wino_workspace(lib, dev, W, H, I, O, variant)
+    want = oracle.conv_winograd(x, w, b, relu=True)
+    first = None
+    for _ in range(3):
+        ok(lib, lib.drhip_fill_f32(out, 7.0, O * H * W, None))
+        ok(lib, lib.drhip_conv3x3_winograd_f32(xd, U, bd, out, W, H, I, O, 1, variant, ws, None))
+        got = dev.get(out, want.shape)
+        assert_close(got, want, floor=float(np.abs(b).max()))
+        first = got if first is None else first
+        assert np.array_equal(got, first)
+        assert np.all(dev.get(ws, (n,)).view(np.uint32) == 0xffa5c3e1)
+    assert_close(first, oracle.conv_f64(x, w, b, relu=True), floor=float(np.abs(b).max()))
+    if W % 2 == 0 and H % 2 == 0:
+        pooled = dev.empty(O * H * W // 4)
+        ok(lib, lib.drhip_conv3x3_winograd_f32(xd, U, bd, pooled, W, H, I, O, 1 | 2, variant, ws, None))
+        assert np.array_equal(dev.get(pooled, (O, H // 2, W // 2)), oracle.pool(first, (2, 2, 1), (2, 2, 1), 0))
+    ok(lib, lib.drhip_conv3x3_winograd_f32(xd, U, None, out, W, H, I, O, 0, variant, ws, None))
+    assert_close(dev.get(out, want.shape), oracle.conv_winograd(x, w, None, relu=False))
+    late = ctypes.c_uint(123)
+    ok(lib, lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)))
+    assert late.value == 0
+    assert lib.drhip_conv3x3_winograd_f32(xd, U, bd, out, W, H, I, O, 1, variant, None, None) == -1
+    # too short to share, or more panels than one round of the CUs: refused
+    for shape in ((W, H, 24, O), (112, 112, 256, 256)):
+        assert lib.drhip_conv3x3_winograd_workspace_floats(*shape, variant) == 0
+        assert lib.drhip_conv3x3_winograd_f32(xd, U, bd, out, *shape, 1, variant, ws, None) == -1
+
+
 def test_winograd_tiered_refused_combinations(lib, dev):
     p = dev.empty(64)
     for variant in (0x1001, 0x1901, 0x1c01, 0x1811, 0x1803, 0x2801):     # not joined, 16-tile blocks, two wave sets, split bits, 128 channels, unknown bit

@@ -736,6 +736,15 @@ def test_split_winograd_workspace_holds_pieces_only(lib):
         assert floats(0x100 | nA << 20 | sA << 12 | sB << 16) == slots * 8 * 8192, (nA, sA, sB)
 
 
+@pytest.mark.parametrize("W,H,I,O,variant", [
+    (56, 56, 256, 256, 0x2c01), (56, 56, 128, 256, 0x401),          # 200 panels: helpers, or too few stages for them
+    (48, 48, 128, 256, 0x2c01), (46, 46, 64, 256, 0x401),           # 144, 136 panels: no halves of them
+    (34, 32, 256, 256, 0xc11), (34, 32, 128, 256, 0xc11), (34, 32, 64, 256, 0x101),     # 72 panels: halves, or the 16-tile form
+    (36, 36, 256, 96, 0x821), (14, 14, 512, 512, 0x831), (28, 28, 512, 512, 0xc11), (56, 56, 64, 64, 0x501)])
+def test_winograd_variant_by_panels_and_stages(lib, W, H, I, O, variant):
+    assert lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O) == variant
+
+
 @pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
 def test_interleaved_to_planes(lib, pixels, channels):
     a = np.random.default_rng(0).standard_normal((pixels, channels)).astype(np.float32)
