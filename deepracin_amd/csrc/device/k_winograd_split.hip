@@ -607,12 +607,12 @@ extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, in
         const int S = std::min(4, cusPerXcd / n), old = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
         if (!(old & 0x100)) {                           // (layers of its 16-tile form are too small)
             const int lg = old >> 4 & 15, panels32 = p.s.nTB * ceil_div(O, 32);
-            // (narrow maps and maps with both sides odd keep their pieces although helpers are faster there too, 33x31 256->512 19.7 / 17.0:
-            // they are what pieces are tested with, in two graphs at once and on their own)
-            const int helped = old & 0x2000 && wide && !(W & H & 1) ? wino_helpers(panels32, ceil_div(I, 8), cusPerXcd).donated : 0;
-            const double stages = (double)ceil_div(2 * nC - helped, 1 << lg) * ceil_div(panels32 << lg, cus);
-            // (with helpers: 48x48 256->256 pieces here 18.6, there 16.2; 512->256 27.5 / 27.2, 36x36 512->512 31.5 / 30.2, 40x40 512->512 33.6 / 33.9)
-            if (2.75 * ceil_div(ceil_div(nC, S), 2) + 10.6 < (helped ? 0.97 : 0.93) * (0.56 * stages + (lg > 0 ? 4.5 : 3)))
+            // Where panels of one round leave CUs idle, that kernel's helpers make it as fast as the pieces or faster (48x48 256->256 pieces 18.6,
+            // helpers 16.1 us; 512->256 27.5 / 27.2), but pieces are more exact (error against 64 bits, rms, 2.4e-7 and 3.0e-7): they stay where
+            // they are faster than that kernel by itself, with halves or quarters below 5/8 of the CUs.
+            const bool few = lg == 0 && 8 * panels32 < 5 * cus;
+            const double stages = few && nC >= 32 && O >= 64 ? 1.5 * nC : (double)ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus);
+            if (2.75 * ceil_div(ceil_div(nC, S), 2) + 10.6 < 0.93 * (0.56 * stages + (lg > 0 || few ? 4.5 : 3)))
                 if (const int v = split(0x101, 0, S, S)) return v;
         }
     }
