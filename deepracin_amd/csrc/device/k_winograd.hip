@@ -357,6 +357,9 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         const __amdgpu_buffer_rsrc_t rHelp = __builtin_amdgcn_make_buffer_rsrc((void*)ws, 0, 0x7ffffff0, kBufferFlags);
         const int helpRegion = (int)(4u * (unsigned)logical * (unsigned)(OB * TB * 4));
         u32x4 helped[OB / EO];
+        // (stores take the whole offset in the vector register: with the region in the scalar one the compiler lets the next vector instruction
+        // overwrite the data of a 16-byte store, and on gfx950 the store then now and then takes the new value)
+        auto help_slot = [&](int ol) { return helpRegion + 16 * (ol * TB + (tid & 31)); };
         auto ask_helper = [&] {
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -411,7 +414,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             if constexpr (kHelping) {
 #pragma unroll
                 for (int q = 0; q < OB / EO; ++q)
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(eo + EO * q)), rHelp, (int)(16u * (unsigned)((eo + EO * q) * TB + et)), helpRegion, kAuxThrough);
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(eo + EO * q)), rHelp, help_slot(eo + EO * q), 0, kAuxThrough);
                 // (the next panel's sums go where these were)
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
                 __builtin_amdgcn_s_barrier();
@@ -434,14 +437,14 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             // (tiered: a workgroup's partial tiles lie at its own index in the grid, its partners' 8 workgroups apart)
             const unsigned region0 = tiered ? blockIdx.x - (unsigned)(kXcds * split) : (unsigned)logical;
             const unsigned regionStep = tiered ? (unsigned)kXcds : (unsigned)nBlocks;
-            // byte address of a slot = region of the split (scalar offset) + place of the tile in the panel (per lane)
+            // byte address of a slot = region of the split + place of the tile in the panel (per lane; of a store together, see above)
             auto region_of = [&](int sp) { return (int)(4u * (region0 + (unsigned)sp * regionStep) * panelFloats); };
             auto place_of = [&](int ol) { return (int)(16u * (unsigned)(ol * TB + et)); };
 #pragma unroll
             for (int q = 0; q < OB / EO; ++q) {
                 const int ol = eo + EO * q;
                 if ((ol >> lgRows) == split) continue;
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(ol)), rWs, place_of(ol), region_of(split), kAuxThrough);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(ol)), rWs, place_of(ol) + region_of(split), 0, kAuxThrough);
             }
             const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
             // (the number of splits as a constant: every access below is unconditional.  The slot of the own split is
@@ -470,7 +473,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
 #pragma unroll
                     for (int u = 0; u < S; ++u) s += (u == split) ? own : __builtin_bit_cast(f32x4, part[u]);
 #pragma unroll
-                    for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, place_of(ol), region_of(u), kAuxThrough);
+                    for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, place_of(ol) + region_of(u), 0, kAuxThrough);
                     if (!ready) {                       // a partner never delivered: say so in the result and in the counter
                         s = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
                         atomicAdd(&g_wino_join_timeouts, 1u);
@@ -504,7 +507,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             for (int spins = 0; spins < kWinoJoinSpins && !arrived; ++spins) { ask_helper(); arrived = all_here(); }
             const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
 #pragma unroll
-            for (int q = 0; q < OB / EO; ++q) __builtin_amdgcn_raw_buffer_store_b128(empty, rHelp, (int)(16u * (unsigned)((eo + EO * q) * TB + et)), helpRegion, kAuxThrough);
+            for (int q = 0; q < OB / EO; ++q) __builtin_amdgcn_raw_buffer_store_b128(empty, rHelp, help_slot(eo + EO * q), 0, kAuxThrough);
             if (!arrived) atomicAdd(&g_wino_join_timeouts, 1u);
         }
 #pragma unroll
