@@ -26,6 +26,7 @@
 // waits for the other splits' partial tiles by watching the workspace slots themselves.
 #include "wino_common.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <type_traits>
@@ -148,7 +149,7 @@ __device__ inline f32x4 buf_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, un
 template <int NT, int KW, bool FEWC = false, bool HELP = false>
 __global__ void __launch_bounds__(kWinoThreads * KW, KW == 2 ? 1 : (NT == 1 ? 3 : (NT == 2 ? 2 : 1)))
 winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__ U, const float* __restrict__ bias,
-                         WINO_ARGS, float* __restrict__ out, float* __restrict__ ws) {
+                         WINO_ARGS, float* __restrict__ out, float* __restrict__ ws, int joinSpins) {
     constexpr int TB = 32, OB = 32 * NT, KC = kWinoKC;
     WINO_UNPACK(TB, OB)
     extern __shared__ float P[];                    // epilogue only: [KW sets][4 rows][2][OB o][32 t] floats
@@ -422,7 +423,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                 return;
             }
         }
-        if (!HELP && joined && nSp > 1) {
+        if (!HELP && !FEWC && joined && nSp > 1) {      // (a single stage is not cut)
             // (the partial tiles go out and are looked for at the highest priority: the other workgroups on this CU
             // are in their channel loops, and a wave at their priority gets an issue slot only when they stall)
             if (tiered) __builtin_amdgcn_s_setprio(3);
@@ -449,6 +450,8 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
             // (the number of splits as a constant: every access below is unconditional.  The slot of the own split is
             // read and reset like the others - nobody ever writes it - and its content replaced by the own tile.)
+            bool asked = false;
+            unsigned givenUp = 0;
             auto collect = [&](auto nSplitsConst) {
                 constexpr int S = decltype(nSplitsConst)::value;
 #pragma unroll
@@ -458,7 +461,8 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                     const f32x4 own = tile_of(ol);
                     u32x4 part[S];
                     bool ready = false;
-                    for (int spins = 0; spins < kWinoJoinSpins && !ready; ++spins) {
+                    for (int spins = 0; spins <= joinSpins && !ready; ++spins) {
+                        if (spins == joinSpins) wino_gives_up(&g_wino_join_timeouts);
                         // (the loads are invariant as far as the compiler can see: without this it issues them once,
                         // in front of the loop)
                         asm volatile("" ::: "memory");
@@ -467,17 +471,17 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                         for (int u = 0; u < S; ++u) part[u] = __builtin_amdgcn_raw_buffer_load_b128(rWs, place_of(ol), region_of(u), kAuxDeviceVolatile);
 #pragma unroll
                         for (int u = 0; u < S; ++u)
-                            ready = ready && (u == split || (part[u][0] != kWinoEmpty && part[u][1] != kWinoEmpty && part[u][2] != kWinoEmpty && part[u][3] != kWinoEmpty));
+                            ready = ready && (u == split || wino_slot_full(part[u]));
                     }
+                    // (what was looked for has come behind the own stores: they have arrived, and this waits for nothing)
+                    if (!asked) { givenUp = wino_given_up(&g_wino_join_timeouts); asked = true; }
                     f32x4 s = {0.f, 0.f, 0.f, 0.f};     // splits added in order, like winograd_split_reduce_kernel
 #pragma unroll
                     for (int u = 0; u < S; ++u) s += (u == split) ? own : __builtin_bit_cast(f32x4, part[u]);
 #pragma unroll
                     for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, place_of(ol) + region_of(u), 0, kAuxThrough);
-                    if (!ready) {                       // a partner never delivered: say so in the result and in the counter
-                        s = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
-                        atomicAdd(&g_wino_join_timeouts, 1u);
-                    }
+                    // a partner never delivered: it shows in the result, too
+                    if (!ready) s = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
                     if (eTileOk && o < O) {
                         if (bias) s += kBiasEarly ? biasEarly[kBiasEarly ? q : 0] : bias[o];
                         if (relu & kEpiRelu) { s[0] = fmaxf(s[0], 0.f); s[1] = fmaxf(s[1], 0.f); s[2] = fmaxf(s[2], 0.f); s[3] = fmaxf(s[3], 0.f); }
@@ -493,6 +497,13 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             else if (lgSp == 2) collect(std::integral_constant<int, 4>{});
             else if (lgSp == 3) collect(std::integral_constant<int, 8>{});
             else collect(std::integral_constant<int, 16>{});
+            if (!asked) givenUp = wino_given_up(&g_wino_join_timeouts);
+            if (__builtin_expect(givenUp != 0, 0)) {
+                int spins = joinSpins;
+#pragma clang loop unroll(disable)
+                for (int q = 0; q < OB / EO; ++q)
+                    if (((eo + EO * q) >> lgRows) != split) wino_see_off(rWs, place_of(eo + EO * q) + region_of(split), spins);
+            }
             return;
         }
         bool arrived = true;
@@ -500,15 +511,18 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
             auto all_here = [&] {
                 bool r = true;
 #pragma unroll
-                for (int q = 0; q < OB / EO; ++q) r = r && helped[q][0] != kWinoEmpty && helped[q][1] != kWinoEmpty && helped[q][2] != kWinoEmpty && helped[q][3] != kWinoEmpty;
+                for (int q = 0; q < OB / EO; ++q) r = r && wino_slot_full(helped[q]);
                 return r;
             };
             arrived = all_here();
-            for (int spins = 0; spins < kWinoJoinSpins && !arrived; ++spins) { ask_helper(); arrived = all_here(); }
+            for (int spins = 0; spins <= joinSpins && !arrived; ++spins) {
+                if (spins == joinSpins) wino_gives_up(&g_wino_join_timeouts);
+                ask_helper();
+                arrived = all_here();
+            }
             const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
 #pragma unroll
             for (int q = 0; q < OB / EO; ++q) __builtin_amdgcn_raw_buffer_store_b128(empty, rHelp, help_slot(eo + EO * q), 0, kAuxThrough);
-            if (!arrived) atomicAdd(&g_wino_join_timeouts, 1u);
         }
 #pragma unroll
         for (int q = 0; q < OB / EO; ++q) {
@@ -543,15 +557,25 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
     // gained nothing.)
     if constexpr (HELP) {
         if (helper) {
+            const int first = logical;
             for (;;) {                                  // every nSplits-th panel of the XCD
                 rest_of_kernel(std::true_type{}, std::true_type{});
                 inXcd += nSplits;
                 logical += nSplits;
-                if (inXcd >= perXcd || logical >= nBlocks) return;
+                if (inXcd >= perXcd || logical >= nBlocks) break;
                 oBlock = fast_div(logical, nTBd);
                 o0 = oBlock * OB;
                 t0 = (logical - oBlock * (int)nTBd.d) * TB;
             }
+            if (__builtin_expect(wino_given_up(&g_wino_join_timeouts) != 0, 0)) {
+                const __amdgpu_buffer_rsrc_t rHelp = __builtin_amdgcn_make_buffer_rsrc((void*)ws, 0, 0x7ffffff0, kBufferFlags);
+                int spins = joinSpins;
+#pragma clang loop unroll(disable)
+                for (int panel = first; panel < logical; panel += nSplits)
+#pragma clang loop unroll(disable)
+                    for (int i = (int)threadIdx.x; i < OB * TB; i += kWinoThreads * KW) wino_see_off(rHelp, 16 * (panel * OB * TB + i), spins);
+            }
+            return;
         }
     }
     if constexpr (KW == 2) {
@@ -919,6 +943,13 @@ WinoHelpers wino_helpers(int nBlocks, int nChunks, int cus) {
 // panel-sized region per workgroup of the grid.
 constexpr int kEpiAvgPool2 = 4;     // (inside this file: of the kernels for images)
 
+// Some 0.2 s; DR_WINO_JOIN_SPINS for tests of what a launch leaves behind whose pieces did not wait.
+int wino_join_spins() {
+    const char* e = getenv("DR_WINO_JOIN_SPINS");
+    const int n = e ? atoi(e) : 0;
+    return n > 0 ? std::min(n, 1 << 18) : 1 << 18;
+}
+
 template <int NT, int TB>
 static int launch_wino(const float* in, const float* U, const float* bias, float* out, float* workspace,
                        int W, int H, int I, int O, int relu, const WinoCfg& c, hipStream_t s) {
@@ -935,7 +966,7 @@ static int launch_wino(const float* in, const float* U, const float* bias, float
             static_assert(4 * 2 * OB * TB * sizeof(float) * 2 <= 65536, "no more LDS than any launch may have");
             launch((winograd_f23_mfma_kernel<1, 2, false, true>), dim3(gridX + h.count * kXcds), dim3(2 * kWinoThreads), 2 * ldsBytes, s, in, U, bias,
                    (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dx.mul, dtb.mul,
-                   dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | (unsigned)h.count << 13, (unsigned)h.donated << 16, out, workspace);
+                   dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | (unsigned)h.count << 13, (unsigned)h.donated << 16, out, workspace, wino_join_spins());
             return launched("winograd_f23_mfma_kernel");
         }
     }
@@ -946,7 +977,7 @@ static int launch_wino(const float* in, const float* U, const float* bias, float
             for (int k = 0; k < t.count; ++k) { lgs |= (unsigned)t.lg[k] << (4 * k); counts |= (unsigned)t.n[k] << (8 * k); }
             launch((winograd_f23_mfma_kernel<NT, 1>), dim3(t.wgsPerXcd * kXcds), dim3(kWinoThreads), ldsBytes, s, in, U, bias,
                    (unsigned)W | (unsigned)H << 16, (unsigned)I | (unsigned)O << 16, dx.mul, dtb.mul,
-                   dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | lgs << 13 | 3u << 30, counts, out, workspace);
+                   dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | lgs << 13 | 3u << 30, counts, out, workspace, wino_join_spins());
             return launched("winograd_f23_mfma_kernel");
         }
     }
@@ -954,6 +985,7 @@ static int launch_wino(const float* in, const float* U, const float* bias, float
                                dx.shift | dtb.shift << 5 | (unsigned)(relu & 3) << 10 | (unsigned)vec2 << 12 | (unsigned)g.splits << 13 |
                                    (relu & kEpiAvgPool2 ? 1u << 29 : 0u) | (joined ? 1u << 31 : 0u),
                                (unsigned)g.chunksPerSplit | (joined ? (unsigned)__builtin_ctz(g.splits) << 24 : 0u)};
+    const int spins = joined ? wino_join_spins() : 0;
     // joined: one grid row, the splits of a panel side by side on one XCD (see the kernel)
     const dim3 grid = joined ? dim3(gridX * g.splits) : dim3(gridX, g.splits);
     if constexpr (TB == 32) {
@@ -974,16 +1006,16 @@ static int launch_wino(const float* in, const float* U, const float* bias, float
             }
             if (c.waveSets == 2)
                 launch((winograd_f23_mfma_kernel<NT, 2>), grid, dim3(2 * kWinoThreads), 2 * ldsBytes, s,
-                       in, U, bias, pa.wh, pa.io, pa.mulX, pa.mulTB, pa.cfg0, pa.cfg1, out, workspace);
+                       in, U, bias, pa.wh, pa.io, pa.mulX, pa.mulTB, pa.cfg0, pa.cfg1, out, workspace, spins);
         }
         if (c.waveSets != 2 || NT > 2) {
             if (NT <= 2 && I <= 4 && g.splits == 1) {       // an image: the stage without its two empty k-steps
                 if constexpr (NT <= 2)
                     launch((winograd_f23_mfma_kernel<NT, 1, true>), grid, dim3(kWinoThreads), ldsBytes, s,
-                           in, U, bias, pa.wh, pa.io, pa.mulX, pa.mulTB, pa.cfg0, pa.cfg1, out, workspace);
+                           in, U, bias, pa.wh, pa.io, pa.mulX, pa.mulTB, pa.cfg0, pa.cfg1, out, workspace, spins);
             } else
                 launch((winograd_f23_mfma_kernel<NT, 1>), grid, dim3(kWinoThreads), ldsBytes, s,
-                       in, U, bias, pa.wh, pa.io, pa.mulX, pa.mulTB, pa.cfg0, pa.cfg1, out, workspace);
+                       in, U, bias, pa.wh, pa.io, pa.mulX, pa.mulTB, pa.cfg0, pa.cfg1, out, workspace, spins);
         }
     } else if (c.waveSets == 2)
         launch((winograd_f23_mfma16_kernel<NT, 2>), grid, dim3(2 * kWinoThreads), 2 * ldsBytes, s,

@@ -50,6 +50,7 @@ struct WsShape {                            // everything but the pointers; by v
     // The first nA output panels of an XCD are cut into sA splits of perA chunks (in nA * sA workgroups), the others into sB of
     // perB; mulA, mulB: division by sA and sB
     int wgsA, nA, sA, sB, perA, perB, mulA, mulB;
+    int joinSpins;
 };
 
 __device__ unsigned g_ws_join_timeouts;     // partial tiles that never arrived, over the life of the process
@@ -392,7 +393,8 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
 #pragma unroll
             for (int i = 0; i < C; ++i) own[i] = tile_of(eo + EO * (q0 + min(i, count - 1)));
             bool ready = false;
-            for (int spins = 0; spins < kWinoJoinSpins && !ready; ++spins) {
+            for (int spins = 0; spins <= s.joinSpins && !ready; ++spins) {
+                if (spins == s.joinSpins) wino_gives_up(&g_ws_join_timeouts);
                 asm volatile("" ::: "memory");          // (to the compiler these loads are invariant)
                 ready = true;
 #pragma unroll
@@ -403,8 +405,9 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                 for (int i = 0; i < C; ++i)
 #pragma unroll
                     for (int u = 0; u < S; ++u)
-                        ready = ready && (u == split || (part[i][u][0] != kWinoEmpty && part[i][u][1] != kWinoEmpty && part[i][u][2] != kWinoEmpty && part[i][u][3] != kWinoEmpty));
+                        ready = ready && (u == split || wino_slot_full(part[i][u]));
             }
+            const unsigned givenUp = wino_given_up(&g_ws_join_timeouts);    // (waits for nothing: the parts have come behind the own stores)
 #pragma unroll
             for (int i = 0; i < C; ++i) {
                 if (i >= count) continue;
@@ -415,12 +418,17 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
 #pragma unroll
                 for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, slot_of(u, q), 0, kAuxThrough);
                 note(q, y);
-                if (!ready) {                           // a partner never delivered: say so in the result and in the counter
+                if (!ready) {                           // a partner never delivered: it shows in the result, too
                     y = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
                     again &= ~(1u << q);
-                    atomicAdd(&g_ws_join_timeouts, 1u);
                 }
                 if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2, kSplitUnscale);
+            }
+            if (__builtin_expect(givenUp != 0, 0)) {
+                int spins = s.joinSpins;
+#pragma clang loop unroll(disable)
+                for (int q = 0; q < NP; ++q)
+                    if (q < q0 || q >= q0 + count) wino_see_off(rWs, slot_of(split, q), spins);
             }
         };
         if (KW == 1 || nSp == 2) join(integral_constant<int, 2>{});
@@ -653,6 +661,7 @@ extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U,
     DRHIP_REQUIRE(ws_plan(W, H, I, O, variant, &p), "drhip_conv3x3_winograd_split_f32: variant %#x does not cover %dx%dx%d -> %d", variant, W, H, I, O);
     DRHIP_REQUIRE(workspace || (p.s.sA == 1 && p.s.sB == 1), "drhip_conv3x3_winograd_split_f32: variant %#x joins splits and needs a prepared workspace", variant);
     p.s.flags = flags;
+    p.s.joinSpins = p.s.sA == 1 && p.s.sB == 1 ? 0 : wino_join_spins();
     p.s.vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
     const unsigned short* F = (const unsigned short*)U;
     hipStream_t st = as_stream(stream);

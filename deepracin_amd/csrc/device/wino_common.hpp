@@ -63,10 +63,34 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr unsigned kWinoEmpty = 0xffa5c3e1u;        // a signalling NaN: marks a workspace slot whose partial tile has not arrived
 struct WinoHelpers { int count, donated; };          // of an XCD; stages of 8 channels they take off each of its panels (k_winograd.hip)
 WinoHelpers wino_helpers(int nBlocks, int nChunks, int cus);
-constexpr int kWinoJoinSpins = 1 << 18;             // bound on the wait for a partner's partial tile (some 0.2 s)
 constexpr int kAuxThrough = 1 | 16;                 // cache policy of a buffer access: sc0 sc1, written through to memory
 constexpr int kAuxDeviceVolatile = 16 | (int)0x80000000u;   // sc1 (device scope: not served from this CU's vector cache), reloaded every time
 int ws_join_timeouts(unsigned* count);              // of the split-operand kernel
+int wino_join_spins();                              // bound on the wait for a partner's partial tile
+
+// Nothing of a launch may lie in its workspace when the launch has ended: the next one would take a partial tile that came too
+// late for its own panel.  Whoever gives a tile up adds to the kernel's counter first and looks once more behind that; whoever has stored
+// tiles reads the counter once they have arrived.  So either the last look finds the tile, or its writer finds the counter not zero.
+// From then on (the counter never goes back) writers see their tiles off: they wait until the reader has put the marker back and
+// do it themselves where it does not.  Both sides are on one XCD, whose L2 orders the two.
+__device__ inline void wino_gives_up(unsigned* counter) {
+    atomicAdd(counter, 1u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+__device__ inline unsigned wino_given_up(unsigned* counter) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (the caller's tiles have arrived)
+    return __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool wino_slot_full(u32x4 v) { return v[0] != kWinoEmpty && v[1] != kWinoEmpty && v[2] != kWinoEmpty && v[3] != kWinoEmpty; }
+// (spins: for all slots of the caller together)
+__device__ inline void wino_see_off(__amdgpu_buffer_rsrc_t r, int at, int& spins) {
+    for (; spins > 0; --spins) {
+        asm volatile("" ::: "memory");
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, kAuxDeviceVolatile);
+        if (v[0] == kWinoEmpty && v[1] == kWinoEmpty && v[2] == kWinoEmpty && v[3] == kWinoEmpty) return;
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4{kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty}, r, at, 0, kAuxThrough);
+}
 
 constexpr int kEpiRelu = DRHIP_EPILOGUE_RELU, kEpiMaxPool2 = DRHIP_EPILOGUE_MAXPOOL2;   // bits of the `relu` argument
 

@@ -258,7 +258,10 @@ size_t drhip_conv3x3_winograd_workspace_floats(int W, int H, int I, int O, int v
  * it must not overlap.  drhip_conv3x3_winograd_f32 with variant 0 never picks a joined variant.  A partner that does
  * not deliver within the kernel's bounded wait (about 0.2 s: the device was shared so that the launch was not
  * resident as a whole) turns the affected outputs into NaN and is counted; drhip_conv3x3_winograd_join_timeouts
- * reads that count (a synchronous copy).  Environment DR_WINO_JOIN=0 keeps pick_variant from returning such variants.
+ * reads that count (a synchronous copy).  Tiles that come after that are taken out of the workspace before the launch ends, so
+ * that the next one finds it prepared all the same; from the first such wait of the process on, joined launches look after their tiles
+ * at the end, some microseconds each.  Environment DR_WINO_JOIN=0 keeps pick_variant from returning such variants, DR_WINO_JOIN_SPINS=n ends
+ * the waits of later launches after n looks (for tests).
  * Bit 0x1000 on top of 0x800 ("tiered", four waves, 32 or 64 channels per workgroup, split bits zero) lets the
  * launcher cut a layer whose blocks do not divide by the compute units into tiers: as many whole blocks per unit as fit,
  * then the rest halved, quartered ... over the input channels (joined as above) so that every unit gets the same
