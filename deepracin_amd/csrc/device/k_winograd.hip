@@ -1069,22 +1069,29 @@ extern "C" int drhip_conv3x3_winograd_pick_variant(int W, int H, int I, int O) {
     const int panels = ceil_div(T, 32) * ceil_div(O, code == 2 ? 64 : 32);
     const int nChunks = ceil_div(I, kWinoKC);
     int lg = 0;
+    // (half of a long layer on the CUs in part: it goes out as quarters of 64-channel panels, below, whose sums are half as long as those of
+    // whole panels with two wave sets.  Eight of them, 0x22 / helpers / whole: error against 64 bits 1 / 1.07 / 1.38, time 1 / 0.70 / 0.96)
+    const bool longHalves = code == 1 && 8 * panels < 5 * cus && O >= 64 && (nChunks >> 1) >= 32;
     // Panels for one round of the CUs and no halves of them: the CUs without one help the others.
-    if (code == 1 && 2 * panels > cus && wino_join_flag(1, 2) && wino_helpers(panels, nChunks, cus / kXcds).count) return 0x2c01;
+    if (code == 1 && 2 * panels > cus && !longHalves && wino_join_flag(1, 2) && wino_helpers(panels, nChunks, cus / kXcds).count) return 0x2c01;
     // (a split costs a second kernel: below 6 stages in all it does not pay, nor where the next cut is too fine to be joined in one round
-    // and this one is whole or can be joined.  us, with / without that cut: 46x46 64->256 10.2 / 7.4, 34x32 256->256 13.7 / 12.4,
-    // 36x36 256->96 9.8 / 8.4)
-    auto enough = [&] { return (panels << (lg + 1)) > cus && (lg == 0 || wino_join_flag(lg, nChunks)); };
-    while (lg < 5 && nChunks >= 6 && !enough() && (panels << lg) < (5 * cus) / 8 && (nChunks >> (lg + 1)) >= 2) ++lg;
+    // and this one is whole or can be joined: with two wave sets its sums are as long as the finer cut's.  Eight of each, finer / this one:
+    // 0x11 / 0x401 error 1 / 1.00, time 1 / 0.76; 0x21 / 0xc11 1.01, 0.91; 0x31 / 0xc21 0.97, 0.90; 0x41 / 0xc31 0.96, 0.87)
+    bool early = false;
+    while (lg < 5 && nChunks >= 6 && (panels << lg) < (5 * cus) / 8 && (nChunks >> (lg + 1)) >= 2) {
+        early = (panels << (lg + 1)) > cus && (lg == 0 ? !longHalves : wino_join_flag(lg, nChunks) != 0);
+        if (early) break;
+        ++lg;
+    }
     // At most one workgroup per CU and at least two stages for each wave set: eight waves per workgroup,
     // so that every SIMD still has two waves to alternate between (56x56 256->256: 23.6 vs 24.8 us;
     // 28x28 512->512 as 112 panels x 2 splits: 26.3 vs 26.9 us for 64-channel panels x 4 splits).
     // A split whose workgroups are all resident at once (one per CU) adds its partial tiles up inside the launch.
-    // (joined splits of fewer than 16 stages each, finer than halves: four waves, 14x14 512->512 as 8 splits: 10.4 vs 11.1 us, 36x36 256->96
-    // as 4 8.4 / 9.4; as halves 34x32 128->256 8.9 / 8.2, 192->256 11.0 / 10.1)
+    // (joined splits of fewer than 16 stages each, finer than halves: four waves, 14x14 512->512 as 8 splits: 10.4 vs 11.1 us; as halves
+    // 34x32 128->256 8.9 / 8.2, 192->256 11.0 / 10.1)
     if ((panels << lg) <= cus && (nChunks >> lg) >= 4) {
         const int join = wino_join_flag(lg, nChunks);
-        return ((join && lg > 1 && (nChunks >> lg) < 16) ? 0 : 0x400) | code | (lg << 4) | join;
+        return ((join && lg > 1 && !early && (nChunks >> lg) < 16) ? 0 : 0x400) | code | (lg << 4) | join;
     }
     // Unsplit layers with more 32-channel panels than CUs, but no multiple of them (112x112 128->128: 392 panels,
     // two on 136 CUs and one on 120): tiers of whole, halved, ... panels even the CUs out (in a replayed VGG16

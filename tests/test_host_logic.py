@@ -740,9 +740,22 @@ def test_split_winograd_workspace_holds_pieces_only(lib):
     (56, 56, 256, 256, 0x2c01), (56, 56, 128, 256, 0x401),          # 200 panels: helpers, or too few stages for them
     (48, 48, 128, 256, 0x2c01), (46, 46, 64, 256, 0x401),           # 144, 136 panels: no halves of them
     (34, 32, 256, 256, 0xc11), (34, 32, 128, 256, 0xc11), (34, 32, 64, 256, 0x101),     # 72 panels: halves, or the 16-tile form
-    (36, 36, 256, 96, 0x821), (14, 14, 512, 512, 0x831), (28, 28, 512, 512, 0xc11), (56, 56, 64, 64, 0x501)])
+    (36, 36, 256, 96, 0xc21), (14, 14, 512, 512, 0x831), (28, 28, 512, 512, 0xc11), (56, 56, 64, 64, 0x501)])
 def test_winograd_variant_by_panels_and_stages(lib, W, H, I, O, variant):
     assert lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O) == variant
+
+
+@pytest.mark.parametrize("W,H,I,O,variant,donated,finer", [
+    (131, 35, 384, 16, 0xc21, 0, 8), (44, 53, 479, 64, 0xc21, 0, 8), (8, 32, 285, 514, 0xc21, 0, 8),    # quarters where eighths would need a second round
+    (349, 5, 571, 5, 0xc31, 0, 16), (7, 268, 250, 3, 0xc31, 0, 16),                                     # eighths, sixteenths
+    (45, 79, 537, 138, 0x22, 0, 4), (188, 30, 627, 93, 0x22, 0, 4),                                     # 129 to 159 panels, long sums: quarters as they were
+    (188, 30, 500, 93, 0x2c01, 20, 2), (45, 386, 600, 1, 0x2c01, 24, 2), (46, 46, 64, 256, 0x401, 0, 2)])   # helpers or two wave sets where there were halves
+def test_sums_of_a_cut_are_as_short_as_the_finer_one_s(lib, W, H, I, O, variant, donated, finer):
+    """Stages of eight channels that one accumulator adds up: where a cut is not made because its pieces would not fit one round, or helpers
+    take its place, no more than with that cut."""
+    v, stages, div = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O), -(-I // 8), lambda a, b: -(-a // b)
+    assert v == variant
+    assert div(div(stages - donated, 1 << (v >> 4 & 15)), 2 if v & 0x400 else 1) <= div(stages, finer)
 
 
 @pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
