@@ -1051,16 +1051,19 @@ static int wino_join_flag(int lg, int nChunks) {
     return (enabled && lg >= 1 && lg <= 3 && (nChunks & ((1 << lg) - 1)) == 0) ? 0x800 : 0;
 }
 
-extern "C" int drhip_conv3x3_winograd_pick_variant(int W, int H, int I, int O) {
+// joins: a launch that joins splits or takes helpers may be picked.  (Without, the choice needs no larger workspace than with: the caller of
+// variant 0 has asked for that one.)
+static int wino_pick(int W, int H, int I, int O, bool joins) {
     const int T = ((W + 1) / 2) * ((H + 1) / 2);
     const int cus = num_cu();
     // Small layers (SqueezeNet's expand convolutions: <= 8 stages, a few dozen 32x32 panels) are bound
     // by the latency of one workgroup, not by throughput: 16x16 blocks, unsplit, one launch
     // (in a replayed launch graph 4.2-5.8 us per layer against 5.1-7.1 us for the 32x32 forms).
     // (Where they would need a second round of the CUs and halves of the 32x32 panels can be joined: those, from 10 stages on.
-    // 48x105 96->64 8.5 / 7.8, 34x32 128->256 10.2 / 8.2; with 8 stages 49x60 64->160 6.8 / 7.3)
+    // 48x105 96->64 8.5 / 7.8, 34x32 128->256 10.2 / 8.2; with 8 stages 49x60 64->160 6.8 / 7.3.  Halves in two launches, 0.91 to 1.13 times the
+    // 16-tile form over eight shapes, or whole panels, 1.05 to 1.17, are not what that rule is for)
     if (ceil_div(T, 32) * ceil_div(O, 32) < cus / 2 && ceil_div(I, kWinoKC) <= 16 &&
-        !(ceil_div(I, kWinoKC) > 8 && ceil_div(T, 16) * ceil_div(O, 16) > cus && wino_join_flag(1, ceil_div(I, kWinoKC))))
+        !(joins && ceil_div(I, kWinoKC) > 8 && ceil_div(T, 16) * ceil_div(O, 16) > cus && wino_join_flag(1, ceil_div(I, kWinoKC))))
         // 6+ stages and at most one workgroup per CU (14x14 maps; 56x56 64->64: 5.3 vs 5.5 us): two wave sets
         return (ceil_div(I, kWinoKC) >= 6 && ceil_div(T, 16) * ceil_div(O, 16) <= cus) ? 0x501 : 0x101;
     // (an image layer has next to no transform work to share, and twice the workgroups of half the size spread its
@@ -1110,6 +1113,8 @@ extern "C" int drhip_conv3x3_winograd_pick_variant(int W, int H, int I, int O) {
     if (code == 1 && lg >= 1 && lg < 5 && O >= 64 && (nChunks >> lg) >= 32) return 2 | ((lg + 1) << 4);
     return code | (lg << 4);
 }
+
+extern "C" int drhip_conv3x3_winograd_pick_variant(int W, int H, int I, int O) { return wino_pick(W, H, I, O, true); }
 
 extern "C" int drhip_conv3x3_winograd_workspace_prepare_f32(float* workspace, size_t floats, void* stream) {
     DRHIP_REQUIRE(workspace || floats == 0, "drhip_conv3x3_winograd_workspace_prepare_f32: NULL workspace");
@@ -1163,7 +1168,7 @@ extern "C" int drhip_conv3x3_winograd_f32(const float* in, const float* U, const
     DRHIP_REQUIRE((relu & ~(DRHIP_EPILOGUE_RELU | DRHIP_EPILOGUE_MAXPOOL2)) == 0, "drhip_conv3x3_winograd_f32: unknown epilogue flags %d", relu);
     DRHIP_REQUIRE(!(relu & DRHIP_EPILOGUE_MAXPOOL2) || ((W | H) & 1) == 0, "drhip_conv3x3_winograd_f32: the fused 2x2 max pool needs even W and H (got %dx%d)", W, H);
     if (variant == 0) {
-        variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
+        variant = wino_pick(W, H, I, O, false);
         if (variant & 0x2000) variant = 0x401;
         if (variant & 0x1000) variant = (variant & 0xf) == 2 ? 2 : 1;      // (joined splits need a prepared workspace: explicit variants only)
         variant &= ~0x800;

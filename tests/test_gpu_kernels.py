@@ -774,6 +774,24 @@ def test_winograd_auto_variant_vgg_shapes(lib, dev, oracle):
         dev.close()
 
 
+@pytest.mark.parametrize("W,H,I,O,split,whole", [
+    (34, 32, 128, 256, 0x101, 0x101), (20, 123, 124, 117, 0x101, 0x101),       # the 16-tile form, which joined halves beat and halves in two launches do not
+    (36, 36, 256, 96, 0x421, 0x401), (28, 28, 512, 512, 0x411, 0x401), (48, 48, 256, 256, 0x401, 0x401), (112, 112, 128, 128, 1, 1)])
+def test_winograd_variant_0_joins_nothing(lib, dev, W, H, I, O, split, whole):
+    """Variant 0 takes the best form without joins, with a workspace (that of the picked variant is enough) or without: the same bits."""
+    U, _ = wino_filters(lib, dev, own(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I))))
+    xd, y = dev.put(own(I, H, W)), dev.empty(O * H * W)
+    n = lib.drhip_conv3x3_winograd_workspace_floats(W, H, I, O, lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O))
+    assert lib.drhip_conv3x3_winograd_workspace_floats(W, H, I, O, split) <= n
+    ws = dev.empty(max(n, 1))
+
+    def run(variant, workspace):
+        ok(lib, lib.drhip_conv3x3_winograd_f32(xd, U, None, y, W, H, I, O, 0, variant, workspace, None))
+        return dev.get(y, (O, H, W))
+
+    assert np.array_equal(run(0, ws), run(split, ws)) and np.array_equal(run(0, None), run(whole, None))
+
+
 def test_winograd_rejects_bad_arguments(lib, dev):
     p = dev.empty(64)
     assert lib.drhip_conv3x3_winograd_f32(p, p, None, p, 0, 4, 1, 1, 0, 0, None, None) == -1
