@@ -1051,6 +1051,23 @@ static int wino_join_flag(int lg, int nChunks) {
     return (enabled && lg >= 1 && lg <= 3 && (nChunks & ((1 << lg) - 1)) == 0) ? 0x800 : 0;
 }
 
+// Layers whose 32x32 panels leave half of the CUs without one and that are not long.
+static bool wino_small(int T, int nChunks, int O, int cus) { return ceil_div(T, 32) * ceil_div(O, 32) < cus / 2 && nChunks <= 16; }
+// Whether 2^lg splits are to be cut once more: fewer workgroups than 5/8 of the CUs, and at least two stages in each.
+static bool wino_cut_more(int panels, int lg, int nChunks, int cus) {
+    return lg < 5 && nChunks >= 6 && (panels << lg) < (5 * cus) / 8 && (nChunks >> (lg + 1)) >= 2;
+}
+
+int drhip::wino_halvings(int W, int H, int I, int O) {
+    const int T = ((W + 1) / 2) * ((H + 1) / 2), nChunks = ceil_div(I, kWinoKC), cus = num_cu();
+    if (wino_small(T, nChunks, O, cus)) return -1;
+    const bool wide = O > 32 && T >= 8192 && I > 4;
+    const int panels = ceil_div(T, 32) * ceil_div(O, wide ? 64 : 32);
+    int lg = 0;
+    while (wino_cut_more(panels, lg, nChunks, cus)) ++lg;
+    return !wide && lg >= 1 && lg < 5 && O >= 64 && (panels << lg) > cus && (nChunks >> lg) >= 32 ? lg + 1 : lg;
+}
+
 // joins: a launch that joins splits or takes helpers may be picked.  (Without, the choice needs no larger workspace than with: the caller of
 // variant 0 has asked for that one.)
 static int wino_pick(int W, int H, int I, int O, bool joins) {
@@ -1062,7 +1079,7 @@ static int wino_pick(int W, int H, int I, int O, bool joins) {
     // (Where they would need a second round of the CUs and halves of the 32x32 panels can be joined: those, from 10 stages on.
     // 48x105 96->64 8.5 / 7.8, 34x32 128->256 10.2 / 8.2; with 8 stages 49x60 64->160 6.8 / 7.3.  Halves in two launches, 0.91 to 1.13 times the
     // 16-tile form over eight shapes, or whole panels, 1.05 to 1.17, are not what that rule is for)
-    if (ceil_div(T, 32) * ceil_div(O, 32) < cus / 2 && ceil_div(I, kWinoKC) <= 16 &&
+    if (wino_small(T, ceil_div(I, kWinoKC), O, cus) &&
         !(joins && ceil_div(I, kWinoKC) > 8 && ceil_div(T, 16) * ceil_div(O, 16) > cus && wino_join_flag(1, ceil_div(I, kWinoKC))))
         // 6+ stages and at most one workgroup per CU (14x14 maps; 56x56 64->64: 5.3 vs 5.5 us): two wave sets
         return (ceil_div(I, kWinoKC) >= 6 && ceil_div(T, 16) * ceil_div(O, 16) <= cus) ? 0x501 : 0x101;
@@ -1081,7 +1098,7 @@ static int wino_pick(int W, int H, int I, int O, bool joins) {
     // and this one is whole or can be joined: with two wave sets its sums are as long as the finer cut's.  Eight of each, finer / this one:
     // 0x11 / 0x401 error 1 / 1.00, time 1 / 0.76; 0x21 / 0xc11 1.01, 0.91; 0x31 / 0xc21 0.97, 0.90; 0x41 / 0xc31 0.96, 0.87)
     bool early = false;
-    while (lg < 5 && nChunks >= 6 && (panels << lg) < (5 * cus) / 8 && (nChunks >> (lg + 1)) >= 2) {
+    while (wino_cut_more(panels, lg, nChunks, cus)) {
         early = (panels << (lg + 1)) > cus && (lg == 0 ? !longHalves : wino_join_flag(lg, nChunks) != 0);
         if (early) break;
         ++lg;

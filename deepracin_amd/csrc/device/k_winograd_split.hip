@@ -612,17 +612,14 @@ extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, in
         return ws_plan(W, H, I, O, v, &p) ? v : 0;
     };
     if (joins && 2 * n <= cusPerXcd) {
-        const int S = std::min(4, cusPerXcd / n), old = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
-        if (!(old & 0x100)) {                           // (layers of its 16-tile form are too small)
-            const int lg = old >> 4 & 15, panels32 = p.s.nTB * ceil_div(O, 32);
-            // Where panels of one round leave CUs idle, that kernel's helpers make it as fast as the pieces or faster (48x48 256->256 pieces 18.6,
-            // helpers 16.1 us; 512->256 27.5 / 27.2), but pieces are more exact (error against 64 bits, rms, 2.4e-7 and 3.0e-7): they stay where
-            // they are faster than that kernel by itself, with halves or quarters below 5/8 of the CUs.
-            const bool few = lg == 0 && 8 * panels32 < 5 * cus;
-            const double stages = few && nC >= 32 && O >= 64 ? 1.5 * nC : (double)ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus);
-            if (2.75 * ceil_div(ceil_div(nC, S), 2) + 10.6 < 0.93 * (0.56 * stages + (lg > 0 || few ? 4.5 : 3)))
-                if (const int v = split(0x101, 0, S, S)) return v;
-        }
+        // Against the fp32 kernel in equal splits and two launches, although its joined halves and helpers may be up to 1.2 times as fast as the
+        // pieces: the pieces are more exact than those (error against 64 bits, 0.70 of joined halves' and 0.86 of helpers' over 15 shapes)
+        // and stay where they gain on a form whose sums are as short.  And against what that kernel takes, where that is the slower one.
+        const int S = std::min(4, cusPerXcd / n), halvings = wino_halvings(W, H, I, O), panels32 = p.s.nTB * ceil_div(O, 32);
+        auto fp32 = [&](int lg) { return 0.56 * ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus) + (lg > 0 ? 4.5 : 3); };
+        if (halvings >= 0 &&                            // (layers of its 16-tile form are too small)
+            2.75 * ceil_div(ceil_div(nC, S), 2) + 10.6 < 0.93 * std::max(fp32(halvings), fp32(drhip_conv3x3_winograd_pick_variant(W, H, I, O) >> 4 & 15)))
+            if (const int v = split(0x101, 0, S, S)) return v;
     }
     if (!wide) return 0;
     const int over = n - cusPerXcd, over2 = n - 2 * cusPerXcd;

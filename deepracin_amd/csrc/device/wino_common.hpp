@@ -67,6 +67,7 @@ constexpr int kAuxThrough = 1 | 16;                 // cache policy of a buffer 
 constexpr int kAuxDeviceVolatile = 16 | (int)0x80000000u;   // sc1 (device scope: not served from this CU's vector cache), reloaded every time
 int ws_join_timeouts(unsigned* count);              // of the split-operand kernel
 int wino_join_spins();                              // bound on the wait for a partner's partial tile
+int wino_halvings(int W, int H, int I, int O);      // of the input channels where the fp32 kernel neither joins nor helps; -1: its 16-tile form
 
 // Nothing of a launch may lie in its workspace when the launch has ended: the next one would take a partial tile that came too
 // late for its own panel.  Whoever gives a tile up adds to the kernel's counter first and looks once more behind that; whoever has stored

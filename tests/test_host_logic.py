@@ -758,6 +758,16 @@ def test_sums_of_a_cut_are_as_short_as_the_finer_one_s(lib, W, H, I, O, variant,
     assert div(div(stages - donated, 1 << (v >> 4 & 15)), 2 if v & 0x400 else 1) <= div(stages, finer)
 
 
+@pytest.mark.parametrize("W,H,I,O,pieces", [
+    (48, 48, 256, 256, 3), (48, 48, 512, 256, 3), (40, 30, 512, 512, 3),        # which helpers, or joined halves, would do as fast
+    (42, 143, 504, 80, 2), (62, 57, 497, 134, 2), (56, 41, 783, 114, 4),        # with an odd number of chunks, too
+    (172, 9, 1020, 154, 4),                                                     # faster than joined halves, not than quarters in two launches
+    (56, 56, 256, 256, 0), (28, 28, 512, 512, 0), (34, 32, 256, 256, 0)])       # no faster than halves and whole panels
+def test_layers_stay_in_pieces_for_their_exactness(lib, W, H, I, O, pieces):
+    """Split-operand pieces are more exact than the joined halves and helpers of the fp32 kernel, and are measured against its other forms."""
+    assert lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O) == (0x101 | pieces << 12 | pieces << 16 if pieces else 0)
+
+
 @pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
 def test_interleaved_to_planes(lib, pixels, channels):
     a = np.random.default_rng(0).standard_normal((pixels, channels)).astype(np.float32)
