@@ -477,8 +477,8 @@ gboolean dR_planBuffers(dR_Graph* net) {
                 else ((dR_Softmax_Data*)consumer->layer)->drDeferredInput = n;
                 dR_Conv2d_Data* cd = (dR_Conv2d_Data*)c->layer;
                 cd->drFusedAvgPool = TRUE;
-                // (at most 64 tiles for the reader to add up: of 32 pixels in larger maps)
-                if (cd->drDirectBank && (cd->variant & 0x20) && c->oshape.s0 * c->oshape.s1 > 64 * 16) cd->variant = 8;
+                // (at most 64 tiles for the reader to add up: of 32 pixels in larger maps, which variant 0 has, with as many waves as there is work for)
+                if (cd->drDirectBank && (cd->variant & 0x20) && c->oshape.s0 * c->oshape.s1 > 64 * 16) cd->variant = 0;
                 ((dR_Pooling_Data*)n->layer)->drFused = TRUE;
             }
         }

@@ -583,6 +583,21 @@ def test_fire_modules_ride_along_where_that_is_faster(lib, W, S, E, modules, joi
         assert ["in the launch of the layers in front" in _kernel_line(s) for s in squeezes[1:]] == [joined] * (modules - 1)
 
 
+@pytest.mark.parametrize("W,H,I,O,stride,variant", [(40, 40, 24, 16, 1, 0), (86, 94, 64, 32, 2, 0), (32, 32, 24, 16, 1, 0x24), (64, 64, 64, 16, 2, 0x28)])
+def test_averaged_layers_have_at_most_64_tiles(lib, monkeypatch, W, H, I, O, stride, variant):
+    """A direct 3x3 layer whose tiles of 16 pixels are more than 64 leaves a global average to tiles of 32 (variant 0: by that form's own rule)."""
+    monkeypatch.setenv("DR_CONV3X3", "direct")
+    w, size = lambda i, o, k: np.ones((i, o, k, k), np.float32), (W // stride, H // stride)
+    with dr.Environment() as env:
+        g = env.create_graph()
+        c = dr.Conv2d_raw(dr.feed_node(g, [H, W, I]), w(I, O, 3), None, (stride, stride), "relu")
+        dr.mark_as_output(dr.Softmax(dr.Pooling(c, "average", [1, *size, 1], [1, *size, 1])))
+        assert lib.dR_propagateShapesAndSchedule(g.ptr) == 1
+        assert int(re.search(r"variant (\d+)", _kernel_line(c))[1]) == lib.drhip_conv3x3_direct_pick_variant(*size, I, O)
+        assert lib.dR_planBuffers(g.ptr) == 1
+        assert int(re.search(r"variant (\d+)", _kernel_line(c))[1]) == variant
+
+
 def test_layers_beyond_32_bit_byte_offsets_take_the_general_kernels(lib):
     """Every dimension fits the 16-bit argument fields, but the input holds 2^29 elements or more: the matrix-core
     3x3 kernels and the pooling-on-load 1x1 kernel (32-bit byte offsets) are not scheduled for such a layer."""
