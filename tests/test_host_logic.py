@@ -598,6 +598,24 @@ def test_averaged_layers_have_at_most_64_tiles(lib, monkeypatch, W, H, I, O, str
         assert int(re.search(r"variant (\d+)", _kernel_line(c))[1]) == variant
 
 
+@pytest.mark.parametrize("W,H,I,O,reader,inLaunch", [
+    (200, 200, 3, 64, True, True), (300, 300, 3, 64, True, True), (96, 96, 3, 24, True, False), (128, 128, 3, 32, True, False), (96, 96, 3, 24, False, True)])
+def test_who_takes_a_pooling_of_three_behind_other_filters(lib, W, H, I, O, reader, inLaunch):
+    """7x7/2 layer -> 3x3/2 max pooling (-> 1x1 layer): the first layer stores the pooled tensor where that beats the pooling's alternative, which is the
+    1x1 layer taking the maxima on load where there is one (96x96 3->24: in the launch without a reader, on load with it)."""
+    w = lambda i, o, k: np.ones((i, o, k, k), np.float32)
+    pick = lambda against: lib.drhip_conv_bank_maxpool3s2_pick_variant(W, H, I, O, 7, 7, 2, 2, against) != 0
+    assert pick(1 if reader else 0) == inLaunch
+    with dr.Environment() as env:
+        g = env.create_graph()
+        c = dr.Conv2d_raw(dr.feed_node(g, [H, W, I]), w(I, O, 7), None, (2, 2), "relu")
+        p = dr.Pooling(c, "max", [1, 3, 3, 1], [1, 2, 2, 1])
+        dr.mark_as_output(dr.Conv2d_raw(p, w(O, 16, 1), None, (1, 1), "relu") if reader else p)
+        assert lib.dR_propagateShapesAndSchedule(g.ptr) == 1 and lib.dR_planBuffers(g.ptr) == 1
+        pixels, pooled = (W // 2) * (H // 2), -(-(W // 2) // 2) * -(-(H // 2) // 2)
+        assert plan_of(g, [c])[0][3] == O * (pooled if inLaunch else pixels)        # (floats)
+
+
 def test_layers_beyond_32_bit_byte_offsets_take_the_general_kernels(lib):
     """Every dimension fits the 16-bit argument fields, but the input holds 2^29 elements or more: the matrix-core
     3x3 kernels and the pooling-on-load 1x1 kernel (32-bit byte offsets) are not scheduled for such a layer."""
