@@ -1016,12 +1016,13 @@ def test_branches_keep_off_memory_that_fusions_touch(oracle, gpu, kind):
             assert np.array_equal(x, y)
 
 
-def test_joined_layers_of_two_graphs_on_two_streams(lib, gpu):
-    """Pieces of a split-operand layer wait for each other inside the launch.  Two graphs with such a layer, each on its own
-    stream, run at the same time: every pass as if it were alone, and no piece waited in vain."""
+@pytest.mark.parametrize("W,H,I,O,helpers", [(33, 31, 256, 512, False), (56, 56, 256, 256, True), (48, 48, 128, 256, True)])
+def test_joined_layers_of_two_graphs_on_two_streams(lib, gpu, W, H, I, O, helpers):
+    """Pieces of a split-operand layer, and panels and their helpers, wait for each other inside the launch.  Two graphs with such a layer, each on its
+    own stream, run at the same time: every pass as if it were alone, and no piece waited in vain."""
     rng = np.random.default_rng(3)
-    W, H, I, O = 33, 31, 256, 512
-    assert lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O) >> 12
+    split = lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O)
+    assert split == 0 and lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O) == 0x2c01 if helpers else split >> 12
     late = ctypes.c_uint(0)
     assert lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)) == 0
     before = late.value

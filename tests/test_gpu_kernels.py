@@ -747,9 +747,34 @@ def test_winograd_helpers(lib, dev, oracle, W, H, I, O):
         assert lib.drhip_conv3x3_winograd_f32(xd, U, bd, out, *shape, 1, variant, ws, None) == -1
 
 
+@pytest.mark.parametrize("variant", [0x2c01, 0xc11, 0x821, 0x1801])
+def test_winograd_joins_keep_infinities(lib, dev, variant):
+    """Infinities and NaN in the share of the one, of the other and of both whose sums are joined (with helpers the first 64 channels are the panel's
+    own): what fp32 Winograd makes of them, also of a NaN that looks like the marker of a tile that has not arrived, and the next launch sees nothing
+    of it.  (Not in the columns at the edge, whose samples the kernel multiplies by zero for their neighbours.)"""
+    W, H, I, O = 13, 9, 128, 33
+    x, w = own(I, H, W), own(I, O, 3, 3, scale=0.02)
+    spoilt = x.copy()
+    spoilt[3, 4, 4], spoilt[100, 4, 4], spoilt[5, 1, 7], spoilt[127, 6, 9], spoilt[70, 7, 3] = np.inf, -np.inf, np.inf, np.inf, np.nan
+    spoilt.view(np.uint32)[[9, 90, 126], 2, 10] = 0xffa5c3e1
+    U, _ = wino_filters(lib, dev, w)
+    n, y = lib.drhip_conv3x3_winograd_workspace_floats(W, H, I, O, variant), dev.empty(O * H * W)
+    ws = wino_workspace(lib, dev, W, H, I, O, variant)
+    for a in (x, spoilt, x, spoilt):
+        ok(lib, lib.drhip_conv3x3_winograd_f32(dev.put(a), U, None, y, W, H, I, O, 0, variant, ws, None))
+        got, want = dev.get(y, (O, H, W)), winograd_replay(a, w)
+        assert np.isnan(want).any() == np.isinf(want).any() == (a is spoilt)
+        assert_same_extremes(got, want)
+        assert np.all(dev.get(ws, (n,)).view(np.uint32) == 0xffa5c3e1)
+    late = ctypes.c_uint(123)
+    ok(lib, lib.drhip_conv3x3_winograd_join_timeouts(ctypes.byref(late)))
+    assert late.value == 0
+
+
 def test_winograd_tiered_refused_combinations(lib, dev):
     p = dev.empty(64)
-    for variant in (0x1001, 0x1901, 0x1c01, 0x1811, 0x1803, 0x2801):     # not joined, 16-tile blocks, two wave sets, split bits, 128 channels, unknown bit
+    # not joined, 16-tile blocks, two wave sets, split bits, 128 channels; helpers with one wave set, 64 channels, split bits, not joined, in tiers; an unknown bit
+    for variant in (0x1001, 0x1901, 0x1c01, 0x1811, 0x1803, 0x2801, 0x2c02, 0x2c11, 0x2001, 0x3c01, 0x4801, 0x4c01):
         assert lib.drhip_conv3x3_winograd_workspace_floats(8, 8, 16, 16, variant) == 0
         assert lib.drhip_conv3x3_winograd_f32(p, p, None, p, 8, 8, 16, 16, 0, variant, p, None) == -1, hex(variant)
 
