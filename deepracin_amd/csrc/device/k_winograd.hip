@@ -137,7 +137,7 @@ __device__ inline f32x4 buf_load4(__amdgpu_buffer_rsrc_t r, unsigned voffset, un
 // loads); layers whose workgroup count leaves one workgroup per CU get their second wave per SIMD this way,
 // without a second workgroup's share of partial tiles in memory.
 // FEWC: a layer with at most four input channels (an image): one stage whose third and fourth k-step would multiply
-// zeros are left out, and nothing is prefetched.
+// zeros are left out, and nothing is prefetched or cut (224x224 3->64 with the code for tiers and joins, which it never reaches, 5.2 us, without 5.0).
 // HELP: a launch with helpers.  Panels that fill one round of the CUs only in part leave the others idle: 56x56 256->256 has 200 panels
 // for 256 CUs.  There the CUs without a panel of their own take the last stages (cfg1, bits 16 to 23: channels in eights) of
 // several panels each, one panel after the other, and leave the sums in the panel's slots of the workspace (as the joined splits do); the panel's
@@ -167,7 +167,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         donated = (int)((cfg1 >> 16) & 255u);
         nSp = 1;
         slot -= nSplits;                                // (the first workgroups of an XCD are its helpers)
-    } else if (tiered) {
+    } else if (!FEWC && tiered) {
         int jj = slot, base = 0;
         bool found = false;
 #pragma unroll
@@ -181,7 +181,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
         if (!found) return;
         nSp = 1 << lgSp;
         chunksHere = ((I + kWinoKC - 1) / kWinoKC) >> lgSp;     // (the launcher makes tiers of equal splits only)
-    } else if (joined) {
+    } else if (!FEWC && joined) {
         split = slot & (nSplits - 1);
         slot >>= lgSplits;
     }
@@ -193,7 +193,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
     int t0 = (logical - oBlock * (int)nTBd.d) * TB;
     // The fewer stages a workgroup has, the sooner its partial tiles can be on their way: small pieces first,
     // so that the workgroups that end a CU's work are whole panels, which wait for nobody.
-    if (tiered) {
+    if (!FEWC && tiered) {
         if (lgSp >= 3) __builtin_amdgcn_s_setprio(3);
         else if (lgSp == 2) __builtin_amdgcn_s_setprio(2);
         else if (lgSp == 1) __builtin_amdgcn_s_setprio(1);
@@ -423,7 +423,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                 return;
             }
         }
-        if (!HELP && !FEWC && joined && nSp > 1) {      // (a single stage is not cut)
+        if (!HELP && !FEWC && joined && nSp > 1) {
             // (the partial tiles go out and are looked for at the highest priority: the other workgroups on this CU
             // are in their channel loops, and a wave at their priority gets an issue slot only when they stall)
             if (tiered) __builtin_amdgcn_s_setprio(3);
