@@ -19,8 +19,8 @@
 //     few tiles fill the chip that way without a second kernel.
 //   * A 2x2/2 max pooling behind the layer is taken from these sums: a pooled pixel a lane.  (28x28 with 5x5 filters and poolings, 16
 //     and 32 channels, its image from the host and its results back: 36.4 -> 32.2 us, two launches less.)
-//   * So is a 3x3/2 max pooling (P3): the pixels of a workgroup are then the 9x7 or 9x9 under 4x3 or 4x4 pooled ones, so that
-//     1.3 times the products are done, and one launch less and a quarter of the outputs stored.  (Figures stand at the choice of the variant.)
+//   * So is a 3x3/2 max pooling (P3): the pixels of a workgroup are then the 9x7 or 9x9 under 4x3 or 4x4 pooled ones, in two or three
+//     blocks of 32, so that 1.33 or 1.5 times the products are done, and one launch less and a quarter of the outputs stored.  (Figures stand at the choice of the variant.)
 //   * Outputs that do not come out finite are worked out again in fp32, at the end.
 // Layers with at most four input channels (images) put four neighbouring pixels x four channels into one step of 16 k
 // (CP = 4) instead of 16 channels of one pixel, most of which would be zero: a 7x7 filter over RGB is 14 steps, not 49.

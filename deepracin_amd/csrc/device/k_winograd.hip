@@ -925,12 +925,14 @@ static bool wino_tiers(int nBlocks, int nChunks, int cus, WinoTiers* t) {
     return t->maxLg > 0;
 }
 
+struct WinoHelpers { int count, donated; };          // of an XCD; stages of 8 channels they take off each of its panels
+
 // Who helps (see the kernel): an XCD has P panels and `cus` CUs; cus - P helpers have up to `each` panels each.  In stages of eight channels
 // (0.47 us on a CU) a panel's own workgroup needs n - d and 11 on top where something is joined, a helper each * (d + 4) and 5 or 6:
 // the largest even d for which the helper is done first.  Below 4 the join costs what is gained (57x55 256->256, d = 2: 20.1 / 20.0).
 // Measured, d = 2, 4, 6, 8, 10: 56x56 256->256 (four panels each) 19.4 18.7 21.3 24.9 28.9; 52x52 (three) 19.0 18.0 17.3 19.7 22.4; 48x48 (two)
 // 19.1 17.9 17.0 16.1 16.5.
-WinoHelpers wino_helpers(int nBlocks, int nChunks, int cus) {
+static WinoHelpers wino_helpers(int nBlocks, int nChunks, int cus) {
     const int P = ceil_div(nBlocks, kXcds);
     WinoHelpers best = {0, 0};
     if (P >= cus) return best;
