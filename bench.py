@@ -17,8 +17,8 @@ of 20 passes is a few milliseconds long and a single sample of it says little), 
                  achieved / 157.3 TFLOP/s.  Winograd F(2x2,3x3) issues 2.25x fewer multiplications than
                  that, so `frac` is credit for the algorithm, NOT matrix-pipe utilisation: that is
                  `issued_tflops` (the FLOPs the kernel really issues, 2*16*tiles*I*O with tiles, I and O
-                 padded to its blocks -- the counters SQ_INSTS_VALU_MFMA_MOPS_F32 and _BF16 read exactly this, see
-                 profiles/; six bf16 products each on the layers of the split-operand kernel) and
+                 padded to its blocks -- the counters SQ_INSTS_VALU_MFMA_MOPS_F32, _BF16 and _F16 read exactly this, see
+                 profiles/; six bf16 or three f16 products each on the layers of the split-operand kernels) and
                  `mfma_busy_frac`, the share of the data-sheet matrix peaks (157.3 fp32, 2500 bf16) the
                  pipe was issuing at; the >= 50 % target is judged on `mfma_busy_frac`.
                  `mfma_busy_frac_counters` is the same share from SQ_VALU_MFMA_BUSY_CYCLES of the
@@ -71,7 +71,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 PEAK_MFMA_F32_TFLOPS = 157.3
-PEAK_MFMA_BF16_TFLOPS = 2500.0      # dense
+PEAK_MFMA_BF16_TFLOPS = 2500.0      # dense, and f16
 PEAK_HBM_GBS = 8000.0
 PEAK_CLOCK_GHZ = 2.4            # the clock the data-sheet peak is quoted at
 COUNTERS_JSON = os.path.join(ROOT, "profiles", "counters.json")
@@ -110,18 +110,20 @@ def winograd_issued_flops(lib, W, H, I, O):
     """FLOPs the Winograd kernel issues for a layer: 16 GEMMs over tiles x I x O, each padded to the blocks of
     the variant the scheduler picks (tile blocks of 32 or 16, 8 input channels per stage, 32/64/128 or 16/32/64
     output channels per workgroup); drhip_conv3x3_winograd_f32 decides the same way.  With it the peak of the matrix cores it
-    runs on: large layers take the split-operand kernel, six bf16 products (32 tiles x 16 channels x 64 channels) for each fp32 one."""
+    runs on and the kernel's name: large layers take a split-operand kernel, six bf16 or three f16 products (32 tiles x 16 channels x
+    64 channels) for each fp32 one (random weights fit two f16 parts)."""
     v = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O)
     tb = 16 if v & 0x100 else 32
     ob = tb * {1: 1, 2: 2, 3: 4}[v & 0xf]
     tiles = ((W + 1) // 2) * ((H + 1) // 2)
     pad = lambda n, m: -(-n // m) * m
-    if lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O):
-        return 6 * 2 * 16 * pad(tiles, 32) * pad(I, 16) * pad(O, 64), PEAK_MFMA_BF16_TFLOPS
+    pair = lib.drhip_conv3x3_winograd_pair_pick_variant(W, H, I, O)
+    if pair or lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O):
+        return (3 if pair else 6) * 2 * 16 * pad(tiles, 32) * pad(I, 16) * pad(O, 64), PEAK_MFMA_BF16_TFLOPS, "winograd_f23_%s_kernel" % ("pair" if pair else "split")
     # (an image layer -- at most 4 input channels, 32-tile blocks, unsplit, four waves -- runs its one stage without
     # the two k-steps that would multiply zeros)
     few = I <= 4 and tb == 32 and (v & 0xf) <= 2 and not (v & 0x400) and not (v >> 4) & 0xf
-    return 2 * 16 * pad(tiles, tb) * (4 if few else pad(I, 8)) * pad(O, ob), PEAK_MFMA_F32_TFLOPS
+    return 2 * 16 * pad(tiles, tb) * (4 if few else pad(I, 8)) * pad(O, ob), PEAK_MFMA_F32_TFLOPS, KERNEL_NAMES["winograd"]
 
 
 def measure(workload, seed, steps, warmup, blocks=BLOCKS, instrument=True, env_vars=None):
@@ -253,10 +255,9 @@ def analyse(lib, m, workload, counters):
         if k == "winograd" and ms[i] > 0:
             W, H, _ = shapes[n["in"]]
             I, O = n["w"].shape[0], joint_o.get(i, n["w"].shape[1])
-            issued, peak = winograd_issued_flops(lib, W, H, I, O)
+            issued, peak, name = winograd_issued_flops(lib, W, H, I, O)
             gk["issued"] += issued
             gk["busy_ms"] += issued / peak / 1e9
-            name = "winograd_f23_split_kernel" if peak == PEAK_MFMA_BF16_TFLOPS else KERNEL_NAMES[k]
             gk.setdefault("names", collections.Counter())[name] += 1
             v = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O)
             if peak == PEAK_MFMA_F32_TFLOPS and (v >> 4) & 0xf and not v & 0x800:       # split layers whose partial tiles are summed by a second kernel
@@ -445,9 +446,9 @@ def summarise(dirs, workload, counters_json, last=0):
                 units = per
             if "SQ_INSTS_VALU_MFMA_MOPS_F32" in per:
                 mfma = per
-                bf16 = {r["dispatch"]: r["value"] for r in per.get("SQ_INSTS_VALU_MFMA_MOPS_BF16", [])}
-                for r in per["SQ_INSTS_VALU_MFMA_MOPS_F32"]:        # a kernel issues the one or the other
-                    r["value"] += bf16.get(r["dispatch"], 0.0)
+                halves = [{r["dispatch"]: r["value"] for r in per.get("SQ_INSTS_VALU_MFMA_MOPS_" + t, [])} for t in ("BF16", "F16")]
+                for r in per["SQ_INSTS_VALU_MFMA_MOPS_F32"]:        # a kernel issues one of them
+                    r["value"] += sum(h.get(r["dispatch"], 0.0) for h in halves)
     if fetch and write:
         cf = [r["value"] for r in fetch if "copy3d" in r["kernel"]][1:]
         cw = [r["value"] for r in write if "copy3d" in r["kernel"]][1:]
@@ -479,7 +480,7 @@ def summarise(dirs, workload, counters_json, last=0):
     if mfma:
         mops = _last_pass(mfma["SQ_INSTS_VALU_MFMA_MOPS_F32"], last)
         busy = {r["dispatch"]: r["value"] for r in mfma.get("SQ_VALU_MFMA_BUSY_CYCLES", [])}
-        print("Matrix-core counters of the launches of the last forward pass that issue MFMAs.  SQ_INSTS_VALU_MFMA_MOPS_F32 (and _BF16, on the "
+        print("Matrix-core counters of the launches of the last forward pass that issue MFMAs.  SQ_INSTS_VALU_MFMA_MOPS_F32 (and _BF16 and _F16, on the "
               "split-operand kernels) counts 512 FLOP per unit; SQ_VALU_MFMA_BUSY_CYCLES is summed over the chip's 1024 SIMDs; `kernel us` is the dispatch's own "
               "End - Start timestamp under the profiler (longer than in a plain run); busy = busy cycles per SIMD / (kernel us x 2.4 GHz).\n")
         print("| # | kernel | grid (lanes) | MOPS | issued GFLOP | MFMA busy cycles/SIMD | kernel us | busy |")

@@ -28,13 +28,17 @@
 // launches that leave at most one workgroup per CU, where a single set is alone on its SIMDs and waits for its own loads.
 // Launches whose panels do not fill the CUs evenly cut the input channels of all or of the last panels into pieces, which add their
 // sums up inside the launch (the rule, and what it measured, stands at the choice of the variant).
-#include "bf16x3.hpp"
+//
+// The second kernel of this file does the same with operands in two f16 parts (f16x2.hpp).
+#include "f16x2.hpp"
 #include "wino_common.hpp"
 
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
+#include <vector>
 
 namespace drhip {
 
@@ -86,84 +90,94 @@ wino_split_filter_kernel(const float* __restrict__ w, unsigned short* __restrict
     }
 }
 
-// TURNS: see `turn`.  (Of its own, because even its few instructions show on layers of three steps: 41x53 254->254 0.17 us.)
+// What a workgroup computes: a split of the input channels of a panel of 32 tiles and 64 output channels.
+template <int KW>
+struct WsPlace {
+    int wave, set, nSp, split, inXcd, first, perSplit, steps, oBlock, o0, t0;      // (wave: the row of the transform, of both sets)
+    bool ok;
+    __device__ __forceinline__ explicit WsPlace(const WsShape& s) {
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+        set = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+        const FastDiv nTBd = {(unsigned)s.nTB, s.mulTB, s.shTB};
+        const int perXcd = (s.nBlocks + kXcds - 1) / kXcds;
+        const int slot = (int)(blockIdx.x >> 3), later = slot - s.wgsA;        // (an XCD works on neighbouring panels)
+        nSp = later < 0 ? s.sA : s.sB;
+        const int place = later < 0 ? slot : later, panel = nSp == 1 ? place : place * (later < 0 ? s.mulA : s.mulB) >> 16;
+        split = nSp == 1 ? 0 : place - panel * nSp;
+        inXcd = (later < 0 ? 0 : s.nA) + panel;
+        const int logical = (int)(blockIdx.x & 7) * perXcd + inXcd;
+        ok = !(inXcd >= perXcd || logical >= s.nBlocks);
+        perSplit = later < 0 ? s.perA : s.perB;
+        first = split * perSplit;
+        steps = (perSplit + KW - 1) / KW;
+        oBlock = fast_div(logical, nTBd);
+        o0 = oBlock * 64;
+        t0 = (logical - oBlock * s.nTB) * 32;
+    }
+};
+
+// The samples of a workgroup's steps on their way from global memory to LDS, and where they lie there.
+// A segment is the part of the panel's 32 tiles that lies in one row of tiles; its samples lie in a row in LDS, from a
+// multiple of 16 bytes on: from column 2*tx-1 of its first tile, or from column 0 where that is left of the map (the sample
+// in front of it is then whatever lies in front of it: it is multiplied by zero).
+// TURNS: panels of an XCD begin at different channels (`turn`) and go round: the first to reach a fragment of the filters brings it
+// from memory, the others find it in L2, and they take turns at that instead of all waiting for it together.  (A template parameter,
+// because even its few instructions show on layers of three steps: 41x53 254->254 0.17 us.)
 template <int KW, int WC, bool TURNS>
-__global__ void __launch_bounds__(256 * KW, 2)
-winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __restrict__ U, const float* __restrict__ bias,
-                          float* __restrict__ out, WsShape s, float* __restrict__ ws) {
-    constexpr int NT = 2, OB = 32 * NT;
-    constexpr int CHB = WC * 16, ROWB = kWsKC * CHB, BUFB = 4 * ROWB;    // bytes of a window row of one channel, of 16, of a step's samples
-    constexpr int NDMA = ROWB / 1024;               // loads of a wave for them: one window row each
-    constexpr int kPA[6] = {0, 0, 0, 1, 1, 2}, kPB[6] = {2, 1, 0, 1, 0, 0}; // partial products: part of the filter, part of the sample
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-    __shared__ float biasT[OB];
+struct WsSamples {
+    static constexpr int CHB = WC * 16, ROWB = kWsKC * CHB, BUFB = 4 * ROWB;    // bytes of a window row of one channel, of 16, of a step's samples
+    static constexpr int NDMA = ROWB / 1024;        // loads of a wave for them: one window row each
+    unsigned voff[NDMA];                            // (never below kOutOfRange where it started from that)
+    unsigned stepB, ldsBase, toNext;
+    int steps, fetching, left;                      // the step whose samples are fetched next; how many are to come
+    __amdgpu_buffer_rsrc_t rIn;
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, set = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
-    const int l32 = lane & 31, half = lane >> 5;
-    const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX}, nTBd = {(unsigned)s.nTB, s.mulTB, s.shTB};
+    __device__ __forceinline__ static int segment_at(const WsShape& s, int off0, int k) { return k == 0 ? 4 : (2 * (k * s.tilesX - off0) + 4 * k + 6) & ~3; }     // in floats
 
-    const int perXcd = (s.nBlocks + kXcds - 1) / kXcds;
-    const int slot = (int)(blockIdx.x >> 3), later = slot - s.wgsA;        // (an XCD works on neighbouring panels)
-    const int nSp = later < 0 ? s.sA : s.sB;
-    const int place = later < 0 ? slot : later, panel = nSp == 1 ? place : place * (later < 0 ? s.mulA : s.mulB) >> 16;
-    const int split = nSp == 1 ? 0 : place - panel * nSp;
-    const int inXcd = (later < 0 ? 0 : s.nA) + panel, logical = (int)(blockIdx.x & 7) * perXcd + inXcd;
-    if (inXcd >= perXcd || logical >= s.nBlocks) return;
-    const int perSplit = later < 0 ? s.perA : s.perB, first = split * perSplit, steps = (perSplit + KW - 1) / KW;
-    const int oBlock = fast_div(logical, nTBd);
-    const int o0 = oBlock * OB, t0 = (logical - oBlock * s.nTB) * 32;
-    const int W = s.W, H = s.H, I = s.I, plane = W * H;
-
-    // ---- samples: global memory -> LDS -------------------------------------------------------------------------------
-    // A segment is the part of the panel's 32 tiles that lies in one row of tiles; its samples lie in a row in LDS, from a
-    // multiple of 16 bytes on: from column 2*tx-1 of its first tile, or from column 0 where that is left of the map (the sample
-    // in front of it is then whatever lies in front of it: it is multiplied by zero).
-    const int ty0 = fast_div(t0, tilesXd), off0 = t0 - ty0 * s.tilesX;
-    // Panels of an XCD begin at different channels and go round: the first to reach a fragment of the filters brings it from
-    // memory, the others find it in L2, and they take turns at that instead of all waiting for it together.
-    const int turn = TURNS ? min(inXcd & 31, steps - 1) : 0;
-    auto segment_at = [&](int k) { return k == 0 ? 4 : (2 * (k * s.tilesX - off0) + 4 * k + 6) & ~3; };     // in floats
-    const unsigned stepB = 64u * KW * (unsigned)plane;
-    const int first16 = 16 * (first + set);
-    // Segment by segment, for a wave's window row and the same in all lanes: where its samples lie in LDS, behind which of them the
-    // row ends (not one of them, for a row beside the map), and the address that the first would have at the row's beginning.
-    constexpr int SEG = ws_segments(WC);
-    const unsigned plane4 = 4u * (unsigned)plane;
-    int segAt[SEG], segEnd[SEG];
-    unsigned segBase[SEG];
+    __device__ __forceinline__ WsSamples(const float* in, const char* lds, const WsShape& s, const WsPlace<KW>& at, int ty0, int off0, int turn) {
+        const int lane = threadIdx.x & 63, W = s.W, H = s.H, plane = W * H;
+        steps = at.steps;
+        stepB = 64u * KW * (unsigned)plane;
+        const int first16 = 16 * (at.first + at.set);
+        // Segment by segment, for a wave's window row and the same in all lanes: where its samples lie in LDS, behind which of them the
+        // row ends (not one of them, for a row beside the map), and the address that the first would have at the row's beginning.
+        constexpr int SEG = ws_segments(WC);
+        const unsigned plane4 = 4u * (unsigned)plane;
+        int segAt[SEG], segEnd[SEG];
+        unsigned segBase[SEG];
 #pragma unroll
-    for (int k = 0; k < SEG; ++k) {
-        const int iy = 2 * (ty0 + k) - 1 + wave, left = k == 0 && off0 > 0 ? 2 * off0 - 1 : 0;
-        segAt[k] = segment_at(k);
-        segEnd[k] = iy >= 0 && iy < H ? W - left + segAt[k] : 0;
-        segBase[k] = 4u * (unsigned)(iy * W + left - segAt[k]) + (unsigned)first16 * plane4;
-    }
-    unsigned voff[NDMA];                                // (never below kOutOfRange where it started from that)
-    int piece = lane % WC;
-    unsigned chOff = (unsigned)(lane / WC) * plane4;
-#pragma unroll
-    for (int i = 0; i < NDMA; ++i) {
-        const int f = 4 * piece;
-        int end = segEnd[0];
-        unsigned base = segBase[0];
-#pragma unroll
-        for (int k = 1; k < SEG; ++k) {
-            end = f >= segAt[k] ? segEnd[k] : end;
-            base = f >= segAt[k] ? segBase[k] : base;
+        for (int k = 0; k < SEG; ++k) {
+            const int iy = 2 * (ty0 + k) - 1 + at.wave, skip = k == 0 && off0 > 0 ? 2 * off0 - 1 : 0;
+            segAt[k] = segment_at(s, off0, k);
+            segEnd[k] = iy >= 0 && iy < H ? W - skip + segAt[k] : 0;
+            segBase[k] = 4u * (unsigned)(iy * W + skip - segAt[k]) + (unsigned)first16 * plane4;
         }
-        voff[i] = (f >= 4 && f < end ? base + 4u * (unsigned)f + chOff : kOutOfRange) + (unsigned)turn * stepB;
-        const bool wrap = piece >= WC - 64 % WC;        // 64 pieces on
-        piece += 64 % WC - (wrap ? WC : 0);
-        chOff += (unsigned)(64 / WC) * plane4 + (wrap ? plane4 : 0u);
+        int piece = lane % WC;
+        unsigned chOff = (unsigned)(lane / WC) * plane4;
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) {
+            const int f = 4 * piece;
+            int end = segEnd[0];
+            unsigned base = segBase[0];
+#pragma unroll
+            for (int k = 1; k < SEG; ++k) {
+                end = f >= segAt[k] ? segEnd[k] : end;
+                base = f >= segAt[k] ? segBase[k] : base;
+            }
+            voff[i] = (f >= 4 && f < end ? base + 4u * (unsigned)f + chOff : kOutOfRange) + (unsigned)turn * stepB;
+            const bool wrap = piece >= WC - 64 % WC;        // 64 pieces on
+            piece += 64 % WC - (wrap ? WC : 0);
+            chOff += (unsigned)(64 / WC) * plane4 + (wrap ? plane4 : 0u);
+        }
+        rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, min(s.I, 16 * (at.first + at.perSplit)) * plane * 4, kBufferFlags);    // (ends with the split)
+        ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(at.set * 3 * BUFB + at.wave * ROWB);
+        fetching = turn;
+        left = steps;
+        toNext = 0;
     }
-    const __amdgpu_buffer_rsrc_t rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, min(I, 16 * (first + perSplit)) * plane * 4, kBufferFlags);    // (ends with the split)
-    const unsigned ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(set * 3 * BUFB);
-    // 16 bytes per lane, lane by lane, to LDS at M0.  The compiler does not count these loads: where it waits for a filter
-    // it waits for a few more loads than it means to, and for the samples this kernel waits itself.
-    int fetching = turn, left = steps;                  // the step whose samples are fetched next; how many are to come
-    unsigned toNext = 0;
-    auto fetch_sample = [&](int buf, int i) {
+    // The i-th load of the next step into buffer `buf`: 16 bytes per lane, lane by lane, to LDS at M0.  The compiler does not count these
+    // loads: where it waits for a filter it waits for a few more loads than it means to, and for the samples the kernels wait themselves.
+    __device__ __forceinline__ void fetch(int buf, int i) {
         if (i == 0) {
             const bool last = TURNS && fetching == steps - 1;
             // (behind the last one out of the map: zeros that nobody uses cost no trip to memory)
@@ -171,184 +185,36 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             --left;
             if (TURNS) fetching = last ? 0 : fetching + 1;
         }
-        const unsigned at = ldsBase + (unsigned)(buf * BUFB + wave * ROWB);
+        const unsigned at = ldsBase + (unsigned)(buf * BUFB);
         unsigned m0;                                    // (put back: the compiler may keep a value there, and takes no clobber for it)
         asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 m0, %0"
                      : "=&s"(m0) : "v"(voff[i]), "s"(rIn), "s"(at + 1024u * i) : "memory");
         voff[i] += toNext;
-    };
-
-    // ---- filters ---------------------------------------------------------------------------------------------------
-    // The waits for samples count the filter loads issued behind them, so these must stay where they stand: an address whose
-    // origin the compiler does not see keeps it from taking them for loads that no memory clobber concerns.
-    const unsigned short* uHere = U;
-    asm volatile("" : "+s"(uHere));
-    const int uBytes = 16 * s.nC * 3 * s.nOB * 1024;
-    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, uBytes, kBufferFlags);
-    unsigned uOb[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) uOb[nt] = (unsigned)((wave * s.nC * s.nOB + min(oBlock * NT + nt, s.nOB - 1)) * 12288);
-    const unsigned uStep = (unsigned)s.nOB * 12288u;
-    // (what the last step requests for one behind it comes from nowhere)
-    __amdgpu_buffer_rsrc_t rNext = rU;
-    // the first part of two positions and the others of one: no more registers are left
-    u32x4b f0[2][NT], f12[NT][2];
-    auto filter = [&](int e, int nt, int q) -> u32x4b& { return q == 0 ? f0[e & 1][nt] : f12[nt][q - 1]; };
-    auto load_filter = [&](const __amdgpu_buffer_rsrc_t& from, int e, int nt, int q, int step) {
-        filter(e, nt, q) = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 3072)), 0));
-    };
-
-    // ---- operands --------------------------------------------------------------------------------------------------
-    const int rowA = wave, rowB = wave < 2 ? 2 : 1;
-    const float sgn = wave == 1 ? 1.0f : -1.0f;
-    const int lr = fast_div(l32 + off0, tilesXd), tx = l32 + off0 - lr * s.tilesX;
-    const int firstTx = lr == 0 ? off0 : 0;
-    const int rLds = half * 8 * CHB + 4 * (segment_at(lr) + 2 * (tx - firstTx) - (firstTx == 0 ? 1 : 0));
-    // the masks of the samples beside the map carry the scale of the split as well
-    const float k0f = tx > 0 ? kSplitScale : 0.0f, k2f = 2 * tx + 1 < W ? kSplitScale : 0.0f, k3f = 2 * tx + 2 < W ? kSplitScale : 0.0f;
-    float mm[8][4];                                 // combined window rows of this lane's tile, 8 channels
-    float ra[4], rb[4];                             // a channel's rows on their way from LDS
-    const char* samples = lds + set * 3 * BUFB;
-    auto read_rows = [&](int buf, int j) {
-        const float* a = (const float*)(samples + buf * BUFB + rowA * ROWB + rLds + j * CHB);
-        const float* b = (const float*)(samples + buf * BUFB + rowB * ROWB + rLds + j * CHB);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) { ra[c] = a[c]; rb[c] = b[c]; }
-    };
-    auto combine = [&](int j) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) mm[j][c] = fmaf(sgn, rb[c], ra[c]);
-        mm[j][1] *= kSplitScale;                    // (the other two are multiplied where they are used)
-        mm[j][2] *= k2f;
-    };
-    u32x4b B[2][3];                                 // [position parity][part]
-    float va[2], vb[2], xa[2], xb[2];               // the two items being split
-    auto vvalue = [&](int e, int c) {
-        return e == 0 ? fmaf(k0f, mm[c][0], -mm[c][2]) : e == 1 ? mm[c][1] + mm[c][2] : e == 2 ? mm[c][2] - mm[c][1] : fmaf(k3f, mm[c][3], -mm[c][1]);
-    };
-    auto pack = [&](float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2b{a, b}, bf16x2)); };
-    // The operands of position e out of mm: 12 ticks for two items (an item is two channels), whose instructions
-    // alternate: a vector instruction that needs the result of the one in front of it waits for it.
-    auto split_tick = [&](int e, int tick) {
-        const int u = tick / 12, k = tick % 12;
-#pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            const int p = 2 * u + x;
-            u32x4b(&d)[3] = B[e & 1];
-            if (k == 0) va[x] = vvalue(e, 2 * p);
-            if (k == 1) vb[x] = vvalue(e, 2 * p + 1);
-            if (k == 2 || k == 7 || k == 11) d[k == 2 ? 0 : k == 7 ? 1 : 2][p] = pack(va[x], vb[x]);
-            if (k == 3 || k == 8) xa[x] = __builtin_bit_cast(float, d[k == 3 ? 0 : 1][p] << 16);
-            if (k == 4 || k == 8) xb[x] = __builtin_bit_cast(float, d[k == 4 ? 0 : 1][p] & 0xffff0000u);
-            if (k == 5 || k == 9) va[x] -= xa[x];
-            if (k == 6 || k == 10) vb[x] -= xb[x];
-        }
-    };
-
-    f32x16b acc[4][NT];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[e][nt][r] = 0.0f;
-
-    auto barrier = [&] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
-
-    // ---- prologue --------------------------------------------------------------------------------------------------
-    float biasEarly = 0.0f;
-    if (tid < OB && bias) biasEarly = bias[min(o0 + tid, s.O - 1)];
-    asm volatile("" ::: "memory");
-    // What the first products need comes first, the rest behind the barrier.
-#pragma unroll
-    for (int i = 0; i < (KW == 1 ? 2 : 1) * NDMA; ++i) fetch_sample(i / NDMA, i % NDMA);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) load_filter(rU, 0, nt, q, first + set + KW * turn);
-    if (tid < OB) biasT[tid] = biasEarly;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NT + (KW == 1 ? NDMA : 0)) : "memory");
-    barrier();
-#pragma unroll
-    for (int i = 0; i < NDMA; ++i) if (KW == 2) fetch_sample(1, i);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) load_filter(rU, 1, nt, 0, first + set + KW * turn);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) { read_rows(0, j); combine(j); }
-#pragma unroll
-    for (int t = 0; t < 24; ++t) split_tick(0, t);
-
-    // ---- steps -----------------------------------------------------------------------------------------------------
-    // A position is 12 MFMAs, one per slot; with each go two ticks of the next position's operands and what else is due.
-    auto position = [&](auto ec, int step, int stepNext, int nxt, int nxt2) {
-        constexpr int e = decltype(ec)::value;
-#pragma unroll
-        for (int i = 0; i < 6 * NT; ++i) {
-            const int q = i / NT, nt = i % NT;
-            acc[e][nt] = mfma_bf16(filter(e, nt, kPA[q]), B[e & 1][kPB[q]], acc[e][nt]);
-            // a part's last product has been issued: its registers take the filters that come next
-            if (q == 2 || q == 4 || q == 5) {
-                const int by = q == 2 ? 2 : 1;
-                load_filter(e + by >= 4 ? rNext : rU, (e + by) & 3, nt, kPA[q], e + by >= 4 ? stepNext : step);
-            }
-#pragma unroll
-            for (int tk = 2 * i; tk < 2 * i + 2; ++tk) {
-                split_tick((e + 1) & 3, tk);
-                const int at = 24 * e + tk;         // 0..95 over the step
-                if (at % 4 == 0 && at / 4 < NDMA) fetch_sample(nxt2, at / 4);
-                // Rows of the next step, one channel after the other: read, and some ticks later combined, behind the last
-                // use of what they replace and in front of their own first use.
-                constexpr int kRead[8] = {46, 52, 57, 62, 67, 71, 76, 80}, kComb[8] = {51, 56, 61, 66, 70, 75, 79, 83};
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if (at == kComb[j]) combine(j);
-                    if (at == kRead[j]) read_rows(nxt, j);
-                }
-            }
-            // The next step's samples, requested a step ago, have to be visible before they are read.  (Younger than them are this
-            // step's fetch and at least the filters of a position: more than the count waited for.)
-            if (24 * e + 2 * i + 2 == 36) {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
-                barrier();
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    using std::integral_constant;
-    int nxt = 1, nxt2 = 2;
-    for (int n = 0, m = turn; n < steps; ++n) {
-        const int step = first + set + KW * m;
-        m = TURNS && m == steps - 1 ? 0 : m + 1;
-        const int stepNext = first + set + KW * m;
-        rNext = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, n + 1 < steps ? uBytes : 0, kBufferFlags);
-        position(integral_constant<int, 0>{}, step, stepNext, nxt, nxt2);
-        position(integral_constant<int, 1>{}, step, stepNext, nxt, nxt2);
-        position(integral_constant<int, 2>{}, step, stepNext, nxt, nxt2);
-        position(integral_constant<int, 3>{}, step, stepNext, nxt, nxt2);
-        nxt = nxt2;
-        nxt2 = nxt2 == 2 ? 0 : nxt2 + 1;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (fetches beyond the last step, of every wave: LDS is about to be used for
-    barrier();                                              // something else)
+};
 
-    // ---- epilogue --------------------------------------------------------------------------------------------------
-    // D of the 32x32 MFMA: lane -> tile lane%32; register r -> channel 8*(r/4) + 4*(lane/32) + r%4.  Each wave reduces its row of the
-    // transform to two columns, the rows (and the two sets) meet in LDS.
-    float* P = (float*)lds;                         // [set][row][2][OB][32]
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float m0 = acc[0][nt][r], m1 = acc[1][nt][r], m2 = acc[2][nt][r], m3 = acc[3][nt][r];
-            const int ol = 32 * nt + 8 * (r / 4) + 4 * half + (r % 4);
-            P[(((set * 4 + wave) * 2 + 0) * OB + ol) * 32 + l32] = m0 + m1 + m2;
-            P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + l32] = m1 - m2 + m3;
-        }
-    barrier();
+__device__ __forceinline__ void ws_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The bank of three bf16 parts: its fragments of 32 output channels by 16 input channels in pieces of 16 bytes, and a weight out of its parts.
+struct WsBf16x3 {
+    static constexpr int PARTS = 3;
+    __device__ __forceinline__ static float whole(const unsigned (&part)[PARTS], float) { return drhip::whole(part[0], part[1], part[2]); }
+};
+
+// The sums of a panel, rows of the transform (and the two wave sets) side by side in LDS as P[set][row][2][64][32], become outputs: joined with
+// those of the other splits, checked, finished.  scaleT: by output channel, what the sums are to be multiplied by (none: kSplitUnscale).
+template <int KW, class Bank>
+__device__ __forceinline__ void ws_finish(const float* P, const float* biasT, const float* scaleT, const WsShape& s, const WsPlace<KW>& at, const float* in, const unsigned short* U, float* out, float* ws) {
+    constexpr int NT = 2, OB = 32 * NT;
+    using std::integral_constant;
+    const int tid = threadIdx.x, lane = tid & 63, nSp = at.nSp, split = at.split, oBlock = at.oBlock, o0 = at.o0, t0 = at.t0;
+    const int W = s.W, H = s.H, I = s.I, plane = W * H;
+    const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX};
+    auto scale = [&](int ol) { return scaleT ? scaleT[ol] : kSplitUnscale; };
     constexpr int EO = 8 * KW, NP = OB / EO;        // output channels finished per pass, passes
     const int et = tid & 31, eo = tid >> 5;
     const int etg = t0 + et;
@@ -422,7 +288,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                     y = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
                     again &= ~(1u << q);
                 }
-                if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2, kSplitUnscale);
+                if (eOk && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, ox, oy, s.vec2, scale(ol));
             }
             if (__builtin_expect(givenUp != 0, 0)) {
                 int spins = s.joinSpins;
@@ -438,16 +304,17 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
         }
     } else {
         f32x4 y[NP];                                    // (read in one go: with each store behind its own reads the notes cost the trunk
-        float b[NP];                                    // 4.5 us)
+        float b[NP], f[NP];                             // 4.5 us)
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
             y[q] = tile_of(eo + EO * q);
             b[q] = biasT[eo + EO * q];
+            f[q] = scale(eo + EO * q);
             note(q, y[q]);
         }
 #pragma unroll
         for (int q = 0; q < NP; ++q)
-            if (eOk && o0 + eo + EO * q < s.O) wino_finish(out, y[q], b[q], s.flags, o0 + eo + EO * q, plane, W, H, ox, oy, s.vec2, kSplitUnscale);
+            if (eOk && o0 + eo + EO * q < s.O) wino_finish(out, y[q], b[q], s.flags, o0 + eo + EO * q, plane, W, H, ox, oy, s.vec2, f[q]);
     }
 
     // ---- tiles that did not come out finite --------------------------------------------------------------------------------
@@ -458,10 +325,11 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     if (__builtin_expect(any == 0, 1)) return;          // (expected: otherwise what follows lies between instructions that every launch
                                                         // fetches, and a trunk of 640x480 takes 713 us instead of 702)
     constexpr int C = 2 * NP, S = 64 / C;               // channels of this wave, lanes per channel
+    constexpr int PARTS = Bank::PARTS, FRAG = 4 * PARTS * 64;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
     const __amdgpu_buffer_rsrc_t rAll = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, I * plane * 4, kBufferFlags);
     const int part = lane / C, pass = lane % C >> 1, ol = 2 * (tid >> 6) + (lane & 1) + EO * pass;
-    const u32x4b* uLane = (const u32x4b*)U + (size_t)min(oBlock * NT + (ol >> 5), s.nOB - 1) * 768 + (ol & 31);
+    const u32x4b* uLane = (const u32x4b*)U + (size_t)min(oBlock * NT + (ol >> 5), s.nOB - 1) * FRAG + (ol & 31);
     for (unsigned bad = (unsigned)any | (unsigned)(any >> 32); bad != 0; bad &= bad - 1) {
         const int t = __builtin_ctz(bad), ty = fast_div(t0 + t, tilesXd), x0 = 2 * (t0 + t - ty * s.tilesX) - 1, y0 = 2 * ty - 1;
         // A NaN among the samples at the tile's own four pixels reaches all four outputs, whatever the others are.
@@ -481,7 +349,7 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
             float m[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma clang loop unroll(disable)
             for (int c8 = part; c8 < 2 * s.nC; c8 += S) {       // eight channels, half of a chunk
-                const u32x4b* u = uLane + (size_t)(r * s.nC + (c8 >> 1)) * s.nOB * 768 + 32 * (c8 & 1);
+                const u32x4b* u = uLane + (size_t)(r * s.nC + (c8 >> 1)) * s.nOB * FRAG + 32 * (c8 & 1);
                 float v[8][4];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
@@ -498,11 +366,15 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
                 }
 #pragma unroll
                 for (int x = 0; x < 4; ++x) {
-                    const u32x4b hi = u[3 * x * 64], mid = u[(3 * x + 1) * 64], lo = u[(3 * x + 2) * 64];
+                    u32x4b parts[PARTS];
+#pragma unroll
+                    for (int q = 0; q < PARTS; ++q) parts[q] = u[(PARTS * x + q) * 64];
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
-                        auto of = [&](u32x4b q) { return j & 1 ? q[j / 2] >> 16 : q[j / 2] & 0xffffu; };
-                        m[x] = fmaf(whole(of(hi), of(mid), of(lo)), v[j][x], m[x]);
+                        unsigned of[PARTS];
+#pragma unroll
+                        for (int q = 0; q < PARTS; ++q) of[q] = j & 1 ? parts[q][j / 2] >> 16 : parts[q][j / 2] & 0xffffu;
+                        m[x] = fmaf(Bank::whole(of, scale(ol)), v[j][x], m[x]);
                     }
                 }
             }
@@ -519,13 +391,484 @@ winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __
     }
 }
 
-struct WsPlan { int kw, wc, perXcd; bool turns; size_t lds; WsShape s; };
+template <int KW, int WC, bool TURNS>
+__global__ void __launch_bounds__(256 * KW, 2)
+winograd_f23_split_kernel(const float* __restrict__ in, const unsigned short* __restrict__ U, const float* __restrict__ bias,
+                          float* __restrict__ out, WsShape s, float* __restrict__ ws) {
+    constexpr int NT = 2, OB = 32 * NT;
+    using Samples = WsSamples<KW, WC, TURNS>;
+    constexpr int CHB = Samples::CHB, ROWB = Samples::ROWB, BUFB = Samples::BUFB, NDMA = Samples::NDMA;
+    constexpr int kPA[6] = {0, 0, 0, 1, 1, 2}, kPB[6] = {2, 1, 0, 1, 0, 0}; // partial products: part of the filter, part of the sample
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ float biasT[OB];
+
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const WsPlace<KW> at(s);
+    if (!at.ok) return;
+    const int wave = at.wave, set = at.set, first = at.first, steps = at.steps, oBlock = at.oBlock, o0 = at.o0, W = s.W;
+    const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX};
+    const int ty0 = fast_div(at.t0, tilesXd), off0 = at.t0 - ty0 * s.tilesX, turn = TURNS ? min(at.inXcd & 31, steps - 1) : 0;
+    Samples fetched(in, lds, s, at, ty0, off0, turn);
+    auto fetch_sample = [&](int buf, int i) { fetched.fetch(buf, i); };
+
+    // ---- filters ---------------------------------------------------------------------------------------------------
+    // The waits for samples count the filter loads issued behind them, so these must stay where they stand: an address whose
+    // origin the compiler does not see keeps it from taking them for loads that no memory clobber concerns.
+    const unsigned short* uHere = U;
+    asm volatile("" : "+s"(uHere));
+    const int uBytes = 16 * s.nC * 3 * s.nOB * 1024;
+    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, uBytes, kBufferFlags);
+    unsigned uOb[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) uOb[nt] = (unsigned)((wave * s.nC * s.nOB + min(oBlock * NT + nt, s.nOB - 1)) * 12288);
+    const unsigned uStep = (unsigned)s.nOB * 12288u;
+    // (what the last step requests for one behind it comes from nowhere)
+    __amdgpu_buffer_rsrc_t rNext = rU;
+    // the first part of two positions and the others of one: no more registers are left
+    u32x4b f0[2][NT], f12[NT][2];
+    auto filter = [&](int e, int nt, int q) -> u32x4b& { return q == 0 ? f0[e & 1][nt] : f12[nt][q - 1]; };
+    auto load_filter = [&](const __amdgpu_buffer_rsrc_t& from, int e, int nt, int q, int step) {
+        filter(e, nt, q) = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 3072)), 0));
+    };
+
+    // ---- operands --------------------------------------------------------------------------------------------------
+    const int rowA = wave, rowB = wave < 2 ? 2 : 1;
+    const float sgn = wave == 1 ? 1.0f : -1.0f;
+    const int lr = fast_div(l32 + off0, tilesXd), tx = l32 + off0 - lr * s.tilesX;
+    const int firstTx = lr == 0 ? off0 : 0;
+    const int rLds = half * 8 * CHB + 4 * (Samples::segment_at(s, off0, lr) + 2 * (tx - firstTx) - (firstTx == 0 ? 1 : 0));
+    // the masks of the samples beside the map carry the scale of the split as well
+    const float k0f = tx > 0 ? kSplitScale : 0.0f, k2f = 2 * tx + 1 < W ? kSplitScale : 0.0f, k3f = 2 * tx + 2 < W ? kSplitScale : 0.0f;
+    float mm[8][4];                                 // combined window rows of this lane's tile, 8 channels
+    float ra[4], rb[4];                             // a channel's rows on their way from LDS
+    const char* samples = lds + set * 3 * BUFB;
+    auto read_rows = [&](int buf, int j) {
+        const float* a = (const float*)(samples + buf * BUFB + rowA * ROWB + rLds + j * CHB);
+        const float* b = (const float*)(samples + buf * BUFB + rowB * ROWB + rLds + j * CHB);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { ra[c] = a[c]; rb[c] = b[c]; }
+    };
+    auto combine = [&](int j) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mm[j][c] = fmaf(sgn, rb[c], ra[c]);
+        mm[j][1] *= kSplitScale;                    // (the other two are multiplied where they are used)
+        mm[j][2] *= k2f;
+    };
+    u32x4b B[2][3];                                 // [position parity][part]
+    float va[2], vb[2], xa[2], xb[2];               // the two items being split
+    auto vvalue = [&](int e, int c) {
+        return e == 0 ? fmaf(k0f, mm[c][0], -mm[c][2]) : e == 1 ? mm[c][1] + mm[c][2] : e == 2 ? mm[c][2] - mm[c][1] : fmaf(k3f, mm[c][3], -mm[c][1]);
+    };
+    auto pack = [&](float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2b{a, b}, bf16x2)); };
+    // The operands of position e out of mm: 12 ticks for two items (an item is two channels), whose instructions
+    // alternate: a vector instruction that needs the result of the one in front of it waits for it.
+    auto split_tick = [&](int e, int tick) {
+        const int u = tick / 12, k = tick % 12;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int p = 2 * u + x;
+            u32x4b(&d)[3] = B[e & 1];
+            if (k == 0) va[x] = vvalue(e, 2 * p);
+            if (k == 1) vb[x] = vvalue(e, 2 * p + 1);
+            if (k == 2 || k == 7 || k == 11) d[k == 2 ? 0 : k == 7 ? 1 : 2][p] = pack(va[x], vb[x]);
+            if (k == 3 || k == 8) xa[x] = __builtin_bit_cast(float, d[k == 3 ? 0 : 1][p] << 16);
+            if (k == 4 || k == 8) xb[x] = __builtin_bit_cast(float, d[k == 4 ? 0 : 1][p] & 0xffff0000u);
+            if (k == 5 || k == 9) va[x] -= xa[x];
+            if (k == 6 || k == 10) vb[x] -= xb[x];
+        }
+    };
+
+    f32x16b acc[4][NT];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[e][nt][r] = 0.0f;
+
+    // ---- prologue --------------------------------------------------------------------------------------------------
+    float biasEarly = 0.0f;
+    if (tid < OB && bias) biasEarly = bias[min(o0 + tid, s.O - 1)];
+    asm volatile("" ::: "memory");
+    // What the first products need comes first, the rest behind the barrier.
+#pragma unroll
+    for (int i = 0; i < (KW == 1 ? 2 : 1) * NDMA; ++i) fetch_sample(i / NDMA, i % NDMA);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) load_filter(rU, 0, nt, q, first + set + KW * turn);
+    if (tid < OB) biasT[tid] = biasEarly;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NT + (KW == 1 ? NDMA : 0)) : "memory");
+    ws_barrier();
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) if (KW == 2) fetch_sample(1, i);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) load_filter(rU, 1, nt, 0, first + set + KW * turn);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { read_rows(0, j); combine(j); }
+#pragma unroll
+    for (int t = 0; t < 24; ++t) split_tick(0, t);
+
+    // ---- steps -----------------------------------------------------------------------------------------------------
+    // A position is 12 MFMAs, one per slot; with each go two ticks of the next position's operands and what else is due.
+    auto position = [&](auto ec, int step, int stepNext, int nxt, int nxt2) {
+        constexpr int e = decltype(ec)::value;
+#pragma unroll
+        for (int i = 0; i < 6 * NT; ++i) {
+            const int q = i / NT, nt = i % NT;
+            acc[e][nt] = mfma_bf16(filter(e, nt, kPA[q]), B[e & 1][kPB[q]], acc[e][nt]);
+            // a part's last product has been issued: its registers take the filters that come next
+            if (q == 2 || q == 4 || q == 5) {
+                const int by = q == 2 ? 2 : 1;
+                load_filter(e + by >= 4 ? rNext : rU, (e + by) & 3, nt, kPA[q], e + by >= 4 ? stepNext : step);
+            }
+#pragma unroll
+            for (int tk = 2 * i; tk < 2 * i + 2; ++tk) {
+                split_tick((e + 1) & 3, tk);
+                const int at = 24 * e + tk;         // 0..95 over the step
+                if (at % 4 == 0 && at / 4 < NDMA) fetch_sample(nxt2, at / 4);
+                // Rows of the next step, one channel after the other: read, and some ticks later combined, behind the last
+                // use of what they replace and in front of their own first use.
+                constexpr int kRead[8] = {46, 52, 57, 62, 67, 71, 76, 80}, kComb[8] = {51, 56, 61, 66, 70, 75, 79, 83};
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    if (at == kComb[j]) combine(j);
+                    if (at == kRead[j]) read_rows(nxt, j);
+                }
+            }
+            // The next step's samples, requested a step ago, have to be visible before they are read.  (Younger than them are this
+            // step's fetch and at least the filters of a position: more than the count waited for.)
+            if (24 * e + 2 * i + 2 == 36) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + 4 * NT) : "memory");
+                ws_barrier();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using std::integral_constant;
+    int nxt = 1, nxt2 = 2;
+    for (int n = 0, m = turn; n < steps; ++n) {
+        const int step = first + set + KW * m;
+        m = TURNS && m == steps - 1 ? 0 : m + 1;
+        const int stepNext = first + set + KW * m;
+        rNext = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, n + 1 < steps ? uBytes : 0, kBufferFlags);
+        position(integral_constant<int, 0>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 1>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 2>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 3>{}, step, stepNext, nxt, nxt2);
+        nxt = nxt2;
+        nxt2 = nxt2 == 2 ? 0 : nxt2 + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (fetches beyond the last step, of every wave: LDS is about to be used for
+    ws_barrier();                                              // something else)
+
+    // ---- epilogue --------------------------------------------------------------------------------------------------
+    // D of the 32x32 MFMA: lane -> tile lane%32; register r -> channel 8*(r/4) + 4*(lane/32) + r%4.  Each wave reduces its row of the
+    // transform to two columns, the rows (and the two sets) meet in LDS.
+    float* P = (float*)lds;                         // [set][row][2][OB][32]
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float m0 = acc[0][nt][r], m1 = acc[1][nt][r], m2 = acc[2][nt][r], m3 = acc[3][nt][r];
+            const int ol = 32 * nt + 8 * (r / 4) + 4 * half + (r % 4);
+            P[(((set * 4 + wave) * 2 + 0) * OB + ol) * 32 + l32] = m0 + m1 + m2;
+            P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + l32] = m1 - m2 + m3;
+        }
+    ws_barrier();
+    ws_finish<KW, WsBf16x3>(P, biasT, nullptr, s, at, in, U, out, ws);
+}
+
+// ---- two f16 parts ---------------------------------------------------------------------------------------------------------
+
+// The bank of two f16 parts: U[row][chunk][o/32][position in the row][part][lane][8], the filters of output channel o multiplied by a power of two;
+// behind it, by output channel, what their sums are to be multiplied by.
+struct WsF16x2 {
+    static constexpr int PARTS = 2;
+    __device__ __forceinline__ static float whole(const unsigned (&part)[PARTS], float scale) {
+        return scale * (float)__builtin_bit_cast(f16x2h, part[0])[0] + scale * (float)__builtin_bit_cast(f16x2h, part[1])[0];
+    }
+};
+
+// scale[o]: 2^-k, where 2^k brings the largest weight of output channel o to 2^13 .. 2^14.  Transformed filters are at most 2.25 times as large, and
+// at least a quarter.
+__global__ void __launch_bounds__(256)
+wino_pair_scale_kernel(const float* __restrict__ w, float* __restrict__ scale, int I, int O) {
+    __shared__ float part[4];
+    const int o = blockIdx.x;
+    float m = 0.0f;
+    if (o < O)
+        for (int k = threadIdx.x; k < 9 * I; k += 256) m = fmaxf(m, fabsf(w[((size_t)(k / 9) * O + o) * 9 + k % 9]));
+    for (int k = 1; k < 64; k *= 2) m = fmaxf(m, __shfl_xor(m, k));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+        const int e = (int)(__float_as_uint(m) >> 23) - 127;
+        scale[o] = m == 0.0f ? 1.0f : __uint_as_float((unsigned)(127 + max(min(e - 13, 114), -126)) << 23);
+    }
+}
+
+__global__ void __launch_bounds__(256)
+wino_pair_filter_kernel(const float* __restrict__ w, unsigned short* __restrict__ U, const float* __restrict__ scale, int I, int O, int nC, int nOB) {
+    const int row = threadIdx.x >> 6, lane = threadIdx.x & 63, ob = blockIdx.x % nOB, chunk = blockIdx.x / nOB;
+    const int c0 = chunk * 16 + 8 * (lane >> 5), o = ob * 32 + (lane & 31);
+    const float up = __uint_as_float((254u << 23) - __float_as_uint(scale[o]));
+    float u[8][4];                                  // the row's four positions of eight channels
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float all[16] = {};
+        if (c0 + e < I && o < O) wino_filter_transform(w + ((size_t)(c0 + e) * O + o) * 9, all);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) u[e][x] = up * (row == 0 ? all[x] : row == 1 ? all[4 + x] : row == 2 ? all[8 + x] : all[12 + x]);
+    }
+    u32x4b* d = (u32x4b*)U + ((size_t)(row * nC + chunk) * nOB + ob) * 8 * 64 + lane;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        u32x4b hi, lo;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            hi[p] = pack_f16(u[2 * p][x], u[2 * p + 1][x]);
+            lo[p] = pack_f16(f16_rest(u[2 * p][x], hi[p], 0, -1.0f), f16_rest(u[2 * p + 1][x], hi[p], 1, -1.0f));
+        }
+        d[(2 * x) * 64] = hi;
+        d[(2 * x + 1) * 64] = lo;
+    }
+}
+
+// One word per lane, by byte offset, to consecutive words of LDS.
+__device__ __forceinline__ void ws_word_to_lds(__amdgpu_buffer_rsrc_t from, int offset, const float* to) {
+    const unsigned at = (unsigned)(size_t)(__attribute__((address_space(3))) const float*)to;
+    unsigned m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0) : "v"(offset), "s"(from), "s"(at) : "memory");
+}
+
+// Winograd on the f16 matrix cores, operands in two parts (f16x2.hpp): the three-part kernel's panels, waves, steps and pieces, with 24 MFMAs a wave and
+// step instead of 48, 16 KiB of filters instead of 24 and 176 vector instructions instead of 270.  Layers, us, three parts / two, with their errors
+// against 64 bits (rms, 1e-7): 640x480 64->64 85 / 67 (2.2 / 1.9), 320x240 128->128 75.0 / 56.9 (2.8 / 2.3), 160x120 256->256 73.6 / 54.1 (3.7 / 2.9),
+// 80x60 512->512 75.7 / 54.7 (3.7 / 2.9), 112x112 128->128 16.0 / 13.0 (2.1 / 1.9), 40x30 512->512 27.8 / 22.0 (2.5 / 2.2).
+// What bounds it: two workgroups of a CU take 4480 clocks a step on 320x240, the fetches without the MFMAs 2630 (168 KB at 64 bytes a clock), MFMAs and vector
+// instructions without fetches 1940: eight fragments of filters under way per wave do not cover the way to L2 while a CU's eight waves queue there.
+template <int KW, int WC, bool TURNS>
+__global__ void __launch_bounds__(256 * KW, 2)
+winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __restrict__ U, const float* __restrict__ bias,
+                         float* __restrict__ out, WsShape s, float* __restrict__ ws) {
+    constexpr int NT = 2, OB = 32 * NT;
+    using Samples = WsSamples<KW, WC, TURNS>;
+    constexpr int CHB = Samples::CHB, ROWB = Samples::ROWB, BUFB = Samples::BUFB, NDMA = Samples::NDMA;
+    constexpr int kPA[3] = {1, 0, 0}, kPB[3] = {0, 1, 0};   // partial products: part of the filter, part of the sample
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ float biasT[OB], scaleT[OB];
+
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const WsPlace<KW> at(s);
+    if (!at.ok) return;
+    const int wave = at.wave, set = at.set, first = at.first, steps = at.steps, oBlock = at.oBlock, o0 = at.o0, W = s.W;
+    const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX};
+    const int ty0 = fast_div(at.t0, tilesXd), off0 = at.t0 - ty0 * s.tilesX, turn = TURNS ? min(at.inXcd & 31, steps - 1) : 0;
+    Samples fetched(in, lds, s, at, ty0, off0, turn);
+
+    // ---- filters ---------------------------------------------------------------------------------------------------
+    // (an address whose origin the compiler does not see, for the reason that the three-part kernel has)
+    const unsigned short* uHere = U;
+    asm volatile("" : "+s"(uHere));
+    const int uBytes = 16 * s.nC * 2 * s.nOB * 1024;
+    const __amdgpu_buffer_rsrc_t rU = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, uBytes, kBufferFlags);
+    unsigned uOb[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) uOb[nt] = (unsigned)((wave * s.nC * s.nOB + min(oBlock * NT + nt, s.nOB - 1)) * 8192);
+    const unsigned uStep = (unsigned)s.nOB * 8192u;
+    __amdgpu_buffer_rsrc_t rNext = rU;              // (what the last step requests for one behind it comes from nowhere)
+    u32x4b f[2][NT][2];                             // of two positions
+    auto load_filter = [&](const __amdgpu_buffer_rsrc_t& from, int e, int nt, int q, int step) {
+        f[e & 1][nt][q] = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 2048)), 0));
+    };
+
+    // ---- operands --------------------------------------------------------------------------------------------------
+    // A column of tiles (a lane and the one 32 on) has its samples multiplied by a power of two of its own, `scale`, so that the largest that the wave
+    // has met is below 2^14 once two rows of the window are combined, and was 2^11 or more when the scale was chosen.  A step that brings a larger one
+    // lowers the scale, and what has been summed up with it, before its products begin.  As long as all samples are zero any scale will do.
+    const int rowA = wave, rowB = wave < 2 ? 2 : 1;
+    const float sgn = wave == 1 ? 1.0f : -1.0f;
+    const int lr = fast_div(l32 + off0, tilesXd), tx = l32 + off0 - lr * s.tilesX;
+    const int firstTx = lr == 0 ? off0 : 0;
+    const int rLds = half * 8 * CHB + 4 * (Samples::segment_at(s, off0, lr) + 2 * (tx - firstTx) - (firstTx == 0 ? 1 : 0));
+    float k[4] = {tx > 0 ? 1.0f : 0.0f, 1.0f, 2 * tx + 1 < W ? 1.0f : 0.0f, 2 * tx + 2 < W ? 1.0f : 0.0f};      // masks of the columns of the window, with the scale
+    constexpr float kLimit = 0x1p14f;
+    float limit = kLimit, most = 0.0f;              // of the samples that come next
+    float minusOne;
+    asm volatile("s_mov_b32 %0, 0xbf800000" : "=s"(minusOne));
+    float mm[8][4];                                 // combined window rows of this lane's tile, 8 channels
+    float ra[3][2], rb[3][2];                       // two channels' samples of a column on their way from LDS, of three columns
+    const char* samples = lds + set * 3 * BUFB;
+    auto read_two = [&](int buf, int slot, int c, int j) {
+        const float* a = (const float*)(samples + buf * BUFB + rowA * ROWB + rLds + j * CHB) + c;
+        const float* b = (const float*)(samples + buf * BUFB + rowB * ROWB + rLds + j * CHB) + c;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) { ra[slot][x] = a[x * (CHB / 4)]; rb[slot][x] = b[x * (CHB / 4)]; }
+    };
+    auto combine_two = [&](int slot, int c, int j) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) mm[j + x][c] = k[c] * fmaf(sgn, rb[slot][x], ra[slot][x]);
+        most = fmaxf(fmaxf(fabsf(mm[j][c]), fabsf(mm[j + 1][c])), most);
+    };
+    u32x4b B[2][2];                                 // [position parity][part]
+    float va[2], vb[2];                             // the two items being split
+    auto vvalue = [&](int e, int c) {
+        return e == 0 ? mm[c][0] - mm[c][2] : e == 1 ? mm[c][1] + mm[c][2] : e == 2 ? mm[c][2] - mm[c][1] : mm[c][3] - mm[c][1];
+    };
+    // The operands of position e out of mm: 6 ticks for two items (an item is two channels), whose instructions alternate.
+    auto split_tick = [&](int e, int tick) {
+        const int u = tick / 6, n = tick % 6;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int p = 2 * u + x;
+            u32x4b(&d)[2] = B[e & 1];
+            if (n == 0) va[x] = vvalue(e, 2 * p);
+            if (n == 1) vb[x] = vvalue(e, 2 * p + 1);
+            if (n == 2) d[0][p] = pack_f16(va[x], vb[x]);
+            if (n == 3) va[x] = f16_rest(va[x], d[0][p], 0, minusOne);
+            if (n == 4) vb[x] = f16_rest(vb[x], d[0][p], 1, minusOne);
+            if (n == 5) d[1][p] = pack_f16(va[x], vb[x]);
+        }
+    };
+
+    f32x16b acc[4][NT];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[e][nt][r] = 0.0f;
+
+    // The scale that suits `most`, and everything that has been multiplied by the old one with it.
+    auto rescale = [&](bool sums) {
+        const float largest = fmaxf(most, __shfl_xor(most, 32));
+        const int e = (int)(__float_as_uint(largest) >> 23) - 127, has = (int)(__float_as_uint(k[1]) >> 23) - 127;
+        const bool lower = largest >= limit && e < 128;         // (an infinity stays one whatever the scale)
+        const int by = lower ? min(11 - e, 126 - has) : 0, by2 = by / 2;       // (in two factors: it goes down to -240)
+        // Samples that no scale makes large enough, fp32 denormals, are left to the pass over what did not come out finite.
+        const float f1 = e + by < 1 && lower ? __builtin_nanf("") : __uint_as_float((unsigned)(127 + by2) << 23), f2 = __uint_as_float((unsigned)(127 + by - by2) << 23);
+        auto times = [&](float x) { return x * f1 * f2; };
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            k[c] = times(k[c]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) mm[j][c] = times(mm[j][c]);
+        }
+        if (lower) limit = kLimit;
+        if (sums)
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[x][nt][r] = times(acc[x][nt][r]);
+#pragma unroll
+        for (int t = 0; t < 12; ++t) split_tick(0, t);
+    };
+
+    // ---- prologue --------------------------------------------------------------------------------------------------
+    if (wave == 0 && set == 0) {                    // to LDS as well; what does not exist, a missing bias among it, arrives as zeros
+        const __amdgpu_buffer_rsrc_t rBias = __builtin_amdgcn_make_buffer_rsrc((void*)bias, 0, bias ? 4 * s.O : 0, kBufferFlags);
+        const __amdgpu_buffer_rsrc_t rScale = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)U + uBytes), 0, 128 * s.nOB, kBufferFlags);
+        ws_word_to_lds(rBias, 4 * (o0 + lane), biasT);
+        ws_word_to_lds(rScale, 4 * (o0 + lane), scaleT);
+    }
+    // What the first products need comes first, the rest behind the barrier.
+#pragma unroll
+    for (int i = 0; i < (KW == 1 ? 2 : 1) * NDMA; ++i) fetched.fetch(i / NDMA, i % NDMA);
+#pragma unroll
+    for (int q = 0; q < 2 * NT; ++q) load_filter(rU, 0, q & 1, kPA[q / 2], first + set + KW * turn);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NT + (KW == 1 ? NDMA : 0)) : "memory");
+    ws_barrier();
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) if (KW == 2) fetched.fetch(1, i);
+#pragma unroll
+    for (int q = 0; q < 2 * NT; ++q) load_filter(rU, 1, q & 1, kPA[q / 2], first + set + KW * turn);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) { read_two(0, n % 3, n / 4, 2 * (n % 4)); combine_two(n % 3, n / 4, 2 * (n % 4)); }
+    {   // the first scale: for `most` where it is not zero
+        limit = 0x1p-149f;
+        rescale(false);
+        const bool none = limit < kLimit;
+        if (none) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) k[c] *= 0x1p64f;
+        }
+        most = 0.0f;
+    }
+
+    // ---- steps -----------------------------------------------------------------------------------------------------
+    // A position is 6 MFMAs, one per slot; with each go two ticks of the next position's operands and what else is due.
+    auto position = [&](auto ec, int step, int stepNext, int nxt, int nxt2) {
+        constexpr int e = decltype(ec)::value;
+#pragma unroll
+        for (int i = 0; i < 3 * NT; ++i) {
+            const int q = i / NT, nt = i % NT, slot = 6 * e + i;        // slot: 0..23 over the step
+            acc[e][nt] = mfma_f16(f[e & 1][nt][kPA[q]], B[e & 1][kPB[q]], acc[e][nt]);
+            // a part's last product has been issued: its registers take the filters of the position after the next
+            if (q != 1) load_filter(e >= 2 ? rNext : rU, (e + 2) & 3, nt, kPA[q], e >= 2 ? stepNext : step);
+            split_tick((e + 1) & 3, 2 * i);
+            split_tick((e + 1) & 3, 2 * i + 1);
+            // The samples of the next step, two channels of a column at a time, read and two slots later combined, behind the last use of
+            // what they replace: the first column is used by the first position alone, the third by the first three.
+            if (slot >= 8) combine_two((slot - 8) % 3, (slot - 8) / 4 == 1 ? 2 : (slot - 8) / 4 == 2 ? 1 : (slot - 8) / 4, 2 * ((slot - 8) % 4));
+            if (slot >= 6 && slot < 22) read_two(nxt, (slot - 6) % 3, (slot - 6) / 4 == 1 ? 2 : (slot - 6) / 4 == 2 ? 1 : (slot - 6) / 4, 2 * ((slot - 6) % 4));
+            if (slot % 4 == 0 && slot / 4 < NDMA) fetched.fetch(nxt2, slot / 4);
+            // The next step's samples, requested a step ago, have to be visible before they are read.  (Younger than them are filters behind
+            // slot 16, or 20, of the step before, or of the prologue, those of this position and two loads for the step after.)
+            if (slot == 5) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA == 5 ? 10 : 8) : "memory");
+                ws_barrier();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using std::integral_constant;
+    int nxt = 1, nxt2 = 2;
+    for (int n = 0, m = turn; n < steps; ++n) {
+        const int step = first + set + KW * m;
+        m = TURNS && m == steps - 1 ? 0 : m + 1;
+        const int stepNext = first + set + KW * m;
+        rNext = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, n + 1 < steps ? uBytes : 0, kBufferFlags);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(most >= limit) != 0, 0)) rescale(true);
+        most = 0.0f;
+        position(integral_constant<int, 0>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 1>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 2>{}, step, stepNext, nxt, nxt2);
+        position(integral_constant<int, 3>{}, step, stepNext, nxt, nxt2);
+        nxt = nxt2;
+        nxt2 = nxt2 == 2 ? 0 : nxt2 + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (fetches beyond the last step, of every wave: LDS is about to be used for
+    ws_barrier();                                           // something else)
+
+    // ---- epilogue --------------------------------------------------------------------------------------------------
+    float* P = (float*)lds;                         // [set][row][2][OB][32]
+    const float back = __uint_as_float((254u << 23) - __float_as_uint(k[1]));
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float m0 = acc[0][nt][r], m1 = acc[1][nt][r], m2 = acc[2][nt][r], m3 = acc[3][nt][r];
+            const int ol = 32 * nt + 8 * (r / 4) + 4 * half + (r % 4);
+            P[(((set * 4 + wave) * 2 + 0) * OB + ol) * 32 + l32] = back * (m0 + m1 + m2);
+            P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + l32] = back * (m1 - m2 + m3);
+        }
+    ws_barrier();
+    ws_finish<KW, WsF16x2>(P, biasT, scaleT, s, at, in, U, out, ws);
+}
+
+struct WsPlan { int kw, wc, perXcd; bool turns, pair; size_t lds; WsShape s; };
 
 // Variant: 0x100 | wave sets - 1 | sA << 12 | sB << 16 | nA << 20, where the first nA output panels of every XCD are cut into
 // sA splits (1 to 4, with one wave set 1 or 2) of their input channels and the others into sB; all zero: nothing is split.
 static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
-    if (variant < 0 || (variant & 0xffe) != 0x100 || W < 1 || H < 1 || I < 1 || O < 1) return false;
+    if (variant < 0 || (variant & 0xdfe) != 0x100 || W < 1 || H < 1 || I < 1 || O < 1) return false;
     p->kw = 1 + (variant & 1);
+    p->pair = (variant & 0x200) != 0;
     WsShape& s = p->s;
     s.W = W; s.H = H; s.I = I; s.O = O;
     s.tilesX = (W + 1) / 2;
@@ -567,12 +910,19 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
            (long long)p->perXcd * kXcds * 32768 < (1ll << 31);
 }
 
-template <int KW, int WC, bool TURNS>
+template <int KW, int WC, bool TURNS, bool PAIR>
 static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, float* ws, const WsPlan& p, hipStream_t st) {
+    constexpr auto kernel = PAIR ? winograd_f23_pair_kernel<KW, WC, TURNS> : winograd_f23_split_kernel<KW, WC, TURNS>;
     static std::atomic<unsigned long long> asked{0};
-    if (int rc = allow_lds((const void*)winograd_f23_split_kernel<KW, WC, TURNS>, p.lds, asked)) return rc;
-    launch((winograd_f23_split_kernel<KW, WC, TURNS>), dim3(p.perXcd * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s, ws);
-    return launched("winograd_f23_split_kernel");
+    if (int rc = allow_lds((const void*)kernel, p.lds, asked)) return rc;
+    launch(kernel, dim3(p.perXcd * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s, ws);
+    return launched(PAIR ? "winograd_f23_pair_kernel" : "winograd_f23_split_kernel");
+}
+template <bool PAIR>
+static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, float* ws, const WsPlan& p, hipStream_t st) {
+    if (p.wc == 24) return p.turns ? launch_ws<2, 24, true, PAIR>(in, U, bias, out, ws, p, st) : launch_ws<2, 24, false, PAIR>(in, U, bias, out, ws, p, st);
+    if (p.kw == 2) return p.turns ? launch_ws<2, 20, true, PAIR>(in, U, bias, out, ws, p, st) : launch_ws<2, 20, false, PAIR>(in, U, bias, out, ws, p, st);
+    return p.turns ? launch_ws<1, 20, true, PAIR>(in, U, bias, out, ws, p, st) : launch_ws<1, 20, false, PAIR>(in, U, bias, out, ws, p, st);
 }
 
 int ws_join_timeouts(unsigned* count) {
@@ -631,6 +981,13 @@ extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, in
     return nC >= 4 || (nC >= 2 && 2 * blocks >= 3 * cus) ? 0x100 : 0;
 }
 
+// Two f16 parts instead of three bf16 ones, where the kernel of split operands is taken at all and from 64 input channels on: with fewer its sums
+// are less exact (16 channels 1.34 against 1.11e-7 rms, 32 channels 1.45 against 1.32).
+extern "C" int drhip_conv3x3_winograd_pair_pick_variant(int W, int H, int I, int O) {
+    const int v = I >= 64 ? drhip_conv3x3_winograd_split_pick_variant(W, H, I, O) : 0;
+    return v ? v | 0x200 : 0;
+}
+
 extern "C" size_t drhip_conv3x3_winograd_split_filter_floats(int I, int O) {
     return I <= 0 || O <= 0 ? 0 : (size_t)ceil_div(I, kWsKC) * ceil_div(O, 32) * 12288;
 }
@@ -650,6 +1007,49 @@ extern "C" int drhip_winograd_split_filter_transform_f32(const float* w, float* 
     return launched("wino_split_filter_kernel");
 }
 
+extern "C" size_t drhip_conv3x3_winograd_pair_filter_floats(int I, int O) {
+    return I <= 0 || O <= 0 ? 0 : (size_t)ceil_div(O, 32) * ((size_t)ceil_div(I, kWsKC) * 8192 + 32);
+}
+
+// Magnitudes by their bits, which are in the same order and put NaN last: of every output channel its smallest filter's and its largest's
+// largest weight.
+template <int TAPS>
+static void filter_range(const float* w, int I, int O, unsigned* least, unsigned* largest) {
+    for (int c = 0; c < I; ++c)
+        for (int o = 0; o < O; ++o, w += TAPS) {
+            unsigned bits[TAPS], most[2] = {0u, 0u};
+            memcpy(bits, w, sizeof bits);
+#pragma unroll
+            for (int k = 0; k < TAPS; ++k) most[k % 2] = std::max(most[k % 2], bits[k] << 1);
+            most[0] = std::max(most[0], most[1]);
+            least[o] = std::min(least[o], most[0]);
+            largest[o] = std::max(largest[o], most[0]);
+        }
+}
+
+// A channel's weights next to the largest of its output channel: where one is below 2^-12 of it, and samples of that channel may be as
+// much larger than the others, what the scaled parts lose could show.  (Weights that are random or trained and not pruned are far from that.)
+extern "C" int drhip_winograd_pair_fits(const float* w, int I, int O, int taps) {
+    if (!w || I <= 0 || O <= 0 || (taps != 1 && taps != 9)) return 0;
+    std::vector<unsigned> least((size_t)O, ~0u), largest((size_t)O, 0u);
+    (taps == 1 ? filter_range<1> : filter_range<9>)(w, I, O, least.data(), largest.data());
+    auto power = [](int e) { return (unsigned)(127 + e) << 24; };       // the bits of 2^e
+    for (int o = 0; o < O; ++o)
+        if (largest[o] != 0 && !(largest[o] >= power(-100) && largest[o] <= power(100) && least[o] + (12u << 24) >= largest[o])) return 0;
+    return 1;
+}
+
+extern "C" int drhip_winograd_pair_filter_transform_f32(const float* w, float* U, int I, int O, void* stream) {
+    DRHIP_REQUIRE(w && U && I > 0 && O > 0, "drhip_winograd_pair_filter_transform_f32: bad arguments");
+    const int nC = ceil_div(I, kWsKC), nOB = ceil_div(O, 32);
+    DRHIP_REQUIRE((long long)nC * nOB * 12288 * 4 < (1ll << 31), "drhip_winograd_pair_filter_transform_f32: %dx%d filters are too many", I, O);
+    float* scale = U + (size_t)nC * nOB * 8192;
+    launch(wino_pair_scale_kernel, dim3(32 * nOB), dim3(256), 0, as_stream(stream), w, scale, I, O);
+    if (int rc = launched("wino_pair_scale_kernel")) return rc;
+    launch(wino_pair_filter_kernel, dim3((unsigned)(nC * nOB)), dim3(256), 0, as_stream(stream), w, (unsigned short*)U, scale, I, O, nC, nOB);
+    return launched("wino_pair_filter_kernel");
+}
+
 extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int flags, int variant, float* workspace, void* stream) {
     DRHIP_REQUIRE(in && U && out, "drhip_conv3x3_winograd_split_f32: NULL tensor");
     DRHIP_REQUIRE((flags & ~(kEpiRelu | kEpiMaxPool2)) == 0, "drhip_conv3x3_winograd_split_f32: unknown epilogue flags %#x", flags);
@@ -662,7 +1062,5 @@ extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U,
     p.s.vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
     const unsigned short* F = (const unsigned short*)U;
     hipStream_t st = as_stream(stream);
-    if (p.wc == 24) return p.turns ? launch_ws<2, 24, true>(in, F, bias, out, workspace, p, st) : launch_ws<2, 24, false>(in, F, bias, out, workspace, p, st);
-    if (p.kw == 2) return p.turns ? launch_ws<2, 20, true>(in, F, bias, out, workspace, p, st) : launch_ws<2, 20, false>(in, F, bias, out, workspace, p, st);
-    return p.turns ? launch_ws<1, 20, true>(in, F, bias, out, workspace, p, st) : launch_ws<1, 20, false>(in, F, bias, out, workspace, p, st);
+    return p.pair ? launch_ws<true>(in, F, bias, out, workspace, p, st) : launch_ws<false>(in, F, bias, out, workspace, p, st);
 }

@@ -17,6 +17,9 @@ inline dR_Conv2d_Data* conv_of(dR_Node* n) { return (dR_Conv2d_Data*)n->layer; }
 inline bool pools_by_three(dR_Node* n) { return ((const dR_Pooling_Data*)((dR_Node*)n->next_layers->first->element)->layer)->shape.s1 == 3; }
 inline int weight_count(const dR_Conv2d_Data* c) { return c->shape.s0 * c->shape.s1 * c->shape.s2 * c->shape.s3; }
 
+// A Winograd layer whose filters lie in two f16 parts.
+inline bool pair_bank(const dR_Conv2d_Data* c) { return c->drWinoSplit && (c->variant & 0x200); }
+
 gboolean conv_propagate(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     if (node->previous_layers->length != 1 && verbose(net))
@@ -67,7 +70,7 @@ gchar* conv_print(dR_Node* node) {
     const char* kernel = c->drFireFrom ? "in the launch of the layers in front"
                        : c->drFire ? (c->drFireNext ? "fire module and the squeeze layer behind it, fp32 MFMA" : "fire module, fp32 MFMA")
                        : c->algo == drConv1x1Gemm ? "1x1 MFMA GEMM"
-                       : c->algo == drConvWinograd ? (c->drWinoSplit ? "Winograd F(2x2,3x3) split-operand bf16 MFMA" : "Winograd F(2x2,3x3) MFMA")
+                       : c->algo == drConvWinograd ? (pair_bank(c) ? "Winograd F(2x2,3x3) split-operand f16 MFMA" : c->drWinoSplit ? "Winograd F(2x2,3x3) split-operand bf16 MFMA" : "Winograd F(2x2,3x3) MFMA")
                        : c->drSplitBank ? "direct, split-operand bf16 MFMA" : c->drDirectBank ? "direct MFMA" : "direct";
     return fmt_dup("Conv2d Layer: %d\n Filter dimensions: %dx%d\n Input channels: %d\n Output channels: %d\n"
                    " Activation: %s\n Stride: %d, %d, %d, %d\n Use bias: %s\n Kernel: %s (variant %d)\n",
@@ -81,6 +84,16 @@ void pick_winograd(dR_Conv2d_Data* c, int O) {
     c->variant = drhip_conv3x3_winograd_split_pick_variant(W, H, I, O);
     c->drWinoSplit = c->variant != 0;
     if (!c->drWinoSplit) c->variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
+}
+
+// Once its weights are known: operands in two f16 parts instead, where those can hold them.
+void pick_winograd_pair(dR_Conv2d_Data* c, int O) {
+    const int v = drhip_conv3x3_winograd_pair_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
+    const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
+    if (v == 0 || !c->hasVariables || (a && !a->hasVariables)) return;
+    if (!drhip_winograd_pair_fits(c->weights, c->shape.s2, c->shape.s3, 9) || (a && !drhip_winograd_pair_fits(a->weights, a->shape.s2, a->shape.s3, 1))) return;
+    c->variant = v;
+    c->drWinoSplit = TRUE;
 }
 
 size_t winograd_workspace_floats(const dR_Conv2d_Data* c, int O) {
@@ -175,10 +188,12 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     const bool wino = c->algo == drConvWinograd;
     const int O = launch_channels(c);
     if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
+    if (wino) pick_winograd_pair(c, O);
     if (c->drSplitBank && c->drFusedPool)
         c->variant = pools_by_three(node) ? drhip_conv_bank_maxpool3s2_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 2)
                                           : drhip_conv_bank_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 1);
-    const int n = c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
+    const int n = pair_bank(c) ? (int)drhip_conv3x3_winograd_pair_filter_floats(c->shape.s2, O)
+                       : c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
                        : wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
                        : c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)
                        : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1)
@@ -251,8 +266,8 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         cl_mem raw = NULL;
         if (!dR_createFloatBuffer(net, &raw, I * O * 9, CL_MEM_READ_ONLY)) return FALSE;
         ok = dR_uploadArray(net, (gchar*)"", (void*)host, 0, rawBytes, raw);
-        if (ok) ok = !device_failed(net, c->drWinoSplit ? drhip_winograd_split_filter_transform_f32((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net))
-                                                       : drhip_winograd_filter_transform_f32((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net)),
+        if (ok) ok = !device_failed(net, (pair_bank(c) ? drhip_winograd_pair_filter_transform_f32 : c->drWinoSplit ? drhip_winograd_split_filter_transform_f32
+                                                       : drhip_winograd_filter_transform_f32)((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net)),
                                     "winograd filter transform");
         if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "winograd filter transform (sync)");
         dR_clMemoryBufferCleanup(net, raw);

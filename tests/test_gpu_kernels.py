@@ -518,6 +518,99 @@ def test_conv_bank_keeps_extreme_weights(lib, dev, I, k, stride, infinite):
     assert_same_extremes(got, want)
 
 
+PAIR = 0x200
+
+
+def pair_winograd(lib, dev, x, w, variant, flags=0, bias=None):
+    """One launch of the kernel of two f16 parts."""
+    (I, H, W), O = x.shape, w.shape[1]
+    F = dev.empty(lib.drhip_conv3x3_winograd_pair_filter_floats(I, O))
+    ok(lib, lib.drhip_winograd_pair_filter_transform_f32(dev.put(w), F, I, O, None))
+    n, ws = lib.drhip_conv3x3_winograd_split_workspace_floats(W, H, I, O, variant | PAIR), None
+    if n:
+        ws = dev.empty(n)
+        ok(lib, lib.drhip_conv3x3_winograd_workspace_prepare_f32(ws, n, None))
+    shape = (O, H // 2, W // 2) if flags & 2 else (O, H, W)
+    y, xd = dev.empty(int(np.prod(shape))), dev.put(x)
+    for _ in range(2):                      # (twice on one workspace)
+        ok(lib, lib.drhip_conv3x3_winograd_split_f32(xd, F, dev.put(bias) if bias is not None else None, y, W, H, I, O, flags, variant | PAIR, ws, None))
+    return dev.get(y, shape)
+
+
+@pytest.mark.parametrize("variant,W,H,I,O", [
+    (0x100, 33, 17, 16, 33), (0x101, 31, 40, 17, 70), (0x100, 61, 63, 64, 128), (0x101, 61, 63, 65, 128), (0x100, 32, 2, 33, 65), (0x101, 75, 1, 48, 1),
+    (0x100, 224, 20, 3, 64), (0x101, 11, 30, 33, 40), (0x101, 320, 6, 200, 96), (0x101, 28, 28, 256, 512), (0x100 | SPLIT_HALVES, 61, 63, 64, 128),
+    (0x101 | SPLIT_HALVES, 28, 28, 256, 512), (0x101 | 3 << 12 | 3 << 16, 27, 14, 112, 200), (0x101 | SPLIT_MIXED, 64, 36, 100, 70)])
+def test_winograd_pair_operands(lib, dev, oracle, variant, W, H, I, O):
+    """Winograd on the f16 matrix cores, operands split into two parts: ragged channels, single steps, narrow and one-row maps, pieces, panels that begin
+    at different channels, the pooling epilogue.  Held to a twentieth of the layer bar, like three parts."""
+    x, w, b = rnd(I, H, W), rnd(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I))), rnd(O, scale=0.1)
+    for flags, bias in ((1, b), (0, None)):
+        want = oracle.conv_f64(x, w, bias, relu=bool(flags))
+        got = pair_winograd(lib, dev, x, w, variant, flags, bias)
+        assert_close(got, want, "two parts")
+        assert rel_err(got, want) <= TOL / 20
+        if W % 2 == 0 and H % 2 == 0:
+            assert np.array_equal(pair_winograd(lib, dev, x, w, variant, flags | 2, bias), oracle.pool(got, (2, 2, 1), (2, 2, 1), 0))
+
+
+@pytest.mark.parametrize("W,H,I,O", [(61, 63, 64, 128), (40, 30, 96, 64), (57, 44, 128, 70), (33, 31, 256, 96), (30, 28, 512, 64)])
+def test_winograd_pair_is_as_exact_as_three_parts(lib, dev, oracle, W, H, I, O):
+    """From 64 channels on, rms against 64 bits on rectified samples: two parts lose 2^-24 of a product and round the accumulator half as often."""
+    x, w = np.maximum(own(I, H, W), 0), own(I, O, 3, 3, scale=np.sqrt(2.0 / (9 * I)))
+    want = oracle.conv_f64(x, w)
+    rms = lambda y: float(np.sqrt(np.mean((y.astype(np.float64) - want) ** 2)))
+    assert rms(pair_winograd(lib, dev, x, w, 0x101)) <= rms(split_winograd(lib, dev, x, w, 0x101)[0])
+
+
+@pytest.mark.parametrize("variant", [0x100, 0x101, 0x101 | SPLIT_HALVES])
+@pytest.mark.parametrize("kind", ["rising", "late", "dark", "tiny", "denormal", "huge", "weights", "zero"])
+def test_winograd_pair_scales(lib, dev, oracle, kind, variant):
+    """Every column of tiles has a scale of its own that follows its largest sample: channels that get larger from step to step, that are zero at first,
+    maps of which one side is 2^-30 of the other, samples of any size, output channels of any size."""
+    W, H, I, O = 70, 6, 100, 40
+    x, w = own(I, H, W), own(I, O, 3, 3, scale=0.1)
+    if kind == "rising":                    # (weights that make up for it: what is lost in a channel would show)
+        up = np.exp2(np.arange(I) // 4).astype(np.float32)
+        x, w = x * up[:, None, None], np.maximum(np.abs(w), 0.05) * np.sign(w)
+    elif kind == "late":
+        x[:40] = 0
+        x[40:90, :, 30:] = 0
+        x[40] *= np.float32(2.0 ** -40)
+    elif kind == "dark":
+        x[:, :, 35:] *= np.float32(2.0 ** -30)
+    elif kind in ("tiny", "denormal", "huge"):
+        x = (x * {"tiny": 2.0 ** -100, "denormal": 2.0 ** -140, "huge": 2.0 ** 120}[kind]).astype(np.float32)
+        w = w * np.float32(2.0 ** (-20 if kind == "huge" else 20))
+    elif kind == "weights":
+        w = w * np.exp2(np.arange(O) * 4.0 - 80)[:, None, None].astype(np.float32)
+    else:
+        x[:] = 0
+    want, got = oracle.conv_f64(x, w), pair_winograd(lib, dev, x, w, variant)
+    if kind == "dark":                      # (the transforms mix neighbouring tiles' samples: the dark side begins a tile further on)
+        assert rel_err(got[:, :, 38:], want[:, :, 38:], floor=0.0) <= TOL / 20
+        got, want = got[:, :, :34], want[:, :, :34]
+    if kind == "weights":
+        for o in range(O):
+            assert rel_err(got[o], want[o], floor=0.0) <= TOL / 20, o
+    elif kind == "zero":
+        assert np.array_equal(got, np.zeros_like(got))
+    else:
+        assert rel_err(got, want, floor=0.0) <= TOL / 20
+
+
+@pytest.mark.parametrize("variant,W,H,I,O", [(0x100, 33, 9, 70, 70), (0x101, 40, 10, 100, 33), (0x101 | SPLIT_HALVES, 28, 9, 272, 33)])
+def test_winograd_pair_keeps_infinities(lib, dev, variant, W, H, I, O):
+    """Infinite, NaN and the largest finite samples come out as fp32 Winograd has them, at the edges of the map too."""
+    x, w = own(I, H, W), own(I, O, 3, 3, scale=0.02)
+    x[1, 4, 12], x[0, 0, 0], x[I - 1, H - 1, W - 1], x[I - 2, 3, 0], x[2, 5, W - 1] = np.inf, -np.inf, np.inf, -np.inf, np.inf
+    x[3, 2, 26], x[4, 2, 27], x[2, 6, 20] = np.inf, -np.inf, np.nan
+    x[5, 7, 5] = x[I - 1, 1, 22] = 3.399e38
+    got, want = pair_winograd(lib, dev, x, w, variant), winograd_replay(x, w)
+    assert np.isinf(want).sum() > O and np.isnan(want).any()
+    assert_same_extremes(got, want)
+
+
 @pytest.mark.parametrize("operand,power", [(o, p) for o in ("samples", "weights") for p in (-146, -136, -126, -112, -60, 60, 100, 116, 124)])
 def test_split_kernels_hold_operands_of_any_size(lib, dev, oracle, operand, power):
     """Samples and weights down to the smallest fp32 number keep all their bits, and what is too large for three parts once it is scaled, the

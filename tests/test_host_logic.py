@@ -746,6 +746,79 @@ def test_split_kernel_waits_for_its_samples(split_kernel_code):
         assert memory(front[first + 1:]) >= wait > 0, (name, front, wait)
 
 
+@pytest.fixture(scope="module")
+def pair_kernel_code(tmp_path_factory):
+    """{kernel: lines} of the two-part kernel's assembly."""
+    import subprocess
+    from deepracin_amd import build
+    out = str(tmp_path_factory.mktemp("asm") / "pair.s")
+    src = os.path.join(build.CSRC, "device", "k_winograd_split.hip")
+    subprocess.run([build.HIPCC] + build.COMMON + build.DEVICE + ["--cuda-device-only", "-S", src, "-o", out], check=True, capture_output=True)
+    kernels, name = {}, None
+    for line in open(out):
+        if line.startswith("_ZN5drhip24winograd_f23_pair_kernel") and line.split(";")[0].strip().endswith(":"):
+            name = line.split(":")[0]
+            kernels[name] = []
+        elif name and line.strip().startswith(".section"):
+            name = None
+        elif name:
+            kernels[name].append(line.strip())
+    assert len(kernels) == 6
+    return kernels
+
+
+def test_pair_kernel_waits_for_its_samples_and_leaves_m0(pair_kernel_code):
+    """As for the three-part kernel: fetches to LDS put M0 back, and a wait for all but the last n memory instructions has at least n behind the fetch
+    that it is for: the first step's in front of the loop, and a step's once round the loop."""
+    for name, lines in pair_kernel_code.items():
+        fetches = 6 if "ILi2ELi24E" in name else 5
+        blocks, inline = [[]], False
+        for k, line in enumerate(lines):
+            inline = (inline or line == ";;#ASMSTART") and line != ";;#ASMEND"
+            if line.startswith(".LBB"):
+                blocks.append([])
+            elif re.match(r"(buffer|global|flat|scratch)_(load|store|atomic)", line):
+                if line.endswith(" lds"):
+                    saved = lines[k - 3].split()[1].rstrip(",")
+                    assert lines[k - 3].split()[2] == "m0" and lines[k - 2].startswith("s_mov_b32 m0, ") and lines[k + 1] == "s_mov_b32 m0, " + saved, name
+                blocks[-1].append("F" if line.startswith("buffer_load_dwordx4") and line.endswith(" lds") else "M")
+            elif inline and line.startswith("s_waitcnt vmcnt"):
+                blocks[-1].append(int(re.search(r"\((\d+)\)", line).group(1)))
+        memory = lambda events: sum(e in ("F", "M") for e in events)
+        fetching = [b for b in blocks if "F" in b]
+        body, front = fetching[-1], [e for b in fetching[:-1] for e in b if e in ("F", "M")]
+        assert body.count("F") == fetches and front.count("F") == 2 * fetches, name
+        waits = [k for k, e in enumerate(body) if isinstance(e, int)]
+        last = max(k for k, e in enumerate(body) if e == "F")
+        assert len(waits) == 1 and memory(body[last + 1:]) + memory(body[:waits[0]]) >= body[waits[0]] > 0, name
+        places = [k for k, e in enumerate(front) if e == "F"]
+        wait = next(e for b in blocks for e in b if isinstance(e, int))
+        assert memory(front[places[fetches - 1] + 1:]) >= wait > 0, (name, front, wait)
+        # and the second step's, which the loop's first wait is for
+        assert memory(front[places[-1] + 1:]) + memory(body[:waits[0]]) >= body[waits[0]], name
+
+
+@pytest.mark.parametrize("what,fits", [("random", True), ("zero channel", True), ("tiny filter", False), ("zero filter", False), ("nan", False), ("inf", False),
+                                       ("small", True), ("too small", False), ("too large", False)])
+def test_filters_that_two_parts_can_hold(lib, what, fits):
+    """Finite, none of an output channel's filters far below its largest; an output channel without any is exact."""
+    w = np.random.default_rng(1).standard_normal((70, 33, 9)).astype(np.float32)
+    if what == "zero channel":
+        w[:, 5] = 0
+    elif what in ("tiny filter", "zero filter", "nan", "inf"):
+        w[69, 32] = {"tiny filter": 2.0 ** -14, "zero filter": 0.0, "nan": w[69, 32], "inf": w[69, 32]}[what]
+        if what in ("nan", "inf"):
+            w[69, 32, 8] = np.nan if what == "nan" else np.inf
+    else:
+        w *= np.float32({"small": 2.0 ** -90, "too small": 2.0 ** -110, "too large": 2.0 ** 110}.get(what, 1.0))
+    p = np.ascontiguousarray(w).ctypes.data_as(ctypes.c_void_p)
+    assert lib.drhip_winograd_pair_fits(p, 70, 33, 9) == fits
+    one = np.ascontiguousarray(w[:, :, 8])
+    if what == "random":
+        one[:] = np.abs(one) + 0.01
+    assert what not in ("random", "nan", "inf") or lib.drhip_winograd_pair_fits(one.ctypes.data_as(ctypes.c_void_p), 70, 33, 1) == fits
+
+
 def test_outputs_of_an_unprepared_graph_are_none_at_all(lib):
     """download_outputs in front of prepare returns an empty list, as the reference's wrapper does: dR_getOutputBuffers counts none."""
     with dr.Environment() as env:
