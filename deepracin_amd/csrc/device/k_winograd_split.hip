@@ -50,7 +50,7 @@ constexpr int ws_segments(int WC) { return (4 * WC - 72) / 4 + 1; }
 struct WsShape {                            // everything but the pointers; by value to the kernel
     int W, H, I, O, tilesX, T, nTB, nBlocks, nC, nOB;   // tiles, panels of 32 tiles, panels of outputs; 16-channel chunks, 32-channel blocks of filters
     unsigned mulX, shX, mulTB, shTB;                    // division by tilesX and by nTB
-    int flags, vec2;
+    int flags, vec2, pairs;                             // pairs: rows of two neighbouring tiles' outputs are 16 bytes, on 8
     // The first nA output panels of an XCD are cut into sA splits of perA chunks (in nA * sA workgroups), the others into sB of
     // perB; mulA, mulB: division by sA and sB
     int wgsA, nA, sA, sB, perA, perB, mulA, mulB;
@@ -180,8 +180,10 @@ struct WsSamples {
     __device__ __forceinline__ void fetch(int buf, int i) {
         if (i == 0) {
             const bool last = TURNS && fetching == steps - 1;
+            toNext = last ? stepB - (unsigned)steps * stepB : stepB;
             // (behind the last one out of the map: zeros that nobody uses cost no trip to memory)
-            toNext = TURNS && left == 1 ? kOutOfRange : TURNS && left < 1 ? 0 : last ? stepB - (unsigned)steps * stepB : stepB;
+            if (TURNS) toNext = left == 1 ? kOutOfRange : toNext;
+            if (TURNS) toNext = left < 1 ? 0u : toNext;
             --left;
             if (TURNS) fetching = last ? 0 : fetching + 1;
         }
@@ -199,6 +201,8 @@ __device__ __forceinline__ void ws_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+__device__ __forceinline__ int ws_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
 // The bank of three bf16 parts: its fragments of 32 output channels by 16 input channels in pieces of 16 bytes, and a weight out of its parts.
 struct WsBf16x3 {
     static constexpr int PARTS = 3;
@@ -211,7 +215,8 @@ template <int KW, class Bank>
 __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, const float* scaleT, const WsShape& s, const WsPlace<KW>& at, const float* in, const unsigned short* U, float* out, float* ws) {
     constexpr int NT = 2, OB = 32 * NT;
     using std::integral_constant;
-    const int tid = threadIdx.x, lane = tid & 63, nSp = at.nSp, split = at.split, oBlock = at.oBlock, o0 = at.o0, t0 = at.t0;
+    // (the lane is asked for once more: what lives through the loop would be spilled there)
+    const int lane = ws_lane(), tid = 64 * (4 * at.set + at.wave) + lane, nSp = at.nSp, split = at.split, oBlock = at.oBlock, o0 = at.o0, t0 = at.t0;
     const int W = s.W, H = s.H, I = s.I, plane = W * H;
     const FastDiv tilesXd = {(unsigned)s.tilesX, s.mulX, s.shX};
     auto scale = [&](int ol) { return scaleT ? scaleT[ol] : kSplitUnscale; };
@@ -302,6 +307,77 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
             if (nSp == 3) join(integral_constant<int, 3>{});
             else join(integral_constant<int, 4>{});
         }
+    } else if (s.pairs) {
+        // Two neighbouring tiles a thread: half of the reads, and rows of 16 bytes to store, without branches between the stores: tiles, rows and output
+        // channels that do not exist lie out of the range of the buffer.  A CU takes 16 bytes a clock of stores of 8 bytes a lane, and 20 to 25 of 16.
+        // (640x480 64->64, clocks of a workgroup: sums 1360 -> 840, stores 4120 -> 2560 of 24800; the layer 69.2 -> 67.8 us, 320x240 64->128 37.0 -> 35.9.)
+        constexpr int EP = 2 * EO, NQ = OB / EP;
+        const int pt = 2 * (tid & 15), po = tid >> 4;
+        const bool pOk = t0 + pt < s.T;
+        const int pTy = pOk ? fast_div(t0 + pt, tilesXd) : 0, px = pOk ? 2 * (t0 + pt - pTy * s.tilesX) : 0;
+        f32x4 rows[NQ][2];
+        float sum = 0.0f;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int ol = po + EP * q;
+            f32x2 p[4][2];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    p[r][x] = *(const f32x2*)&P[((r * 2 + x) * OB + ol) * 32 + pt];
+                    if (KW == 2) {
+                        const f32x2 other = *(const f32x2*)&P[(((4 + r) * 2 + x) * OB + ol) * 32 + pt];
+                        p[r][x] = f32x2{p[r][x][0] + other[0], p[r][x][1] + other[1]};
+                    }
+                }
+            const float b = biasT[ol], f = scale(ol);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const float top = p[0][x][t] + p[1][x][t] + p[2][x][t], bottom = p[1][x][t] - p[2][x][t] + p[3][x][t];
+                    sum += fabsf(top) + fabsf(bottom);
+                    rows[q][0][2 * t + x] = fmaf(top, f, b);
+                    rows[q][1][2 * t + x] = fmaf(bottom, f, b);
+                }
+        }
+        if (s.flags & kEpiRelu)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { rows[q][0][k] = fmaxf(rows[q][0][k], 0.f); rows[q][1][k] = fmaxf(rows[q][1][k], 0.f); }
+        const bool pool = s.flags & kEpiMaxPool2;
+        const int outPlane = pool ? plane >> 2 : plane;
+        auto channels = [&](int q) {                    // (their buffer: the EP output channels of pass q)
+            return __builtin_amdgcn_make_buffer_rsrc((void*)(out + (size_t)(o0 + EP * q) * outPlane), 0, max(min(s.O - o0 - EP * q, EP), 0) * outPlane * 4, kBufferFlags);
+        };
+        if (pool) {
+            const int to = pOk ? 4 * (po * outPlane + pTy * (W >> 1) + (px >> 1)) : (int)kOutOfRange;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const f32x2 most = {fmaxf(fmaxf(rows[q][0][0], rows[q][0][1]), fmaxf(rows[q][1][0], rows[q][1][1])), fmaxf(fmaxf(rows[q][0][2], rows[q][0][3]), fmaxf(rows[q][1][2], rows[q][1][3]))};
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2b, most), channels(q), to, 0, kAuxThrough);
+            }
+        } else {
+            const int to = pOk ? 4 * (po * plane + 2 * pTy * W + px) : (int)kOutOfRange, below = pOk && 2 * pTy + 1 < H ? to + 4 * W : (int)kOutOfRange;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const __amdgpu_buffer_rsrc_t r = channels(q);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, rows[q][0]), r, to, 0, kAuxThrough);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, rows[q][1]), r, below, 0, kAuxThrough);
+            }
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(pOk && !(sum < __builtin_inff())) != 0, 0)) {
+#pragma clang loop unroll(disable)
+            for (int n = 0; n < 2 * NQ; ++n) {          // bit 2 * pass + tile of the pair
+                auto at = [&](int r, int x) { const float* row = &P[((r * 2 + x) * OB + po + EP * (n >> 1)) * 32 + pt + (n & 1)]; return KW == 2 ? row[0] + row[8 * OB * 32] : row[0]; };
+                float all = 0.0f;
+#pragma unroll
+                for (int x = 0; x < 2; ++x) all += fabsf(at(0, x) + at(1, x) + at(2, x)) + fabsf(at(1, x) - at(2, x) + at(3, x));
+                again |= pOk && !(all < __builtin_inff()) ? 1u << n : 0u;
+            }
+        }
     } else {
         f32x4 y[NP];                                    // (read in one go: with each store behind its own reads the notes cost the trunk
         float b[NP], f[NP];                             // 4.5 us)
@@ -321,16 +397,29 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
     // Once more in fp32, step by step as the fp32 kernel does it, and with the samples beside the map left out.  Every wave
     // for itself, tile by tile: its 2 * NP output channels side by side, the lanes left over share the input channels.  (Us, without
     // and with one NaN and one infinity among the samples: 56x56 512->512 58 / 241, 224x224 64->64 18 / 39; all NaN 68 and 30.)
-    const unsigned long long any = __builtin_amdgcn_ballot_w64(eOk && again != 0u);
+    const bool pairs = nSp == 1 && s.pairs;
+    const unsigned long long any = __builtin_amdgcn_ballot_w64((pairs || eOk) && again != 0u);
     if (__builtin_expect(any == 0, 1)) return;          // (expected: otherwise what follows lies between instructions that every launch
                                                         // fetches, and a trunk of 640x480 takes 713 us instead of 702)
     constexpr int C = 2 * NP, S = 64 / C;               // channels of this wave, lanes per channel
     constexpr int PARTS = Bank::PARTS, FRAG = 4 * PARTS * 64;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (what is stored below lies where other lanes have stored)
     const __amdgpu_buffer_rsrc_t rAll = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, I * plane * 4, kBufferFlags);
-    const int part = lane / C, pass = lane % C >> 1, ol = 2 * (tid >> 6) + (lane & 1) + EO * pass;
+    // (the channels that this wave has stored: of 2 a pass, or, of pairs of tiles, of 4)
+    const int part = lane / C, first = pairs ? lane & 3 : lane & 1, pass = pairs ? lane % C >> 2 : lane % C >> 1, ol = pairs ? 4 * (tid >> 6) + first + 2 * EO * pass : 2 * (tid >> 6) + first + EO * pass;
     const u32x4b* uLane = (const u32x4b*)U + (size_t)min(oBlock * NT + (ol >> 5), s.nOB - 1) * FRAG + (ol & 31);
-    for (unsigned bad = (unsigned)any | (unsigned)(any >> 32); bad != 0; bad &= bad - 1) {
+    unsigned bad = (unsigned)any | (unsigned)(any >> 32);
+    if (pairs) {                                        // lanes with pairs become tiles
+        bad = 0;
+#pragma clang loop unroll(disable)
+        for (int x = 0; x < 2; ++x) {
+            const unsigned long long odd = __builtin_amdgcn_ballot_w64((again & 0x55555555u << x) != 0u);
+            unsigned m = (unsigned)(odd | odd >> 16 | odd >> 32 | odd >> 48) & 0xffffu;
+            m = (m | m << 8) & 0x00ff00ffu; m = (m | m << 4) & 0x0f0f0f0fu; m = (m | m << 2) & 0x33333333u; m = (m | m << 1) & 0x55555555u;
+            bad |= m << x;
+        }
+    }
+    for (; bad != 0; bad &= bad - 1) {
         const int t = __builtin_ctz(bad), ty = fast_div(t0 + t, tilesXd), x0 = 2 * (t0 + t - ty * s.tilesX) - 1, y0 = 2 * ty - 1;
         // A NaN among the samples at the tile's own four pixels reaches all four outputs, whatever the others are.
         bool own = false;
@@ -386,8 +475,8 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
         for (int k = C; k < 64; k *= 2)
 #pragma unroll
             for (int c = 0; c < 4; ++c) y[c] += __shfl_xor(y[c], k);
-        const unsigned noted = (unsigned)__shfl((int)again, 32 * (lane & 1) + t);
-        if (part == 0 && (noted >> pass & 1u) && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, x0 + 1, y0 + 1, s.vec2);
+        const unsigned noted = (unsigned)__shfl((int)again, pairs ? 16 * first + (t >> 1) : 32 * first + t);
+        if (part == 0 && (noted >> (pairs ? 2 * pass + (t & 1) : pass) & 1u) && o0 + ol < s.O) wino_finish(out, y, biasT[ol], s.flags, o0 + ol, plane, W, H, x0 + 1, y0 + 1, s.vec2);
     }
 }
 
@@ -648,6 +737,7 @@ __device__ __forceinline__ void ws_word_to_lds(__amdgpu_buffer_rsrc_t from, int 
 // step instead of 48, 16 KiB of filters instead of 24 and 176 vector instructions instead of 270.  Layers, us, three parts / two, with their errors
 // against 64 bits (rms, 1e-7): 640x480 64->64 85 / 67 (2.2 / 1.9), 320x240 128->128 75.0 / 56.9 (2.8 / 2.3), 160x120 256->256 73.6 / 54.1 (3.7 / 2.9),
 // 80x60 512->512 75.7 / 54.7 (3.7 / 2.9), 112x112 128->128 16.0 / 13.0 (2.1 / 1.9), 40x30 512->512 27.8 / 22.0 (2.5 / 2.2).
+// No value may go to scratch: a kernel that has any starts about 1 us later (the eight such layers of VGG16 293 -> 287 us a pass).
 // What bounds it: two workgroups of a CU take 4480 clocks a step on 320x240, the fetches without the MFMAs 2630 (168 KB at 64 bytes a clock), MFMAs and vector
 // instructions without fetches 1940: eight fragments of filters under way per wave do not cover the way to L2 while a CU's eight waves queue there.
 template <int KW, int WC, bool TURNS>
@@ -681,8 +771,9 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
     const unsigned uStep = (unsigned)s.nOB * 8192u;
     __amdgpu_buffer_rsrc_t rNext = rU;              // (what the last step requests for one behind it comes from nowhere)
     u32x4b f[2][NT][2];                             // of two positions
+    int lane16 = lane * 16;                         // (told to the compiler anew in every step: the other part's offset goes in the instruction then)
     auto load_filter = [&](const __amdgpu_buffer_rsrc_t& from, int e, int nt, int q, int step) {
-        f[e & 1][nt][q] = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 2048)), 0));
+        f[e & 1][nt][q] = __builtin_bit_cast(u32x4b, __builtin_amdgcn_raw_buffer_load_b128(from, lane16 + q * 1024, (int)(uOb[nt] + (unsigned)min(step, s.nC - 1) * uStep + (unsigned)(e * 2048)), 0));
     };
 
     // ---- operands --------------------------------------------------------------------------------------------------
@@ -696,11 +787,13 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
     const int rLds = half * 8 * CHB + 4 * (Samples::segment_at(s, off0, lr) + 2 * (tx - firstTx) - (firstTx == 0 ? 1 : 0));
     float k[4] = {tx > 0 ? 1.0f : 0.0f, 1.0f, 2 * tx + 1 < W ? 1.0f : 0.0f, 2 * tx + 2 < W ? 1.0f : 0.0f};      // masks of the columns of the window, with the scale
     constexpr float kLimit = 0x1p14f;
-    float limit = kLimit, most = 0.0f;              // of the samples that come next
+    float most = 0.0f;                              // of the samples that come next
+    unsigned long long noneYet = ~0ull;             // lanes that have met zeros only: any other sample sets their scale
     float minusOne;
     asm volatile("s_mov_b32 %0, 0xbf800000" : "=s"(minusOne));
     float mm[8][4];                                 // combined window rows of this lane's tile, 8 channels
-    float ra[3][2], rb[3][2];                       // two channels' samples of a column on their way from LDS, of three columns
+    constexpr int RING = WC == 24 ? 2 : 3;
+    float ra[RING][2], rb[RING][2];                 // two channels' samples of a column on their way from LDS, of three columns (two: registers)
     const char* samples = lds + set * 3 * BUFB;
     auto read_two = [&](int buf, int slot, int c, int j) {
         const float* a = (const float*)(samples + buf * BUFB + rowA * ROWB + rLds + j * CHB) + c;
@@ -744,9 +837,10 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
 
     // The scale that suits `most`, and everything that has been multiplied by the old one with it.
     auto rescale = [&](bool sums) {
-        const float largest = fmaxf(most, __shfl_xor(most, 32));
+        const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(most), __float_as_uint(most), false, false);
+        const float largest = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
         const int e = (int)(__float_as_uint(largest) >> 23) - 127, has = (int)(__float_as_uint(k[1]) >> 23) - 127;
-        const bool lower = largest >= limit && e < 128;         // (an infinity stays one whatever the scale)
+        const bool lower = (largest >= kLimit || (largest != 0.0f && __builtin_amdgcn_inverse_ballot_w64(noneYet))) && e < 128;    // (an infinity stays one whatever the scale)
         const int by = lower ? min(11 - e, 126 - has) : 0, by2 = by / 2;       // (in two factors: it goes down to -240)
         // Samples that no scale makes large enough, fp32 denormals, are left to the pass over what did not come out finite.
         const float f1 = e + by < 1 && lower ? __builtin_nanf("") : __uint_as_float((unsigned)(127 + by2) << 23), f2 = __uint_as_float((unsigned)(127 + by - by2) << 23);
@@ -757,7 +851,7 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
 #pragma unroll
             for (int j = 0; j < 8; ++j) mm[j][c] = times(mm[j][c]);
         }
-        if (lower) limit = kLimit;
+        noneYet &= ~__builtin_amdgcn_ballot_w64(lower);
         if (sums)
 #pragma unroll
             for (int x = 0; x < 4; ++x)
@@ -788,12 +882,10 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
 #pragma unroll
     for (int q = 0; q < 2 * NT; ++q) load_filter(rU, 1, q & 1, kPA[q / 2], first + set + KW * turn);
 #pragma unroll
-    for (int n = 0; n < 16; ++n) { read_two(0, n % 3, n / 4, 2 * (n % 4)); combine_two(n % 3, n / 4, 2 * (n % 4)); }
+    for (int n = 0; n < 16; ++n) { read_two(0, n % RING, n / 4, 2 * (n % 4)); combine_two(n % RING, n / 4, 2 * (n % 4)); }
     {   // the first scale: for `most` where it is not zero
-        limit = 0x1p-149f;
         rescale(false);
-        const bool none = limit < kLimit;
-        if (none) {
+        if (__builtin_amdgcn_inverse_ballot_w64(noneYet)) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) k[c] *= 0x1p64f;
         }
@@ -814,8 +906,8 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
             split_tick((e + 1) & 3, 2 * i + 1);
             // The samples of the next step, two channels of a column at a time, read and two slots later combined, behind the last use of
             // what they replace: the first column is used by the first position alone, the third by the first three.
-            if (slot >= 8) combine_two((slot - 8) % 3, (slot - 8) / 4 == 1 ? 2 : (slot - 8) / 4 == 2 ? 1 : (slot - 8) / 4, 2 * ((slot - 8) % 4));
-            if (slot >= 6 && slot < 22) read_two(nxt, (slot - 6) % 3, (slot - 6) / 4 == 1 ? 2 : (slot - 6) / 4 == 2 ? 1 : (slot - 6) / 4, 2 * ((slot - 6) % 4));
+            if (slot >= 8) combine_two((slot - 8) % RING, (slot - 8) / 4 == 1 ? 2 : (slot - 8) / 4 == 2 ? 1 : (slot - 8) / 4, 2 * ((slot - 8) % 4));
+            if (slot >= 6 && slot < 22) read_two(nxt, (slot - 6) % RING, (slot - 6) / 4 == 1 ? 2 : (slot - 6) / 4 == 2 ? 1 : (slot - 6) / 4, 2 * ((slot - 6) % 4));
             if (slot % 4 == 0 && slot / 4 < NDMA) fetched.fetch(nxt2, slot / 4);
             // The next step's samples, requested a step ago, have to be visible before they are read.  (Younger than them are filters behind
             // slot 16, or 20, of the step before, or of the prologue, those of this position and two loads for the step after.)
@@ -833,8 +925,9 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
         m = TURNS && m == steps - 1 ? 0 : m + 1;
         const int stepNext = first + set + KW * m;
         rNext = __builtin_amdgcn_make_buffer_rsrc((void*)uHere, 0, n + 1 < steps ? uBytes : 0, kBufferFlags);
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(most >= limit) != 0, 0)) rescale(true);
+        if (__builtin_expect((__builtin_amdgcn_ballot_w64(most >= kLimit) | (__builtin_amdgcn_ballot_w64(most != 0.0f) & noneYet)) != 0, 0)) rescale(true);
         most = 0.0f;
+        asm volatile("" : "+v"(lane16));
         position(integral_constant<int, 0>{}, step, stepNext, nxt, nxt2);
         position(integral_constant<int, 1>{}, step, stepNext, nxt, nxt2);
         position(integral_constant<int, 2>{}, step, stepNext, nxt, nxt2);
@@ -847,15 +940,16 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
 
     // ---- epilogue --------------------------------------------------------------------------------------------------
     float* P = (float*)lds;                         // [set][row][2][OB][32]
+    const int at32 = ws_lane() & 31, atHalf = ws_lane() >> 5;
     const float back = __uint_as_float((254u << 23) - __float_as_uint(k[1]));
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const float m0 = acc[0][nt][r], m1 = acc[1][nt][r], m2 = acc[2][nt][r], m3 = acc[3][nt][r];
-            const int ol = 32 * nt + 8 * (r / 4) + 4 * half + (r % 4);
-            P[(((set * 4 + wave) * 2 + 0) * OB + ol) * 32 + l32] = back * (m0 + m1 + m2);
-            P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + l32] = back * (m1 - m2 + m3);
+            const int ol = 32 * nt + 8 * (r / 4) + 4 * atHalf + (r % 4);
+            P[(((set * 4 + wave) * 2 + 0) * OB + ol) * 32 + at32] = back * (m0 + m1 + m2);
+            P[(((set * 4 + wave) * 2 + 1) * OB + ol) * 32 + at32] = back * (m1 - m2 + m3);
         }
     ws_barrier();
     ws_finish<KW, WsF16x2>(P, biasT, scaleT, s, at, in, U, out, ws);
@@ -920,7 +1014,10 @@ static int launch_ws(const float* in, const unsigned short* U, const float* bias
 }
 template <bool PAIR>
 static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, float* ws, const WsPlan& p, hipStream_t st) {
-    if (p.wc == 24) return p.turns ? launch_ws<2, 24, true, PAIR>(in, U, bias, out, ws, p, st) : launch_ws<2, 24, false, PAIR>(in, U, bias, out, ws, p, st);
+    if (p.wc == 24) {
+        if constexpr (!PAIR) { if (!p.turns) return launch_ws<2, 24, false, PAIR>(in, U, bias, out, ws, p, st); }
+        return launch_ws<2, 24, true, PAIR>(in, U, bias, out, ws, p, st);       // (of the pair kernel always: without turns the compiler keeps a value in scratch)
+    }
     if (p.kw == 2) return p.turns ? launch_ws<2, 20, true, PAIR>(in, U, bias, out, ws, p, st) : launch_ws<2, 20, false, PAIR>(in, U, bias, out, ws, p, st);
     return p.turns ? launch_ws<1, 20, true, PAIR>(in, U, bias, out, ws, p, st) : launch_ws<1, 20, false, PAIR>(in, U, bias, out, ws, p, st);
 }
@@ -951,7 +1048,14 @@ using namespace drhip;
 //     channels more than 6: nothing gained (81x239 256->128, 7 over: 48.6 against 47.6).
 //   * a few more than two per CU: the rest in halves (160x120 256->256 76.1 us against 84.3, 128->256 43.8 against 46.5).
 //     After more rounds than one the workgroups do not end together any more (320x240 128->128, 2.3 rounds: 80 against 74).
-extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, int O) {
+//
+// Two f16 parts take less (measured like that, 70 shapes drawn and VGG16's, with other filters each time, us fp32 kernel / this):
+//   * pieces 7.8, 2 more per pair of chunks and 0.22 per MB of filters (56x56 256->256 20.5 / 16.5, 28x28 512->512 23.4 / 20.4, 61x75 320->140 23.3 / 19.8,
+//     62x41 376->106 19.0 / 14.1, 51x41 191->384 18.0 / 15.5; 56x56 128->256 12.0 / 12.2, 28x28 256->512 14.6 / 16.9, 84x68 224->64 12.0 / 12.2 and fewer panels
+//     stay there).
+//   * one workgroup for more than half of the CUs from 4 chunks on (112x112 64->128 12.0 / 9.4, 48x56 64->448 12.0 / 9.4, 55x57 93->305 17.1 / 12.1), with
+//     two wave sets from 8 (118x112 160->70 18.0 / 15.5, one set 16.2; 85x111 288->128 23.4 and 26.7).
+static int ws_pick(int W, int H, int I, int O, bool pair) {
     WsPlan p;
     if (O <= 32 || !ws_plan(W, H, I, O, 0x101, &p)) return 0;
     const int blocks = p.s.nBlocks, nC = p.s.nC, cus = num_cu(), cusPerXcd = cus / kXcds, n = ceil_div(blocks, kXcds);
@@ -967,8 +1071,10 @@ extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, in
         // and stay where they gain on a form whose sums are as short.  And against what that kernel takes, where that is the slower one.
         const int S = std::min(4, cusPerXcd / n), halvings = wino_halvings(W, H, I, O), panels32 = p.s.nTB * ceil_div(O, 32);
         auto fp32 = [&](int lg) { return 0.56 * ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus) + (lg > 0 ? 4.5 : 3); };
+        const int pairs = ceil_div(ceil_div(nC, S), 2);
+        const double taken = fp32(drhip_conv3x3_winograd_pick_variant(W, H, I, O) >> 4 & 15);
         if (halvings >= 0 &&                            // (layers of its 16-tile form are too small)
-            2.75 * ceil_div(ceil_div(nC, S), 2) + 10.6 < 0.93 * std::max(fp32(halvings), fp32(drhip_conv3x3_winograd_pick_variant(W, H, I, O) >> 4 & 15)))
+            (2.75 * pairs + 10.6 < 0.93 * std::max(fp32(halvings), taken) || (pair && 2.0 * pairs + 7.8 + 0.22e-6 * 64 * I * O < 0.93 * taken)))
             if (const int v = split(0x101, 0, S, S)) return v;
     }
     if (!wide) return 0;
@@ -977,14 +1083,17 @@ extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, in
         if (const int v = split(0x101, cusPerXcd, 1, 4 * over <= cusPerXcd ? 4 : 3)) return v;
     if (joins && nC >= 8 && over2 > 0 && 2 * over2 <= cusPerXcd)
         if (const int v = split(0x100, 2 * cusPerXcd, 1, 2)) return v;
+    if (pair && blocks <= cus) return 2 * n > cusPerXcd && nC >= 4 ? (nC >= 8 ? 0x101 : 0x100) : 0;
     if (blocks <= cus) return nC >= 8 && 20 * blocks >= 11 * cus ? 0x101 : 0;
     return nC >= 4 || (nC >= 2 && 2 * blocks >= 3 * cus) ? 0x100 : 0;
 }
 
-// Two f16 parts instead of three bf16 ones, where the kernel of split operands is taken at all and from 64 input channels on: with fewer its sums
-// are less exact (16 channels 1.34 against 1.11e-7 rms, 32 channels 1.45 against 1.32).
+extern "C" int drhip_conv3x3_winograd_split_pick_variant(int W, int H, int I, int O) { return ws_pick(W, H, I, O, false); }
+
+// Two f16 parts from 64 input channels on: with fewer their sums are less exact than three bf16 parts' (16 channels 1.34 against 1.11e-7 rms, 32 channels
+// 1.45 against 1.32).
 extern "C" int drhip_conv3x3_winograd_pair_pick_variant(int W, int H, int I, int O) {
-    const int v = I >= 64 ? drhip_conv3x3_winograd_split_pick_variant(W, H, I, O) : 0;
+    const int v = I >= 64 ? ws_pick(W, H, I, O, true) : 0;
     return v ? v | 0x200 : 0;
 }
 
@@ -1060,6 +1169,7 @@ extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U,
     p.s.flags = flags;
     p.s.joinSpins = p.s.sA == 1 && p.s.sB == 1 ? 0 : wino_join_spins();
     p.s.vec2 = ((W & 1) == 0) && (((size_t)out & 7) == 0);
+    p.s.pairs = (W & 3) == 0 && ((size_t)out & 7) == 0 && (long long)W * H * 32 * p.kw < (1ll << 31) / 2;
     const unsigned short* F = (const unsigned short*)U;
     hipStream_t st = as_stream(stream);
     return p.pair ? launch_ws<true>(in, F, bias, out, workspace, p, st) : launch_ws<false>(in, F, bias, out, workspace, p, st);

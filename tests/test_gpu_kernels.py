@@ -599,7 +599,7 @@ def test_winograd_pair_scales(lib, dev, oracle, kind, variant):
         assert rel_err(got, want, floor=0.0) <= TOL / 20
 
 
-@pytest.mark.parametrize("variant,W,H,I,O", [(0x100, 33, 9, 70, 70), (0x101, 40, 10, 100, 33), (0x101 | SPLIT_HALVES, 28, 9, 272, 33)])
+@pytest.mark.parametrize("variant,W,H,I,O", [(0x100, 33, 9, 70, 70), (0x100, 40, 10, 70, 70), (0x101, 40, 10, 100, 33), (0x101 | SPLIT_HALVES, 28, 9, 272, 33)])
 def test_winograd_pair_keeps_infinities(lib, dev, variant, W, H, I, O):
     """Infinite, NaN and the largest finite samples come out as fp32 Winograd has them, at the edges of the map too."""
     x, w = own(I, H, W), own(I, O, 3, 3, scale=0.02)
@@ -609,6 +609,32 @@ def test_winograd_pair_keeps_infinities(lib, dev, variant, W, H, I, O):
     got, want = pair_winograd(lib, dev, x, w, variant), winograd_replay(x, w)
     assert np.isinf(want).sum() > O and np.isnan(want).any()
     assert_same_extremes(got, want)
+
+
+@pytest.mark.parametrize("variant", [0x100, 0x101, 0x100 | PAIR, 0x101 | PAIR])
+@pytest.mark.parametrize("W,H,I,O", [(40, 10, 70, 33), (36, 17, 64, 65), (64, 1, 64, 70), (72, 34, 65, 128)])
+def test_winograd_stores_pairs_of_tiles(lib, dev, oracle, variant, W, H, I, O):
+    """Rows of two neighbouring tiles are stored together where they lie on 8 bytes, one tile at a time elsewhere: the same bits, on odd heights, ragged
+    channels and part of a panel, with an infinity and a NaN among the samples, and nothing behind the outputs is written."""
+    x, w, b = own(I, H, W), own(I, O, 3, 3, scale=0.05), own(O)
+    xs = [x, x.copy()]
+    xs[1][3, H // 2, 5], xs[1][I - 1, 0, W - 2] = np.inf, np.nan
+    kind = "pair" if variant & PAIR else "split"
+    F = dev.empty(getattr(lib, "drhip_conv3x3_winograd_%s_filter_floats" % kind)(I, O))
+    ok(lib, getattr(lib, "drhip_winograd_%s_filter_transform_f32" % kind)(dev.put(w), F, I, O, None))
+    for x in xs:
+        for flags in (0, 1, 3):
+            if flags & 2 and (W | H) & 1:
+                continue
+            shape = (O, H // 2, W // 2) if flags & 2 else (O, H, W)
+            n, outs = int(np.prod(shape)), []
+            for first in (0, 2, 1):                     # on 16 bytes, on 8, on 4
+                y = dev.put(np.full(n + 8, 7, np.float32))
+                ok(lib, lib.drhip_conv3x3_winograd_split_f32(dev.put(x), F, dev.put(b), ctypes.c_void_p((y.value if hasattr(y, "value") else y) + 4 * first), W, H, I, O, flags, variant, None, None))
+                got = dev.get(y, (n + 8,))
+                assert np.all(got[:first] == 7) and np.all(got[first + n:] == 7)
+                outs.append(got[first:first + n])
+            assert np.array_equal(outs[0], outs[2], equal_nan=True) and np.array_equal(outs[1], outs[2], equal_nan=True)
 
 
 @pytest.mark.parametrize("operand,power", [(o, p) for o in ("samples", "weights") for p in (-146, -136, -126, -112, -60, 60, 100, 116, 124)])

@@ -874,6 +874,15 @@ def test_layers_stay_in_pieces_for_their_exactness(lib, W, H, I, O, pieces):
     assert lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O) == (0x101 | pieces << 12 | pieces << 16 if pieces else 0)
 
 
+@pytest.mark.parametrize("W,H,I,O,variant", [
+    (56, 56, 256, 256, 0x22301), (28, 28, 512, 512, 0x44301), (62, 41, 376, 106, 0x44301), (47, 61, 192, 192, 0x33301),     # pieces where they are the faster ones
+    (56, 56, 128, 256, 0), (28, 28, 256, 512, 0), (84, 68, 224, 64, 0), (14, 14, 512, 512, 0), (45, 60, 480, 64, 0),
+    (112, 112, 64, 128, 0x300), (112, 112, 127, 128, 0x301), (112, 112, 112, 128, 0x300), (112, 112, 63, 128, 0),           # one round that fills more than half of the CUs
+    (64, 64, 64, 256, 0), (64, 66, 64, 256, 0x300), (28, 30, 64, 1024, 0)])                                                # 128 panels, 132, and none of them on maps that narrow
+def test_winograd_pair_variant_by_panels_and_chunks(lib, W, H, I, O, variant):
+    assert lib.drhip_conv3x3_winograd_pair_pick_variant(W, H, I, O) == variant
+
+
 @pytest.mark.parametrize("pixels,channels", [(1, 1), (1, 5), (63, 7), (64, 2), (65, 3), (1000, 64)])
 def test_interleaved_to_planes(lib, pixels, channels):
     a = np.random.default_rng(0).standard_normal((pixels, channels)).astype(np.float32)
