@@ -260,7 +260,7 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, tile_of(eo + EO * q)), rWs, slot_of(split, q), 0, kAuxThrough);
             const u32x4 empty = {kWinoEmpty, kWinoEmpty, kWinoEmpty, kWinoEmpty};
             f32x4 own[C];
-            u32x4 part[C][S];
+            u32x4 part[C][S] = {};
 #pragma unroll
             for (int i = 0; i < C; ++i) own[i] = tile_of(eo + EO * (q0 + min(i, count - 1)));
             bool ready = false;
@@ -271,7 +271,7 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
 #pragma unroll
                 for (int i = 0; i < C; ++i)
 #pragma unroll
-                    for (int u = 0; u < S; ++u) part[i][u] = __builtin_amdgcn_raw_buffer_load_b128(rWs, slot_of(u, q0 + min(i, count - 1)), 0, kAuxDeviceVolatile);
+                    for (int u = 0; u < S; ++u) if (u != split) part[i][u] = __builtin_amdgcn_raw_buffer_load_b128(rWs, slot_of(u, q0 + min(i, count - 1)), 0, kAuxDeviceVolatile);
 #pragma unroll
                 for (int i = 0; i < C; ++i)
 #pragma unroll
@@ -287,7 +287,7 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
 #pragma unroll
                 for (int u = 0; u < S; ++u) y += u == split ? own[i] : __builtin_bit_cast(f32x4, part[i][u]);
 #pragma unroll
-                for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, slot_of(u, q), 0, kAuxThrough);
+                for (int u = 0; u < S; ++u) if (u != split) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, slot_of(u, q), 0, kAuxThrough);
                 note(q, y);
                 if (!ready) {                           // a partner never delivered: it shows in the result, too
                     y = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
