@@ -152,23 +152,27 @@ struct WsSamples {
             segEnd[k] = iy >= 0 && iy < H ? W - skip + segAt[k] : 0;
             segBase[k] = 4u * (unsigned)(iy * W + skip - segAt[k]) + (unsigned)first16 * plane4;
         }
-        int piece = lane % WC;
-        unsigned chOff = (unsigned)(lane / WC) * plane4;
+        auto offsets = [&](auto segments) {
+            int piece = lane % WC;
+            unsigned chOff = (unsigned)(lane / WC) * plane4;
 #pragma unroll
-        for (int i = 0; i < NDMA; ++i) {
-            const int f = 4 * piece;
-            int end = segEnd[0];
-            unsigned base = segBase[0];
+            for (int i = 0; i < NDMA; ++i) {
+                const int f = 4 * piece;
+                int end = segEnd[0];
+                unsigned base = segBase[0];
 #pragma unroll
-            for (int k = 1; k < SEG; ++k) {
-                end = f >= segAt[k] ? segEnd[k] : end;
-                base = f >= segAt[k] ? segBase[k] : base;
+                for (int k = 1; k < decltype(segments)::value; ++k) {
+                    end = f >= segAt[k] ? segEnd[k] : end;
+                    base = f >= segAt[k] ? segBase[k] : base;
+                }
+                voff[i] = (f >= 4 && f < end ? base + 4u * (unsigned)f + chOff : kOutOfRange) + (unsigned)turn * stepB;
+                const bool wrap = piece >= WC - 64 % WC;        // 64 pieces on
+                piece += 64 % WC - (wrap ? WC : 0);
+                chOff += (unsigned)(64 / WC) * plane4 + (wrap ? plane4 : 0u);
             }
-            voff[i] = (f >= 4 && f < end ? base + 4u * (unsigned)f + chOff : kOutOfRange) + (unsigned)turn * stepB;
-            const bool wrap = piece >= WC - 64 % WC;        // 64 pieces on
-            piece += 64 % WC - (wrap ? WC : 0);
-            chOff += (unsigned)(64 / WC) * plane4 + (wrap ? plane4 : 0u);
-        }
+        };
+        if (WC == 20 && s.tilesX >= 31) offsets(std::integral_constant<int, 2>{});      // (no panel touches three rows of tiles)
+        else offsets(std::integral_constant<int, SEG>{});
         rIn = __builtin_amdgcn_make_buffer_rsrc((void*)in, 0, min(s.I, 16 * (at.first + at.perSplit)) * plane * 4, kBufferFlags);    // (ends with the split)
         ldsBase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds + (unsigned)(at.set * 3 * BUFB + at.wave * ROWB);
         fetching = turn;
@@ -841,10 +845,10 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
         const float largest = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
         const int e = (int)(__float_as_uint(largest) >> 23) - 127, has = (int)(__float_as_uint(k[1]) >> 23) - 127;
         const bool lower = (largest >= kLimit || (largest != 0.0f && __builtin_amdgcn_inverse_ballot_w64(noneYet))) && e < 128;    // (an infinity stays one whatever the scale)
-        const int by = lower ? min(11 - e, 126 - has) : 0, by2 = by / 2;       // (in two factors: it goes down to -240)
+        const int by = lower ? min(11 - e, 126 - has) : 0, by2 = sums ? by / 2 : by;       // (in two factors: it goes down to -240.  The first one does not)
         // Samples that no scale makes large enough, fp32 denormals, are left to the pass over what did not come out finite.
         const float f1 = e + by < 1 && lower ? __builtin_nanf("") : __uint_as_float((unsigned)(127 + by2) << 23), f2 = __uint_as_float((unsigned)(127 + by - by2) << 23);
-        auto times = [&](float x) { return x * f1 * f2; };
+        auto times = [&](float x) { return sums ? x * f1 * f2 : x * f1; };
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             k[c] = times(k[c]);
@@ -882,7 +886,19 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
 #pragma unroll
     for (int q = 0; q < 2 * NT; ++q) load_filter(rU, 1, q & 1, kPA[q / 2], first + set + KW * turn);
 #pragma unroll
-    for (int n = 0; n < 16; ++n) { read_two(0, n % RING, n / 4, 2 * (n % 4)); combine_two(n % RING, n / 4, 2 * (n % 4)); }
+    for (int c = 0; c < 4; c += 2) {                // (eight reads under way: the sums' registers are still free)
+        float pa[8][2], pb[8][2];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            read_two(0, 0, c + i / 4, 2 * (i % 4));
+            pa[i][0] = ra[0][0]; pa[i][1] = ra[0][1]; pb[i][0] = rb[0][0]; pb[i][1] = rb[0][1];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            ra[0][0] = pa[i][0]; ra[0][1] = pa[i][1]; rb[0][0] = pb[i][0]; rb[0][1] = pb[i][1];
+            combine_two(0, c + i / 4, 2 * (i % 4));
+        }
+    }
     {   // the first scale: for `most` where it is not zero
         rescale(false);
         if (__builtin_amdgcn_inverse_ballot_w64(noneYet)) {
