@@ -1069,6 +1069,11 @@ using namespace drhip;
 //   * pieces 7.8, 2 more per pair of chunks and 0.22 per MB of filters (56x56 256->256 20.5 / 16.5, 28x28 512->512 23.4 / 20.4, 61x75 320->140 23.3 / 19.8,
 //     62x41 376->106 19.0 / 14.1, 51x41 191->384 18.0 / 15.5; 56x56 128->256 12.0 / 12.2, 28x28 256->512 14.6 / 16.9, 84x68 224->64 12.0 / 12.2 and fewer panels
 //     stay there).
+//   * one to one and a half panels per CU: with one wave set, whole panels on seven CUs of eight and all others in halves, everything at once (whole
+//     panels / whole ones on every CU and the rest in quarters / this: 80x60 512->512 64.1 / 55.8 / 53.2, 256->512 35.2 / 34.3 / 30.1, 120x80 256->256
+//     36.8 / 34.1 / 29.7; whole / this: 88x64 512->512 65.2 / 58.7, 132x66 200->256 31.1 / 25.5, 122x93 128->256 21.7 / 20.7; with fewer chunks
+//     than 8 no more than 4 %).  Six to eight of eight CUs with whole panels measure the same within 2 %; with more than one and a half panels
+//     per CU halves do not fit in beside them (100x78 400->400 56.0 / 61.8).
 //   * one workgroup for more than half of the CUs from 4 chunks on (112x112 64->128 12.0 / 9.4, 48x56 64->448 12.0 / 9.4, 55x57 93->305 17.1 / 12.1), with
 //     two wave sets from 8 (118x112 160->70 18.0 / 15.5, one set 16.2; 85x111 288->128 23.4 and 26.7).
 static int ws_pick(int W, int H, int I, int O, bool pair) {
@@ -1095,6 +1100,8 @@ static int ws_pick(int W, int H, int I, int O, bool pair) {
     }
     if (!wide) return 0;
     const int over = n - cusPerXcd, over2 = n - 2 * cusPerXcd;
+    if (pair && joins && over > 0 && 2 * over <= cusPerXcd && nC >= 8)
+        if (const int v = split(0x100, std::max(cusPerXcd * 7 / 8, 2 * over), 1, 2)) return v;
     if (joins && over > 0 && (nC >= 24 ? 3 * over <= cusPerXcd : nC >= 16 && 5 * over <= cusPerXcd))
         if (const int v = split(0x101, cusPerXcd, 1, 4 * over <= cusPerXcd ? 4 : 3)) return v;
     if (joins && nC >= 8 && over2 > 0 && 2 * over2 <= cusPerXcd)
