@@ -41,6 +41,7 @@ static Touched touched_by(dR_Node* n) {
         const dR_Conv2d_Data* c = (const dR_Conv2d_Data*)n->layer;
         if (c->drPooledInput) reads_inputs_of(c->drPooledInput);
         if (c->drAbsorbed1x1) t.writes.push_back(out_range(c->drAbsorbed1x1));
+        if (c->drJoins) t.writes.push_back(Range{(const char*)c->workspaceBuf, (const char*)c->workspaceBuf + 1});
         if (c->drFusedPool && c->drPoolAverage) t.writes.push_back(out_range((dR_Node*)n->next_layers->first->element));
     }
     if (n->type == tSoftmax && ((const dR_Softmax_Data*)n->layer)->drFcInput) reads_inputs_of(((const dR_Softmax_Data*)n->layer)->drFcInput);

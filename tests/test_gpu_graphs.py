@@ -991,6 +991,8 @@ def _branches_spec(kind):
     elif kind == "on load":         # node 6 writes where node 1 was, which node 3 in front of it pools on load
         spec = [{"op": "feed", "shape": (37, 29, 8)}, conv(st, 0, 5, 8, 16), pool(1, 3, 2), conv(st, 2, 1, 16, 24), conv(st, 0, 1, 8, 16), conv(st, 4, 3, 16, 12),
                 conv(st, 5, 1, 12, 16), conv(st, 3, 1, 24, 6), conv(st, 6, 1, 16, 4)]
+    elif kind == "joins":           # both leave partial tiles in the graph's one region for them
+        spec = [{"op": "feed", "shape": (33, 31, 256)}, conv(st, 0, 3, 256, 512), conv(st, 0, 3, 256, 256)]
     else:                           # node 6 writes where node 1 was, which the softmax in front of it reads for the layer that it computes
         fc = lambda src, k, n: {"op": "fc", "in": src, "w": (st.next().standard_normal((k, n)) * k ** -0.5).astype(np.float32), "b": None, "relu": True}
         spec = [{"op": "feed", "shape": (60, 1, 1)}, fc(0, 60, 60), fc(1, 60, 20), {"op": "softmax", "in": 2}, fc(0, 60, 50), fc(4, 50, 60), fc(5, 60, 60), fc(6, 60, 30), {"op": "softmax", "in": 7}]
@@ -998,7 +1000,7 @@ def _branches_spec(kind):
     return spec, [i for i in range(1, len(spec)) if i not in read]
 
 
-@pytest.mark.parametrize("kind", ["average", "on load", "softmax"])
+@pytest.mark.parametrize("kind", ["average", "on load", "softmax", "joins"])
 def test_branches_keep_off_memory_that_fusions_touch(oracle, gpu, kind):
     """Independent nodes on side streams (DR_BRANCHES=1): every replay as node by node."""
     spec, outs = _branches_spec(kind)
@@ -1007,13 +1009,34 @@ def test_branches_keep_off_memory_that_fusions_touch(oracle, gpu, kind):
     inputs = [rng.standard_normal((c, h, w)).astype(np.float32) for _ in range(4)]
     eager, _ = _run_many(spec, outs, inputs, graph_mode=False)
     forked, used = _run_many(spec, outs, inputs, graph_mode=True, branches=True)
-    assert used
+    assert used and (kind != "joins" or _run_many.groups == 0)
     want = oracle.run_spec(spec, {0: inputs[0]})
     for i, a in zip(outs, eager[0]):
         assert rel_err(a, want[i]) <= LAYER_TOL
     for a, b in zip(eager, forked):
         for x, y in zip(a, b):
             assert np.array_equal(x, y)
+
+
+def test_joined_layers_share_one_region(oracle, gpu):
+    """Halves, quarters, helpers and pieces of one graph, one behind the other, leave the region as they found it: every pass gives the same bits, and
+    those of the layers in graphs of their own."""
+    st = configs._Streams(81)
+    conv = configs._conv
+    spec = [{"op": "feed", "shape": (48, 48, 256)}, conv(st, 0, 3, 256, 256), conv(st, 1, 3, 256, 256), {"op": "pool", "in": 2, "window": (2, 2, 1), "stride": (2, 2, 1), "kind": 0},
+            conv(st, 3, 3, 256, 512), conv(st, 4, 3, 512, 512), {"op": "pool", "in": 5, "window": (2, 2, 1), "stride": (2, 2, 1), "kind": 0}, conv(st, 6, 3, 512, 512)]
+    x = np.random.default_rng(6).standard_normal((256, 48, 48)).astype(np.float32)
+    (first, second, third), _ = _run_many(spec, [3, 4, 6, 7], [x, 2 * x, x], graph_mode=False)
+    for a, b in zip(first, third):
+        assert np.array_equal(a, b)
+    got, src = first, x
+    for layers, a in (((1, 2, 3), got[0]), ((4,), got[1]), ((5, 6), got[2]), ((7,), got[3])):
+        own = [{"op": "feed", "shape": src.shape[::-1]}] + [dict(spec[i], **{"in": k}) for k, i in enumerate(layers)]
+        alone, _ = _run_many(own, [len(own) - 1], [src], graph_mode=False)
+        assert np.array_equal(alone[0][0], a), layers
+        want = oracle.run_spec(own, {0: src})[-1]
+        assert rel_err(a, want) <= LAYER_TOL
+        src = a
 
 
 @pytest.mark.parametrize("W,H,I,O,helpers", [(33, 31, 256, 512, False), (56, 56, 256, 256, True), (48, 48, 128, 256, True)])
