@@ -306,8 +306,9 @@ __device__ __forceinline__ void ws_finish(const float* P, const float* biasT, co
                     if (q < q0 || q >= q0 + count) wino_see_off(rWs, slot_of(split, q), spins);
             }
         };
-        if (KW == 1 || nSp == 2) join(integral_constant<int, 2>{});
-        else if constexpr (KW == 2) {
+        constexpr bool kHalvesOnly = KW == 1 && Bank::PARTS == 3;
+        if (kHalvesOnly || nSp == 2) join(integral_constant<int, 2>{});
+        else if constexpr (!kHalvesOnly) {
             if (nSp == 3) join(integral_constant<int, 3>{});
             else join(integral_constant<int, 4>{});
         }
@@ -1015,7 +1016,7 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
     if (s.sA == 1 && s.sB == 1) return true;
     // A workgroup waits for the other splits of its panel, which are its neighbours in dispatch order on the same XCD: as long
     // as one XCD holds more workgroups than a panel has splits, they all get to run.
-    auto allowed = [&](int n) { return n >= 1 && n <= 2 * p->kw && (n - 1) * ceil_div(s.nC, n) < s.nC; };
+    auto allowed = [&](int n) { return n >= 1 && n <= (p->pair ? 4 : 2 * p->kw) && (n - 1) * ceil_div(s.nC, n) < s.nC; };
     return s.nA <= panels && allowed(s.sA) && allowed(s.sB) && std::max(s.sA, s.sB) < num_cu() / kXcds && p->perXcd < 8192 &&
            (long long)p->perXcd * kXcds * 32768 < (1ll << 31);
 }
@@ -1069,11 +1070,12 @@ using namespace drhip;
 //   * pieces 7.8, 2 more per pair of chunks and 0.22 per MB of filters (56x56 256->256 20.5 / 16.5, 28x28 512->512 23.4 / 20.4, 61x75 320->140 23.3 / 19.8,
 //     62x41 376->106 19.0 / 14.1, 51x41 191->384 18.0 / 15.5; 56x56 128->256 12.0 / 12.2, 28x28 256->512 14.6 / 16.9, 84x68 224->64 12.0 / 12.2 and fewer panels
 //     stay there).
-//   * one to one and a half panels per CU: with one wave set, whole panels on seven CUs of eight and all others in halves, everything at once (whole
-//     panels / whole ones on every CU and the rest in quarters / this: 80x60 512->512 64.1 / 55.8 / 53.2, 256->512 35.2 / 34.3 / 30.1, 120x80 256->256
-//     36.8 / 34.1 / 29.7; whole / this: 88x64 512->512 65.2 / 58.7, 132x66 200->256 31.1 / 25.5, 122x93 128->256 21.7 / 20.7; with fewer chunks
+//   * one to one and a half panels per CU: with one wave set, whole panels on seven CUs of eight and all others in halves, or, where there is room for
+//     those at once as well, in thirds or quarters (whole panels / whole ones on every CU and the rest in quarters / this: 80x60 512->512 64.1 / 55.8 / 52.0,
+//     256->512 35.2 / 34.3 / 30.2, 120x80 256->256 36.8 / 34.1 / 29.8, 80x52 512->512 61.0 / 51.6 / 46.4 and in halves 48.8; whole / this: 88x64 512->512 65.2 / 58.7, 132x66 200->256 31.1 / 25.5, 122x93 128->256 21.7 / 20.7; with fewer chunks
 //     than 8 no more than 4 %).  Six to eight of eight CUs with whole panels measure the same within 2 %; with more than one and a half panels
 //     per CU halves do not fit in beside them (100x78 400->400 56.0 / 61.8).
+//   * no more than one in six CUs over two panels each: those in quarters (144x120 256->256 in halves 51.8, in quarters 48.5; 160x120, one in three, 53.8 and 57.4).
 //   * one workgroup for more than half of the CUs from 4 chunks on (112x112 64->128 12.0 / 9.4, 48x56 64->448 12.0 / 9.4, 55x57 93->305 17.1 / 12.1), with
 //     two wave sets from 8 (118x112 160->70 18.0 / 15.5, one set 16.2; 85x111 288->128 23.4 and 26.7).
 static int ws_pick(int W, int H, int I, int O, bool pair) {
@@ -1084,7 +1086,7 @@ static int ws_pick(int W, int H, int I, int O, bool pair) {
     static const bool joins = [] { const char* e = getenv("DR_WINO_JOIN"); return !(e && e[0] == '0'); }();
     auto split = [&](int base, int nA, int sA, int sB) {
         const int v = base | sA << 12 | sB << 16 | nA << 20;
-        return ws_plan(W, H, I, O, v, &p) ? v : 0;
+        return ws_plan(W, H, I, O, v | (pair ? 0x200 : 0), &p) ? v : 0;
     };
     if (joins && 2 * n <= cusPerXcd) {
         // Against the fp32 kernel in equal splits and two launches, although its joined halves and helpers may be up to 1.2 times as fast as the
@@ -1100,10 +1102,15 @@ static int ws_pick(int W, int H, int I, int O, bool pair) {
     }
     if (!wide) return 0;
     const int over = n - cusPerXcd, over2 = n - 2 * cusPerXcd;
-    if (pair && joins && over > 0 && 2 * over <= cusPerXcd && nC >= 8)
-        if (const int v = split(0x100, std::max(cusPerXcd * 7 / 8, 2 * over), 1, 2)) return v;
+    if (pair && joins && over > 0 && 2 * over <= cusPerXcd && nC >= 8) {
+        const int whole = std::max(cusPerXcd * 7 / 8, 2 * over);
+        for (int k = std::min(4, (2 * cusPerXcd - whole) / (n - whole)); k >= 2; --k)
+            if (const int v = split(0x100, whole, 1, k)) return v;
+    }
     if (joins && over > 0 && (nC >= 24 ? 3 * over <= cusPerXcd : nC >= 16 && 5 * over <= cusPerXcd))
         if (const int v = split(0x101, cusPerXcd, 1, 4 * over <= cusPerXcd ? 4 : 3)) return v;
+    if (pair && joins && nC >= 8 && over2 > 0 && 6 * over2 <= cusPerXcd)
+        if (const int v = split(0x100, 2 * cusPerXcd, 1, 4)) return v;
     if (joins && nC >= 8 && over2 > 0 && 2 * over2 <= cusPerXcd)
         if (const int v = split(0x100, 2 * cusPerXcd, 1, 2)) return v;
     if (pair && blocks <= cus) return 2 * n > cusPerXcd && nC >= 4 ? (nC >= 8 ? 0x101 : 0x100) : 0;

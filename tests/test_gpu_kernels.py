@@ -541,7 +541,8 @@ def pair_winograd(lib, dev, x, w, variant, flags=0, bias=None):
     (0x100, 33, 17, 16, 33), (0x101, 31, 40, 17, 70), (0x100, 61, 63, 64, 128), (0x101, 61, 63, 65, 128), (0x100, 32, 2, 33, 65), (0x101, 75, 1, 48, 1),
     (0x100, 224, 20, 3, 64), (0x101, 11, 30, 33, 40), (0x101, 320, 6, 200, 96), (0x101, 28, 28, 256, 512), (0x100 | SPLIT_HALVES, 61, 63, 64, 128),
     (0x101 | SPLIT_HALVES, 28, 28, 256, 512), (0x101 | 3 << 12 | 3 << 16, 27, 14, 112, 200), (0x101 | SPLIT_MIXED, 64, 36, 100, 70),
-    (0x100 | 3 << 20 | 1 << 12 | 2 << 16, 64, 36, 130, 70)])
+    (0x100 | 3 << 20 | 1 << 12 | 2 << 16, 64, 36, 130, 70), (0x100 | 4 << 20 | 1 << 12 | 3 << 16, 64, 36, 130, 70),
+    (0x100 | 4 << 20 | 1 << 12 | 4 << 16, 63, 36, 200, 70), (0x100 | 3 << 12 | 3 << 16, 61, 20, 79, 65)])
 def test_winograd_pair_operands(lib, dev, oracle, variant, W, H, I, O):
     """Winograd on the f16 matrix cores, operands split into two parts: ragged channels, single steps, narrow and one-row maps, pieces, panels that begin
     at different channels, the pooling epilogue.  Held to a twentieth of the layer bar, like three parts."""

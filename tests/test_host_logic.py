@@ -834,6 +834,11 @@ def test_split_winograd_variants_are_those_that_the_rule_can_pick(lib):
     assert [n for n in range(16) if joins(0x100, n)] == [2] and [n for n in range(16) if joins(0x101, n)] == [2, 3, 4]
 
 
+def test_pair_winograd_joins_up_to_four_pieces(lib):
+    joins = lambda base, n: lib.drhip_conv3x3_winograd_split_workspace_floats(160, 120, 256, 256, base | n << 12 | n << 16) > 0
+    assert [n for n in range(16) if joins(0x300, n)] == [n for n in range(16) if joins(0x301, n)] == [2, 3, 4]
+
+
 def test_split_winograd_workspace_holds_pieces_only(lib):
     """160x120 256->256 is 600 panels, 75 per XCD: slots of 32 KiB for the pieces, none for panels that stay whole."""
     floats = lambda v: lib.drhip_conv3x3_winograd_split_workspace_floats(160, 120, 256, 256, v)
@@ -878,7 +883,7 @@ def test_layers_stay_in_pieces_for_their_exactness(lib, W, H, I, O, pieces):
     (56, 56, 256, 256, 0x22301), (28, 28, 512, 512, 0x44301), (62, 41, 376, 106, 0x44301), (47, 61, 192, 192, 0x33301),     # pieces where they are the faster ones
     (56, 56, 128, 256, 0), (28, 28, 256, 512, 0), (84, 68, 224, 64, 0), (14, 14, 512, 512, 0), (45, 60, 480, 64, 0),
     (112, 112, 64, 128, 0x300), (112, 112, 127, 128, 0x301), (112, 112, 112, 128, 0x300), (112, 112, 63, 128, 0),           # one round that fills more than half of the CUs
-    (80, 60, 512, 512, 0x1c21300), (80, 52, 192, 512, 0x1c21300), (128, 96, 128, 256, 0x2021300), (122, 93, 256, 256, 0x1c21300),   # whole panels beside halves
+    (80, 60, 512, 512, 0x1c31300), (80, 52, 192, 512, 0x1c41300), (144, 120, 256, 256, 0x4041300), (160, 120, 256, 256, 0x4021300), (128, 96, 128, 256, 0x2021300), (122, 93, 256, 256, 0x1c21300),   # whole panels beside halves
     (124, 101, 384, 200, 0x300), (108, 90, 112, 256, 0x300), (112, 128, 112, 128, 0x300),
     (64, 64, 64, 256, 0), (64, 66, 64, 256, 0x300), (28, 30, 64, 1024, 0)])                                                # 128 panels, 132, and none of them on maps that narrow
 def test_winograd_pair_variant_by_panels_and_chunks(lib, W, H, I, O, variant):
