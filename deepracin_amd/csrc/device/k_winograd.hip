@@ -459,7 +459,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                     const int ol = eo + EO * q, o = o0 + ol;
                     if ((ol >> lgRows) != split) continue;
                     const f32x4 own = tile_of(ol);
-                    u32x4 part[S] = {};
+                    u32x4 part[S];
                     bool ready = false;
                     for (int spins = 0; spins <= joinSpins && !ready; ++spins) {
                         if (spins == joinSpins) wino_gives_up(&g_wino_join_timeouts);
@@ -468,7 +468,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
                         asm volatile("" ::: "memory");
                         ready = true;
 #pragma unroll
-                        for (int u = 0; u < S; ++u) if (u != split) part[u] = __builtin_amdgcn_raw_buffer_load_b128(rWs, place_of(ol), region_of(u), kAuxDeviceVolatile);
+                        for (int u = 0; u < S; ++u) part[u] = __builtin_amdgcn_raw_buffer_load_b128(rWs, place_of(ol), region_of(u), kAuxDeviceVolatile);
 #pragma unroll
                         for (int u = 0; u < S; ++u)
                             ready = ready && (u == split || wino_slot_full(part[u]));
@@ -479,7 +479,7 @@ winograd_f23_mfma_kernel(const float* __restrict__ in, const float* __restrict__
 #pragma unroll
                     for (int u = 0; u < S; ++u) s += (u == split) ? own : __builtin_bit_cast(f32x4, part[u]);
 #pragma unroll
-                    for (int u = 0; u < S; ++u) if (u != split) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, place_of(ol) + region_of(u), 0, kAuxThrough);
+                    for (int u = 0; u < S; ++u) __builtin_amdgcn_raw_buffer_store_b128(empty, rWs, place_of(ol) + region_of(u), 0, kAuxThrough);
                     // a partner never delivered: it shows in the result, too
                     if (!ready) s = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
                     if (eTileOk && o < O) {
