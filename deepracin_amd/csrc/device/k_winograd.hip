@@ -1070,6 +1070,10 @@ int drhip::wino_halvings(int W, int H, int I, int O) {
     return !wide && lg >= 1 && lg < 5 && O >= 64 && (panels << lg) > cus && (nChunks >> lg) >= 32 ? lg + 1 : lg;
 }
 
+int drhip::wino_donated(int W, int H, int I, int O) {
+    return wino_helpers(ceil_div(((W + 1) / 2) * ((H + 1) / 2), 32) * ceil_div(O, 32), ceil_div(I, kWinoKC), num_cu() / kXcds).donated;
+}
+
 // joins: a launch that joins splits or takes helpers may be picked.  (Without, the choice needs no larger workspace than with: the caller of
 // variant 0 has asked for that one.)
 static int wino_pick(int W, int H, int I, int O, bool joins) {

@@ -740,8 +740,8 @@ __device__ __forceinline__ void ws_word_to_lds(__amdgpu_buffer_rsrc_t from, int 
 
 // Winograd on the f16 matrix cores, operands in two parts (f16x2.hpp): the three-part kernel's panels, waves, steps and pieces, with 24 MFMAs a wave and
 // step instead of 48, 16 KiB of filters instead of 24 and 176 vector instructions instead of 270.  Layers, us, three parts / two, with their errors
-// against 64 bits (rms, 1e-7): 640x480 64->64 85 / 67 (2.2 / 1.9), 320x240 128->128 75.0 / 56.9 (2.8 / 2.3), 160x120 256->256 73.6 / 54.1 (3.7 / 2.9),
-// 80x60 512->512 75.7 / 54.7 (3.7 / 2.9), 112x112 128->128 16.0 / 13.0 (2.1 / 1.9), 40x30 512->512 27.8 / 22.0 (2.5 / 2.2).
+// against 64 bits (rms, 1e-7): 640x480 64->64 81.8 / 66.2 (1.82 / 1.62), 320x240 128->128 75.0 / 55.7 (2.40 / 2.01), 160x120 256->256 73.7 / 53.9
+// (3.23 / 2.56), 112x112 128->128 16.9 / 13.4 (1.85 / 1.66), 40x30 512->512 29.2 / 22.9 (2.24 / 1.96), 80x60 512->512 76.4 / 54.0 (3.16 / 3.05).
 // No value may go to scratch: a kernel that has any starts about 1 us later (the eight such layers of VGG16 293 -> 287 us a pass).
 // What bounds it: two workgroups of a CU take 4480 clocks a step on 320x240, the fetches without the MFMAs 2630 (168 KB at 64 bytes a clock), MFMAs and vector
 // instructions without fetches 1940: eight fragments of filters under way per wave do not cover the way to L2 while a CU's eight waves queue there.
@@ -1067,17 +1067,24 @@ using namespace drhip;
 //     After more rounds than one the workgroups do not end together any more (320x240 128->128, 2.3 rounds: 80 against 74).
 //
 // Two f16 parts take less (measured like that, 70 shapes drawn and VGG16's, with other filters each time, us fp32 kernel / this):
-//   * pieces 7.8, 2 more per pair of chunks and 0.22 per MB of filters (56x56 256->256 20.5 / 16.5, 28x28 512->512 23.4 / 20.4, 61x75 320->140 23.3 / 19.8,
-//     62x41 376->106 19.0 / 14.1, 51x41 191->384 18.0 / 15.5; 56x56 128->256 12.0 / 12.2, 28x28 256->512 14.6 / 16.9, 84x68 224->64 12.0 / 12.2 and fewer panels
-//     stay there).
-//   * one to one and a half panels per CU: with one wave set, whole panels on seven CUs of eight and all others in halves, or, where there is room for
-//     those at once as well, in thirds or quarters (whole panels / whole ones on every CU and the rest in quarters / this: 80x60 512->512 64.1 / 55.8 / 52.0,
-//     256->512 35.2 / 34.3 / 30.2, 120x80 256->256 36.8 / 34.1 / 29.8, 80x52 512->512 61.0 / 51.6 / 46.4 and in halves 48.8; whole / this: 88x64 512->512 65.2 / 58.7, 132x66 200->256 31.1 / 25.5, 122x93 128->256 21.7 / 20.7; with fewer chunks
-//     than 8 no more than 4 %).  Six to eight of eight CUs with whole panels measure the same within 2 %; with more than one and a half panels
-//     per CU halves do not fit in beside them (100x78 400->400 56.0 / 61.8).
+//   * pieces 7.8, 2 more per pair of chunks and 0.22 per MB of filters (56x56 256->256 20.3 / 16.4, 28x28 512->512 23.2 / 18.9, 61x75 320->140 23.3 / 19.8,
+//     62x41 376->106 19.0 / 14.1, 51x41 191->384 18.0 / 15.5; 56x56 128->256 12.2 / 11.7, 28x28 256->512 14.0 / 14.4, 84x68 224->64 12.0 / 12.2 and fewer panels
+//     stay there).  Where that kernel has helpers it takes 0.56 per stage that its own workgroups keep and 3.6 (39x152 198->68 13.6 / 15.2, 18x74 230->466
+//     16.0 / 17.8 stay there).  300 drawn shapes of up to 16 panels: 0.90 to 1.003 times the fp32 kernel's time but for one (21x148 232->79, 12.7 / 14.2).
+//   * two thirds of a panel per CU at most, and fp32 panels for more than half of a round: from 19 chunks on all in thirds, with one wave set (73x28 400->476
+//     32 / 28, 52x56 440->330 35.3 / 30.7; two wave sets unsplit 30.0 and 33.5; 80x60 512->256 33.6 against 35.8, 256->256 23.5 against 21.0).
+//   * up to one and a half panels per CU: with one wave set, whole panels on seven CUs of eight and all others in halves, or, where there is room for
+//     those at once as well, in thirds or quarters (whole / this: 88x64 512->512 65.2 / 58.7, 132x66 200->256 31.1 / 25.5, 122x93 128->256 21.7 / 20.7;
+//     with fewer chunks than 8 no more than 4 %).  With more than one and a half panels per CU halves do not fit in beside them (100x78 400->400 56.0 / 61.8).
+//   * Where three parts would have whole panels of two wave sets, whose sums are half as long, that would be less exact than they (by up to 3 %).  Up to
+//     1/4 over, without padded outputs: half of the panels in halves, or, with 1/16 over, as many in quarters as leave two slots of the XCD empty (three parts /
+//     seven of eight / this, and the errors against 64 bits, 1e-7: 80x60 512->512 76.4 / 52.9 / 54.0, 3.16 / 3.18 / 3.05; 80x60 256->512 43.7 / 30.7 / 31.2,
+//     2.37 / 2.44 / 2.36; 71x119 256->256 42.8 / 28.8 / 29.5, 2.60 / 2.63 / 2.56; all slots taken 63 against 57 where 10 fewer are).  Otherwise two wave
+//     sets here too (81x86 384->384 65.2 / 45.4 / 49.2, 2.79 / 2.89 / 2.30).  Over 100 drawn shapes the error is 0.62 to 0.998 times three parts'.
 //   * no more than one in six CUs over two panels each: those in quarters (144x120 256->256 in halves 51.8, in quarters 48.5; 160x120, one in three, 53.8 and 57.4).
 //   * one workgroup for more than half of the CUs from 4 chunks on (112x112 64->128 12.0 / 9.4, 48x56 64->448 12.0 / 9.4, 55x57 93->305 17.1 / 12.1), with
-//     two wave sets from 8 (118x112 160->70 18.0 / 15.5, one set 16.2; 85x111 288->128 23.4 and 26.7).
+//     two wave sets from 8 (118x112 160->70 18.0 / 15.5, one set 16.2; 85x111 288->128 23.4 and 26.7), but none where the fp32 kernel's panels, of 32 outputs,
+//     are a round (73x28 66->476 9.0 / 11.0, 34x159 140->141 12.9 / 16.2, 38x74 300->344 24.4 / 25.2).
 static int ws_pick(int W, int H, int I, int O, bool pair) {
     WsPlan p;
     if (O <= 32 || !ws_plan(W, H, I, O, 0x101, &p)) return 0;
@@ -1094,26 +1101,34 @@ static int ws_pick(int W, int H, int I, int O, bool pair) {
         // and stay where they gain on a form whose sums are as short.  And against what that kernel takes, where that is the slower one.
         const int S = std::min(4, cusPerXcd / n), halvings = wino_halvings(W, H, I, O), panels32 = p.s.nTB * ceil_div(O, 32);
         auto fp32 = [&](int lg) { return 0.56 * ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus) + (lg > 0 ? 4.5 : 3); };
-        const int pairs = ceil_div(ceil_div(nC, S), 2);
-        const double taken = fp32(drhip_conv3x3_winograd_pick_variant(W, H, I, O) >> 4 & 15);
+        const int pairs = ceil_div(ceil_div(nC, S), 2), picked = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
+        const double taken = fp32(picked >> 4 & 15);
+        const double helped = picked & 0x2000 ? 0.56 * (ceil_div(I, 8) - wino_donated(W, H, I, O)) + 3.6 : taken;
         if (halvings >= 0 &&                            // (layers of its 16-tile form are too small)
-            (2.75 * pairs + 10.6 < 0.93 * std::max(fp32(halvings), taken) || (pair && 2.0 * pairs + 7.8 + 0.22e-6 * 64 * I * O < 0.93 * taken)))
+            (2.75 * pairs + 10.6 < 0.93 * std::max(fp32(halvings), taken) || (pair && 2.0 * pairs + 7.8 + 0.22e-6 * 64 * I * O < 0.93 * helped)))
             if (const int v = split(0x101, 0, S, S)) return v;
     }
     if (!wide) return 0;
     const int over = n - cusPerXcd, over2 = n - 2 * cusPerXcd;
-    if (pair && joins && over > 0 && 2 * over <= cusPerXcd && nC >= 8) {
+    const bool fewMore = joins && over > 0 && (nC >= 24 ? 3 * over <= cusPerXcd : nC >= 16 && 5 * over <= cusPerXcd);      // than one panel per CU
+    if (pair && fewMore && O % 64 == 0 && 4 * over <= cusPerXcd) {
+        const int k = 16 * over <= cusPerXcd ? 4 : 2, whole = k == 4 ? ceil_div(4 * n - 2 * cusPerXcd + 2, 3) : n / 2;
+        if (const int v = split(0x100, whole, 1, k)) return v;
+    }
+    if (pair && joins && !fewMore && over > 0 && 2 * over <= cusPerXcd && nC >= 8) {
         const int whole = std::max(cusPerXcd * 7 / 8, 2 * over);
         for (int k = std::min(4, (2 * cusPerXcd - whole) / (n - whole)); k >= 2; --k)
             if (const int v = split(0x100, whole, 1, k)) return v;
     }
-    if (joins && over > 0 && (nC >= 24 ? 3 * over <= cusPerXcd : nC >= 16 && 5 * over <= cusPerXcd))
+    if (fewMore)
         if (const int v = split(0x101, cusPerXcd, 1, 4 * over <= cusPerXcd ? 4 : 3)) return v;
     if (pair && joins && nC >= 8 && over2 > 0 && 6 * over2 <= cusPerXcd)
         if (const int v = split(0x100, 2 * cusPerXcd, 1, 4)) return v;
     if (joins && nC >= 8 && over2 > 0 && 2 * over2 <= cusPerXcd)
         if (const int v = split(0x100, 2 * cusPerXcd, 1, 2)) return v;
-    if (pair && blocks <= cus) return 2 * n > cusPerXcd && nC >= 4 ? (nC >= 8 ? 0x101 : 0x100) : 0;
+    if (pair && joins && over <= 0 && 3 * n <= 2 * cusPerXcd && 2 * n > cusPerXcd && nC >= 19)
+        if (const int v = split(0x100, 0, 3, 3)) return v;
+    if (pair && blocks <= cus) return p.s.nTB * ceil_div(O, 32) > cus && nC >= 4 ? (nC >= 8 ? 0x101 : 0x100) : 0;
     if (blocks <= cus) return nC >= 8 && 20 * blocks >= 11 * cus ? 0x101 : 0;
     return nC >= 4 || (nC >= 2 && 2 * blocks >= 3 * cus) ? 0x100 : 0;
 }

@@ -66,6 +66,7 @@ constexpr int kAuxDeviceVolatile = 16 | (int)0x80000000u;   // sc1 and volatile,
 int ws_join_timeouts(unsigned* count);              // of the split-operand kernel
 int wino_join_spins();                              // bound on the wait for a partner's partial tile
 int wino_halvings(int W, int H, int I, int O);      // of the input channels where the fp32 kernel neither joins nor helps; -1: its 16-tile form
+int wino_donated(int W, int H, int I, int O);       // stages of 8 channels that helpers take off each of its panels where it has helpers (0x2c01)
 
 // Nothing of a launch may lie in its workspace when the launch has ended: the next one would take a partial tile that came too
 // late for its own panel.  Whoever gives a tile up adds to the kernel's counter first and looks once more behind that; whoever has stored

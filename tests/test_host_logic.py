@@ -883,7 +883,10 @@ def test_layers_stay_in_pieces_for_their_exactness(lib, W, H, I, O, pieces):
     (56, 56, 256, 256, 0x22301), (28, 28, 512, 512, 0x44301), (62, 41, 376, 106, 0x44301), (47, 61, 192, 192, 0x33301),     # pieces where they are the faster ones
     (56, 56, 128, 256, 0), (28, 28, 256, 512, 0), (84, 68, 224, 64, 0), (14, 14, 512, 512, 0), (45, 60, 480, 64, 0),
     (112, 112, 64, 128, 0x300), (112, 112, 127, 128, 0x301), (112, 112, 112, 128, 0x300), (112, 112, 63, 128, 0),           # one round that fills more than half of the CUs
-    (80, 60, 512, 512, 0x1c31300), (80, 52, 192, 512, 0x1c41300), (144, 120, 256, 256, 0x4041300), (160, 120, 256, 256, 0x4021300), (128, 96, 128, 256, 0x2021300), (122, 93, 256, 256, 0x1c21300),   # whole panels beside halves
+    (73, 28, 128, 476, 0), (34, 159, 69, 141, 0), (40, 40, 146, 294, 0), (39, 152, 198, 68, 0),                             # one round or helpers of the fp32 kernel
+    (73, 28, 400, 476, 0x33300), (80, 60, 304, 256, 0x33300), (80, 60, 288, 256, 0x301), (88, 64, 304, 256, 0x301),         # thirds, all at once
+    (75, 53, 256, 512, 0x1841300), (71, 119, 256, 256, 0x1941300), (62, 71, 512, 512, 0x1121300), (80, 60, 512, 512, 0x1321300), (113, 44, 384, 512, 0x1421300),    # half in halves, for short sums
+    (80, 60, 500, 500, 0x2041301), (114, 91, 384, 256, 0x2031301), (80, 52, 192, 512, 0x1c41300), (144, 120, 256, 256, 0x4041300), (160, 120, 256, 256, 0x4021300), (128, 96, 128, 256, 0x2021300), (122, 93, 256, 256, 0x1c21300),   # whole panels beside halves
     (124, 101, 384, 200, 0x300), (108, 90, 112, 256, 0x300), (112, 128, 112, 128, 0x300),
     (64, 64, 64, 256, 0), (64, 66, 64, 256, 0x300), (28, 30, 64, 1024, 0)])                                                # 128 panels, 132, and none of them on maps that narrow
 def test_winograd_pair_variant_by_panels_and_chunks(lib, W, H, I, O, variant):
