@@ -87,19 +87,26 @@ void pick_winograd(dR_Conv2d_Data* c, int O) {
     if (!c->drWinoSplit) c->variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
 }
 
-// Once its weights are known: operands in two f16 parts instead, where those can hold them.
+// Operands in two f16 parts instead, as far as the shape goes.
 void pick_winograd_pair(dR_Conv2d_Data* c, int O) {
     const int v = drhip_conv3x3_winograd_pair_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
-    const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
-    if (v == 0 || !c->hasVariables || (a && !a->hasVariables)) return;
-    if (!drhip_winograd_pair_fits(c->weights, c->shape.s2, c->shape.s3, 9) || (a && !drhip_winograd_pair_fits(a->weights, a->shape.s2, a->shape.s3, 1))) return;
+    if (v == 0) return;
     c->variant = v;
     c->drWinoSplit = TRUE;
+}
+bool fits_pair(const dR_Conv2d_Data* c) {
+    const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
+    return drhip_winograd_pair_fits(c->weights, c->shape.s2, c->shape.s3, 9) && (!a || drhip_winograd_pair_fits(a->weights, a->shape.s2, a->shape.s3, 1));
 }
 
 size_t winograd_workspace_floats(const dR_Conv2d_Data* c, int O) {
     return (c->drWinoSplit ? drhip_conv3x3_winograd_split_workspace_floats : drhip_conv3x3_winograd_workspace_floats)(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->variant);
 }
+size_t winograd_filter_floats(const dR_Conv2d_Data* c, int O) {
+    return (pair_bank(c) ? drhip_conv3x3_winograd_pair_filter_floats : c->drWinoSplit ? drhip_conv3x3_winograd_split_filter_floats : drhip_conv3x3_winograd_filter_floats)(c->shape.s2, O);
+}
+// Of the graph's region for partial tiles that are joined in their launch.
+size_t winograd_join_floats(const dR_Conv2d_Data* c, int O) { return c->drWinoSplit || (c->variant & 0x800) ? winograd_workspace_floats(c, O) : 0; }
 
 // ---- schedule: kernel variant and tile parameters for gfx950 -------------------------------------
 gboolean conv_schedule(dR_Graph* net, dR_Node* node) {
@@ -173,6 +180,32 @@ inline bool launch_has_bias(const dR_Conv2d_Data* c) {
     return c->useBias || (c->drAbsorbed1x1 && conv_of(c->drAbsorbed1x1)->useBias);
 }
 
+// Filters and split-K partial tiles of a Winograd layer in its present form.  Joined inside a launch the tiles have left the region when it ends, so
+// all such layers of a graph share one: in memory that was in use a few us ago a tile reaches its reader sooner.  (A region each, one for all: VGG16
+// 284.6 / 274.4 us a pass, its convolutions over 640x480 514.0 / 501.3.)
+gboolean allocate_winograd(dR_Graph* net, dR_Conv2d_Data* c) {
+    const int O = launch_channels(c);
+    gboolean ok = dR_createFloatBuffer(net, &c->weightsBuf, (gint)winograd_filter_floats(c, O), CL_MEM_READ_ONLY);
+    const size_t joins = winograd_join_floats(c, O), ws = winograd_workspace_floats(c, O);
+    c->drJoins = joins > 0;
+    net->drJoinFloats = std::max(net->drJoinFloats, (gsize)joins);
+    if (c->drJoins) c->workspaceBuf = net->drJoinBuf;       // (which dR_prepare makes when all layers have said what they need)
+    else if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);
+    return ok;
+}
+
+// A layer whose weights two f16 parts cannot hold, at first or because it got others since: the form that holds all, from here on.
+gboolean leave_pair(dR_Graph* net, dR_Conv2d_Data* c) {
+    const int O = launch_channels(c);
+    if (device_failed(net, drhip_stream_sync(stream_of(net)), "winograd filters (sync)")) return FALSE;     // (passes that read them)
+    if (net->drGraphExec) { drhip_graph_destroy(net->drGraphExec); net->drGraphExec = NULL; }               // (recorded with them)
+    net->clConfig->memConsumptionGPU -= (glong)(winograd_filter_floats(c, O) * sizeof(float));
+    if (!dR_clMemoryBufferCleanup(net, c->weightsBuf)) return FALSE;
+    c->weightsBuf = c->workspaceBuf = NULL;                 // (pieces in two parts are always joined)
+    pick_winograd(c, O);
+    return allocate_winograd(net, c);
+}
+
 gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     dR_Conv2d_Data* c = conv_of(node);
     if (c->drAbsorbedBy) return TRUE;           // the 3x3 sibling carries this node's filters and bias
@@ -188,26 +221,19 @@ gboolean conv_allocate(dR_Graph* net, dR_Node* node) {
     }
     const bool wino = c->algo == drConvWinograd;
     const int O = launch_channels(c);
-    if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
-    if (wino) pick_winograd_pair(c, O);
+    if (wino) {
+        if (c->drAbsorbed1x1) pick_winograd(c, O);  // the joint layer is wider than the one schedule() saw
+        net->drJoinFloats = std::max(net->drJoinFloats, (gsize)winograd_join_floats(c, O));     // (room for the form that a layer may have to go back to)
+        pick_winograd_pair(c, O);
+    }
     if (c->drSplitBank && c->drFusedPool)
         c->variant = pools_by_three(node) ? drhip_conv_bank_maxpool3s2_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 2)
                                           : drhip_conv_bank_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O, c->shape.s0, c->shape.s1, c->stride.s1, c->stride.s2, 1);
-    const int n = pair_bank(c) ? (int)drhip_conv3x3_winograd_pair_filter_floats(c->shape.s2, O)
-                       : c->drWinoSplit ? (int)drhip_conv3x3_winograd_split_filter_floats(c->shape.s2, O)
-                       : wino ? (int)drhip_conv3x3_winograd_filter_floats(c->shape.s2, O)
-                       : c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)
-                       : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1)
-                       : c->drByPixel ? ((O + 15) & ~15) * c->shape.s2 : weight_count(c);
-    gboolean ok = dR_createFloatBuffer(net, &c->weightsBuf, n, CL_MEM_READ_ONLY);
+    const int n = c->drDirectBank ? (int)drhip_conv3x3_direct_filter_floats(c->shape.s2, O)
+                : c->drSplitBank ? (int)drhip_conv_bank_floats(c->shape.s2, O, c->shape.s0, c->shape.s1)
+                : c->drByPixel ? ((O + 15) & ~15) * c->shape.s2 : weight_count(c);
+    gboolean ok = wino ? allocate_winograd(net, c) : dR_createFloatBuffer(net, &c->weightsBuf, n, CL_MEM_READ_ONLY);
     if (launch_has_bias(c)) ok = ok && dR_createFloatBuffer(net, &c->biasBuf, O, CL_MEM_READ_ONLY);
-    const size_t ws = wino ? winograd_workspace_floats(c, O) : 0;
-    // Split-K partial tiles.  Joined inside a launch they have left the region when it ends, so all such layers of a graph share one: in memory
-    // that was in use a few us ago a tile reaches its reader sooner.  (A region each, one for all: VGG16 284.6 / 274.4 us a pass, its
-    // convolutions over 640x480 514.0 / 501.3.)
-    c->drJoins = ws > 0 && (c->drWinoSplit || (c->variant & 0x800));
-    if (c->drJoins) net->drJoinFloats = std::max(net->drJoinFloats, (gsize)ws);
-    else if (ws > 0) ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, (gint)ws, CL_MEM_READ_WRITE);
     if (c->drFusedAvgPool)                      // per-tile pixel sums for the pooling behind this layer
         ok = ok && dR_createFloatBuffer(net, &c->workspaceBuf, avgpool_slices(c) * O, CL_MEM_READ_WRITE);
     return ok;
@@ -257,6 +283,7 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         // channels first (they sit just below this node's in the concat), centre tap only.
         const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
         if (a && !a->hasVariables) { say("Conv2d Layer %d has no weights: call dR_Conv2d_setVariables first! \n", c->drAbsorbed1x1->layerID); return FALSE; }
+        if (pair_bank(c) && !fits_pair(c) && !leave_pair(net, c)) return FALSE;
         const int I = c->shape.s2, O3 = c->shape.s3, O1 = a ? a->shape.s3 : 0, O = O1 + O3;
         std::vector<float> joint;
         const float* host = c->weights;

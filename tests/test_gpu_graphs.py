@@ -1039,6 +1039,67 @@ def test_joined_layers_share_one_region(oracle, gpu):
         src = a
 
 
+def _kernels(nodes):
+    """What the convolutions say that they run."""
+    fn = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_void_p)
+    texts = [ctypes.string_at(fn(dr.node_struct(n).printLayer)(n.ptr)).decode() for n in nodes if n.desc == "Conv2D"]
+    return [next(l for l in t.splitlines() if "Kernel:" in l) for t in texts]
+
+
+@pytest.mark.parametrize("replay", [False, True])
+@pytest.mark.parametrize("what", ["infinite", "nan", "far below"])
+@pytest.mark.parametrize("W,H,I,O", [(64, 66, 64, 256), (56, 56, 256, 256), (73, 28, 400, 476)])       # whole panels, halves behind which helpers join, thirds
+def test_refilled_weights_that_two_parts_cannot_hold(oracle, gpu, monkeypatch, W, H, I, O, what, replay):
+    """dR_Conv2d_setVariables and dR_fillBuffers on a prepared graph: weights that the first ones' bank has no room for are computed as a graph that was
+    prepared with them computes them, and so are the next ones; the other layer stays as it is."""
+    monkeypatch.setenv("DR_HIPGRAPH", "1" if replay else "0")
+    st = configs._Streams(83)
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, 3, I, O, relu=False), configs._conv(st, 0, 3, I, O, relu=False)]
+    x = np.random.default_rng(7).standard_normal((I, H, W)).astype(np.float32)
+    w0, b = spec[2]["w"], spec[2]["b"]
+    w1 = np.ascontiguousarray(w0[:, ::-1]).copy()
+    w1[3, 5, 1, 1] = {"infinite": np.inf, "nan": np.nan, "far below": 1.0}[what]
+    if what == "far below":                         # (and samples that make up for it)
+        w1[3] *= np.float32(2.0 ** -24)
+    xs = x.copy()
+    xs[3] *= np.float32(2.0 ** 24 if what == "far below" else 1.0)
+
+    def run(g, nodes, a):
+        configs.feed_chw(nodes[0], a)
+        assert g.lib.dR_apply(g.ptr)
+        return [y.copy() for y in configs.fetch_chw(g)]
+
+    def refill(g, node, w):
+        g.lib.dR_Conv2d_setVariables(node.ptr, dr._fptr(w), dr._fptr(b))
+        assert g.lib.dR_fillBuffers(ctypes.c_void_p(g.ptr)) == 1
+
+    with dr.Environment() as env:
+        g, own = env.create_graph(), env.create_graph()
+        nodes = configs.build_graph(g, spec, [1, 2])
+        dr.prepare(g)
+        before = _kernels(nodes)
+        assert all("f16" in k for k in before)
+        first = [run(g, nodes, a) for a in (x, xs, x)]
+        refill(g, nodes[2], w1)
+        got = [run(g, nodes, a) for a in (x, xs, x)]
+        assert _kernels(nodes)[0] == before[0]
+        there = configs.build_graph(own, spec[:2] + [dict(spec[2], w=w1)], [1, 2])
+        dr.prepare(own)
+        for a, old, now in zip((x, xs, x), first, got):
+            alone = run(own, there, a)
+            assert np.array_equal(now[0], old[0]) and np.array_equal(now[1], alone[1], equal_nan=True)
+            if what == "far below":
+                assert rel_err(now[1], oracle.conv_f64(a, w1, b, relu=False)) <= LAYER_TOL / 20
+            else:
+                assert np.isfinite(now[1][:5]).all() and not np.isfinite(now[1][5]).all()
+        assert _kernels(nodes) == _kernels(there) and "f16" not in _kernels(nodes)[1]
+        refill(g, nodes[2], w0)                     # weights that would fit again
+        again = [run(g, nodes, a) for a in (x, xs, x)]
+        for old, now in zip(first, again):
+            assert np.array_equal(now[0], old[0]) and rel_err(now[1], old[1]) <= LAYER_TOL / 20
+        assert all(np.array_equal(a, b) for a, b in zip(again[0], again[2]))
+
+
 @pytest.mark.parametrize("W,H,I,O,helpers", [(33, 31, 256, 512, False), (56, 56, 256, 256, True), (48, 48, 128, 256, True)])
 def test_joined_layers_of_two_graphs_on_two_streams(lib, gpu, W, H, I, O, helpers):
     """Pieces of a split-operand layer, and panels and their helpers, wait for each other inside the launch.  Two graphs with such a layer, each on its
