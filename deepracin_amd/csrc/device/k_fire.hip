@@ -426,6 +426,7 @@ extern "C" float drhip_fire_us(int W, int H, int S, int E, int Sn, int pool, int
     const double patches = std::max(0.0, 16.0 * p.S16 * 4 / 48 / 2400 * p.hpx * slicesIn * perCu - 2);
     return 0.97f * (float)(pool ? 1.6 + 1.12 * us + patches : Sn > 0 ? 2.1 + (0.73 + 0.06 * p.S16) * us + 1.8 * patches : 1.95 + 0.89 * us + 1.8 * patches);
 }
+// (An expand pair apart is a launch in three bf16 parts or in fp32: with a 1x1 layer riding along it never is one in two f16 parts.)
 extern "C" float drhip_fire_expand_us(int W, int H, int S, int E) {
     const double mpxE = 1e-6 * W * H * E;
     if (drhip_conv3x3_winograd_split_pick_variant(W, H, S, 2 * E)) return (float)(5.4 + (W & 1 ? 5.4 : 2.9) * mpxE + 0.094 * mpxE * S + 0.000009 * E * S);

@@ -87,16 +87,14 @@ void pick_winograd(dR_Conv2d_Data* c, int O) {
     if (!c->drWinoSplit) c->variant = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
 }
 
-// Operands in two f16 parts instead, as far as the shape goes.
+// Operands in two f16 parts instead, as far as the shape goes.  Not where a 1x1 sibling rides along: one weight is a filter there, and few sets of those
+// have none below 2^-12 of the largest (0 of 20 normally distributed ones of 64x256, 1 of the stored SqueezeNet's 8), so that the planner, which has to price
+// such a launch before it knows the weights, counts on the other forms.
 void pick_winograd_pair(dR_Conv2d_Data* c, int O) {
-    const int v = drhip_conv3x3_winograd_pair_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
+    const int v = c->drAbsorbed1x1 ? 0 : drhip_conv3x3_winograd_pair_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
     if (v == 0) return;
     c->variant = v;
     c->drWinoSplit = TRUE;
-}
-bool fits_pair(const dR_Conv2d_Data* c) {
-    const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
-    return drhip_winograd_pair_fits(c->weights, c->shape.s2, c->shape.s3, 9) && (!a || drhip_winograd_pair_fits(a->weights, a->shape.s2, a->shape.s3, 1));
 }
 
 size_t winograd_workspace_floats(const dR_Conv2d_Data* c, int O) {
@@ -283,8 +281,8 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         // channels first (they sit just below this node's in the concat), centre tap only.
         const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
         if (a && !a->hasVariables) { say("Conv2d Layer %d has no weights: call dR_Conv2d_setVariables first! \n", c->drAbsorbed1x1->layerID); return FALSE; }
-        if (pair_bank(c) && !fits_pair(c) && !leave_pair(net, c)) return FALSE;
         const int I = c->shape.s2, O3 = c->shape.s3, O1 = a ? a->shape.s3 : 0, O = O1 + O3;
+        if (pair_bank(c) && !drhip_winograd_pair_fits(c->weights, I, O, 9) && !leave_pair(net, c)) return FALSE;
         std::vector<float> joint;
         const float* host = c->weights;
         if (a) {

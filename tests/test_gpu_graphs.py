@@ -1100,6 +1100,28 @@ def test_refilled_weights_that_two_parts_cannot_hold(oracle, gpu, monkeypatch, W
         assert all(np.array_equal(a, b) for a, b in zip(again[0], again[2]))
 
 
+@pytest.mark.parametrize("W,H,S,E,kernel", [(56, 56, 64, 256, "Winograd F(2x2,3x3) MFMA"), (112, 112, 64, 128, "split-operand bf16 MFMA"), (33, 31, 256, 256, "split-operand bf16 MFMA")])
+def test_expand_pairs_keep_three_parts(oracle, gpu, W, H, S, E, kernel):
+    """The 3x3 layer of a pair that is one launch has the kernel that the planner prices, also with weights that two parts could hold."""
+    st = configs._Streams(85)
+    spec = [{"op": "feed", "shape": (W, H, S)}, configs._conv(st, 0, 1, S, E), configs._conv(st, 0, 3, S, E), {"op": "concat", "ins": [1, 2], "dim": 2}]
+    spec[1]["w"] = spec[1]["w"] + np.copysign(np.float32(0.01), spec[1]["w"])
+    x = np.random.default_rng(8).standard_normal((S, H, W)).astype(np.float32)
+    with dr.Environment() as env:
+        g = env.create_graph()
+        nodes = configs.build_graph(g, spec, [3])
+        assert g.lib.drhip_conv3x3_winograd_pair_pick_variant(W, H, S, 2 * E)
+        for n in (1, 2):
+            w = spec[n]["w"]
+            assert g.lib.drhip_winograd_pair_fits(w.ctypes.data_as(ctypes.c_void_p), S, E, w.shape[2] * w.shape[3])
+        dr.prepare(g)
+        assert kernel in _kernels(nodes)[1]
+        configs.feed_chw(nodes[0], x)
+        assert g.lib.dR_apply(g.ptr)
+        got = configs.fetch_chw(g)[0]
+    assert rel_err(got, oracle.run_spec(spec, {0: x})[3]) <= LAYER_TOL
+
+
 @pytest.mark.parametrize("W,H,I,O,helpers", [(33, 31, 256, 512, False), (56, 56, 256, 256, True), (48, 48, 128, 256, True)])
 def test_joined_layers_of_two_graphs_on_two_streams(lib, gpu, W, H, I, O, helpers):
     """Pieces of a split-operand layer, and panels and their helpers, wait for each other inside the launch.  Two graphs with such a layer, each on its
