@@ -22,6 +22,10 @@ def ok(lib, rc):
     ("fp32", 0x1801, 112, 112, 128, 128),       # tiers
     ("split", 0x101 | 2 << 12 | 2 << 16, 28, 28, 256, 512), ("split", 0x101 | 4 << 12 | 4 << 16, 27, 13, 256, 130), ("split", 0x100 | 2 << 12 | 2 << 16, 64, 36, 96, 70),
     ("split", 0x101 | 3 << 12 | 3 << 16, 88, 72, 256, 128),     # 39 pieces for the 32 CUs of an XCD: some wait for others that have not begun
+    # two f16 parts: quarters with two wave sets, thirds and halves with one, whole panels in front of quarters, thirds and halves, and pieces of two kinds
+    ("pair", 0x301 | 4 << 12 | 4 << 16, 27, 13, 256, 130), ("pair", 0x300 | 3 << 12 | 3 << 16, 73, 28, 400, 130), ("pair", 0x300 | 2 << 12 | 2 << 16, 64, 36, 96, 70),
+    ("pair", 0x300 | 4 << 20 | 1 << 12 | 4 << 16, 64, 36, 256, 70), ("pair", 0x300 | 4 << 20 | 1 << 12 | 3 << 16, 63, 36, 200, 70),
+    ("pair", 0x300 | 3 << 20 | 1 << 12 | 2 << 16, 64, 36, 130, 70), ("pair", 0x301 | 2 << 20 | 2 << 12 | 3 << 16, 64, 36, 130, 70),
 ])
 def test_tiles_that_come_too_late_are_gone_with_the_launch(lib, dev, monkeypatch, kind, variant, W, H, I, O, spins):
     """A workgroup that does not wait for its partners gives NaN for what is missing, and their tiles, which come later, are not
@@ -30,9 +34,10 @@ def test_tiles_that_come_too_late_are_gone_with_the_launch(lib, dev, monkeypatch
     rng = np.random.default_rng(W * I + variant)
     draw = lambda *shape: rng.standard_normal(shape).astype(np.float32)
     w, out = draw(I, O, 3, 3), dev.empty(O * H * W)
-    split = kind == "split"
-    U = dev.empty((lib.drhip_conv3x3_winograd_split_filter_floats if split else lib.drhip_conv3x3_winograd_filter_floats)(I, O))
-    ok(lib, (lib.drhip_winograd_split_filter_transform_f32 if split else lib.drhip_winograd_filter_transform_f32)(dev.put(w), U, I, O, None))
+    split = kind != "fp32"
+    named = {"fp32": "", "split": "split_", "pair": "pair_"}[kind]
+    U = dev.empty(getattr(lib, "drhip_conv3x3_winograd_%sfilter_floats" % named)(I, O))
+    ok(lib, getattr(lib, "drhip_winograd_%sfilter_transform_f32" % named)(dev.put(w), U, I, O, None))
     n = (lib.drhip_conv3x3_winograd_split_workspace_floats if split else lib.drhip_conv3x3_winograd_workspace_floats)(W, H, I, O, variant)
     assert n
     ws = dev.empty(n)
