@@ -298,7 +298,8 @@ int drhip_conv3x3_winograd_split_f32(const float* in, const float* F, const floa
  * filters' bytes.  F is then the bank of drhip_winograd_pair_filter_transform_f32 (drhip_conv3x3_winograd_pair_filter_floats(I,O)
  * floats, 16-byte aligned).  drhip_winograd_pair_fits (on the host: w is host memory, taps weights a filter, 9 or 1)
  * tells whether these weights may be held that way: finite, and none of an output channel's filters smaller than 2^-12 of its largest;
- * otherwise the three-part bank is the one to use.  Samples may be anything.  drhip_conv3x3_winograd_pair_pick_variant: 0, or the variant
+ * otherwise the three-part bank is the one to use (a filter of zeros among others: samples of its channel would set a scale that leaves the other channels' few
+ * bits).  Samples may be anything.  drhip_conv3x3_winograd_pair_pick_variant: 0, or the variant
  * for such a bank. */
 int drhip_conv3x3_winograd_pair_pick_variant(int W, int H, int I, int O);
 size_t drhip_conv3x3_winograd_pair_filter_floats(int I, int O);

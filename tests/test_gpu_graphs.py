@@ -1100,6 +1100,29 @@ def test_refilled_weights_that_two_parts_cannot_hold(oracle, gpu, monkeypatch, W
         assert all(np.array_equal(a, b) for a, b in zip(again[0], again[2]))
 
 
+@pytest.mark.parametrize("what,kernel", [("fit", "f16"), ("zero filter", None), ("tiny filter", None)])
+@pytest.mark.parametrize("W,H,I,O,other", [(56, 56, 256, 256, "Winograd F(2x2,3x3) MFMA"), (112, 112, 128, 128, "split-operand bf16 MFMA"), (33, 31, 256, 512, "split-operand bf16 MFMA")])
+def test_samples_behind_filters_of_nothing_are_no_measure(oracle, gpu, W, H, I, O, other, what, kernel):
+    """The samples of a column of tiles share a scale in the two-part kernel, which follows the largest.  Where that is of a channel whose filters are zero, or next
+    to it, the outputs are made of the others, which the scale would leave few bits: such a layer is prepared in a form that holds all of them."""
+    st = configs._Streams(87)
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, 3, I, O)]
+    x = np.random.default_rng(9).random((I, H, W), dtype=np.float32)
+    if what != "fit":
+        spec[1]["w"][7] *= np.float32(0.0 if what == "zero filter" else 2.0 ** -24)
+        x[7] *= np.float32(2.0 ** 24)
+    with dr.Environment() as env:
+        g = env.create_graph()
+        nodes = configs.build_graph(g, spec, [1])
+        dr.prepare(g)
+        assert (kernel or other) in _kernels(nodes)[0]
+        configs.feed_chw(nodes[0], x)
+        for _ in range(2):
+            assert g.lib.dR_apply(g.ptr)
+        got = configs.fetch_chw(g)[0]
+    assert rel_err(got, oracle.conv_f64(x, spec[1]["w"], spec[1]["b"], relu=True)) <= LAYER_TOL / 20
+
+
 @pytest.mark.parametrize("W,H,S,E,kernel", [(56, 56, 64, 256, "Winograd F(2x2,3x3) MFMA"), (112, 112, 64, 128, "split-operand bf16 MFMA"), (33, 31, 256, 256, "split-operand bf16 MFMA")])
 def test_expand_pairs_keep_three_parts(oracle, gpu, W, H, S, E, kernel):
     """The 3x3 layer of a pair that is one launch has the kernel that the planner prices, also with weights that two parts could hold."""
