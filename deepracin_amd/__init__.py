@@ -195,6 +195,7 @@ def load_library(path=None):
         "drhip_conv3x3_winograd_pair_filter_floats": (c_size_t, [c_int, c_int]),
         "drhip_winograd_pair_fits": (c_int, [vp, c_int, c_int, c_int]),
         "drhip_conv3x3_winograd_pair_pick_variant": (c_int, [c_int] * 4),
+        "drhip_winograd_pair_holds": (c_int, [vp, c_int, c_int, POINTER(c_int), vp]),
         "drhip_winograd_pair_filter_transform_f32": (c_int, [vp, vp, c_int, c_int, vp]),
         "drhip_conv3x3_winograd_join_timeouts": (c_int, [POINTER(ctypes.c_uint)]),
         "drhip_conv1x1_f32": (c_int, [vp, vp, vp, vp] + [c_int] * 5 + [vp]),

@@ -684,30 +684,81 @@ struct WsF16x2 {
     }
 };
 
-// scale[o]: 2^-k, where 2^k brings the largest weight of output channel o to 2^13 .. 2^14.  Transformed filters are at most 2.25 times as large, and
-// at least a quarter.
+// A bank's tail, in words: by output channel (rounded up to 32) what its sums are multiplied by; by 32 of them, how many the bank cannot hold; by
+// 16-channel chunk and output channel the bits of the largest weight of the largest filter and of the smallest.
+struct WsPairTail {
+    float* scale;
+    int *unfit, *largest, *least;
+    __host__ __device__ WsPairTail(float* tail, int nC, int nOB) : scale(tail), unfit((int*)tail + 32 * nOB), largest(unfit + nOB), least(largest + 32 * nC * nOB) {}
+    static __host__ __device__ size_t words(int nC, int nOB) { return (size_t)nOB * (33 + 64 * (size_t)nC); }
+};
+// Magnitudes by their bits, which are in the same order and put NaN last.  Where the largest weight of an output channel is in range and no filter's is below
+// 2^-12 of it (why: drhip_winograd_pair_fits), two parts can hold the channel; one without any weight is exact.
+__host__ __device__ inline bool ws_pair_holds(int largest, int least) {
+    constexpr int low = (127 - 100) << 23, high = (127 + 100) << 23;        // the bits of 2^-100 and 2^100
+    return largest == 0 || (largest >= low && largest <= high && least + (12 << 23) >= largest);
+}
+
+// On the device, where the weights are for the next kernel anyway: a pass over them on the host, 0.28 ns each, made dR_prepare of VGG16's convolutions over
+// 640x480 8.4 ms (5.9 now, 5.4 with three parts) and that of three layers 56x56 128->256 0.99 (0.74, 0.76).
 __global__ void __launch_bounds__(256)
-wino_pair_scale_kernel(const float* __restrict__ w, float* __restrict__ scale, int I, int O) {
-    __shared__ float part[4];
-    const int o = blockIdx.x;
-    float m = 0.0f;
+wino_pair_range_kernel(const float* __restrict__ w, int* __restrict__ largest, int* __restrict__ least, int I, int O, int outputs) {
+    __shared__ int part[2][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, o = blockIdx.x * 64 + lane, chunk = blockIdx.y;
+    int most = 0, fewest = 0x7fffffff;
     if (o < O)
-        for (int k = threadIdx.x; k < 9 * I; k += 256) m = fmaxf(m, fabsf(w[((size_t)(k / 9) * O + o) * 9 + k % 9]));
-    for (int k = 1; k < 64; k *= 2) m = fmaxf(m, __shfl_xor(m, k));
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+        for (int c = 16 * chunk + wave; c < min(16 * chunk + 16, I); c += 4) {
+            const float* f = w + ((size_t)c * O + o) * 9;
+            int m = 0;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) m = max(m, (int)(__float_as_uint(f[k]) & 0x7fffffffu));
+            most = max(most, m);
+            fewest = min(fewest, m);
+        }
+    part[0][wave][lane] = most;
+    part[1][wave][lane] = fewest;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        m = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-        const int e = (int)(__float_as_uint(m) >> 23) - 127;
-        scale[o] = m == 0.0f ? 1.0f : __uint_as_float((unsigned)(127 + max(min(e - 13, 114), -126)) << 23);
+    if (wave == 0 && o < outputs) {
+        largest[(size_t)chunk * outputs + o] = max(max(part[0][0][lane], part[0][1][lane]), max(part[0][2][lane], part[0][3][lane]));
+        least[(size_t)chunk * outputs + o] = min(min(part[1][0][lane], part[1][1][lane]), min(part[1][2][lane], part[1][3][lane]));
     }
 }
 
+// scale[o]: 2^-k, where 2^k brings the largest weight of output channel o to 2^13 .. 2^14.  Transformed filters are at most 2.25 times as large, and
+// at least a quarter.
 __global__ void __launch_bounds__(256)
-wino_pair_filter_kernel(const float* __restrict__ w, unsigned short* __restrict__ U, const float* __restrict__ scale, int I, int O, int nC, int nOB) {
+wino_pair_filter_kernel(const float* __restrict__ w, unsigned short* __restrict__ U, float* tail, int I, int O, int nC, int nOB) {
+    const WsPairTail t(tail, nC, nOB);
+    __shared__ int range[2][8][32];
+    __shared__ float upOf[32];
     const int row = threadIdx.x >> 6, lane = threadIdx.x & 63, ob = blockIdx.x % nOB, chunk = blockIdx.x / nOB;
+    {
+        const int ol = threadIdx.x & 31, eighth = threadIdx.x >> 5;
+        int most = 0, fewest = 0x7fffffff;
+        for (int c = eighth; c < nC; c += 8) {
+            most = max(most, t.largest[(size_t)c * 32 * nOB + ob * 32 + ol]);
+            fewest = min(fewest, t.least[(size_t)c * 32 * nOB + ob * 32 + ol]);
+        }
+        range[0][eighth][ol] = most;
+        range[1][eighth][ol] = fewest;
+    }
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        const int ol = threadIdx.x;
+        int most = 0, fewest = 0x7fffffff;
+        for (int k = 0; k < 8; ++k) { most = max(most, range[0][k][ol]); fewest = min(fewest, range[1][k][ol]); }
+        const int e = (most >> 23) - 127;
+        const float scale = most == 0 ? 1.0f : __uint_as_float((unsigned)(127 + max(min(e - 13, 114), -126)) << 23);
+        upOf[ol] = __uint_as_float((254u << 23) - __float_as_uint(scale));
+        if (chunk == 0) {
+            t.scale[ob * 32 + ol] = scale;
+            const unsigned long long unfit = __builtin_amdgcn_ballot_w64(!ws_pair_holds(most, fewest));
+            if (ol == 0) t.unfit[ob] = __builtin_popcountll(unfit);
+        }
+    }
+    __syncthreads();
     const int c0 = chunk * 16 + 8 * (lane >> 5), o = ob * 32 + (lane & 31);
-    const float up = __uint_as_float((254u << 23) - __float_as_uint(scale[o]));
+    const float up = upOf[lane & 31];
     float u[8][4];                                  // the row's four positions of eight channels
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -1162,48 +1213,7 @@ extern "C" int drhip_winograd_split_filter_transform_f32(const float* w, float* 
 }
 
 extern "C" size_t drhip_conv3x3_winograd_pair_filter_floats(int I, int O) {
-    return I <= 0 || O <= 0 ? 0 : (size_t)ceil_div(O, 32) * ((size_t)ceil_div(I, kWsKC) * 8192 + 32);
-}
-
-// Magnitudes by their bits, which are in the same order and put NaN last: of every output channel its smallest filter's and its largest's
-// largest weight.  Four filters at a time (0.64 ns a weight one at a time, 0.28 now).
-typedef int i32x4h __attribute__((ext_vector_type(4)));
-static inline i32x4h larger_of(i32x4h a, i32x4h b) { return a > b ? a : b; }
-static inline i32x4h largest_of_nine(const float* w) {     // in some order: three loads of four, one weight twice in them
-    i32x4h v[3];
-    memcpy(&v[0], w, 16);
-    memcpy(&v[1], w + 4, 16);
-    memcpy(&v[2], w + 5, 16);
-    return larger_of(v[0] & 0x7fffffff, larger_of(v[1] & 0x7fffffff, v[2] & 0x7fffffff));
-}
-
-template <int TAPS>
-static void filter_range(const float* w, int I, int O, int* least, int* largest) {
-    for (int c = 0; c < I; ++c) {
-        int o = 0;
-        if (TAPS == 9)
-            for (; o + 4 <= O; o += 4, w += 36) {
-                const i32x4h m0 = largest_of_nine(w), m1 = largest_of_nine(w + 9), m2 = largest_of_nine(w + 18), m3 = largest_of_nine(w + 27);
-                const i32x4h even = larger_of(__builtin_shufflevector(m0, m1, 0, 4, 1, 5), __builtin_shufflevector(m0, m1, 2, 6, 3, 7)),
-                             odd = larger_of(__builtin_shufflevector(m2, m3, 0, 4, 1, 5), __builtin_shufflevector(m2, m3, 2, 6, 3, 7)),
-                             most = larger_of(__builtin_shufflevector(even, odd, 0, 1, 4, 5), __builtin_shufflevector(even, odd, 2, 3, 6, 7));
-                i32x4h l, g;
-                memcpy(&l, least + o, 16);
-                memcpy(&g, largest + o, 16);
-                l = most < l ? most : l;
-                g = larger_of(most, g);
-                memcpy(least + o, &l, 16);
-                memcpy(largest + o, &g, 16);
-            }
-        for (; o < O; ++o, w += TAPS) {
-            int bits[TAPS], most = 0;
-            memcpy(bits, w, sizeof bits);
-#pragma unroll
-            for (int k = 0; k < TAPS; ++k) most = std::max(most, bits[k] & 0x7fffffff);
-            least[o] = std::min(least[o], most);
-            largest[o] = std::max(largest[o], most);
-        }
-    }
+    return I <= 0 || O <= 0 ? 0 : (size_t)ceil_div(O, 32) * ceil_div(I, kWsKC) * 8192 + WsPairTail::words(ceil_div(I, kWsKC), ceil_div(O, 32));
 }
 
 // A filter next to the largest of its output channel.  This is about samples: those of a column of tiles share a scale that follows the largest, so each
@@ -1214,10 +1224,19 @@ static void filter_range(const float* w, int I, int O, int* least, int* largest)
 extern "C" int drhip_winograd_pair_fits(const float* w, int I, int O, int taps) {
     if (!w || I <= 0 || O <= 0 || (taps != 1 && taps != 9)) return 0;
     std::vector<int> least((size_t)O, 0x7fffffff), largest((size_t)O, 0);
-    (taps == 1 ? filter_range<1> : filter_range<9>)(w, I, O, least.data(), largest.data());
-    auto power = [](int e) { return (127 + e) << 23; };         // the bits of 2^e
+    for (int c = 0; c < I; ++c)
+        for (int o = 0; o < O; ++o, w += taps) {
+            int most = 0;
+            for (int k = 0; k < taps; ++k) {
+                int bits;
+                memcpy(&bits, w + k, sizeof bits);
+                most = std::max(most, bits & 0x7fffffff);
+            }
+            least[o] = std::min(least[o], most);
+            largest[o] = std::max(largest[o], most);
+        }
     for (int o = 0; o < O; ++o)
-        if (largest[o] != 0 && !(largest[o] >= power(-100) && largest[o] <= power(100) && least[o] + (12 << 23) >= largest[o])) return 0;
+        if (!ws_pair_holds(largest[o], least[o])) return 0;
     return 1;
 }
 
@@ -1225,11 +1244,22 @@ extern "C" int drhip_winograd_pair_filter_transform_f32(const float* w, float* U
     DRHIP_REQUIRE(w && U && I > 0 && O > 0, "drhip_winograd_pair_filter_transform_f32: bad arguments");
     const int nC = ceil_div(I, kWsKC), nOB = ceil_div(O, 32);
     DRHIP_REQUIRE((long long)nC * nOB * 12288 * 4 < (1ll << 31), "drhip_winograd_pair_filter_transform_f32: %dx%d filters are too many", I, O);
-    float* scale = U + (size_t)nC * nOB * 8192;
-    launch(wino_pair_scale_kernel, dim3(32 * nOB), dim3(256), 0, as_stream(stream), w, scale, I, O);
-    if (int rc = launched("wino_pair_scale_kernel")) return rc;
-    launch(wino_pair_filter_kernel, dim3((unsigned)(nC * nOB)), dim3(256), 0, as_stream(stream), w, (unsigned short*)U, scale, I, O, nC, nOB);
+    float* tail = U + (size_t)nC * nOB * 8192;
+    const WsPairTail t(tail, nC, nOB);
+    launch(wino_pair_range_kernel, dim3((32 * nOB + 63) / 64, nC), dim3(256), 0, as_stream(stream), w, t.largest, t.least, I, O, 32 * nOB);
+    if (int rc = launched("wino_pair_range_kernel")) return rc;
+    launch(wino_pair_filter_kernel, dim3((unsigned)(nC * nOB)), dim3(256), 0, as_stream(stream), w, (unsigned short*)U, tail, I, O, nC, nOB);
     return launched("wino_pair_filter_kernel");
+}
+
+extern "C" int drhip_winograd_pair_holds(const float* U, int I, int O, int* holds, void* stream) {
+    DRHIP_REQUIRE(U && holds && I > 0 && O > 0, "drhip_winograd_pair_holds: bad arguments");
+    const int nC = ceil_div(I, kWsKC), nOB = ceil_div(O, 32);
+    std::vector<int> unfit((size_t)nOB);
+    const WsPairTail t((float*)U + (size_t)nC * nOB * 8192, nC, nOB);
+    if (int rc = drhip_download(unfit.data(), t.unfit, 0, unfit.size() * sizeof(int), stream)) return rc;
+    *holds = std::all_of(unfit.begin(), unfit.end(), [](int n) { return n == 0; });
+    return DRHIP_OK;
 }
 
 extern "C" int drhip_conv3x3_winograd_split_f32(const float* in, const float* U, const float* bias, float* out, int W, int H, int I, int O, int flags, int variant, float* workspace, void* stream) {

@@ -282,7 +282,6 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         const dR_Conv2d_Data* a = c->drAbsorbed1x1 ? conv_of(c->drAbsorbed1x1) : NULL;
         if (a && !a->hasVariables) { say("Conv2d Layer %d has no weights: call dR_Conv2d_setVariables first! \n", c->drAbsorbed1x1->layerID); return FALSE; }
         const int I = c->shape.s2, O3 = c->shape.s3, O1 = a ? a->shape.s3 : 0, O = O1 + O3;
-        if (pair_bank(c) && !drhip_winograd_pair_fits(c->weights, I, O, 9) && !leave_pair(net, c)) return FALSE;
         std::vector<float> joint;
         const float* host = c->weights;
         if (a) {
@@ -297,9 +296,17 @@ gboolean conv_fill(dR_Graph* net, dR_Node* node) {
         cl_mem raw = NULL;
         if (!dR_createFloatBuffer(net, &raw, I * O * 9, CL_MEM_READ_ONLY)) return FALSE;
         ok = dR_uploadArray(net, (gchar*)"", (void*)host, 0, rawBytes, raw);
-        if (ok) ok = !device_failed(net, (pair_bank(c) ? drhip_winograd_pair_filter_transform_f32 : c->drWinoSplit ? drhip_winograd_split_filter_transform_f32
-                                                       : drhip_winograd_filter_transform_f32)((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net)),
-                                    "winograd filter transform");
+        auto transform = [&]() {
+            return !device_failed(net, (pair_bank(c) ? drhip_winograd_pair_filter_transform_f32 : c->drWinoSplit ? drhip_winograd_split_filter_transform_f32
+                                                     : drhip_winograd_filter_transform_f32)((const float*)raw, (float*)c->weightsBuf, I, O, stream_of(net)),
+                                  "winograd filter transform");
+        };
+        if (ok) ok = transform();
+        if (ok && pair_bank(c)) {
+            int holds = 0;
+            ok = !device_failed(net, drhip_winograd_pair_holds((const float*)c->weightsBuf, I, O, &holds, stream_of(net)), "winograd filter transform (sync)");
+            if (ok && !holds) ok = leave_pair(net, c) && transform();
+        }
         if (ok) ok = !device_failed(net, drhip_stream_sync(stream_of(net)), "winograd filter transform (sync)");
         dR_clMemoryBufferCleanup(net, raw);
         net->clConfig->memConsumptionGPU -= (glong)rawBytes;

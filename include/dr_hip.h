@@ -296,15 +296,17 @@ int drhip_conv3x3_winograd_split_f32(const float* in, const float* F, const floa
                                      int W, int H, int I, int O, int relu, int variant, float* workspace, void* stream);
 /* Variant bit 0x200: operands in two f16 parts instead of three bf16 ones, half of the matrix instructions and two thirds of the
  * filters' bytes.  F is then the bank of drhip_winograd_pair_filter_transform_f32 (drhip_conv3x3_winograd_pair_filter_floats(I,O)
- * floats, 16-byte aligned).  drhip_winograd_pair_fits (on the host: w is host memory, taps weights a filter, 9 or 1)
- * tells whether these weights may be held that way: finite, and none of an output channel's filters smaller than 2^-12 of its largest;
- * otherwise the three-part bank is the one to use (a filter of zeros among others: samples of its channel would set a scale that leaves the other channels' few
- * bits).  Samples may be anything.  drhip_conv3x3_winograd_pair_pick_variant: 0, or the variant
- * for such a bank. */
+ * floats, 16-byte aligned).  drhip_winograd_pair_fits (on the host: w is host memory, taps weights a filter, 9 or 1) tells whether these
+ * weights may be held that way: finite, and none of an output channel's filters smaller than 2^-12 of its largest; otherwise the
+ * three-part bank is the one to use (a filter of zeros among others: samples of its channel would set a scale that leaves the other
+ * channels' few bits).  drhip_winograd_pair_holds: the same of a bank that has been filled, told by the device, which looks at the weights
+ * when it lays them out; waits for the stream.  Samples may be anything.  drhip_conv3x3_winograd_pair_pick_variant: 0, or the variant for
+ * such a bank. */
 int drhip_conv3x3_winograd_pair_pick_variant(int W, int H, int I, int O);
 size_t drhip_conv3x3_winograd_pair_filter_floats(int I, int O);
 int drhip_winograd_pair_fits(const float* w /* [I][O][taps] */, int I, int O, int taps);
 int drhip_winograd_pair_filter_transform_f32(const float* w /* [I][O][3][3] */, float* F, int I, int O, void* stream);
+int drhip_winograd_pair_holds(const float* F, int I, int O, int* holds, void* stream);
 
 /* 1x1 convolution as an fp32 MFMA GEMM out[O][P] = w[O x I] . in[I][P], P = H*W; w is the
  * original [I][O] array (no transpose needed).  Replaces kernel `conv2d1x1`, its launch and the

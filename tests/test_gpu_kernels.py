@@ -639,6 +639,40 @@ def test_winograd_stores_pairs_of_tiles(lib, dev, oracle, variant, W, H, I, O):
             assert np.array_equal(outs[0], outs[2], equal_nan=True) and np.array_equal(outs[1], outs[2], equal_nan=True)
 
 
+@pytest.mark.parametrize("I,O", [(64, 32), (65, 33), (200, 300), (17, 64), (1, 1), (257, 97)])
+def test_a_pair_bank_knows_whether_it_holds_its_weights(lib, dev, I, O):
+    """The device tells it of all weights as the host does: at either end of the channels, in chunks that end early, for the first and the last tap, whatever the sign,
+    and has the scales that the largest weights ask for."""
+    def both(w):
+        F, holds = dev.put(np.full(lib.drhip_conv3x3_winograd_pair_filter_floats(I, O), np.nan, np.float32)), ctypes.c_int(-1)
+        ok(lib, lib.drhip_winograd_pair_filter_transform_f32(dev.put(w), F, I, O, None))
+        ok(lib, lib.drhip_winograd_pair_holds(F, I, O, ctypes.byref(holds), None))
+        assert holds.value == lib.drhip_winograd_pair_fits(np.ascontiguousarray(w).ctypes.data_as(ctypes.c_void_p), I, O, 9)
+        at = -(-I // 16) * -(-O // 32) * 8192
+        scale = dev.get(F, (at + -(-O // 32) * 32,))[at:at + O]
+        if np.isfinite(w).all() and (np.abs(w).max(axis=(0, 2, 3)) > 0).all():
+            assert np.array_equal(scale, np.exp2(np.floor(np.log2(np.abs(w).max(axis=(0, 2, 3)))) - 13).astype(np.float32))
+        return holds.value
+
+    w0 = own(I, O, 3, 3)
+    w0[:, :, 1, 1] = np.copysign(np.maximum(np.abs(w0[:, :, 1, 1]), 0.01), w0[:, :, 1, 1])
+    assert both(w0) == 1
+    for c in {0, I - 1, I // 2}:
+        for o in {0, O - 1, O // 2}:
+            for value, alone in ((np.inf, 0), (-np.nan, 0), (2.0 ** 101, 0)):
+                w = w0.copy()
+                w[c, o, 2 * (c & 1), 2 * (o & 1)] = value
+                assert both(w) == alone
+            for value in (0.0, 2.0 ** -16):
+                w = w0.copy()
+                w[c, o] = value
+                assert both(w) == (I == 1)          # (the only filter of its output channel is the largest)
+    assert both(w0 * np.float32(2.0 ** -99 * 2.0 ** -10)) == 0
+    w = w0.copy()
+    w[:, O // 2] = 0
+    assert both(w) == 1
+
+
 @pytest.mark.parametrize("operand,power", [(o, p) for o in ("samples", "weights") for p in (-146, -136, -126, -112, -60, 60, 100, 116, 124)])
 def test_split_kernels_hold_operands_of_any_size(lib, dev, oracle, operand, power):
     """Samples and weights down to the smallest fp32 number keep all their bits, and what is too large for three parts once it is scaled, the
