@@ -1121,7 +1121,10 @@ using namespace drhip;
 //   * pieces 7.8, 2 more per pair of chunks and 0.22 per MB of filters (56x56 256->256 20.3 / 16.4, 28x28 512->512 23.2 / 18.9, 61x75 320->140 23.3 / 19.8,
 //     62x41 376->106 19.0 / 14.1, 51x41 191->384 18.0 / 15.5; 56x56 128->256 12.2 / 11.7, 28x28 256->512 14.0 / 14.4, 84x68 224->64 12.0 / 12.2 and fewer panels
 //     stay there).  Where that kernel has helpers it takes 0.56 per stage that its own workgroups keep and 3.6 (39x152 198->68 13.6 / 15.2, 18x74 230->466
-//     16.0 / 17.8 stay there).  300 drawn shapes of up to 16 panels: 0.90 to 1.003 times the fp32 kernel's time but for one (21x148 232->79, 12.7 / 14.2).
+//     16.0 / 17.8 stay there).  300 drawn shapes of up to 16 panels: 0.90 to 1.003 times the fp32 kernel's time but for one, on a narrow map.
+//     Those (six loads a step, each of more pieces of rows) take 6.5 around the pairs, 0.1 more for each workgroup of an XCD and 0.09 per MB, and the fp32 kernel's
+//     time is taken for 0.4 less, or with a second launch for 1.5 more.  Of 20000 drawn shapes 32 stay in fp32 for it (21x148 232->79 12.9 / 14.2, 12x359 236->48
+//     12.1 / 13.8, 17x236 237->55 12.0 / 13.5, 12x433 196->134 17.9 / 19.9; of the 32 half within 4 % of even, three 6 to 10 % slower in fp32).
 //   * two thirds of a panel per CU at most, and fp32 panels for more than half of a round: from 19 chunks on all in thirds, with one wave set (73x28 400->476
 //     32 / 28, 52x56 440->330 35.3 / 30.7; two wave sets unsplit 30.0 and 33.5; 80x60 512->256 33.6 against 35.8, 256->256 23.5 against 21.0).
 //   * up to one and a half panels per CU: with one wave set, whole panels on seven CUs of eight and all others in halves, or, where there is room for
@@ -1154,9 +1157,11 @@ static int ws_pick(int W, int H, int I, int O, bool pair) {
         auto fp32 = [&](int lg) { return 0.56 * ceil_div(2 * nC, 1 << lg) * ceil_div(panels32 << lg, cus) + (lg > 0 ? 4.5 : 3); };
         const int pairs = ceil_div(ceil_div(nC, S), 2), picked = drhip_conv3x3_winograd_pick_variant(W, H, I, O);
         const double taken = fp32(picked >> 4 & 15);
-        const double helped = picked & 0x2000 ? 0.56 * (ceil_div(I, 8) - wino_donated(W, H, I, O)) + 3.6 : taken;
+        const double helped = picked & 0x2000 ? 0.56 * (ceil_div(I, 8) - wino_donated(W, H, I, O)) + 3.6 : taken, filterMB = 64e-6 * I * O;
+        const double summed = (picked & 0xf00) == 0x400 && picked & 0xf0 ? 1.9 : 0;        // (two wave sets a panel, and a second launch)
+        const bool gains = 2.0 * pairs + 7.8 + 0.22 * filterMB < 0.93 * helped && (wide || 2.0 * pairs + 6.9 + 0.105 * n * S + 0.09 * filterMB < helped + summed);
         if (halvings >= 0 &&                            // (layers of its 16-tile form are too small)
-            (2.75 * pairs + 10.6 < 0.93 * std::max(fp32(halvings), taken) || (pair && 2.0 * pairs + 7.8 + 0.22e-6 * 64 * I * O < 0.93 * helped)))
+            (2.75 * pairs + 10.6 < 0.93 * std::max(fp32(halvings), taken) || (pair && gains)))
             if (const int v = split(0x101, 0, S, S)) return v;
     }
     if (!wide) return 0;

@@ -881,6 +881,7 @@ def test_layers_stay_in_pieces_for_their_exactness(lib, W, H, I, O, pieces):
 
 @pytest.mark.parametrize("W,H,I,O,variant", [
     (56, 56, 256, 256, 0x22301), (28, 28, 512, 512, 0x44301), (62, 41, 376, 106, 0x44301), (47, 61, 192, 192, 0x33301),     # pieces where they are the faster ones
+    (21, 148, 232, 79, 0), (12, 359, 236, 48, 0), (12, 75, 304, 304, 0), (22, 107, 380, 281, 0x22301), (25, 32, 434, 296, 0x44301), (23, 46, 453, 472, 0x33301),      # narrow maps
     (56, 56, 128, 256, 0), (28, 28, 256, 512, 0), (84, 68, 224, 64, 0), (14, 14, 512, 512, 0), (45, 60, 480, 64, 0),
     (112, 112, 64, 128, 0x300), (112, 112, 127, 128, 0x301), (112, 112, 112, 128, 0x300), (112, 112, 63, 128, 0),           # one round that fills more than half of the CUs
     (73, 28, 128, 476, 0), (34, 159, 69, 141, 0), (40, 40, 146, 294, 0), (39, 152, 198, 68, 0),                             # one round or helpers of the fp32 kernel
