@@ -1074,7 +1074,7 @@ static bool ws_plan(int W, int H, int I, int O, int variant, WsPlan* p) {
 
 template <int KW, int WC, bool TURNS, bool PAIR>
 static int launch_ws(const float* in, const unsigned short* U, const float* bias, float* out, float* ws, const WsPlan& p, hipStream_t st) {
-    constexpr auto kernel = PAIR ? winograd_f23_pair_kernel<KW, WC, TURNS> : winograd_f23_split_kernel<KW, WC, TURNS>;
+    constexpr auto kernel = [] { if constexpr (PAIR) return winograd_f23_pair_kernel<KW, WC, TURNS>; else return winograd_f23_split_kernel<KW, WC, TURNS>; }();
     static std::atomic<unsigned long long> asked{0};
     if (int rc = allow_lds((const void*)kernel, p.lds, asked)) return rc;
     launch(kernel, dim3(p.perXcd * kXcds), dim3(256 * KW), p.lds, st, in, U, bias, out, p.s, ws);

@@ -761,10 +761,21 @@ def pair_kernel_code(tmp_path_factory):
             kernels[name] = []
         elif name and line.strip().startswith(".section"):
             name = None
+        elif line.strip().startswith(".amdhsa_kernel"):
+            described = line.split()[1]
+        elif ".amdhsa_private_segment_fixed_size" in line and described in kernels:
+            kernels[described].append(line.strip())
         elif name:
             kernels[name].append(line.strip())
-    assert len(kernels) == 6
+    assert len(kernels) == 5                # (narrow maps always take turns)
     return kernels
+
+
+def test_pair_kernel_keeps_nothing_in_scratch(pair_kernel_code):
+    """A kernel that has scratch starts about 1 us later."""
+    for name, lines in pair_kernel_code.items():
+        assert not [l for l in lines if l.startswith("scratch_")], name
+        assert ".amdhsa_private_segment_fixed_size 0" in lines, name
 
 
 def test_pair_kernel_waits_for_its_samples_and_leaves_m0(pair_kernel_code):
