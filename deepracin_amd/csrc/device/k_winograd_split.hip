@@ -835,7 +835,9 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
     // ---- operands --------------------------------------------------------------------------------------------------
     // A column of tiles (a lane and the one 32 on) has its samples multiplied by a power of two of its own, `scale`, so that the largest that the wave
     // has met is below 2^14 once two rows of the window are combined, and was 2^11 or more when the scale was chosen.  A step that brings a larger one
-    // lowers the scale, and what has been summed up with it, before its products begin.  As long as all samples are zero any scale will do.
+    // lowers the scale, and what has been summed up with it, before its products begin.  As long as all samples are zero any scale will do.  A sample that the
+    // scale takes beyond fp32 (2^64 behind nothing but zeros, 2^114 or more times as large as the ones in front of it) becomes an infinity, and its tile is worked out
+    // again at the end.
     const int rowA = wave, rowB = wave < 2 ? 2 : 1;
     const float sgn = wave == 1 ? 1.0f : -1.0f;
     const int lr = fast_div(l32 + off0, tilesXd), tx = l32 + off0 - lr * s.tilesX;
@@ -897,15 +899,14 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
         const float largest = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
         const int e = (int)(__float_as_uint(largest) >> 23) - 127, has = (int)(__float_as_uint(k[1]) >> 23) - 127;
         const bool lower = (largest >= kLimit || (largest != 0.0f && __builtin_amdgcn_inverse_ballot_w64(noneYet))) && e < 128;    // (an infinity stays one whatever the scale)
-        const int by = lower ? min(11 - e, 126 - has) : 0, by2 = sums ? by / 2 : by;       // (in two factors: it goes down to -240.  The first one does not)
+        const int by = lower ? min(11 - e, 126 - has) : 0;         // (-116 to 126: one factor)
         // Samples that no scale makes large enough, fp32 denormals, are left to the pass over what did not come out finite.
-        const float f1 = e + by < 1 && lower ? __builtin_nanf("") : __uint_as_float((unsigned)(127 + by2) << 23), f2 = __uint_as_float((unsigned)(127 + by - by2) << 23);
-        auto times = [&](float x) { return sums ? x * f1 * f2 : x * f1; };
+        const float factor = e + by < 1 && lower ? __builtin_nanf("") : __uint_as_float((unsigned)(127 + by) << 23);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            k[c] = times(k[c]);
+            k[c] *= factor;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) mm[j][c] = times(mm[j][c]);
+            for (int j = 0; j < 8; ++j) mm[j][c] *= factor;
         }
         noneYet &= ~__builtin_amdgcn_ballot_w64(lower);
         if (sums)
@@ -914,7 +915,7 @@ winograd_f23_pair_kernel(const float* __restrict__ in, const unsigned short* __r
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[x][nt][r] = times(acc[x][nt][r]);
+                    for (int r = 0; r < 16; ++r) acc[x][nt][r] *= factor;
 #pragma unroll
         for (int t = 0; t < 12; ++t) split_tick(0, t);
     };

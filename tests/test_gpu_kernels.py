@@ -566,10 +566,10 @@ def test_winograd_pair_is_as_exact_as_three_parts(lib, dev, oracle, W, H, I, O):
 
 
 @pytest.mark.parametrize("variant", [0x100, 0x101, 0x101 | SPLIT_HALVES])
-@pytest.mark.parametrize("kind", ["rising", "late", "dark", "tiny", "denormal", "huge", "weights", "zero"])
+@pytest.mark.parametrize("kind", ["rising", "late", "leap", "late leap", "dark", "tiny", "denormal", "huge", "weights", "zero"])
 def test_winograd_pair_scales(lib, dev, oracle, kind, variant):
     """Every column of tiles has a scale of its own that follows its largest sample: channels that get larger from step to step, that are zero at first,
-    maps of which one side is 2^-30 of the other, samples of any size, output channels of any size."""
+    or that leap beyond what the scale has room for, maps of which one side is 2^-30 of the other, samples of any size, output channels of any size."""
     W, H, I, O = 70, 6, 100, 40
     x, w = own(I, H, W), own(I, O, 3, 3, scale=0.1)
     if kind == "rising":                    # (weights that make up for it: what is lost in a channel would show)
@@ -579,6 +579,9 @@ def test_winograd_pair_scales(lib, dev, oracle, kind, variant):
         x[:40] = 0
         x[40:90, :, 30:] = 0
         x[40] *= np.float32(2.0 ** -40)
+    elif kind in ("leap", "late leap"):     # from one step to the next by more than the scale leaves room for
+        x[:40] *= np.float32(2.0 ** -70 if kind == "leap" else 0.0)
+        x[40:] *= np.float32(2.0 ** 70)
     elif kind == "dark":
         x[:, :, 35:] *= np.float32(2.0 ** -30)
     elif kind in ("tiny", "denormal", "huge"):
