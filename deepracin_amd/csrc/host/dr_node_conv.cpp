@@ -89,9 +89,10 @@ void pick_winograd(dR_Conv2d_Data* c, int O) {
 
 // Operands in two f16 parts instead, as far as the shape goes.  Not where a 1x1 sibling rides along: one weight is a filter there, and few sets of those
 // have none below 2^-12 of the largest (0 of 20 normally distributed ones of 64x256, 1 of the stored SqueezeNet's 8), so that the planner, which has to price
-// such a launch before it knows the weights, counts on the other forms.
+// such a launch before it knows the weights, counts on the other forms.  (DR_WINO_PAIR=0: nowhere; three parts or fp32 instead, which hold all bits of an operand.)
 void pick_winograd_pair(dR_Conv2d_Data* c, int O) {
-    const int v = c->drAbsorbed1x1 ? 0 : drhip_conv3x3_winograd_pair_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
+    const char* env = getenv("DR_WINO_PAIR");
+    const int v = c->drAbsorbed1x1 || (env && strcmp(env, "0") == 0) ? 0 : drhip_conv3x3_winograd_pair_pick_variant(c->ishape.s0, c->ishape.s1, c->shape.s2, O);
     if (v == 0) return;
     c->variant = v;
     c->drWinoSplit = TRUE;

@@ -1123,6 +1123,28 @@ def test_samples_behind_filters_of_nothing_are_no_measure(oracle, gpu, W, H, I, 
     assert rel_err(got, oracle.conv_f64(x, spec[1]["w"], spec[1]["b"], relu=True)) <= LAYER_TOL / 20
 
 
+@pytest.mark.parametrize("W,H,I,O,other", [(56, 56, 256, 256, "Winograd F(2x2,3x3) MFMA"), (33, 31, 256, 512, "split-operand bf16 MFMA")])
+def test_two_parts_can_be_declined(oracle, gpu, monkeypatch, W, H, I, O, other):
+    """DR_WINO_PAIR=0 in front of dR_prepare: the forms that hold all bits of an operand.  A flat map under one box filter shows them: three parts are exact to
+    2^-22 there."""
+    st = configs._Streams(89)
+    spec = [{"op": "feed", "shape": (W, H, I)}, configs._conv(st, 0, 3, I, O, relu=False, bias=False)]
+    x = np.full((I, H, W), 0.7310586, np.float32)
+    spec[1]["w"][:] = np.float32(1 / 9)
+    want = oracle.conv_f64(x, spec[1]["w"])
+    for env_var, kernel in (("0", other), ("1", "f16"), (None, "f16")):
+        monkeypatch.delenv("DR_WINO_PAIR", raising=False) if env_var is None else monkeypatch.setenv("DR_WINO_PAIR", env_var)
+        with dr.Environment() as env:
+            g = env.create_graph()
+            nodes = configs.build_graph(g, spec, [1])
+            dr.prepare(g)
+            assert kernel in _kernels(nodes)[0]
+            configs.feed_chw(nodes[0], x)
+            assert g.lib.dR_apply(g.ptr)
+            got = configs.fetch_chw(g)[0]
+        assert rel_err(got, want) <= LAYER_TOL / 20 and ("bf16" not in kernel or rel_err(got, want) <= 2.0 ** -21)
+
+
 @pytest.mark.parametrize("W,H,S,E,kernel", [(56, 56, 64, 256, "Winograd F(2x2,3x3) MFMA"), (112, 112, 64, 128, "split-operand bf16 MFMA"), (33, 31, 256, 256, "split-operand bf16 MFMA")])
 def test_expand_pairs_keep_three_parts(oracle, gpu, W, H, S, E, kernel):
     """The 3x3 layer of a pair that is one launch has the kernel that the planner prices, also with weights that two parts could hold."""
