@@ -111,13 +111,13 @@ def winograd_issued_flops(lib, W, H, I, O):
     the variant the scheduler picks (tile blocks of 32 or 16, 8 input channels per stage, 32/64/128 or 16/32/64
     output channels per workgroup); drhip_conv3x3_winograd_f32 decides the same way.  With it the peak of the matrix cores it
     runs on and the kernel's name: large layers take a split-operand kernel, six bf16 or three f16 products (32 tiles x 16 channels x
-    64 channels) for each fp32 one (random weights fit two f16 parts)."""
+    64 channels) for each fp32 one (random weights fit two f16 parts, which DR_WINO_PAIR=0 declines)."""
     v = lib.drhip_conv3x3_winograd_pick_variant(W, H, I, O)
     tb = 16 if v & 0x100 else 32
     ob = tb * {1: 1, 2: 2, 3: 4}[v & 0xf]
     tiles = ((W + 1) // 2) * ((H + 1) // 2)
     pad = lambda n, m: -(-n // m) * m
-    pair = lib.drhip_conv3x3_winograd_pair_pick_variant(W, H, I, O)
+    pair = 0 if os.environ.get("DR_WINO_PAIR") == "0" else lib.drhip_conv3x3_winograd_pair_pick_variant(W, H, I, O)
     if pair or lib.drhip_conv3x3_winograd_split_pick_variant(W, H, I, O):
         return (3 if pair else 6) * 2 * 16 * pad(tiles, 32) * pad(I, 16) * pad(O, 64), PEAK_MFMA_BF16_TFLOPS, "winograd_f23_%s_kernel" % ("pair" if pair else "split")
     # (an image layer -- at most 4 input channels, 32-tile blocks, unsplit, four waves -- runs its one stage without

@@ -1,6 +1,6 @@
 // fp32 products on the f16 matrix cores, at the accuracy of an fp32 kernel.
 //
-// hi = f16(x), lo = f16(x - hi), both rounded to nearest: 2 x 11 significant bits and the sign of lo hold 22 to 24 bits of x, all of them
+// hi = f16(x), lo = f16(x - hi), both rounded to nearest: 2 x 11 significant bits and the sign of lo hold 23 to 24 bits of x, all of them
 // for three numbers in four and all but the last for the fourth.  A product is the sum of hi*hi, hi*lo and lo*hi; lo*lo, up to 2^-22 of it, is left out.  That is
 // three matrix instructions per 16 values of k where three bf16 parts (bf16x3.hpp) take six, and 4 bytes an operand instead of 6.
 // What it loses in the operands, 2^-24 of a product at random, it gains back in the accumulator, which is rounded once per matrix instruction:
